@@ -110,8 +110,12 @@ int mx_sample(const void* logits, int is_bf16, int64_t* out, int B, int V, float
 int mx_sample_temp_rows(const void* logits, int is_bf16, int64_t* out, int B, int V, const float* temps,
                         const int64_t* seeds, const int32_t* steps, float* ws, hipStream_t stream);
 // sampling.hip
+int64_t mx_sample_rows_ws(int B, int V);
 int mx_sample_rows(const void* logits, int is_bf16, int64_t* out, int B, int V, const float* temps,
-                   const float* top_ps, const int32_t* top_ks, const int64_t* seeds, const int32_t* steps,
+                   const float* top_ps, const int32_t* top_ks, const int64_t* seeds, const int32_t* steps, void* ws,
+                   hipStream_t stream);
+int mx_sample_list(const void* logits, int is_bf16, int64_t* out, int B, int V, const double* temps,
+                   const double* top_ps, const int64_t* top_ks, const int64_t* seeds, const int64_t* steps, void* ws,
                    hipStream_t stream);
 }
 

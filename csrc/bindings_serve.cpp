@@ -151,10 +151,29 @@ at::Tensor sample_rows(const at::Tensor& logits, const at::Tensor& temps, const 
   chk(steps, at::kInt, "steps i32 [B]");
   DevGuard g(logits.device());
   auto out = at::empty({B}, logits.options().dtype(at::kLong));
+  auto ws = at::empty({mx_sample_rows_ws((int)B, (int)logits.size(1))}, logits.options().dtype(at::kByte));
   MX_OK(mx_sample_rows(logits.data_ptr(), logits.scalar_type() == at::kBFloat16 ? 1 : 0, out.data_ptr<int64_t>(),
                        (int)B, (int)logits.size(1), temps.data_ptr<float>(), top_p.data_ptr<float>(),
                        top_k.data_ptr<int32_t>(), seeds.data_ptr<int64_t>(), steps.data_ptr<int32_t>(),
-                       cur_stream()));
+                       ws.data_ptr(), cur_stream()));
+  return out;
+}
+
+// the parameters as lists: nothing is copied to the device for them
+at::Tensor sample_list(const at::Tensor& logits, at::ArrayRef<double> temps, at::ArrayRef<double> top_p,
+                       at::IntArrayRef top_k, at::IntArrayRef seeds, at::IntArrayRef steps) {
+  MX_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.dim() == 2, "logits [B, V] contiguous GPU");
+  MX_CHECK(logits.scalar_type() == at::kBFloat16 || logits.scalar_type() == at::kFloat, "logits bf16/f32");
+  const int64_t B = logits.size(0);
+  MX_CHECK((int64_t)temps.size() == B && (int64_t)top_p.size() == B && (int64_t)top_k.size() == B &&
+               (int64_t)seeds.size() == B && (int64_t)steps.size() == B,
+           "one temperature, top_p, top_k, seed and step a row");
+  DevGuard g(logits.device());
+  auto out = at::empty({B}, logits.options().dtype(at::kLong));
+  auto ws = at::empty({mx_sample_rows_ws((int)B, (int)logits.size(1))}, logits.options().dtype(at::kByte));
+  MX_OK(mx_sample_list(logits.data_ptr(), logits.scalar_type() == at::kBFloat16 ? 1 : 0, out.data_ptr<int64_t>(),
+                       (int)B, (int)logits.size(1), temps.data(), top_p.data(), top_k.data(), seeds.data(),
+                       steps.data(), ws.data_ptr(), cur_stream()));
   return out;
 }
 
@@ -283,6 +302,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
   m.def("sample(Tensor logits, float temperature, int seed, int step) -> Tensor");
   m.def("sample_rows(Tensor logits, Tensor temps, Tensor top_p, Tensor top_k, Tensor seeds, Tensor steps) -> Tensor");
+  m.def("sample_list(Tensor logits, float[] temps, float[] top_p, int[] top_k, int[] seeds, int[] steps) -> Tensor");
   m.def("sample_temp_rows(Tensor logits, Tensor temps, Tensor seeds, Tensor steps) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear_swiglu(Tensor x, Tensor w) -> Tensor");
@@ -297,6 +317,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn", &decode_attn);
   m.impl("sample", &sample);
   m.impl("sample_rows", &sample_rows);
+  m.impl("sample_list", &sample_list);
   m.impl("sample_temp_rows", &sample_temp_rows);
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny_linear_swiglu", &skinny_linear_swiglu);

@@ -98,9 +98,9 @@ def sample_rows(logits: torch.Tensor, temps, top_ps, top_ks, seeds, steps) -> to
     """Batched sampling with per-row parameters (OpenAI semantics): softmax of
     logits / T, keep the top_k most likely (k <= 0: all), then the smallest
     most-likely prefix whose mass reaches top_p, renormalise, draw; T <= 0 is
-    greedy.  GPU: ONE launch for the whole batch (csrc/kernels/sampling.hip:
-    radix-select thresholds + Gumbel-max over the kept set, keyed by
-    (seed, step, token) so a request's draws do not depend on batching).
+    greedy.  GPU: csrc/kernels/sampling.hip (thresholds from a histogram of the row +
+    Gumbel-max over the kept set, keyed by (seed, step, token) so a request's draws do
+    not depend on batching; the parameters travel with the launches).
     CPU: ``filter_probs`` + torch.multinomial.  ``top_p <= 0`` (an empty nucleus)
     is the limit of a vanishing nucleus: that row is sampled greedily on both paths;
     a NaN top_p / temperature is rejected."""
@@ -117,16 +117,8 @@ def sample_rows(logits: torch.Tensor, temps, top_ps, top_ks, seeds, steps) -> to
         x = x.contiguous()
         if all(t <= 0 for t in temps):
             return ops.sample(x, 0.0, 0, 0)  # batched greedy: one argmax pass
-        dev = logits.device
-        prm = torch.tensor([[float(t), float(p), float(k)] for t, p, k in zip(temps, top_ps, top_ks)],
-                           dtype=torch.float32).pin_memory().to(dev, non_blocking=True)
-        st = torch.tensor([[int(sd), int(sp)] for sd, sp in zip(seeds, steps)], dtype=torch.int64).pin_memory()
-        st = st.to(dev, non_blocking=True)
-        if all(p >= 1.0 for p in top_ps) and all(k <= 0 for k in top_ks):
-            # temperature / greedy rows only: the vocabulary-split kernel (same draws)
-            return ops.sample_temp_rows(x, prm[:, 0].contiguous(), st[:, 0].contiguous(), st[:, 1].int().contiguous())
-        return ops.sample_rows(x, prm[:, 0].contiguous(), prm[:, 1].contiguous(), prm[:, 2].int().contiguous(),
-                               st[:, 0].contiguous(), st[:, 1].int().contiguous())
+        return ops.sample_list(x, [float(t) for t in temps], [float(p) for p in top_ps], [int(k) for k in top_ks],
+                               [int(sd) for sd in seeds], [int(sp) for sp in steps])
     out = torch.empty(B, dtype=torch.long)
     for i in range(B):
         if temps[i] <= 0:

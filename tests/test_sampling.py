@@ -128,3 +128,77 @@ def test_concurrent_samplers_on_two_streams(gpu):
     for k in range(2):
         for o in outs[k]:
             assert torch.equal(o, want[k])
+
+
+def _scores(V: int, seed: int, step: int):
+    """The sampler's Gumbel noise of a row, and how far the hardware logarithm may be from it: its error of 2^-23
+    weighs as much more as -log(u) is below one."""
+    import numpy as np
+
+    u32 = np.uint32
+    with np.errstate(over="ignore"):
+        a, b = u32(seed & 0xFFFFFFFF) * u32(0x9E3779B1), (u32(step) + u32(0x7F4A7C15)) * u32(0x85EBCA77)
+        h = a ^ b ^ ((np.arange(V, dtype=u32) + u32(0x165667B1)) * u32(0xC2B2AE3D))
+        h ^= h >> u32(15)
+        h *= u32(0x2C1B3C6D)
+        h ^= h >> u32(12)
+        h *= u32(0x297A2D39)
+        h ^= h >> u32(15)
+    u = ((h >> u32(8)).astype(np.float32) + np.float32(0.5)).astype(np.float64) / 16777216.0  # rounded as on the device
+    e = np.maximum(-np.log(u), 2.0 ** -25)
+    return torch.from_numpy(-np.log(e)), torch.from_numpy(2.0 ** -22 / e + 1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,dtype", [(16383, torch.float32), (16384, torch.bfloat16), (16385, torch.float32),
+                                     (50257, torch.bfloat16), (128256, torch.float32), (128256, torch.bfloat16)])
+@pytest.mark.parametrize("shape", ["normal", "flat", "equal", "masked", "peaked"])
+def test_gpu_split_sampler_draws(gpu, V, dtype, shape):
+    """The draw of every row is the best Gumbel score among the tokens that top-k and top-p keep, both computed in
+    f64 (rows whose runner-up or boundary lies within rounding are left out; 70 rows: two launches)."""
+    g = torch.Generator().manual_seed(V)
+    B = 70
+    x = torch.randn(B, V, generator=g) * {"normal": 2.5, "flat": 0.01, "equal": 0.0, "masked": 2.0, "peaked": 9.0}[shape]
+    x += 1.5 * (shape == "equal")
+    if shape == "masked":
+        x[:, torch.rand(V, generator=g) < 0.7] = float("-inf")
+    x = x.to(dtype)
+    temps = [[0.8, 1.0, 0.0, 0.6, 1.7][i % 5] for i in range(B)]
+    tops = [[0.9, 1.0, 0.5, 0.999, 0.02, 0.95, 0.7][i % 7] for i in range(B)]
+    ks = [[0, 40, 1, 5000, 0, V, 3, 0, 900][i % 9] for i in range(B)]
+    seeds, steps = [(i * 2654435761) % (1 << 40) for i in range(B)], [i * 3 for i in range(B)]
+    got = dops.sample_rows(x.to(gpu), temps, tops, ks, seeds, steps).cpu()
+    from mxllm.ops import native
+
+    dev = [torch.tensor(t, dtype=d, device=gpu) for t, d in zip(
+        (temps, tops, ks, seeds, steps), (torch.float32, torch.float32, torch.int32, torch.int64, torch.int32))]
+    assert torch.equal(native().sample_rows(x.to(gpu), *dev).cpu(), got)
+    checked = 0
+    for i in range(B):
+        row = x[i].double()
+        if temps[i] <= 0:
+            assert got[i] == row.argmax()
+            continue
+        t = float(torch.tensor(temps[i], dtype=torch.float32))
+        keep = row > float("-inf")
+        if 0 < ks[i] < V:
+            keep &= row >= torch.topk(row, ks[i]).values[-1]
+        w = torch.where(keep, torch.exp((row - row.max()) / t), 0.0)
+        vals, inv = torch.unique(row, return_inverse=True)  # tokens of one value stay together
+        mass = torch.zeros(len(vals), dtype=torch.float64).index_add_(0, inv, w)
+        above = (mass.flip(0).cumsum(0).flip(0) - mass)[inv]
+        if tops[i] < 1:
+            p = float(torch.tensor(tops[i], dtype=torch.float32)) * w.sum()
+            if (above[keep] - p).abs().min() < 1e-5 * w.sum():  # 2^17 masses of 2^-24 relative rounding, in f32
+                continue
+            keep &= above < p
+        noise, err = _scores(V, seeds[i], steps[i])
+        s = torch.where(keep, row / t + noise, float("-inf"))
+        best = int((s - err).argmax())
+        assert keep[got[i]], (i, temps[i], tops[i], ks[i])
+        rest = s + err
+        rest[best] = float("-inf")
+        if (s - err)[best] > rest.max():
+            assert got[i] == best, (i, temps[i], tops[i], ks[i])
+            checked += 1
+    assert checked > B // 5
