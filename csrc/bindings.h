@@ -123,6 +123,8 @@ extern "C" {
 // fp8_gemm.hip
 int mx_skinny_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y, int64_t ldy,
                    int M, int N, int K, hipStream_t stream);
+int mx_skinny_gemm_half(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y, int64_t ldy, int M,
+                        int N, int K, hipStream_t stream);
 int mx_skinny_gemm_swiglu(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y,
                           int64_t ldy, int M, int F, int K, hipStream_t stream);
 int mx_skinny_rope_gemm(const uint16_t* h, int64_t ldh, int norm, const uint16_t* delta, int64_t ldd,

@@ -194,6 +194,19 @@ at::Tensor skinny_linear(const at::Tensor& x, const at::Tensor& w) {
   return y;
 }
 
+// the same for M <= 8 by groups of 8 channels: projections whose groups of 16 leave CUs idle
+at::Tensor skinny_linear_half(const at::Tensor& x, const at::Tensor& w) {
+  MX_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1, "x: bf16 [M, K] rows");
+  MX_CHECK(w.is_cuda() && w.scalar_type() == at::kBFloat16 && w.dim() == 2 && w.stride(1) == 1, "w: bf16 [N, K] rows");
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  MX_CHECK(w.size(1) == K && M >= 1 && M <= 8 && N % 8 == 0 && K % 1024 == 0 && x.stride(0) % 8 == 0 &&
+               w.stride(0) % 8 == 0, "skinny_linear_half shape contract");
+  DevGuard g(x.device());
+  auto y = at::empty({M, N}, x.options());
+  MX_OK(mx_skinny_gemm_half(bf(x), x.stride(0), bf(w), w.stride(0), bfm(y), N, (int)M, (int)N, (int)K, cur_stream()));
+  return y;
+}
+
 // y[M, F] = swiglu(x[M, K] . w[2F, K]^T) for M <= 32 tokens, w = [gate; up] rows: the decode
 // MLP's first projection with SwiGLU in the GEMM epilogue (csrc/kernels/skinny_gemm.hip).
 at::Tensor skinny_linear_swiglu(const at::Tensor& x, const at::Tensor& w) {
@@ -305,6 +318,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("sample_list(Tensor logits, float[] temps, float[] top_p, int[] top_k, int[] seeds, int[] steps) -> Tensor");
   m.def("sample_temp_rows(Tensor logits, Tensor temps, Tensor seeds, Tensor steps) -> Tensor");
   m.def("skinny_linear(Tensor x, Tensor w) -> Tensor");
+  m.def("skinny_linear_half(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_linear_swiglu(Tensor x, Tensor w) -> Tensor");
   m.def("skinny_qkv_rope(Tensor h, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor cos, Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, Tensor? block_table=None) -> (Tensor, Tensor)");
   m.def("skinny_norm_linear(Tensor h, Tensor? delta, Tensor gamma, float eps, Tensor w, bool swiglu) -> (Tensor, Tensor)");
@@ -320,6 +334,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("sample_list", &sample_list);
   m.impl("sample_temp_rows", &sample_temp_rows);
   m.impl("skinny_linear", &skinny_linear);
+  m.impl("skinny_linear_half", &skinny_linear_half);
   m.impl("skinny_linear_swiglu", &skinny_linear_swiglu);
   m.impl("skinny_qkv_rope", &skinny_qkv_rope);
   m.impl("skinny_norm_linear", &skinny_norm_linear);

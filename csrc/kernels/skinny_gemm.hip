@@ -38,7 +38,9 @@ namespace mx {
 // MB: 16-token blocks (1 or 2); X rows >= M are clamped to M-1 and discarded.
 // NC: 16-channel groups per workgroup: each X fragment then feeds NC MFMAs, so X traffic per
 // streamed weight byte drops NC-fold (it equals the weight traffic at 16 tokens with NC = 1).
-template <int MB, int NC, bool SWO = false, bool NORM = false, bool ROPE = false, bool MERGE = false>
+// HALF: 8 channels a workgroup (M <= 8): fragment row r takes channel r & 7 and half r >> 3 of the wave's K part,
+// token column c token c & 7 and the same half, and the two diagonal blocks of the product are added.
+template <int MB, int NC, bool SWO = false, bool NORM = false, bool ROPE = false, bool MERGE = false, bool HALF = false>
 __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __restrict__ X, int64_t ldx,
                                                           const uint16_t* __restrict__ W, int64_t ldw,
                                                           uint16_t* __restrict__ Y, int64_t ldy, int M, int K,
@@ -48,24 +50,26 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
   static_assert(!ROPE || (NC == 1 && !SWO), "RoPE epilogue: one channel group");
   static_assert(!NORM || (MB == 1 && NC == 1), "fused RMSNorm: <= 16 rows, one channel group");
   static_assert(!MERGE || (MB == 1 && NC == 1 && !NORM && !SWO && !ROPE), "fused split merge: plain GEMM rows");
+  static_assert(!HALF || (MB == 1 && NC == 1 && !SWO && !NORM && !ROPE && !MERGE), "half groups: plain GEMM rows");
   constexpr bool LDSX = NORM || MERGE;  // X rows built in LDS by the prologue
   constexpr int NW = kSkWaves, UNR = sk_unr(NC);
   __shared__ f32x4 red[NW][NC][MB][64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NC;
+  const int n0 = blockIdx.x * (HALF ? 8 : 16 * NC);
   const int kq = K / NW;  // this wave's K part
+  const int kh = HALF && c >= 8 ? kq / 2 : 0;
   const uint16_t* wrow[NC];
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
     // SWO: channel c < 8 -> gate row blockIdx.x * 8 + c, c >= 8 -> the matching up row
     // ROPE: head blockIdx.x / 8, pair base 8 (blockIdx.x % 8); c >= 8 -> the second-half row
-    const int64_t wr = (SWO || ROPE) ? dfuse_row<SWO>(blockIdx.x, c, F) : (int64_t)(n0 + 16 * j + c);
-    wrow[j] = W + wr * ldw + (int64_t)w * kq + 16 * g;
+    const int64_t wr = (SWO || ROPE) ? dfuse_row<SWO>(blockIdx.x, c, F) : (int64_t)(n0 + 16 * j + (HALF ? c & 7 : c));
+    wrow[j] = W + wr * ldw + (int64_t)w * kq + kh + 16 * g;
   }
   const uint16_t* xr[MB];
-  const int nit = kq / 64;
+  const int nit = kq / (HALF ? 128 : 64);
   // NORM: the first UNR chunks' weight loads go out before the prologue, so the weight stream's
   // latency overlaps the RMSNorm instead of following it
   u16x8 apre[UNR][NC][2];
@@ -83,7 +87,8 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
     for (int mb = 0; mb < MB; ++mb) xr[mb] = xs + (int64_t)min(mb * 16 + c, M - 1) * K + (int64_t)w * kq + 16 * g;
   } else {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) xr[mb] = X + (int64_t)min(mb * 16 + c, M - 1) * ldx + (int64_t)w * kq + 16 * g;
+    for (int mb = 0; mb < MB; ++mb)
+      xr[mb] = X + (int64_t)min(mb * 16 + (HALF ? c & 7 : c), M - 1) * ldx + (int64_t)w * kq + kh + 16 * g;
   }
 
   f32x4 acc[NC][MB];
@@ -103,7 +108,12 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
 #pragma unroll
         for (int ww = 1; ww < NW; ++ww) s += red[ww][j][mb][lane];
         const int m = mb * 16 + c;
-        if constexpr (ROPE) {
+        if constexpr (HALF) {  // (channel, token) of the first halves + (channel + 8, token + 8) of the second
+          u16x4 o;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i] + __shfl_xor(s[i], 40, 64));
+          if (c < 8 && g < 2 && c < M) *reinterpret_cast<u16x4*>(Y + (int64_t)c * ldy + n0 + 4 * g) = o;
+        } else if constexpr (ROPE) {
           dfuse_rope_store(s, g, m, M, blockIdx.x, rp);
         } else if constexpr (SWO) {
           dfuse_swiglu_store(s, g, m, M, Y, ldy, blockIdx.x);
@@ -210,6 +220,18 @@ extern "C" int mx_skinny_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w,
     if (nc >= 4) SKG(2, 4); else if (nc == 2) SKG(2, 2); else SKG(2, 1);
   }
 #undef SKG
+  return (int)hipGetLastError();
+}
+
+// The same for up to 8 rows by groups of 8 channels (HALF): twice the workgroups, where 16 channels each leave CUs
+// without one.  2048 channels, one row: K 8192 13.1 -> 10.0 us, K 12288 19.2 -> 13.0, K 2048 5.1 -> 4.1 (8 rows:
+// 15.0 -> 12.9, 21.9 -> 17.3, 5.4 -> 4.7).  The halves of a wave's K part are summed apart: other bits than above.
+// K % 1024 == 0, N % 8 == 0.
+extern "C" int mx_skinny_gemm_half(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y,
+                                   int64_t ldy, int M, int N, int K, hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > 8 || N % 8 || K % 1024 || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K || ldw < K || ldy < N) return -1;
+  skinny_gemm_kernel<1, 1, false, false, false, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
   return (int)hipGetLastError();
 }
 

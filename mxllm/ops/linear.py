@@ -569,6 +569,9 @@ def normed_linear(x: torch.Tensor, h: torch.Tensor, nw: torch.Tensor, eps: float
 # projections; the 70B ones lost at 4 rows).  MXLLM_SKINNY_M=0 keeps every GEMM on hipBLASLt.
 SKINNY_M = int(os.environ.get("MXLLM_SKINNY_M", "8"))
 _SKINNY_SMALL_W = 128 << 20
+# output channels below which 16 a workgroup leave some of the 256 CUs without one: 8 a workgroup (at 4096 and
+# more no gain)
+_HALF_N = 4096
 
 
 def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
@@ -586,7 +589,9 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and x.numel() // max(x.shape[-1], 1) <= SKINNY_M:
         x2 = x.reshape(-1, x.shape[-1])
         if x2.shape[0] > 0 and _skinny_ok(x2, w):
-            return native().skinny_linear(x2, w).view(*x.shape[:-1], w.shape[0])
+            half = w.shape[0] < _HALF_N and w.shape[1] % 1024 == 0 and x2.shape[0] <= 8
+            fn = native().skinny_linear_half if half else native().skinny_linear
+            return fn(x2, w).view(*x.shape[:-1], w.shape[0])
     return F.linear(x, w)
 
 

@@ -855,3 +855,14 @@ def test_embedding_bwd_sorted_dominant_id(gpu, f32):
     ref = torch.zeros(V, H, device=gpu, dtype=torch.float64).index_add_(0, ids, dy.double())
     assert rel_err(outs[0], ref) < (1e-5 if f32 else 5e-3)
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 2048, 8192), (8, 8, 1024), (5, 2056, 3072), (3, 40, 12288), (7, 4080, 2048)])
+def test_skinny_linear_half(gpu, M, N, K):
+    """Decode GEMM by groups of 8 channels against fp64: one group, odd row counts, K parts of one to twelve chunks."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K + 64, device=gpu, dtype=torch.bfloat16)[:, :K]
+    w = torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05
+    y = _ops().skinny_linear_half(x, w)
+    assert y.shape == (M, N) and rel_err(y, x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
