@@ -100,6 +100,98 @@ at::Tensor skinny_merge_linear(const at::Tensor& ml, const at::Tensor& po, const
   return y;
 }
 
+// ---------------------------------------------------------------- decode GEMMs that stay (csrc/kernels/stream_gemm.hip)
+// w bf16 [N, K] rows, or e4m3 codes (uint8) with scale f32 [N]
+struct StreamOperands {
+  const uint16_t *x, *delta = nullptr, *gamma = nullptr;
+  const float* scale = nullptr;
+  int64_t M, K, N, ldd = 0;
+  at::Tensor h_out;
+};
+
+StreamOperands stream_operands(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
+                               const c10::optional<at::Tensor>& gamma, const at::Tensor& w,
+                               const c10::optional<at::Tensor>& scale) {
+  StreamOperands o;
+  MX_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1, "x: bf16 [M, K] rows");
+  MX_CHECK(w.is_cuda() && w.dim() == 2 && w.stride(1) == 1 && w.device() == x.device(), "w: [N, K] rows on x's device");
+  o.M = x.size(0), o.K = x.size(1), o.N = w.size(0);
+  if (scale.has_value() && scale->defined()) {
+    MX_CHECK(w.scalar_type() == at::kByte && scale->is_cuda() && scale->scalar_type() == at::kFloat &&
+                 scale->is_contiguous() && scale->numel() == o.N && w.stride(0) % 16 == 0,
+             "e4m3 weights: uint8 [N, K] rows, scale f32 [N]");
+    o.scale = scale->data_ptr<float>();
+  } else {
+    MX_CHECK(w.scalar_type() == at::kBFloat16 && w.stride(0) % 8 == 0, "w: bf16 [N, K] rows");
+  }
+  const bool norm = gamma.has_value() && gamma->defined();
+  MX_CHECK(w.size(1) == o.K && o.N % 16 == 0 && x.stride(0) % 8 == 0 && mx_stream_ok((int)o.M, (int)o.K, norm),
+           "stream GEMM shape contract");
+  o.x = bf(x);
+  o.h_out = x;
+  if (norm) {
+    MX_CHECK(gamma->is_cuda() && gamma->scalar_type() == at::kBFloat16 && gamma->is_contiguous() && gamma->numel() == o.K,
+             "gamma: bf16 [K]");
+    o.gamma = bf(*gamma);
+    if (delta.has_value() && delta->defined()) {
+      const at::Tensor& d = *delta;
+      MX_CHECK(d.is_cuda() && d.scalar_type() == at::kBFloat16 && d.dim() == 2 && d.size(0) == o.M && d.size(1) == o.K &&
+                   d.stride(1) == 1 && d.stride(0) % 8 == 0, "delta: bf16 [M, K] rows");
+      o.delta = bf(d);
+      o.ldd = d.stride(0);
+      o.h_out = at::empty({o.M, o.K}, x.options());
+    }
+  }
+  return o;
+}
+
+// y = [swiglu](x . w^T); with gamma x = rmsnorm(h + delta), up to 4 rows.  Returns (y, h + delta).
+std::tuple<at::Tensor, at::Tensor> stream_linear(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
+                                                 const c10::optional<at::Tensor>& gamma, double eps, const at::Tensor& w,
+                                                 const c10::optional<at::Tensor>& scale, bool swiglu) {
+  DevGuard g(x.device());
+  StreamOperands o = stream_operands(x, delta, gamma, w, scale);
+  const int64_t Ny = swiglu ? o.N / 2 : o.N;
+  auto y = at::empty({o.M, Ny}, x.options());
+  MX_OK(mx_stream_gemm(o.x, x.stride(0), w.data_ptr(), w.stride(0), o.scale, bfm(y), Ny, (int)o.M, (int)o.N, (int)o.K,
+                       swiglu ? 1 : 0, o.delta, o.ldd, o.gamma, (float)eps, o.delta ? bfm(o.h_out) : nullptr, nullptr,
+                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0, cur_stream()));
+  return {y, o.h_out};
+}
+
+// the QKV projection with RoPE and the cache append in the epilogue, heads of 64 or 128: (q [M, Hq, D], h + delta)
+std::tuple<at::Tensor, at::Tensor> stream_qkv_rope(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
+                                                   const c10::optional<at::Tensor>& gamma, double eps,
+                                                   const at::Tensor& w, const c10::optional<at::Tensor>& scale,
+                                                   const at::Tensor& cosb, const at::Tensor& sinb,
+                                                   const at::Tensor& pos, const c10::optional<at::Tensor>& slots,
+                                                   at::Tensor& k_cache, at::Tensor& v_cache, int64_t Hq, int64_t Hkv,
+                                                   const c10::optional<at::Tensor>& block_table) {
+  DevGuard g(x.device());
+  StreamOperands o = stream_operands(x, delta, gamma, w, scale);
+  const int64_t D = k_cache.size(3);
+  MX_CHECK((D == 64 || D == 128) && o.N == (Hq + 2 * Hkv) * D, "heads of 64 or 128");
+  MX_CHECK(cosb.scalar_type() == at::kFloat && sinb.scalar_type() == at::kFloat && cosb.is_contiguous() &&
+               sinb.is_contiguous() && cosb.size(-1) == D / 2 && sinb.size(-1) == D / 2, "cos/sin f32 [max_pos, D / 2]");
+  MX_CHECK(pos.scalar_type() == at::kInt && pos.numel() == o.M && pos.is_contiguous(), "pos int32 [M]");
+  check_bf16(k_cache, "k_cache");
+  check_bf16(v_cache, "v_cache");
+  MX_CHECK(k_cache.size(1) == Hkv && v_cache.sizes() == k_cache.sizes() && k_cache.is_contiguous() &&
+               v_cache.is_contiguous(), "caches [slots, Hkv, max_seq, D]");
+  const int32_t* sl = nullptr;
+  if (slots.has_value() && slots->defined()) {
+    MX_CHECK(slots->scalar_type() == at::kInt && slots->numel() == o.M && slots->is_contiguous(), "slots int32 [M]");
+    sl = slots->data_ptr<int32_t>();
+  }
+  const KvPages pg = kv_pages(block_table, k_cache);
+  auto q = at::empty({o.M, Hq, D}, x.options());
+  MX_OK(mx_stream_gemm(o.x, x.stride(0), w.data_ptr(), w.stride(0), o.scale, nullptr, 0, (int)o.M, (int)o.N, (int)o.K,
+                       D == 128 ? 2 : 3, o.delta, o.ldd, o.gamma, (float)eps, o.delta ? bfm(o.h_out) : nullptr,
+                       cosb.data_ptr<float>(), sinb.data_ptr<float>(), pos.data_ptr<int32_t>(), sl, bfm(q), bfm(k_cache),
+                       bfm(v_cache), (int)Hq, (int)Hkv, (int)k_cache.size(2), pg.bt, pg.maxb, cur_stream()));
+  return {q, o.h_out};
+}
+
 at::Tensor sample(const at::Tensor& logits, double temperature, int64_t seed, int64_t step) {
   MX_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.dim() == 2, "logits [B, V] contiguous GPU");
   MX_CHECK(logits.scalar_type() == at::kBFloat16 || logits.scalar_type() == at::kFloat, "logits bf16/f32");
@@ -313,6 +405,10 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor lens, Tensor? slots, int max_len, float scale, int len_off=0, Tensor? block_table=None, Tensor? counters=None) -> Tensor");
   m.def("decode_attn_partials(Tensor q, Tensor k_cache, Tensor v_cache, Tensor lens, Tensor? slots, int max_len, float scale, int len_off=0, Tensor? block_table=None) -> (Tensor, Tensor)");
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
+  m.def("stream_linear(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, bool swiglu) -> (Tensor, Tensor)");
+  m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
+        "Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, "
+        "Tensor? block_table) -> (Tensor, Tensor)");
   m.def("sample(Tensor logits, float temperature, int seed, int step) -> Tensor");
   m.def("sample_rows(Tensor logits, Tensor temps, Tensor top_p, Tensor top_k, Tensor seeds, Tensor steps) -> Tensor");
   m.def("sample_list(Tensor logits, float[] temps, float[] top_p, int[] top_k, int[] seeds, int[] steps) -> Tensor");
@@ -329,6 +425,8 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn_partials", &decode_attn_partials);
   m.impl("skinny_merge_linear", &skinny_merge_linear);
   m.impl("decode_attn", &decode_attn);
+  m.impl("stream_linear", &stream_linear);
+  m.impl("stream_qkv_rope", &stream_qkv_rope);
   m.impl("sample", &sample);
   m.impl("sample_rows", &sample_rows);
   m.impl("sample_list", &sample_list);

@@ -20,12 +20,12 @@ struct SkNorm {
 };
 
 struct SkRope {
-  const float* cosb;     // [max_pos, 64]
+  const float* cosb;     // [max_pos, D / 2]
   const float* sinb;
   const int32_t* pos;    // [M] position of the new token
   const int32_t* slots;  // [M] cache slot (nullptr: row index)
-  uint16_t* q;           // [M, Hq, 128]
-  uint16_t* kc;          // [slots, Hkv, max_seq, 128], or paged [blocks, Hkv, block, 128]
+  uint16_t* q;           // [M, Hq, D]
+  uint16_t* kc;          // [slots, Hkv, max_seq, D], or paged [blocks, Hkv, block, D]
   uint16_t* vc;
   int Hq, Hkv, max_seq;  // max_seq: the cache's sequence dimension (the block size when paged)
   const int32_t* bt;     // paged: block table [slots, maxb] (nullptr: contiguous)
@@ -34,18 +34,21 @@ struct SkRope {
 
 // Weight row of channel c (0..15) of workgroup blk in the paired layouts:
 //  SWO : 8 gate rows blk*8 .. +7 and the matching up rows F + blk*8 .. +7;
-//  ROPE: head blk/8, first-half rows 8 (blk%8) .. +7 and the matching second-half rows (+64).
-template <bool SWO>
+//  ROPE (heads of D = 2 HD): D / 16 workgroups a head, each 8 first-half rows and the matching second-half
+//  rows (+ HD).
+template <bool SWO, int HD = 64>
 __device__ __forceinline__ int64_t dfuse_row(int blk, int c, int F) {
+  constexpr int PH = HD / 8;
   if constexpr (SWO) return (int64_t)blk * 8 + (c & 7) + (c >= 8 ? F : 0);
-  else return (int64_t)(blk >> 3) * 128 + (blk & 7) * 8 + (c & 7) + (c >= 8 ? 64 : 0);
+  else return (int64_t)(blk / PH) * (2 * HD) + (blk % PH) * 8 + (c & 7) + (c >= 8 ? HD : 0);
 }
 
-// RMSNorm (with the residual add when na.delta) of M <= 4 rows of X into xs [M, K] (LDS),
+// RMSNorm (with the residual add when na.delta) of M <= 4 rows of X into xs [M, K] (LDS, row stride lds),
 // by a 512-thread workgroup: rows m = q, q + 2, ... by wave group q, each group with
 // rmsnorm.hip's 256-thread mapping and summation order.  Workgroup 0 stores h + delta.
 __device__ __forceinline__ void dfuse_norm_rows(const uint16_t* __restrict__ X, int64_t ldx, int M, int K,
-                                                const SkNorm& na, uint16_t* xs, float (*nscr)[4], float* nrs) {
+                                                const SkNorm& na, uint16_t* xs, int lds, float (*nscr)[4],
+                                                float* nrs) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int q = w >> 2, tq = tid & 255;
   for (int m0 = 0; m0 < M; m0 += 2) {
@@ -66,7 +69,7 @@ __device__ __forceinline__ void dfuse_norm_rows(const uint16_t* __restrict__ X, 
           const float v = bf2f(hb[j]);
           ss += v * v;
         }
-        *reinterpret_cast<u16x8*>(xs + (int64_t)m * K + cc) = hb;
+        *reinterpret_cast<u16x8*>(xs + (int64_t)m * lds + cc) = hb;
       }
     }
     ss = wave_sum(ss);
@@ -86,7 +89,7 @@ __device__ __forceinline__ void dfuse_norm_rows(const uint16_t* __restrict__ X, 
     if (m < M) {
       const float rs = nrs[m];
       for (int cc = tq * 8; cc < K; cc += 2048) {
-        u16x8* px = reinterpret_cast<u16x8*>(xs + (int64_t)m * K + cc);
+        u16x8* px = reinterpret_cast<u16x8*>(xs + (int64_t)m * lds + cc);
         const u16x8 hb = *px;
         const u16x8 gw = *reinterpret_cast<const u16x8*>(na.gamma + cc);
         u16x8 o;
@@ -184,12 +187,14 @@ __device__ __forceinline__ void dfuse_swiglu_store(const f32x4& v, int g, int m,
   }
 }
 
+template <int HD = 64>
 __device__ __forceinline__ void dfuse_rope_store(const f32x4& v, int g, int m, int M, int blk, const SkRope& rp) {
   f32x4 hi;
 #pragma unroll
   for (int i = 0; i < 4; ++i) hi[i] = __shfl_xor(v[i], 32, 64);
   if (g < 2 && m < M) {
-    const int head = blk >> 3, i0 = (blk & 7) * 8 + 4 * g;
+    constexpr int PH = HD / 8;
+    const int head = blk / PH, i0 = (blk % PH) * 8 + 4 * g;
     const int p = rp.pos[m];
     const int slot = rp.slots ? rp.slots[m] : m;
     u16x4 y1, y2;
@@ -197,21 +202,21 @@ __device__ __forceinline__ void dfuse_rope_store(const f32x4& v, int g, int m, i
     if (head >= rp.Hq + rp.Hkv) {  // v: no rotation
 #pragma unroll
       for (int i = 0; i < 4; ++i) y1[i] = f2bf(v[i]), y2[i] = f2bf(hi[i]);
-      dst = rp.vc + kv_row(rp.bt, rp.maxb, rp.max_seq, slot, rp.Hkv, head - rp.Hq - rp.Hkv, p) * 128;
+      dst = rp.vc + kv_row(rp.bt, rp.maxb, rp.max_seq, slot, rp.Hkv, head - rp.Hq - rp.Hkv, p) * (2 * HD);
     } else {
-      const float* cp = rp.cosb + (int64_t)p * 64 + i0;
-      const float* sp = rp.sinb + (int64_t)p * 64 + i0;
+      const float* cp = rp.cosb + (int64_t)p * HD + i0;
+      const float* sp = rp.sinb + (int64_t)p * HD + i0;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {  // rope_append's arithmetic on the bf16-rounded projection
         const float a = bf2f(f2bf(v[i])), bb = bf2f(f2bf(hi[i]));
         y1[i] = f2bf(a * cp[i] - bb * sp[i]);
         y2[i] = f2bf(bb * cp[i] + a * sp[i]);
       }
-      dst = head < rp.Hq ? rp.q + ((int64_t)m * rp.Hq + head) * 128
-                         : rp.kc + kv_row(rp.bt, rp.maxb, rp.max_seq, slot, rp.Hkv, head - rp.Hq, p) * 128;
+      dst = head < rp.Hq ? rp.q + ((int64_t)m * rp.Hq + head) * (2 * HD)
+                         : rp.kc + kv_row(rp.bt, rp.maxb, rp.max_seq, slot, rp.Hkv, head - rp.Hq, p) * (2 * HD);
     }
     *reinterpret_cast<u16x4*>(dst + i0) = y1;
-    *reinterpret_cast<u16x4*>(dst + 64 + i0) = y2;
+    *reinterpret_cast<u16x4*>(dst + HD + i0) = y2;
   }
 }
 

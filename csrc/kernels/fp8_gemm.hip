@@ -14,37 +14,14 @@
 //  * each lane loads 16 contiguous fp8 bytes (k = 16g .. 16g+15 of a 64-k chunk), so
 //    the two MFMA k-steps of the chunk take k = 16g + 8s + j (permuted inside the
 //    chunk); the X fragments use the same permutation (16-B bf16 loads);
-//  * dequantisation without a conversion table: the quantiser never emits a zero or
-//    subnormal code (see mxllm/serve/quant.py), so for every code
-//    bf16 = sign<<15 | ((e4m3 & 0x7F) << 4) + (120 << 7)   (exponent rebias 7 -> 127),
-//    two bytes at a time with 32-bit ALU ops (byte permute, and, shift-add, and-or);
+//  * dequantisation by the hardware's fp8 -> bf16 pair conversion (e4m3.h; exact);
 //  * the per-channel scale is applied once in the epilogue.
 #include <cstdlib>
 
-#include "common.h"
+#include "e4m3.h"
+#include "skinny_core.h"
 
 namespace mx {
-
-typedef __bf16 bf16x8_f8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f32x4 mfma16_f8(const u16x8& a, const u16x8& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_f8, a), __builtin_bit_cast(bf16x8_f8, b),
-                                                 c, 0, 0, 0);
-}
-
-// two e4m3 bytes (bits 0-7 and 8-15 of w16) -> packed bf16x2
-__device__ __forceinline__ uint32_t e4m3x2_to_bf16x2(uint32_t w) {
-  const uint32_t x = __builtin_amdgcn_perm(0u, w, 0x0c010c00u);  // b0 -> bits 0-7, b1 -> bits 16-23
-  const uint32_t mag = ((x & 0x007F007Fu) << 4) + 0x3C003C00u;
-  return mag | ((x << 8) & 0x80008000u);
-}
-
-__device__ __forceinline__ u16x8 dequant8(uint32_t lo, uint32_t hi) {
-  const uint32_t a = e4m3x2_to_bf16x2(lo), b = e4m3x2_to_bf16x2(lo >> 16);
-  const uint32_t c = e4m3x2_to_bf16x2(hi), d = e4m3x2_to_bf16x2(hi >> 16);
-  return __builtin_bit_cast(u16x8, u32x4{a, b, c, d});
-}
 
 // MB: 16-token blocks (1 or 2); X rows >= M are clamped to M-1 and discarded.
 // NW waves per workgroup split K into NW contiguous parts (more loads in flight for
@@ -85,8 +62,8 @@ __global__ void __launch_bounds__(64 * NW) w8a16_gemm_kernel(const uint16_t* __r
       const u16x8 a1 = dequant8(q[j][2], q[j][3]);  // k = 16g + 8..15  (MFMA step 1)
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        acc[j][mb] = mfma16_f8(a0, b[mb][0], acc[j][mb]);
-        acc[j][mb] = mfma16_f8(a1, b[mb][1], acc[j][mb]);
+        acc[j][mb] = mfma16_sk(a0, b[mb][0], acc[j][mb]);
+        acc[j][mb] = mfma16_sk(a1, b[mb][1], acc[j][mb]);
       }
     }
   };

@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
     if constexpr (NORM) {
       __shared__ float nscr[2][4];
       __shared__ float nrs[4];
-      dfuse_norm_rows(X, ldx, M, K, na, xs, nscr, nrs);
+      dfuse_norm_rows(X, ldx, M, K, na, xs, K, nscr, nrs);
     } else {
       dfuse_merge_rows(M, K, mg, xs);
     }

@@ -36,7 +36,8 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
               ("attn_fwd", "chunk_attn", "decode", "hybrid", "hybrid_skinny", "latent", "latent_mfma", "mingru",
-               "moe", "moe_mfma", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm"),
+               "moe", "moe_mfma", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
+               "stream_gemm"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),
 }
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")

@@ -583,87 +583,161 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
             and x2.stride(0) % 8 == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0 and use_native(x2))
 
 
+# Rows past which a projection of _STREAM_N and more channels goes to the workgroups that stay
+# (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of once 16 channels), by rows x width: the X that the
+# others read beside 16 channels of weights.  At 16,384 both are level (28672 x 4096, 4 rows: 48.0 -> 43.6 us;
+# 16384 x 2048, 4 rows 14.9 -> 15.9, 8 rows 16.9 -> 16.3; 28672 x 4096, 16 rows 67 -> 48, hipBLASLt 60-67).
+# Past 16 rows two token blocks halve what a fragment of weights is read for: hipBLASLt up to 32,768 channels
+# (16384 x 2048, 32 rows: 18.4 us against 21.4; 128256 x 2048: 119 against 112).
+_STREAM_MK, _STREAM_N, _STREAM_N2 = 16384, 8192, 32768
+# Rows x width up to which a projection of at most 4096 channels (one group a CU) runs on skinny_gemm.hip past
+# SKINNY_M rows: 4096 x 4096, 16 rows 11.2 us against hipBLASLt's 15.6, 24 rows 14.5 against 13.4; 3072 x 2048,
+# 32 rows 9.1 against 11.7.
+_WIDE_MK, _WIDE_N = 65536, 4096
+
+
+def _rows_ok(x2: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> bool:
+    """Operands that the decode GEMMs take: bf16 rows, and weights of bf16 or of e4m3 codes with ``scale``."""
+    return (x2.is_cuda and x2.dtype == torch.bfloat16 and w.dtype == (torch.bfloat16 if scale is None else torch.uint8)
+            and x2.shape[1] == w.shape[1] and w.shape[0] % 16 == 0 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
+            and w.stride(1) == 1 and w.stride(0) % (8 if scale is None else 16) == 0 and use_native(x2))
+
+
+def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
+    """Rows of K that csrc/kernels/stream_gemm.hip holds in LDS beside its partial sums (``norm``: and norms)."""
+    return SKINNY_M > 0 and 0 < M <= (4 if norm else 32) and K % 2048 == 0 and 16384 + 2 * M * (K + 8) <= 158 * 1024
+
+
+def _stream_wins(M: int, N: int, K: int) -> bool:
+    return _stream_fits(M, K) and N >= _STREAM_N and M * K >= _STREAM_MK
+
+
+def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    M, (N, K) = x2.shape[0], w.shape
+    if _stream_wins(M, N, K) and (M <= 16 or N >= _STREAM_N2):
+        return native().stream_linear(x2, None, None, 0.0, w, None, False)[0] if _rows_ok(x2, w) else None
+    if M <= SKINNY_M:
+        # many rows of a large weight outside the kernel above: hipBLASLt
+        ok = _skinny_ok(x2, w) or (M * K < _STREAM_MK and K % 512 == 0 and _rows_ok(x2, w))
+        half = N < _HALF_N and K % 1024 == 0 and M <= 8
+        return (native().skinny_linear_half if half else native().skinny_linear)(x2, w) if ok else None
+    if M * K <= _WIDE_MK and N <= _WIDE_N and K % 512 == 0 and _rows_ok(x2, w):
+        return native().skinny_linear(x2, w)
+    return None
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if w.requires_grad and torch.is_grad_enabled():
         return _LinearFn.apply(x, w)
-    if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and x.numel() // max(x.shape[-1], 1) <= SKINNY_M:
-        x2 = x.reshape(-1, x.shape[-1])
-        if x2.shape[0] > 0 and _skinny_ok(x2, w):
-            half = w.shape[0] < _HALF_N and w.shape[1] % 1024 == 0 and x2.shape[0] <= 8
-            fn = native().skinny_linear_half if half else native().skinny_linear
-            return fn(x2, w).view(*x.shape[:-1], w.shape[0])
+    if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= 32:
+        y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
+        if y is not None:
+            return y.view(*x.shape[:-1], w.shape[0])
     return F.linear(x, w)
 
 
-def linear_swiglu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
     """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts as ONE launch, with
-    ``w = [gate; up]`` [2F, K] (csrc/kernels/skinny_gemm.hip SWO variant: the SwiGLU in
-    the GEMM epilogue, bit-identical to the GEMM + SwiGLU kernels).  None when the fused
-    kernel does not take the call (the caller then runs the two ops)."""
+    ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip or
+    stream_gemm.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
+    the fused kernels do not take the call (the caller then runs the two ops)."""
     if SKINNY_M <= 0 or x.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return None
-    if x.shape[1] != w.shape[1] or w.shape[0] % 16 or not 0 < x.shape[0] <= SKINNY_M:
+    if x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
         return None
-    if not _skinny_ok(x, w):
+    if scale is not None:
+        if not (_stream_fits(*x.shape) and _rows_ok(x, w, scale)):
+            return None
+        return native().stream_linear(x, None, None, 0.0, w, scale, True)[0]
+    if _stream_wins(x.shape[0], *w.shape) and _rows_ok(x, w):
+        return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
+    if x.shape[0] > SKINNY_M or not _skinny_ok(x, w):
         return None
     return native().skinny_linear_swiglu(x, w)
 
 
-# rows up to which the RMSNorm runs in the decode GEMM's prologue (every workgroup recomputes the
+# rows up to which the RMSNorm runs in the prologue of skinny_gemm.hip (every workgroup recomputes the
 # rows): measured same box, 8B decode batch 1 3.607 -> 3.479 ms and 70B 26.22 -> 24.98 ms, but batch 4
-# 3.83 -> 4.04 ms (archive/profiles/r2s3_decode_ab/); the kernel takes up to 4
+# 3.83 -> 4.04 ms (archive/profiles/r2s3_decode_ab/); the kernel takes up to 4.  stream_gemm.hip's workgroups
+# do it once for all their channels: up to 4 rows.
 NORM_M = int(os.environ.get("MXLLM_NORM_FUSED_M", "2"))
 
 
+def _norm_stream(M: int, K: int, scale) -> bool:
+    """Whether the RMSNorm goes into stream_gemm.hip's prologue."""
+    return _stream_fits(M, K, True) and NORM_M > 0 and (scale is not None or M > min(NORM_M, SKINNY_M))
+
+
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,
-                norm: bool) -> bool:
+                norm: bool, scale: torch.Tensor | None = None) -> bool:
     """Whether :func:`qkv_rope_linear` takes these shapes (``norm``: with the RMSNorm prologue)."""
     if SKINNY_M <= 0 or h.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return False
-    M, K = h.shape
-    if not 0 < M <= (min(NORM_M, SKINNY_M) if norm else SKINNY_M) or (norm and M * K > 32768):
+    (M, K), D = h.shape, k_cache.shape[-1]
+    if D not in (64, 128) or w.shape != ((Hq + 2 * Hkv) * D, K) or k_cache.dtype != torch.bfloat16:
         return False
-    if w.shape != ((Hq + 2 * Hkv) * 128, K) or k_cache.shape[-1] != 128 or k_cache.dtype != torch.bfloat16:
+    if not (cos.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous() and k_cache.is_contiguous()
+            and v_cache.is_contiguous()):
         return False
-    return bool(_skinny_ok(h, w) and cos.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous()
-                and k_cache.is_contiguous() and v_cache.is_contiguous())
+    if _qkv_stream(M, K, D, norm, scale):
+        return _rows_ok(h, w, scale)
+    if scale is not None or D != 128 or not 0 < M <= (min(NORM_M, SKINNY_M) if norm else SKINNY_M):
+        return False
+    return bool((not norm or M * K <= 32768) and _skinny_ok(h, w))
+
+
+def _qkv_stream(M: int, K: int, D: int, norm: bool, scale) -> bool:
+    """bf16 heads of 128 up to SKINNY_M rows have their kernel in skinny_gemm.hip."""
+    if norm:
+        return NORM_M > 0 and _stream_fits(M, K, True) and (scale is not None or D == 64 or M > min(NORM_M, SKINNY_M))
+    return _stream_fits(M, K) and (scale is not None or D == 64 or M > SKINNY_M)
 
 
 def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, cos, sin, pos, slots, k_cache,
-                    v_cache, Hq: int, Hkv: int, block_table=None):
+                    v_cache, Hq: int, Hkv: int, block_table=None, scale: torch.Tensor | None = None):
     """Inference, decode rows: the QKV projection with RoPE and the KV-cache append in the GEMM
-    epilogue (csrc/kernels/skinny_gemm.hip ROPE) and, for 1-NORM_M rows, the (residual-add +)
+    epilogue (csrc/kernels/skinny_gemm.hip ROPE, stream_gemm.hip) and, for a few rows, the (residual-add +)
     RMSNorm in its prologue; ``gamma`` None: ``h`` is already normalised; ``block_table``:
-    paged caches (mxllm/serve/kvcache.py).  Returns
-    (q [M, Hq, 128] rotated, new residual) or None when the fused kernel does not take the call."""
-    if not qkv_rope_ok(h, w, cos, sin, k_cache, v_cache, Hq, Hkv, gamma is not None):
-        return None
+    paged caches (mxllm/serve/kvcache.py); ``scale``: w is e4m3 codes.  Returns
+    (q [M, Hq, D] rotated, new residual) or None when the fused kernels do not take the call."""
     norm = gamma is not None
+    if not qkv_rope_ok(h, w, cos, sin, k_cache, v_cache, Hq, Hkv, norm, scale):
+        return None
     if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous()):
         return None
     if delta is not None and (not norm or delta.shape != h.shape or delta.stride(1) != 1 or delta.stride(0) % 8):
         return None
+    if _qkv_stream(h.shape[0], h.shape[1], k_cache.shape[-1], norm, scale):
+        return native().stream_qkv_rope(h, delta, gamma, float(eps), w, scale, cos, sin, pos, slots, k_cache, v_cache,
+                                        Hq, Hkv, block_table)
     return native().skinny_qkv_rope(h, delta, gamma, float(eps), w, cos, sin, pos, slots, k_cache, v_cache, Hq, Hkv,
                                     block_table)
 
 
 def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor, eps: float, w: torch.Tensor,
-                swiglu: bool = False):
+                swiglu: bool = False, scale: torch.Tensor | None = None):
     """Inference, decode rows: ``(linear(rmsnorm(h + delta) * gamma, w), h + delta)`` as ONE
-    launch (csrc/kernels/skinny_gemm.hip NORM: the RMSNorm in the GEMM prologue, same bits as
+    launch (the RMSNorm in the prologue of csrc/kernels/skinny_gemm.hip or stream_gemm.hip, same bits as
     the RMSNorm kernel + decode GEMM); with ``swiglu`` w = [gate; up] and the first output is
-    silu(g) * u.  ``delta`` None: plain RMSNorm, the residual is ``h``.  None when the fused
-    kernel does not take the call."""
+    silu(g) * u; ``scale``: w is e4m3 codes.  ``delta`` None: plain RMSNorm, the residual is ``h``.  None
+    when the fused kernels do not take the call."""
     if SKINNY_M <= 0 or h.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return None
     M, K = h.shape
-    if not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768 or h.stride(1) != 1 or w.shape[1] != K or w.shape[0] % 16:
+    stream = _norm_stream(M, K, scale) and w.shape[0] >= _STREAM_N
+    if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
-    if gamma.dtype != torch.bfloat16 or not gamma.is_contiguous() or not _skinny_ok(h, w):
+    if h.stride(1) != 1 or w.shape[1] != K or w.shape[0] % 16:
+        return None
+    if gamma.dtype != torch.bfloat16 or not gamma.is_contiguous():
+        return None
+    if not (_rows_ok(h, w, scale) if stream else _skinny_ok(h, w)):
         return None
     if delta is not None and (delta.shape != h.shape or delta.dtype != h.dtype or delta.stride(1) != 1
                               or delta.stride(0) % 8):
         return None
+    if stream:
+        return native().stream_linear(h, delta, gamma, float(eps), w, scale, bool(swiglu))
     return native().skinny_norm_linear(h, delta, gamma, float(eps), w, bool(swiglu))
 
 

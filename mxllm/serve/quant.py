@@ -74,6 +74,10 @@ class W8Linear(nn.Module):
         self.register_buffer("scale", s)
         self.out_features, self.in_features = q.shape
 
+    def streams(self, rows: int) -> bool:
+        """Whether calls of ``rows`` rows run on the weight-only kernels (which the fused decode steps extend)."""
+        return rows <= SMALL_M
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         x2 = x.reshape(-1, self.in_features)
         if x2.stride(1) != 1 or x2.stride(0) % 8:

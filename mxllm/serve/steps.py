@@ -27,6 +27,7 @@ from ..ops import decode as dops
 from ..ops.hybrid import PromptRows, SeqCaches, TokenRows
 from ..ops.latent import LatentCache
 from .kvcache import KVCache, StateCache
+from .quant import W8Linear
 
 _SWIGLU_FUSED = os.environ.get("MXLLM_SWIGLU_FUSED", "1") != "0"  # A/B switch (bench/serve_bench.py)
 _NORM_FUSED = os.environ.get("MXLLM_NORM_FUSED", "1") != "0"  # A/B switch: RMSNorm in the decode GEMM prologue
@@ -89,14 +90,24 @@ class LlamaSteps:
 
         return self._layers(x, attn)
 
+    @staticmethod
+    def _stream_weight(lin, rows: int):
+        """(weight, scale) of a projection that the fused decode GEMMs take: plain bf16 (scale None), or e4m3 codes
+        where ``rows`` rows keep bf16 activations; (None, None): neither."""
+        if type(lin) is FusedLinear and lin.lora_r == 0:
+            return lin.weight, None
+        if type(lin) is W8Linear and lin.streams(rows):
+            return lin.q, lin.scale
+        return None, None
+
     def _norm_proj(self, delta, h, gamma, lin, swiglu: bool):
         """(proj(rmsnorm(h + delta) * gamma), h + delta); ``swiglu``: proj = swiglu(lin(.)).
-        Decode rows of a plain bf16 projection run as ONE launch (RMSNorm in the GEMM
+        Decode rows of a plain bf16 or e4m3 projection run as ONE launch (RMSNorm in the GEMM
         prologue, SwiGLU in its epilogue: csrc/kernels/skinny_gemm.hip)."""
         eps = self.cfg.norm_eps
-        plain = type(lin) is FusedLinear and lin.lora_r == 0
-        if _NORM_FUSED and plain:
-            r = ops.norm_linear(delta, h, gamma, eps, lin.weight, swiglu)
+        w, scale = self._stream_weight(lin, h.shape[0])
+        if _NORM_FUSED and w is not None:
+            r = ops.norm_linear(delta, h, gamma, eps, w, swiglu, scale)
             if r is not None:
                 return r
         if delta is None:
@@ -106,8 +117,8 @@ class LlamaSteps:
         if not swiglu:
             return lin(xn), h
         mid = None
-        if _SWIGLU_FUSED and plain and xn.dim() == 2:
-            mid = ops.linear_swiglu(xn, lin.weight)  # decode rows: SwiGLU in the GEMM epilogue
+        if _SWIGLU_FUSED and w is not None and xn.dim() == 2:
+            mid = ops.linear_swiglu(xn, w, scale)  # decode rows: SwiGLU in the GEMM epilogue
         if mid is None:
             mid = ops.swiglu(lin(xn))
         return mid, h
@@ -190,18 +201,18 @@ class LlamaSteps:
                                          c.n_heads, c.n_kv_heads, c.head_dim, max_len, bt, cnt)
 
         def qkv_fn(i, delta, h, gamma, layer):
-            # QKV GEMM with the RoPE/cache-append epilogue; 1-2 rows also with the RMSNorm prologue
+            # QKV GEMM with the RoPE/cache-append epilogue; a few rows also with the RMSNorm prologue
             # (one launch), more rows after the RMSNorm kernel
-            if not (_ROPE_FUSED and self.eng.tp is None and c.head_dim == 128
-                    and type(layer.wqkv) is FusedLinear and layer.wqkv.lora_r == 0):
+            w, scale = self._stream_weight(layer.wqkv, B)
+            if not (_ROPE_FUSED and self.eng.tp is None and w is not None):
                 return None
-            rope = (layer.wqkv.weight, m.rope_cos, m.rope_sin, pos, sl, self.eng.kv.k[i], self.eng.kv.v[i],
-                    c.n_heads, c.n_kv_heads, bt)
+            rope = (w, m.rope_cos, m.rope_sin, pos, sl, self.eng.kv.k[i], self.eng.kv.v[i],
+                    c.n_heads, c.n_kv_heads, bt, scale)
             if _NORM_FUSED:
                 r = ops.qkv_rope_linear(delta, h, gamma, c.norm_eps, *rope)
                 if r is not None:
                     return r
-            if not ops.qkv_rope_ok(h, rope[0], rope[1], rope[2], rope[5], rope[6], rope[7], rope[8], False):
+            if not ops.qkv_rope_ok(h, rope[0], rope[1], rope[2], rope[5], rope[6], rope[7], rope[8], False, scale):
                 return None
             if delta is None:
                 xn = ops.rms_norm(h, gamma, c.norm_eps)

@@ -866,3 +866,68 @@ def test_skinny_linear_half(gpu, M, N, K):
     w = torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05
     y = _ops().skinny_linear_half(x, w)
     assert y.shape == (M, N) and rel_err(y, x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
+
+
+def _stream_weight(w, f8):
+    from mxllm.serve.quant import quantize_e4m3
+
+    return quantize_e4m3(w) if f8 else (w, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f8", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 16, 2048), (3, 16 * 513, 4096), (16, 16 * 257, 4096), (17, 8192, 2048),
+                                   (32, 16 * 600, 2048), (9, 48, 6144), (4, 96, 16384), (2, 16 * 1025, 8192)])
+def test_stream_linear(gpu, M, N, K, f8):
+    """Decode GEMM of workgroups that stay (csrc/kernels/stream_gemm.hip): the bits of the one-group kernels, with
+    fewer, as many and more groups than workgroups, one and two workgroups a CU, both block sizes; row-strided x."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K + 64, device=gpu, dtype=torch.bfloat16)[:, :K]
+    w, s = _stream_weight(torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05, f8)
+    y = _ops().stream_linear(x, None, None, 0.0, w, s, False)[0]
+    assert torch.equal(y, _ops().w8_linear(x, w, s) if f8 else _ops().skinny_linear(x, w))
+    wd = w.view(torch.float8_e4m3fn).double() * s.double()[:, None] if f8 else w.double()
+    assert rel_err(y, x.double() @ wd.t()) < 2 ** -8  # one bf16 rounding
+    from mxllm import ops
+
+    two = ops.swiglu(y)
+    assert torch.equal(_ops().stream_linear(x, None, None, 0.0, w, s, True)[0], two)
+    if M <= 4:
+        for resid in (False, True):
+            d = torch.randn(M, K, device=gpu, dtype=torch.bfloat16) if resid else None
+            gamma = (1.0 + 0.1 * torch.randn(K, device=gpu)).to(torch.bfloat16)
+            xn, hn = ops.add_rms_norm(d, x, gamma, 1e-5) if resid else (ops.rms_norm(x, gamma, 1e-5), x)
+            for sw in (False, True):
+                got, h2 = _ops().stream_linear(x, d, gamma, 1e-5, w, s, sw)
+                assert torch.equal(h2, hn)
+                assert torch.equal(got, _ops().stream_linear(xn, None, None, 0.0, w, s, sw)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f8", [False, True])
+@pytest.mark.parametrize("M,Hq,Hkv,D,K,norm", [(1, 32, 8, 64, 2048, True), (16, 32, 8, 128, 4096, False),
+                                               (32, 5, 1, 64, 2048, False), (4, 64, 8, 128, 8192, True)])
+def test_stream_qkv_rope(gpu, M, Hq, Hkv, D, K, norm, f8):
+    """The QKV projection with RoPE and the cache append in the epilogue, heads of 64 and 128, contiguous and paged
+    caches: q, cache rows and residual of RMSNorm + projection + rope_append."""
+    from mxllm import ops
+
+    torch.manual_seed(M * 3 + Hq)
+    max_seq, nslots = 256, M + 2
+    h = torch.randn(M, K, device=gpu, dtype=torch.bfloat16)
+    d = torch.randn(M, K, device=gpu, dtype=torch.bfloat16) if norm else None
+    gamma = (1.0 + 0.1 * torch.randn(K, device=gpu)).to(torch.bfloat16) if norm else None
+    w, s = _stream_weight(torch.randn((Hq + 2 * Hkv) * D, K, device=gpu, dtype=torch.bfloat16) * 0.05, f8)
+    cos, sin = ref.rope_tables(1024, D, 500000.0, None, gpu)
+    slots = torch.randperm(nslots, device=gpu)[:M].to(torch.int32)
+    xn, hn = ops.add_rms_norm(d, h, gamma, 1e-5) if norm else (h, h)
+    qkv = _ops().stream_linear(xn, None, None, 0.0, w, s, False)[0]
+    for bt in (None, torch.randperm(4 * nslots, device=gpu).to(torch.int32).view(nslots, 4)):
+        pos = torch.randint(0, max_seq if bt is None else 1024, (M,), device=gpu, dtype=torch.int32)
+        kc = torch.randn(nslots if bt is None else 4 * nslots, Hkv, max_seq, D, device=gpu, dtype=torch.bfloat16)
+        vc = torch.randn_like(kc)
+        kc2, vc2 = kc.clone(), vc.clone()
+        q, h2 = _ops().stream_qkv_rope(h, d, gamma, 1e-5, w, s, cos, sin, pos, slots, kc, vc, Hq, Hkv, bt)
+        q_ref = _ops().rope_append(qkv, cos, sin, pos, slots, kc2, vc2, Hq, Hkv, D, bt)
+        assert torch.equal(h2, hn) and torch.equal(q.view(M, -1), q_ref.reshape(M, -1))
+        assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
