@@ -65,125 +65,8 @@ __global__ void __launch_bounds__(256) rope_append_kernel(const uint16_t* __rest
 constexpr int kSplit = 256;  // keys per workgroup
 constexpr int kMaxRep = 16;  // q-heads per kv-head supported
 
-// grid (nsplit, Hkv, B); block 256 = one key per thread for the score phase.
-template <int D>
-__global__ void __launch_bounds__(256) decode_attn_kernel(const uint16_t* __restrict__ q,
-                                                          const uint16_t* __restrict__ kc,
-                                                          const uint16_t* __restrict__ vc,
-                                                          const int32_t* __restrict__ lens, int len_off,
-                                                          const int32_t* __restrict__ slots,
-                                                          float* __restrict__ part_ml, float* __restrict__ part_o,
-                                                          int Hq, int Hkv, int max_seq, int nsplit, float sl,
-                                                          const int32_t* __restrict__ bt, int maxb) {
-  __shared__ float qs[kMaxRep][D];
-  __shared__ float ps[kMaxRep][kSplit];
-  __shared__ float red[kMaxRep][4];
-  __shared__ __attribute__((aligned(16))) uint16_t vs[kSplit * D];
-  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
-  const int rep = Hq / Hkv;
-  const int len = lens[b] + len_off;
-  const int slot = slots ? slots[b] : b;
-  const int k_lo = split * kSplit;
-  const int k_hi = min(len, k_lo + kSplit);
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  float* pml = part_ml + (((int64_t)b * Hq + hk * rep) * nsplit + split) * 2;
-  if (k_lo >= k_hi) {  // empty split: neutral partial
-    if (tid < rep) {
-      pml[(int64_t)tid * nsplit * 2] = -INFINITY;
-      pml[(int64_t)tid * nsplit * 2 + 1] = 0.f;
-    }
-    return;
-  }
-  for (int i = tid; i < rep * D; i += 256) {
-    const int h = i / D, d = i % D;
-    qs[h][d] = bf2f(q[((int64_t)b * Hq + hk * rep + h) * D + d]);
-  }
-  // base such that base + key * D addresses every key of this split (a paged split lies in
-  // one block: the block size is a multiple of kSplit)
-  const int64_t kvb = (kv_row(bt, maxb, max_seq, slot, Hkv, hk, k_lo) - k_lo) * D;
-  const uint16_t* kbase = kc + kvb;
-  const uint16_t* vbase = vc + kvb;
-  // stage V rows of this split into LDS (coalesced 16-B chunks)
-  constexpr int CH = D / 8;
-  for (int c = tid; c < kSplit * CH; c += 256) {
-    const int row = c / CH, ch = c % CH, key = k_lo + row;
-    u16x8 v = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (key < k_hi) v = *reinterpret_cast<const u16x8*>(vbase + (int64_t)key * D + ch * 8);
-    *reinterpret_cast<u16x8*>(vs + row * D + ch * 8) = v;
-  }
-  __syncthreads();
-  const int key = k_lo + tid;
-  float s[kMaxRep];
-#pragma unroll
-  for (int h = 0; h < kMaxRep; ++h) s[h] = -INFINITY;
-  if (key < k_hi) {
-#pragma unroll
-    for (int h = 0; h < kMaxRep; ++h) s[h] = 0.f;
-    const uint16_t* kr = kbase + (int64_t)key * D;
-#pragma unroll 4
-    for (int c = 0; c < D; c += 8) {
-      const u16x8 kv = *reinterpret_cast<const u16x8*>(kr + c);
-      float kf[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) kf[j] = bf2f(kv[j]);
-#pragma unroll
-      for (int h = 0; h < kMaxRep; ++h) {
-        if (h < rep) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) s[h] += qs[h][c + j] * kf[j];
-        }
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < kMaxRep; ++h) s[h] *= sl;
-  }
-  // per-head max over the split
-#pragma unroll
-  for (int h = 0; h < kMaxRep; ++h) {
-    if (h < rep) {
-      const float m = wave_max(s[h]);
-      if (lane == 0) red[h][wid] = m;
-    }
-  }
-  __syncthreads();
-  float mh[kMaxRep];
-#pragma unroll
-  for (int h = 0; h < kMaxRep; ++h)
-    mh[h] = h < rep ? fmaxf(fmaxf(red[h][0], red[h][1]), fmaxf(red[h][2], red[h][3])) : 0.f;
-  __syncthreads();
-#pragma unroll
-  for (int h = 0; h < kMaxRep; ++h) {
-    if (h < rep) {
-      const float p = key < k_hi ? __builtin_amdgcn_exp2f(s[h] - mh[h]) : 0.f;
-      ps[h][tid] = p;
-      const float l = wave_sum(p);
-      if (lane == 0) red[h][wid] = l;
-    }
-  }
-  __syncthreads();
-  if (tid < rep) {
-    pml[(int64_t)tid * nsplit * 2] = mh[tid];
-    pml[(int64_t)tid * nsplit * 2 + 1] = red[tid][0] + red[tid][1] + red[tid][2] + red[tid][3];
-  }
-  // o[h][d] = sum_key p[h][key] v[key][d]: thread -> (h, d pair)
-  const int nkeys = k_hi - k_lo;
-  for (int o = tid; o < rep * (D / 2); o += 256) {
-    const int h = o / (D / 2), d = (o % (D / 2)) * 2;
-    float a0 = 0.f, a1 = 0.f;
-    for (int kk = 0; kk < nkeys; ++kk) {
-      const float p = ps[h][kk];
-      const uint32_t pr = *reinterpret_cast<const uint32_t*>(vs + kk * D + d);
-      a0 += p * bf2f((uint16_t)(pr & 0xffff));
-      a1 += p * bf2f((uint16_t)(pr >> 16));
-    }
-    float* po = part_o + ((((int64_t)b * Hq + hk * rep + h) * nsplit + split) * D) + d;
-    po[0] = a0;
-    po[1] = a1;
-  }
-}
-
 // ---------------------------------------------------------------------------
-// MFMA decode attention, D = 128 (every Llama-3.x model).  Memory-bound: the
+// Decode attention, heads of D = 128, 64 or 32.  Memory-bound: the
 // whole point is to stream each (seq, kv-head)'s cached K/V rows once at HBM
 // rate, so
 //   * a workgroup = 4 waves = 256 keys of one (seq, kv-head); each wave owns 64
@@ -194,15 +77,19 @@ __global__ void __launch_bounds__(256) decode_attn_kernel(const uint16_t* __rest
 //     as the B fragment;
 //   * the S^T accumulator (head on the lane, keys in registers) converted to
 //     bf16 IS the B operand of O^T[d][head] += V^T . P (keys permuted inside
-//     each 32-key k-step to match the accumulator's row order);
+//     each 32-key k-step to match the accumulator's row order).  D = 128: one
+//     bf16 rounding of P.  D < 128: P as the sum of three bf16 (24 bits, what f32
+//     holds) in three products, so the weights keep their f32 precision;
 //   * V^T fragments come from a row-major V image in LDS through
 //     ds_read_b64_tr_b16; the image is filled by LDS-DMA (global_load_lds,
 //     source-swizzled so the transposed reads are conflict-free);
 //   * the four waves' partials are merged through LDS (each wave reuses its own
 //     V region) into one (m, l, o) partial per split, the format of
-//     decode_combine_kernel.
-// 64 KiB LDS and < 128 VGPRs: two workgroups (8 waves) per CU, 256 KiB of K/V
-// in flight per CU.
+//     decode_combine_kernel; a single split is the output itself.
+// D = 128: 64 KiB LDS and < 128 VGPRs: two workgroups (8 waves) per CU, 256 KiB of
+// K/V in flight per CU.  D = 64, bound by latency at the few workgroups of a small
+// batch: 32 q-heads of 8 kv-heads, one sequence of 700 keys 6.4 us; with one key a
+// thread for the scores and a serial walk over the split's keys for the outputs 17.5.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(1))) const void* gptr_t;
@@ -218,8 +105,14 @@ __device__ __forceinline__ u16x4 tr_read16(const char* p) {
   return __builtin_bit_cast(u16x4, v);
 }
 
-// 16-B chunk swizzle of a 256-B row (conflict-free row and transposed reads)
-__device__ __forceinline__ int dswz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+// 16-B chunk swizzle of a row of 2 D bytes: transposed reads take 32 B of each of 16 rows, and rows that start in
+// the same bank take different pairs of chunks
+template <int D>
+__device__ __forceinline__ int dswz(int row) {
+  if constexpr (D == 128) return ((row & 3) << 2) | ((row >> 2) & 3);
+  else if constexpr (D == 64) return ((row >> 1) & 3) << 1;
+  else return ((row >> 2) & 1) << 1;
+}
 
 // stores / loads of the split partials that another workgroup of the SAME launch merges:
 // write-through (sc1, relaxed agent-scope atomic store), so no release fence (an L2
@@ -240,14 +133,16 @@ __device__ __forceinline__ float ld_part(const float* p, int ld) {
 }
 
 // one split of decode_attn_mfma_kernel: (m, l, o) partial of 256 keys for every
-// q-head of the GQA group (see the kernel's header comment)
+// q-head of the GQA group (see the kernel's header comment); out: the only split, and its output
+template <int D>
 __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc,
                                                   const uint16_t* __restrict__ vc, float* __restrict__ part_o,
                                                   float* __restrict__ pml, char* smem, float (*mls)[2][16], int b,
                                                   int hk, int rep, int Hq, int split, int nsplit, int k_lo, int k_hi,
                                                   int slot, int max_seq, float sl, const int32_t* __restrict__ bt,
-                                                  int maxb, int Hkv, int st) {
-  constexpr int D = 128, ROWB = 256, WKEYS = 64, WTILE = WKEYS * ROWB;
+                                                  int maxb, int Hkv, int st, uint16_t* __restrict__ out) {
+  constexpr int ROWB = 2 * D, CPR = D / 8, WKEYS = 64, WTILE = WKEYS * ROWB, KS = D / 32, DB = D / 16;
+  constexpr int NP = D == 128 ? 1 : 3;  // bf16 parts of a weight
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
@@ -257,40 +152,40 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
   const int wk0 = k_lo + WKEYS * w;
   char* vs = smem + w * WTILE;
 
-  // V rows of this wave -> LDS (16 x 1-KiB lane-linear DMA pieces; swizzle by
+  // V rows of this wave -> LDS (D / 8 x 1-KiB lane-linear DMA pieces; swizzle by
   // permuting each lane's SOURCE chunk).  Rows past k_hi duplicate a valid row
   // (finite; their probabilities are exactly 0).
 #pragma unroll
-  for (int seg = 0; seg < 16; ++seg) {
-    const int row = seg * 4 + (lane >> 4), slt = lane & 15;
-    const int ch = slt ^ dswz(row);
+  for (int seg = 0; seg < CPR; ++seg) {
+    const int row = seg * (64 / CPR) + lane / CPR, slt = lane % CPR;
+    const int ch = slt ^ dswz<D>(row);
     const int key = min(wk0 + row, k_hi - 1);
     __builtin_amdgcn_global_load_lds((gptr_t)(vbase + (int64_t)key * D + ch * 8), (lptr_t)(vs + seg * 1024), 16, 0,
                                      0);
   }
   // Q^T fragments (B operand): lane (c, g) holds Q[head c][32 s + 8 g .. +7]
-  u16x8 qf[4];
+  u16x8 qf[KS];
   const uint16_t* qrow = q + ((int64_t)b * Hq + hk * rep + min(c, rep - 1)) * D;
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
+  for (int s = 0; s < KS; ++s) {
     qf[s] = *reinterpret_cast<const u16x8*>(qrow + 32 * s + 8 * g);
     if (c >= rep) qf[s] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
   }
   // K fragments (A operand), straight from HBM: block j, k-step s ->
   // K[wk0 + 16 j + c][32 s + 8 g .. +7]
-  u16x8 kf[4][4];
+  u16x8 kf[4][KS];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int key = min(wk0 + 16 * j + c, k_hi - 1);
 #pragma unroll
-    for (int s = 0; s < 4; ++s) kf[j][s] = *reinterpret_cast<const u16x8*>(kbase + (int64_t)key * D + 32 * s + 8 * g);
+    for (int s = 0; s < KS; ++s) kf[j][s] = *reinterpret_cast<const u16x8*>(kbase + (int64_t)key * D + 32 * s + 8 * g);
   }
   f32x4 sacc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     sacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) sacc[j] = mfma16(kf[j][s], qf[s], sacc[j]);
+    for (int s = 0; s < KS; ++s) sacc[j] = mfma16(kf[j][s], qf[s], sacc[j]);
   }
   // softmax over this wave's 64 keys, per head (= lane column c); lane (c, g)
   // holds keys wk0 + 16 j + 4 g + i
@@ -308,41 +203,46 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   const float mref = mx == -INFINITY ? 0.f : mx;  // wave with no valid key: all p = 0
   float ls = 0.f;
-  u16x8 pb[2];
+  u16x8 pb[NP][2];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float p = __builtin_amdgcn_exp2f(sacc[j][i] - mref);
+      float p = __builtin_amdgcn_exp2f(sacc[j][i] - mref);
       ls += p;
-      pb[j >> 1][4 * (j & 1) + i] = f2bf(p);
+#pragma unroll
+      for (int n = 0; n < NP; ++n) {
+        pb[n][j >> 1][4 * (j & 1) + i] = f2bf(p);
+        p -= bf2f(pb[n][j >> 1][4 * (j & 1) + i]);
+      }
     }
   ls += __shfl_xor(ls, 16, 64);
   ls += __shfl_xor(ls, 32, 64);
 
   // O^T[d][head] += V^T . P; k-step t covers keys 32 t + {16 h + 4 g + i}
-  f32x4 oacc[8];
+  f32x4 oacc[DB];
 #pragma unroll
-  for (int db = 0; db < 8; ++db) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's V DMA has landed (only it reads vs)
   const int qq = c >> 2, pp = c & 3;
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
     const int r0 = 32 * t + 4 * g + qq, r1 = r0 + 16;
 #pragma unroll
-    for (int db = 0; db < 8; ++db) {
+    for (int db = 0; db < DB; ++db) {
       const int ch = 2 * db + (pp >> 1);
-      const u16x4 va = tr_read16(vs + r0 * ROWB + 16 * (ch ^ dswz(r0)) + 8 * (pp & 1));
-      const u16x4 vb = tr_read16(vs + r1 * ROWB + 16 * (ch ^ dswz(r1)) + 8 * (pp & 1));
+      const u16x4 va = tr_read16(vs + r0 * ROWB + 16 * (ch ^ dswz<D>(r0)) + 8 * (pp & 1));
+      const u16x4 vb = tr_read16(vs + r1 * ROWB + 16 * (ch ^ dswz<D>(r1)) + 8 * (pp & 1));
       const u16x8 a = u16x8{va[0], va[1], va[2], va[3], vb[0], vb[1], vb[2], vb[3]};
-      oacc[db] = mfma16(a, pb[t], oacc[db]);
+#pragma unroll
+      for (int n = NP - 1; n >= 0; --n) oacc[db] = mfma16(a, pb[n][t], oacc[db]);  // the smallest parts first
     }
   }
   // merge the four waves: each wave parks (m, l, O^T) in its own V region
   __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's transposed reads retired
   float* so = reinterpret_cast<float*>(vs);  // [d][16 heads]
 #pragma unroll
-  for (int db = 0; db < 8; ++db)
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 4; ++i) so[(16 * db + 4 * g + i) * 16 + c] = oacc[db][i];
   if (g == 0) {
@@ -363,6 +263,10 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
       L += f * mls[ww][1][h];
       acc += f * reinterpret_cast<const float*>(smem + ww * WTILE)[d * 16 + h];
     }
+    if (out) {  // as decode_combine_kernel writes one split
+      out[((int64_t)b * Hq + hk * rep + h) * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
+      continue;
+    }
     st_part(&part_o[(((int64_t)b * Hq + hk * rep + h) * nsplit + split) * D + d], acc, st);
     if (d == 0) {
       st_part(&pml[(int64_t)h * nsplit * 2], M, st);
@@ -378,6 +282,7 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
 //   3 = agent-scope stores, an agent-scope acquire fence in the merger, plain loads;
 //   4 = plain stores, one agent-scope release fence per workgroup (lane 0, after every wave's
 //       vmcnt drain), acquire fence in the merger, plain loads (guide §5 in-launch split-K recipe).
+template <int D>
 __global__ void __launch_bounds__(256, 2) decode_attn_mfma_kernel(const uint16_t* __restrict__ q,
                                                                   const uint16_t* __restrict__ kc,
                                                                   const uint16_t* __restrict__ vc,
@@ -389,7 +294,7 @@ __global__ void __launch_bounds__(256, 2) decode_attn_mfma_kernel(const uint16_t
                                                                   const int32_t* __restrict__ bt, int maxb,
                                                                   uint16_t* __restrict__ out,
                                                                   unsigned int* __restrict__ cnt, int proto) {
-  constexpr int D = 128, WTILE = 64 * 256;  // 16 KiB per wave
+  constexpr int WTILE = 64 * 2 * D;  // 16 KiB per wave at D = 128
   __shared__ __attribute__((aligned(16))) char smem[4 * WTILE];
   __shared__ float mls[4][2][16];
   __shared__ int s_last;
@@ -403,16 +308,21 @@ __global__ void __launch_bounds__(256, 2) decode_attn_mfma_kernel(const uint16_t
   const bool fused = cnt != nullptr;
   const int st = !fused ? 0 : proto == 2 ? 2 : proto == 4 ? 0 : 1;  // store mode of the partials
   float* pml = part_ml + (((int64_t)b * Hq + hk * rep) * nsplit + split) * 2;
+  uint16_t* const only = out && nsplit == 1 ? out : nullptr;
   if (k_lo >= k_hi) {  // empty split (workgroup-uniform): neutral partial
+    if (only) {
+      for (int i = tid; i < rep * D; i += 256) only[((int64_t)b * Hq + hk * rep) * D + i] = 0;
+      return;
+    }
     if (tid < rep) {
       st_part(&pml[(int64_t)tid * nsplit * 2], -INFINITY, st);
       st_part(&pml[(int64_t)tid * nsplit * 2 + 1], 0.f, st);
     }
   } else {
-    decode_split_body(q, kc, vc, part_o, pml, smem, mls, b, hk, rep, Hq, split, nsplit, k_lo, k_hi, slot, max_seq,
-                      sl, bt, maxb, Hkv, st);
+    decode_split_body<D>(q, kc, vc, part_o, pml, smem, mls, b, hk, rep, Hq, split, nsplit, k_lo, k_hi, slot, max_seq,
+                         sl, bt, maxb, Hkv, st, only);
   }
-  if (!fused) return;
+  if (!fused || only) return;
   // In-launch combine: the last of the nsplit workgroups of this (seq, kv-head) to arrive
   // merges the partials and resets the counter (zero again for the next call).
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave: its partial stores done
@@ -626,23 +536,17 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
   dim3 grid(nsplit, Hkv, B);
   const float sl = scale * 1.4426950408889634f;
   // out == nullptr: partials only, merged by the caller (skinny_gemm.hip MERGE, hybrid.hip attn_combine)
-  if (D == 128) {
-    // cnt (zeroed [B * Hkv] counters, owned by the caller): the splits merge in-launch
-    // MXLLM_DECODE_HANDOFF: hand-off protocol of the in-launch merge (see the kernel; read per call)
-    const char* pe = getenv("MXLLM_DECODE_HANDOFF");
-    const int proto = pe && *pe ? atoi(pe) : 4;
-    const bool fused = out && cnt && proto >= 1 && proto <= 4;
-    decode_attn_mfma_kernel<<<grid, 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, Hq, Hkv,
-                                                      max_seq, nsplit, sl, bt, maxb, out, fused ? cnt : nullptr,
-                                                      proto);
-    if (out && !fused) decode_combine_kernel<128><<<B * Hq, 128, 0, stream>>>(part_ml, part_o, out, nsplit);
-    return (int)hipGetLastError();
-  }
-#define DA(DD)                                                                                                  \
-  decode_attn_kernel<DD><<<grid, 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, Hq, Hkv, \
-                                                   max_seq, nsplit, sl, bt, maxb);                              \
-  if (out) decode_combine_kernel<DD><<<B * Hq, DD, 0, stream>>>(part_ml, part_o, out, nsplit)
-  if (D == 64) { DA(64); } else if (D == 32) { DA(32); } else return -1;
+  // cnt (zeroed [B * Hkv] counters, owned by the caller; D = 128): the splits merge in-launch
+  // MXLLM_DECODE_HANDOFF: hand-off protocol of the in-launch merge (see the kernel; read per call)
+  const char* pe = getenv("MXLLM_DECODE_HANDOFF");
+  const int proto = pe && *pe ? atoi(pe) : 4;
+  const bool fused = out && cnt && D == 128 && proto >= 1 && proto <= 4;
+#define DA(DD)                                                                                                      \
+  decode_attn_mfma_kernel<DD><<<grid, 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, Hq, Hkv, \
+                                                        max_seq, nsplit, sl, bt, maxb, fused || nsplit == 1 ? out : nullptr, \
+                                                        fused ? cnt : nullptr, proto);                              \
+  if (out && !fused && nsplit > 1) decode_combine_kernel<DD><<<B * Hq, DD, 0, stream>>>(part_ml, part_o, out, nsplit)
+  if (D == 128) { DA(128); } else if (D == 64) { DA(64); } else if (D == 32) { DA(32); } else return -1;
 #undef DA
   return (int)hipGetLastError();
 }

@@ -931,3 +931,45 @@ def test_stream_qkv_rope(gpu, M, Hq, Hkv, D, K, norm, f8):
         q_ref = _ops().rope_append(qkv, cos, sin, pos, slots, kc2, vc2, Hq, Hkv, D, bt)
         assert torch.equal(h2, hn) and torch.equal(q.view(M, -1), q_ref.reshape(M, -1))
         assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Hq,Hkv,lens", [(8, 2, [1, 255, 256, 257]), (4, 4, [64, 65, 700]), (16, 1, [1300, 3]),
+                                         (6, 2, [31, 256])])
+def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
+    """Split-K decode attention on paged caches with stale rows (NaN past a sequence's end), every group size up to
+    16: merged partials against f64.  Heads of 64 and 32 keep f32 softmax weights (an f32 sum of up to 1300 terms);
+    heads of 128 round them to bf16.  The output of a single split equals the merge of its partials."""
+    torch.manual_seed(D + Hq)
+    B, blk = len(lens), 256
+    maxb = (max(lens) + blk - 1) // blk
+    bt = torch.randperm(B * maxb, device=gpu).to(torch.int32).view(B, maxb)
+    kc = torch.full((B * maxb, Hkv, blk, D), float("nan"), device=gpu, dtype=torch.bfloat16)
+    vc = kc.clone()
+    q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+    want = torch.empty(B, Hq, D, dtype=torch.float64, device=gpu)
+    for b, n in enumerate(lens):
+        k, v = (torch.randn(Hkv, n, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        for j in range(0, n, blk):
+            kc[int(bt[b, j // blk]), :, :min(blk, n - j)] = k[:, j:j + blk]
+            vc[int(bt[b, j // blk]), :, :min(blk, n - j)] = v[:, j:j + blk]
+        for h in range(Hq):
+            s = k[h * Hkv // Hq].double() @ q[b, h].double() * D ** -0.5
+            want[b, h] = torch.softmax(s, 0) @ v[h * Hkv // Hq].double()
+    pos = torch.tensor(lens, dtype=torch.int32, device=gpu) - 1
+    slots = torch.arange(B, dtype=torch.int32, device=gpu)
+    ml, po = _ops().decode_attn_partials(q, kc, vc, pos, slots, max(lens), D ** -0.5, 1, bt)
+    m, l = ml[..., 0].double(), ml[..., 1].double()
+    w = torch.where(m > float("-inf"), torch.exp2(m - m.amax(-1, keepdim=True)), 0.0)
+    o = torch.where(w[..., None] > 0, po.double(), 0.0)
+    got = (w[..., None] * o).sum(2) / (w * l).sum(-1, keepdim=True)
+    err = float((got - want).norm() / want.norm())
+    assert err < (2 ** -8 if D == 128 else 2e-6), err
+    out = _ops().decode_attn(q, kc, vc, pos, slots, max(lens), D ** -0.5, 1, bt, None).view(B, Hq, D)
+    assert rel_err(out, want) < 2 ** -7
+    one = [b for b, n in enumerate(lens) if n <= blk]
+    if one:
+        i = torch.tensor(one, device=gpu)
+        y = _ops().decode_attn(q[i], kc, vc, pos[i], slots[i], blk, D ** -0.5, 1, bt, None).view(-1, Hq, D)
+        assert torch.equal(y, out[i])
