@@ -662,6 +662,37 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> rope_split(const at::Tensor& qkv,
   return {q, k, v};
 }
 
+// Causal attention of several prompts in two launches: RoPE + head split + cache append of all rows, then flash
+// attention over a table of query blocks.  qkv [T, (Hq + 2 Hkv) D], rows int32 [T, 4] (position, slot, -, -), blocks
+// int32 [n, 4] (first row of the sequence, its rows, block of 128 queries, -); positions are below max_len.
+at::Tensor prompt_attention(const at::Tensor& qkv, const at::Tensor& cos, const at::Tensor& sin, const at::Tensor& rows,
+                            const at::Tensor& blocks, int64_t max_len, int64_t Hq, int64_t Hkv, at::Tensor& k_cache,
+                            at::Tensor& v_cache, const at::Tensor& block_table, double scale) {
+  check_bf16(qkv, "qkv");
+  check_bf16(k_cache, "k_cache");
+  check_bf16(v_cache, "v_cache");
+  check_f32(cos, "cos");
+  check_f32(sin, "sin");
+  MX_CHECK(k_cache.dim() == 4 && k_cache.size(1) == Hkv && v_cache.sizes() == k_cache.sizes(), "cache shape");
+  const int64_t T = qkv.size(0), D = k_cache.size(3);
+  MX_CHECK(qkv.dim() == 2 && qkv.size(1) == (Hq + 2 * Hkv) * D && T * D * 2 < INT32_MAX, "qkv [T, (Hq + 2 Hkv) D]");
+  MX_CHECK(cos.size(-1) == D / 2 && sin.sizes() == cos.sizes() && cos.size(0) >= max_len, "rope table");
+  auto table = [&](const at::Tensor& t, const char* name) {
+    MX_CHECK(t.is_cuda() && t.scalar_type() == at::kInt && t.is_contiguous() && t.dim() == 2, name);
+    return t.data_ptr<int32_t>();
+  };
+  MX_CHECK(rows.size(0) == T && rows.size(1) == 4 && blocks.size(1) == 4, "rows [T, 4], blocks [n, 4]");
+  DevGuard g(qkv.device());
+  auto q = at::empty({Hq, T, D}, qkv.options()), k = at::empty({Hkv, T, D}, qkv.options()), v = at::empty_like(k);
+  MX_OK(mx_rope_prompts(bf(qkv), cos.data_ptr<float>(), sin.data_ptr<float>(), table(rows, "rows int32"), bfm(q), bfm(k),
+                        bfm(v), bfm(k_cache), bfm(v_cache), table(block_table, "block_table int32"),
+                        (int)block_table.size(1), (int)k_cache.size(2), (int)T, (int)Hq, (int)Hkv, (int)D, cur_stream()));
+  auto o = at::empty({T, Hq * D}, qkv.options());
+  MX_OK(mx_attn_fwd_prompts(bf(q), bf(k), bf(v), table(blocks, "blocks int32"), (int)blocks.size(0), bfm(o), (int)T,
+                            (int)Hq, (int)Hkv, (int)D, (float)scale, cur_stream()));
+  return o;
+}
+
 at::Tensor rope_merge_bwd(const at::Tensor& dq, const at::Tensor& dkp, const at::Tensor& dvp, const at::Tensor& cos,
                           const at::Tensor& sin, int64_t B, int64_t S, int64_t Hq, int64_t Hkv, int64_t D,
                           int64_t out_pad) {
@@ -956,6 +987,7 @@ TORCH_LIBRARY(mxllm, m) {
   m.def("ce_chunk(Tensor(a!) logits, Tensor labels, int ignore_index, Tensor inv_n) -> Tensor");
   m.def("ce_chunk_f32(Tensor logits, Tensor(a!) dl, Tensor labels, int ignore_index, Tensor inv_n) -> Tensor");
   m.def("rope_split(Tensor qkv, Tensor cos, Tensor sin, int B, int S, int Hq, int Hkv, int D, Tensor? positions=None) -> (Tensor, Tensor, Tensor)");
+  m.def("prompt_attention(Tensor qkv, Tensor cos, Tensor sin, Tensor rows, Tensor blocks, int max_len, int Hq, int Hkv, Tensor(a!) k_cache, Tensor(b!) v_cache, Tensor block_table, float scale) -> Tensor");
   m.def("rope_merge_bwd(Tensor dq, Tensor dkp, Tensor dvp, Tensor cos, Tensor sin, int B, int S, int Hq, int Hkv, int D, int out_pad=0) -> Tensor");
   m.def("attn_fwd(Tensor q, Tensor k, Tensor v, bool causal, float scale, int out_pad=0) -> (Tensor, Tensor)");
   m.def("w8_linear(Tensor x, Tensor q, Tensor scale) -> Tensor");
@@ -998,6 +1030,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("embedding_bwd_sorted", &embedding_bwd_sorted);
   m.impl("ce_fwd_bwd", &ce_fwd_bwd);
   m.impl("rope_split", &rope_split);
+  m.impl("prompt_attention", &prompt_attention);
   m.impl("rope_merge_bwd", &rope_merge_bwd);
   m.impl("attn_fwd", &attn_fwd);
   m.impl("attn_bwd", &attn_bwd);

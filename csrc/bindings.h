@@ -169,6 +169,11 @@ int mx_attn_combine(const float* ml, const float* po, const uint16_t* gate, int6
 int mx_attn_fwd_seg(const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* blocks, int nblk,
                     const uint16_t* gate, int64_t ldg, uint16_t* o, int T, int Hq, int Hkv, int D, int E, float scale,
                     hipStream_t stream);
+int mx_attn_fwd_prompts(const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* blocks, int nblk,
+                        uint16_t* o, int T, int Hq, int Hkv, int D, float scale, hipStream_t stream);
+int mx_rope_prompts(const uint16_t* qkv, const float* cosb, const float* sinb, const int32_t* rows, uint16_t* q,
+                    uint16_t* k, uint16_t* v, uint16_t* kc, uint16_t* vc, const int32_t* bt, int maxb, int block, int T,
+                    int Hq, int Hkv, int D, hipStream_t stream);
 int mx_chunk_attn(const void* q, int64_t qh, int64_t qt, const void* k, const void* v, int64_t kh, int64_t vh, int Dp,
                   int Ep, const int32_t* pos, const int32_t* slots, const int32_t* bt, int maxb, int block,
                   const void* gate, int64_t ldg, void* out, int f32, int64_t rows, int H, int G, int D, int E,

@@ -74,9 +74,13 @@ __device__ __forceinline__ u16x4 tr_read(const char* p) {
 // Tile kt issues K(kt + 2) and V(kt + 1) during its QK^T steps, so a K tile has two tiles of MFMAs
 // to land and a V tile one and a half, where the symmetric 2-slot ring gives both one.
 // SEG (ragged prompts): q / k / v are [heads, T, D] over the rows of all sequences and every
-// workgroup takes its query block from a table of segments that attend only to themselves (a chunk
-// of one sequence).  The softmax has a sink (a key of score 0 without a value: the running max starts
-// at 0 and the sum at 1), and the output (E <= D dims per head) is multiplied by sigmoid(gate).
+// workgroup takes its query block from a table of segments that attend only to themselves (a
+// sequence, or a chunk of one).  kSegSink: the softmax has a sink (a key of score 0 without a value: the
+// running max starts at 0 and the sum at 1), and the output (E <= D dims per head) is multiplied by
+// sigmoid(gate).  kSegPlain: neither, rows of ldo; the bits of one launch a sequence, which 6 prompts of
+// 17 - 901 tokens spent 67 us a layer on (32 heads of 64; each launch lasts as long as its longest block)
+// where the table takes 22.8.
+enum { kSegNone, kSegSink, kSegPlain };
 struct AttnSeg {
   const int4* blocks;    // [gridDim / Hq] (first row of the segment, its rows, query block, -)
   const uint16_t* gate;  // [T, ldg]: head h's gate at column h * E
@@ -84,7 +88,7 @@ struct AttnSeg {
   int T, E;
 };
 
-template <int D, bool CAUSAL, int NW, bool PROF = false, int R = 2, bool SR = false, bool SEG = false>
+template <int D, bool CAUSAL, int NW, bool PROF = false, int R = 2, bool SR = false, int SEG = kSegNone>
 __global__ void __launch_bounds__(64 * NW, 8 / NW)
 attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
                 uint16_t* __restrict__ O, float* __restrict__ LSE, int B, int Hq, int Hkv, int S, int Sk,
@@ -208,7 +212,7 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, 
     for (int j = 0; j < 16; ++j) o[d][j] = 0.f;
   // m_i: the (deferred) running max of this row in the log2 domain of the scaled
   // scores; l_i: running sum of exp2(s*sl - m_i)
-  float m_i = SEG ? 0.f : -1e30f, l_i = SEG && hh == 0 ? 1.f : 0.f;
+  float m_i = SEG == kSegSink ? 0.f : -1e30f, l_i = SEG == kSegSink && hh == 0 ? 1.f : 0.f;
 
   // Loop-invariant LDS byte addresses.  The XOR swizzle of a row depends only on
   // row & 15, so for every (n, s2) k-step and both ring buffers a fragment address
@@ -453,7 +457,7 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, 
     l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-  if constexpr (SEG) {
+  if constexpr (SEG == kSegSink) {
     if (qrow < S) {
       const uint16_t* gp = seg.gate + (row0 + qrow) * (size_t)seg.ldg + (size_t)h * seg.E;
       uint16_t* op = O + (row0 + qrow) * (size_t)ldo + (size_t)h * seg.E;
@@ -482,7 +486,7 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, 
         }
     }
   } else if (qrow < S) {
-    uint16_t* op = O + ((size_t)b * S + qrow) * (size_t)ldo + (size_t)h * D;
+    uint16_t* op = O + ((size_t)(SEG ? 0 : b) * S + row0 + qrow) * (size_t)ldo + (size_t)h * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -493,7 +497,7 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, 
         for (int j = 0; j < 4; ++j) v4[j] = f2bf(o[db][4 * gq + j] * inv);
         *reinterpret_cast<u16x4*>(op + d) = v4;
       }
-    if (hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
+    if (!SEG && hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
   }
   if constexpr (PROF) {
     const uint64_t t_end = __builtin_amdgcn_s_memtime();
@@ -785,7 +789,7 @@ attn_fwd_pp_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (qrow < S) {
-    uint16_t* op = O + ((size_t)b * S + qrow) * (size_t)ldo + (size_t)h * D;
+    uint16_t* op = O + ((size_t)(SEG ? 0 : b) * S + row0 + qrow) * (size_t)ldo + (size_t)h * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -796,7 +800,7 @@ attn_fwd_pp_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
         for (int j = 0; j < 4; ++j) v4[j] = f2bf(o[db][4 * gq + j] * inv);
         *reinterpret_cast<u16x4*>(op + d) = v4;
       }
-    if (hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
+    if (!SEG && hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
   }
 }
 
@@ -1282,12 +1286,31 @@ extern "C" int mx_attn_fwd_seg(const uint16_t* q, const uint16_t* k, const uint1
   const AttnSeg sg{reinterpret_cast<const int4*>(blocks), gate, ldg, T, E};
   const float sl = scale * 1.4426950408889634f;
 #define FWDS(DD)                                                                                                \
-  attn_fwd_kernel<DD, true, 4, false, 2, false, true><<<nblk * Hq, 256, 0, stream>>>(                           \
+  attn_fwd_kernel<DD, true, 4, false, 2, false, kSegSink><<<nblk * Hq, 256, 0, stream>>>(                           \
       q, k, v, o, nullptr, 1, Hq, Hkv, T, T, 0, sl, Hq * E, 1, nullptr, sg)
   if (D == 128) FWDS(128);
   else if (D == 64) FWDS(64);
   else if (D == 32) FWDS(32);
   else return -1;
 #undef FWDS
+  return (int)hipGetLastError();
+}
+
+// The same without sink and gate: causal attention inside every segment, o [T, Hq * D].
+extern "C" int mx_attn_fwd_prompts(const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* blocks,
+                                   int nblk, uint16_t* o, int T, int Hq, int Hkv, int D, float scale,
+                                   hipStream_t stream) {
+  if (T <= 0 || nblk <= 0) return 0;
+  if (Hkv <= 0 || Hq % Hkv) return -1;
+  const AttnSeg sg{reinterpret_cast<const int4*>(blocks), nullptr, 0, T, D};
+  const float sl = scale * 1.4426950408889634f;
+#define FWDP(DD)                                                                                                \
+  attn_fwd_kernel<DD, true, 4, false, 2, false, kSegPlain><<<nblk * Hq, 256, 0, stream>>>(                      \
+      q, k, v, o, nullptr, 1, Hq, Hkv, T, T, 0, sl, Hq * D, 1, nullptr, sg)
+  if (D == 128) FWDP(128);
+  else if (D == 64) FWDP(64);
+  else if (D == 32) FWDP(32);
+  else return -1;
+#undef FWDP
   return (int)hipGetLastError();
 }

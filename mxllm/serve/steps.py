@@ -72,7 +72,7 @@ class LlamaSteps:
         return self.model.hidden_states(torch.tensor([ids], dtype=torch.long, device=self.eng.device))
 
     def prefill_hidden(self, slots: list[int], prompts: list[list[int]]) -> torch.Tensor:
-        """Concatenated tokens through the GEMMs; attention per sequence into its own cache slot."""
+        """Concatenated tokens through the GEMMs; every sequence attends to itself and is kept in its cache slot."""
         m, c, eng = self.model, self.cfg, self.eng
         lens = [len(p) for p in prompts]
         t = torch.tensor([tok for p in prompts for tok in p], dtype=torch.long, device=eng.device)
@@ -81,7 +81,16 @@ class LlamaSteps:
         for S in lens:
             offs.append(offs[-1] + S)
 
+        rows = None
+        if ops.use_native(x):
+            rows = PromptRows(lens, eng.device, slots)
+            blocks, longest = rows.attn_blocks(max(lens)), max(lens)
+
         def attn(i, qkv):
+            if rows is not None:
+                return ops.native().prompt_attention(qkv.contiguous(), m.rope_cos, m.rope_sin, rows.rowinfo, blocks, longest,
+                                                     c.n_heads, c.n_kv_heads, eng.kv.k[i], eng.kv.v[i], eng.kv.bt,
+                                                     1.0 / math.sqrt(c.head_dim))
             outs = [dops.prefill_attention(qkv[offs[j]:offs[j + 1]], m.rope_cos, m.rope_sin,
                                            lambda k, v, j=j: eng.kv.write(i, slots[j], k, v), lens[j], c.n_heads,
                                            c.n_kv_heads, c.head_dim)

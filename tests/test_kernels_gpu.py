@@ -973,3 +973,36 @@ def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
         i = torch.tensor(one, device=gpu)
         y = _ops().decode_attn(q[i], kc, vc, pos[i], slots[i], blk, D ** -0.5, 1, bt, None).view(-1, Hq, D)
         assert torch.equal(y, out[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,Hq,Hkv", [(32, 4, 2), (64, 32, 8), (128, 8, 1)])
+@pytest.mark.parametrize("lens", [[1], [127, 1, 129], [256, 65, 700, 128, 3]])
+def test_prompt_attention(gpu, D, Hq, Hkv, lens):
+    """Prompts of several sequences in two launches: the bits of RoPE split, cache copies and attention sequence by
+    sequence; cache rows that no prompt owns stay as they are."""
+    from mxllm.ops.hybrid import PromptRows
+
+    torch.manual_seed(D + len(lens))
+    T, nslots, blk = sum(lens), len(lens) + 1, 256
+    maxb = (max(lens) + blk - 1) // blk
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=gpu, dtype=torch.bfloat16)
+    cos, sin = ref.rope_tables(max(lens), D, 500000.0, None, gpu)
+    bt = torch.randperm(nslots * maxb, device=gpu).to(torch.int32).view(nslots, maxb)
+    slots = torch.randperm(nslots)[:len(lens)].tolist()
+    kc = torch.randn(nslots * maxb, Hkv, blk, D, device=gpu, dtype=torch.bfloat16)
+    vc = torch.randn_like(kc)
+    kc2, vc2 = kc.clone(), vc.clone()
+    rows = PromptRows(lens, gpu, slots)
+    o = _ops().prompt_attention(qkv, cos, sin, rows.rowinfo, rows.attn_blocks(max(lens)), max(lens), Hq, Hkv, kc, vc, bt,
+                                D ** -0.5)
+    at = 0
+    for n, slot in zip(lens, slots):
+        q, k, v = _ops().rope_split(qkv[at:at + n].contiguous(), cos, sin, 1, n, Hq, Hkv, D, None)
+        assert torch.equal(o[at:at + n], _ops().attn_fwd(q, k, v, True, D ** -0.5)[0].view(n, Hq * D))
+        for j in range(0, n, blk):
+            m = min(blk, n - j)
+            kc2[int(bt[slot, j // blk]), :, :m] = k[0, :, j:j + m]
+            vc2[int(bt[slot, j // blk]), :, :m] = v[0, :, j:j + m]
+        at += n
+    assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
