@@ -111,7 +111,7 @@ struct G8Epi {
 
 // MOE / MOE_GLU
 struct G8Moe {
-  const int4* tiles;   // (expert, first sorted row, rows, -) of each 256-row tile; rows 0: none
+  const int4* tiles;   // (expert, first sorted row, rows, number of tiles) of each 256-row tile, the unused ones last
   const int32_t* src;  // row of A of each sorted row (nullptr: the row itself)
   uint32_t arec;       // bytes of A
   int F;               // output columns
@@ -395,10 +395,19 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
   }
   // ONE __shared__ array (a second LDS object makes hipcc drain vmcnt before LDS reads: guide §5 item 4a)
   __shared__ __attribute__((aligned(1024))) char smem[2 * G8_TILE];
-  const int nM = M >> 8, nN = N >> 8;
-  int pm, pn;
+  const int nN = N >> 8;
+  int nM = M >> 8, pm, pn;
   {
-    const int L = xcd_remap(blockIdx.x, gridDim.x);
+    // MOE: the grid is as large as any choice of experts may need.  The tiles there are, over all XCDs: by the
+    // grid's size the last XCDs had none while the first ones' 36 tiles took their 32 CUs two turns (2048 tokens, 4
+    // of 16 experts of 768, K 4096: 240 tiles of a grid of 288, 158 us; 93 by the tiles' number)
+    int grid = gridDim.x;
+    if constexpr (g8_moe(EPI)) {
+      nM = mo.tiles[0].w;
+      grid = nM * nN;
+      if ((int)blockIdx.x >= grid) return;
+    }
+    const int L = xcd_remap(blockIdx.x, grid);
     constexpr int GM = 8;
     const int per = GM * nN, grp = L / per, first = grp * GM;
     const int rows = min(GM, nM - first), in = L - grp * per;
@@ -408,7 +417,6 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
   int4 tl = {0, 0, 0, 0};
   if constexpr (g8_moe(EPI)) {
     tl = mo.tiles[pm];
-    if (tl.z == 0) return;
     B += (int64_t)tl.x * (EPI == G8_EPI_MOE_GLU ? 2 : 1) * mo.F * ldb;
   }
   // (MOE: rows are taken from the table, m0 = 0)

@@ -44,7 +44,8 @@ __global__ void __launch_bounds__(256) moe_route_kernel(const T* __restrict__ x,
 }
 
 // ------------------------------------------------------------------ grouping
-// ids [P] -> src (token of each sorted row), inv (sorted row of each pair), tiles of at most bm rows
+// ids [P] -> src (token of each sorted row), inv (sorted row of each pair), tiles of at most bm rows (expert, first
+// row, rows, number of tiles), the unused ones last
 __global__ void __launch_bounds__(1024) moe_group_kernel(const int32_t* __restrict__ ids, int P, int top, int E, int bm,
                                                          int32_t* __restrict__ src, int32_t* __restrict__ inv,
                                                          int4* __restrict__ tiles, int ntiles) {
@@ -73,9 +74,9 @@ __global__ void __launch_bounds__(1024) moe_group_kernel(const int32_t* __restri
   for (int e = t; e < E; e += 1024) {
     const int n = cnt[e];
     for (int j = 0, r = 0; r < n; ++j, r += bm)
-      if (tfirst[e] + j < ntiles) tiles[tfirst[e] + j] = int4{e, first[e] + r, min(bm, n - r), 0};
+      if (tfirst[e] + j < ntiles) tiles[tfirst[e] + j] = int4{e, first[e] + r, min(bm, n - r), tfirst[E]};
   }
-  for (int i = tfirst[E] + t; i < ntiles; i += 1024) tiles[i] = int4{0, 0, 0, 0};
+  for (int i = tfirst[E] + t; i < ntiles; i += 1024) tiles[i] = int4{0, 0, 0, tfirst[E]};
   __syncthreads();
   for (int i = t; i < P; i += 1024) {
     const int pos = atomicAdd(&first[min(max(ids[i], 0), E - 1)], 1);
