@@ -76,136 +76,157 @@ __global__ void __launch_bounds__(512) moe_route_mfma_kernel(const uint16_t* __r
 // ------------------------------------------------------------------ few tokens
 constexpr int kFewTokens = 64, kFewPairs = 1024;
 
-// GLU: y[pair] = clipped unit of x[token] through [gate | up]; else y[pair] = W x[pair].
-// Workgroups: the shared expert's slices (its rows are the tokens), then those of every expert, or - fewer pairs
-// than experts - of every pair whose expert no earlier pair has chosen.  A slice is 16 weight rows, 8 gate and
-// the 8 matching up rows where GLU; KW of the 8 waves share the K of NC slices (a fragment of the rows feeds
-// NC products), 8 / KW such sets a workgroup.
-// a.logits (GLU): the choices are made here from the router's logits; one workgroup stores them.
-template <bool GLU, int KW, int NC, int MB>
-__global__ void __launch_bounds__(512) moe_few_kernel(MoeFew a) {
-  constexpr int SL = 8 / KW * NC, CH = GLU ? 8 : 16, U = 2;
-  __shared__ int16_t sel[kFewPairs], list[kFewPairs];
-  __shared__ int count;
-  __shared__ f32x4 red[8][NC][MB][64];
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 15, g = lane >> 4;
-  const int snx = a.sw ? (a.sN + SL * CH - 1) / (SL * CH) : 0, nx = (a.N + SL * CH - 1) / (SL * CH);
-  const bool shared = (int)blockIdx.x < snx;
-  const int N = shared ? a.sN : a.N, K = shared ? a.sK : a.K, P = a.T * a.top;
-  const int bx = shared ? blockIdx.x : (blockIdx.x - snx) % nx, unit = shared ? 0 : (blockIdx.x - snx) / nx;
-  const int ks = w % KW, n0 = (bx * SL + w / KW * NC) * CH;
-  int n = a.T, expert = 0;
-  if (!shared) {
-    if (GLU && a.logits) {
-      for (int t = w; t < a.T; t += 8) {
-        const int store = (int)blockIdx.x == snx;
-        moe_choose64(lane < a.E ? a.logits[(int64_t)t * a.E + lane] : 0.f, a.E, a.top, lane, [&](int k, float wt) {
-          sel[t * a.top + k] = (int16_t)lane;
-          if (store) {
-            a.ids_out[t * a.top + k] = lane;
-            a.wts_out[t * a.top + k] = wt;
-          }
-        });
-      }
-    } else {
-      for (int i = tid; i < P; i += 512) sel[i] = (int16_t)min(max(a.ids[i], 0), a.E - 1);
-    }
-    __syncthreads();
-    expert = P <= a.E ? sel[unit] : unit;
-    if (w == 0) {  // pairs whose choice this expert is
-      int at = 0, first = P;
-      for (int i0 = 0; i0 < P; i0 += 64) {
-        const bool hit = i0 + lane < P && sel[i0 + lane] == expert;
-        const uint64_t m = __ballot(hit);
-        if (hit) list[at + __popcll(m & ((1ull << lane) - 1))] = (int16_t)(i0 + lane);
-        if (m && first == P) first = i0 + __ffsll((unsigned long long)m) - 1;
-        at += __popcll(m);
-      }
-      if (lane == 0) count = P <= a.E && first < unit ? 0 : at;
-    }
-    __syncthreads();
-    n = count;
-    if (n == 0) return;
-  }
-  const uint16_t* W = shared ? a.sw : a.w + (int64_t)expert * (GLU ? 2 : 1) * a.N * a.K;
+// What bounds them: weights read once (67 MB up, 34 MB down for 32 tokens at 1B sizes), and behind one another the
+// choices, the list of an expert's pairs, its rows and its weights; several workgroups a CU hide each other's waits,
+// so more loads in flight a wave, which cost registers, lose (blocks of 4 chunks issued ahead of the choices: up
+// 22.5 -> 33.9 us).
+// One slice set: 16 weight rows a slice, 8 gate and the 8 matching up rows where GLU; KW of the 8 waves share the K
+// of NC slices (a fragment of the rows feeds NC products), 8 / KW such sets a workgroup.
+template <bool GLU, int KW, int NC>
+struct FewSlices {
+  static constexpr int SL = 8 / KW * NC, CH = GLU ? 8 : 16, U = 2;
   const uint16_t* wr[NC];
-#pragma unroll
-  for (int j = 0; j < NC; ++j)
-    wr[j] = W + ((int64_t)(GLU && c >= 8 ? N : 0) + min(n0 + j * CH + (GLU ? c & 7 : c), N - 1)) * K;
-  const int steps = (K + 63) / 64, per = (steps + KW - 1) / KW;
-  const int k0 = ks * per * 64, k1 = min(K, k0 + per * 64);
-  uint16_t* const y = shared ? a.sy : a.y;
-  for (int r0 = 0; r0 < n; r0 += 16 * MB) {
-    const uint16_t* xr[MB];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int r = min(r0 + 16 * mb + c, n - 1);
-      if (GLU) xr[mb] = a.x + (int64_t)(shared ? r : list[r] / a.top) * a.ldx;
-      else xr[mb] = shared ? a.sx + (int64_t)r * a.sK : a.x + (int64_t)list[r] * a.ldx;
-    }
-    f32x4 acc[NC][MB];
+  int n0, k0, k1, ks;
+
+  __device__ __forceinline__ FewSlices(const uint16_t* W, int bx, int N, int K, int w, int c) {
+    ks = w % KW;
+    n0 = (bx * SL + w / KW * NC) * CH;
+    const int steps = (K + 63) / 64, per = (steps + KW - 1) / KW;
+    k0 = ks * per * 64, k1 = min(K, k0 + per * 64);
 #pragma unroll
     for (int j = 0; j < NC; ++j)
+      wr[j] = W + ((int64_t)(GLU && c >= 8 ? N : 0) + min(n0 + j * CH + (GLU ? c & 7 : c), N - 1)) * K;
+  }
+  // n rows: xrow(r) reads, yrow(r) is the output's; limit of the unit
+  template <int MB, typename X, typename Y>
+  __device__ __forceinline__ void run(int n, int N, X xrow, Y yrow, uint16_t* y, float limit, f32x4* red, int w, int lane,
+                                      int c, int g) {
+    auto slot = [&](int wv, int j, int mb) -> f32x4& { return red[((wv * NC + j) * MB + mb) * 64 + lane]; };
+    for (int r0 = 0; r0 < n; r0 += 16 * MB) {
+      const uint16_t* xr[MB];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int kb = k0; kb < k1; kb += 64 * U) {
-      u16x8 fa[U][NC][2], fb[U][MB][2];
+      for (int mb = 0; mb < MB; ++mb) xr[mb] = xrow(min(r0 + 16 * mb + c, n - 1));
+      f32x4 acc[NC][MB];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = kb + 64 * u + 16 * g;
-        const bool on = k < k1;  // K is a multiple of 16
-        const int kk = on ? k : 0;
+      for (int j = 0; j < NC; ++j)
 #pragma unroll
-        for (int j = 0; j < NC; ++j) {
-          fa[u][j][0] = *reinterpret_cast<const u16x8*>(wr[j] + kk);
-          fa[u][j][1] = *reinterpret_cast<const u16x8*>(wr[j] + kk + 8);
-        }
+        for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int kb = k0; kb < k1; kb += 64 * U) {
+        u16x8 fa[U][NC][2], fb[U][MB][2];
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          fb[u][mb][0] = *reinterpret_cast<const u16x8*>(xr[mb] + kk);
-          fb[u][mb][1] = *reinterpret_cast<const u16x8*>(xr[mb] + kk + 8);
-          if (!on) fb[u][mb][0] = fb[u][mb][1] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
+        for (int u = 0; u < U; ++u) {
+          const int k = kb + 64 * u + 16 * g;
+          const bool on = k < k1;  // K is a multiple of 16
+          const int kk = on ? k : 0;
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int j = 0; j < NC; ++j)
+          for (int j = 0; j < NC; ++j) {
+            fa[u][j][0] = *reinterpret_cast<const u16x8*>(wr[j] + kk);
+            fa[u][j][1] = *reinterpret_cast<const u16x8*>(wr[j] + kk + 8);
+          }
 #pragma unroll
           for (int mb = 0; mb < MB; ++mb) {
-            acc[j][mb] = mfma16_sk(fa[u][j][0], fb[u][mb][0], acc[j][mb]);
-            acc[j][mb] = mfma16_sk(fa[u][j][1], fb[u][mb][1], acc[j][mb]);
+            fb[u][mb][0] = *reinterpret_cast<const u16x8*>(xr[mb] + kk);
+            fb[u][mb][1] = *reinterpret_cast<const u16x8*>(xr[mb] + kk + 8);
+            if (!on) fb[u][mb][0] = fb[u][mb][1] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
           }
-    }
-    if (r0) __syncthreads();  // the previous rows' sums are read
-#pragma unroll
-    for (int j = 0; j < NC; ++j)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) red[w][j][mb][lane] = acc[j][mb];
-    __syncthreads();
-    for (int jm = ks; jm < NC * MB; jm += KW) {  // the K parts' waves share the sums
-      const int j = jm % NC, mb = jm / NC;
-      f32x4 s = red[w - ks][j][mb][lane];
-#pragma unroll
-      for (int i = 1; i < KW; ++i) s += red[w - ks + i][j][mb][lane];
-      const int r = r0 + 16 * mb + c, ch = n0 + j * CH + 4 * g;
-      u16x4 o;
-      if constexpr (GLU) {  // rows 4 g .. of the slice: gate in groups 0 and 1, up in 2 and 3
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float up = __shfl_xor(s[i], 32, 64);
-          o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, shared ? a.slimit : a.limit));
         }
-      } else {
+        __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
 #pragma unroll
-        for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int j = 0; j < NC; ++j)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+              acc[j][mb] = mfma16_sk(fa[u][j][0], fb[u][mb][0], acc[j][mb]);
+              acc[j][mb] = mfma16_sk(fa[u][j][1], fb[u][mb][1], acc[j][mb]);
+            }
       }
-      if (r < n && ch < N && (!GLU || g < 2))
-        *reinterpret_cast<u16x4*>(y + (int64_t)(shared ? r : list[r]) * N + ch) = o;
+      if (r0) __syncthreads();  // the previous rows' sums are read
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) slot(w, j, mb) = acc[j][mb];
+      __syncthreads();
+      for (int jm = ks; jm < NC * MB; jm += KW) {  // the K parts' waves share the sums
+        const int j = jm % NC, mb = jm / NC;
+        f32x4 s = slot(w - ks, j, mb);
+#pragma unroll
+        for (int i = 1; i < KW; ++i) s += slot(w - ks + i, j, mb);
+        const int r = r0 + 16 * mb + c, ch = n0 + j * CH + 4 * g;
+        u16x4 o;
+        if constexpr (GLU) {  // rows 4 g .. of the slice: gate in groups 0 and 1, up in 2 and 3
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float up = __shfl_xor(s[i], 32, 64);
+            o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, limit));
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+        }
+        if (r < n && ch < N && (!GLU || g < 2)) *reinterpret_cast<u16x4*>(y + (int64_t)yrow(r) * N + ch) = o;
+      }
     }
   }
+};
+
+// GLU: y[pair] = clipped unit of x[token] through [gate | up]; else y[pair] = W x[pair].
+// Workgroups: the shared expert's slices (its rows are the tokens), then those of every expert, or - fewer pairs
+// than experts - of every pair whose expert no earlier pair has chosen.  KW, NC, MB: the experts' slices (MB blocks
+// of 16 rows at a time); SKW, SNC, SMB the shared one's, whose K is longer and whose rows are all tokens.
+// a.logits (GLU): the choices are made here from the router's logits; one workgroup stores them.
+template <bool GLU, int KW, int NC, int MB, int SKW, int SNC, int SMB>
+__global__ void __launch_bounds__(512) moe_few_kernel(MoeFew a) {
+  using Own = FewSlices<GLU, KW, NC>;
+  using Shared = FewSlices<GLU, SKW, SNC>;
+  __shared__ int16_t sel[kFewPairs], list[kFewPairs];
+  __shared__ int count;
+  __shared__ f32x4 red[8 * 64 * (NC * MB > SNC * SMB ? NC * MB : SNC * SMB)];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  constexpr int SCOLS = Shared::SL * Shared::CH, COLS = Own::SL * Own::CH;
+  const int snx = a.sw ? (a.sN + SCOLS - 1) / SCOLS : 0, nx = (a.N + COLS - 1) / COLS, P = a.T * a.top;
+  if ((int)blockIdx.x < snx) {
+    Shared s(a.sw, blockIdx.x, a.sN, a.sK, w, c);
+    s.template run<SMB>(
+        a.T, a.sN, [&](int r) { return GLU ? a.x + (int64_t)r * a.ldx : a.sx + (int64_t)r * a.sK; },
+        [](int r) { return r; }, a.sy, a.slimit, red, w, lane, c, g);
+    return;
+  }
+  const int bx = (blockIdx.x - snx) % nx, unit = (blockIdx.x - snx) / nx;
+  if (GLU && a.logits) {
+    for (int t = w; t < a.T; t += 8) {
+      const int store = (int)blockIdx.x == snx;
+      moe_choose64(lane < a.E ? a.logits[(int64_t)t * a.E + lane] : 0.f, a.E, a.top, lane, [&](int k, float wt) {
+        sel[t * a.top + k] = (int16_t)lane;
+        if (store) {
+          a.ids_out[t * a.top + k] = lane;
+          a.wts_out[t * a.top + k] = wt;
+        }
+      });
+    }
+  } else {
+    for (int i = tid; i < P; i += 512) sel[i] = (int16_t)min(max(a.ids[i], 0), a.E - 1);
+  }
+  __syncthreads();
+  const int expert = P <= a.E ? sel[unit] : unit;
+  if (w == 0) {  // pairs whose choice this expert is
+    int at = 0, first = P;
+    for (int i0 = 0; i0 < P; i0 += 64) {
+      const bool hit = i0 + lane < P && sel[i0 + lane] == expert;
+      const uint64_t m = __ballot(hit);
+      if (hit) list[at + __popcll(m & ((1ull << lane) - 1))] = (int16_t)(i0 + lane);
+      if (m && first == P) first = i0 + __ffsll((unsigned long long)m) - 1;
+      at += __popcll(m);
+    }
+    if (lane == 0) count = P <= a.E && first < unit ? 0 : at;
+  }
+  __syncthreads();
+  if (count == 0) return;
+  Own s(a.w + (int64_t)expert * (GLU ? 2 : 1) * a.N * a.K, bx, a.N, a.K, w, c);
+  s.template run<MB>(
+      count, a.N, [&](int r) { return a.x + (int64_t)(GLU ? list[r] / a.top : list[r]) * a.ldx; },
+      [&](int r) { return list[r]; }, a.y, a.limit, red, w, lane, c, g);
 }
 
 }  // namespace mx
@@ -261,24 +282,30 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
       (a.sw && (a.sN <= 0 || a.sN % 4 || a.sK <= 0 || a.sK % 16)))
     return -1;
   // channels of a workgroup: up 16, from 33 tokens on 32 (the rows' fragments are then most of the traffic);
-  // down 64, for a few pairs 32 with K in four parts
+  // down 64, for a few pairs 32 with K in four parts; the shared expert's down, whose K is the longest, 16 with K in
+  // eight (its few workgroups were the last to end: K 2048 in two parts are 16 waits for memory one after another;
+  // 32 tokens, 1B sizes 30.5 -> 16.1 us, 4 tokens 15.6 -> 10.3; 8B sizes 38.4 -> 33.1, 22.2 -> 18.7)
   const bool split = !glu && a.T * a.top <= 8;
-  const int64_t cols = glu ? (a.T <= 32 ? 16 : 32) : split ? 32 : 64, units = a.T * a.top <= a.E ? a.T * a.top : a.E;
-  const int64_t g = units * ((a.N + cols - 1) / cols) + (a.sw ? (a.sN + cols - 1) / cols : 0);
-  if (g > INT32_MAX) return -1;
-#define MF(GLU, KW, NC, MB) moe_few_kernel<GLU, KW, NC, MB><<<(unsigned)g, 512, 0, stream>>>(a)
+  const int64_t units = a.T * a.top <= a.E ? a.T * a.top : a.E;
+#define MF(GLU, KW, NC, MB, SKW, SNC, SMB)                                                                       \
+  do {                                                                                                           \
+    const int64_t cols = 8 / KW * NC * (GLU ? 8 : 16), sc = 8 / SKW * SNC * (GLU ? 8 : 16);                      \
+    const int64_t gr = units * ((a.N + cols - 1) / cols) + (a.sw ? (a.sN + sc - 1) / sc : 0);                    \
+    if (gr > INT32_MAX) return -1;                                                                               \
+    moe_few_kernel<GLU, KW, NC, MB, SKW, SNC, SMB><<<(unsigned)gr, 512, 0, stream>>>(a);                         \
+  } while (0)
   if (glu) {
-    if (a.T <= 16) MF(true, 8, 2, 1);
-    else if (a.T <= 32) MF(true, 8, 2, 2);
-    else MF(true, 8, 4, 4);
+    if (a.T <= 16) MF(true, 8, 2, 1, 8, 2, 1);
+    else if (a.T <= 32) MF(true, 8, 2, 2, 8, 2, 2);
+    else MF(true, 8, 4, 4, 8, 4, 4);
   } else if (split) {
-    MF(false, 4, 1, 1);
+    MF(false, 4, 1, 1, 8, 1, 1);
   } else if (a.T <= 16) {
-    MF(false, 2, 1, 1);
+    MF(false, 2, 1, 1, 8, 1, 1);
   } else if (a.T <= 32) {
-    MF(false, 2, 1, 2);
+    MF(false, 2, 1, 2, 8, 1, 2);
   } else {
-    MF(false, 2, 1, 4);
+    MF(false, 2, 1, 4, 8, 1, 4);
   }
 #undef MF
   return (int)hipGetLastError();
