@@ -9,14 +9,14 @@ Every training GEMM of a Llama step is one of four operand orders over row-major
   tt    [K][M]     [K][N]     A^T @ B           weight gradient dW = dY^T X (token-major operands)
   nt    [K][M]     [N][K]     A^T @ B^T         (unused; for completeness)
 
-``gemm8`` is selected per (form, M, N, K, output dtype) only where it was measured faster
-(entries with ``tail``: the tail-balanced launch, ``mx_gemm8_tail`` -- a last wave of at most half
-the CUs runs as twice as many half-K workgroups, e.g. the 16 x 40-tile 70B qkv forward)
-(``mxllm/tuning/gemm8_gfx950.json``, written from ``bench/gemm8_probe.py`` runs), or for every
-shape it takes in deterministic mode (``MXLLM_DETERMINISTIC=1``: one workgroup per output tile,
-a fixed K order, no split-K or atomics — the step is bitwise reproducible; vendor stream-K
-solutions are not, archive/profiles/r3aa).  ``MXLLM_GEMM8=0`` disables it, ``=all`` forces it wherever
-it takes the shape (A/B runs).
+``gemm8`` is selected only where it was measured faster: per (form, M, N, K, output dtype) from a
+table (``mxllm/tuning/gemm8_gfx950.json``, written from ``bench/gemm8_probe.py`` runs; entries with
+``tail``: the tail-balanced launch, ``mx_gemm8_tail`` -- a last wave of at most half the CUs runs as
+twice as many half-K workgroups, e.g. the 16 x 40-tile 70B qkv forward), by the rule of ``_gains``
+for the sizes that the table does not hold, or for every shape it takes in deterministic mode
+(``MXLLM_DETERMINISTIC=1``: one workgroup per output tile, a fixed K order, no split-K or atomics —
+the step is bitwise reproducible; vendor stream-K solutions are not, archive/profiles/r3aa).
+``MXLLM_GEMM8=0`` disables it, ``=all`` forces it wherever it takes the shape (A/B runs).
 """
 from __future__ import annotations
 
@@ -111,7 +111,31 @@ def schedule(form: str, M: int, N: int, K: int, out_dtype: torch.dtype) -> int:
         ph = 4  # persistent kernel: world 1 only (see _multi_rank)
     if ph:
         return ph
+    if out_dtype == torch.bfloat16 and _gains(form, M, N, K):
+        return 4
     return DEFAULT_PH if (pol == "all" or deterministic()) else 0
+
+
+def _gains(form: str, M: int, N: int, K: int) -> bool:
+    """bf16-output shapes outside the table that gemm8 (4-phase, one 256 x 256 tile a CU) runs faster.
+
+    ``tt``: what it saves is the two transposes and their launches; what it loses to hipBLASLt is the split of
+    a long K when the tiles leave CUs idle.  (us: transposes + hipBLASLt -> gemm8; M x N, K tokens)
+      * a short K, at any number of tiles: 512 x 512, 1000: 40 -> 23; 2048 x 2048, 300: 41 -> 14
+        (4 to 64 tiles at 2048: 37 -> 38..41, at 4096: 36..56 -> 70..75);
+      * a K that is no multiple of 64, which hipBLASLt reads slowly: 16384 x 2048, 3606: 271 -> 179;
+      * else a last wave that is full enough.  One wave: 144 tiles 4096: 89 -> 77, 8192: 161 -> 146 (128 tiles 77 ->
+        78 and 144 -> 154).  More: 256 tiles 118 -> 98, 512 237 -> 200, 384 172 -> 167 (288 tiles 149 -> 160).
+    ``nn``: both read the operands as they are; gemm8 from 11 sixteenths of the CUs on (28672 -> 4096 at 2816
+    rows, 176 tiles: 864 -> 552; 224 tiles, 6144 -> 4096: 148 -> 129; 160 tiles of 8192: 176 -> 182)."""
+    tiles = (M // 256) * (N // 256)
+    # past the kernel's 32-bit offsets (it would decline: the caller's other path stays)
+    if K < 128 or (K + 63) // 64 * 64 * max(M if form == "tt" else 0, N) >= 1 << 30:
+        return False
+    if form == "tt":
+        full = tiles / (-(-tiles // CUS) * CUS)
+        return K <= 1536 or (K % 64 != 0 and tiles >= 64) or (tiles >= 144 and full >= (0.56 if tiles <= CUS else 0.7))
+    return form == "nn" and tiles >= CUS * 11 // 16
 
 
 DEFAULT_PH = int(os.environ.get("MXLLM_GEMM8_DEFAULT_PH", "4"))

@@ -95,6 +95,21 @@ def test_gemm8_weight_grad_odd_tokens(gpu, T, ph, monkeypatch):
     _check(out, dy.float().t() @ x.float(), 1e-5)
 
 
+@pytest.mark.parametrize("T,N,K", [(128, 256, 256), (150, 256, 512), (1536, 512, 256), (1537, 2048, 2048), (1600, 3072, 3072)])
+def test_weight_grad_route(gpu, T, N, K):
+    """Weight gradients that the rule puts on gemm8, first written and accumulated, against float32."""
+    from mxllm.ops import gemm
+    from mxllm.ops.linear import weight_grad_
+
+    assert gemm.schedule("tt", N, K, T, torch.bfloat16) == 4
+    dy, x = _mat(T, N, gpu, pad=8, seed=6), _mat(T, K, gpu, pad=8, seed=7)
+    ref = dy.float().t() @ x.float()
+    out = weight_grad_(torch.full((N, K), float("nan"), device=gpu, dtype=torch.bfloat16), dy, x, beta=0.0)
+    _check(out, ref, 5e-3)
+    base = out.clone()
+    _check(weight_grad_(out, dy, x, beta=1.0), ref + base.float(), 5e-3)
+
+
 @pytest.mark.parametrize("ph", ["8", "4"])
 def test_gemm8_odd_ktiles_nn(gpu, ph, monkeypatch):
     """the LoRA-augmented dX shape: K = N_out + 64 (an odd number of 64-deep K-tiles)."""
