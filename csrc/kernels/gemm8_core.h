@@ -89,9 +89,14 @@ __device__ __forceinline__ int g8_map_a(int r, int h) { return (r >> 6) * 128 + 
 //               to 256 rows of one expert out of a table; A's rows are gathered through it, rows, columns and
 //               K past the end read as zeros and are not stored (K, F and the strides are multiples of 8).
 //               GLU: columns as SWIGLU (gate and up of one channel in one lane), output [rows, F]
+//  G8_EPI_ROWS / G8_EPI_ROWS_SWIGLU: any number of rows (A k-contiguous; the last tile's rows past M read as zeros
+//               through the descriptor's range and are not stored).  SWIGLU: only m = silu(g) u is stored, the
+//               projection itself never leaves the registers
 constexpr int G8_EPI_NONE = 0, G8_EPI_ROPE = 1, G8_EPI_SWIGLU = 2, G8_EPI_SWIGLU_BWD = 3, G8_EPI_MOE = 4,
-              G8_EPI_MOE_GLU = 5;
+              G8_EPI_MOE_GLU = 5, G8_EPI_ROWS = 6, G8_EPI_ROWS_SWIGLU = 7;
 constexpr bool g8_moe(int epi) { return epi == G8_EPI_MOE || epi == G8_EPI_MOE_GLU; }
+constexpr bool g8_rows(int epi) { return epi == G8_EPI_ROWS || epi == G8_EPI_ROWS_SWIGLU; }
+constexpr bool g8_pairs(int epi) { return epi == G8_EPI_SWIGLU || epi == G8_EPI_ROWS_SWIGLU; }
 constexpr uint32_t G8_OOB = 0x80000000u;  // past every descriptor's range: reads as zeros
 
 struct G8Epi {
@@ -123,7 +128,7 @@ template <int EPI>
 __device__ __forceinline__ int g8_epi_row(int v, int pn, int F) {
   if constexpr (EPI == G8_EPI_ROPE) {
     return (v & ~127) + ((v >> 6) & 1) * 32 + ((v >> 5) & 1) * 64 + (v & 31);
-  } else if constexpr (EPI == G8_EPI_SWIGLU || EPI == G8_EPI_MOE_GLU) {
+  } else if constexpr (g8_pairs(EPI) || EPI == G8_EPI_MOE_GLU) {
     return (((v >> 5) & 1) ? F : 0) + 128 * pn + (v >> 6) * 32 + (v & 31);
   } else {
     return v;
@@ -214,7 +219,7 @@ __device__ __forceinline__ void g8_store8(uint16_t* dst, const f32x4& va, const 
 
 template <int EPI>
 __device__ __forceinline__ void g8_epilogue_fused(f32x4 (&acc)[8][4], float alpha, int ml, int pn, int wc, int lane,
-                                                  int N, const G8Epi& ep, void* C, int64_t ldc, const G8Moe& mo, const int4& tl) {
+                                                  int M, int N, const G8Epi& ep, void* C, int64_t ldc, const G8Moe& mo, const int4& tl) {
   // this lane's 8 stored columns start at offset u8 inside a 32-column group (after the swap)
   const int u8 = 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
   if constexpr (g8_moe(EPI)) {
@@ -343,6 +348,38 @@ __device__ __forceinline__ void g8_epilogue_fused(f32x4 (&acc)[8][4], float alph
         }
       }
     }
+  } else if constexpr (EPI == G8_EPI_ROWS) {
+#pragma unroll
+    for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = ml + qa * 64 + 16 * i;
+#pragma unroll
+        for (int jp = 0; jp < 2; ++jp) {
+          const f32x4 va = acc[4 * qa + i][2 * jp] * alpha, vb = acc[4 * qa + i][2 * jp + 1] * alpha;
+          const uint4 o = g8_pack8(va, vb);  // lanes exchange: outside the row test
+          if (m < M)
+            *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(C) + m * ldc + 256 * pn + 64 * wc + 32 * jp + u8) = o;
+        }
+      }
+  } else if constexpr (EPI == G8_EPI_ROWS_SWIGLU) {
+    const int col = 128 * pn + 32 * wc + u8;
+#pragma unroll
+    for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = ml + qa * 64 + 16 * i;
+        f32x4 mm[2];
+#pragma unroll
+        for (int jl = 0; jl < 2; ++jl)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const float g = g8_rbf(acc[4 * qa + i][jl][c] * alpha), u = g8_rbf(acc[4 * qa + i][2 + jl][c] * alpha);
+            mm[jl][c] = g * g8_sigmoid(g) * u;
+          }
+        const uint4 o = g8_pack8(mm[0], mm[1]);
+        if (m < M) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(C) + m * ldc + col) = o;
+      }
   } else {  // G8_EPI_SWIGLU
     const int F = N / 2;
     const int col = 128 * pn + 32 * wc + u8;  // gate column (up: + F; m: the same column)
@@ -380,7 +417,7 @@ __global__ void __launch_bounds__(512, 1)
 gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
              void* __restrict__ C, int64_t ldc, int M, int N, int K, const float* __restrict__ alpha_t,
              float alpha_f, int k0 = 0, int64_t cpart = 0, G8Epi ep = G8Epi{}, G8Moe mo = G8Moe{}) {
-  static_assert(EPI == G8_EPI_NONE || (!OUT_F32 && !BETA && (EPI == G8_EPI_SWIGLU_BWD ? A_KC && !B_KC : A_KC && B_KC)),
+  static_assert(EPI == G8_EPI_NONE || (!OUT_F32 && !BETA && (EPI == G8_EPI_ROWS ? A_KC : EPI == G8_EPI_SWIGLU_BWD ? A_KC && !B_KC : A_KC && B_KC)),
                 "fused epilogues: bf16, beta 0; TN-form forwards, NN-form SwiGLU backward");
   // K split in two (gridDim.y == 2, k0 = K of part 0): part 1 covers K rows / columns k0 .. K-1 of
   // both operands and writes its own output image C + cpart (mx_gemm8_tail: the last, partial wave
@@ -396,7 +433,7 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
   // ONE __shared__ array (a second LDS object makes hipcc drain vmcnt before LDS reads: guide §5 item 4a)
   __shared__ __attribute__((aligned(1024))) char smem[2 * G8_TILE];
   const int nN = N >> 8;
-  int nM = M >> 8, pm, pn;
+  int nM = (g8_rows(EPI) ? M + 255 : M) >> 8, pm, pn;
   {
     // MOE: the grid is as large as any choice of experts may need.  The tiles there are, over all XCDs: by the
     // grid's size the last XCDs had none while the first ones' 36 tiles took their 32 CUs two turns (2048 tokens, 4
@@ -439,10 +476,10 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
   // ---- operand descriptors (range-checked: mn-contiguous rows past K read as zeros)
   const uint16_t* abase = A_KC ? A + (int64_t)m0 * lda : A + m0;
   // SWIGLU: gate and up rows are F apart -> absolute weight rows off the start of B
-  const uint16_t* bbase = B_KC ? B + (int64_t)(EPI == G8_EPI_SWIGLU || g8_moe(EPI) ? 0 : n0) * ldb : B + n0;
-  const uint32_t arec = g8_moe(EPI) ? mo.arec : A_KC ? (uint32_t)((255 * lda + (int64_t)nk * G8_BK) * 2) : (uint32_t)(((int64_t)K * lda - m0) * 2);
+  const uint16_t* bbase = B_KC ? B + (int64_t)(g8_pairs(EPI) || g8_moe(EPI) ? 0 : n0) * ldb : B + n0;
+  const uint32_t arec = g8_moe(EPI) ? mo.arec : A_KC ? (uint32_t)(((g8_rows(EPI) ? min(255, M - 1 - m0) : 255) * lda + (int64_t)nk * G8_BK) * 2) : (uint32_t)(((int64_t)K * lda - m0) * 2);
   const uint32_t brec = g8_moe(EPI) ? (uint32_t)((int64_t)(EPI == G8_EPI_MOE_GLU ? 2 : 1) * mo.F * ldb * 2)
-                        : EPI == G8_EPI_SWIGLU ? (uint32_t)(((int64_t)(N - 1) * ldb + (int64_t)nk * G8_BK) * 2)
+                        : g8_pairs(EPI) ? (uint32_t)(((int64_t)(N - 1) * ldb + (int64_t)nk * G8_BK) * 2)
                         : B_KC ? (uint32_t)((255 * ldb + (int64_t)nk * G8_BK) * 2)
                                : (uint32_t)(((int64_t)K * ldb - n0) * 2);
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void*)abase, 0, arec, 0x00020000);
@@ -734,7 +771,7 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
   const int ml = m0 + wr * 128 + (lane & 15);
   const int nl = n0 + wc * 64 + 4 * (lane >> 4);
   if constexpr (EPI != G8_EPI_NONE) {
-    g8_epilogue_fused<EPI>(acc, alpha, ml, pn, wc, lane, N, ep, C, ldc, mo, tl);
+    g8_epilogue_fused<EPI>(acc, alpha, ml, pn, wc, lane, M, N, ep, C, ldc, mo, tl);
     return;
   }
 #pragma unroll

@@ -126,16 +126,60 @@ def _gains(form: str, M: int, N: int, K: int) -> bool:
       * a K that is no multiple of 64, which hipBLASLt reads slowly: 16384 x 2048, 3606: 271 -> 179;
       * else a last wave that is full enough.  One wave: 144 tiles 4096: 89 -> 77, 8192: 161 -> 146 (128 tiles 77 ->
         78 and 144 -> 154).  More: 256 tiles 118 -> 98, 512 237 -> 200, 384 172 -> 167 (288 tiles 149 -> 160).
-    ``nn``: both read the operands as they are; gemm8 from 11 sixteenths of the CUs on (28672 -> 4096 at 2816
-    rows, 176 tiles: 864 -> 552; 224 tiles, 6144 -> 4096: 148 -> 129; 160 tiles of 8192: 176 -> 182)."""
+    ``nn``: :func:`_gains_nn`."""
     tiles = (M // 256) * (N // 256)
     # past the kernel's 32-bit offsets (it would decline: the caller's other path stays)
     if K < 128 or (K + 63) // 64 * 64 * max(M if form == "tt" else 0, N) >= 1 << 30:
         return False
     if form == "tt":
-        full = tiles / (-(-tiles // CUS) * CUS)
+        full = _wave_fill(tiles)
         return K <= 1536 or (K % 64 != 0 and tiles >= 64) or (tiles >= 144 and full >= (0.56 if tiles <= CUS else 0.7))
-    return form == "nn" and tiles >= CUS * 11 // 16
+    return form == "nn" and _gains_nn(tiles)
+
+
+def _wave_fill(tiles: int) -> float:
+    """Part of the CUs' turns that ``tiles`` of one workgroup a CU use."""
+    return tiles / (max(-(-tiles // CUS), 1) * CUS)
+
+
+def _gains_nn(tiles: int) -> bool:
+    """Input gradients: both kernels read the operands as they are; gemm8 where its tiles fill their waves (us,
+    library -> gemm8): 176 tiles, 28672 -> 4096 at 2600 rows 830 -> 536, 6144 -> 4096 115 -> 109; 192, 8192 -> 8192 at
+    1300 149 -> 142; 352 at 2600 300 -> 300; 784, 4096 -> 14336 at 3606 417 -> 336; but 160 tiles 176 -> 182, 280
+    133 -> 152, 320 at 5000 219 -> 228."""
+    return _wave_fill(tiles) >= 0.68
+
+
+def rows_ok(a: torch.Tensor, b: torch.Tensor, b_kc: bool, swiglu: bool = False) -> bool:
+    """What mx_gemm8_rows (csrc/kernels/gemm8.hip) takes: any number of rows of ``a`` [M, K]."""
+    if not (use_native(a) and a.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16):
+        return False
+    K, N = a.shape[1], b.shape[0 if b_kc else 1]
+    ldb = b.stride(0)
+    return bool(a.shape[0] > 0 and K % 64 == 0 and K > 0 and N % 256 == 0 and N > 0
+                and a.stride(1) == 1 and b.stride(1) == 1 and a.stride(0) % 8 == 0 and ldb % 8 == 0
+                and a.stride(0) >= K and ldb >= (K if b_kc else N)
+                and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
+                and 256 * a.stride(0) < 1 << 30 and (N if swiglu else 256 if b_kc else K) * ldb < 1 << 30)
+
+
+def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> bool:
+    """Whether the rows kernel is the faster one; the library is tuned for round numbers of rows, and falls behind
+    between them (us, library -> gemm8; H x N at rows):
+      * projections (``b_kc``) from 700 tiles on: 4096 x 28672 at 2600 542 -> 450, 3606 612 -> 617, 5000 904 -> 820;
+        8192 x 57344 at 700 559 -> 530 (4096 x 28672 at 1025, 560 tiles: 235 -> 241; 14336 x 4096 at 2600, 176: 237 -> 243);
+      * input gradients: :func:`_gains_nn`;
+      * gate-up with SwiGLU, which saves the projection's trip through HBM at any size: where the last tile's rows are
+        not mostly padding and half the CUs have a tile.  2048 x 16384 at 700 57 -> 46, 2600 205 -> 142, 4096 236 -> 198;
+        4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 1025 249 -> 241, 4096 706 -> 640."""
+    if _policy() == "0":
+        return False
+    tiles = -(-M // 256) * (N // 256)
+    if swiglu:
+        return tiles >= CUS // 2 and 4 * M >= 3 * (-(-M // 256) * 256)
+    if M % 256 == 0:
+        return False
+    return tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles)
 
 
 DEFAULT_PH = int(os.environ.get("MXLLM_GEMM8_DEFAULT_PH", "4"))
@@ -166,6 +210,9 @@ def mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = N
     ``alpha_t``: optional 1-element f32 device scalar (no host sync)."""
     M, N, K = _dims(form, a, b)
     odt = out.dtype if out is not None else (out_dtype or a.dtype)
+    if (out is None and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16
+            and rows_gain(M, N, K, form == "tn") and rows_ok(a, b, form == "tn")):
+        return native().gemm8_rows(a, b, form == "tn", False)
     if out is None:
         out = torch.empty(M, N, dtype=odt, device=a.device)
         beta = 0.0

@@ -31,6 +31,7 @@ from typing import Sequence
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from ..parallel.grad_ready import direct_grad, direct_grad32, mark_ready
 from . import gemm
@@ -626,6 +627,11 @@ def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     return None
 
 
+def _no_autograd(x: torch.Tensor) -> bool:
+    """No gradient is asked of ``x``, backward or forward mode (kernels without a derivative)."""
+    return not (torch.is_grad_enabled() and x.requires_grad) and forward_ad.unpack_dual(x).tangent is None
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if w.requires_grad and torch.is_grad_enabled():
         return _LinearFn.apply(x, w)
@@ -633,13 +639,19 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
         if y is not None:
             return y.view(*x.shape[:-1], w.shape[0])
+    if x.shape[-1] == w.shape[1] and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() > 1:
+        M = x.numel() // max(x.shape[-1], 1)
+        if gemm.rows_gain(M, *w.shape, True) and _no_autograd(x):
+            x2 = x.reshape(M, x.shape[-1])
+            if gemm.rows_ok(x2, w, True):
+                return native().gemm8_rows(x2, w, True, False).view(*x.shape[:-1], w.shape[0])
     return F.linear(x, w)
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
-    """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts as ONE launch, with
-    ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip or
-    stream_gemm.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
+    """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch, with
+    ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
+    stream_gemm.hip or gemm8.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
     if SKINNY_M <= 0 or x.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return None
@@ -651,9 +663,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
         return native().stream_linear(x, None, None, 0.0, w, scale, True)[0]
     if _stream_wins(x.shape[0], *w.shape) and _rows_ok(x, w):
         return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
-    if x.shape[0] > SKINNY_M or not _skinny_ok(x, w):
-        return None
-    return native().skinny_linear_swiglu(x, w)
+    if 0 < x.shape[0] <= SKINNY_M and _skinny_ok(x, w):
+        return native().skinny_linear_swiglu(x, w)
+    if gemm.rows_gain(x.shape[0], w.shape[0], w.shape[1], True, True) and gemm.rows_ok(x, w, True, True) and _no_autograd(x):
+        return native().gemm8_rows(x, w, True, True)  # a prompt pass
+    return None
 
 
 # rows up to which the RMSNorm runs in the prologue of skinny_gemm.hip (every workgroup recomputes the

@@ -110,6 +110,42 @@ def test_weight_grad_route(gpu, T, N, K):
     _check(weight_grad_(out, dy, x, beta=1.0), ref + base.float(), 5e-3)
 
 
+@pytest.mark.parametrize("M", [1, 255, 256, 257, 700])
+@pytest.mark.parametrize("N,K", [(256, 64), (512, 192), (768, 320)])
+def test_gemm8_rows(gpu, M, N, K):
+    """Any number of rows, in both orders of the weight and with SwiGLU; nothing is read or kept past the last row."""
+    from mxllm import ops
+
+    x = _mat(M, K, gpu, pad=8, seed=1)
+    for b_kc in (True, False):
+        w = _mat(N, K, gpu, pad=8, seed=2) if b_kc else _mat(K, N, gpu, pad=8, seed=2)
+        y = _ops().gemm8_rows(x, w, b_kc, False)
+        _check(y, x.float() @ (w.float().t() if b_kc else w.float()), 5e-3)
+        if b_kc:
+            assert torch.equal(_ops().gemm8_rows(x, w, True, True), ops.swiglu(y))  # the same roundings
+
+
+def test_rows_routes(gpu):
+    """The public entry points at a ragged prompt's size, against float32; a gradient keeps them off the kernel."""
+    from mxllm import ops
+    from mxllm.ops import gemm
+
+    M, N, K = 2560 + 3, 18432, 256
+    x, w = _mat(M, K, gpu, seed=1), _mat(N, K, gpu, seed=2)
+    assert gemm.rows_gain(M, N, K, True) and gemm.rows_gain(M, N, K, True, True)
+    ref = x.float() @ w.float().t()
+    with torch.no_grad():
+        y = ops.linear(x.view(1, M, K), w)
+        _check(y[0], ref, 5e-3)
+        assert torch.equal(ops.linear_swiglu(x, w), ops.swiglu(y[0]))
+        dy = _mat(M, N, gpu, seed=3)
+        _check(gemm.mm("nn", dy, _mat(N, 11 * 256, gpu, seed=4)), dy.float() @ _mat(N, 11 * 256, gpu, seed=4).float(), 5e-3)
+    xg = x.clone().requires_grad_()
+    ops.linear(xg, w).sum().backward()
+    _check(xg.grad, w.float().sum(0).expand(M, K), 5e-3)
+    assert ops.linear_swiglu(xg, w) is None
+
+
 @pytest.mark.parametrize("ph", ["8", "4"])
 def test_gemm8_odd_ktiles_nn(gpu, ph, monkeypatch):
     """the LoRA-augmented dX shape: K = N_out + 64 (an odd number of 64-deep K-tiles)."""
