@@ -179,7 +179,8 @@ bool gemm8_sq(const at::Tensor& a, bool a_kc, const at::Tensor& b, bool b_kc, at
 
 // a op(b) (bf16) for any number of rows: a [M, K], b [N, K] when b_kc else [K, N] -> [M, N]; swiglu: b = [gate; up]
 // -> silu(gate) up [M, N / 2] (mx_gemm8_rows; callers ask mxllm/ops/gemm.py rows_ok first).
-at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool swiglu) {
+// parts > 1: K in that many parts (mx_gemm8_parts).
+at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool swiglu, int64_t parts) {
   MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm8_rows: GPU tensors of one device");
   MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm8_rows: bf16 operands");
   MX_CHECK(a.dim() == 2 && b.dim() == 2, "gemm8_rows: 2-D operands");
@@ -189,8 +190,16 @@ at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool 
            "gemm8_rows: row-major operands");
   DevGuard g(a.device());
   auto out = at::empty({M, swiglu ? N / 2 : N}, a.options());
-  const int rc = mx_gemm8_rows(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M,
-                               (int)N, (int)K, swiglu ? 1 : 0, cur_stream());
+  int rc;
+  if (parts > 1) {
+    MX_CHECK(parts <= K / 64, "gemm8_rows: parts of at least 64 of K");
+    auto ws = at::empty({parts * M * N}, a.options().dtype(at::kFloat));
+    rc = mx_gemm8_parts(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
+                        (int)K, swiglu ? 1 : 0, (int)parts, ws.data_ptr<float>(), cur_stream());
+  } else {
+    rc = mx_gemm8_rows(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
+                       (int)K, swiglu ? 1 : 0, cur_stream());
+  }
   MX_CHECK(rc != -1, "gemm8_rows: shape, stride or alignment not taken");
   MX_OK(rc);
   return out;
@@ -981,7 +990,7 @@ TORCH_LIBRARY(mxllm, m) {
   m.def("segmented_mean(Tensor codes, Tensor offsets) -> Tensor");
   m.def("copy2d_batched(Tensor desc, int total_blocks) -> ()");
   m.def("transpose2d(Tensor x, Tensor? scale=None) -> Tensor");
-  m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu) -> Tensor");
+  m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
   m.def("gemm8(Tensor a, bool a_kc, Tensor b, bool b_kc, Tensor(a!) out, float beta, Tensor? alpha_t=None, float alpha=1.0, int ph=8) -> bool");
   m.def("prefetch(Tensor t, int wgs) -> ()");
   m.def("cu_masked_stream(int device, int[] mask) -> int", &cu_masked_stream);  // no tensor args: catch-all

@@ -60,6 +60,8 @@ int mx_gemm8_epi(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                  int N, int K, int mode, MxG8Epi ep, hipStream_t stream);
 int mx_gemm8_rows(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, int b_kc, uint16_t* C, int64_t ldc,
                   int M, int N, int K, int swiglu, hipStream_t stream);
+int mx_gemm8_parts(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, int b_kc, uint16_t* C, int64_t ldc,
+                   int M, int N, int K, int swiglu, int S, float* ws, hipStream_t stream);
 int mx_gemm8_sq(const uint16_t* A, int64_t lda, int a_kc, const uint16_t* B, int64_t ldb, int b_kc, uint16_t* C,
                 int64_t ldc, int M, int N, int K, const float* alpha_t, float alpha_f, float* sq, hipStream_t stream);
 int mx_gemm8_tail(const uint16_t* A, int64_t lda, int a_kc, const uint16_t* B, int64_t ldb, int b_kc, uint16_t* C,

@@ -92,10 +92,11 @@ __device__ __forceinline__ int g8_map_a(int r, int h) { return (r >> 6) * 128 + 
 //  G8_EPI_ROWS / G8_EPI_ROWS_SWIGLU: any number of rows (A k-contiguous; the last tile's rows past M read as zeros
 //               through the descriptor's range and are not stored).  SWIGLU: only m = silu(g) u is stored, the
 //               projection itself never leaves the registers
+//  G8_EPI_PART  one of k0 parts of K, as fp32 into image `part` (cpart elements on) of C; any number of rows
 constexpr int G8_EPI_NONE = 0, G8_EPI_ROPE = 1, G8_EPI_SWIGLU = 2, G8_EPI_SWIGLU_BWD = 3, G8_EPI_MOE = 4,
-              G8_EPI_MOE_GLU = 5, G8_EPI_ROWS = 6, G8_EPI_ROWS_SWIGLU = 7;
+              G8_EPI_MOE_GLU = 5, G8_EPI_ROWS = 6, G8_EPI_ROWS_SWIGLU = 7, G8_EPI_PART = 8;
 constexpr bool g8_moe(int epi) { return epi == G8_EPI_MOE || epi == G8_EPI_MOE_GLU; }
-constexpr bool g8_rows(int epi) { return epi == G8_EPI_ROWS || epi == G8_EPI_ROWS_SWIGLU; }
+constexpr bool g8_rows(int epi) { return epi >= G8_EPI_ROWS && epi <= G8_EPI_PART; }
 constexpr bool g8_pairs(int epi) { return epi == G8_EPI_SWIGLU || epi == G8_EPI_ROWS_SWIGLU; }
 constexpr uint32_t G8_OOB = 0x80000000u;  // past every descriptor's range: reads as zeros
 
@@ -362,6 +363,19 @@ __device__ __forceinline__ void g8_epilogue_fused(f32x4 (&acc)[8][4], float alph
             *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(C) + m * ldc + 256 * pn + 64 * wc + 32 * jp + u8) = o;
         }
       }
+  } else if constexpr (EPI == G8_EPI_PART) {
+    const int n = 256 * pn + 64 * wc + 4 * (lane >> 4);
+#pragma unroll
+    for (int qa = 0; qa < 2; ++qa)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = ml + qa * 64 + 16 * i;
+        float* row = reinterpret_cast<float*>(C) + m * ldc + n;
+        if (m < M) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4*>(row + 32 * (j >> 1) + 16 * (j & 1)) = acc[4 * qa + i][j];
+        }
+      }
   } else if constexpr (EPI == G8_EPI_ROWS_SWIGLU) {
     const int col = 128 * pn + 32 * wc + u8;
 #pragma unroll
@@ -417,12 +431,12 @@ __global__ void __launch_bounds__(512, 1)
 gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb,
              void* __restrict__ C, int64_t ldc, int M, int N, int K, const float* __restrict__ alpha_t,
              float alpha_f, int k0 = 0, int64_t cpart = 0, G8Epi ep = G8Epi{}, G8Moe mo = G8Moe{}) {
-  static_assert(EPI == G8_EPI_NONE || (!OUT_F32 && !BETA && (EPI == G8_EPI_ROWS ? A_KC : EPI == G8_EPI_SWIGLU_BWD ? A_KC && !B_KC : A_KC && B_KC)),
+  static_assert(EPI == G8_EPI_NONE || EPI == G8_EPI_PART || (!OUT_F32 && !BETA && (EPI == G8_EPI_ROWS ? A_KC : EPI == G8_EPI_SWIGLU_BWD ? A_KC && !B_KC : A_KC && B_KC)),
                 "fused epilogues: bf16, beta 0; TN-form forwards, NN-form SwiGLU backward");
   // K split in two (gridDim.y == 2, k0 = K of part 0): part 1 covers K rows / columns k0 .. K-1 of
   // both operands and writes its own output image C + cpart (mx_gemm8_tail: the last, partial wave
   // of tiles of a GEMM runs as twice as many half-K workgroups; the images are summed after)
-  if (gridDim.y > 1) {
+  if (EPI != G8_EPI_PART && gridDim.y > 1) {
     const int kp = blockIdx.y;
     const int64_t koff = kp ? k0 : 0;
     A += A_KC ? koff : koff * lda;
@@ -444,7 +458,16 @@ gemm8_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __rest
       grid = nM * nN;
       if ((int)blockIdx.x >= grid) return;
     }
-    const int L = xcd_remap(blockIdx.x, grid);
+    int L = xcd_remap(blockIdx.x, grid);
+    if constexpr (EPI == G8_EPI_PART) {  // parts after each other: an XCD's tiles share the panels of one part of K
+      const int tiles = nM * nN, kp = L / tiles, nkt = (K + G8_BK - 1) / G8_BK;
+      const int t0 = nkt * kp / k0, t1 = nkt * (kp + 1) / k0;
+      L -= kp * tiles;
+      A += A_KC ? (int64_t)t0 * G8_BK : (int64_t)t0 * G8_BK * lda;
+      B += B_KC ? (int64_t)t0 * G8_BK : (int64_t)t0 * G8_BK * ldb;
+      C = reinterpret_cast<float*>(C) + kp * cpart;
+      K = (kp + 1 == k0 ? K : t1 * G8_BK) - t0 * G8_BK;
+    }
     constexpr int GM = 8;
     const int per = GM * nN, grp = L / per, first = grp * GM;
     const int rows = min(GM, nM - first), in = L - grp * per;

@@ -163,23 +163,34 @@ def rows_ok(a: torch.Tensor, b: torch.Tensor, b_kc: bool, swiglu: bool = False) 
                 and 256 * a.stride(0) < 1 << 30 and (N if swiglu else 256 if b_kc else K) * ldb < 1 << 30)
 
 
-def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> bool:
-    """Whether the rows kernel is the faster one; the library is tuned for round numbers of rows, and falls behind
-    between them (us, library -> gemm8; H x N at rows):
+def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
+    """Parts of K (1: whole) in which the rows kernel is the faster one, else 0.
+
+    In parts where the tiles leave half the CUs without one and K is long; each part costs its fp32 image's trip (us,
+    library -> gemm8; K x N at rows):
+      * projections (``b_kc``): K of 12,288 and 64 rows on.  14336 x 4096 at 64 35 -> 31, 128 59 -> 36, 400 80 -> 57,
+        1000 122 -> 97, 2048 191 -> 171; 28672 x 8192 at 200 312 -> 122 (14336 x 4096 at 48 28 -> 30; 8192 x 2048 at
+        512 29 -> 37, 2048 69 -> 67);
+      * input gradients: K of 6144 on.  16384 x 2048 at 1000 124 -> 68, 4096 237 -> 211; 6144 x 4096 at 512 53 -> 43
+        (3072 x 2048 at 512 26 -> 30).
+    Whole, where the library, which is tuned for round numbers of rows, falls behind between them:
       * projections (``b_kc``) from 700 tiles on: 4096 x 28672 at 2600 542 -> 450, 3606 612 -> 617, 5000 904 -> 820;
         8192 x 57344 at 700 559 -> 530 (4096 x 28672 at 1025, 560 tiles: 235 -> 241; 14336 x 4096 at 2600, 176: 237 -> 243);
       * input gradients: :func:`_gains_nn`;
       * gate-up with SwiGLU, which saves the projection's trip through HBM at any size: where the last tile's rows are
-        not mostly padding and half the CUs have a tile.  2048 x 16384 at 700 57 -> 46, 2600 205 -> 142, 4096 236 -> 198;
-        4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 1025 249 -> 241, 4096 706 -> 640."""
+        not mostly padding and five eighths of the CUs have a tile.  2048 x 16384 at 700 48 -> 42, 2600 205 -> 142, 4096
+        236 -> 198 (512, 128 tiles: 38 -> 40); 4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 1025 249 -> 241, 4096
+        706 -> 640."""
     if _policy() == "0":
-        return False
+        return 0
     tiles = -(-M // 256) * (N // 256)
+    if 0 < tiles <= CUS // 2 and not swiglu and (M >= 64 and K >= 12288 if b_kc else K >= 6144):
+        return min(CUS // tiles, 16)
     if swiglu:
-        return tiles >= CUS // 2 and 4 * M >= 3 * (-(-M // 256) * 256)
+        return int(tiles >= CUS * 5 // 8 and 4 * M >= 3 * (-(-M // 256) * 256))
     if M % 256 == 0:
-        return False
-    return tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles)
+        return 0
+    return int(tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles))
 
 
 DEFAULT_PH = int(os.environ.get("MXLLM_GEMM8_DEFAULT_PH", "4"))
@@ -210,9 +221,10 @@ def mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = N
     ``alpha_t``: optional 1-element f32 device scalar (no host sync)."""
     M, N, K = _dims(form, a, b)
     odt = out.dtype if out is not None else (out_dtype or a.dtype)
-    if (out is None and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16
-            and rows_gain(M, N, K, form == "tn") and rows_ok(a, b, form == "tn")):
-        return native().gemm8_rows(a, b, form == "tn", False)
+    if out is None and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16:
+        parts = rows_gain(M, N, K, form == "tn")
+        if parts and rows_ok(a, b, form == "tn"):
+            return native().gemm8_rows(a, b, form == "tn", False, parts)
     if out is None:
         out = torch.empty(M, N, dtype=odt, device=a.device)
         beta = 0.0

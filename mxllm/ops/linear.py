@@ -641,10 +641,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             return y.view(*x.shape[:-1], w.shape[0])
     if x.shape[-1] == w.shape[1] and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() > 1:
         M = x.numel() // max(x.shape[-1], 1)
-        if gemm.rows_gain(M, *w.shape, True) and _no_autograd(x):
+        parts = gemm.rows_gain(M, *w.shape, True)
+        if parts and _no_autograd(x):
             x2 = x.reshape(M, x.shape[-1])
             if gemm.rows_ok(x2, w, True):
-                return native().gemm8_rows(x2, w, True, False).view(*x.shape[:-1], w.shape[0])
+                return native().gemm8_rows(x2, w, True, False, parts).view(*x.shape[:-1], w.shape[0])
     return F.linear(x, w)
 
 
@@ -665,8 +666,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
         return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
     if 0 < x.shape[0] <= SKINNY_M and _skinny_ok(x, w):
         return native().skinny_linear_swiglu(x, w)
-    if gemm.rows_gain(x.shape[0], w.shape[0], w.shape[1], True, True) and gemm.rows_ok(x, w, True, True) and _no_autograd(x):
-        return native().gemm8_rows(x, w, True, True)  # a prompt pass
+    parts = gemm.rows_gain(x.shape[0], *w.shape, True, True)  # a prompt pass
+    if parts and gemm.rows_ok(x, w, True, True) and _no_autograd(x):
+        return native().gemm8_rows(x, w, True, True, parts)
     return None
 
 

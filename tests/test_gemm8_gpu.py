@@ -111,7 +111,7 @@ def test_weight_grad_route(gpu, T, N, K):
 
 
 @pytest.mark.parametrize("M", [1, 255, 256, 257, 700])
-@pytest.mark.parametrize("N,K", [(256, 64), (512, 192), (768, 320)])
+@pytest.mark.parametrize("N,K", [(256, 64), (512, 192), (768, 320), (256, 1088)])
 def test_gemm8_rows(gpu, M, N, K):
     """Any number of rows, in both orders of the weight and with SwiGLU; nothing is read or kept past the last row."""
     from mxllm import ops
@@ -123,27 +123,38 @@ def test_gemm8_rows(gpu, M, N, K):
         _check(y, x.float() @ (w.float().t() if b_kc else w.float()), 5e-3)
         if b_kc:
             assert torch.equal(_ops().gemm8_rows(x, w, True, True), ops.swiglu(y))  # the same roundings
+        for parts in range(2, min(K // 64, 16) + 1, 2):
+            yp = _ops().gemm8_rows(x, w, b_kc, False, parts)
+            _check(yp, x.float() @ (w.float().t() if b_kc else w.float()), 5e-3)
+            if b_kc:
+                assert torch.equal(_ops().gemm8_rows(x, w, True, True, parts), ops.swiglu(yp))
 
 
-def test_rows_routes(gpu):
-    """The public entry points at a ragged prompt's size, against float32; a gradient keeps them off the kernel."""
+@pytest.mark.parametrize("M,N,K,form", [(2563, 18432, 256, "tn"), (64, 256, 12288, "tn"), (300, 512, 12288, "tn"),
+                                        (1000, 10240, 512, "swiglu"), (2563, 18432, 256, "swiglu"), (2563, 4096, 256, "nn"),
+                                        (512, 512, 6144, "nn")])
+def test_rows_routes(gpu, M, N, K, form):
+    """The entry points at sizes that the rule gives to the rows kernel, whole and in parts, against float32; where a
+    gradient is asked for the result has one."""
     from mxllm import ops
     from mxllm.ops import gemm
 
-    M, N, K = 2560 + 3, 18432, 256
-    x, w = _mat(M, K, gpu, seed=1), _mat(N, K, gpu, seed=2)
-    assert gemm.rows_gain(M, N, K, True) and gemm.rows_gain(M, N, K, True, True)
-    ref = x.float() @ w.float().t()
-    with torch.no_grad():
-        y = ops.linear(x.view(1, M, K), w)
-        _check(y[0], ref, 5e-3)
-        assert torch.equal(ops.linear_swiglu(x, w), ops.swiglu(y[0]))
-        dy = _mat(M, N, gpu, seed=3)
-        _check(gemm.mm("nn", dy, _mat(N, 11 * 256, gpu, seed=4)), dy.float() @ _mat(N, 11 * 256, gpu, seed=4).float(), 5e-3)
+    assert gemm.rows_gain(M, N, K, form != "nn", form == "swiglu")
+    x = _mat(M, K, gpu, seed=1)
+    w = _mat(K, N, gpu, seed=2) if form == "nn" else _mat(N, K, gpu, seed=2)
+    ref = x.float() @ (w.float() if form == "nn" else w.float().t())
     xg = x.clone().requires_grad_()
-    ops.linear(xg, w).sum().backward()
-    _check(xg.grad, w.float().sum(0).expand(M, K), 5e-3)
-    assert ops.linear_swiglu(xg, w) is None
+    if form == "nn":
+        _check(gemm.mm("nn", x, w), ref, 5e-3)
+    elif form == "tn":
+        _check(ops.linear(x.view(1, M, K), w)[0], ref, 5e-3)
+        ops.linear(xg, w).sum().backward()
+        _check(xg.grad, w.float().sum(0).expand(M, K), 5e-3)
+    else:
+        g, u = ref.to(torch.bfloat16).float().chunk(2, 1)
+        # g and u rounded to bf16 may differ by an ulp (2^-8) each from a sum in another order
+        _check(ops.linear_swiglu(x, w), torch.nn.functional.silu(g) * u, 1e-2)
+        assert ops.linear_swiglu(xg, w) is None
 
 
 @pytest.mark.parametrize("ph", ["8", "4"])
