@@ -40,11 +40,13 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> rmsnorm_fwd(const at::Tensor& x,
 }
 
 // returns (dx, dw_f32 or empty).  dres may be a row-strided [T, H] view;
-// out_pad > 0: dx is the left part of a [T, H + out_pad] buffer.
+// out_pad > 0: dx is the left part of a [T, H + out_pad] buffer.  dw_into (contiguous [H], bf16 or f32): the sum goes
+// there, over what it held or (dw_add) onto it, and the second result is empty.
 std::tuple<at::Tensor, at::Tensor> rmsnorm_bwd(const at::Tensor& dy, const at::Tensor& x,
                                                const at::Tensor& w, const at::Tensor& rstd,
                                                const c10::optional<at::Tensor>& dres, bool need_dw,
-                                               int64_t out_pad) {
+                                               int64_t out_pad, const c10::optional<at::Tensor>& dw_into,
+                                               bool dw_add) {
   check_bf16(dy, "dy");
   check_bf16(x, "x");
   check_bf16(w, "w");
@@ -76,17 +78,27 @@ std::tuple<at::Tensor, at::Tensor> rmsnorm_bwd(const at::Tensor& dy, const at::T
   float* dwpp = nullptr;
   if (need_dw) {
     dwp = at::empty({nblk, H}, x.options().dtype(at::kFloat));
-    dw = at::empty({H}, x.options().dtype(at::kFloat));
+    if (dw_into.has_value()) {
+      dw = *dw_into;
+      MX_CHECK(dw.device() == x.device() && dw.is_contiguous() && dw.numel() == H &&
+                   (dw.scalar_type() == at::kFloat || dw.scalar_type() == at::kBFloat16),
+               "dw_into: contiguous [H], bf16 or f32, on the device");
+    } else {
+      dw = at::empty({H}, x.options().dtype(at::kFloat));
+      dw_add = false;
+    }
     dwpp = dwp.data_ptr<float>();
   }
   if (T > 0) {
     MX_OK(mx_rmsnorm_bwd(bf(dy), bf(x), bf(w), rstd.data_ptr<float>(), drp, bfm(dx), dwpp, (int)T, (int)H,
                          (int)ldr, (int)(H + out_pad), rpb, cur_stream()));
-    if (need_dw) MX_OK(mx_colsum_f32(dwpp, dw.data_ptr<float>(), (int)nblk, (int)H, cur_stream()));
-  } else if (need_dw) {
+    if (need_dw)
+      MX_OK(mx_colsum(dwpp, dw.data_ptr(), dw.scalar_type() == at::kFloat ? 1 : 0, (int)nblk, (int)H, dw_add ? 1 : 0,
+                      cur_stream()));
+  } else if (need_dw && !dw_add) {
     dw.zero_();
   }
-  return {dx, need_dw ? dw : at::Tensor()};
+  return {dx, need_dw && !dw_into.has_value() ? dw : at::Tensor()};
 }
 
 // ---------------------------------------------------------------- misc
@@ -986,7 +998,7 @@ void lora_grads(const at::Tensor& x, const at::Tensor& dy, const at::Tensor& g, 
 
 TORCH_LIBRARY(mxllm, m) {
   m.def("rmsnorm_fwd(Tensor x, Tensor? res, Tensor w, float eps, int out_pad=0) -> (Tensor, Tensor, Tensor)");
-  m.def("rmsnorm_bwd(Tensor dy, Tensor x, Tensor w, Tensor rstd, Tensor? dres, bool need_dw, int out_pad=0) -> (Tensor, Tensor)");
+  m.def("rmsnorm_bwd(Tensor dy, Tensor x, Tensor w, Tensor rstd, Tensor? dres, bool need_dw, int out_pad=0, Tensor(a!)? dw_into=None, bool dw_add=False) -> (Tensor, Tensor)");
   m.def("segmented_mean(Tensor codes, Tensor offsets) -> Tensor");
   m.def("copy2d_batched(Tensor desc, int total_blocks) -> ()");
   m.def("transpose2d(Tensor x, Tensor? scale=None) -> Tensor");

@@ -15,7 +15,7 @@ int mx_rmsnorm_fwd(const uint16_t* x, const uint16_t* res, const uint16_t* w, ui
 int mx_rmsnorm_bwd(const uint16_t* dy, const uint16_t* x, const uint16_t* w, const float* rstd,
                    const uint16_t* dres, uint16_t* dx, float* dwp, int T, int H, int ldr, int ldx, int rpb,
                    hipStream_t stream);
-int mx_colsum_f32(const float* p, float* out, int nblk, int H, hipStream_t stream);
+int mx_colsum(const float* p, void* out, int out_f32, int nblk, int H, int add, hipStream_t stream);
 
 // misc.hip
 int mx_segmented_mean_i32(const int32_t* codes, const int64_t* offs, float* out, int nseg,

@@ -158,24 +158,39 @@ __global__ void __launch_bounds__(256) rmsnorm_bwd_kernel(
   }
 }
 
-// Sum partials [nblk, H] over nblk -> out[H] f32.  Block = 64 column-lanes x 4
-// row-slices, each lane owning 4 consecutive columns (16-B loads); the 4 slices
-// are combined through LDS.  Deterministic (fixed order, no atomics).
-__global__ void __launch_bounds__(256) colsum_kernel(const float* __restrict__ p, float* __restrict__ out,
-                                                     int nblk, int H) {
-  __shared__ f32x4 red[4][64];
-  const int cl = threadIdx.x & 63, sl = threadIdx.x >> 6;
-  const int c = (blockIdx.x * 64 + cl) * 4;
+// Sum partials [nblk, H] over nblk -> out[H], f32 or bf16, added to what it held (`add`, in f32, rounded once) or
+// over it: a gradient's own slot, so that no second kernel adds the sum there.  Block = 8 column-lanes of 4
+// consecutive columns x 32 row-slices, combined through LDS in a fixed order.  Bound by latency: 512 partials of 2048,
+// 64 workgroups 5.0 us (4 slices, 8 workgroups: 9.5 us, and 47 us for the elementwise sum into the slot).
+template <typename O>
+__global__ void __launch_bounds__(256) colsum_kernel(const float* __restrict__ p, O* __restrict__ out,
+                                                     int nblk, int H, int add) {
+  __shared__ f32x4 red[32][8];
+  const int cl = threadIdx.x & 7, sl = threadIdx.x >> 3;
+  const int c = (blockIdx.x * 8 + cl) * 4;
   f32x4 s = {0.f, 0.f, 0.f, 0.f};
   if (c < H) {
 #pragma unroll 8
-    for (int b = sl; b < nblk; b += 4) s += *reinterpret_cast<const f32x4*>(p + (size_t)b * H + c);
+    for (int b = sl; b < nblk; b += 32) s += *reinterpret_cast<const f32x4*>(p + (size_t)b * H + c);
   }
   red[sl][cl] = s;
   __syncthreads();
   if (sl == 0 && c < H) {
-    f32x4 t = red[0][cl] + red[1][cl] + red[2][cl] + red[3][cl];
-    *reinterpret_cast<f32x4*>(out + c) = t;
+    f32x4 t = red[0][cl];
+#pragma unroll
+    for (int i = 1; i < 32; ++i) t += red[i][cl];
+    if constexpr (sizeof(O) == 4) {
+      f32x4* o = reinterpret_cast<f32x4*>(out + c);
+      *o = add ? *o + t : t;
+    } else {
+      uint2* o = reinterpret_cast<uint2*>(out + c);
+      if (add) {
+        const uint2 v = *o;
+        t += f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                   __uint_as_float(v.y & 0xffff0000u)};
+      }
+      *o = uint2{pack_bf16x2(t[0], t[1]), pack_bf16x2(t[2], t[3])};
+    }
   }
 }
 
@@ -231,8 +246,13 @@ extern "C" int mx_rmsnorm_bwd(const uint16_t* dy, const uint16_t* x, const uint1
   return (int)hipGetLastError();
 }
 
-extern "C" int mx_colsum_f32(const float* p, float* out, int nblk, int H, hipStream_t stream) {
-  if (H % 4 != 0) return -1;
-  colsum_kernel<<<(H / 4 + 63) / 64, 256, 0, stream>>>(p, out, nblk, H);
+// out: H elements, 16-B aligned (f32) or 8-B aligned (bf16)
+extern "C" int mx_colsum(const float* p, void* out, int out_f32, int nblk, int H, int add, hipStream_t stream) {
+  if (H % 4 != 0 || ((uintptr_t)out & (out_f32 ? 15 : 7))) return -1;
+  const int grid = (H / 4 + 7) / 8;
+  if (out_f32)
+    colsum_kernel<<<grid, 256, 0, stream>>>(p, reinterpret_cast<float*>(out), nblk, H, add);
+  else
+    colsum_kernel<<<grid, 256, 0, stream>>>(p, reinterpret_cast<uint16_t*>(out), nblk, H, add);
   return (int)hipGetLastError();
 }

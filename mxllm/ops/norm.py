@@ -10,7 +10,7 @@ from __future__ import annotations
 import torch
 
 from . import reference as ref
-from ..parallel.grad_ready import accum_grad
+from ..parallel.grad_ready import accum_grad, grad_slot, slot_written
 from ._ext import native, rows_view, use_native
 
 # ``out_pad`` / ``grad_pad``: the normalised output (forward) or the input
@@ -30,19 +30,25 @@ class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, w, rstd = ctx.saved_tensors
-        dx, dw = native().rmsnorm_bwd(dy.contiguous(), x, w, rstd, None, ctx.needs_input_grad[1])
-        return dx, _wgrad(ctx, dw, w, 1), None, None
+        dx, dw = _backward(ctx, dy, x, w, rstd, None, 1)
+        return dx, dw, None, None
 
 
-def _wgrad(ctx, dw, w, idx: int):
-    """dγ (fp32 from the kernel; ``idx``: w's input position): added straight into
-    an fp32 gradient target when the owner keeps one (no bf16 rounding), else
-    handed to autograd as w.dtype."""
-    if dw is None or not ctx.needs_input_grad[idx]:
-        return None
-    if accum_grad(ctx.wp, dw):
-        return None
-    return dw.to(w.dtype)
+def _backward(ctx, dy, h, w, rstd, dres, idx: int, grad_pad: int = 0):
+    """(dx, dγ for autograd).  dγ (``idx``: w's input position) goes straight into the owner's gradient slot where
+    there is one — fp32 sums, rounded once to the slot's type — else to autograd as w.dtype."""
+    need = ctx.needs_input_grad[idx]
+    wp = ctx.wp
+    slot = grad_slot(wp) if need else None
+    if slot is not None and slot.dtype in (torch.float32, torch.bfloat16) and slot.device == h.device:
+        dx, _ = native().rmsnorm_bwd(dy.contiguous(), h, w, rstd, dres, True, grad_pad, slot,
+                                     not getattr(wp, "_mx_grad_fresh", False))
+        slot_written(wp)
+        return dx, None
+    dx, dw = native().rmsnorm_bwd(dy.contiguous(), h, w, rstd, dres, need, grad_pad)
+    if not need or accum_grad(wp, dw):
+        return dx, None
+    return dx, dw.to(w.dtype)
 
 
 class _AddRMSNormFn(torch.autograd.Function):
@@ -62,8 +68,8 @@ class _AddRMSNormFn(torch.autograd.Function):
         if dy is None:
             dy = torch.zeros_like(h)
         dres = rows_view(dh) if dh is not None else None
-        dx, dw = native().rmsnorm_bwd(dy.contiguous(), h, w, rstd, dres, ctx.needs_input_grad[2], ctx.grad_pad)
-        return dx, dx, _wgrad(ctx, dw, w, 2), None, None, None
+        dx, dw = _backward(ctx, dy, h, w, rstd, dres, 2, ctx.grad_pad)
+        return dx, dx, dw, None, None, None
 
 
 def rms_norm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-5, out_pad: int = 0) -> torch.Tensor:

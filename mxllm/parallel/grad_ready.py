@@ -33,6 +33,24 @@ def direct_grad32(p):
     return getattr(p, "_mx_grad32", None)
 
 
+def grad_slot(p):
+    """``p``'s owner-attached gradient target as a kernel may write it whole (dense, aligned for vector
+    stores), or None.  The caller adds to it, or overwrites it where ``_mx_grad_fresh`` is set, and then calls
+    :func:`slot_written`."""
+    if p is None:
+        return None
+    t = direct_grad32(p)
+    if t is None:
+        t = direct_grad(p)
+    return t if t is not None and t.is_contiguous() and t.data_ptr() % 16 == 0 else None
+
+
+def slot_written(p) -> None:
+    if getattr(p, "_mx_grad_fresh", False):
+        p._mx_grad_fresh = False
+    mark_ready(p)
+
+
 def accum_grad(p, g) -> bool:
     """Add a computed gradient ``g`` (any float dtype, e.g. the fp32 partials of the
     RMSNorm dγ / embedding kernels) into ``p``'s owner-attached target — the fp32

@@ -41,6 +41,23 @@ def test_rmsnorm_fwd_bwd(gpu, T, H):
     assert rel_err(dw, wf.grad) < 1e-3
 
 
+@pytest.mark.parametrize("T,H", [(1, 8), (33, 1000), (700, 2048), (20000, 72)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rmsnorm_backward_into_slot(gpu, T, H, dtype):
+    """The weight's gradient over or onto what an owner's slot held, rounded once."""
+    x, dy = torch.randn(2, T, H, device=gpu).to(torch.bfloat16)
+    w = torch.ones(H, device=gpu, dtype=torch.bfloat16)
+    _, rstd, _ = _ops().rmsnorm_fwd(x, None, w, 1e-5)
+    dx, dw = _ops().rmsnorm_bwd(dy, x, w, rstd, None, True)
+    old = torch.randn(H, device=gpu).to(dtype)
+    for add in (False, True):
+        buf = torch.cat([old, old.new_full((8,), 3.0)])
+        slot = buf[:H]
+        dx2, none = _ops().rmsnorm_bwd(dy, x, w, rstd, None, True, 0, slot, add)
+        assert none is None and torch.equal(dx, dx2) and (buf[H:] == 3.0).all()
+        assert torch.equal(slot, (old.float() + dw if add else dw).to(dtype))  # the same sum, one rounding
+
+
 def test_add_rmsnorm(gpu):
     torch.manual_seed(1)
     x = torch.randn(300, 1024, device=gpu, dtype=torch.bfloat16)
