@@ -390,3 +390,26 @@ def test_fused_grad_norm_matches_full_pass(gpu, monkeypatch):
     assert torch.equal(g1, g0)  # the fused dW GEMMs store the same gradient bits
     for k in m0:
         assert torch.allclose(m1[k].float(), m0[k].float(), rtol=0, atol=1e-6), k
+
+
+@pytest.mark.parametrize("gdt,accum", [(None, 1), (None, 2), (torch.float32, 1)])
+def test_tied_fresh_gradients_bitwise(gpu, gdt, accum, monkeypatch):
+    """Tied embeddings, whose gradient autograd sums: slots that hold an earlier step's gradient give the weights of
+    slots that the optimizer clears."""
+    monkeypatch.setenv("MXLLM_FUSED_GRAD_NORM", "0")  # the norm summed in one order on both sides
+    cfg = _cfg().replace(tie_embeddings=True)
+    g = torch.Generator(device=gpu).manual_seed(1)
+    batches = [torch.randint(0, cfg.vocab_size, (2, 256), device=gpu, generator=g) for _ in range(3 * accum)]
+    out = {}
+    for fresh in ("0", "1"):
+        monkeypatch.setenv("MXLLM_FRESH_GRADS", fresh)
+        tr = _ddp_trainer(gpu, cfg, 7, grad_dtype=gdt)
+        assert tr.fresh_grads == (fresh == "1")
+        for k in range(3):
+            if tr.fresh_grads:
+                for s in tr.flat.slots:
+                    tr.flat.grads[s.offset:s.offset + s.numel].fill_(7.0)
+            tr.train_step([(b, b) for b in batches[k * accum:(k + 1) * accum]])
+        out[fresh] = _masters(tr)
+    for n, w in out["0"].items():
+        assert torch.equal(w, out["1"][n]), n
