@@ -102,6 +102,93 @@ __device__ __forceinline__ void dfuse_norm_rows(const uint16_t* __restrict__ X, 
   __syncthreads();
 }
 
+// LDS traffic of this wave done, then the workgroup's barrier: loads from memory stay in flight (__syncthreads waits
+// for them)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The same for a caller that stays (stream_gemm.hip), at 40 registers more.
+// What it reads of the first 4096 columns is asked for before `ahead`, the caller's first weight loads: loads return
+// in order, so that the norm would wait for weights asked for before it, and those after it for the norm.
+template <typename Ahead>
+__device__ __forceinline__ void dfuse_norm_ahead(const uint16_t* __restrict__ X, int64_t ldx, int M, int K,
+                                                 const SkNorm& na, uint16_t* xs, int lds, float (*nscr)[4],
+                                                 const Ahead& ahead) {
+  constexpr int NP = 2;  // 2048-column chunks held in registers
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int q = w >> 2, tq = tid & 255;
+  u16x8 hb[2][NP] = {}, dv[2][NP] = {}, gw[NP] = {};
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int cc = tq * 8 + 2048 * i;
+    if (cc >= K) continue;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int m = 2 * p + q;
+      if (m >= M) continue;
+      hb[p][i] = *reinterpret_cast<const u16x8*>(X + (int64_t)m * ldx + cc);
+      if (na.delta) dv[p][i] = *reinterpret_cast<const u16x8*>(na.delta + (int64_t)m * na.ldd + cc);
+    }
+    gw[i] = *reinterpret_cast<const u16x8*>(na.gamma + cc);
+  }
+  ahead();
+  auto residual = [&](u16x8& h, const u16x8& d, int m, int cc, float& ss) {
+    if (na.delta) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) h[j] = f2bf(bf2f(d[j]) + bf2f(h[j]));
+      if (blockIdx.x == 0) *reinterpret_cast<u16x8*>(na.h_out + (int64_t)m * K + cc) = h;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = bf2f(h[j]);
+      ss += v * v;
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int m = 2 * p + q;
+    float ss = 0.f;
+    if (m < M) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i)
+        if (tq * 8 + 2048 * i < K) residual(hb[p][i], dv[p][i], m, tq * 8 + 2048 * i, ss);
+      for (int cc = tq * 8 + 2048 * NP; cc < K; cc += 2048) {
+        u16x8 h = *reinterpret_cast<const u16x8*>(X + (int64_t)m * ldx + cc), d = {};
+        if (na.delta) d = *reinterpret_cast<const u16x8*>(na.delta + (int64_t)m * na.ldd + cc);
+        residual(h, d, m, cc, ss);
+        *reinterpret_cast<u16x8*>(xs + (int64_t)m * lds + cc) = h;
+      }
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) nscr[m][w & 3] = ss;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int m = 2 * p + q;
+    if (m >= M) continue;
+    float r = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r += nscr[m][i];
+    const float rs = rsqrtf(r / (float)K + na.eps);
+    auto normed = [&](const u16x8& h, const u16x8& g) {
+      u16x8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = f2bf(bf2f(h[j]) * rs * bf2f(g[j]));
+      return o;
+    };
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int cc = tq * 8 + 2048 * i;
+      if (cc < K) *reinterpret_cast<u16x8*>(xs + (int64_t)m * lds + cc) = normed(hb[p][i], gw[i]);
+    }
+    for (int cc = tq * 8 + 2048 * NP; cc < K; cc += 2048) {  // each thread the chunks it stored
+      u16x8* px = reinterpret_cast<u16x8*>(xs + (int64_t)m * lds + cc);
+      *px = normed(*px, *reinterpret_cast<const u16x8*>(na.gamma + cc));
+    }
+  }
+  lds_barrier();
+}
+
 // Split-K decode attention partials (decode.hip decode_attn_*: per (row, q-head, split) the
 // running max / sum in part_ml [M, Hq, nsplit, 2] and the unnormalised output in part_o
 // [M, Hq, nsplit, 128]) merged into the attention output rows xs [M, Hq * 128] (LDS) -- the

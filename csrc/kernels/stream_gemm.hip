@@ -8,17 +8,20 @@
 // is in flight while the last one is multiplied and summed.
 //  * 8 waves split K in eight contiguous parts, 64-k chunks of two v_mfma_f32_16x16x32_bf16 with the weights as
 //    the A operand, partial sums in wave order: the products and sums of the kernels above, bit for bit;
+//  * X is asked for in front of the first weights and worked on behind them: loads return in order, and __syncthreads
+//    waits for all of them (with the weights in front and that barrier, 6144 x 4096 at 16 rows 17.6 us in a step, now
+//    14.8; the e4m3 gate-up projection of 4 rows with its norm 26.5, now 23.6);
 //  * blocks of U chunks, two in flight: 8 (K a multiple of 4096) or 4 (of 2048): 128 or 64 registers, so that
 //    with up to 80 KB of LDS two workgroups share a CU;
 //  * LDS rows are K + 8 long: the 16 rows that a fragment read touches start 4 banks apart;
 //  * the waves take turns at a group's sum and epilogue (two LDS images, one barrier a group), the others go on;
 //  * epilogues: plain, SwiGLU (8 gate and the matching 8 up channels), RoPE + cache append (heads of 64 or 128);
 //    prologue: the RMSNorm with the residual add, up to 4 rows (decode_fuse.h).
-// 28672 x 4096 (235 MB), rows 1 / 4 / 8 / 16: 42.1 / 43.6 / 45.1 / 48.2 us (5.6 - 4.9 TB/s) against skinny_gemm's 44.7 /
-// 48.0 / 56.0 / 67.1 and hipBLASLt's 60 - 67; in a step of 16 rows, SwiGLU included, 44.4 against 59.7 + 5.2.  The same
-// in e4m3, rows 1 / 4 / 8: 24.9 / 25.8 / 28.6 against fp8_gemm's 28.4 / 32.2 / 36.4.  128256 x 2048, 8 rows: 97 against
-// 108 and 115.  Projections of one group a CU or less gain nothing (4096 x 4096, 16 rows: 13.4 against 11.2).
-// Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 17 us for 50 MB).
+// 28672 x 4096 (235 MB) with SwiGLU, rows 1 / 4 / 8 / 16: 42.6 / 42.9 / 43.3 / 43.8 us (5.5 TB/s) against skinny_gemm's
+// 43.6 / 47.3 / 54.9 / 67.1 and hipBLASLt's 67; in e4m3, rows 1 / 4 / 8: 24.9 / 25.8 / 28.6 against fp8_gemm's 28.4 / 32.2
+// / 36.4.  128256 x 2048, 8 rows: 98 against 109 and 114.
+// Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 14.8 us for 50 MB; the last 128 as
+// 256 halves: no change, a half's loads take a whole one's turns).
 #include <algorithm>
 
 #include "decode_fuse.h"
@@ -67,11 +70,8 @@ struct WFrag<true, U> {
   }
 };
 
-// LDS traffic of this wave done, then the workgroup's barrier: weight loads stay in flight
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <bool F8, int MB, int EPI, bool NORM, int U>
-__global__ void __launch_bounds__(512) stream_gemm_kernel(StreamArgs a) {
+__global__ void __launch_bounds__(512, MB == 1 && (F8 || U == 4) ? 4 : 2) stream_gemm_kernel(StreamArgs a) {
   constexpr int NW = kSkWaves, NRED = MB == 1 ? 2 : 1, WB = F8 ? 1 : 2;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -99,18 +99,37 @@ __global__ void __launch_bounds__(512) stream_gemm_kernel(StreamArgs a) {
     }
   };
   WFrag<F8, U> f0, f1;
-  load(f0);  // ahead of the prologue
+  // the first block goes out behind the reads of X, which return before it, and in front of the work on them
   if constexpr (NORM) {
-    __shared__ float nscr[2][4];
-    __shared__ float nrs[4];
-    dfuse_norm_rows(a.X, a.ldx, M, K, a.na, xs, ldx, nscr, nrs);
+    __shared__ float nscr[4][4];
+    dfuse_norm_ahead(a.X, a.ldx, M, K, a.na, xs, ldx, nscr, [&]() __attribute__((always_inline)) { load(f0); });
   } else {
-    const int per = K / 8;
-    for (int p = tid; p < M * per; p += 512) {
-      const int m = p / per, k = (p - m * per) * 8;
-      *reinterpret_cast<u16x8*>(xs + m * ldx + k) = *reinterpret_cast<const u16x8*>(a.X + (int64_t)m * a.ldx + k);
+    constexpr int XP = !F8 && U == 8 ? 16 : 8;  // 16-B pieces of X a thread holds: all, or the last ones
+    const int per = K / 8, total = M * per;
+    u16x8 v[XP];
+    auto fetch = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < XP; ++i) {
+        const int p = min(p0 + tid + 512 * i, total - 1), m = p / per;
+        v[i] = *reinterpret_cast<const u16x8*>(a.X + (int64_t)m * a.ldx + (p - m * per) * 8);
+      }
+    };
+    auto put = [&](int p0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < XP; ++i) {
+        const int p = p0 + tid + 512 * i, m = p / per;
+        if (p < total) *reinterpret_cast<u16x8*>(xs + m * ldx + (p - m * per) * 8) = v[i];
+      }
+    };
+    int p0 = 0;
+    for (; p0 + XP * 512 < total; p0 += XP * 512) {
+      fetch(p0);
+      put(p0);
     }
-    __syncthreads();
+    fetch(p0);
+    load(f0);
+    put(p0);
+    lds_barrier();
   }
   const uint16_t* xr[MB];
 #pragma unroll
@@ -170,19 +189,25 @@ __global__ void __launch_bounds__(512) stream_gemm_kernel(StreamArgs a) {
     cg += gridDim.x;
   };
   const int steps = (a.groups - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * nblk;
+  if (steps == 1) {
+    multiply(f0);
+    return;
+  }
+  load(f1);
   int s = 0;
-  for (; s + 2 < steps; s += 2) {
-    load(f1);
+  for (; s + 3 < steps; s += 2) {
     multiply(f0);
     load(f0);
     multiply(f1);
-  }
-  if (steps - s == 2) {
     load(f1);
-    multiply(f0);
+  }
+  multiply(f0);
+  if (steps - s == 3) {
+    load(f0);
     multiply(f1);
-  } else {
     multiply(f0);
+  } else {
+    multiply(f1);
   }
 }
 

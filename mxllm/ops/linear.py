@@ -584,13 +584,13 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
             and x2.stride(0) % 8 == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0 and use_native(x2))
 
 
-# Rows past which a projection of _STREAM_N and more channels goes to the workgroups that stay
-# (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of once 16 channels), by rows x width: the X that the
-# others read beside 16 channels of weights.  At 16,384 both are level (28672 x 4096, 4 rows: 48.0 -> 43.6 us;
-# 16384 x 2048, 4 rows 14.9 -> 15.9, 8 rows 16.9 -> 16.3; 28672 x 4096, 16 rows 67 -> 48, hipBLASLt 60-67).
-# Past 16 rows two token blocks halve what a fragment of weights is read for: hipBLASLt up to 32,768 channels
-# (16384 x 2048, 32 rows: 18.4 us against 21.4; 128256 x 2048: 119 against 112).
-_STREAM_MK, _STREAM_N, _STREAM_N2 = 16384, 8192, 32768
+# Where a projection goes to the workgroups that stay (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of
+# once 16 channels).  A K of 4096s, whose blocks are long: from 6144 channels on at any rows (us, skinny -> stream,
+# 6144 x 4096, 1 row 14.6 -> 13.6, 8 rows 15.7 -> 13.5; 28672 x 4096, 1 / 16 rows 43.6 / 67 -> 42.6 / 43.8; 4096 x 4096
+# level), an LM head from 2 rows on (128256 x 4096, 1 row 173 -> 175, 4 rows 192 -> 178).  Else by rows x width, the X
+# that the others read beside 16 channels of weights: 16384 x 2048, 4 rows 15.0 -> 15.6, 8 rows 16.8 -> 15.3, 32 rows
+# 18.0 with SwiGLU against hipBLASLt's 19.6; 8192 x 2048, 8 rows 9.2 -> 10.4, 24 rows 14.2 -> 11.2 (hipBLASLt 13.2).
+_STREAM_MK, _STREAM_N, _STREAM_N4, _STREAM_N2 = 16384, 8192, 6144, 32768
 # Rows x width up to which a projection of at most 4096 channels (one group a CU) runs on skinny_gemm.hip past
 # SKINNY_M rows: 4096 x 4096, 16 rows 11.2 us against hipBLASLt's 15.6, 24 rows 14.5 against 13.4; 3072 x 2048,
 # 32 rows 9.1 against 11.7.
@@ -610,12 +610,16 @@ def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
 
 
 def _stream_wins(M: int, N: int, K: int) -> bool:
-    return _stream_fits(M, K) and N >= _STREAM_N and M * K >= _STREAM_MK
+    if not _stream_fits(M, K):
+        return False
+    if K % 4096 == 0 and N >= _STREAM_N4:
+        return M > 1 or N < _STREAM_N2
+    return N >= _STREAM_N and M * K >= _STREAM_MK
 
 
 def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     M, (N, K) = x2.shape[0], w.shape
-    if _stream_wins(M, N, K) and (M <= 16 or N >= _STREAM_N2):
+    if _stream_wins(M, N, K):
         return native().stream_linear(x2, None, None, 0.0, w, None, False)[0] if _rows_ok(x2, w) else None
     if M <= SKINNY_M:
         # many rows of a large weight outside the kernel above: hipBLASLt
@@ -675,13 +679,15 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
 # rows up to which the RMSNorm runs in the prologue of skinny_gemm.hip (every workgroup recomputes the
 # rows): measured same box, 8B decode batch 1 3.607 -> 3.479 ms and 70B 26.22 -> 24.98 ms, but batch 4
 # 3.83 -> 4.04 ms (archive/profiles/r2s3_decode_ab/); the kernel takes up to 4.  stream_gemm.hip's workgroups
-# do it once for all their channels: up to 4 rows.
+# do it once for all their channels, up to 4 rows and behind no weights (us, skinny -> stream, 1 / 2 / 4 rows: 28672 x
+# 4096 with SwiGLU 45.9 / 49.1 / 56.4 -> 42.3 / 42.8 / 43.7; 6144 x 4096 13.6 / 14.4 / 17.2 -> 13.1 / 13.8 / 15.0; 2048 x
+# 2048 5.0 / 5.5 / 6.8 -> 4.6 / 4.9 / 5.6): wherever it takes the shape and 2048 channels keep its workgroups busy.
 NORM_M = int(os.environ.get("MXLLM_NORM_FUSED_M", "2"))
 
 
-def _norm_stream(M: int, K: int, scale) -> bool:
+def _norm_stream(M: int, K: int) -> bool:
     """Whether the RMSNorm goes into stream_gemm.hip's prologue."""
-    return _stream_fits(M, K, True) and NORM_M > 0 and (scale is not None or M > min(NORM_M, SKINNY_M))
+    return _stream_fits(M, K, True) and NORM_M > 0
 
 
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,
@@ -695,18 +701,17 @@ def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq
     if not (cos.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous() and k_cache.is_contiguous()
             and v_cache.is_contiguous()):
         return False
-    if _qkv_stream(M, K, D, norm, scale):
+    if _qkv_stream(M, K, norm):
         return _rows_ok(h, w, scale)
     if scale is not None or D != 128 or not 0 < M <= (min(NORM_M, SKINNY_M) if norm else SKINNY_M):
         return False
     return bool((not norm or M * K <= 32768) and _skinny_ok(h, w))
 
 
-def _qkv_stream(M: int, K: int, D: int, norm: bool, scale) -> bool:
-    """bf16 heads of 128 up to SKINNY_M rows have their kernel in skinny_gemm.hip."""
-    if norm:
-        return NORM_M > 0 and _stream_fits(M, K, True) and (scale is not None or D == 64 or M > min(NORM_M, SKINNY_M))
-    return _stream_fits(M, K) and (scale is not None or D == 64 or M > SKINNY_M)
+def _qkv_stream(M: int, K: int, norm: bool) -> bool:
+    """Whether the QKV projection goes to stream_gemm.hip (us, skinny -> stream, 6144 x 4096 without norm: 1 row 13.9 ->
+    13.1, 4 rows 14.8 -> 13.7, 8 rows 16.2 -> 14.6); bf16 heads of 128 whose K it does not take to skinny_gemm.hip."""
+    return _norm_stream(M, K) if norm else _stream_fits(M, K)
 
 
 def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, cos, sin, pos, slots, k_cache,
@@ -723,7 +728,7 @@ def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, 
         return None
     if delta is not None and (not norm or delta.shape != h.shape or delta.stride(1) != 1 or delta.stride(0) % 8):
         return None
-    if _qkv_stream(h.shape[0], h.shape[1], k_cache.shape[-1], norm, scale):
+    if _qkv_stream(h.shape[0], h.shape[1], norm):
         return native().stream_qkv_rope(h, delta, gamma, float(eps), w, scale, cos, sin, pos, slots, k_cache, v_cache,
                                         Hq, Hkv, block_table)
     return native().skinny_qkv_rope(h, delta, gamma, float(eps), w, cos, sin, pos, slots, k_cache, v_cache, Hq, Hkv,
@@ -740,7 +745,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     if SKINNY_M <= 0 or h.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return None
     M, K = h.shape
-    stream = _norm_stream(M, K, scale) and w.shape[0] >= _STREAM_N
+    stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else _STREAM_N)
     if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
     if h.stride(1) != 1 or w.shape[1] != K or w.shape[0] % 16:
