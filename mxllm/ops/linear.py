@@ -590,9 +590,10 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 # level), an LM head from 2 rows on (128256 x 4096, 1 row 173 -> 175, 4 rows 192 -> 178).  Else by rows x width, the X
 # that the others read beside 16 channels of weights: 16384 x 2048, 4 rows 15.0 -> 15.6, 8 rows 16.8 -> 15.3, 32 rows
 # 18.0 with SwiGLU against hipBLASLt's 19.6; 8192 x 2048, 8 rows 9.2 -> 10.4, 24 rows 14.2 -> 11.2 (hipBLASLt 13.2).
+# Past 8 rows also with few channels: 2048 x 4096, 16 rows 10.3 -> 9.1; 2048 x 2048, 12 / 32 rows 5.8 / 8.7 -> 5.8 / 7.5.
 _STREAM_MK, _STREAM_N, _STREAM_N4, _STREAM_N2 = 16384, 8192, 6144, 32768
-# Rows x width up to which a projection of at most 4096 channels (one group a CU) runs on skinny_gemm.hip past
-# SKINNY_M rows: 4096 x 4096, 16 rows 11.2 us against hipBLASLt's 15.6, 24 rows 14.5 against 13.4; 3072 x 2048,
+# Rows x width up to which a projection of at most 4096 channels (one group a CU) that the kernel above does not take
+# runs on skinny_gemm.hip past SKINNY_M rows: 4096 x 4096, 16 rows 11.2 us against hipBLASLt's 15.6, 24 rows 14.5 against 13.4; 3072 x 2048,
 # 32 rows 9.1 against 11.7.
 _WIDE_MK, _WIDE_N = 65536, 4096
 
@@ -612,9 +613,21 @@ def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
 def _stream_wins(M: int, N: int, K: int) -> bool:
     if not _stream_fits(M, K):
         return False
+    if M > 8 and N >= 2048:
+        return True
     if K % 4096 == 0 and N >= _STREAM_N4:
         return M > 1 or N < _STREAM_N2
     return N >= _STREAM_N and M * K >= _STREAM_MK
+
+
+def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
+    """Inference: ``x2 W^T`` for a few rows and e4m3 weights.  A long K on stream_gemm.hip where X fits its LDS (us,
+    fp8_gemm.hip -> there: 4096 x 14336, 1 / 4 rows 16.8 / 18.2 -> 15.2 / 16.9; 2048 x 8192, 8 rows 10.9 -> 10.1; but
+    4096 x 4096, 4 rows 6.5 -> 7.2)."""
+    M, K = x2.shape
+    if K >= 8192 and _stream_fits(M, K) and _rows_ok(x2, q, scale):
+        return native().stream_linear(x2, None, None, 0.0, q, scale, False)[0]
+    return native().w8_linear(x2, q, scale)
 
 
 def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:

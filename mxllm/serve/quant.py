@@ -28,6 +28,7 @@ import torch
 import torch.nn as nn
 
 from ..ops._ext import native, use_native
+from ..ops.linear import w8_rows
 
 E4M3_MAX = 448.0
 # Calls of up to SMALL_M tokens use the weight-only HIP kernel (bf16 activations, the fp8
@@ -86,9 +87,9 @@ class W8Linear(nn.Module):
         if not use_native(x2):
             y = torch.matmul(x2, dequantize_e4m3(self.q, self.scale).to(x2.dtype).t())
         elif M <= SMALL_M or self.in_features % 16 or self.out_features % 16:
-            # weight-streaming HIP kernel: bf16 activations, weights dequantised in registers
-            # (it falls back to dequantise + hipBLASLt for shapes it does not take)
-            y = native().w8_linear(x2, self.q, self.scale)
+            # weight-streaming HIP kernels: bf16 activations, weights dequantised in registers
+            # (w8_linear falls back to dequantise + hipBLASLt for shapes it does not take)
+            y = w8_rows(x2, self.q, self.scale)
         else:
             # larger batches / prefill: fp8 x fp8 MFMA GEMM (hipBLASLt), per-token activation
             # scales and the per-channel weight scales applied by the GEMM epilogue
