@@ -181,16 +181,15 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
         not mostly padding and five eighths of the CUs have a tile.  2048 x 16384 at 700 48 -> 42, 2600 205 -> 142, 4096
         236 -> 198 (512, 128 tiles: 38 -> 40); 4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 1025 249 -> 241, 4096
         706 -> 640."""
-    if _policy() == "0":
-        return 0
-    tiles = -(-M // 256) * (N // 256)
+    rows = -(-M // 256)
+    tiles = rows * (N // 256)
     if 0 < tiles <= CUS // 2 and not swiglu and (M >= 64 and K >= 12288 if b_kc else K >= 6144):
-        return min(CUS // tiles, 16)
-    if swiglu:
-        return int(tiles >= CUS * 5 // 8 and 4 * M >= 3 * (-(-M // 256) * 256))
-    if M % 256 == 0:
-        return 0
-    return int(tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles))
+        parts = min(CUS // tiles, 16)
+    elif swiglu:
+        parts = int(tiles >= CUS * 5 // 8 and 4 * M >= 768 * rows)
+    else:
+        parts = int(M % 256 != 0 and (tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles)))
+    return parts if parts and _policy() != "0" else 0
 
 
 DEFAULT_PH = int(os.environ.get("MXLLM_GEMM8_DEFAULT_PH", "4"))

@@ -656,13 +656,14 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
         if y is not None:
             return y.view(*x.shape[:-1], w.shape[0])
-    if x.shape[-1] == w.shape[1] and x.dtype == torch.bfloat16 and x.is_cuda and x.dim() > 1:
-        M = x.numel() // max(x.shape[-1], 1)
-        parts = gemm.rows_gain(M, *w.shape, True)
-        if parts and _no_autograd(x):
-            x2 = x.reshape(M, x.shape[-1])
+    if x.is_cuda and x.dim() > 1:
+        N, K = w.shape
+        M = x.numel() // max(K, 1)
+        parts = gemm.rows_gain(M, N, K, True)
+        if parts and x.shape[-1] == K and _no_autograd(x):
+            x2 = x.reshape(M, K)
             if gemm.rows_ok(x2, w, True):
-                return native().gemm8_rows(x2, w, True, False, parts).view(*x.shape[:-1], w.shape[0])
+                return native().gemm8_rows(x2, w, True, False, parts).view(*x.shape[:-1], N)
     return F.linear(x, w)
 
 
