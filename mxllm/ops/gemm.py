@@ -174,8 +174,9 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
       * input gradients: K of 6144 on.  16384 x 2048 at 1000 124 -> 68, 4096 237 -> 211; 6144 x 4096 at 512 53 -> 43
         (3072 x 2048 at 512 26 -> 30).
     Whole, where the library, which is tuned for round numbers of rows, falls behind between them:
-      * projections (``b_kc``) from 700 tiles on: 4096 x 28672 at 2600 542 -> 450, 3606 612 -> 617, 5000 904 -> 820;
-        8192 x 57344 at 700 559 -> 530 (4096 x 28672 at 1025, 560 tiles: 235 -> 241; 14336 x 4096 at 2600, 176: 237 -> 243);
+      * projections (``b_kc``) of K 8192 and more from 500 tiles on: 8192 x 57344 at 700 559 -> 530, 2600 1916 -> 1740;
+        8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321).  With a shorter K the library is up to 27 %
+        slower at some row counts and 3 to 6 % faster at others (4096 x 28672 at 2700 543 -> 441, 4003 600 -> 634);
       * input gradients: :func:`_gains_nn`;
       * gate-up with SwiGLU, which saves the projection's trip through HBM at any size: where the last tile's rows are
         not mostly padding and five eighths of the CUs have a tile.  2048 x 16384 at 700 48 -> 42, 2600 205 -> 142, 4096
@@ -188,7 +189,7 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
     elif swiglu:
         parts = int(tiles >= CUS * 5 // 8 and 4 * M >= 768 * rows)
     else:
-        parts = int(M % 256 != 0 and (tiles >= 700 if b_kc else K >= 128 and _gains_nn(tiles)))
+        parts = int(M % 256 != 0 and (K >= 8192 and tiles >= 500 if b_kc else K >= 128 and _gains_nn(tiles)))
     return parts if parts and _policy() != "0" else 0
 
 

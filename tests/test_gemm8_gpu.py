@@ -130,7 +130,7 @@ def test_gemm8_rows(gpu, M, N, K):
                 assert torch.equal(_ops().gemm8_rows(x, w, True, True, parts), ops.swiglu(yp))
 
 
-@pytest.mark.parametrize("M,N,K,form", [(2563, 18432, 256, "tn"), (64, 256, 12288, "tn"), (300, 512, 12288, "tn"),
+@pytest.mark.parametrize("M,N,K,form", [(2563, 12800, 8192, "tn"), (64, 256, 12288, "tn"), (300, 512, 12288, "tn"),
                                         (1000, 10240, 512, "swiglu"), (2563, 18432, 256, "swiglu"), (2563, 4096, 256, "nn"),
                                         (512, 512, 6144, "nn")])
 def test_rows_routes(gpu, M, N, K, form):
