@@ -189,34 +189,6 @@ bool gemm8_sq(const at::Tensor& a, bool a_kc, const at::Tensor& b, bool b_kc, at
   return true;
 }
 
-// a op(b) (bf16) for any number of rows: a [M, K], b [N, K] when b_kc else [K, N] -> [M, N]; swiglu: b = [gate; up]
-// -> silu(gate) up [M, N / 2] (mx_gemm8_rows; callers ask mxllm/ops/gemm.py rows_ok first).
-// parts > 1: K in that many parts (mx_gemm8_parts).
-at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool swiglu, int64_t parts) {
-  MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm8_rows: GPU tensors of one device");
-  MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm8_rows: bf16 operands");
-  MX_CHECK(a.dim() == 2 && b.dim() == 2, "gemm8_rows: 2-D operands");
-  const int64_t M = a.size(0), K = a.size(1), N = b_kc ? b.size(0) : b.size(1);
-  MX_CHECK(K == (b_kc ? b.size(1) : b.size(0)), "gemm8_rows: shape mismatch");
-  MX_CHECK(a.stride(1) == 1 && b.stride(1) == 1 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX,
-           "gemm8_rows: row-major operands");
-  DevGuard g(a.device());
-  auto out = at::empty({M, swiglu ? N / 2 : N}, a.options());
-  int rc;
-  if (parts > 1) {
-    MX_CHECK(parts <= K / 64, "gemm8_rows: parts of at least 64 of K");
-    auto ws = at::empty({parts * M * N}, a.options().dtype(at::kFloat));
-    rc = mx_gemm8_parts(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
-                        (int)K, swiglu ? 1 : 0, (int)parts, ws.data_ptr<float>(), cur_stream());
-  } else {
-    rc = mx_gemm8_rows(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
-                       (int)K, swiglu ? 1 : 0, cur_stream());
-  }
-  MX_CHECK(rc != -1, "gemm8_rows: shape, stride or alignment not taken");
-  MX_OK(rc);
-  return out;
-}
-
 // out[M, N] (bf16) = op(a) op(b) with the tail-balanced launch (mx_gemm8_tail): the output split at
 // `at` columns (rows when `rows`) -- whole waves of tiles before it, half-K workgroups summed through
 // an fp32 workspace after it.  Returns false (nothing launched) for shapes it does not take.
@@ -1002,7 +974,6 @@ TORCH_LIBRARY(mxllm, m) {
   m.def("segmented_mean(Tensor codes, Tensor offsets) -> Tensor");
   m.def("copy2d_batched(Tensor desc, int total_blocks) -> ()");
   m.def("transpose2d(Tensor x, Tensor? scale=None) -> Tensor");
-  m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
   m.def("gemm8(Tensor a, bool a_kc, Tensor b, bool b_kc, Tensor(a!) out, float beta, Tensor? alpha_t=None, float alpha=1.0, int ph=8) -> bool");
   m.def("prefetch(Tensor t, int wgs) -> ()");
   m.def("cu_masked_stream(int device, int[] mask) -> int", &cu_masked_stream);  // no tensor args: catch-all
@@ -1048,7 +1019,6 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("segmented_mean", &segmented_mean);
   m.impl("copy2d_batched", &copy2d_batched);
   m.impl("transpose2d", &transpose2d);
-  m.impl("gemm8_rows", &gemm8_rows);
   m.impl("gemm8", &gemm8);
   m.impl("gemm8_tail", &gemm8_tail);
   m.impl("gemm8_rope", &gemm8_rope);

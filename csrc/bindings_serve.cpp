@@ -145,6 +145,34 @@ StreamOperands stream_operands(const at::Tensor& x, const c10::optional<at::Tens
   return o;
 }
 
+// a op(b) (bf16) for any number of rows: a [M, K], b [N, K] when b_kc else [K, N] -> [M, N]; swiglu: b = [gate; up]
+// -> silu(gate) up [M, N / 2] (mx_gemm8_rows; callers ask mxllm/ops/gemm.py rows_ok first).
+// parts > 1: K in that many parts (mx_gemm8_parts).
+at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool swiglu, int64_t parts) {
+  MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm8_rows: GPU tensors of one device");
+  MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm8_rows: bf16 operands");
+  MX_CHECK(a.dim() == 2 && b.dim() == 2, "gemm8_rows: 2-D operands");
+  const int64_t M = a.size(0), K = a.size(1), N = b_kc ? b.size(0) : b.size(1);
+  MX_CHECK(K == (b_kc ? b.size(1) : b.size(0)), "gemm8_rows: shape mismatch");
+  MX_CHECK(a.stride(1) == 1 && b.stride(1) == 1 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX,
+           "gemm8_rows: row-major operands");
+  DevGuard g(a.device());
+  auto out = at::empty({M, swiglu ? N / 2 : N}, a.options());
+  int rc;
+  if (parts > 1) {
+    MX_CHECK(parts <= K / 64, "gemm8_rows: parts of at least 64 of K");
+    auto ws = at::empty({parts * M * N}, a.options().dtype(at::kFloat));
+    rc = mx_gemm8_parts(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
+                        (int)K, swiglu ? 1 : 0, (int)parts, ws.data_ptr<float>(), cur_stream());
+  } else {
+    rc = mx_gemm8_rows(bf(a), a.stride(0), bf(b), b.stride(0), b_kc ? 1 : 0, bfm(out), out.stride(0), (int)M, (int)N,
+                       (int)K, swiglu ? 1 : 0, cur_stream());
+  }
+  MX_CHECK(rc != -1, "gemm8_rows: shape, stride or alignment not taken");
+  MX_OK(rc);
+  return out;
+}
+
 // y = [swiglu](x . w^T); with gamma x = rmsnorm(h + delta), up to 4 rows.  Returns (y, h + delta).
 std::tuple<at::Tensor, at::Tensor> stream_linear(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
                                                  const c10::optional<at::Tensor>& gamma, double eps, const at::Tensor& w,
@@ -405,6 +433,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("decode_attn(Tensor q, Tensor k_cache, Tensor v_cache, Tensor lens, Tensor? slots, int max_len, float scale, int len_off=0, Tensor? block_table=None, Tensor? counters=None) -> Tensor");
   m.def("decode_attn_partials(Tensor q, Tensor k_cache, Tensor v_cache, Tensor lens, Tensor? slots, int max_len, float scale, int len_off=0, Tensor? block_table=None) -> (Tensor, Tensor)");
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
+  m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
   m.def("stream_linear(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, bool swiglu) -> (Tensor, Tensor)");
   m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
         "Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, "
@@ -425,6 +454,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn_partials", &decode_attn_partials);
   m.impl("skinny_merge_linear", &skinny_merge_linear);
   m.impl("decode_attn", &decode_attn);
+  m.impl("gemm8_rows", &gemm8_rows);
   m.impl("stream_linear", &stream_linear);
   m.impl("stream_qkv_rope", &stream_qkv_rope);
   m.impl("sample", &sample);

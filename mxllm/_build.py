@@ -35,8 +35,8 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 # component -> (library, kernel files, op binding files)
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
-              ("attn_fwd", "chunk_attn", "decode", "hybrid", "hybrid_skinny", "latent", "latent_mfma", "mingru",
-               "moe", "moe_mfma", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
+              ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
+               "mingru", "moe", "moe_mfma", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
                "stream_gemm"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),
 }

@@ -151,7 +151,7 @@ def _gains_nn(tiles: int) -> bool:
 
 
 def rows_ok(a: torch.Tensor, b: torch.Tensor, b_kc: bool, swiglu: bool = False) -> bool:
-    """What mx_gemm8_rows (csrc/kernels/gemm8.hip) takes: any number of rows of ``a`` [M, K]."""
+    """What mx_gemm8_rows (csrc/kernels/gemm8_rows.hip) takes: any number of rows of ``a`` [M, K]."""
     if not (use_native(a) and a.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16):
         return False
     K, N = a.shape[1], b.shape[0 if b_kc else 1]

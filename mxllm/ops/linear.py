@@ -670,7 +670,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
     """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch, with
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
-    stream_gemm.hip or gemm8.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
+    stream_gemm.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
     if SKINNY_M <= 0 or x.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
         return None
