@@ -644,14 +644,17 @@ def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     return None
 
 
-def _no_autograd(x: torch.Tensor) -> bool:
-    """No gradient is asked of ``x``, backward or forward mode (kernels without a derivative)."""
-    return not (torch.is_grad_enabled() and x.requires_grad) and forward_ad.unpack_dual(x).tangent is None
+def _no_autograd(*ts: torch.Tensor | None) -> bool:
+    """No gradient is asked of any of these, backward or forward mode (kernels without a derivative)."""
+    grad = torch.is_grad_enabled()
+    return all(t is None or (not (grad and t.requires_grad) and forward_ad.unpack_dual(t).tangent is None) for t in ts)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if w.requires_grad and torch.is_grad_enabled():
         return _LinearFn.apply(x, w)
+    if not _no_autograd(x, w):
+        return F.linear(x, w)
     if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= 32:
         y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
         if y is not None:
@@ -660,7 +663,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         N, K = w.shape
         M = x.numel() // max(K, 1)
         parts = gemm.rows_gain(M, N, K, True)
-        if parts and x.shape[-1] == K and _no_autograd(x):
+        if parts and x.shape[-1] == K:
             x2 = x.reshape(M, K)
             if gemm.rows_ok(x2, w, True):
                 return native().gemm8_rows(x2, w, True, False, parts).view(*x.shape[:-1], N)
@@ -672,7 +675,7 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
     stream_gemm.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
-    if SKINNY_M <= 0 or x.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
+    if SKINNY_M <= 0 or x.dim() != 2 or not _no_autograd(x, w):
         return None
     if x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
         return None
@@ -685,7 +688,7 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     if 0 < x.shape[0] <= SKINNY_M and _skinny_ok(x, w):
         return native().skinny_linear_swiglu(x, w)
     parts = gemm.rows_gain(x.shape[0], *w.shape, True, True)  # a prompt pass
-    if parts and gemm.rows_ok(x, w, True, True) and _no_autograd(x):
+    if parts and gemm.rows_ok(x, w, True, True):
         return native().gemm8_rows(x, w, True, True, parts)
     return None
 
@@ -707,7 +710,7 @@ def _norm_stream(M: int, K: int) -> bool:
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,
                 norm: bool, scale: torch.Tensor | None = None) -> bool:
     """Whether :func:`qkv_rope_linear` takes these shapes (``norm``: with the RMSNorm prologue)."""
-    if SKINNY_M <= 0 or h.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
+    if SKINNY_M <= 0 or h.dim() != 2 or not _no_autograd(h, w):
         return False
     (M, K), D = h.shape, k_cache.shape[-1]
     if D not in (64, 128) or w.shape != ((Hq + 2 * Hkv) * D, K) or k_cache.dtype != torch.bfloat16:
@@ -738,7 +741,7 @@ def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, 
     norm = gamma is not None
     if not qkv_rope_ok(h, w, cos, sin, k_cache, v_cache, Hq, Hkv, norm, scale):
         return None
-    if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous()):
+    if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous() or not _no_autograd(delta, gamma)):
         return None
     if delta is not None and (not norm or delta.shape != h.shape or delta.stride(1) != 1 or delta.stride(0) % 8):
         return None
@@ -756,7 +759,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     the RMSNorm kernel + decode GEMM); with ``swiglu`` w = [gate; up] and the first output is
     silu(g) * u; ``scale``: w is e4m3 codes.  ``delta`` None: plain RMSNorm, the residual is ``h``.  None
     when the fused kernels do not take the call."""
-    if SKINNY_M <= 0 or h.dim() != 2 or (w.requires_grad and torch.is_grad_enabled()):
+    if SKINNY_M <= 0 or h.dim() != 2 or not _no_autograd(delta, h, gamma, w):
         return None
     M, K = h.shape
     stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else _STREAM_N)

@@ -1,0 +1,58 @@
+"""What the inference kernels behind ``ops.linear`` and its fused forms must not take: they have neither derivatives nor
+batching rules, and read whole 16-byte pieces of dense rows."""
+import pytest
+import torch
+
+from mxllm import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _bf16(gpu, *shape, seed=0, std=1.0):
+    g = torch.Generator(device=gpu).manual_seed(seed)
+    return torch.empty(*shape, device=gpu).normal_(0, std, generator=g).bfloat16()
+
+
+def _close(got, want, tol):
+    err = float((got.double() - want.double()).norm() / want.double().norm())
+    assert err < tol, err
+
+
+# rows on each side of the decode GEMMs' limits (8, 16, 32) and of a prompt pass; 12,288: K in parts from 64 rows on
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 64])
+@pytest.mark.parametrize("N,K", [(2048, 2048), (8192, 4096), (512, 12288)])
+def test_frozen_weight_passes_gradients(gpu, M, N, K):
+    """A frozen weight: the input's gradient is dy W, backward and forward mode (one bf16 rounding: 2^-8)."""
+    x, w, dy = _bf16(gpu, M, K, seed=1).requires_grad_(), _bf16(gpu, N, K, seed=2, std=0.03), _bf16(gpu, M, N, seed=3)
+    y = ops.linear(x, w)
+    y.backward(dy)
+    _close(x.grad, dy.double() @ w.double(), 2 ** -8)
+    t = _bf16(gpu, M, K, seed=4)
+    _, tan = torch.func.jvp(lambda a: ops.linear(a, w), (x.detach(),), (t,))
+    _close(tan, t.double() @ w.double().t(), 2 ** -8)
+    with torch.autograd.forward_ad.dual_level():  # a tangent of the weight alone
+        dual = torch.autograd.forward_ad.make_dual(w, torch.ones_like(w))
+        tan = torch.autograd.forward_ad.unpack_dual(ops.linear(x.detach(), dual)).tangent
+    _close(tan, x.detach().double().sum(1, keepdim=True).expand(M, N), 2 ** -6)
+
+
+@pytest.mark.parametrize("M", [1, 4, 16])
+def test_fused_forms_decline_gradients(gpu, M):
+    """The fused decode forms leave calls whose inputs ask for gradients to the caller's differentiable parts."""
+    K, F, H, D = 4096, 4096, 4, 128
+    x, w, gamma = _bf16(gpu, M, K), _bf16(gpu, 2 * F, K, seed=1, std=0.03), torch.ones(K, device=gpu).bfloat16()
+    wq = _bf16(gpu, 3 * H * D, K, seed=2, std=0.03)
+    cos = torch.ones(64, D // 2, device=gpu)
+    pos = torch.zeros(M, dtype=torch.int32, device=gpu)
+    kc, vc = torch.zeros(2, M, H, 64, D, device=gpu, dtype=torch.bfloat16)
+
+    def forms(x, delta, gamma):
+        a = ops.linear_swiglu(x, w), ops.qkv_rope_linear(None, x, None, 1e-5, wq, cos, cos, pos, None, kc, vc, H, H)
+        return a + ((ops.norm_linear(delta, x, gamma, 1e-5, w, True),
+                     ops.qkv_rope_linear(delta, x, gamma, 1e-5, wq, cos, cos, pos, None, kc, vc, H, H)) if M <= 4 else ())
+
+    assert all(r is not None for r in forms(x, x, gamma))
+    assert all(r is None for r in forms(x.clone().requires_grad_(), x, gamma))
+    if M <= 4:
+        for delta, g in ((x.clone().requires_grad_(), gamma), (x, gamma.clone().requires_grad_())):
+            assert all(r is None for r in forms(x, delta, g)[2:])
