@@ -644,16 +644,22 @@ def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     return None
 
 
-def _no_autograd(*ts: torch.Tensor | None) -> bool:
-    """No gradient is asked of any of these, backward or forward mode (kernels without a derivative)."""
+def _plain(*ts: torch.Tensor | None) -> bool:
+    """Tensors that a kernel without a derivative, a batching rule or a shape function may take: no gradient is asked of
+    any, backward or forward mode, none is a transform's (``torch.func``) or a subclass, and nothing records the call
+    (compilers, tracers, dispatch modes), which would keep the choice made for these sizes, or not know the op."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
+        return False
     grad = torch.is_grad_enabled()
-    return all(t is None or (not (grad and t.requires_grad) and forward_ad.unpack_dual(t).tangent is None) for t in ts)
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)
+                             and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+                             and forward_ad.unpack_dual(t).tangent is None) for t in ts)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if w.requires_grad and torch.is_grad_enabled():
         return _LinearFn.apply(x, w)
-    if not _no_autograd(x, w):
+    if not _plain(x, w):
         return F.linear(x, w)
     if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= 32:
         y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
@@ -675,7 +681,7 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
     stream_gemm.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
-    if SKINNY_M <= 0 or x.dim() != 2 or not _no_autograd(x, w):
+    if SKINNY_M <= 0 or x.dim() != 2 or not _plain(x, w):
         return None
     if x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
         return None
@@ -710,7 +716,7 @@ def _norm_stream(M: int, K: int) -> bool:
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,
                 norm: bool, scale: torch.Tensor | None = None) -> bool:
     """Whether :func:`qkv_rope_linear` takes these shapes (``norm``: with the RMSNorm prologue)."""
-    if SKINNY_M <= 0 or h.dim() != 2 or not _no_autograd(h, w):
+    if SKINNY_M <= 0 or h.dim() != 2 or not _plain(h, w):
         return False
     (M, K), D = h.shape, k_cache.shape[-1]
     if D not in (64, 128) or w.shape != ((Hq + 2 * Hkv) * D, K) or k_cache.dtype != torch.bfloat16:
@@ -741,7 +747,7 @@ def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, 
     norm = gamma is not None
     if not qkv_rope_ok(h, w, cos, sin, k_cache, v_cache, Hq, Hkv, norm, scale):
         return None
-    if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous() or not _no_autograd(delta, gamma)):
+    if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous() or not _plain(delta, gamma)):
         return None
     if delta is not None and (not norm or delta.shape != h.shape or delta.stride(1) != 1 or delta.stride(0) % 8):
         return None
@@ -759,7 +765,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     the RMSNorm kernel + decode GEMM); with ``swiglu`` w = [gate; up] and the first output is
     silu(g) * u; ``scale``: w is e4m3 codes.  ``delta`` None: plain RMSNorm, the residual is ``h``.  None
     when the fused kernels do not take the call."""
-    if SKINNY_M <= 0 or h.dim() != 2 or not _no_autograd(delta, h, gamma, w):
+    if SKINNY_M <= 0 or h.dim() != 2 or not _plain(delta, h, gamma, w):
         return None
     M, K = h.shape
     stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else _STREAM_N)

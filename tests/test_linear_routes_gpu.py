@@ -56,3 +56,26 @@ def test_fused_forms_decline_gradients(gpu, M):
     if M <= 4:
         for delta, g in ((x.clone().requires_grad_(), gamma), (x, gamma.clone().requires_grad_())):
             assert all(r is None for r in forms(x, delta, g)[2:])
+
+
+@pytest.mark.parametrize("M", [4, 16, 64])
+def test_transforms_and_tracers_take_the_library(gpu, M):
+    """vmap, torch.func.grad, compilation, tracing and shape propagation of an inference call, on each side of the
+    decode GEMMs' rows; a traced call is right at rows that it was not traced with."""
+    from torch._subclasses import FakeTensorMode
+
+    K, N = (2048, 4096) if M < 64 else (12288, 512)
+    w, xs = _bf16(gpu, N, K, seed=1, std=0.03), _bf16(gpu, 3, M, K, seed=2)
+    want = xs.double() @ w.double().t()
+    _close(torch.func.vmap(lambda a: ops.linear(a, w))(xs), want, 2 ** -8)
+    _close(torch.func.vmap(lambda b: ops.linear(xs[0], b))(torch.stack([w, 2 * w]))[1], 2 * want[0], 2 ** -8)
+    dx = torch.func.grad(lambda a: ops.linear(a, w).double().sum())(xs[0])
+    _close(dx, w.double().sum(0).expand(M, K), 2 ** -8)
+    _close(torch.compile(lambda a: ops.linear(a, w), backend="eager", fullgraph=True)(xs[0]), want[0], 2 ** -8)
+    traced = torch.jit.trace(lambda a: ops.linear(a, w), xs[0], check_trace=False)
+    _close(traced(xs.reshape(-1, K)), want.reshape(-1, N), 2 ** -8)
+    mode = FakeTensorMode()
+    fakes = mode.from_tensor(xs[0]), mode.from_tensor(w)
+    with mode:
+        y = ops.linear(*fakes)
+        assert y.shape == (M, N) and y.device == w.device
