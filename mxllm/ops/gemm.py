@@ -101,8 +101,8 @@ def takes(form: str, M: int, N: int, K: int) -> bool:
     return K % 64 == 0 or form == "tt"
 
 
-def schedule(form: str, M: int, N: int, K: int, out_dtype: torch.dtype) -> int:
-    """0 = not on gemm8; else its phase schedule (8 or 4) for this shape."""
+def schedule(form: str, M: int, N: int, K: int, out_dtype: torch.dtype, rules: bool = True) -> int:
+    """0 = not on gemm8; else its phase schedule (8 or 4) for this shape (``rules`` False: by the table alone)."""
     pol = _policy()
     if pol == "0" or not takes(form, M, N, K):
         return 0
@@ -111,7 +111,7 @@ def schedule(form: str, M: int, N: int, K: int, out_dtype: torch.dtype) -> int:
         ph = 4  # persistent kernel: world 1 only (see _multi_rank)
     if ph:
         return ph
-    if out_dtype == torch.bfloat16 and _gains(form, M, N, K):
+    if rules and out_dtype == torch.bfloat16 and _gains(form, M, N, K):
         return 4
     return DEFAULT_PH if (pol == "all" or deterministic()) else 0
 
@@ -196,8 +196,14 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
 DEFAULT_PH = int(os.environ.get("MXLLM_GEMM8_DEFAULT_PH", "4"))
 
 
-def want(form: str, M: int, N: int, K: int, out_dtype: torch.dtype) -> bool:
-    return schedule(form, M, N, K, out_dtype) > 0
+def want(form: str, M: int, N: int, K: int, out_dtype: torch.dtype, rules: bool = True) -> bool:
+    return schedule(form, M, N, K, out_dtype, rules) > 0
+
+
+def asks_grad(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """A backward pass that is itself to be differentiated (``create_graph``).  The sizes that go to a kernel by rule
+    then stay with torch, which refuses what it cannot differentiate; a kernel would leave the gradient out."""
+    return torch.is_grad_enabled() and (a.requires_grad or b.requires_grad)
 
 
 # (A k-contiguous, B k-contiguous) per form
@@ -221,14 +227,15 @@ def mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = N
     ``alpha_t``: optional 1-element f32 device scalar (no host sync)."""
     M, N, K = _dims(form, a, b)
     odt = out.dtype if out is not None else (out_dtype or a.dtype)
-    if out is None and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16:
+    asked = asks_grad(a, b)
+    if out is None and not asked and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16:
         parts = rows_gain(M, N, K, form == "tn")
         if parts and rows_ok(a, b, form == "tn"):
             return native().gemm8_rows(a, b, form == "tn", False, parts)
     if out is None:
         out = torch.empty(M, N, dtype=odt, device=a.device)
         beta = 0.0
-    ph = (schedule(form, M, N, K, odt) if use_native(a) and a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16
+    ph = (schedule(form, M, N, K, odt, not asked) if use_native(a) and a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16
           and odt in (torch.bfloat16, torch.float32) else 0)
     if ph:
         a_kc, b_kc = _KC[form]

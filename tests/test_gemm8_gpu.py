@@ -287,3 +287,19 @@ def test_gemm8_persistent_bitwise(gpu, a_kc, b_kc, f32, beta, monkeypatch):
     assert torch.equal(outs["0"], outs["1"])
     ref = A @ B + (c0.float() if beta else 0.0)
     _check(outs["1"], ref, 1e-5 if f32 else 5e-3)
+
+
+@pytest.mark.parametrize("form,M,N,K", [("nn", 512, 512, 6144), ("nn", 2563, 4096, 256), ("tn", 64, 256, 12288),
+                                        ("tt", 256, 512, 1000)])
+def test_second_derivatives_are_refused(gpu, form, M, N, K):
+    """Sizes that go to gemm8 by rule: where the product itself is to be differentiated it is refused as elsewhere, and
+    not answered by a kernel that leaves the gradient out."""
+    from mxllm.ops import gemm
+
+    a = _mat(K, M, gpu, seed=1) if form == "tt" else _mat(M, K, gpu, seed=1)
+    b = _mat(N, K, gpu, seed=2) if form == "tn" else _mat(K, N, gpu, seed=2)
+    assert gemm.rows_gain(M, N, K, form == "tn") or gemm.want(form, M, N, K, torch.bfloat16)
+    with pytest.raises(RuntimeError, match="automatic differentiation"):
+        gemm.mm(form, a.clone().requires_grad_(), b)
+    with torch.no_grad():
+        assert gemm.mm(form, a.clone().requires_grad_(), b).shape == (M, N)
