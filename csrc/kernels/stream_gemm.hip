@@ -250,7 +250,8 @@ extern "C" int mx_stream_ok(int M, int K, int norm) {
 
 // epi 0: y [M, N]; 1: w = [gate; up], y [M, N / 2] = silu(g) u; 2 / 3: the QKV projection of heads of 128 / 64 (N =
 // (Hq + 2 Hkv) heads), q rotated, K / V appended to the caches at (slot, pos).  scale: w is e4m3 codes, else bf16.
-// gamma: X = rmsnorm(h + delta) of up to 4 rows (x = h; delta may be null, else h_out gets h + delta).
+// gamma: X = rmsnorm(h + delta) of up to 4 rows (x = h; delta may be null, else h_out gets h + delta).  What is read,
+// and h_out, 16-B aligned, the other outputs 8-B; other sizes, strides and addresses: -1, nothing launched.
 extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
                               int64_t ldy, int M, int N, int K, int epi, const uint16_t* delta, int64_t ldd,
                               const uint16_t* gamma, float eps, uint16_t* h_out, const float* cosb, const float* sinb,
@@ -259,6 +260,9 @@ extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int
   if (M <= 0) return 0;
   if (!mx_stream_ok(M, K, gamma != nullptr) || N % 16 || ldx % 8 || ldw % (scale ? 16 : 8) || ldx < K || ldw < K ||
       epi < 0 || epi > 3 || (delta && (!gamma || ldd % 8 || ldd < K || !h_out)))
+    return -1;
+  if (((uintptr_t)x | (uintptr_t)w | (uintptr_t)scale | (uintptr_t)delta | (uintptr_t)gamma | (uintptr_t)h_out) & 15 ||
+      ((uintptr_t)y | (uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 7)
     return -1;
   if (epi >= 2 ? N != (Hq + 2 * Hkv) * (epi == 2 ? 128 : 64) : (ldy % 4 || ldy < (epi == 1 ? N / 2 : N))) return -1;
   StreamArgs a{x, ldx, w, ldw, scale, y, ldy, M, K, N / 2, N / 16, SkNorm{delta, ldd, gamma, h_out, eps},

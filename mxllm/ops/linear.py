@@ -575,13 +575,19 @@ _SKINNY_SMALL_W = 128 << 20
 _HALF_N = 4096
 
 
+def _dense_rows(t: torch.Tensor) -> bool:
+    """[rows, n] that a kernel may read in 16-byte pieces: rows that do not overlap, every piece aligned."""
+    return (t.stride(1) == 1 and t.stride(0) * t.element_size() % 16 == 0 and t.stride(0) >= t.shape[1]
+            and t.data_ptr() % 16 == 0)
+
+
 def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
     K, M = x2.shape[1], x2.shape[0]
     if M > 1 and w.shape[0] * K > _SKINNY_SMALL_W:
         return False
     return (M <= SKINNY_M and x2.is_cuda and x2.dtype == torch.bfloat16
-            and w.dtype == torch.bfloat16 and K % 512 == 0 and w.shape[0] % 16 == 0 and x2.stride(1) == 1
-            and x2.stride(0) % 8 == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0 and use_native(x2))
+            and w.dtype == torch.bfloat16 and K % 512 == 0 and w.shape[0] % 16 == 0 and _dense_rows(x2) and _dense_rows(w)
+            and use_native(x2))
 
 
 # Where a projection goes to the workgroups that stay (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of
@@ -601,8 +607,8 @@ _WIDE_MK, _WIDE_N = 65536, 4096
 def _rows_ok(x2: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> bool:
     """Operands that the decode GEMMs take: bf16 rows, and weights of bf16 or of e4m3 codes with ``scale``."""
     return (x2.is_cuda and x2.dtype == torch.bfloat16 and w.dtype == (torch.bfloat16 if scale is None else torch.uint8)
-            and x2.shape[1] == w.shape[1] and w.shape[0] % 16 == 0 and x2.stride(1) == 1 and x2.stride(0) % 8 == 0
-            and w.stride(1) == 1 and w.stride(0) % (8 if scale is None else 16) == 0 and use_native(x2))
+            and x2.shape[1] == w.shape[1] and w.shape[0] % 16 == 0 and _dense_rows(x2) and _dense_rows(w)
+            and (scale is None or scale.data_ptr() % 16 == 0) and use_native(x2))
 
 
 def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
@@ -708,6 +714,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
 NORM_M = int(os.environ.get("MXLLM_NORM_FUSED_M", "2"))
 
 
+def _norm_operands(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor) -> bool:
+    return (gamma.dtype == torch.bfloat16 and gamma.is_contiguous() and gamma.data_ptr() % 16 == 0
+            and (delta is None or (delta.shape == h.shape and delta.dtype == h.dtype and _dense_rows(delta))))
+
+
 def _norm_stream(M: int, K: int) -> bool:
     """Whether the RMSNorm goes into stream_gemm.hip's prologue."""
     return _stream_fits(M, K, True) and NORM_M > 0
@@ -747,9 +758,9 @@ def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, 
     norm = gamma is not None
     if not qkv_rope_ok(h, w, cos, sin, k_cache, v_cache, Hq, Hkv, norm, scale):
         return None
-    if norm and (gamma.dtype != torch.bfloat16 or not gamma.is_contiguous() or not _plain(delta, gamma)):
+    if norm and not (_plain(delta, gamma) and _norm_operands(delta, h, gamma)):
         return None
-    if delta is not None and (not norm or delta.shape != h.shape or delta.stride(1) != 1 or delta.stride(0) % 8):
+    if delta is not None and not norm:
         return None
     if _qkv_stream(h.shape[0], h.shape[1], norm):
         return native().stream_qkv_rope(h, delta, gamma, float(eps), w, scale, cos, sin, pos, slots, k_cache, v_cache,
@@ -771,14 +782,9 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else _STREAM_N)
     if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
-    if h.stride(1) != 1 or w.shape[1] != K or w.shape[0] % 16:
-        return None
-    if gamma.dtype != torch.bfloat16 or not gamma.is_contiguous():
+    if w.shape[1] != K or w.shape[0] % 16 or not _norm_operands(delta, h, gamma):
         return None
     if not (_rows_ok(h, w, scale) if stream else _skinny_ok(h, w)):
-        return None
-    if delta is not None and (delta.shape != h.shape or delta.dtype != h.dtype or delta.stride(1) != 1
-                              or delta.stride(0) % 8):
         return None
     if stream:
         return native().stream_linear(h, delta, gamma, float(eps), w, scale, bool(swiglu))

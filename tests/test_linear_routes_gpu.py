@@ -79,3 +79,31 @@ def test_transforms_and_tracers_take_the_library(gpu, M):
     with mode:
         y = ops.linear(*fakes)
         assert y.shape == (M, N) and y.device == w.device
+
+
+def _odd_rows(gpu, kind, M, K):
+    """Rows whose layout the decode GEMMs do not read: overlapping, shorter apart than long, off 16-byte addresses."""
+    if kind == "expanded":
+        return _bf16(gpu, 1, K, seed=5).expand(M, K)
+    if kind == "overlapping":
+        return _bf16(gpu, M * 64 + K, seed=5).as_strided((M, K), (64, 1))
+    buf = _bf16(gpu, M * (K + 8) + 8, seed=5)
+    return buf[4:4 + M * (K + 8)].view(M, K + 8)[:, :K]
+
+
+@pytest.mark.parametrize("M", [2, 8, 16, 32, 64])
+@pytest.mark.parametrize("kind", ["expanded", "overlapping", "misaligned"])
+def test_odd_layouts_take_the_library(gpu, kind, M):
+    K, N = (2048, 4096) if M < 64 else (12288, 512)
+    w, x = _bf16(gpu, N, K, seed=1, std=0.03), _odd_rows(gpu, kind, M, K)
+    _close(ops.linear(x, w), x.double() @ w.double().t(), 2 ** -8)
+    wk = _odd_rows(gpu, kind, N, K)
+    _close(ops.linear(_bf16(gpu, M, K), wk), _bf16(gpu, M, K).double() @ wk.double().t(), 2 ** -8)
+    gamma = torch.ones(K, device=gpu).bfloat16()
+    for delta, h, v in ((x, _bf16(gpu, M, K), w), (None, x, w), (None, _bf16(gpu, M, K), wk)):
+        assert ops.norm_linear(delta, h, gamma, 1e-5, v) is None
+    if kind == "misaligned":
+        odd = torch.ones(K + 4, device=gpu).bfloat16()[4:]
+        assert ops.norm_linear(None, _bf16(gpu, M, K), odd, 1e-5, w) is None
+        q, s = torch.zeros(N, K, device=gpu, dtype=torch.uint8), torch.ones(N + 1, device=gpu)[1:]
+        assert ops.linear_swiglu(_bf16(gpu, M, K), q, s) is None
