@@ -789,7 +789,7 @@ attn_fwd_pp_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
   }
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   if (qrow < S) {
-    uint16_t* op = O + ((size_t)(SEG ? 0 : b) * S + row0 + qrow) * (size_t)ldo + (size_t)h * D;
+    uint16_t* op = O + ((size_t)b * S + qrow) * (size_t)ldo + (size_t)h * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -800,7 +800,7 @@ attn_fwd_pp_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ 
         for (int j = 0; j < 4; ++j) v4[j] = f2bf(o[db][4 * gq + j] * inv);
         *reinterpret_cast<u16x4*>(op + d) = v4;
       }
-    if (!SEG && hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
+    if (hh == 0) LSE[(size_t)(b * Hq + h) * S + qrow] = m_i + __log2f(l_tot);
   }
 }
 
