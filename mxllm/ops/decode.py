@@ -15,9 +15,15 @@ from ._ext import native, use_native
 
 
 def prefill_attention(qkv: torch.Tensor, cos, sin, write_kv, S: int, Hq: int, Hkv: int, D: int) -> torch.Tensor:
-    """One sequence (positions 0..S-1), CPU tensors (GPU: ``prompt_attention``, all sequences at once): RoPE,
-    hand the rotated K and V [Hkv, S, D] to ``write_kv(k, v)`` (the engine's KV cache), causal attention.
-    qkv [S, NH*D] -> o [S, Hq*D]."""
+    """One sequence (positions 0..S-1): RoPE, hand the rotated K and V [Hkv, S, D] to
+    ``write_kv(k, v)`` (a KV cache), causal attention.  qkv [S, NH*D] -> o [S, Hq*D].
+    (The engine's prompt passes on the GPU: ``prompt_attention``, all sequences at once.)"""
+    if use_native(qkv):
+        ops = native()
+        q, k, v = ops.rope_split(qkv.contiguous(), cos, sin, 1, S, Hq, Hkv, D, None)
+        write_kv(k[0], v[0])
+        o, _ = ops.attn_fwd(q, k, v, True, 1.0 / math.sqrt(D))
+        return o.view(S, Hq * D)
     x = qkv.view(1, S, Hq + 2 * Hkv, D)
     q = ref.apply_rope(x[:, :, :Hq], cos, sin)
     k = ref.apply_rope(x[:, :, Hq:Hq + Hkv], cos, sin)

@@ -1023,3 +1023,19 @@ def test_prompt_attention(gpu, D, Hq, Hkv, lens):
             vc2[int(bt[slot, j // blk]), :, :m] = v[0, :, j:j + m]
         at += n
     assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,Hq,Hkv,S", [(32, 4, 2, 1), (64, 8, 2, 300), (128, 8, 8, 129)])
+def test_prefill_attention_runs_the_kernels(gpu, D, Hq, Hkv, S):
+    """One sequence on the GPU: the bits of RoPE split and flash attention, K and V handed out as [Hkv, S, D]."""
+    from mxllm.ops.decode import prefill_attention
+
+    torch.manual_seed(D + S)
+    qkv = torch.randn(S, (Hq + 2 * Hkv) * D, device=gpu, dtype=torch.bfloat16)
+    cos, sin = ref.rope_tables(S, D, 500000.0, None, gpu)
+    kept = []
+    o = prefill_attention(qkv, cos, sin, lambda k, v: kept.extend((k, v)), S, Hq, Hkv, D)
+    q, k, v = _ops().rope_split(qkv, cos, sin, 1, S, Hq, Hkv, D, None)
+    assert torch.equal(kept[0], k[0]) and torch.equal(kept[1], v[0])
+    assert torch.equal(o, _ops().attn_fwd(q, k, v, True, D ** -0.5)[0].view(S, Hq * D))
