@@ -206,6 +206,7 @@ __device__ __forceinline__ int topkp_row(const T* __restrict__ x, int V, const S
       if (red[w2] > b || (red[w2] == b && redi[w2] < i)) { b = red[w2]; i = redi[w2]; }
   };
   argmax_reduce(best, bi);
+  if (bi >= V) bi = 0;  // no logit is a number
   if (!(temp > 0.f)) return bi;
   const float mx = best;
   const float c = 1.4426950408889634f / temp;  // exp2 domain

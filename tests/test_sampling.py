@@ -202,3 +202,21 @@ def test_gpu_split_sampler_draws(gpu, V, dtype, shape):
             assert got[i] == best, (i, temps[i], tops[i], ks[i])
             checked += 1
     assert checked > B // 5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [1000, 16384, 50257])
+@pytest.mark.parametrize("temp,p,k", [(0.8, 1.0, 0), (0.8, 0.9, 0), (0.8, 1.0, 40), (0.8, 0.9, 40), (0.0, 1.0, 0)])
+def test_gpu_sampler_without_numbers(gpu, V, temp, p, k):
+    """Rows that hold no number give token 0, never an id outside the vocabulary; tokens without a number are not
+    drawn; an infinite logit is.  Both forms of the sampler, beside a row that needs neither."""
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(5, V, generator=g)
+    x[0] = float("nan")
+    x[1] = float("-inf")
+    x[2, torch.rand(V, generator=g) < 0.1] = float("nan")
+    x[3, V // 2] = float("inf")
+    ids = dops.sample_rows(x.to(gpu), [temp] * 4 + [1.0], [p] * 5, [k] * 5, list(range(5)), [7] * 5).tolist()
+    assert ids[:2] == [0, 0] and ids[3] == V // 2 and 0 <= ids[4] < V
+    assert 0 <= ids[2] < V and not x[2, ids[2]].isnan()
+    assert temp > 0 or ids[2] == x[2].nan_to_num(-1e9).argmax()
