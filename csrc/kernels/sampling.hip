@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(kSampThreads) sample_topkp_kernel(const T* __r
 // Shorter rows: one workgroup, one launch.  32 top-p rows of 8,191: 30 us against 41 split; of 32,768: about 80
 // (its time grows with the row) against 47.
 constexpr int kSplitV = 16384;
-constexpr int kSplitMaxV = 1 << 22;  // 2^22 masses of up to 2^42 fit 64 bits
+constexpr int kSplitMaxV = (1 << 22) - 1;  // as many masses of up to 2^42 stay below 2^64
 constexpr int kMBins = 2048;
 constexpr int kMaxCh = 64;         // chunks a row (= one wave over their partials)
 constexpr int kListCap = 1024;     // listed tokens a row
@@ -414,7 +414,7 @@ __global__ void __launch_bounds__(kChThreads) samp_hist_kernel(const T* __restri
 // Where a row's cuts lie: tokens of bins below `all` are kept, those of bins all .. last and of bin `bk` (the one
 // the k-th token is in; kMBins: no top-k) are listed.
 struct RowCut {
-  int all, last, bk, none;
+  int all, last, bk;
 };
 // pm / pc [kMBins]: mass and count of the bins ahead of each; every thread of NT calls it
 template <int NT>
@@ -441,7 +441,7 @@ __device__ __forceinline__ RowCut row_cut(const SampWs& ws, int row, const SampR
     if (lane >= o) { im += y; in += z; }
   }
   if (lane == 63) { wm[wv] = im; wc[wv] = in; }
-  if (t == 0) *out = RowCut{0, kMBins - 1, hk ? kMBins - 1 : kMBins, 0};
+  if (t == 0) *out = RowCut{0, kMBins - 1, hk ? kMBins - 1 : kMBins};
   __syncthreads();
   unsigned long long bm = im - sm, tot = 0;
   uint32_t bn = in - sn;
@@ -504,7 +504,7 @@ __global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restri
   if (!(rp.temp > 0.f)) return;
   const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f;
   const RowScale rs = row_scale(ws, row, gridDim.x, rp.temp);
-  RowCut r{kMBins, kMBins - 1, kMBins, 0};
+  RowCut r{kMBins, kMBins - 1, kMBins};
   if (hk || hp) r = row_cut<kChThreads>(ws, row, rp, hk, hp, pm, pc, wm, wc, &cut);
   const float inv_t = 1.f / rp.temp;
   float gb = -INFINITY;

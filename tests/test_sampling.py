@@ -220,3 +220,18 @@ def test_gpu_sampler_without_numbers(gpu, V, temp, p, k):
     assert ids[:2] == [0, 0] and ids[3] == V // 2 and 0 <= ids[4] < V
     assert 0 <= ids[2] < V and not x[2, ids[2]].isnan()
     assert temp > 0 or ids[2] == x[2].nan_to_num(-1e9).argmax()
+
+
+def test_split_sampler_masses_fit():
+    """The split form takes no row whose masses, each up to 2^42, could sum to 2^64 (a total of zero restricts nothing);
+    it alone has a workspace."""
+    import ctypes
+
+    from mxllm.ops import _ext
+
+    if not _ext.available():
+        pytest.skip("native library not built")
+    ws = ctypes.CDLL(_ext.LIB).mx_sample_rows_ws
+    ws.restype = ctypes.c_int64
+    taken = [V for V in (1, 16383, 16384, (1 << 22) - 1, 1 << 22, 1 << 23) if ws(1, V) > 0]
+    assert taken == [16384, (1 << 22) - 1] and max(taken) << 42 < 1 << 64
