@@ -567,8 +567,10 @@ def normed_linear(x: torch.Tensor, h: torch.Tensor, nw: torch.Tensor, eps: float
 # (csrc/kernels/skinny_gemm.hip) where it beat hipBLASLt inside the decode step
 # (bench/serve_bench.py A/B, archive/profiles/r2x_skinny_gemm.md): one token row for every projection
 # and the LM head; 2..SKINNY_M rows for weights of <= 128 M elements (all Llama-3.1-8B
-# projections; the 70B ones lost at 4 rows).  MXLLM_SKINNY_M=0 keeps every GEMM on hipBLASLt.
+# projections; the 70B ones lost at 4 rows).  MXLLM_SKINNY_M set bounds the rows of every decode GEMM; 0 keeps all
+# forward GEMMs of inference on hipBLASLt.
 SKINNY_M = int(os.environ.get("MXLLM_SKINNY_M", "8"))
+_DECODE_M = SKINNY_M if "MXLLM_SKINNY_M" in os.environ else 32  # rows of the kernels that take more than skinny_gemm.hip
 _SKINNY_SMALL_W = 128 << 20
 # output channels below which 16 a workgroup leave some of the 256 CUs without one: 8 a workgroup (at 4096 and
 # more no gain)
@@ -613,7 +615,7 @@ def _rows_ok(x2: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = Non
 
 def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
     """Rows of K that csrc/kernels/stream_gemm.hip holds in LDS beside its partial sums (``norm``: and norms)."""
-    return SKINNY_M > 0 and 0 < M <= (4 if norm else 32) and K % 2048 == 0 and 16384 + 2 * M * (K + 8) <= 158 * 1024
+    return 0 < M <= min(4 if norm else 32, _DECODE_M) and K % 2048 == 0 and 16384 + 2 * M * (K + 8) <= 158 * 1024
 
 
 def _stream_wins(M: int, N: int, K: int) -> bool:
@@ -667,11 +669,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         return _LinearFn.apply(x, w)
     if not _plain(x, w):
         return F.linear(x, w)
-    if SKINNY_M > 0 and x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= 32:
+    if x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= _DECODE_M:
         y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
         if y is not None:
             return y.view(*x.shape[:-1], w.shape[0])
-    if x.is_cuda and x.dim() > 1:
+    if SKINNY_M > 0 and x.is_cuda and x.dim() > 1:
         N, K = w.shape
         M = x.numel() // max(K, 1)
         parts = gemm.rows_gain(M, N, K, True)
@@ -711,7 +713,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
 # do it once for all their channels, up to 4 rows and behind no weights (us, skinny -> stream, 1 / 2 / 4 rows: 28672 x
 # 4096 with SwiGLU 45.9 / 49.1 / 56.4 -> 42.3 / 42.8 / 43.7; 6144 x 4096 13.6 / 14.4 / 17.2 -> 13.1 / 13.8 / 15.0; 2048 x
 # 2048 5.0 / 5.5 / 6.8 -> 4.6 / 4.9 / 5.6): wherever it takes the shape and 2048 channels keep its workgroups busy.
+# MXLLM_NORM_FUSED_M set bounds both.
 NORM_M = int(os.environ.get("MXLLM_NORM_FUSED_M", "2"))
+_NORM_STREAM_M = NORM_M if "MXLLM_NORM_FUSED_M" in os.environ else 4
 
 
 def _norm_operands(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor) -> bool:
@@ -721,7 +725,7 @@ def _norm_operands(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Ten
 
 def _norm_stream(M: int, K: int) -> bool:
     """Whether the RMSNorm goes into stream_gemm.hip's prologue."""
-    return _stream_fits(M, K, True) and NORM_M > 0
+    return M <= _NORM_STREAM_M and _stream_fits(M, K, True)
 
 
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,

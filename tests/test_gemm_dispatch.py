@@ -2,6 +2,8 @@
 guard for multi-rank runs."""
 import os
 import socket
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -52,3 +54,18 @@ def test_persistent_gemm_is_world1_only():
         p.join(60)
         assert p.exitcode == 0
     assert got == {0: 4, 1: 4}
+
+
+@pytest.mark.parametrize("env,rows,norm_rows", [({}, 32, 4), ({"MXLLM_SKINNY_M": "0"}, 0, 0), ({"MXLLM_SKINNY_M": "3"}, 3, 3),
+                                                ({"MXLLM_SKINNY_M": "16"}, 16, 4), ({"MXLLM_NORM_FUSED_M": "1"}, 32, 1),
+                                                ({"MXLLM_NORM_FUSED_M": "0"}, 32, 0)])
+def test_switches_bound_every_decode_gemm(env, rows, norm_rows):
+    """MXLLM_SKINNY_M and MXLLM_NORM_FUSED_M are upper limits for the rows of all decode kernels where they are set."""
+    code = ("import sys; import mxllm.ops; m = sys.modules['mxllm.ops.linear']; r = range(1, 40); "
+            "print(max([M for M in r if m._stream_fits(M, 2048)], default=0), "
+            "max([M for M in r if m._norm_stream(M, 2048)], default=0), m._DECODE_M)")
+    base = {k: v for k, v in os.environ.items() if k not in ("MXLLM_SKINNY_M", "MXLLM_NORM_FUSED_M")}
+    out = subprocess.run([sys.executable, "-c", code], env={**base, **env}, capture_output=True, text=True, timeout=300,
+                         cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert out.returncode == 0, out.stderr[-2000:]
+    assert [int(v) for v in out.stdout.split()] == [rows, norm_rows, rows]

@@ -1,5 +1,7 @@
 """What the inference kernels behind ``ops.linear`` and its fused forms must not take: they have neither derivatives nor
 batching rules, and read whole 16-byte pieces of dense rows."""
+import sys
+
 import pytest
 import torch
 
@@ -107,3 +109,15 @@ def test_odd_layouts_take_the_library(gpu, kind, M):
         assert ops.norm_linear(None, _bf16(gpu, M, K), odd, 1e-5, w) is None
         q, s = torch.zeros(N, K, device=gpu, dtype=torch.uint8), torch.ones(N + 1, device=gpu)[1:]
         assert ops.linear_swiglu(_bf16(gpu, M, K), q, s) is None
+
+
+@pytest.mark.parametrize("M", [1, 16, 64])
+def test_switch_off_is_the_library(gpu, M, monkeypatch):
+    """MXLLM_SKINNY_M=0: no forward GEMM of inference runs on a kernel of ours."""
+    lin = sys.modules["mxllm.ops.linear"]
+    monkeypatch.setattr(lin, "SKINNY_M", 0)
+    monkeypatch.setattr(lin, "_DECODE_M", 0)
+    monkeypatch.setattr(lin, "native", lambda: pytest.fail("a kernel was asked for"))
+    x, w = _bf16(gpu, M, 12288), _bf16(gpu, 512, 12288, seed=1, std=0.03)
+    _close(ops.linear(x, w), x.double() @ w.double().t(), 2 ** -8)
+    assert ops.linear_swiglu(x, w) is None and ops.norm_linear(None, x, x[0].contiguous(), 1e-5, w) is None
