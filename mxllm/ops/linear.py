@@ -572,9 +572,11 @@ def normed_linear(x: torch.Tensor, h: torch.Tensor, nw: torch.Tensor, eps: float
 SKINNY_M = int(os.environ.get("MXLLM_SKINNY_M", "8"))
 _DECODE_M = SKINNY_M if "MXLLM_SKINNY_M" in os.environ else 32  # rows of the kernels that take more than skinny_gemm.hip
 _SKINNY_SMALL_W = 128 << 20
-# output channels below which 16 a workgroup leave some of the 256 CUs without one: 8 a workgroup (at 4096 and
-# more no gain)
-_HALF_N = 4096
+# Output channels up to which 8 a workgroup leave every one of the 256 CUs at most one (us, 16 a workgroup -> 8: 2048 x
+# 2048, 1 / 8 rows 4.6 / 5.3 -> 3.9 / 4.5; 2048 x 8192 13.4 / 15.1 -> 9.2 / 11.7).  More channels are a second turn for
+# some: 3072 x 2048, 1 / 8 rows 5.1 / 5.7 -> 5.3 / 6.6, 2304 x 8192, 8 rows 15.2 -> 19.3; one row of a longer K gains even
+# so, below the channels whose groups of 16 fill the CUs: 3584 x 3072 7.6 -> 7.0, 4080 x 4096 9.6 -> 8.6.
+_HALF_N, _HALF_N1, _HALF_K1 = 2048, 4096, 3072
 
 
 def _dense_rows(t: torch.Tensor) -> bool:
@@ -638,18 +640,28 @@ def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Ten
     return native().w8_linear(x2, q, scale)
 
 
-def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
-    M, (N, K) = x2.shape[0], w.shape
+def _decode_route(M: int, N: int, K: int) -> str:
+    """The decode GEMM of M rows of K times [N, K]: "stream" (stream_gemm.hip), "half" or "skinny" (skinny_gemm.hip, 8 or
+    16 channels a workgroup), or "" (hipBLASLt)."""
     if _stream_wins(M, N, K):
-        return native().stream_linear(x2, None, None, 0.0, w, None, False)[0] if _rows_ok(x2, w) else None
+        return "stream"
+    if K % 512:
+        return ""
     if M <= SKINNY_M:
-        # many rows of a large weight outside the kernel above: hipBLASLt
-        ok = _skinny_ok(x2, w) or (M * K < _STREAM_MK and K % 512 == 0 and _rows_ok(x2, w))
-        half = N < _HALF_N and K % 1024 == 0 and M <= 8
-        return (native().skinny_linear_half if half else native().skinny_linear)(x2, w) if ok else None
-    if M * K <= _WIDE_MK and N <= _WIDE_N and K % 512 == 0 and _rows_ok(x2, w):
-        return native().skinny_linear(x2, w)
-    return None
+        if M > 1 and N * K > _SKINNY_SMALL_W and M * K >= _STREAM_MK:
+            return ""
+        half = N <= _HALF_N or (M == 1 and N < _HALF_N1 and K >= _HALF_K1)
+        return "half" if half and K % 1024 == 0 and M <= 8 else "skinny"
+    return "skinny" if M * K <= _WIDE_MK and N <= _WIDE_N else ""
+
+
+def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    route = _decode_route(x2.shape[0], *w.shape)
+    if not route or not _rows_ok(x2, w):
+        return None
+    if route == "stream":
+        return native().stream_linear(x2, None, None, 0.0, w, None, False)[0]
+    return (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
 
 
 def _plain(*ts: torch.Tensor | None) -> bool:

@@ -9,6 +9,7 @@ import pytest
 import torch
 import torch.multiprocessing as mp
 
+import mxllm.ops  # noqa: F401
 from mxllm.ops import gemm
 
 
@@ -69,3 +70,16 @@ def test_switches_bound_every_decode_gemm(env, rows, norm_rows):
                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     assert out.returncode == 0, out.stderr[-2000:]
     assert [int(v) for v in out.stdout.split()] == [rows, norm_rows, rows]
+
+
+# (M, N, K): both sides of each line of the decode GEMMs' dispatch, as measured beside it in mxllm/ops/linear.py
+DECODE_ROUTES = {
+    "half": [(1, 2048, 2048), (8, 2048, 8192), (1, 3584, 3072), (8, 512, 4096)],
+    "skinny": [(1, 3072, 2048), (8, 3072, 2048), (2, 3584, 3072), (8, 2064, 8192), (1, 4096, 3072), (4, 512, 1536)],
+}
+
+
+@pytest.mark.parametrize("route,M,N,K", [(r, *s) for r, sizes in DECODE_ROUTES.items() for s in sizes])
+def test_decode_routes(route, M, N, K):
+    lin = sys.modules["mxllm.ops.linear"]
+    assert lin._decode_route(M, N, K) == route
