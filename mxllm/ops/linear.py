@@ -602,10 +602,18 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 # 18.0 with SwiGLU against hipBLASLt's 19.6; 8192 x 2048, 8 rows 9.2 -> 10.4, 24 rows 14.2 -> 11.2 (hipBLASLt 13.2).
 # Past 8 rows also with few channels: 2048 x 4096, 16 rows 10.3 -> 9.1; 2048 x 2048, 12 / 32 rows 5.8 / 8.7 -> 5.8 / 7.5.
 _STREAM_MK, _STREAM_N, _STREAM_N4, _STREAM_N2 = 16384, 8192, 6144, 32768
-# Rows x width up to which a projection of at most 4096 channels (one group a CU) that the kernel above does not take
-# runs on skinny_gemm.hip past SKINNY_M rows: 4096 x 4096, 16 rows 11.2 us against hipBLASLt's 15.6, 24 rows 14.5 against 13.4; 3072 x 2048,
-# 32 rows 9.1 against 11.7.
-_WIDE_MK, _WIDE_N = 65536, 4096
+# Past SKINNY_M rows the kernel of 16 channels a workgroup keeps projections of at most 4096 channels (one group a CU) that
+# the one above does not take: of up to 16 rows where the rows' fragments stay few, and from 768 channels on (us, hipBLASLt
+# -> here: 1024 x 2048, 9 / 32 rows 8.4 / 8.5 -> 5.3 / 7.9; 4096 x 1536, 32 rows 9.8 -> 7.7; 3072 x 3072, 16 rows 12.6 -> 8.4;
+# 64 x 2048, 16 rows 5.5 -> 5.4).  Beyond, each workgroup's walk over the rows is what lasts: 64 x 2048, 24 rows 5.5 -> 6.7;
+# 1024 x 4096, 32 rows 8.9 -> 13.3; 2560 x 2560, 24 rows 9.6 -> 10.5; 1024 x 6144, 9 rows 10.5 -> 11.7.
+_WIDE_N = 4096
+
+
+def _wide_wins(M: int, N: int, K: int) -> bool:
+    if N > _WIDE_N:
+        return False
+    return (M <= 16 and M * K <= 32768) or (N >= 768 and (K <= 2048 or (K <= 4096 and M * K <= 49152)))
 
 
 def _rows_ok(x2: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> bool:
@@ -652,7 +660,7 @@ def _decode_route(M: int, N: int, K: int) -> str:
             return ""
         half = N <= _HALF_N or (M == 1 and N < _HALF_N1 and K >= _HALF_K1)
         return "half" if half and K % 1024 == 0 and M <= 8 else "skinny"
-    return "skinny" if M * K <= _WIDE_MK and N <= _WIDE_N else ""
+    return "skinny" if M <= _DECODE_M and _wide_wins(M, N, K) else ""
 
 
 def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:

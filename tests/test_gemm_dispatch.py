@@ -75,7 +75,10 @@ def test_switches_bound_every_decode_gemm(env, rows, norm_rows):
 # (M, N, K): both sides of each line of the decode GEMMs' dispatch, as measured beside it in mxllm/ops/linear.py
 DECODE_ROUTES = {
     "half": [(1, 2048, 2048), (8, 2048, 8192), (1, 3584, 3072), (8, 512, 4096)],
-    "skinny": [(1, 3072, 2048), (8, 3072, 2048), (2, 3584, 3072), (8, 2064, 8192), (1, 4096, 3072), (4, 512, 1536)],
+    "skinny": [(1, 3072, 2048), (8, 3072, 2048), (2, 3584, 3072), (8, 2064, 8192), (1, 4096, 3072), (4, 512, 1536),
+               (16, 64, 2048), (32, 1024, 2048), (32, 4096, 1536), (16, 3072, 3072), (12, 1024, 4096)],
+    "": [(17, 64, 2048), (32, 512, 1024), (16, 64, 4096), (13, 1024, 4096), (20, 2560, 2560), (9, 1024, 6144),
+         (9, 4112, 1536), (33, 1024, 2048)],
 }
 
 
