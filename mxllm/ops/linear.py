@@ -595,13 +595,20 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # Where a projection goes to the workgroups that stay (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of
-# once 16 channels).  A K of 4096s, whose blocks are long: from 6144 channels on at any rows (us, skinny -> stream,
-# 6144 x 4096, 1 row 14.6 -> 13.6, 8 rows 15.7 -> 13.5; 28672 x 4096, 1 / 16 rows 43.6 / 67 -> 42.6 / 43.8; 4096 x 4096
-# level), an LM head from 2 rows on (128256 x 4096, 1 row 173 -> 175, 4 rows 192 -> 178).  Else by rows x width, the X
-# that the others read beside 16 channels of weights: 16384 x 2048, 4 rows 15.0 -> 15.6, 8 rows 16.8 -> 15.3, 32 rows
-# 18.0 with SwiGLU against hipBLASLt's 19.6; 8192 x 2048, 8 rows 9.2 -> 10.4, 24 rows 14.2 -> 11.2 (hipBLASLt 13.2).
-# Past 8 rows also with few channels: 2048 x 4096, 16 rows 10.3 -> 9.1; 2048 x 2048, 12 / 32 rows 5.8 / 8.7 -> 5.8 / 7.5.
-_STREAM_MK, _STREAM_N, _STREAM_N4, _STREAM_N2 = 16384, 8192, 6144, 32768
+# once 16 channels), as far as X fits the LDS (32 rows of 2048, 17 of 4096, 11 of 6144, 8 of 8192, 5 of 14336).
+#  * Up to 8 rows (us, skinny -> stream): a K of 4096s, whose blocks are long, from 6144 channels on (6144 x 4096, 1 / 8
+#    rows 14.6 / 15.9 -> 13.6 / 13.7; 28672 x 4096, 1 row 43.6 -> 42.6; 4096 x 4096 level), an LM head from 2 rows on (128256 x
+#    4096, 1 row 173 -> 175, 4 rows 192 -> 178).  Else by rows x width, the X that the other reads beside 16 channels
+#    of weights: 8192 x 6144, 8 rows 24.4 -> 22.3; a K of 2048 at 8 rows with enough channels to spread the end (28672
+#    26.4 -> 24.8, 16384 15.7 -> 16.1, 8192 9.1 -> 10.4; with SwiGLU 16384 15.6 -> 15.2, 8192 9.5 -> 10.2).
+#  * Past 8 rows (hipBLASLt -> stream): a K of 2048 at any width (2048 x 2048, 12 / 32 rows 8.5 / 8.6 -> 5.3 / 7.1; 128256, 32
+#    rows 111 -> 104), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 17.1 / 16.8 -> 17.3 / 17.9;
+#    14336 15.8 / 15.7 -> 16.7 / 17.7; 20480 22.0 / 22.1 -> 20.4 / 21.1), which gain with SwiGLU only (19.2 -> 18.0).  A K of 4096 up
+#    to 16 rows (2048 x 4096 and wider; 12288, 16 rows 26.7 -> 21.0), a 17th only where there is much to stream (16384 30.7 ->
+#    29.2, 12288 22.2 -> 24.1).  Longer ones from 12288 channels on (12288 x 6144, 9 rows 35.5 -> 32.2, 6144 18.4 -> 20.2).
+_STREAM_MK, _STREAM_N4, _STREAM_N2 = 16384, 6144, 32768
+
+
 # Past SKINNY_M rows the kernel of 16 channels a workgroup keeps projections of at most 4096 channels (one group a CU) that
 # the one above does not take: of up to 16 rows where the rows' fragments stay few, and from 768 channels on (us, hipBLASLt
 # -> here: 1024 x 2048, 9 / 32 rows 8.4 / 8.5 -> 5.3 / 7.9; 4096 x 1536, 32 rows 9.8 -> 7.7; 3072 x 3072, 16 rows 12.6 -> 8.4;
@@ -628,14 +635,18 @@ def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
     return 0 < M <= min(4 if norm else 32, _DECODE_M) and K % 2048 == 0 and 16384 + 2 * M * (K + 8) <= 158 * 1024
 
 
-def _stream_wins(M: int, N: int, K: int) -> bool:
+def _stream_wins(M: int, N: int, K: int, swiglu: bool = False) -> bool:
     if not _stream_fits(M, K):
         return False
-    if M > 8 and N >= 2048:
-        return True
+    if M > 8:
+        if K > 4096:
+            return N >= 12288
+        if K == 4096:
+            return N >= (2048 if M <= 16 else 16384)
+        return N >= 2048 and (swiglu or M <= 16 or not 12288 < N < 20480)
     if K % 4096 == 0 and N >= _STREAM_N4:
         return M > 1 or N < _STREAM_N2
-    return N >= _STREAM_N and M * K >= _STREAM_MK
+    return M * K >= _STREAM_MK and N >= (8192 if K > 2048 else 10240 if swiglu else 20480)
 
 
 def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
@@ -717,7 +728,7 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
         if not (_stream_fits(*x.shape) and _rows_ok(x, w, scale)):
             return None
         return native().stream_linear(x, None, None, 0.0, w, scale, True)[0]
-    if _stream_wins(x.shape[0], *w.shape) and _rows_ok(x, w):
+    if _stream_wins(x.shape[0], *w.shape, True) and _rows_ok(x, w):
         return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
     if 0 < x.shape[0] <= SKINNY_M and _skinny_ok(x, w):
         return native().skinny_linear_swiglu(x, w)
@@ -803,7 +814,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     if SKINNY_M <= 0 or h.dim() != 2 or not _plain(delta, h, gamma, w):
         return None
     M, K = h.shape
-    stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else _STREAM_N)
+    stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else 8192)
     if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
     if w.shape[1] != K or w.shape[0] % 16 or not _norm_operands(delta, h, gamma):

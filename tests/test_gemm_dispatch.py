@@ -74,10 +74,14 @@ def test_switches_bound_every_decode_gemm(env, rows, norm_rows):
 
 # (M, N, K): both sides of each line of the decode GEMMs' dispatch, as measured beside it in mxllm/ops/linear.py
 DECODE_ROUTES = {
+    "stream": [(1, 6144, 4096), (2, 128256, 4096), (8, 20480, 2048), (8, 8192, 6144), (9, 2048, 2048), (32, 12288, 2048),
+               (16, 16384, 2048), (32, 20480, 2048), (16, 2048, 4096), (17, 16384, 4096), (9, 12288, 6144)],
     "half": [(1, 2048, 2048), (8, 2048, 8192), (1, 3584, 3072), (8, 512, 4096)],
     "skinny": [(1, 3072, 2048), (8, 3072, 2048), (2, 3584, 3072), (8, 2064, 8192), (1, 4096, 3072), (4, 512, 1536),
-               (16, 64, 2048), (32, 1024, 2048), (32, 4096, 1536), (16, 3072, 3072), (12, 1024, 4096)],
-    "": [(17, 64, 2048), (32, 512, 1024), (16, 64, 4096), (13, 1024, 4096), (20, 2560, 2560), (9, 1024, 6144),
+               (16, 64, 2048), (32, 1024, 2048), (32, 4096, 1536), (16, 3072, 3072), (12, 1024, 4096),
+               (8, 16384, 2048), (8, 4096, 4096), (1, 128256, 4096), (4, 16384, 2048)],
+    "": [(17, 16384, 2048), (32, 14336, 2048), (17, 12288, 4096), (18, 28672, 4096), (9, 6144, 6144), (9, 28672, 8192),
+         (17, 64, 2048), (32, 512, 1024), (16, 64, 4096), (13, 1024, 4096), (20, 2560, 2560), (9, 1024, 6144),
          (9, 4112, 1536), (33, 1024, 2048)],
 }
 
@@ -86,3 +90,10 @@ DECODE_ROUTES = {
 def test_decode_routes(route, M, N, K):
     lin = sys.modules["mxllm.ops.linear"]
     assert lin._decode_route(M, N, K) == route
+
+
+def test_swiglu_route_of_decode_rows():
+    """With SwiGLU in the epilogue the GEMM that stays gains from fewer channels on, and past 16 rows at any."""
+    wins = sys.modules["mxllm.ops.linear"]._stream_wins
+    assert wins(8, 10240, 2048, True) and not wins(8, 8192, 2048, True) and not wins(8, 10240, 2048)
+    assert wins(32, 16384, 2048, True) and not wins(32, 16384, 2048) and not wins(33, 16384, 2048, True)
