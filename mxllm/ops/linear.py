@@ -571,6 +571,9 @@ def normed_linear(x: torch.Tensor, h: torch.Tensor, nw: torch.Tensor, eps: float
 # forward GEMMs of inference on hipBLASLt.
 SKINNY_M = int(os.environ.get("MXLLM_SKINNY_M", "8"))
 _DECODE_M = SKINNY_M if "MXLLM_SKINNY_M" in os.environ else 32  # rows of the kernels that take more than skinny_gemm.hip
+# Larger weights that the kernel with its rows in LDS does not take: up to 5 rows of 2048, 8192 / K of longer ones (us,
+# hipBLASLt -> skinny: 128256 x 2048, 2 / 5 rows 95.6 / 92.2 -> 88.6 / 89.7, 7 rows 92.4 -> 99.1; 128256 x 1536, 4 / 6 rows 72.1 /
+# 72.2 -> 70.8 / 76.4; 65536 x 2560, 2 / 5 rows 61.8 / 59.6 -> 60.7 / 65.0).
 _SKINNY_SMALL_W = 128 << 20
 # Output channels up to which 8 a workgroup leave every one of the 256 CUs at most one (us, 16 a workgroup -> 8: 2048 x
 # 2048, 1 / 8 rows 4.6 / 5.3 -> 3.9 / 4.5; 2048 x 8192 13.4 / 15.1 -> 9.2 / 11.7).  More channels are a second turn for
@@ -667,7 +670,7 @@ def _decode_route(M: int, N: int, K: int) -> str:
     if K % 512:
         return ""
     if M <= SKINNY_M:
-        if M > 1 and N * K > _SKINNY_SMALL_W and M * K >= _STREAM_MK:
+        if M > 1 and N * K > _SKINNY_SMALL_W and not (M <= 5 and M * K <= (10240 if K <= 2048 else 8192)):
             return ""
         half = N <= _HALF_N or (M == 1 and N < _HALF_N1 and K >= _HALF_K1)
         return "half" if half and K % 1024 == 0 and M <= 8 else "skinny"
