@@ -80,7 +80,7 @@ DECODE_ROUTES = {
     "skinny": [(1, 3072, 2048), (8, 3072, 2048), (2, 3584, 3072), (8, 2064, 8192), (1, 4096, 3072), (4, 512, 1536),
                (16, 64, 2048), (32, 1024, 2048), (32, 4096, 1536), (16, 3072, 3072), (12, 1024, 4096),
                (8, 16384, 2048), (8, 4096, 4096), (1, 128256, 4096), (4, 16384, 2048),
-               (5, 128256, 2048), (3, 65536, 2560), (5, 128256, 1536), (8, 65536, 2048)],
+               (5, 128256, 2048), (3, 65536, 2560), (5, 128256, 1536), (7, 65536, 2048)],
     "": [(6, 128256, 2048), (4, 65536, 2560), (6, 128256, 1536), (17, 16384, 2048), (32, 14336, 2048), (17, 12288, 4096), (18, 28672, 4096), (9, 6144, 6144), (9, 28672, 8192),
          (17, 64, 2048), (32, 512, 1024), (16, 64, 4096), (13, 1024, 4096), (20, 2560, 2560), (9, 1024, 6144),
          (9, 4112, 1536), (33, 1024, 2048)],
