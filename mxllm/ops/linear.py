@@ -773,17 +773,20 @@ def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq
     if not (cos.dtype == torch.float32 and cos.is_contiguous() and sin.is_contiguous() and k_cache.is_contiguous()
             and v_cache.is_contiguous()):
         return False
-    if _qkv_stream(M, K, norm):
+    if _qkv_stream(M, K, norm, D, scale is not None):
         return _rows_ok(h, w, scale)
     if scale is not None or D != 128 or not 0 < M <= (min(NORM_M, SKINNY_M) if norm else SKINNY_M):
         return False
     return bool((not norm or M * K <= 32768) and _skinny_ok(h, w))
 
 
-def _qkv_stream(M: int, K: int, norm: bool) -> bool:
-    """Whether the QKV projection goes to stream_gemm.hip (us, skinny -> stream, 6144 x 4096 without norm: 1 row 13.9 ->
-    13.1, 4 rows 14.8 -> 13.7, 8 rows 16.2 -> 14.6); bf16 heads of 128 whose K it does not take to skinny_gemm.hip."""
-    return _norm_stream(M, K) if norm else _stream_fits(M, K)
+def _qkv_stream(M: int, K: int, norm: bool, D: int, f8: bool) -> bool:
+    """Whether the QKV projection goes to stream_gemm.hip; what it leaves, bf16 heads of 128 up to 8 rows, to
+    skinny_gemm.hip.  (us, skinny -> stream, 6144 x 4096 without norm: 1 row 15.2 -> 14.4, 8 rows 16.4 -> 14.9; 3072 x 2048,
+    heads of 128, 5.5 -> 6.1 and 6.2 -> 6.4, with the norm 5.9 -> 5.5; 17 rows of 4096 18.1 -> 18.6.)"""
+    if norm:
+        return _norm_stream(M, K)
+    return _stream_fits(M, K) and (K == 2048 or M <= 16) and (f8 or D != 128 or K > 2048 or M > 8)
 
 
 def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, cos, sin, pos, slots, k_cache,
@@ -800,7 +803,7 @@ def qkv_rope_linear(delta, h: torch.Tensor, gamma, eps: float, w: torch.Tensor, 
         return None
     if delta is not None and not norm:
         return None
-    if _qkv_stream(h.shape[0], h.shape[1], norm):
+    if _qkv_stream(*h.shape, norm, k_cache.shape[-1], scale is not None):
         return native().stream_qkv_rope(h, delta, gamma, float(eps), w, scale, cos, sin, pos, slots, k_cache, v_cache,
                                         Hq, Hkv, block_table)
     return native().skinny_qkv_rope(h, delta, gamma, float(eps), w, cos, sin, pos, slots, k_cache, v_cache, Hq, Hkv,

@@ -98,3 +98,13 @@ def test_swiglu_route_of_decode_rows():
     wins = sys.modules["mxllm.ops.linear"]._stream_wins
     assert wins(8, 10240, 2048, True) and not wins(8, 8192, 2048, True) and not wins(8, 10240, 2048)
     assert wins(32, 16384, 2048, True) and not wins(32, 16384, 2048) and not wins(33, 16384, 2048, True)
+
+
+def test_qkv_route_of_decode_rows():
+    stream = sys.modules["mxllm.ops.linear"]._qkv_stream
+    for M, K, norm, D, f8, want in ((1, 4096, False, 128, False, True), (8, 2048, False, 128, False, False),
+                                    (9, 2048, False, 128, False, True), (1, 2048, True, 128, False, True),
+                                    (1, 2048, False, 64, False, True), (8, 2048, False, 128, True, True),
+                                    (16, 4096, False, 128, False, True), (17, 4096, False, 128, False, False),
+                                    (5, 4096, True, 128, False, False)):
+        assert stream(M, K, norm, D, f8) == want, (M, K, norm, D, f8)
