@@ -746,7 +746,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
 # 3.83 -> 4.04 ms (archive/profiles/r2s3_decode_ab/); the kernel takes up to 4.  stream_gemm.hip's workgroups
 # do it once for all their channels, up to 4 rows and behind no weights (us, skinny -> stream, 1 / 2 / 4 rows: 28672 x
 # 4096 with SwiGLU 45.9 / 49.1 / 56.4 -> 42.3 / 42.8 / 43.7; 6144 x 4096 13.6 / 14.4 / 17.2 -> 13.1 / 13.8 / 15.0; 2048 x
-# 2048 5.0 / 5.5 / 6.8 -> 4.6 / 4.9 / 5.6): wherever it takes the shape and 2048 channels keep its workgroups busy.
+# 2048 5.0 / 5.5 / 6.8 -> 4.6 / 4.9 / 5.6): where it takes the shape, for 2048 channels and more.  A long K of as few
+# channels gains only past 2 rows (4096 x 4096, 1 / 4 rows 9.3 / 13.0 -> 9.7 / 11.2; 8192 x 8192 26.0 / 31.2 -> 26.8 / 30.5), and past
+# 8192 not at all (4096 x 14336, 4 rows 31.5 -> 34.0).
 # MXLLM_NORM_FUSED_M set bounds both.
 NORM_M = int(os.environ.get("MXLLM_NORM_FUSED_M", "2"))
 _NORM_STREAM_M = NORM_M if "MXLLM_NORM_FUSED_M" in os.environ else 4
@@ -760,6 +762,10 @@ def _norm_operands(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Ten
 def _norm_stream(M: int, K: int) -> bool:
     """Whether the RMSNorm goes into stream_gemm.hip's prologue."""
     return M <= _NORM_STREAM_M and _stream_fits(M, K, True)
+
+
+def _norm_wins(M: int, N: int, K: int) -> bool:
+    return N >= 2048 and (N > K or K < 4096 or (M > 2 and K <= 8192))
 
 
 def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq: int, Hkv: int,
@@ -820,7 +826,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     if SKINNY_M <= 0 or h.dim() != 2 or not _plain(delta, h, gamma, w):
         return None
     M, K = h.shape
-    stream = _norm_stream(M, K) and w.shape[0] >= (2048 if scale is None else 8192)
+    stream = _norm_stream(M, K) and (_norm_wins(M, w.shape[0], K) if scale is None else w.shape[0] >= 8192)
     if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
     if w.shape[1] != K or w.shape[0] % 16 or not _norm_operands(delta, h, gamma):

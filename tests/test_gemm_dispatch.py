@@ -108,3 +108,10 @@ def test_qkv_route_of_decode_rows():
                                     (16, 4096, False, 128, False, True), (17, 4096, False, 128, False, False),
                                     (5, 4096, True, 128, False, False)):
         assert stream(M, K, norm, D, f8) == want, (M, K, norm, D, f8)
+
+
+def test_norm_route_of_decode_rows():
+    wins = sys.modules["mxllm.ops.linear"]._norm_wins
+    yes = [(1, 2048, 2048), (4, 3072, 2048), (1, 6144, 4096), (4, 4096, 4096), (3, 8192, 8192), (1, 10240, 8192)]
+    no = [(1, 1024, 2048), (2, 4096, 4096), (1, 8192, 8192), (4, 4096, 14336), (1, 2048, 8192)]
+    assert [s for s in yes if not wins(*s)] == [] and [s for s in no if wins(*s)] == []
