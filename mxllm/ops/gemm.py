@@ -126,6 +126,10 @@ def _gains(form: str, M: int, N: int, K: int) -> bool:
       * a K that is no multiple of 64, which hipBLASLt reads slowly: 16384 x 2048, 3606: 271 -> 179;
       * else a last wave that is full enough.  One wave: 144 tiles 4096: 89 -> 77, 8192: 161 -> 146 (128 tiles 77 ->
         78 and 144 -> 154).  More: 256 tiles 118 -> 98, 512 237 -> 200, 384 172 -> 167 (288 tiles 149 -> 160).
+    But not where there is little to save: a long K in multiples of 8 on 64 tiles (2048 x 2048, 3608 75 -> 74, 5160 93 -> 97,
+    5600 93 -> 104), and round token counts of very many tiles, whose transposes are small beside the product or whose
+    time is the output's (57344 x 8192, 256 520 -> 595, 1536 1270 -> 1355; 8192 x 28672, 2304 840 -> 880; 128256 x 2048, 256 320 ->
+    355, but 768 553 -> 528 and 5120 2542 -> 2054).
     ``nn``: :func:`_gains_nn`."""
     tiles = (M // 256) * (N // 256)
     # past the kernel's 32-bit offsets (it would decline: the caller's other path stays)
@@ -133,6 +137,10 @@ def _gains(form: str, M: int, N: int, K: int) -> bool:
         return False
     if form == "tt":
         full = _wave_fill(tiles)
+        if K % 64 == 0 and tiles >= 3584 and (min(M, N) >= 8192 or K <= 512):
+            return False
+        if K % 8 == 0 and K > 4096 and tiles < 96:
+            return False
         return K <= 1536 or (K % 64 != 0 and tiles >= 64) or (tiles >= 144 and full >= (0.56 if tiles <= CUS else 0.7))
     return form == "nn" and _gains_nn(tiles)
 

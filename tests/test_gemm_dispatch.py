@@ -115,3 +115,14 @@ def test_norm_route_of_decode_rows():
     yes = [(1, 2048, 2048), (4, 3072, 2048), (1, 6144, 4096), (4, 4096, 4096), (3, 8192, 8192), (1, 10240, 8192)]
     no = [(1, 1024, 2048), (2, 4096, 4096), (1, 8192, 8192), (4, 4096, 14336), (1, 2048, 8192)]
     assert [s for s in yes if not wins(*s)] == [] and [s for s in no if wins(*s)] == []
+
+
+def test_weight_gradient_rule():
+    """Both sides of the lines that mxllm/ops/gemm.py draws for weight gradients outside the table (M, N, tokens)."""
+    def on(M, N, T):
+        return gemm._gains("tt", M, N, T)
+
+    assert on(2048, 2048, 300) and on(2048, 2048, 3608) and on(2048, 2048, 5161) and on(3072, 2048, 5600)
+    assert not on(2048, 2048, 4104) and not on(2048, 2048, 5600)
+    assert on(128256, 2048, 768) and on(128256, 4096, 1280) and on(57344, 8192, 1537) and on(16384, 4096, 2304)
+    assert not on(57344, 8192, 256) and not on(57344, 8192, 1536) and not on(8192, 28672, 2304) and not on(128256, 2048, 512)
