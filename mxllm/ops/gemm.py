@@ -177,27 +177,41 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
     In parts where the tiles leave half the CUs without one and K is long; each part costs its fp32 image's trip (us,
     library -> gemm8; K x N at rows):
       * projections (``b_kc``): K of 12,288 and 64 rows on.  14336 x 4096 at 64 35 -> 31, 128 59 -> 36, 400 80 -> 57,
-        1000 122 -> 97, 2048 191 -> 171; 28672 x 8192 at 200 312 -> 122 (14336 x 4096 at 48 28 -> 30; 8192 x 2048 at
-        512 29 -> 37, 2048 69 -> 67);
+        1000 122 -> 97, 2048 191 -> 171; 28672 x 8192 at 200 312 -> 122, 512 327 -> 192 (14336 x 4096 at 48 28 -> 30; 8192 x
+        2048 at 512 29 -> 37, 2048 69 -> 67); in two or three parts not past a K of 24,576 (28672 x 8192 at 559 277 -> 315,
+        768 304 -> 321);
       * input gradients: K of 6144 on.  16384 x 2048 at 1000 124 -> 68, 4096 237 -> 211; 6144 x 4096 at 512 53 -> 43
         (3072 x 2048 at 512 26 -> 30).
     Whole, where the library, which is tuned for round numbers of rows, falls behind between them:
       * projections (``b_kc``) of K 8192 and more from 500 tiles on: 8192 x 57344 at 700 559 -> 530, 2600 1916 -> 1740;
-        8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321).  With a shorter K the library is up to 27 %
+        8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321), up to 4096 tiles (8192 x 128256 at 1700 2650 ->
+        2550, 2210 3378 -> 3555, 4445 6338 -> 6656).  With a shorter K the library is up to 27 %
         slower at some row counts and 3 to 6 % faster at others (4096 x 28672 at 2700 543 -> 441, 4003 600 -> 634);
-      * input gradients: :func:`_gains_nn`;
+      * input gradients: :func:`_gains_nn`, with the last tile's rows not mostly padding (8192 -> 28672 at
+        300 175 -> 184, 371 180 -> 190, 408 0.92);
       * gate-up with SwiGLU, which saves the projection's trip through HBM at any size: where the last tile's rows are
         not mostly padding and five eighths of the CUs have a tile.  2048 x 16384 at 700 48 -> 42, 2600 205 -> 142, 4096
-        236 -> 198 (512, 128 tiles: 38 -> 40); 4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 1025 249 -> 241, 4096
-        706 -> 640."""
+        236 -> 198 (512, 128 tiles: 38 -> 40); 4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 4096 706 -> 640.  The longer K,
+        the less the trip counts beside CUs that wait in the last turn or multiply padding: of a K of 4096 three fifths of
+        the turns' places have to be outputs (10240 at 1792 rows, .55: 156 -> 163; 6144 at 3328, .61: 0.90), of a longer one .63
+        (8192 x 8192 at 1105, .54: 143 -> 153; 1377, .67: 0.88; 21504 x 4096 at 5120, .62: 724 -> 844), from three turns on .7
+        (8192 x 10240 at 3328, .68: 447 -> 479; 3693, .75: 0.71)."""
     rows = -(-M // 256)
     tiles = rows * (N // 256)
+    turns = -(-tiles // CUS)
+    dense = 4 * M >= 3 * 256 * rows  # the last tile's missing rows are a quarter of the tiles at most
+    useful = M * N / (max(turns, 1) * CUS * 65536)  # outputs of the places that the turns have
     if 0 < tiles <= CUS // 2 and not swiglu and (M >= 64 and K >= 12288 if b_kc else K >= 6144):
         parts = min(CUS // tiles, 16)
+        if b_kc and parts < 4 and K > 24576:
+            parts = 0
     elif swiglu:
-        parts = int(tiles >= CUS * 5 // 8 and 4 * M >= 768 * rows)
+        fill = 0.0 if K <= 2048 else 0.7 if turns > 2 else 0.6 if K <= 4096 else 0.63
+        parts = int(tiles >= CUS * 5 // 8 and dense and useful >= fill)
+    elif b_kc:
+        parts = int(M % 256 != 0 and K >= 8192 and 500 <= tiles <= 4096)
     else:
-        parts = int(M % 256 != 0 and (K >= 8192 and tiles >= 500 if b_kc else K >= 128 and _gains_nn(tiles)))
+        parts = int(M % 256 != 0 and K >= 128 and _gains_nn(tiles) and dense)
     return parts if parts and _policy() != "0" else 0
 
 
