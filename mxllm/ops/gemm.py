@@ -128,8 +128,8 @@ def _gains(form: str, M: int, N: int, K: int) -> bool:
         78 and 144 -> 154).  More: 256 tiles 118 -> 98, 512 237 -> 200, 384 172 -> 167 (288 tiles 149 -> 160).
     But not where there is little to save: a long K in multiples of 8 on 64 tiles (2048 x 2048, 3608 75 -> 74, 5160 93 -> 97,
     5600 93 -> 104), and round token counts of very many tiles, whose transposes are small beside the product or whose
-    time is the output's (57344 x 8192, 256 520 -> 595, 1536 1270 -> 1355; 8192 x 28672, 2304 840 -> 880; 128256 x 2048, 256 320 ->
-    355, but 768 553 -> 528 and 5120 2542 -> 2054).
+    time is the output's (57344 x 8192, 256 520 -> 595, 416 662 -> 694, 1536 1270 -> 1355, but 1544 1293 -> 1165; 8192 x
+    28672, 2304 840 -> 880; 128256 x 2048, 256 320 -> 355, but 768 553 -> 528 and 5120 2542 -> 2054).
     ``nn``: :func:`_gains_nn`."""
     tiles = (M // 256) * (N // 256)
     # past the kernel's 32-bit offsets (it would decline: the caller's other path stays)
@@ -137,7 +137,7 @@ def _gains(form: str, M: int, N: int, K: int) -> bool:
         return False
     if form == "tt":
         full = _wave_fill(tiles)
-        if K % 64 == 0 and tiles >= 3584 and (min(M, N) >= 8192 or K <= 512):
+        if K % 32 == 0 and tiles >= 3584 and (min(M, N) >= 8192 or K <= 512):
             return False
         if K % 8 == 0 and K > 4096 and tiles < 96:
             return False
@@ -181,12 +181,14 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
         2048 at 512 29 -> 37, 2048 69 -> 67); in two or three parts not past a K of 24,576 (28672 x 8192 at 559 277 -> 315,
         768 304 -> 321);
       * input gradients: K of 6144 on.  16384 x 2048 at 1000 124 -> 68, 4096 237 -> 211; 6144 x 4096 at 512 53 -> 43
-        (3072 x 2048 at 512 26 -> 30).
+        (3072 x 2048 at 512 26 -> 30); in two or three parts of a K over 24,576 with the last tile's rows not mostly
+        padding (57344 x 8192 at 560 524 -> 576, 700 595 -> 591, 1000 738 -> 656).
     Whole, where the library, which is tuned for round numbers of rows, falls behind between them:
       * projections (``b_kc``) of K 8192 and more from 500 tiles on: 8192 x 57344 at 700 559 -> 530, 2600 1916 -> 1740;
-        8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321), up to 4096 tiles (8192 x 128256 at 1700 2650 ->
-        2550, 2210 3378 -> 3555, 4445 6338 -> 6656).  With a shorter K the library is up to 27 %
-        slower at some row counts and 3 to 6 % faster at others (4096 x 28672 at 2700 543 -> 441, 4003 600 -> 634);
+        8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321), up to 4096 tiles and from 128 rows on (8192 x
+        128256 at 64 414 -> 394 to 454, 158 540 -> 450, 1700 2650 -> 2550, 2210 3378 -> 3555, 4445 6338 -> 6656).  With a
+        shorter K the library is up to 27 % slower at some row counts and 3 to 6 % faster at others (4096 x 28672 at 2700 543
+        -> 441, 4003 600 -> 634);
       * input gradients: :func:`_gains_nn`, with the last tile's rows not mostly padding (8192 -> 28672 at
         300 175 -> 184, 371 180 -> 190, 408 0.92);
       * gate-up with SwiGLU, which saves the projection's trip through HBM at any size: where the last tile's rows are
@@ -194,8 +196,9 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
         236 -> 198 (512, 128 tiles: 38 -> 40); 4096 x 28672 at 450 109 -> 97 (300: 77 -> 85), 4096 706 -> 640.  The longer K,
         the less the trip counts beside CUs that wait in the last turn or multiply padding: of a K of 4096 three fifths of
         the turns' places have to be outputs (10240 at 1792 rows, .55: 156 -> 163; 6144 at 3328, .61: 0.90), of a longer one .63
-        (8192 x 8192 at 1105, .54: 143 -> 153; 1377, .67: 0.88; 21504 x 4096 at 5120, .62: 724 -> 844), from three turns on .7
-        (8192 x 10240 at 3328, .68: 447 -> 479; 3693, .75: 0.71)."""
+        (8192 x 8192 at 1105, .54: 143 -> 153; 1377, .67: 0.88), from three turns on .7
+        (8192 x 10240 at 3328, .68: 447 -> 479; 3693, .75: 0.71), and past 8192 N at least as large (21504 x 4096 at 4013,
+        .98: 465 -> 487, at 5120, .62: 724 -> 844)."""
     rows = -(-M // 256)
     tiles = rows * (N // 256)
     turns = -(-tiles // CUS)
@@ -203,13 +206,13 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
     useful = M * N / (max(turns, 1) * CUS * 65536)  # outputs of the places that the turns have
     if 0 < tiles <= CUS // 2 and not swiglu and (M >= 64 and K >= 12288 if b_kc else K >= 6144):
         parts = min(CUS // tiles, 16)
-        if b_kc and parts < 4 and K > 24576:
+        if parts < 4 and K > 24576 and (b_kc or not dense):
             parts = 0
     elif swiglu:
         fill = 0.0 if K <= 2048 else 0.7 if turns > 2 else 0.6 if K <= 4096 else 0.63
-        parts = int(tiles >= CUS * 5 // 8 and dense and useful >= fill)
+        parts = int(tiles >= CUS * 5 // 8 and dense and useful >= fill and (K <= 8192 or N >= K))
     elif b_kc:
-        parts = int(M % 256 != 0 and K >= 8192 and 500 <= tiles <= 4096)
+        parts = int(M >= 128 and M % 256 != 0 and K >= 8192 and 500 <= tiles <= 4096)
     else:
         parts = int(M % 256 != 0 and K >= 128 and _gains_nn(tiles) and dense)
     return parts if parts and _policy() != "0" else 0

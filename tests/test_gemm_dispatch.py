@@ -124,8 +124,8 @@ def test_weight_gradient_rule():
 
     assert on(2048, 2048, 300) and on(2048, 2048, 3608) and on(2048, 2048, 5161) and on(3072, 2048, 5600)
     assert not on(2048, 2048, 4104) and not on(2048, 2048, 5600)
-    assert on(128256, 2048, 768) and on(128256, 4096, 1280) and on(57344, 8192, 1537) and on(16384, 4096, 2304)
-    assert not on(57344, 8192, 256) and not on(57344, 8192, 1536) and not on(8192, 28672, 2304) and not on(128256, 2048, 512)
+    assert on(128256, 2048, 768) and on(128256, 4096, 1280) and on(57344, 8192, 1544) and on(16384, 4096, 2304)
+    assert not on(57344, 8192, 256) and not on(57344, 8192, 416) and not on(57344, 8192, 1536) and not on(8192, 28672, 2304) and not on(128256, 2048, 512)
 
 
 def test_ragged_row_rules():
@@ -134,9 +134,9 @@ def test_ragged_row_rules():
         return gemm.rows_gain(M, N, K, form != "nn", form == "swiglu")
 
     on = [(512, 8192, 28672, "tn"), (1100, 2048, 12288, "tn"), (1700, 128256, 8192, "tn"), (408, 28672, 8192, "nn"),
-          (2635, 8192, 8192, "nn"), (3328, 6144, 4096, "swiglu"), (1280, 16384, 2048, "swiglu"), (1377, 8192, 8192, "swiglu"),
+          (2635, 8192, 8192, "nn"), (1000, 8192, 57344, "nn"), (158, 128256, 8192, "tn"), (3328, 6144, 4096, "swiglu"), (1280, 16384, 2048, "swiglu"), (1377, 8192, 8192, "swiglu"),
           (3693, 10240, 8192, "swiglu"), (765, 21504, 4096, "swiglu")]
     off = [(559, 8192, 28672, "tn"), (768, 8192, 28672, "tn"), (2210, 128256, 8192, "tn"), (300, 28672, 8192, "nn"),
-           (371, 28672, 8192, "nn"), (1792, 10240, 4096, "swiglu"), (1105, 8192, 8192, "swiglu"),
+           (371, 28672, 8192, "nn"), (560, 8192, 57344, "nn"), (64, 128256, 8192, "tn"), (4013, 4096, 21504, "swiglu"), (1792, 10240, 4096, "swiglu"), (1105, 8192, 8192, "swiglu"),
            (3328, 10240, 8192, "swiglu"), (5120, 4096, 21504, "swiglu"), (512, 16384, 2048, "swiglu")]
     assert [s for s in on if not gain(*s)] == [] and [s for s in off if gain(*s)] == []
