@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(256) sample_kernel(const T* __restrict__ logit
   const T* x = logits + row * V;
   const int c0 = blockIdx.x * chunk, c1 = min(V, c0 + chunk);
   uint32_t nseed = seed + (uint32_t)row * 7919u;
-  if (temps) {  // per-row parameters (sample_rows without top-k / top-p): noise of sampling.hip
+  if (temps) {  // per-row parameters (mx_sample_temp_rows): noise of sampling.hip
     const float t = temps[row];
     inv_temp = t > 0.f ? 1.f / t : 0.f;
     nseed = (uint32_t)seeds[row];

@@ -65,8 +65,8 @@ def test_gpu_sampler_mixed_batch_and_vocab_128k(gpu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.float32, 50001)])
 def test_gpu_temperature_rows_split_kernel_matches_topkp_kernel(gpu, dtype, V):
-    """Rows without top-k / top-p go to the vocabulary-split kernel (decode.hip); its draws
-    equal the radix-select kernel's (sampling.hip) for the same (seed, step) noise."""
+    """Rows without top-k / top-p: the draws of the temperature-only kernel (decode.hip, parameters in device
+    arrays) equal the sampler's with thresholds (sampling.hip) for the same (seed, step) noise."""
     from mxllm.ops import native
 
     B = 6
@@ -235,3 +235,28 @@ def test_split_sampler_masses_fit():
     ws.restype = ctypes.c_int64
     taken = [V for V in (1, 16383, 16384, (1 << 22) - 1, 1 << 22, 1 << 23) if ws(1, V) > 0]
     assert taken == [16384, (1 << 22) - 1] and max(taken) << 42 < 1 << 64
+
+
+@pytest.mark.gpu
+def test_concurrent_mixed_samplers_on_two_streams(gpu):
+    """Two samplers of rows with their own temperature, top-k and top-p on different streams at once: every call has its
+    own histograms, lists and counters, so the draws are those of the calls one by one."""
+    B, V = 40, 128256
+    g = torch.Generator(device=gpu).manual_seed(1)
+    xs = [torch.empty(B, V, device=gpu).normal_(0, 2.5, generator=g).bfloat16() for _ in range(2)]
+    ways = [(0.8, 0.9, 0), (0.7, 0.95, 50), (1.0, 1.0, 0), (0.0, 1.0, 0), (1.3, 1.0, 40)]
+    temps, tops, ks = zip(*(ways[i % 5] for i in range(B)))
+
+    def draw(k, step):
+        return dops.sample_rows(xs[k], temps, tops, ks, [100 * k + i for i in range(B)], [step] * B)
+
+    want = [[draw(k, step).clone() for step in range(10)] for k in range(2)]
+    streams = [torch.cuda.Stream(gpu) for _ in range(2)]
+    torch.cuda.synchronize(gpu)
+    got = [[], []]
+    for step in range(10):
+        for k in range(2):
+            with torch.cuda.stream(streams[k]):
+                got[k].append(draw(k, step))
+    torch.cuda.synchronize(gpu)
+    assert all(torch.equal(a, b) for k in range(2) for a, b in zip(got[k], want[k]))

@@ -413,3 +413,34 @@ def test_tied_fresh_gradients_bitwise(gpu, gdt, accum, monkeypatch):
         out[fresh] = _masters(tr)
     for n, w in out["0"].items():
         assert torch.equal(w, out["1"][n]), n
+
+
+def test_fused_grad_norm_of_tied_embeddings(gpu, monkeypatch):
+    """The default path of models with tied embeddings: their slot, which autograd sums and no GEMM's partials cover, is
+    read by the direct pass, with nothing of the values that the slots held before the step; the first step's gradients
+    and norm are those of the full pass."""
+    from mxllm import ops
+
+    monkeypatch.setenv("MXLLM_GEMM8", "all")  # the tiny shapes on gemm8
+    cfg = _cfg().replace(tie_embeddings=True)
+    g = torch.Generator(device=gpu).manual_seed(3)
+    batches = [torch.randint(0, cfg.vocab_size, (2, 256), device=gpu, generator=g) for _ in range(3)]
+    res = {}
+    for fused in ("1", "0"):
+        monkeypatch.setenv("MXLLM_FUSED_GRAD_NORM", fused)
+        tr = _ddp_trainer(gpu, cfg, 5)
+        assert tr.fresh_grads and bool(tr._sq_params) == (fused == "1")
+        tied = tr.model.tok_emb
+        for i, b in enumerate(batches):
+            for s in tr.flat.slots:
+                tr.flat.grads[s.offset:s.offset + s.numel].fill_(7.0)
+            tr.train_step([(b, b)])
+            got, want = float(tr.last_grad_norm), float(ops.sq_norm(tr.flat.grads).sqrt())
+            assert abs(got - want) <= 1e-6 * want, (fused, i, got, want)
+            if i == 0:
+                res[fused] = got, tr.flat.grads.clone()
+        if fused == "1":
+            assert any(p is tied for p in tr._sq_params) and tied._mx_sq_done is False
+            assert any(p._mx_sq_done is True for p in tr._sq_params)
+    (n1, g1), (n0, g0) = res["1"], res["0"]
+    assert torch.equal(g1, g0) and abs(n1 - n0) <= 1e-6 * n0
