@@ -688,9 +688,12 @@ def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
 
 def _plain(*ts: torch.Tensor | None) -> bool:
     """Tensors that a kernel without a derivative, a batching rule or a shape function may take: no gradient is asked of
-    any, backward or forward mode, none is a transform's (``torch.func``) or a subclass, and nothing records the call
-    (compilers, tracers, dispatch modes), which would keep the choice made for these sizes, or not know the op."""
+    any, backward or forward mode, none is a transform's (``torch.func``) or a subclass, autocast asks for no other type,
+    and nothing records the call (compilers, tracers, dispatch modes), which would keep the choice made for these sizes, or
+    not know the op."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
+        return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
     grad = torch.is_grad_enabled()
     return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)

@@ -121,3 +121,13 @@ def test_switch_off_is_the_library(gpu, M, monkeypatch):
     x, w = _bf16(gpu, M, 12288), _bf16(gpu, 512, 12288, seed=1, std=0.03)
     _close(ops.linear(x, w), x.double() @ w.double().t(), 2 ** -8)
     assert ops.linear_swiglu(x, w) is None and ops.norm_linear(None, x, x[0].contiguous(), 1e-5, w) is None
+
+
+@pytest.mark.parametrize("M", [4, 16, 64])
+def test_autocast_decides_the_type(gpu, M):
+    x, w = _bf16(gpu, M, 12288), _bf16(gpu, 2048, 12288, seed=1, std=0.03)
+    for dtype in (torch.float16, torch.bfloat16):
+        with torch.autocast("cuda", dtype):
+            y = ops.linear(x, w)
+        assert y.dtype == dtype
+        _close(y, x.double() @ w.double().t(), 2 ** -8)
