@@ -677,48 +677,55 @@ def _decode_route(M: int, N: int, K: int) -> str:
     return "skinny" if M <= _DECODE_M and _wide_wins(M, N, K) else ""
 
 
-def _decode_linear(x2: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
-    route = _decode_route(x2.shape[0], *w.shape)
-    if not route or not _rows_ok(x2, w):
-        return None
-    if route == "stream":
-        return native().stream_linear(x2, None, None, 0.0, w, None, False)[0]
-    return (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
-
-
 def _plain(*ts: torch.Tensor | None) -> bool:
     """Tensors that a kernel without a derivative, a batching rule or a shape function may take: no gradient is asked of
-    any, backward or forward mode, none is a transform's (``torch.func``) or a subclass, autocast asks for no other type,
-    and nothing records the call (compilers, tracers, dispatch modes), which would keep the choice made for these sizes, or
-    not know the op."""
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack():
+    any, none is a subclass, autocast asks for no other type, and nothing transforms or records the call (forward-mode
+    levels, ``torch.func``, compilers, tracers, dispatch modes), which would not see what the kernel does, or keep the
+    choice made for these sizes.  Asked where a kernel would be taken only: 2 us of host time."""
+    if (torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+            or torch._C._functorch.maybe_current_level() is not None or torch._C._get_tracing_state() is not None):
         return False
-    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
+    if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False
     grad = torch.is_grad_enabled()
-    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)
-                             and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-                             and forward_ad.unpack_dual(t).tangent is None) for t in ts)
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter) and not (grad and t.requires_grad)) for t in ts)
+
+
+def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    """``x w^T`` by the kernel that its sizes go to; None: the library."""
+    if w.dim() != 2:
+        return None
+    N, K = w.shape
+    M = x.numel() // max(K, 1)
+    if x.shape[-1] != K or M == 0:
+        return None
+    if M <= _DECODE_M:
+        route = _decode_route(M, N, K)
+        if not route or not _plain(x, w):
+            return None
+        x2 = x.reshape(M, K)
+        if not _rows_ok(x2, w):
+            return None
+        if route == "stream":
+            y = native().stream_linear(x2, None, None, 0.0, w, None, False)[0]
+        else:
+            y = (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
+    else:
+        parts = gemm.rows_gain(M, N, K, True) if SKINNY_M > 0 and x.is_cuda and x.dim() > 1 else 0
+        if not parts or not _plain(x, w):
+            return None
+        x2 = x.reshape(M, K)
+        if not gemm.rows_ok(x2, w, True):
+            return None
+        y = native().gemm8_rows(x2, w, True, False, parts)
+    return y.view(*x.shape[:-1], N)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if w.requires_grad and torch.is_grad_enabled():
         return _LinearFn.apply(x, w)
-    if not _plain(x, w):
-        return F.linear(x, w)
-    if x.shape[-1] == w.shape[1] and 0 < x.numel() // max(x.shape[-1], 1) <= _DECODE_M:
-        y = _decode_linear(x.reshape(-1, x.shape[-1]), w)
-        if y is not None:
-            return y.view(*x.shape[:-1], w.shape[0])
-    if SKINNY_M > 0 and x.is_cuda and x.dim() > 1:
-        N, K = w.shape
-        M = x.numel() // max(K, 1)
-        parts = gemm.rows_gain(M, N, K, True)
-        if parts and x.shape[-1] == K:
-            x2 = x.reshape(M, K)
-            if gemm.rows_ok(x2, w, True):
-                return native().gemm8_rows(x2, w, True, False, parts).view(*x.shape[:-1], N)
-    return F.linear(x, w)
+    y = None if torch.compiler.is_compiling() else _inference_linear(x, w)
+    return F.linear(x, w) if y is None else y
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
@@ -726,20 +733,19 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
     stream_gemm.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
-    if SKINNY_M <= 0 or x.dim() != 2 or not _plain(x, w):
+    if SKINNY_M <= 0 or x.dim() != 2 or x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
         return None
-    if x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
-        return None
+    (M, K), N = x.shape, w.shape[0]
     if scale is not None:
-        if not (_stream_fits(*x.shape) and _rows_ok(x, w, scale)):
+        if not (_stream_fits(M, K) and _plain(x, w) and _rows_ok(x, w, scale)):
             return None
         return native().stream_linear(x, None, None, 0.0, w, scale, True)[0]
-    if _stream_wins(x.shape[0], *w.shape, True) and _rows_ok(x, w):
+    if _stream_wins(M, N, K, True) and _plain(x, w) and _rows_ok(x, w):
         return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
-    if 0 < x.shape[0] <= SKINNY_M and _skinny_ok(x, w):
+    if M <= SKINNY_M and _plain(x, w) and _skinny_ok(x, w):
         return native().skinny_linear_swiglu(x, w)
-    parts = gemm.rows_gain(x.shape[0], *w.shape, True, True)  # a prompt pass
-    if parts and gemm.rows_ok(x, w, True, True):
+    parts = gemm.rows_gain(M, N, K, True, True)  # a prompt pass
+    if parts and _plain(x, w) and gemm.rows_ok(x, w, True, True):
         return native().gemm8_rows(x, w, True, True, parts)
     return None
 
@@ -826,13 +832,13 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
     the RMSNorm kernel + decode GEMM); with ``swiglu`` w = [gate; up] and the first output is
     silu(g) * u; ``scale``: w is e4m3 codes.  ``delta`` None: plain RMSNorm, the residual is ``h``.  None
     when the fused kernels do not take the call."""
-    if SKINNY_M <= 0 or h.dim() != 2 or not _plain(delta, h, gamma, w):
+    if SKINNY_M <= 0 or h.dim() != 2:
         return None
     M, K = h.shape
     stream = _norm_stream(M, K) and (_norm_wins(M, w.shape[0], K) if scale is None else w.shape[0] >= 8192)
     if not stream and (scale is not None or not 0 < M <= min(NORM_M, SKINNY_M) or M * K > 32768):
         return None
-    if w.shape[1] != K or w.shape[0] % 16 or not _norm_operands(delta, h, gamma):
+    if w.shape[1] != K or w.shape[0] % 16 or not (_plain(delta, h, gamma, w) and _norm_operands(delta, h, gamma)):
         return None
     if not (_rows_ok(h, w, scale) if stream else _skinny_ok(h, w)):
         return None
