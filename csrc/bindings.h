@@ -114,13 +114,6 @@ int mx_sample(const void* logits, int is_bf16, int64_t* out, int B, int V, float
 int mx_sample_temp_rows(const void* logits, int is_bf16, int64_t* out, int B, int V, const float* temps,
                         const int64_t* seeds, const int32_t* steps, float* ws, hipStream_t stream);
 // sampling.hip
-// stream_gemm.hip
-int mx_stream_ok(int M, int K, int norm);
-int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
-                   int64_t ldy, int M, int N, int K, int epi, const uint16_t* delta, int64_t ldd, const uint16_t* gamma,
-                   float eps, uint16_t* h_out, const float* cosb, const float* sinb, const int32_t* pos,
-                   const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq, int Hkv, int max_seq,
-                   const int32_t* bt, int maxb, hipStream_t stream);
 int64_t mx_sample_rows_ws(int B, int V);
 int mx_sample_rows(const void* logits, int is_bf16, int64_t* out, int B, int V, const float* temps,
                    const float* top_ps, const int32_t* top_ks, const int64_t* seeds, const int32_t* steps, void* ws,
@@ -128,6 +121,13 @@ int mx_sample_rows(const void* logits, int is_bf16, int64_t* out, int B, int V, 
 int mx_sample_list(const void* logits, int is_bf16, int64_t* out, int B, int V, const double* temps,
                    const double* top_ps, const int64_t* top_ks, const int64_t* seeds, const int64_t* steps, void* ws,
                    hipStream_t stream);
+// stream_gemm.hip
+int mx_stream_ok(int M, int K, int norm);
+int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
+                   int64_t ldy, int M, int N, int K, int epi, const uint16_t* delta, int64_t ldd, const uint16_t* gamma,
+                   float eps, uint16_t* h_out, const float* cosb, const float* sinb, const int32_t* pos,
+                   const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq, int Hkv, int max_seq,
+                   const int32_t* bt, int maxb, hipStream_t stream);
 }
 
 extern "C" {

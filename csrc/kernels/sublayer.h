@@ -142,7 +142,7 @@ struct MoeGemm {
   const void* x;         // [*, K]
   int64_t ldx;
   const int32_t* src;    // row of x of each sorted row (nullptr: the row itself)
-  const int32_t* tiles;  // [ntiles, 4]: (expert, first sorted row, rows, -); rows 0: none
+  const int32_t* tiles;  // [ntiles, 4]: (expert, first sorted row, rows, tiles in use), the unused ones last with rows 0
   int ntiles;
   const void* w;         // [experts, N, K], GLU: [experts, 2 N, K] (gate rows, then up rows)
   void* y;               // [rows, N]
