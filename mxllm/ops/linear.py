@@ -693,7 +693,7 @@ def _plain(*ts: torch.Tensor | None) -> bool:
 
 def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     """``x w^T`` by the kernel that its sizes go to; None: the library."""
-    if w.dim() != 2:
+    if not x.is_cuda or w.dim() != 2:
         return None
     N, K = w.shape
     M = x.numel() // max(K, 1)
@@ -711,7 +711,7 @@ def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
         else:
             y = (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
     else:
-        parts = gemm.rows_gain(M, N, K, True) if SKINNY_M > 0 and x.is_cuda and x.dim() > 1 else 0
+        parts = gemm.rows_gain(M, N, K, True) if SKINNY_M > 0 and x.dim() > 1 else 0
         if not parts or not _plain(x, w):
             return None
         x2 = x.reshape(M, K)
