@@ -11,17 +11,23 @@
 // sample of the renormalised distribution over them, with the same (seed, step, index) noise as the
 // greedy / temperature kernel in decode.hip, so a request's stream does not depend on batching.
 //
-// Split form (vocabularies of kSplitV and more): four launches over (chunk, row), so a step's few rows fill the
+// Split form (vocabularies of kSplitV and more): three launches over (chunk, row), so a step's few rows fill the
 // chip.  One workgroup a row kept 32 of 256 CUs on six to nine passes whose LDS atomics and logarithms bound it:
-// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the four launches take 63 us (stats 6,
-// hist 15, pick 24, final 18; all top-p 85 us, all top-k 38, temperature alone 26).
+// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the three launches take 35 us (stats 6, hist
+// 11, pick 17; all top-p 33, all top-k 25, temperature alone 20).  What bounds them now: dependent steps inside each
+// launch (row parameters, the chunks' partials, scans over bins, the counter of a row), and for few rows the host's
+// three launches (22 - 25 us a call).
 //  * stats: a chunk's largest (with its index) and smallest logit;
 //  * hist: masses exp2((x - max) log2e / T) and counts in 2048 bins, linear in the exponent (64 bins a power of
 //    two, finer where the row's whole range is under 32 of them).  A bin holds all tokens of a value, so bins
-//    order tokens as their logits do.  Masses are summed as integers (2^-42): any order gives the same sums;
+//    order tokens as their logits do.  Masses are summed as integers (2^-42): any order gives the same sums.
+//    Rows without cuts compete here already;
 //  * pick: the bins where top-k and top-p cross, from the sums; tokens ahead of them compete at once, those
-//    inside are listed (a value or two: tens to hundreds of tokens), the rest is dropped;
-//  * final: exact counts and masses above each listed token, the kept ones compete with the chunks' winners.
+//    inside are listed (a value or two: tens to hundreds of tokens), the rest is dropped.  A row's last workgroup has
+//    exact counts and masses above each listed token; the kept ones compete with the chunks' winners.
+// One workgroup of 1,024 threads a CU: each clears, adds up and scans 2,048 bins, so that four times as many of 256
+// threads took 61 us for the 32 mixed rows (a global counter asked for each listed token, and a fourth launch with a
+// scan of its own for the listed ones, were the other half of that).
 // A row whose list overflows (thousands of tokens of one value at the boundary), and short vocabularies, take the
 // one-workgroup form: no sort, the k-th largest key and then the top-p boundary key by a radix select over
 // order-preserving 32-bit keys, 11 + 11 + 10 bits, over LDS histograms.  Its mass histogram uses float atomics: a
@@ -272,22 +278,32 @@ __global__ void __launch_bounds__(kSampThreads) sample_topkp_kernel(const T* __r
 }
 
 // ------------------------------------------------------------------ split form
-// Shorter rows: one workgroup, one launch.  32 top-p rows of 8,191: 30 us against 41 split; of 32,768: about 80
-// (its time grows with the row) against 47.
+// Shorter rows: one workgroup, one launch.  32 top-p rows of 8,191: 30 us against 41 split when that was four launches;
+// of 32,768: about 80 (its time grows with the row) against 27 now.
 constexpr int kSplitV = 16384;
 constexpr int kSplitMaxV = (1 << 22) - 1;  // as many masses of up to 2^42 stay below 2^64
 constexpr int kMBins = 2048;
 constexpr int kMaxCh = 64;         // chunks a row (= one wave over their partials)
 constexpr int kListCap = 1024;     // listed tokens a row
-constexpr int kChThreads = 256;
+constexpr int kChThreads = 1024;
+
+// A token that only exact sums decide about, with the mass and count of the bins ahead of its own.
+struct Listed {
+  unsigned long long id, pm;  // id: key << 32 | index
+  uint32_t pc, pad;
+};
+struct RowInfo {
+  unsigned long long tot, pmk;  // mass of the row; of the bins ahead of the one the k-th token is in
+  int bk;                       // that bin
+};
 
 struct SampWs {
-  float *mx, *mn, *gv;   // [rows, nch]: largest, smallest finite logit; best score among tokens kept at once
-  int *mi, *gi;          // their indexes
   unsigned long long* mass;  // [rows, kMBins]
+  Listed* list;              // [rows, kListCap]
   uint32_t* cnt;             // [rows, kMBins]
-  unsigned long long* list;  // [rows, kListCap] key << 32 | index
-  uint32_t* nlist;           // [rows]
+  float *mx, *mn, *gv;       // [rows, kMaxCh]: largest, smallest finite logit; best score among tokens kept at once
+  int *mi, *gi;              // their indexes
+  uint32_t *nlist, *done;    // [rows]: listed tokens, workgroups that are through
 };
 
 __device__ __forceinline__ void pick(float& b, int& i, float ov, int oi) {
@@ -298,60 +314,110 @@ __device__ __forceinline__ void wave_pick(float& b, int& i) {
   for (int o = 32; o > 0; o >>= 1) pick(b, i, __shfl_xor(b, o, 64), __shfl_xor(i, o, 64));
 }
 
-// f(index, value) over [c0, c1) of a row; 16-B loads where the row and the chunk allow it
-template <typename T, typename F>
-__device__ __forceinline__ void each_in(const T* __restrict__ x, int c0, int c1, F&& f) {
-  int c = c0;
-  if ((((uintptr_t)(x + c0)) & 15) == 0) {
-    const int ve = c0 + (c1 - c0) / 8 * 8;
-    for (int b = c0 + (int)threadIdx.x * 8; b < ve; b += kChThreads * 8) {
-      if constexpr (sizeof(T) == 2) {
-        const u16x8 v = *reinterpret_cast<const u16x8*>(x + b);
+// [c0, c1) of a row by 16-B loads, two pieces of 8 a thread and turn; rows of any alignment (an odd vocabulary
+// shifts every row) have their first and last few values apart
+template <typename T>
+struct Chunk {
+  const T* x;
+  int c0, c1, head, ve;
+  struct Pieces {
+    u16x8 u, v;
+    __device__ __forceinline__ float at(int j) const { return bf2f(j < 8 ? u[j & 7] : v[j & 7]); }
+  };
+  struct Pieces32 {
+    f32x4 u[2], v[2];
+    __device__ __forceinline__ float at(int j) const { return j < 8 ? u[(j >> 2) & 1][j & 3] : v[(j >> 2) & 1][j & 3]; }
+  };
+  using P = std::conditional_t<sizeof(T) == 2, Pieces, Pieces32>;
+  static constexpr int S = kChThreads * 8;
+
+  __device__ __forceinline__ Chunk(const T* row, int a, int b) : x(row), c0(a), c1(b) {
+    head = min(c1, c0 + (int)((16 - ((uintptr_t)(x + c0) & 15)) & 15) / (int)sizeof(T));
+    ve = head + (c1 - head) / 8 * 8;
+  }
+  __device__ __forceinline__ int start() const { return head + (int)threadIdx.x * 8; }
+  // pieces at b and, where the chunk has it, b + S (else the first again)
+  __device__ __forceinline__ P load(int b) const {
+    const T *p = x + b, *q = x + (b + S < ve ? b + S : b);
+    P r;
+    if constexpr (sizeof(T) == 2) {
+      r.u = *reinterpret_cast<const u16x8*>(p), r.v = *reinterpret_cast<const u16x8*>(q);
+    } else {
+      r.u[0] = *reinterpret_cast<const f32x4*>(p), r.u[1] = *reinterpret_cast<const f32x4*>(p + 4);
+      r.v[0] = *reinterpret_cast<const f32x4*>(q), r.v[1] = *reinterpret_cast<const f32x4*>(q + 4);
+    }
+    return r;
+  }
+  // the thread's values outside the pieces: f(index, value)
+  template <typename F>
+  __device__ __forceinline__ void ends(F&& f) const {
+    const int t = threadIdx.x;
+    auto one = [&](int c) {
+      if constexpr (sizeof(T) == 2) f(c, bf2f(x[c]));
+      else f(c, x[c]);
+    };
+    if (c0 + t < head) one(c0 + t);
+    if (ve + t < c1) one(ve + t);
+  }
+  __device__ __forceinline__ P first() const {
+    P p = {};
+    if (start() < ve) p = load(start());
+    return p;
+  }
+  template <typename F>
+  __device__ __forceinline__ void each(F&& f) const {
+    each(first(), f);
+  }
+  template <typename F>
+  __device__ __forceinline__ void each(P p, F&& f) const {
+    ends(f);
+    for (int b = start(); b < ve; b += 2 * S) {
+      if (b != start()) p = load(b);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) f(b + j, bf2f(v[j]));
-      } else {
-        const f32x4 u = *reinterpret_cast<const f32x4*>(x + b), v = *reinterpret_cast<const f32x4*>(x + b + 4);
+      for (int j = 0; j < 8; ++j) f(b + j, p.at(j));
+      if (b + S < ve) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) f(b + j, u[j]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) f(b + 4 + j, v[j]);
+        for (int j = 8; j < 16; ++j) f(b + S + j - 8, p.at(j));
       }
     }
-    c = ve;
   }
-  for (c += threadIdx.x; c < c1; c += kChThreads) {
-    if constexpr (sizeof(T) == 2) f(c, bf2f(x[c]));
-    else f(c, x[c]);
+};
+
+// thread 0's (b, i): the best of the workgroup
+__device__ __forceinline__ void group_pick(float& b, int& i, float* sv, int* si) {
+  wave_pick(b, i);
+  if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = b; si[threadIdx.x >> 6] = i; }
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    b = threadIdx.x < kChThreads / 64 ? sv[threadIdx.x] : -INFINITY;
+    i = threadIdx.x < kChThreads / 64 ? si[threadIdx.x] : 0x7fffffff;
+    wave_pick(b, i);
   }
 }
 
 template <typename T>
 __global__ void __launch_bounds__(kChThreads) samp_stats_kernel(const T* __restrict__ logits, int V, int chunk,
                                                                 SampWs ws) {
-  __shared__ float sv[4], sm[4];
-  __shared__ int si[4];
+  __shared__ float sv[kChThreads / 64], sm[kChThreads / 64];
+  __shared__ int si[kChThreads / 64];
   const int row = blockIdx.y, nch = gridDim.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   for (int i = blockIdx.x * kChThreads + threadIdx.x; i < kMBins; i += nch * kChThreads) {
     ws.mass[row * kMBins + i] = 0;
     ws.cnt[row * kMBins + i] = 0;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) ws.nlist[row] = 0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) ws.nlist[row] = ws.done[row] = 0;
   const int c0 = blockIdx.x * chunk;
   float b = -INFINITY, m = INFINITY;
   int bi = 0x7fffffff;
-  each_in(logits + (size_t)row * V, c0, min(V, c0 + chunk), [&](int i, float v) {
+  Chunk<T>(logits + (size_t)row * V, c0, min(V, c0 + chunk)).each([&](int i, float v) {
     pick(b, bi, v, i);
     if (v > -INFINITY) m = fminf(m, v);
   });
-  wave_pick(b, bi);
   m = -wave_max(-m);
-  if (lane == 0) { sv[wv] = b; si[wv] = bi; sm[wv] = m; }
-  __syncthreads();
+  if (lane == 0) sm[wv] = m;
+  group_pick(b, bi, sv, si);
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kChThreads / 64; ++w) {
-      pick(b, bi, sv[w], si[w]);
-      m = fminf(m, sm[w]);
-    }
+    for (int w = 1; w < kChThreads / 64; ++w) m = fminf(m, sm[w]);
     ws.mx[row * kMaxCh + blockIdx.x] = b;
     ws.mi[row * kMaxCh + blockIdx.x] = bi;
     ws.mn[row * kMaxCh + blockIdx.x] = m;
@@ -375,8 +441,13 @@ __device__ __forceinline__ RowScale row_scale(const SampWs& ws, int row, int nch
   const int lane = threadIdx.x & 63;
   float b = lane < nch ? ws.mx[row * kMaxCh + lane] : -INFINITY, m = lane < nch ? ws.mn[row * kMaxCh + lane] : INFINITY;
   int bi = lane < nch ? ws.mi[row * kMaxCh + lane] : 0x7fffffff;
-  wave_pick(b, bi);
-  m = -wave_max(-m);
+  for (int o = 1; o < nch; o <<= 1) {  // lane 0's; few chunks, few turns
+    pick(b, bi, __shfl_xor(b, o, 64), __shfl_xor(bi, o, 64));
+    m = fminf(m, __shfl_xor(m, o, 64));
+  }
+  b = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(b)));
+  m = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m)));
+  bi = __builtin_amdgcn_readfirstlane(bi);
   RowScale r;
   r.mx = b;
   r.mi = bi;
@@ -391,15 +462,31 @@ __global__ void __launch_bounds__(kChThreads) samp_hist_kernel(const T* __restri
                                                                SampArgs a, int row0, SampWs ws) {
   __shared__ unsigned long long mass[kMBins];
   __shared__ uint32_t cnt[kMBins];
+  __shared__ float sv[kChThreads / 64];
+  __shared__ int si[kChThreads / 64];
   const int row = blockIdx.y;
   const SampRow rp = samp_row(a, row0 + row);
   const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f;
-  if (!(rp.temp > 0.f) || !(hk || hp)) return;
-  const RowScale rs = row_scale(ws, row, gridDim.x, rp.temp);
-  for (int i = threadIdx.x; i < kMBins; i += kChThreads) { mass[i] = 0; cnt[i] = 0; }
-  __syncthreads();
+  if (!(rp.temp > 0.f)) return;
   const int c0 = blockIdx.x * chunk;
-  each_in(logits + (size_t)row * V, c0, min(V, c0 + chunk), [&](int, float v) {
+  const Chunk<T> ch(logits + (size_t)row * V, c0, min(V, c0 + chunk));
+  if (!(hk || hp)) {  // every token competes: nothing to wait for
+    const float inv_t = 1.f / rp.temp;
+    float gb = -INFINITY;
+    int gi = 0x7fffffff;
+    ch.each([&](int i, float v) { pick(gb, gi, gumbel_score(v, inv_t, rp.seed, rp.step, i), i); });
+    group_pick(gb, gi, sv, si);
+    if (threadIdx.x == 0) {
+      ws.gv[row * kMaxCh + blockIdx.x] = gb;
+      ws.gi[row * kMaxCh + blockIdx.x] = gi;
+    }
+    return;
+  }
+  const typename Chunk<T>::P first = ch.first();  // on its way while the row's scale is found
+  for (int i = threadIdx.x; i < kMBins; i += kChThreads) { mass[i] = 0; cnt[i] = 0; }
+  const RowScale rs = row_scale(ws, row, gridDim.x, rp.temp);
+  __syncthreads();
+  ch.each(first, [&](int, float v) {
     const int b = rs.bin(v);
     if (hp) atomicAdd(&mass[b], rs.weight(v));
     if (hk) atomicAdd(&cnt[b], 1u);
@@ -415,23 +502,33 @@ __global__ void __launch_bounds__(kChThreads) samp_hist_kernel(const T* __restri
 // the k-th token is in; kMBins: no top-k) are listed.
 struct RowCut {
   int all, last, bk;
+  unsigned long long klo, khi;  // mass of the bins ahead of bk, and with it
 };
-// pm / pc [kMBins]: mass and count of the bins ahead of each; every thread of NT calls it
-template <int NT>
-__device__ __forceinline__ RowCut row_cut(const SampWs& ws, int row, const SampRow& rp, bool hk, bool hp,
-                                          unsigned long long* pm, uint32_t* pc, unsigned long long* wm, uint32_t* wc,
-                                          RowCut* out) {
-  constexpr int PER = kMBins / NT, NW = NT / 64;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  unsigned long long m[PER], sm = 0;
-  uint32_t n[PER], sn = 0;
+// a thread's bins
+struct Bins {
+  static constexpr int PER = kMBins / kChThreads;
+  unsigned long long m[PER];
+  uint32_t n[PER];
+  __device__ __forceinline__ Bins(const SampWs& ws, int row, bool hk, bool hp) {
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    m[i] = hp ? ws.mass[row * kMBins + t * PER + i] : 0;
-    n[i] = hk ? ws.cnt[row * kMBins + t * PER + i] : 0;
-    sm += m[i];
-    sn += n[i];
+    for (int i = 0; i < PER; ++i) {
+      m[i] = hp ? ws.mass[row * kMBins + threadIdx.x * PER + i] : 0;
+      n[i] = hk ? ws.cnt[row * kMBins + threadIdx.x * PER + i] : 0;
+    }
   }
+};
+// pm / pc [kMBins]: mass and count of the bins ahead of each; every thread calls it
+__device__ __forceinline__ RowCut row_cut(const Bins& bins, const SampRow& rp, bool hk, bool hp,
+                                          unsigned long long* pm, uint32_t* pc, unsigned long long* wm, uint32_t* wc,
+                                          RowCut* out, unsigned long long& tot) {
+  constexpr int PER = Bins::PER, NW = kChThreads / 64;
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const auto &m = bins.m;
+  const auto &n = bins.n;
+  unsigned long long sm = 0;
+  uint32_t sn = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) sm += m[i], sn += n[i];
   unsigned long long im = sm;
   uint32_t in = sn;
 #pragma unroll
@@ -441,47 +538,52 @@ __device__ __forceinline__ RowCut row_cut(const SampWs& ws, int row, const SampR
     if (lane >= o) { im += y; in += z; }
   }
   if (lane == 63) { wm[wv] = im; wc[wv] = in; }
-  if (t == 0) *out = RowCut{0, kMBins - 1, hk ? kMBins - 1 : kMBins};
+  if (t == 0) *out = RowCut{0, 0, hk ? kMBins - 1 : kMBins, 0, 0};
   __syncthreads();
-  unsigned long long bm = im - sm, tot = 0;
-  uint32_t bn = in - sn;
-  for (int w = 0; w < NW; ++w) {
-    if (w < wv) { bm += wm[w]; bn += wc[w]; }
-    tot += wm[w];
+  unsigned long long vm = lane < NW ? wm[lane] : 0;
+  uint32_t vn = lane < NW ? wc[lane] : 0;
+#pragma unroll
+  for (int o = 1; o < NW; o <<= 1) {
+    const unsigned long long y = __shfl_up(vm, o, 64);
+    const uint32_t z = __shfl_up(vn, o, 64);
+    if (lane >= o) { vm += y; vn += z; }
   }
+  tot = __shfl(vm, NW - 1, 64);
+  unsigned long long bm = im - sm + (wv ? __shfl(vm, wv - 1, 64) : 0);
+  uint32_t bn = in - sn + (wv ? __shfl(vn, wv - 1, 64) : 0);
+  const unsigned long long bm0 = bm;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int b = t * PER + i;
     pm[b] = bm;
     pc[b] = bn;
-    if (hk && bn < (uint32_t)rp.k && bn + n[i] >= (uint32_t)rp.k) out->bk = b;
+    if (hk && bn < (uint32_t)rp.k && bn + n[i] >= (uint32_t)rp.k) {
+      out->bk = b;
+      out->klo = bm;
+      out->khi = bm + m[i];
+    }
     bm += m[i];
     bn += n[i];
   }
   __syncthreads();
   RowCut r = *out;
-  __syncthreads();
   const bool lim = hp && tot > 0 && rp.p > 0.f;  // an empty mass restricts nothing
   if (lim) {
-    // the kept set's mass lies between that of the bins ahead of bk and that with bk
-    const double lo = (double)rp.p * (double)(hk ? pm[r.bk] : tot);
-    const double hi = (double)rp.p * (double)(hk && r.bk + 1 < kMBins ? pm[r.bk + 1] : tot);
-    // bins whose tokens are wholly under a target: a prefix of them
-    int nlo = 0, nhi = 0;
+    // the kept set's mass lies between that of the bins ahead of bk and that with bk; the bin that brings the mass
+    // to p of either: no bin ahead of it does
+    const double lo = (double)rp.p * (double)(hk ? r.klo : tot);
+    const double hi = (double)rp.p * (double)(hk ? r.khi : tot);
+    bm = bm0;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int b = t * PER + i;
-      const double incl = (double)(b + 1 < kMBins ? pm[b + 1] : tot);
-      nlo += incl < lo;
-      nhi += incl < hi;
+      const double excl = (double)bm, incl = (double)(bm + m[i]);
+      if (excl < lo && incl >= lo) out->all = t * PER + i;
+      if (excl < hi && incl >= hi) out->last = t * PER + i;
+      bm += m[i];
     }
-    if (t == 0) { out->all = 0; out->last = 0; }
-    __syncthreads();
-    atomicAdd(&out->all, nlo);
-    atomicAdd(&out->last, nhi);
     __syncthreads();
     r.all = out->all;
-    r.last = min(out->last, kMBins - 1);
+    r.last = out->last;
     r.all = min(r.all, min(r.bk, r.last));
     r.last = min(r.last, r.bk);
   } else {
@@ -491,143 +593,199 @@ __device__ __forceinline__ RowCut row_cut(const SampWs& ws, int row, const SampR
   return r;
 }
 
+// Values that another workgroup of the same launch reads: written through to and read from where all XCDs see them, so
+// that no fence has to write a whole L2 back (with a fence on each side 32 top-p rows took 69 us instead of 33).
 template <typename T>
-__global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restrict__ logits, int V, int chunk,
-                                                               SampArgs a, int row0, SampWs ws) {
-  __shared__ unsigned long long pm[kMBins], wm[4];
-  __shared__ uint32_t pc[kMBins], wc[4];
-  __shared__ RowCut cut;
-  __shared__ float sv[4];
-  __shared__ int si[4];
-  const int row = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+__device__ __forceinline__ void put_shared(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T get_shared(T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The listed tokens of a row (thread t: the t-th of n <= kListCap) against the exact counts and masses above them;
+// those that stay compete with (gb, gi), every wave's best so far.
+struct FinalScratch {
+  struct {
+    uint32_t key, bin;
+    unsigned long long w;
+  } e[kListCap];
+  unsigned long long above[kListCap], zk;
+  uint32_t more[kListCap];
+};
+__device__ __forceinline__ void final_listed(const Listed& e, int n, const RowScale& rs, const RowInfo& info,
+                                             const SampRow& rp, bool hk, bool hp, FinalScratch& f, float& gb, int& gi) {
+  const int t = threadIdx.x;
+  const bool in = t < n;
+  const float v = key2f((uint32_t)(e.id >> 32));
+  const int b = rs.bin(v);
+  const unsigned long long w = rs.weight(v);
+  if (in) {
+    f.e[t] = {(uint32_t)(e.id >> 32), (uint32_t)b, w};
+    f.above[t] = 0;
+    f.more[t] = 0;
+  }
+  if (t == 0) f.zk = 0;
+  __syncthreads();
+  // mass and count of the tokens above each listed one in its bin: the workgroup's threads over (token, part)
+  const int parts = kChThreads / n, i = t % n, part = t / n;
+  if (part < parts) {
+    const uint32_t key = f.e[i].key, bin = f.e[i].bin;
+    unsigned long long m = 0;
+    uint32_t c = 0;
+#pragma unroll 4
+    for (int j = part; j < n; j += parts) {
+      const auto o = f.e[j];
+      const bool over = o.bin == bin && o.key > key;
+      m += over ? o.w : 0;
+      c += over;
+    }
+    if (m) atomicAdd(&f.above[i], m);
+    if (c) atomicAdd(&f.more[i], c);
+  }
+  __syncthreads();
+  const bool keep_k = in && (!hk || e.pc + f.more[t] < (uint32_t)rp.k);
+  if (hk) {
+    if (keep_k && b == info.bk) atomicAdd(&f.zk, w);
+    __syncthreads();
+  }
+  const unsigned long long z = hk ? info.pmk + f.zk : info.tot;
+  const bool lim = hp && info.tot > 0 && rp.p > 0.f;
+  if (keep_k && (!lim || (double)(e.pm + f.above[t]) < (double)rp.p * (double)z))
+    pick(gb, gi, gumbel_score(v, 1.f / rp.temp, rp.seed, rp.step, (int)(uint32_t)e.id), (int)(uint32_t)e.id);
+}
+
+// Picks over a row's chunks; the workgroup that comes last to a row's counter, with all of its lists in memory, ends
+// it (rows without cuts: the first chunk's, from what the launches before left).
+template <typename T>
+__global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restrict__ logits, int64_t* __restrict__ out,
+                                                               int V, int chunk, SampArgs a, int row0, SampWs ws) {
+  __shared__ union {
+    struct {
+      unsigned long long pm[kMBins], wm[kChThreads / 64], own[kListCap];
+      uint32_t pc[kMBins], wc[kChThreads / 64];
+      RowCut cut;
+    } c;
+    FinalScratch f;
+    SampScratch slow;
+  } sh;
+  static_assert(kSampThreads == kChThreads && kListCap == kChThreads, "one workgroup shape; a thread a listed token");
+  __shared__ uint32_t nown, at0, last;
+  __shared__ float sv[kChThreads / 64];
+  __shared__ int si[kChThreads / 64];
+  const int row = blockIdx.y, nch = gridDim.x, t = threadIdx.x, lane = t & 63;
   const SampRow rp = samp_row(a, row0 + row);
-  if (!(rp.temp > 0.f)) return;
-  const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f;
-  const RowScale rs = row_scale(ws, row, gridDim.x, rp.temp);
-  RowCut r{kMBins, kMBins - 1, kMBins};
-  if (hk || hp) r = row_cut<kChThreads>(ws, row, rp, hk, hp, pm, pc, wm, wc, &cut);
+  const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f, cutting = rp.temp > 0.f && (hk || hp);
+  const T* x = logits + (size_t)row * V;
+  if (!cutting && blockIdx.x) return;
+  const Bins bins(ws, row, cutting && hk, cutting && hp);
+  const int c0 = blockIdx.x * chunk;
+  const Chunk<T> ch(x, c0, min(V, c0 + chunk));
+  typename Chunk<T>::P p = {};
+  if (cutting) p = ch.first();  // on its way while the cut is found
+  const RowScale rs = row_scale(ws, row, nch, rp.temp);
+  auto end = [&](float gb, int gi) {  // thread 0
+    out[row] = gi < V ? gi : (rs.mi < V ? rs.mi : 0);
+  };
+  if (!cutting) {
+    float gb = lane < nch && rp.temp > 0.f ? ws.gv[row * kMaxCh + lane] : -INFINITY;
+    int gi = lane < nch && rp.temp > 0.f ? ws.gi[row * kMaxCh + lane] : 0x7fffffff;
+    wave_pick(gb, gi);
+    if (t == 0) end(gb, gi);
+    return;
+  }
+  if (t == 0) nown = 0;
+  RowInfo info;
+  const RowCut r = row_cut(bins, rp, hk, hp, sh.c.pm, sh.c.pc, sh.c.wm, sh.c.wc, &sh.c.cut, info.tot);
+  info.pmk = r.klo;
+  info.bk = r.bk;
   const float inv_t = 1.f / rp.temp;
   float gb = -INFINITY;
   int gi = 0x7fffffff;
-  const int c0 = blockIdx.x * chunk;
-  each_in(logits + (size_t)row * V, c0, min(V, c0 + chunk), [&](int i, float v) {
-    const int b = hk || hp ? rs.bin(v) : 0;
+  auto token = [&](int i, float v) {
+    const int b = rs.bin(v);
     if (b < r.all) {
       pick(gb, gi, gumbel_score(v, inv_t, rp.seed, rp.step, i), i);
     } else if (b <= r.last || b == r.bk) {
-      const uint32_t at = atomicAdd(&ws.nlist[row], 1u);
-      if (at < kListCap) ws.list[row * kListCap + at] = ((unsigned long long)okey(v) << 32) | (uint32_t)i;
+      const uint32_t n = atomicAdd(&nown, 1u);
+      if (n < kListCap) sh.c.own[n] = ((unsigned long long)okey(v) << 32) | (uint32_t)i;
     }
-  });
-  wave_pick(gb, gi);
-  if (lane == 0) { sv[wv] = gb; si[wv] = gi; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kChThreads / 64; ++w) pick(gb, gi, sv[w], si[w]);
-    ws.gv[row * kMaxCh + blockIdx.x] = gb;
-    ws.gi[row * kMaxCh + blockIdx.x] = gi;
+  };
+  // Most tokens lie further from the largest than the last bin that counts reaches: a difference and a comparison
+  // mark the others (and not-a-numbers), which then go one a lane and turn.  With bins for all, and a score at each of
+  // a wave's 16 places that any lane keeps, 32 top-p rows took 36 us, now 33.
+  const int lim = max(max(r.last, hk ? r.bk : 0), r.all - 1);
+  const float far = lim >= kMBins - 1 ? INFINITY : (float)(lim + 1) / (rs.c * rs.scale) * 1.0001f + 1e-30f;
+  ch.ends(token);
+  for (int at = ch.start(); at < ch.ve; at += 2 * ch.S) {
+    if (at != ch.start()) p = ch.load(at);
+    uint32_t near = 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) near |= !(rs.mx - p.at(j) > far) ? 1u << j : 0u;
+    if (at + ch.S >= ch.ve) near &= 0xffu;
+    for (; near; near &= near - 1) {
+      const int j = __builtin_ctz(near);
+      float v = p.at(0);
+#pragma unroll
+      for (int k = 1; k < 16; ++k) v = j == k ? p.at(k) : v;
+      token(at + (j & 7) + (j & 8 ? ch.S : 0), v);
+    }
   }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kSampThreads) samp_final_kernel(const T* __restrict__ logits,
-                                                                  int64_t* __restrict__ out, int V, int nch,
-                                                                  SampArgs a, int row0, SampWs ws) {
-  __shared__ union {
-    SampScratch slow;
-    struct {
-      unsigned long long pm[kMBins], wm[16], w[kListCap], above[kListCap], zk;
-      uint32_t pc[kMBins], wc[16], key[kListCap], idx[kListCap], more[kListCap];
-      uint16_t bin[kListCap];
-      RowCut cut;
-      float red[16];
-      int redi[16];
-    } f;
-  } sh;
-  const int row = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  const SampRow rp = samp_row(a, row0 + row);
-  const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f;
-  if (rp.temp > 0.f && (hk || hp) && ws.nlist[row] > kListCap) {
-    const int id = topkp_row(logits + (size_t)row * V, V, rp, sh.slow);
+  group_pick(gb, gi, sv, si);  // its barrier: the workgroup's list is whole
+  const uint32_t mine = nown;
+  if (t == 0) {
+    put_shared(&ws.gv[row * kMaxCh + blockIdx.x], gb);
+    put_shared(&ws.gi[row * kMaxCh + blockIdx.x], gi);
+    at0 = mine ? atomicAdd(&ws.nlist[row], mine) : 0;
+  }
+  if (mine) {
+    __syncthreads();
+    if (t < mine && at0 + t < kListCap) {
+      const unsigned long long id = sh.c.own[t];
+      const int b = rs.bin(key2f((uint32_t)(id >> 32)));
+      Listed* l = ws.list + row * kListCap + at0 + t;
+      put_shared(&l->id, id);
+      put_shared(&l->pm, sh.c.pm[b]);
+      put_shared(&l->pc, sh.c.pc[b]);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // every wave: what it wrote is where all XCDs see it
+  __syncthreads();
+  if (t == 0) last = atomicAdd(&ws.done[row], 1u) == (uint32_t)nch - 1;
+  __syncthreads();
+  if (!last) return;
+  const int n = (int)get_shared(&ws.nlist[row]);
+  Listed* l = ws.list + row * kListCap + t;  // asked for with its count: past it, used by no one
+  const Listed e{get_shared(&l->id), get_shared(&l->pm), get_shared(&l->pc), 0};
+  gb = lane < nch ? get_shared(&ws.gv[row * kMaxCh + lane]) : -INFINITY;
+  gi = lane < nch ? get_shared(&ws.gi[row * kMaxCh + lane]) : 0x7fffffff;
+  if (n > kListCap) {
+    const int id = topkp_row(x, V, rp, sh.slow);
     if (t == 0) out[row] = id;
     return;
   }
-  const RowScale rs = row_scale(ws, row, nch, rp.temp);
-  if (!(rp.temp > 0.f)) {
-    if (t == 0) out[row] = rs.mi < V ? rs.mi : 0;
-    return;
-  }
-  float gb = lane < nch ? ws.gv[row * kMaxCh + lane] : -INFINITY;
-  int gi = lane < nch ? ws.gi[row * kMaxCh + lane] : 0x7fffffff;
-  if (hk || hp) {
-    const int n = (int)ws.nlist[row];
-    row_cut<kSampThreads>(ws, row, rp, hk, hp, sh.f.pm, sh.f.pc, sh.f.wm, sh.f.wc, &sh.f.cut);
-    const int bk = [&] {  // row_cut leaves it in place
-      __syncthreads();
-      return sh.f.cut.bk;
-    }();
-    unsigned long long tot = 0;
-    for (int w = 0; w < kSampThreads / 64; ++w) tot += sh.f.wm[w];
-    for (int i = t; i < n; i += kSampThreads) {
-      const unsigned long long e = ws.list[row * kListCap + i];
-      const float v = key2f((uint32_t)(e >> 32));
-      sh.f.key[i] = (uint32_t)(e >> 32);
-      sh.f.idx[i] = (uint32_t)e;
-      sh.f.bin[i] = (uint16_t)rs.bin(v);
-      sh.f.w[i] = rs.weight(v);
-      sh.f.above[i] = 0;
-      sh.f.more[i] = 0;
-    }
-    if (t == 0) sh.f.zk = 0;
-    __syncthreads();
-    // mass and count of the tokens above each listed one in its bin: the workgroup's threads over (token, part)
-    if (n > 0) {
-      const int parts = max(1, kSampThreads / n), i = t % n, part = t / n;
-      if (part < parts) {
-        const uint32_t key = sh.f.key[i];
-        const uint16_t bin = sh.f.bin[i];
-        unsigned long long m = 0;
-        uint32_t c = 0;
-        for (int j = part; j < n; j += parts)
-          if (sh.f.bin[j] == bin && sh.f.key[j] > key) { m += sh.f.w[j]; ++c; }
-        if (m) atomicAdd(&sh.f.above[i], m);
-        if (c) atomicAdd(&sh.f.more[i], c);
-      }
-    }
-    __syncthreads();
-    const bool in = t < n;
-    const int b = in ? sh.f.bin[t] : 0;
-    const bool keep_k = in && (!hk || sh.f.pc[b] + sh.f.more[t] < (uint32_t)rp.k);
-    if (hk && keep_k && b == bk) atomicAdd(&sh.f.zk, sh.f.w[t]);
-    __syncthreads();
-    const unsigned long long z = hk ? sh.f.pm[bk] + sh.f.zk : tot;
-    const bool lim = hp && tot > 0 && rp.p > 0.f;
-    if (keep_k && (!lim || (double)(sh.f.pm[b] + sh.f.above[t]) < (double)rp.p * (double)z))
-      pick(gb, gi, gumbel_score(key2f(sh.f.key[t]), 1.f / rp.temp, rp.seed, rp.step, (int)sh.f.idx[t]),
-           (int)sh.f.idx[t]);
-  }
-  wave_pick(gb, gi);
-  __syncthreads();
-  if (lane == 0) { sh.f.red[wv] = gb; sh.f.redi[wv] = gi; }
-  __syncthreads();
-  if (t == 0) {
-    for (int w = 1; w < kSampThreads / 64; ++w) pick(gb, gi, sh.f.red[w], sh.f.redi[w]);
-    out[row] = gi < V ? gi : (rs.mi < V ? rs.mi : 0);
-  }
+  if (n > 0) final_listed(e, n, rs, info, rp, hk, hp, sh.f, gb, gi);
+  group_pick(gb, gi, sv, si);
+  if (t == 0) end(gb, gi);
 }
 
 }  // namespace mx
 
 using namespace mx;
 
-static int samp_chunks(int V) { return std::min(kMaxCh, (V + 4095) / 4096); }
+// Chunks of a row: as many workgroups of 1,024 threads as CUs over all rows, each with at least 8,192 logits (one
+// 16-B piece a thread) and every chunk with a histogram of its own to clear, add up and scan.
+static int samp_chunks(int B, int V) {
+  return std::max(1, std::min({kMaxCh, (256 + B - 1) / B, (V + 8191) / 8192}));
+}
 static bool samp_split(int V) { return V >= kSplitV && V <= kSplitMaxV; }
 
 // bytes of workspace of one call of mx_sample_rows / mx_sample_list
 extern "C" int64_t mx_sample_rows_ws(int B, int V) {
   if (!samp_split(V)) return 0;
   const int64_t rows = std::min(B, kSampGroup);
-  return rows * (kMBins * 12 + kListCap * 8 + kMaxCh * 20 + 8);
+  return rows * (kMBins * 12 + kListCap * (int64_t)sizeof(Listed) + kMaxCh * 20 + 8);
 }
 
 template <typename T>
@@ -644,7 +802,7 @@ static void samp_launch(const T* x, int64_t* out, int B, int V, const SampArgs& 
   const size_t R = B;
   SampWs ws;
   ws.mass = (unsigned long long*)w;
-  ws.list = ws.mass + R * kMBins;
+  ws.list = (Listed*)(ws.mass + R * kMBins);
   ws.cnt = (uint32_t*)(ws.list + R * kListCap);
   ws.mx = (float*)(ws.cnt + R * kMBins);
   ws.mn = ws.mx + R * kMaxCh;
@@ -652,12 +810,12 @@ static void samp_launch(const T* x, int64_t* out, int B, int V, const SampArgs& 
   ws.mi = (int*)(ws.gv + R * kMaxCh);
   ws.gi = ws.mi + R * kMaxCh;
   ws.nlist = (uint32_t*)(ws.gi + R * kMaxCh);
-  const int nch0 = samp_chunks(V), chunk = ((V + nch0 - 1) / nch0 + 7) / 8 * 8, nch = (V + chunk - 1) / chunk;
+  ws.done = ws.nlist + R;
+  const int nch0 = samp_chunks(B, V), chunk = ((V + nch0 - 1) / nch0 + 7) / 8 * 8, nch = (V + chunk - 1) / chunk;
   const dim3 grid(nch, B);
   samp_stats_kernel<T><<<grid, kChThreads, 0, stream>>>(x, V, chunk, ws);
   samp_hist_kernel<T><<<grid, kChThreads, 0, stream>>>(x, V, chunk, a, row0, ws);
-  samp_pick_kernel<T><<<grid, kChThreads, 0, stream>>>(x, V, chunk, a, row0, ws);
-  samp_final_kernel<T><<<B, kSampThreads, 0, stream>>>(x, out, V, nch, a, row0, ws);
+  samp_pick_kernel<T><<<grid, kChThreads, 0, stream>>>(x, out, V, chunk, a, row0, ws);
 }
 
 // logits [B, V] bf16 (is_bf16) or f32; per-row parameters (device arrays of B):

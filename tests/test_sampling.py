@@ -260,3 +260,21 @@ def test_concurrent_mixed_samplers_on_two_streams(gpu):
                 got[k].append(draw(k, step))
     torch.cuda.synchronize(gpu)
     assert all(torch.equal(a, b) for k in range(2) for a, b in zip(got[k], want[k]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,dtype", [(16384, torch.bfloat16), (16389, torch.bfloat16), (50257, torch.float32)])
+def test_gpu_split_sampler_does_not_depend_on_the_batch(gpu, V, dtype):
+    """Rows by themselves, in sevens and all 70 at once (other chunks of a row, other alignments of its start): the masses
+    are sums of integers, so every way draws the same tokens."""
+    B = 70
+    x = (torch.randn(B, V, generator=torch.Generator().manual_seed(V)) * 2.5).to(dtype).to(gpu)
+    ways = [(0.8, 0.9, 0), (0.7, 0.95, 50), (1.0, 1.0, 0), (1.3, 0.999, 0), (0.0, 1.0, 0), (0.9, 1.0, 3000)]
+    temps, tops, ks = zip(*(ways[i % 6] for i in range(B)))
+
+    def draw(n):
+        return torch.cat([dops.sample_rows(x[i:i + n], temps[i:i + n], tops[i:i + n], ks[i:i + n], range(i, min(B, i + n)),
+                                           [9] * min(n, B - i)) for i in range(0, B, n)])
+
+    want = draw(70)
+    assert torch.equal(draw(1), want) and torch.equal(draw(7), want)
