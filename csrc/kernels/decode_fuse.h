@@ -102,10 +102,6 @@ __device__ __forceinline__ void dfuse_norm_rows(const uint16_t* __restrict__ X, 
   __syncthreads();
 }
 
-// LDS traffic of this wave done, then the workgroup's barrier: loads from memory stay in flight (__syncthreads waits
-// for them)
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // The same for a caller that stays (stream_gemm.hip), at 40 registers more.
 // What it reads of the first 4096 columns is asked for before `ahead`, the caller's first weight loads: loads return
 // in order, so that the norm would wait for weights asked for before it, and those after it for the norm.

@@ -12,40 +12,13 @@
 //                values, the pair rotation and the KV-cache append on the 4 consecutive channels a
 //                lane holds; the gate's channels go out as they are.
 // Each replaces two to four launches of a decode step.
-#include "conv_rope.h"
-#include "hybrid.h"
+#include "hybrid_fuse.h"
 #include "skinny_core.h"
 
 namespace mx {
 
 enum { kProNone, kProNorm, kProPoly };
 enum { kEpiPlain, kEpiGru, kEpiConv };
-
-struct HsNorm {
-  const uint16_t* delta;  // [M, K] or nullptr
-  int64_t ldd;
-  const float* h;         // [M, K] f32 residual
-  const float* gamma;     // [K]
-  float* h_out;           // [M, K]: h + delta (when delta)
-  int groups;
-  float eps;
-};
-struct HsPoly {
-  const float* coef;
-  float eps;
-};
-struct HsGru {
-  const float* bias;      // [2 W]: z | u
-  const int32_t* slots;
-  float* state;           // [slots, W]
-  int W;
-};
-struct HsConv {
-  ConvRope a;             // x unused; q [M, H, Dp]
-  const int32_t* pos;
-  const int32_t* slots;
-  uint16_t* gate;         // [M, H E]
-};
 
 constexpr int kHsMaxChunks = 4;  // 8-element pieces per thread: M K <= 512 * 8 * 4
 
@@ -144,99 +117,27 @@ __device__ __forceinline__ void hs_poly_rows(const uint16_t* __restrict__ z, int
   }
 }
 
-// lane (c, g): v[i] = projection g (z, u, gate) of channel 4 blk + i for token c
-__device__ __forceinline__ void hs_gru_store(const f32x4& v, int lane, int M, int blk, const HsGru& gr, uint16_t* Y) {
-  f32x4 u, gt;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    u[i] = __shfl(v[i], (lane & 15) + 16, 64);
-    gt[i] = __shfl(v[i], (lane & 15) + 32, 64);
-  }
-  const int m = lane & 15, c = blk * 4;
-  if (lane < 16 && m < M) {
-    float* sp = gr.state + (int64_t)gr.slots[m] * gr.W + c;
-    float bz[4], bu[4], s[4], o[4];
-    ldv<4>(gr.bias + c, bz);
-    ldv<4>(gr.bias + gr.W + c, bu);
-    ldv<4>(sp, s);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float keep, add;
-      mingru_gate<uint16_t>(v[i] + bz[i], u[i] + bu[i], keep, add);
-      s[i] = keep * s[i] + add;
-      o[i] = s[i] * (gt[i] * sigmoid_t<uint16_t>(gt[i]));
-    }
-    stv<4>(sp, s);
-    stv<4>(Y + (int64_t)m * gr.W + c, o);
-  }
-}
-
-// v: channels [ch, ch + 4) of token m, all of one section and head
-__device__ __forceinline__ void hs_conv_store(const f32x4& v, int ch, int m, int M, const HsConv& cv) {
-  if (m >= M) return;
-  const ConvRope& a = cv.a;
-  const int qk = (a.H + a.G) * a.D, C = qk + a.G * a.E;
-  float u[4], y[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) u[i] = bf2f(f2bf(v[i]));  // the projection as the ring stores it
-  if (ch >= C) {
-    stv<4>(cv.gate + (int64_t)m * a.H * a.E + (ch - C), u);
-    return;
-  }
-  const int p = cv.pos[m], slot = cv.slots[m];
-  uint16_t* ring = reinterpret_cast<uint16_t*>(a.ring) + (int64_t)slot * a.taps * C + ch;
-  float wv[4];
-  ldv<4>(a.w + (int64_t)(a.taps - 1) * C + ch, wv);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = wv[i] * u[i];
-  for (int back = 1; back < a.taps && back <= p; ++back) {
-    float o[4];
-    ldv<4>(ring + (int64_t)((p - back) % a.taps) * C, o);
-    ldv<4>(a.w + (int64_t)(a.taps - 1 - back) * C + ch, wv);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] += wv[i] * o[i];
-  }
-  stv<4>(ring + (int64_t)(p % a.taps) * C, u);
-  const int sec = ch < a.H * a.D ? 0 : ch < qk ? 1 : 2;
-  const int rel = sec == 0 ? ch : sec == 1 ? ch - a.H * a.D : ch - qk;
-  const int dim = sec < 2 ? a.D : a.E, Wp = sec < 2 ? a.Dp : a.Ep;
-  const int head = rel / dim, d0 = rel % dim;
-  if (sec < 2) {
-#pragma unroll
-    for (int i = 0; i < 4; i += 2) {
-      if (d0 + i + 1 < a.rd) {
-        const int64_t t = (int64_t)p * (a.rd >> 1) + ((d0 + i) >> 1);
-        const float c = a.cosb[t], s = a.sinb[t], e = y[i], f = y[i + 1];
-        y[i] = e * c - f * s;
-        y[i + 1] = f * c + e * s;
-      }
-    }
-  }
-  if (sec == 0) {
-    uint16_t* q = reinterpret_cast<uint16_t*>(a.q) + head * a.qh + (int64_t)m * a.qt;
-    stv<4>(q + d0, y);
-    if (d0 + 4 >= dim)
-      for (int d = dim; d < Wp; ++d) q[d] = 0;
-  } else {
-    uint16_t* cache = reinterpret_cast<uint16_t*>(sec == 1 ? a.kc : a.vc);
-    stv<4>(cache + kv_row(a.bt, a.maxb, a.block, slot, a.G, head, p % a.chunk) * Wp + d0, y);
-  }
-}
-
-template <int PRO, int EPI>
+template <int PRO, int EPI, int TB, int KP>
 __global__ void __launch_bounds__(512) hybrid_skinny_kernel(const uint16_t* __restrict__ X, int64_t ldx,
                                                             const uint16_t* __restrict__ W, int64_t ldw,
                                                             uint16_t* __restrict__ Y, int64_t ldy, int M, int K,
                                                             HsNorm na, HsPoly pp, HsGru gr, HsConv cv) {
-  __shared__ f32x4 red[kSkWaves][64];
+  typedef SkSum<TB, 1, KP> Sum;
+  constexpr int RB = Sum::RB;
+  __shared__ f32x4 red[Sum::PLACES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int blk = blockIdx.x, kq = K / kSkWaves, nit = kq / 64;
-  const int64_t row = EPI == kEpiGru ? (int64_t)min(c >> 2, 2) * gr.W + blk * 4 + (c & 3) : (int64_t)blk * 16 + c;
-  const uint16_t* wrow[1] = {W + row * ldw + (int64_t)w * kq + 16 * g};
-  const uint16_t* xr[1];
-  u16x8 apre[sk_unr(1)][1][2];
+  const int blk = blockIdx.x, kq = K / KP, nit = kq / 64;
+  const int64_t k0 = (int64_t)sk_part<KP>(w) * kq + sk_lane_k(c, g);
+  const uint16_t* wrow[RB];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int ch = 8 * sk_half<KP>(w, rb) + (c & 7);
+    wrow[rb] = W + (EPI == kEpiGru ? hs_gru_row(blk, ch, gr.W) : (int64_t)blk * 16 + ch) * ldw + k0;
+  }
+  const uint16_t* xr[TB];
+  u16x8 apre[sk_unr(1)][RB];
   if constexpr (PRO != kProNone) {
     extern __shared__ __attribute__((aligned(16))) uint16_t xs[];  // [M, K], then the norm's scratch
     sk_prefetch<1>(wrow, nit, apre);
@@ -247,18 +148,19 @@ __global__ void __launch_bounds__(512) hybrid_skinny_kernel(const uint16_t* __re
       __shared__ float pred[3][kSkWaves];
       hs_poly_rows(X, ldx, pp, M, K, xs, pred);
     }
-    xr[0] = xs + (int64_t)min(c, M - 1) * K + (int64_t)w * kq + 16 * g;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) xr[tb] = xs + (int64_t)min(8 * tb + (c & 7), M - 1) * K + k0;
   } else {
-    xr[0] = X + (int64_t)min(c, M - 1) * ldx + (int64_t)w * kq + 16 * g;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) xr[tb] = X + (int64_t)min(8 * tb + (c & 7), M - 1) * ldx + k0;
   }
-  f32x4 acc[1][1];
-  sk_stream<1, 1, PRO != kProNone>(wrow, xr, nit, apre, acc);
-  red[w][lane] = acc[0][0];
+  f32x4 acc[RB][TB];
+  sk_stream<TB, 1, PRO != kProNone>(wrow, xr, nit, apre, acc);
+  const Sum sum{red};
+  sum.put(w, c, g, acc);
   __syncthreads();
   if (w == 0) {
-    f32x4 s = red[0][lane];
-#pragma unroll
-    for (int ww = 1; ww < kSkWaves; ++ww) s += red[ww][lane];
+    const f32x4 s = sum.get(c, g, 0, 0);
     if constexpr (EPI == kEpiGru) {
       hs_gru_store(s, lane, M, blk, gr, Y);
     } else if constexpr (EPI == kEpiConv) {
@@ -270,6 +172,29 @@ __global__ void __launch_bounds__(512) hybrid_skinny_kernel(const uint16_t* __re
       *reinterpret_cast<u16x4*>(Y + (int64_t)c * ldy + blk * 16 + 4 * g) = o;
     }
   }
+}
+
+struct HsRun {
+  int groups;
+  size_t lds;
+  const uint16_t* x;
+  int64_t ldx;
+  const uint16_t* w;
+  int64_t ldw;
+  uint16_t* y;
+  int64_t ldy;
+  int M, K;
+};
+template <int PRO, int EPI>
+static void hs_launch(const HsRun& r, const HsNorm& na, const HsPoly& pp, const HsGru& gr, const HsConv& cv, hipStream_t stream) {
+#define HS_RUN(TB, KP) \
+  hybrid_skinny_kernel<PRO, EPI, TB, KP><<<r.groups, 512, r.lds, stream>>>(r.x, r.ldx, r.w, r.ldw, r.y, r.ldy, r.M, r.K, na, pp, gr, cv)
+  if (sk_parts(r.M, r.K) == 4) {
+    if (r.M <= 8) HS_RUN(1, 4); else HS_RUN(2, 4);
+  } else {
+    if (r.M <= 8) HS_RUN(1, 8); else HS_RUN(2, 8);
+  }
+#undef HS_RUN
 }
 
 static int hs_check(const uint16_t* x, int64_t ldx, int64_t ldw, int M, int K, int N) {
@@ -298,8 +223,7 @@ extern "C" int mx_hs_norm_gemm(const uint16_t* delta, int64_t ldd, const float* 
   if (M <= 0) return 0;
   const HsNorm na{delta, ldd, h, gamma, h_out, groups, eps};
   if (hs_check(nullptr, 0, ldw, M, K, N) || hs_norm_check(na, M, K) || N % 16 || ldy % 4 || ldy < N) return -1;
-  hybrid_skinny_kernel<kProNorm, kEpiPlain><<<N / 16, 512, hs_norm_lds(M, K, groups), stream>>>(
-      nullptr, 0, w, ldw, y, ldy, M, K, na, {}, {}, {});
+  hs_launch<kProNorm, kEpiPlain>({N / 16, hs_norm_lds(M, K, groups), nullptr, 0, w, ldw, y, ldy, M, K}, na, {}, {}, {}, stream);
   return (int)hipGetLastError();
 }
 
@@ -308,8 +232,7 @@ extern "C" int mx_hs_poly_gemm(const uint16_t* z, int64_t ldz, const float* coef
                                int64_t ldw, uint16_t* y, int64_t ldy, int M, int N, int K, hipStream_t stream) {
   if (M <= 0) return 0;
   if (hs_check(z, ldz, ldw, M, K, N) || (int64_t)M * K > 32768 || N % 16 || ldy % 4 || ldy < N) return -1;
-  hybrid_skinny_kernel<kProPoly, kEpiPlain><<<N / 16, 512, (size_t)M * K * 2, stream>>>(
-      z, ldz, w, ldw, y, ldy, M, K, {}, HsPoly{coef, eps}, {}, {});
+  hs_launch<kProPoly, kEpiPlain>({N / 16, (size_t)M * K * 2, z, ldz, w, ldw, y, ldy, M, K}, {}, HsPoly{coef, eps}, {}, {}, stream);
   return (int)hipGetLastError();
 }
 
@@ -324,10 +247,9 @@ extern "C" int mx_hs_gru_gemm(const uint16_t* x, int64_t ldx, int norm, const ui
     return -1;
   const HsGru gr{bias, slots, state, W};
   if (norm)
-    hybrid_skinny_kernel<kProNorm, kEpiGru><<<W / 4, 512, hs_norm_lds(M, K, groups), stream>>>(
-        nullptr, 0, w, ldw, y, W, M, K, na, {}, gr, {});
+    hs_launch<kProNorm, kEpiGru>({W / 4, hs_norm_lds(M, K, groups), nullptr, 0, w, ldw, y, W, M, K}, na, {}, gr, {}, stream);
   else
-    hybrid_skinny_kernel<kProNone, kEpiGru><<<W / 4, 512, 0, stream>>>(x, ldx, w, ldw, y, W, M, K, {}, {}, gr, {});
+    hs_launch<kProNone, kEpiGru>({W / 4, 0, x, ldx, w, ldw, y, W, M, K}, {}, {}, gr, {}, stream);
   return (int)hipGetLastError();
 }
 
@@ -339,18 +261,12 @@ extern "C" int mx_hs_conv_gemm(const uint16_t* x, int64_t ldx, int norm, const u
   if (M <= 0) return 0;
   const HsNorm na{delta, ldd, h, gamma, h_out, groups, eps};
   const ConvRope& a = *pa;
-  const int N = (a.H + a.G) * a.D + a.G * a.E + a.H * a.E;
+  const int N = hs_conv_rows(a);
   if (hs_check(norm ? nullptr : x, ldx, ldw, M, K, N) || (norm && hs_norm_check(na, M, K)) || (!norm && !x)) return -1;
-  if (N % 16 || a.D % 4 || a.E % 4 || a.Dp % 4 || a.Ep % 4 || a.rd % 2 || a.rd > a.D || a.H <= 0 || a.G <= 0 ||
-      a.H % a.G || a.taps < 1 || a.chunk <= 0 || a.block <= 0 || !a.ring || !a.kc || !a.vc || !a.bt || a.Dp < a.D ||
-      a.Ep < a.E)
-    return -1;
   const HsConv cv{a, pos, slots, gate};
   if (norm)
-    hybrid_skinny_kernel<kProNorm, kEpiConv><<<N / 16, 512, hs_norm_lds(M, K, groups), stream>>>(
-        nullptr, 0, w, ldw, nullptr, 0, M, K, na, {}, {}, cv);
+    hs_launch<kProNorm, kEpiConv>({N / 16, hs_norm_lds(M, K, groups), nullptr, 0, w, ldw, nullptr, 0, M, K}, na, {}, {}, cv, stream);
   else
-    hybrid_skinny_kernel<kProNone, kEpiConv><<<N / 16, 512, 0, stream>>>(x, ldx, w, ldw, nullptr, 0, M, K, {}, {}, {},
-                                                                           cv);
+    hs_launch<kProNone, kEpiConv>({N / 16, 0, x, ldx, w, ldw, nullptr, 0, M, K}, {}, {}, {}, cv, stream);
   return (int)hipGetLastError();
 }

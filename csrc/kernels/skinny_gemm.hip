@@ -4,14 +4,9 @@
 // 1.7-4.5 TB/s (archive/profiles/r2x_skinny_gemm.md), latency-bound: too few bytes in flight per CU.
 //
 // Same structure as the fp8 weight kernel (fp8_gemm.hip) without the dequantisation:
-//  * workgroup = 8 waves = 16 output channels; the waves split K in eight contiguous parts
-//    and meet in LDS; N/16 workgroups;
-//  * v_mfma_f32_16x16x32_bf16 with the WEIGHTS as the A operand (16 channels x 32 k) and X^T
-//    as the B operand (32 k x 16 tokens); lane (c, g) loads k = 16g .. 16g+15 of each 64-k
-//    chunk of channel c as two 16-B loads = the A fragments of the chunk's two MFMA k-steps,
-//    and the X fragments use the same k permutation;
-//  * 8 chunks' loads are issued before the first is used: 256 B of weights per lane in
-//    flight, 128 KB per workgroup.
+//  * workgroup = 8 waves = 16 output channels, N/16 workgroups; the waves split K (skinny_core.h) and meet in LDS;
+//  * v_mfma_f32_16x16x32_bf16 with the WEIGHTS as the A operand and X^T as the B operand;
+//  * 8 chunks' loads are issued before the first is used: 256 B of weights per lane in flight, 128 KB per workgroup.
 //  * SWO (SwiGLU output, the decode MLP's gate|up projection, W = [gate; up] [2F, K]): a
 //    workgroup's 16 channels are 8 gate rows n..n+7 and the matching 8 up rows F+n..F+n+7, so
 //    the epilogue holds both halves of its 8 outputs and writes silu(g) * u [M, F] directly
@@ -35,12 +30,13 @@
 
 namespace mx {
 
-// MB: 16-token blocks (1 or 2); X rows >= M are clamped to M-1 and discarded.
+// TB: 8-token blocks (1, 2 or 4); X rows >= M are clamped to M-1 and discarded.
 // NC: 16-channel groups per workgroup: each X fragment then feeds NC MFMAs, so X traffic per
 // streamed weight byte drops NC-fold (it equals the weight traffic at 16 tokens with NC = 1).
-// HALF: 8 channels a workgroup (M <= 8): fragment row r takes channel r & 7 and half r >> 3 of the wave's K part,
-// token column c token c & 7 and the same half, and the two diagonal blocks of the product are added.
-template <int MB, int NC, bool SWO = false, bool NORM = false, bool ROPE = false, bool MERGE = false, bool HALF = false>
+// KP: K parts (sk_parts).  HALF: 8 channels a workgroup, 8 K parts, M <= 8.  WIDE: 16-row fragments and TB blocks of 16 tokens
+// (sk_wide).
+template <int TB, int NC, int KP, bool SWO = false, bool NORM = false, bool ROPE = false, bool MERGE = false,
+          bool HALF = false, bool WIDE = false, bool DEEP = false>
 __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __restrict__ X, int64_t ldx,
                                                           const uint16_t* __restrict__ W, int64_t ldw,
                                                           uint16_t* __restrict__ Y, int64_t ldy, int M, int K,
@@ -48,31 +44,34 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
                                                           SkMerge mg = {}) {
   static_assert(!SWO || NC == 1, "SwiGLU epilogue: one channel group");
   static_assert(!ROPE || (NC == 1 && !SWO), "RoPE epilogue: one channel group");
-  static_assert(!NORM || (MB == 1 && NC == 1), "fused RMSNorm: <= 16 rows, one channel group");
-  static_assert(!MERGE || (MB == 1 && NC == 1 && !NORM && !SWO && !ROPE), "fused split merge: plain GEMM rows");
-  static_assert(!HALF || (MB == 1 && NC == 1 && !SWO && !NORM && !ROPE && !MERGE), "half groups: plain GEMM rows");
+  static_assert(!NORM || (TB == 1 && NC == 1), "fused RMSNorm: <= 8 rows, one channel group");
+  static_assert(!MERGE || (TB == 1 && NC == 1 && !NORM && !SWO && !ROPE), "fused split merge: plain GEMM rows");
+  static_assert(!HALF || (TB == 1 && NC == 1 && KP == 8 && !SWO && !NORM && !ROPE && !MERGE), "half groups: plain GEMM rows");
   constexpr bool LDSX = NORM || MERGE;  // X rows built in LDS by the prologue
-  constexpr int NW = kSkWaves, UNR = sk_unr(NC);
-  __shared__ f32x4 red[NW][NC][MB][64];
+  static_assert(!WIDE || (NC == 1 && KP == 8 && !NORM && !ROPE && !MERGE && !HALF), "16-row fragments: plain rows, SwiGLU");
+  constexpr int UNR = sk_unr(NC), RB = HALF ? 1 : kSkBlocks<KP, NC>, BT = WIDE ? 16 : 8;  // tokens of a block
+  typedef SkSum<TB, NC, KP> Sum;
+  __shared__ f32x4 red[HALF ? kSkWaves * 16 : WIDE ? kSkWaves * TB * 64 : Sum::PLACES];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (HALF ? 8 : 16 * NC);
-  const int kq = K / NW;  // this wave's K part
-  const int kh = HALF && c >= 8 ? kq / 2 : 0;
-  const uint16_t* wrow[NC];
+  const int kq = K / KP;  // this wave's K part
+  const int64_t k0 = (int64_t)sk_part<KP>(w) * kq + (WIDE ? 8 * g : sk_lane_k(c, g));
+  const uint16_t* wrow[RB];
 #pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    // SWO: channel c < 8 -> gate row blockIdx.x * 8 + c, c >= 8 -> the matching up row
-    // ROPE: head blockIdx.x / 8, pair base 8 (blockIdx.x % 8); c >= 8 -> the second-half row
-    const int64_t wr = (SWO || ROPE) ? dfuse_row<SWO>(blockIdx.x, c, F) : (int64_t)(n0 + 16 * j + (HALF ? c & 7 : c));
-    wrow[j] = W + wr * ldw + (int64_t)w * kq + kh + 16 * g;
+  for (int rb = 0; rb < RB; ++rb) {
+    const int ch = WIDE ? c : (HALF ? 0 : 8 * sk_half<KP>(w, rb)) + (c & 7), j = KP == 8 ? rb >> 1 : rb;
+    // SWO: channels 0 .. 7: gate rows blockIdx.x * 8 + ch, 8 .. 15: the matching up rows
+    // ROPE: head blockIdx.x / 8, pair base 8 (blockIdx.x % 8); channels 8 .. 15: the second-half rows
+    const int64_t wr = (SWO || ROPE) ? dfuse_row<SWO>(blockIdx.x, ch, F) : (int64_t)(n0 + 16 * j + ch);
+    wrow[rb] = W + wr * ldw + k0 + (WIDE ? 32 * rb : 0);
   }
-  const uint16_t* xr[MB];
-  const int nit = kq / (HALF ? 128 : 64);
+  const uint16_t* xr[TB];
+  const int nit = kq / 64;
   // NORM: the first UNR chunks' weight loads go out before the prologue, so the weight stream's
   // latency overlaps the RMSNorm instead of following it
-  u16x8 apre[UNR][NC][2];
+  u16x8 apre[UNR][RB];
   if constexpr (LDSX) sk_prefetch<NC>(wrow, nit, apre);
   if constexpr (LDSX) {
     extern __shared__ __attribute__((aligned(16))) uint16_t xs[];  // [M, K] normalised / merged rows
@@ -84,50 +83,89 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
       dfuse_merge_rows(M, K, mg, xs);
     }
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) xr[mb] = xs + (int64_t)min(mb * 16 + c, M - 1) * K + (int64_t)w * kq + 16 * g;
+    for (int tb = 0; tb < TB; ++tb) xr[tb] = xs + (int64_t)min(tb * 8 + (c & 7), M - 1) * K + k0;
   } else {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-      xr[mb] = X + (int64_t)min(mb * 16 + (HALF ? c & 7 : c), M - 1) * ldx + (int64_t)w * kq + kh + 16 * g;
+    for (int tb = 0; tb < TB; ++tb) xr[tb] = X + (int64_t)min(tb * BT + (c & (BT - 1)), M - 1) * ldx + k0;
   }
 
-  f32x4 acc[NC][MB];
-  sk_stream<MB, NC, LDSX>(wrow, xr, nit, apre, acc);
-  // C[row = channel 4g + i][col = token c] per (group, m-block): sum the NW K parts
+  f32x4 acc[RB][TB];
+  sk_stream<TB, NC, LDSX, WIDE, DEEP>(wrow, xr, nit, apre, acc);
+  if constexpr (HALF) {
+    const f32x4 part = sk_both_halves(acc[0][0]);
+    if (c < 8 && g < 2) red[w * 16 + 8 * g + c] = part;
+    __syncthreads();
+    if (w == 0 && g < 2 && c < M) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < NC; ++j)
+      for (int ww = 0; ww < kSkWaves; ++ww) s += red[ww * 16 + 8 * g + c];
+      u16x4 o;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) red[w][j][mb][lane] = acc[j][mb];
-  __syncthreads();
-  if (w == 0) {
+      for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+      *reinterpret_cast<u16x4*>(Y + (int64_t)c * ldy + n0 + 4 * g) = o;
+    }
+  } else {
+    const Sum sum{red};
+    if constexpr (WIDE) {
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
+      for (int tb = 0; tb < TB; ++tb) red[(w * TB + tb) * 64 + lane] = acc[0][tb];
+    } else {
+      sum.put(w, c, g, acc);
+    }
+    __syncthreads();
+    if (w == 0) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        f32x4 s = red[0][j][mb][lane];
+      for (int j = 0; j < NC; ++j)
 #pragma unroll
-        for (int ww = 1; ww < NW; ++ww) s += red[ww][j][mb][lane];
-        const int m = mb * 16 + c;
-        if constexpr (HALF) {  // (channel, token) of the first halves + (channel + 8, token + 8) of the second
-          u16x4 o;
+        for (int mb = 0; mb < (WIDE ? TB : (TB + 1) / 2); ++mb) {
+          f32x4 s = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (WIDE) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i] + __shfl_xor(s[i], 40, 64));
-          if (c < 8 && g < 2 && c < M) *reinterpret_cast<u16x4*>(Y + (int64_t)c * ldy + n0 + 4 * g) = o;
-        } else if constexpr (ROPE) {
-          dfuse_rope_store(s, g, m, M, blockIdx.x, rp);
-        } else if constexpr (SWO) {
-          dfuse_swiglu_store(s, g, m, M, Y, ldy, blockIdx.x);
-        } else if (m < M) {
-          u16x4 o;
+            for (int ww = 0; ww < kSkWaves; ++ww) s += red[(ww * TB + mb) * 64 + lane];
+          } else {
+            s = sum.get(c, g, j, mb);
+          }
+          const int m = mb * 16 + c;
+          if constexpr (ROPE) {
+            dfuse_rope_store(s, g, m, M, blockIdx.x, rp);
+          } else if constexpr (SWO) {
+            dfuse_swiglu_store(s, g, m, M, Y, ldy, blockIdx.x);
+          } else if (m < M) {
+            u16x4 o;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
-          *reinterpret_cast<u16x4*>(Y + (int64_t)m * ldy + n0 + 16 * j + 4 * g) = o;
+            for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+            *reinterpret_cast<u16x4*>(Y + (int64_t)m * ldy + n0 + 16 * j + 4 * g) = o;
+          }
         }
-      }
+    }
   }
 }
 
 }  // namespace mx
+
+// Where the kernel whose workgroups stay (stream_gemm.hip: X in LDS once a CU) has the same bits and takes less time (us, here ->
+// there: K 2048, 3 / 8 / 32 rows: 3072 channels 5.2 / 6.1 / 8.8 -> 5.1 / 5.3 / 8.5, 16384 13.8 / 17.0 / 29.7 -> 13.0 / 13.4 / 18.6,
+// 2 rows 12.8 -> 13.0; K 4096, 16 rows: 1024 channels 9.7 -> 9.1, 4096, one group a CU, 10.2 -> 10.5).
+extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
+                              int64_t ldy, int M, int N, int K, int epi, const uint16_t* delta, int64_t ldd,
+                              const uint16_t* gamma, float eps, uint16_t* h_out, const float* cosb, const float* sinb,
+                              const int32_t* pos, const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq,
+                              int Hkv, int max_seq, const int32_t* bt, int maxb, hipStream_t stream);
+static bool sk_stays(int M, int N, int K) {
+  return K == 2048 ? M > 2 : K == 4096 && M > 8 && M <= 16 && !(N > 3072 && N <= 4096);
+}
+// epi 0: plain, 1: SwiGLU (N = 2 F); -1: not taken
+static int sk_stream_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y, int64_t ldy, int M, int N,
+                          int K, int epi, hipStream_t stream) {
+  if (!sk_stays(M, N, K)) return -1;
+  return mx_stream_gemm(x, ldx, w, ldw, nullptr, y, ldy, M, N, K, epi, nullptr, 0, nullptr, 0.f, nullptr, nullptr, nullptr,
+                        nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0, stream);
+}
+
+// the kernel of the sizes' K parts: KERNEL(4) or KERNEL(8)
+#define SK_PARTS(KERNEL) \
+  if (sk_parts(M, K) == 4) KERNEL(4); \
+  else KERNEL(8)
 
 using namespace mx;
 
@@ -151,11 +189,22 @@ extern "C" int mx_skinny_rope_gemm(const uint16_t* h, int64_t ldh, int norm, con
   const SkRope rp{cosb, sinb, pos, slots, q, kc, vc, Hq, Hkv, max_seq, bt, maxb};
   if (norm) {
     const SkNorm na{delta, ldd, gamma, h_out, eps};
-    skinny_gemm_kernel<1, 1, false, true, true><<<N / 16, 512, (size_t)M * K * 2, stream>>>(
-        h, ldh, w, ldw, nullptr, 0, M, K, 0, na, rp);
+#define SKR(KP) skinny_gemm_kernel<1, 1, KP, false, true, true><<<N / 16, 512, (size_t)M * K * 2, stream>>>( \
+      h, ldh, w, ldw, nullptr, 0, M, K, 0, na, rp)
+    SK_PARTS(SKR);
+#undef SKR
   } else {
-    skinny_gemm_kernel<1, 1, false, false, true><<<N / 16, 512, 0, stream>>>(h, ldh, w, ldw, nullptr, 0, M, K, 0,
-                                                                               SkNorm{}, rp);
+#define SKR(KP) skinny_gemm_kernel<1, 1, KP, false, false, true><<<N / 16, 512, 0, stream>>>(h, ldh, w, ldw, nullptr, 0, M, K, \
+                                                                                            0, SkNorm{}, rp)
+#define SKR2(KP) skinny_gemm_kernel<2, 1, KP, false, false, true><<<N / 16, 512, 0, stream>>>(h, ldh, w, ldw, nullptr, 0, M, K, \
+                                                                                             0, SkNorm{}, rp)
+    if (M <= 8) {
+      SK_PARTS(SKR);
+    } else {
+      SK_PARTS(SKR2);
+    }
+#undef SKR
+#undef SKR2
   }
   return (int)hipGetLastError();
 }
@@ -172,8 +221,10 @@ extern "C" int mx_skinny_merge_gemm(const float* ml, const float* po, int nsplit
       nsplit < 1)
     return -1;
   const SkMerge mg{ml, po, nsplit};
-  skinny_gemm_kernel<1, 1, false, false, false, true><<<N / 16, 512, (size_t)M * K * 2, stream>>>(
-      nullptr, 0, w, ldw, y, ldy, M, K, 0, SkNorm{}, SkRope{}, mg);
+#define SKM(KP) skinny_gemm_kernel<1, 1, KP, false, false, false, true><<<N / 16, 512, (size_t)M * K * 2, stream>>>( \
+      nullptr, 0, w, ldw, y, ldy, M, K, 0, SkNorm{}, SkRope{}, mg)
+  SK_PARTS(SKM);
+#undef SKM
   return (int)hipGetLastError();
 }
 
@@ -190,10 +241,14 @@ extern "C" int mx_skinny_norm_gemm(const uint16_t* h, int64_t ldh, const uint16_
   if (swiglu) {
     const int Fh = N / 2;
     if (Fh % 8 || ldy < Fh) return -1;
-    skinny_gemm_kernel<1, 1, true, true><<<Fh / 8, 512, lds, stream>>>(h, ldh, w, ldw, y, ldy, M, K, Fh, na);
+#define SKN(KP) skinny_gemm_kernel<1, 1, KP, true, true><<<Fh / 8, 512, lds, stream>>>(h, ldh, w, ldw, y, ldy, M, K, Fh, na)
+    SK_PARTS(SKN);
+#undef SKN
   } else {
     if (ldy < N) return -1;
-    skinny_gemm_kernel<1, 1, false, true><<<N / 16, 512, lds, stream>>>(h, ldh, w, ldw, y, ldy, M, K, 0, na);
+#define SKN(KP) skinny_gemm_kernel<1, 1, KP, false, true><<<N / 16, 512, lds, stream>>>(h, ldh, w, ldw, y, ldy, M, K, 0, na)
+    SK_PARTS(SKN);
+#undef SKN
   }
   return (int)hipGetLastError();
 }
@@ -211,27 +266,53 @@ extern "C" int mx_skinny_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w,
     const char* e = getenv("MXLLM_SKINNY_NC");
     return e && *e ? atoi(e) : 0;
   }();
+  if (!nc_env && sk_stream_gemm(x, ldx, w, ldw, y, ldy, M, N, K, 0, stream) == 0) return 0;
   int nc = nc_env ? nc_env : 1;
   while (nc > 1 && (N % (16 * nc) || N / (16 * nc) < 128)) nc >>= 1;
-#define SKG(MBV, NCV) skinny_gemm_kernel<MBV, NCV><<<N / (16 * NCV), 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K)
-  if (M <= 16) {
-    if (nc >= 4) SKG(1, 4); else if (nc == 2) SKG(1, 2); else SKG(1, 1);
-  } else {
-    if (nc >= 4) SKG(2, 4); else if (nc == 2) SKG(2, 2); else SKG(2, 1);
+#define SKG(TBV, NCV, KPV) \
+  skinny_gemm_kernel<TBV, NCV, KPV><<<N / (16 * NCV), 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K)
+#define SKT(NCV, KPV) \
+  do { \
+    if (M <= 8) SKG(1, NCV, KPV); else if (M <= 16) SKG(2, NCV, KPV); else SKG(4, NCV, KPV); \
+  } while (0)
+  // up to two workgroups a CU (us, compiler's order -> DEEP, one row: 4096 x 4096 7.7 -> 7.6, 4096 x 14336 23.1 -> 21.9; 128256 x
+  // 2048 82 -> 88)
+  if (M <= 8 && nc == 1 && N <= 16 * 512) {
+#define SKD(KPV) \
+  skinny_gemm_kernel<1, 1, KPV, false, false, false, false, false, false, true><<<N / 16, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K)
+    SK_PARTS(SKD);
+#undef SKD
+    return (int)hipGetLastError();
   }
+#define SKC(KPV) \
+  do { \
+    if (nc >= 4) SKT(4, KPV); else if (nc == 2) SKT(2, KPV); else SKT(1, KPV); \
+  } while (0)
+  if (sk_wide(M, K) && nc == 1) {
+    if (M <= 16) skinny_gemm_kernel<1, 1, 8, false, false, false, false, false, true><<<N / 16, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+    else skinny_gemm_kernel<2, 1, 8, false, false, false, false, false, true><<<N / 16, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+    return (int)hipGetLastError();
+  }
+  SK_PARTS(SKC);
+#undef SKC
+#undef SKT
 #undef SKG
   return (int)hipGetLastError();
 }
 
 // The same for up to 8 rows by groups of 8 channels (HALF): twice the workgroups, where 16 channels each leave CUs
-// without one.  2048 channels, one row: K 8192 13.1 -> 10.0 us, K 12288 19.2 -> 13.0, K 2048 5.1 -> 4.1 (8 rows:
-// 15.0 -> 12.9, 21.9 -> 17.3, 5.4 -> 4.7).  The halves of a wave's K part are summed apart: other bits than above.
+// without one.  2048 channels, one row: K 8192 10.5 -> 8.0 us, K 12288 14.5 -> 11.0, K 2048 4.5 -> 3.7 (8 rows:
+// 13.1 -> 9.9, 18.5 -> 14.0, 5.8 -> 4.4).  Always 8 K parts: for a K of 2048 other bits than above.
 // K % 1024 == 0, N % 8 == 0.
 extern "C" int mx_skinny_gemm_half(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y,
                                    int64_t ldy, int M, int N, int K, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > 8 || N % 8 || K % 1024 || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K || ldw < K || ldy < N) return -1;
-  skinny_gemm_kernel<1, 1, false, false, false, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+  // DEEP up to where the waves that it leaves are busy (2048 x 2048, one row 3.9 -> 3.7 us, 4096 x 4096 7.7 -> 7.5, 2048 x 8192 8.0 -> 8.4)
+  if (K <= 4096)
+    skinny_gemm_kernel<1, 1, 8, false, false, false, false, true, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+  else
+    skinny_gemm_kernel<1, 1, 8, false, false, false, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
   return (int)hipGetLastError();
 }
 
@@ -242,9 +323,19 @@ extern "C" int mx_skinny_gemm_swiglu(const uint16_t* x, int64_t ldx, const uint1
                                      int64_t ldy, int M, int F, int K, hipStream_t stream) {
   if (M <= 0) return 0;
   if (M > 32 || F % 8 || K % 512 || ldx % 8 || ldw % 8 || ldy % 4 || ldx < K || ldw < K || ldy < F) return -1;
-  if (M <= 16)
-    skinny_gemm_kernel<1, 1, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F);
-  else
-    skinny_gemm_kernel<2, 1, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F);
+  if (sk_stream_gemm(x, ldx, w, ldw, y, ldy, M, 2 * F, K, 1, stream) == 0) return 0;
+#define SKS(TBV, KPV) skinny_gemm_kernel<TBV, 1, KPV, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F)
+#define SKT(KPV) \
+  do { \
+    if (M <= 8) SKS(1, KPV); else if (M <= 16) SKS(2, KPV); else SKS(4, KPV); \
+  } while (0)
+  if (sk_wide(M, K)) {
+    if (M <= 16) skinny_gemm_kernel<1, 1, 8, true, false, false, false, false, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F);
+    else skinny_gemm_kernel<2, 1, 8, true, false, false, false, false, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F);
+    return (int)hipGetLastError();
+  }
+  SK_PARTS(SKT);
+#undef SKT
+#undef SKS
   return (int)hipGetLastError();
 }

@@ -6,27 +6,26 @@
 // bytes as the weights' at 16 rows (at 8 for e4m3), through the same load queue.  Here a workgroup stages X in LDS
 // once (2 M K bytes) and walks over channel groups; only weights are left in the queue, and the next block of them
 // is in flight while the last one is multiplied and summed.
-//  * 8 waves split K in eight contiguous parts, 64-k chunks of two v_mfma_f32_16x16x32_bf16 with the weights as
-//    the A operand, partial sums in wave order: the products and sums of the kernels above, bit for bit;
+//  * fragments, K parts and sums of skinny_core.h, or of fp8_gemm.hip for e4m3: the products and sums of the kernels
+//    above, bit for bit;
 //  * X is asked for in front of the first weights and worked on behind them: loads return in order, and __syncthreads
 //    waits for all of them (with the weights in front and that barrier, 6144 x 4096 at 16 rows 17.6 us in a step, now
 //    14.8; the e4m3 gate-up projection of 4 rows with its norm 26.5, now 23.6);
-//  * blocks of U chunks, two in flight: 8 (K a multiple of 4096) or 4 (of 2048): 128 or 64 registers, so that
-//    with up to 80 KB of LDS two workgroups share a CU;
+//  * blocks of 16 loads (K a multiple of 4096) or 8 (of 2048), two in flight: 128 or 64 registers, so that with up to
+//    80 KB of LDS two workgroups share a CU;
 //  * LDS rows are K + 8 long: the 16 rows that a fragment read touches start 4 banks apart;
 //  * the waves take turns at a group's sum and epilogue (two LDS images, one barrier a group), the others go on;
 //  * epilogues: plain, SwiGLU (8 gate and the matching 8 up channels), RoPE + cache append (heads of 64 or 128);
 //    prologue: the RMSNorm with the residual add, up to 4 rows (decode_fuse.h).
-// 28672 x 4096 (235 MB) with SwiGLU, rows 1 / 4 / 8 / 16: 42.6 / 42.9 / 43.3 / 43.8 us (5.5 TB/s) against skinny_gemm's
-// 43.6 / 47.3 / 54.9 / 67.1 and hipBLASLt's 67; in e4m3, rows 1 / 4 / 8: 24.9 / 25.8 / 28.6 against fp8_gemm's 28.4 / 32.2
-// / 36.4.  128256 x 2048, 8 rows: 98 against 109 and 114.
-// Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 14.8 us for 50 MB; the last 128 as
-// 256 halves: no change, a half's loads take a whole one's turns).
+// 28672 x 4096 (235 MB), rows 1 / 4 / 8 / 16: 39.4 / 39.6 / 39.4 / 41.4 us (6.0 TB/s; in fragments of 16 rows x 64 B 43.0 / 43.5 /
+// 43.7 / 44.4) against skinny_gemm's 39.8 / 41.0 / 42.8 / 54.6 and hipBLASLt's 61 to 64; 16384 x 2048 (67 MB), 4 / 8 / 16 rows 12.9 /
+// 13.4 / 15.4 (15.8 / 16.4 / 16.5); in e4m3, rows 1 / 4 / 8: 24.9 / 25.8 / 28.6 against fp8_gemm's 28.4 / 32.2 / 36.4.
+// Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 13.0 us for 50 MB; the last 128 as
+// 256 halves: no change, a half's loads take a whole one's turns), and the launch's own 2 us before the first bytes arrive.
 #include <algorithm>
 
 #include "decode_fuse.h"
-#include "e4m3.h"
-#include "skinny_core.h"
+#include "stream_core.h"
 
 namespace mx {
 
@@ -45,197 +44,92 @@ struct StreamArgs {
   SkRope rp;
 };
 
-template <bool F8, int U>
-struct WFrag {
-  u16x8 a[U][2];
-  __device__ __forceinline__ void load(const char* p) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      a[u][0] = *reinterpret_cast<const u16x8*>(p + u * 128);
-      a[u][1] = *reinterpret_cast<const u16x8*>(p + u * 128 + 16);
-    }
-  }
-  __device__ __forceinline__ void get(int u, u16x8& x, u16x8& y) const { x = a[u][0], y = a[u][1]; }
-};
-template <int U>
-struct WFrag<true, U> {
-  u32x4 a[U];
-  __device__ __forceinline__ void load(const char* p) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const u32x4*>(p + u * 64);
-  }
-  __device__ __forceinline__ void get(int u, u16x8& x, u16x8& y) const {
-    x = dequant8(a[u][0], a[u][1]);
-    y = dequant8(a[u][2], a[u][3]);
-  }
-};
+// workgroups of up to 128 registers: two a CU where LDS allows it (X of 9 rows and more of a K over 2048 does not)
+template <int KIND, int TB, int KP, int NL>
+constexpr int kStWaves = KIND == kStF8 ? (TB == 1 ? 4 : 2) : NL == 8 && (TB == 1 || KP == 4) ? 4 : 2;
 
-template <bool F8, int MB, int EPI, bool NORM, int U>
-__global__ void __launch_bounds__(512, MB == 1 && (F8 || U == 4) ? 4 : 2) stream_gemm_kernel(StreamArgs a) {
-  constexpr int NW = kSkWaves, NRED = MB == 1 ? 2 : 1, WB = F8 ? 1 : 2;
+template <int KIND, int TB, int KP, int EPI, bool NORM, int NL>
+__global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm_kernel(StreamArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int c = lane & 15, g = lane >> 4;
-  const int M = a.M, K = a.K, kq = K / NW, nblk = kq / (64 * U), ldx = K + 8;
-  f32x4(*red)[NW][MB][64] = reinterpret_cast<f32x4(*)[NW][MB][64]>(smem);
-  uint16_t* xs = reinterpret_cast<uint16_t*>(smem + sizeof(f32x4) * NRED * NW * MB * 64);
-  auto row = [&](int grp, int ch) -> int64_t {
-    if constexpr (EPI == kStSwiglu) return dfuse_row<true>(grp, ch, a.F);
-    else if constexpr (EPI == kStRope128) return dfuse_row<false, 64>(grp, ch, 0);
-    else if constexpr (EPI == kStRope64) return dfuse_row<false, 32>(grp, ch, 0);
-    else return (int64_t)grp * 16 + ch;
+  const int tid = threadIdx.x, c = tid & 15, g = tid >> 4 & 3;
+  const int M = a.M, K = a.K;
+  auto row = [&](int grp) __attribute__((always_inline)) -> int64_t {
+    if constexpr (EPI == kStSwiglu) return dfuse_row<true>(grp, 0, a.F);
+    else if constexpr (EPI == kStRope128) return dfuse_row<false, 64>(grp, 0, 0);
+    else if constexpr (EPI == kStRope64) return dfuse_row<false, 32>(grp, 0, 0);
+    else return (int64_t)grp * 16;
   };
-  // the block to load next: group lg, block lb
-  int lg = blockIdx.x, lb = 0;
-  const char* base = reinterpret_cast<const char*>(a.W) + ((int64_t)w * kq + 16 * g) * WB;
-  const char* lp = base + row(lg, c) * a.ldw * WB;
-  auto load = [&](WFrag<F8, U>& f) {
-    f.load(lp + (int64_t)lb * (U * 64 * WB));
-    if (++lb == nblk) {
-      lb = 0;
-      lg += gridDim.x;
-      lp = base + row(min(lg, a.groups - 1), c) * a.ldw * WB;
+  auto off = [&](int ch) __attribute__((always_inline)) -> int {
+    if constexpr (EPI == kStSwiglu) return (int)dfuse_row<true>(0, ch, a.F);
+    else if constexpr (EPI == kStRope128) return (int)dfuse_row<false, 64>(0, ch, 0);
+    else if constexpr (EPI == kStRope64) return (int)dfuse_row<false, 32>(0, ch, 0);
+    else return ch;
+  };
+  auto stage = [&](uint16_t* xs, int ldx, auto ahead) __attribute__((always_inline)) {
+    if constexpr (NORM) {
+      __shared__ float nscr[4][4];
+      dfuse_norm_ahead(a.X, a.ldx, M, K, a.na, xs, ldx, nscr, ahead);
+    } else {
+      stream_rows_in<KIND != kStF8 && NL == 16 ? 16 : 8>(a.X, a.ldx, M, K, xs, ldx, ahead);
     }
   };
-  WFrag<F8, U> f0, f1;
-  // the first block goes out behind the reads of X, which return before it, and in front of the work on them
-  if constexpr (NORM) {
-    __shared__ float nscr[4][4];
-    dfuse_norm_ahead(a.X, a.ldx, M, K, a.na, xs, ldx, nscr, [&]() __attribute__((always_inline)) { load(f0); });
-  } else {
-    constexpr int XP = !F8 && U == 8 ? 16 : 8;  // 16-B pieces of X a thread holds: all, or the last ones
-    const int per = K / 8, total = M * per;
-    u16x8 v[XP];
-    auto fetch = [&](int p0) __attribute__((always_inline)) {
+  auto finish = [&](const f32x4& s, int mb, int cg) __attribute__((always_inline)) {
+    const int m = mb * 16 + c;
+    if constexpr (EPI == kStRope128) {
+      dfuse_rope_store<64>(s, g, m, M, cg, a.rp);
+    } else if constexpr (EPI == kStRope64) {
+      dfuse_rope_store<32>(s, g, m, M, cg, a.rp);
+    } else if constexpr (EPI == kStSwiglu) {
+      dfuse_swiglu_store(s, g, m, M, a.Y, a.ldy, cg);
+    } else if (m < M) {
+      u16x4 o;
 #pragma unroll
-      for (int i = 0; i < XP; ++i) {
-        const int p = min(p0 + tid + 512 * i, total - 1), m = p / per;
-        v[i] = *reinterpret_cast<const u16x8*>(a.X + (int64_t)m * a.ldx + (p - m * per) * 8);
-      }
-    };
-    auto put = [&](int p0) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < XP; ++i) {
-        const int p = p0 + tid + 512 * i, m = p / per;
-        if (p < total) *reinterpret_cast<u16x8*>(xs + m * ldx + (p - m * per) * 8) = v[i];
-      }
-    };
-    int p0 = 0;
-    for (; p0 + XP * 512 < total; p0 += XP * 512) {
-      fetch(p0);
-      put(p0);
+      for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+      *reinterpret_cast<u16x4*>(a.Y + (int64_t)m * a.ldy + (int64_t)cg * 16 + 4 * g) = o;
     }
-    fetch(p0);
-    load(f0);
-    put(p0);
-    lds_barrier();
-  }
-  const uint16_t* xr[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) xr[mb] = xs + min(mb * 16 + c, M - 1) * ldx + w * kq + 16 * g;
-
-  f32x4 acc[MB];
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int cg = blockIdx.x, cb = 0, turn = 0;
-  auto multiply = [&](const WFrag<F8, U>& f) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      u16x8 a0, a1;
-      f.get(u, a0, a1);
-      const int k = (cb * U + u) * 64;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        acc[mb] = mfma16_sk(a0, *reinterpret_cast<const u16x8*>(xr[mb] + k), acc[mb]);
-        acc[mb] = mfma16_sk(a1, *reinterpret_cast<const u16x8*>(xr[mb] + k + 8), acc[mb]);
-      }
-    }
-    if (++cb < nblk) return;
-    cb = 0;
-    const int par = NRED == 2 ? turn & 1 : 0;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      red[par][w][mb][lane] = acc[mb];
-      acc[mb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    lds_barrier();
-    if (w == (turn & (NW - 1))) {
-      f32x4 sc = {1.f, 1.f, 1.f, 1.f};
-      if constexpr (F8) sc = *reinterpret_cast<const f32x4*>(a.scale + row(cg, 4 * g));
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        f32x4 s = red[par][0][mb][lane];
-#pragma unroll
-        for (int ww = 1; ww < NW; ++ww) s += red[par][ww][mb][lane];
-        if constexpr (F8) s *= sc;
-        const int m = mb * 16 + c;
-        if constexpr (EPI == kStRope128) {
-          dfuse_rope_store<64>(s, g, m, M, cg, a.rp);
-        } else if constexpr (EPI == kStRope64) {
-          dfuse_rope_store<32>(s, g, m, M, cg, a.rp);
-        } else if constexpr (EPI == kStSwiglu) {
-          dfuse_swiglu_store(s, g, m, M, a.Y, a.ldy, cg);
-        } else if (m < M) {
-          u16x4 o;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
-          *reinterpret_cast<u16x4*>(a.Y + (int64_t)m * a.ldy + (int64_t)cg * 16 + 4 * g) = o;
-        }
-      }
-    }
-    if constexpr (NRED == 1) lds_barrier();  // one image: its sum is read before the next group's parts
-    ++turn;
-    cg += gridDim.x;
   };
-  const int steps = (a.groups - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * nblk;
-  if (steps == 1) {
-    multiply(f0);
-    return;
-  }
-  load(f1);
-  int s = 0;
-  for (; s + 3 < steps; s += 2) {
-    multiply(f0);
-    load(f0);
-    multiply(f1);
-    load(f1);
-  }
-  multiply(f0);
-  if (steps - s == 3) {
-    load(f0);
-    multiply(f1);
-    multiply(f0);
-  } else {
-    multiply(f1);
-  }
+  stream_walk<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, a.groups, smem, row, off, stage, finish);
 }
 
-constexpr int kRedBytes = 16 * 1024;  // the partial sums' images
-constexpr int kTwoLds = 80 * 1024;    // LDS up to which two workgroups share a CU
+constexpr int kTwoLds = 80 * 1024;  // LDS up to which two workgroups share a CU
 
-template <bool F8, int MB, int EPI, bool NORM, int U>
+template <int KIND, int TB, int KP, int EPI, bool NORM, int NL>
 static int stream_launch(const StreamArgs& a, int per_cu, size_t lds, hipStream_t stream) {
-  static const bool big = hipFuncSetAttribute((const void*)stream_gemm_kernel<F8, MB, EPI, NORM, U>,
+  static const bool big = hipFuncSetAttribute((const void*)stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL>,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) == hipSuccess;
   if (!big) return -1;
-  stream_gemm_kernel<F8, MB, EPI, NORM, U><<<std::min(a.groups, 256 * per_cu), 512, lds, stream>>>(a);
+  stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL><<<std::min(a.groups, 256 * per_cu), 512, lds, stream>>>(a);
   return (int)hipGetLastError();
 }
 
-// bf16 blocks of 8 chunks (152 registers) leave a CU to one workgroup: where its LDS does that anyway
-template <bool F8, int MB, int EPI, bool NORM>
-static int stream_u(const StreamArgs& a, hipStream_t stream) {
-  const size_t lds = kRedBytes + (size_t)a.M * (a.K + 8) * 2;
+// bf16 blocks of 16 loads (150 registers and more) leave a CU to one workgroup: where its LDS does that anyway
+template <int KIND, int TB, int EPI, bool NORM>
+static int stream_blocks(const StreamArgs& a, hipStream_t stream) {
+  const bool four = KIND == kStLines && sk_parts(a.M, a.K) == 4;
+  const size_t lds = (four ? kStreamRed<KIND, TB, 4> : kStreamRed<KIND, TB, 8>) + (size_t)a.M * (a.K + 8) * 2;
   const int per_cu = lds <= kTwoLds ? 2 : 1;
-  return a.K % 4096 == 0 && (F8 || per_cu == 1) ? stream_launch<F8, MB, EPI, NORM, 8>(a, per_cu, lds, stream)
-                                                : stream_launch<F8, MB, EPI, NORM, 4>(a, per_cu, lds, stream);
+  if constexpr (KIND == kStF8) {
+    return a.K % 4096 == 0 ? stream_launch<KIND, TB, 8, EPI, NORM, 8>(a, per_cu, lds, stream)
+                           : stream_launch<KIND, TB, 8, EPI, NORM, 4>(a, per_cu, lds, stream);
+  } else {
+    if constexpr (KIND == kStLines)
+      if (four) return stream_launch<KIND, TB, 4, EPI, NORM, 8>(a, per_cu, lds, stream);
+    return a.K % 4096 == 0 && per_cu == 1 ? stream_launch<KIND, TB, 8, EPI, NORM, 16>(a, per_cu, lds, stream)
+                                          : stream_launch<KIND, TB, 8, EPI, NORM, 8>(a, per_cu, lds, stream);
+  }
 }
 
 template <bool F8, int EPI>
 static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
-  if (norm) return stream_u<F8, 1, EPI, true>(a, stream);
-  return a.M <= 16 ? stream_u<F8, 1, EPI, false>(a, stream) : stream_u<F8, 2, EPI, false>(a, stream);
+  constexpr int LINES = F8 ? kStF8 : kStLines, WIDE = F8 ? kStF8 : kStWide;
+  if (norm) return stream_blocks<LINES, 1, EPI, true>(a, stream);
+  if constexpr (F8) {
+    if (a.M <= 16) return stream_blocks<kStF8, 1, EPI, false>(a, stream);
+  } else {
+    if (a.M <= 8) return stream_blocks<kStLines, 1, EPI, false>(a, stream);
+    if (a.M <= 16) return stream_blocks<kStLines, 2, EPI, false>(a, stream);
+  }
+  return stream_blocks<WIDE, 2, EPI, false>(a, stream);
 }
 
 }  // namespace mx
@@ -244,7 +138,7 @@ using namespace mx;
 
 // Whether mx_stream_gemm takes M rows of K: X and the partial sums in 160 KB of LDS, whole blocks a wave.
 extern "C" int mx_stream_ok(int M, int K, int norm) {
-  const int64_t lds = kRedBytes + (int64_t)M * (K + 8) * 2;
+  const int64_t lds = 16 * 1024 + (int64_t)M * (K + 8) * 2;
   return M >= 1 && M <= (norm ? 4 : 32) && K % 2048 == 0 && lds <= 158 * 1024;
 }
 
@@ -265,6 +159,7 @@ extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int
       ((uintptr_t)y | (uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) & 7)
     return -1;
   if (epi >= 2 ? N != (Hq + 2 * Hkv) * (epi == 2 ? 128 : 64) : (ldy % 4 || ldy < (epi == 1 ? N / 2 : N))) return -1;
+  if ((int64_t)(epi == 1 ? N / 2 + 16 : 256) * ldw * (scale ? 1 : 2) >> 32) return -1;  // offsets inside a group
   StreamArgs a{x, ldx, w, ldw, scale, y, ldy, M, K, N / 2, N / 16, SkNorm{delta, ldd, gamma, h_out, eps},
                SkRope{cosb, sinb, pos, slots, q, kc, vc, Hq, Hkv, max_seq, bt, maxb}};
   const bool norm = gamma != nullptr;

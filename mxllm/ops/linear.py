@@ -576,9 +576,9 @@ _DECODE_M = SKINNY_M if "MXLLM_SKINNY_M" in os.environ else 32  # rows of the ke
 # 72.2 -> 70.8 / 76.4; 65536 x 2560, 2 / 5 rows 61.8 / 59.6 -> 60.7 / 65.0).
 _SKINNY_SMALL_W = 128 << 20
 # Output channels up to which 8 a workgroup leave every one of the 256 CUs at most one (us, 16 a workgroup -> 8: 2048 x
-# 2048, 1 / 8 rows 4.6 / 5.3 -> 3.9 / 4.5; 2048 x 8192 13.4 / 15.1 -> 9.2 / 11.7).  More channels are a second turn for
-# some: 3072 x 2048, 1 / 8 rows 5.1 / 5.7 -> 5.3 / 6.6, 2304 x 8192, 8 rows 15.2 -> 19.3; one row of a longer K gains even
-# so, below the channels whose groups of 16 fill the CUs: 3584 x 3072 7.6 -> 7.0, 4080 x 4096 9.6 -> 8.6.
+# 2048, 1 / 8 rows 4.5 / 5.0 -> 3.7 / 4.4; 2048 x 8192 10.5 / 13.1 -> 8.0 / 9.9).  More channels are a second turn for
+# some: 3072 x 2048, 1 / 8 rows 4.8 / 5.3 -> 4.9 / 6.2; one row of a longer K gains even so, below the channels whose groups
+# of 16 fill the CUs: 3072 x 3072 6.4 -> 5.9.
 _HALF_N, _HALF_N1, _HALF_K1 = 2048, 4096, 3072
 
 
@@ -598,31 +598,37 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # Where a projection goes to the workgroups that stay (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of
-# once 16 channels), as far as X fits the LDS (32 rows of 2048, 17 of 4096, 11 of 6144, 8 of 8192, 5 of 14336).
-#  * Up to 8 rows (us, skinny -> stream): a K of 4096s, whose blocks are long, from 6144 channels on (6144 x 4096, 1 / 8
-#    rows 14.6 / 15.9 -> 13.6 / 13.7; 28672 x 4096, 1 row 43.6 -> 42.6; 4096 x 4096 level), an LM head from 2 rows on (128256 x
-#    4096, 1 row 173 -> 175, 4 rows 192 -> 178).  Else by rows x width, the X that the other reads beside 16 channels
-#    of weights: 8192 x 6144, 8 rows 24.4 -> 22.3; a K of 2048 at 8 rows with enough channels to spread the end (28672
-#    26.4 -> 24.8, 16384 15.7 -> 16.1, 8192 9.1 -> 10.4; with SwiGLU 16384 15.6 -> 15.2, 8192 9.5 -> 10.2).
-#  * Past 8 rows (hipBLASLt -> stream): a K of 2048 at any width (2048 x 2048, 12 / 32 rows 8.5 / 8.6 -> 5.3 / 7.1; 128256, 32
-#    rows 111 -> 104), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 17.1 / 16.8 -> 17.3 / 17.9;
+# once 16 channels), as far as X fits the LDS (32 rows of 2048, 17 of 4096, 11 of 6144, 8 of 8192, 5 of 14336).  (skinny_linear
+# itself goes there too where that has the same bits and takes less time: a K of 2048 from 3 rows on, one of 4096 from 9.)
+# Weights from memory in a chain of launches:
+#  * Up to 8 rows (us, skinny -> stream): a K of 4096s, whose blocks are long, from 6144 channels on (6144 x 4096, 1 / 8 rows
+#    12.1 / 14.0 -> 12.0 / 13.0; 28672 39.8 / 42.8 -> 39.4 / 41.1; 4096 x 4096, 8 rows 8.4 -> 9.5), an LM head from 2 rows on
+#    (128256 x 4096).  Else by rows x width, the X that the other reads beside 16 channels of weights: 8192 x 6144, 8 rows
+#    24.4 -> 22.3.
+#  * Past 8 rows (hipBLASLt -> stream): a K of 2048 at any width (2048 x 2048, 12 / 32 rows 11.0 / 11.3 -> 5.6 / 7.7; 16384, 16
+#    rows 17.9 -> 16.3), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 18.0 / 18.1 -> 17.9 / 18.6;
 #    14336 15.8 / 15.7 -> 16.7 / 17.7; 20480 22.0 / 22.1 -> 20.4 / 21.1), which gain with SwiGLU only (19.2 -> 18.0).  A K of 4096 up
-#    to 16 rows (2048 x 4096 and wider; 12288, 16 rows 26.7 -> 21.0), a 17th only where there is much to stream (16384 30.7 ->
-#    29.2, 12288 22.2 -> 24.1).  Longer ones from 12288 channels on (12288 x 6144, 9 rows 35.5 -> 32.2, 6144 18.4 -> 20.2).
+#    to 16 rows (6144, 16 rows 14.7 -> 14.6; 28672 61 -> 41), but for one group a CU (4096, 9 / 16 rows skinny 9.0 / 10.2
+#    against 10.1 / 10.5), a 17th only where there is much to stream (16384 30.7 -> 29.2, 12288 22.2 -> 24.1).  Longer ones
+#    from 12288 channels on (12288 x 6144, 9 rows 35.5 -> 32.2, 6144 18.4 -> 20.2).
 _STREAM_MK, _STREAM_N4, _STREAM_N2 = 16384, 6144, 32768
 
 
 # Past SKINNY_M rows the kernel of 16 channels a workgroup keeps projections of at most 4096 channels (one group a CU) that
 # the one above does not take: of up to 16 rows where the rows' fragments stay few, and from 768 channels on (us, hipBLASLt
-# -> here: 1024 x 2048, 9 / 32 rows 8.4 / 8.5 -> 5.3 / 7.9; 4096 x 1536, 32 rows 9.8 -> 7.7; 3072 x 3072, 16 rows 12.6 -> 8.4;
-# 64 x 2048, 16 rows 5.5 -> 5.4).  Beyond, each workgroup's walk over the rows is what lasts: 64 x 2048, 24 rows 5.5 -> 6.7;
-# 1024 x 4096, 32 rows 8.9 -> 13.3; 2560 x 2560, 24 rows 9.6 -> 10.5; 1024 x 6144, 9 rows 10.5 -> 11.7.
+# -> here: 1024 x 2048, 9 / 32 rows 10.9 / 11.0 -> 5.1 / 7.3; 4096 x 1536, 32 rows 9.8 -> 7.8; 3072 x 3072, 16 rows 12.4 -> 8.3;
+# 4096 x 4096, 16 rows 15.5 -> 10.2).  Beyond, each workgroup's walk over the rows is what lasts (1024 x 4096, 32 rows 8.9 ->
+# 13.3; 2560 x 2560, 24 rows 9.6 -> 10.5; 1024 x 6144, 9 rows 10.5 -> 11.7), unless the K is one that the library has no good
+# kernel for (4096 channels, 9 / 16 rows: K 16384 31.5 / 31.8 against 35.7 / 39.6 here; 18432 51 / 48 -> 36 / 42; 21504 54 / 54 ->
+# 38 / 43; 28672 65 / 69 -> 54 / 63).
 _WIDE_N = 4096
 
 
 def _wide_wins(M: int, N: int, K: int) -> bool:
     if N > _WIDE_N:
         return False
+    if M <= 16 and N > 3072 and (K == 4096 or K > 16384):
+        return True
     return (M <= 16 and M * K <= 32768) or (N >= 768 and (K <= 2048 or (K <= 4096 and M * K <= 49152)))
 
 
@@ -645,7 +651,7 @@ def _stream_wins(M: int, N: int, K: int, swiglu: bool = False) -> bool:
         if K > 4096:
             return N >= 12288
         if K == 4096:
-            return N >= (2048 if M <= 16 else 16384)
+            return N >= 2048 and not 3072 < N <= 4096 if M <= 16 else N >= 16384
         return N >= 2048 and (swiglu or M <= 16 or not 12288 < N < 20480)
     if K % 4096 == 0 and N >= _STREAM_N4:
         return M > 1 or N < _STREAM_N2

@@ -1039,3 +1039,19 @@ def test_prefill_attention_runs_the_kernels(gpu, D, Hq, Hkv, S):
     q, k, v = _ops().rope_split(qkv, cos, sin, 1, S, Hq, Hkv, D, None)
     assert torch.equal(kept[0], k[0]) and torch.equal(kept[1], v[0])
     assert torch.equal(o, _ops().attn_fwd(q, k, v, True, D ** -0.5)[0].view(S, Hq * D))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 48, 2048), (2, 8208, 2048), (3, 48, 2048), (8, 8208, 3072), (7, 16, 512), (9, 32, 1536),
+                                   (12, 1040, 3072), (16, 3088, 4096), (16, 48, 2048), (17, 48, 2560), (31, 16, 512)])
+def test_skinny_linear_fragments(gpu, M, N, K):
+    """The decode GEMM's ways to read (4 and 8 K parts, all loads of a block ahead or not, blocks of 8 and of 16 rows and tokens,
+    the kernel that stays) against fp64, plain and with SwiGLU; row-strided x, rows and groups at their edges."""
+    from mxllm import ops
+
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 64, device=gpu, dtype=torch.bfloat16)[:, :K]
+    w = torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05
+    y = _ops().skinny_linear(x, w)
+    assert rel_err(y, x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
+    assert torch.equal(_ops().skinny_linear_swiglu(x, w), ops.swiglu(y))
