@@ -123,6 +123,61 @@ __global__ void __launch_bounds__(64 * NW) w8a16_gemm_kernel(const uint16_t* __r
   }
 }
 
+// Up to 8 rows, by 8 weight rows x 128 codes (whole cache lines, nontemporal: skinny_core.h) in 4 K parts, waves 4 .. 7 the other
+// 8 channels.  A lane's 16 codes are k = 64 (c >> 3) + 16 g .. + 15 of a 128-k chunk, a product's useful parts those of the bf16
+// kernel.
+__global__ void __launch_bounds__(512) w8_lines_kernel(const uint16_t* __restrict__ X, int64_t ldx, const uint8_t* __restrict__ Q,
+                                                       const float* __restrict__ scale, uint16_t* __restrict__ Y, int64_t ldy,
+                                                       int M, int K) {
+  typedef SkSum<1, 1, 4> Sum;
+  __shared__ f32x4 red[Sum::PLACES];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16, kq = K / 4, nit = kq / 128;
+  const int64_t k0 = (int64_t)sk_part<4>(w) * kq + 2 * sk_lane_k(c, g);
+  const uint8_t* qrow = Q + (int64_t)(n0 + 8 * sk_half<4>(w, 0) + (c & 7)) * K + k0;
+  const uint16_t* xr = X + (int64_t)min(c & 7, M - 1) * ldx + k0;
+  f32x4 acc[1][1] = {{f32x4{0.f, 0.f, 0.f, 0.f}}};
+  // all loads of a block of U chunks ahead of its products; K's rest by smaller blocks
+  auto block = [&](auto n, int it) {
+    constexpr int U = n;
+    u32x4 q[U];
+    u16x8 b[U][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      q[u] = sk_weights<u32x4>(qrow + (it + u) * 128);
+      b[u][0] = *reinterpret_cast<const u16x8*>(xr + (it + u) * 128);
+      b[u][1] = *reinterpret_cast<const u16x8*>(xr + (it + u) * 128 + 8);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      acc[0][0] = mfma16_sk(dequant8(q[u][0], q[u][1]), b[u][0], acc[0][0]);
+      acc[0][0] = mfma16_sk(dequant8(q[u][2], q[u][3]), b[u][1], acc[0][0]);
+    }
+  };
+  using std::integral_constant;
+  int it = 0;
+  for (; it + 8 <= nit; it += 8) block(integral_constant<int, 8>{}, it);
+  if (it + 4 <= nit) { block(integral_constant<int, 4>{}, it); it += 4; }
+  if (it + 2 <= nit) { block(integral_constant<int, 2>{}, it); it += 2; }
+  if (it < nit) block(integral_constant<int, 1>{}, it);
+  const Sum sum{red};
+  sum.put(w, c, g, acc);
+  __syncthreads();
+  if (w == 0) {
+    const f32x4 s = sum.get(c, g, 0, 0);
+    if (c < M) {
+      const int n = n0 + 4 * g;
+      const f32x4 sc = *reinterpret_cast<const f32x4*>(scale + n);
+      u16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i] * sc[i]);
+      *reinterpret_cast<u16x4*>(Y + (int64_t)c * ldy + n) = o;
+    }
+  }
+}
+
 // Per-token activation quantisation for the fp8 x fp8 GEMM path: one workgroup per
 // row, amax -> scale = amax / 448, codes = e4m3(x / scale) by the hardware pack
 // conversion (OCP e4m3 on gfx950, round to nearest even).  16-B loads; the second
@@ -161,6 +216,13 @@ __global__ void __launch_bounds__(256) quant_rows_e4m3_kernel(const uint16_t* __
 
 using namespace mx;
 
+extern "C" int mx_stream_ok(int M, int K, int norm);
+extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
+                              int64_t ldy, int M, int N, int K, int epi, const uint16_t* delta, int64_t ldd,
+                              const uint16_t* gamma, float eps, uint16_t* h_out, const float* cosb, const float* sinb,
+                              const int32_t* pos, const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq,
+                              int Hkv, int max_seq, const int32_t* bt, int maxb, hipStream_t stream);
+
 // X [M, K] bf16 (row stride ldx), Q [N, K] e4m3 codes, scale [N] f32 (per output channel),
 // Y [M, N] bf16 (row stride ldy).  Requires M in 1..32, N % 16 == 0, K % 512 == 0,
 // ldx a multiple of 8, ldy of 4.
@@ -179,10 +241,25 @@ extern "C" int mx_w8a16_gemm(const uint16_t* x, int64_t ldx, const uint8_t* q, c
   // wherever the grid keeps >= 128 workgroups
   const char* e = getenv("MXLLM_W8_NC");
   const int force = e && *e ? atoi(e) : 0;
+  const bool two = N % 32 == 0 && ((force == 2 && N / 32 >= 128) || (!force && N / 32 >= 256 && (M >= 6 || (M >= 4 && K >= 16384))));
+  // Up to 8 rows whole cache lines, which from 3 rows on pay where X is in LDS (us, 16-row fragments -> lines -> stream_gemm.hip, whose
+  // bits are those of the lines: 4096 x 4096, 1 / 4 / 8 rows 6.1 / 6.5 / 7.1 -> 5.3 / 6.4 / 7.7 -> 5.9 / 5.9 / 6.5; 28672 x 4096 27.1 /
+  // 31.5 / 34.1 -> 25.3 / 34.3 / 33.0 -> 22.2 / 22.4 / 22.8).  Else the 16-row fragments, which read X half as often (4096 x 14336,
+  // 8 rows 18.3 -> 21.5).
+  if (!force && M <= 8) {
+    const bool fits = mx_stream_ok(M, K, 0) != 0;
+    if (fits && M > 2 &&
+        mx_stream_gemm(x, ldx, q, K, scale, y, ldy, M, N, K, 0, nullptr, 0, nullptr, 0.f, nullptr, nullptr, nullptr, nullptr,
+                       nullptr, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0, stream) == 0)
+      return 0;
+    if (fits || M <= 2) {
+      w8_lines_kernel<<<N / 16, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, K);
+      return (int)hipGetLastError();
+    }
+  }
   if (force == 4 && M <= 16 && N % 64 == 0 && N / 64 >= 128)
     w8a16_gemm_kernel<1, 8, 4><<<N / 64, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, N, K);
-  else if (M <= 16 && N % 32 == 0 &&
-           ((force == 2 && N / 32 >= 128) || (!force && N / 32 >= 256 && (M >= 6 || (M >= 4 && K >= 16384)))))
+  else if (M <= 16 && two)
     w8a16_gemm_kernel<1, 8, 2><<<N / 32, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, N, K);
   else if (M <= 16) w8a16_gemm_kernel<1, 8, 1><<<N / 16, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, N, K);
   else w8a16_gemm_kernel<2, 8, 1><<<N / 16, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, N, K);

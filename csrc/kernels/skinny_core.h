@@ -23,8 +23,9 @@ __device__ __forceinline__ f32x4 mfma16_sk(const u16x8& a, const u16x8& b, const
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_sk, a), __builtin_bit_cast(bf16x8_sk, b),
                                                  c, 0, 0, 0);
 }
-__device__ __forceinline__ u16x8 sk_weights(const void* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u16x8*>(p));
+template <typename V = u16x8>
+__device__ __forceinline__ V sk_weights(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
 }
 
 constexpr int kSkWaves = 8;

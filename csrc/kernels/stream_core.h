@@ -14,8 +14,9 @@
 namespace mx {
 
 // How a kernel reads its weights: bf16 in blocks of 8 rows x 128 B and of 8 tokens (up to 16 rows of X), or of 16 rows x 64 B
-// and 16 tokens; e4m3: 16 rows x 64 codes, which a lane widens to the two MFMA operands of a chunk, and 16 tokens.
-enum { kStLines, kStWide, kStF8 };
+// and 16 tokens; e4m3 codes, which a lane widens to the two MFMA operands of a chunk, the same two ways: 8 rows x 128 codes and 8
+// tokens (4 K parts), or 16 rows x 64 and 16.
+enum { kStLines, kStWide, kStF8, kStF8Lines };
 
 // NL loads of weights in flight, chunk by chunk and block by block
 template <int KIND, int NL, int RB>
@@ -28,18 +29,24 @@ struct WFrag {
       for (int rb = 0; rb < RB; ++rb) a[u][rb] = KIND == kStWide ? *reinterpret_cast<const u16x8*>(p + o[rb] + u * 128) : sk_weights(p + o[rb] + u * 128);
   }
 };
-template <int NL>
-struct WFrag<kStF8, NL, 1> {
+template <bool LINES, int NL>
+struct WCodes {
   u32x4 a[NL];
   __device__ __forceinline__ void load(const char* p, const uint32_t (&o)[1]) {
 #pragma unroll
-    for (int u = 0; u < NL; ++u) a[u] = *reinterpret_cast<const u32x4*>(p + o[0] + u * 64);
+    for (int u = 0; u < NL; ++u)
+      a[u] = LINES ? sk_weights<u32x4>(p + o[0] + u * 128) : *reinterpret_cast<const u32x4*>(p + o[0] + u * 64);
   }
   __device__ __forceinline__ void get(int u, u16x8& x, u16x8& y) const {
     x = dequant8(a[u][0], a[u][1]);
     y = dequant8(a[u][2], a[u][3]);
   }
 };
+
+template <int NL>
+struct WFrag<kStF8, NL, 1> : WCodes<false, NL> {};
+template <int NL>
+struct WFrag<kStF8Lines, NL, 1> : WCodes<true, NL> {};
 
 // rows of X [M, K] as they are: XP 16-B pieces a thread holds at once, all or the last ones
 template <int XP, typename Ahead>
@@ -75,30 +82,31 @@ __device__ __forceinline__ void stream_rows_in(const uint16_t* __restrict__ X, i
 // the partial sums' images: two of up to 8 KB (the waves take turns at a group's sum and what follows, the others go
 // on), or one of 16
 template <int KIND, int TB, int KP>
-constexpr int kStreamPlaces = KIND == kStLines ? SkSum<TB, 1, KP>::PLACES : kSkWaves * TB * 64;
+constexpr int kStreamPlaces = KIND == kStLines || KIND == kStF8Lines ? SkSum<TB, 1, KP>::PLACES : kSkWaves * TB * 64;
 template <int KIND, int TB, int KP>
 constexpr int kStreamImages = kStreamPlaces<KIND, TB, KP> * 16 <= 8192 ? 2 : 1;
 template <int KIND, int TB, int KP>
 constexpr int kStreamRed = kStreamPlaces<KIND, TB, KP> * kStreamImages<KIND, TB, KP> * 16;  // bytes, 16 KB at most
 
-// TB blocks of 8 (kStLines) or 16 tokens, KP K parts (8 but for kStLines)
+// TB blocks of 8 (lines) or 16 tokens, KP K parts (kStF8Lines: 4, without lines: 8)
 template <int KIND, int TB, int KP, int NL, typename Row, typename Off, typename Stage, typename Finish>
 __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const float* scale, int M, int K, int groups,
                                             char* smem, const Row& row, const Off& off, const Stage& stage,
                                             const Finish& finish) {
-  constexpr bool F8 = KIND == kStF8, LINES = KIND == kStLines;
+  constexpr bool F8 = KIND == kStF8 || KIND == kStF8Lines, LINES = KIND == kStLines || KIND == kStF8Lines;
+  static_assert(KIND != kStF8Lines || KP == 4, "one block of codes a wave");
   constexpr int NW = kSkWaves, WB = F8 ? 1 : 2, RB = F8 ? 1 : kSkBlocks<KP, 1>, MB = LINES ? (TB + 1) / 2 : TB;
   constexpr int AB = LINES ? RB : 1;  // blocks with sums of their own (kStWide: the halves of a chunk share them)
-  constexpr int CH = NL / RB;         // 64-k chunks of a block
+  constexpr int CK = KIND == kStF8Lines ? 128 : 64, CH = NL / RB;  // k of a chunk, chunks of a block
   typedef SkSum<TB, 1, KP> Sum;  // kStLines
   constexpr int PLACES = kStreamPlaces<KIND, TB, KP>, NRED = kStreamImages<KIND, TB, KP>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
-  const int kq = K / KP, nblk = kq / (64 * CH), ldx = K + 8;
+  const int kq = K / KP, nblk = kq / (CK * CH), ldx = K + 8;
   f32x4* red = reinterpret_cast<f32x4*>(smem);
   uint16_t* xs = reinterpret_cast<uint16_t*>(smem + kStreamRed<KIND, TB, KP>);
-  const int k0 = sk_part<KP>(w) * kq + (LINES ? sk_lane_k(c, g) : F8 ? 16 * g : 8 * g);
+  const int k0 = sk_part<KP>(w) * kq + (F8 && LINES ? 2 * sk_lane_k(c, g) : LINES ? sk_lane_k(c, g) : F8 ? 16 * g : 8 * g);
   // the block to load next: group lg, block lb
   int lg = blockIdx.x, lb = 0;
   uint32_t lo[RB];
@@ -109,7 +117,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
   const char* lp = reinterpret_cast<const char*>(W) + row(lg) * ldw * WB;
   auto load = [&](WFrag<KIND, NL, RB>& f) __attribute__((always_inline)) {
     f.load(lp, lo);
-    lp += CH * 64 * WB;
+    lp += CH * CK * WB;
     if (++lb == nblk) {
       lb = 0;
       lg += gridDim.x;
@@ -134,7 +142,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
   auto multiply = [&](const WFrag<KIND, NL, RB>& f) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const int k = (cb * CH + u) * 64;
+      const int k = (cb * CH + u) * CK;
       if constexpr (F8) {
         u16x8 a0, a1;
         f.get(u, a0, a1);
@@ -182,8 +190,8 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
           s = img[mb * 64 + lane];
 #pragma unroll
           for (int ww = 1; ww < NW; ++ww) s += img[(ww * MB + mb) * 64 + lane];
-          if constexpr (F8) s *= sc;
         }
+        if constexpr (F8) s *= sc;
         finish(s, mb, cg);
       }
     }

@@ -19,7 +19,8 @@
 //    prologue: the RMSNorm with the residual add, up to 4 rows (decode_fuse.h).
 // 28672 x 4096 (235 MB), rows 1 / 4 / 8 / 16: 39.4 / 39.6 / 39.4 / 41.4 us (6.0 TB/s; in fragments of 16 rows x 64 B 43.0 / 43.5 /
 // 43.7 / 44.4) against skinny_gemm's 39.8 / 41.0 / 42.8 / 54.6 and hipBLASLt's 61 to 64; 16384 x 2048 (67 MB), 4 / 8 / 16 rows 12.9 /
-// 13.4 / 15.4 (15.8 / 16.4 / 16.5); in e4m3, rows 1 / 4 / 8: 24.9 / 25.8 / 28.6 against fp8_gemm's 28.4 / 32.2 / 36.4.
+// 13.4 / 15.4 (15.8 / 16.4 / 16.5); in e4m3, 28672 x 4096, rows 1 / 4 / 8: 22.2 / 22.4 / 22.8 (24.6 / 25.4 / 25.7 in
+// 16 rows x 64 B) against fp8_gemm's 27.1 / 31.5 / 34.1; 4096 x 14336, 1 / 4 rows 12.9 / 14.3 (14.3 / 16.1).
 // Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 13.0 us for 50 MB; the last 128 as
 // 256 halves: no change, a half's loads take a whole one's turns), and the launch's own 2 us before the first bytes arrive.
 #include <algorithm>
@@ -46,7 +47,7 @@ struct StreamArgs {
 
 // workgroups of up to 128 registers: two a CU where LDS allows it (X of 9 rows and more of a K over 2048 does not)
 template <int KIND, int TB, int KP, int NL>
-constexpr int kStWaves = KIND == kStF8 ? (TB == 1 ? 4 : 2) : NL == 8 && (TB == 1 || KP == 4) ? 4 : 2;
+constexpr int kStWaves = KIND >= kStF8 ? (TB == 1 ? 4 : 2) : NL == 8 && (TB == 1 || KP == 4) ? 4 : 2;
 
 template <int KIND, int TB, int KP, int EPI, bool NORM, int NL>
 __global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm_kernel(StreamArgs a) {
@@ -70,7 +71,7 @@ __global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm
       __shared__ float nscr[4][4];
       dfuse_norm_ahead(a.X, a.ldx, M, K, a.na, xs, ldx, nscr, ahead);
     } else {
-      stream_rows_in<KIND != kStF8 && NL == 16 ? 16 : 8>(a.X, a.ldx, M, K, xs, ldx, ahead);
+      stream_rows_in<KIND < kStF8 && NL == 16 ? 16 : 8>(a.X, a.ldx, M, K, xs, ldx, ahead);
     }
   };
   auto finish = [&](const f32x4& s, int mb, int cg) __attribute__((always_inline)) {
@@ -106,11 +107,12 @@ static int stream_launch(const StreamArgs& a, int per_cu, size_t lds, hipStream_
 template <int KIND, int TB, int EPI, bool NORM>
 static int stream_blocks(const StreamArgs& a, hipStream_t stream) {
   const bool four = KIND == kStLines && sk_parts(a.M, a.K) == 4;
-  const size_t lds = (four ? kStreamRed<KIND, TB, 4> : kStreamRed<KIND, TB, 8>) + (size_t)a.M * (a.K + 8) * 2;
+  constexpr int KP8 = KIND == kStF8Lines ? 4 : 8;
+  const size_t lds = (four ? kStreamRed<KIND, TB, 4> : kStreamRed<KIND, TB, KP8>) + (size_t)a.M * (a.K + 8) * 2;
   const int per_cu = lds <= kTwoLds ? 2 : 1;
-  if constexpr (KIND == kStF8) {
-    return a.K % 4096 == 0 ? stream_launch<KIND, TB, 8, EPI, NORM, 8>(a, per_cu, lds, stream)
-                           : stream_launch<KIND, TB, 8, EPI, NORM, 4>(a, per_cu, lds, stream);
+  if constexpr (KIND >= kStF8) {
+    return a.K % 4096 == 0 ? stream_launch<KIND, TB, KP8, EPI, NORM, 8>(a, per_cu, lds, stream)
+                           : stream_launch<KIND, TB, KP8, EPI, NORM, 4>(a, per_cu, lds, stream);
   } else {
     if constexpr (KIND == kStLines)
       if (four) return stream_launch<KIND, TB, 4, EPI, NORM, 8>(a, per_cu, lds, stream);
@@ -121,14 +123,10 @@ static int stream_blocks(const StreamArgs& a, hipStream_t stream) {
 
 template <bool F8, int EPI>
 static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
-  constexpr int LINES = F8 ? kStF8 : kStLines, WIDE = F8 ? kStF8 : kStWide;
+  constexpr int LINES = F8 ? kStF8Lines : kStLines, WIDE = F8 ? kStF8 : kStWide;
   if (norm) return stream_blocks<LINES, 1, EPI, true>(a, stream);
-  if constexpr (F8) {
-    if (a.M <= 16) return stream_blocks<kStF8, 1, EPI, false>(a, stream);
-  } else {
-    if (a.M <= 8) return stream_blocks<kStLines, 1, EPI, false>(a, stream);
-    if (a.M <= 16) return stream_blocks<kStLines, 2, EPI, false>(a, stream);
-  }
+  if (a.M <= 8) return stream_blocks<LINES, 1, EPI, false>(a, stream);
+  if (a.M <= 16) return F8 ? stream_blocks<kStF8, 1, EPI, false>(a, stream) : stream_blocks<LINES, F8 ? 1 : 2, EPI, false>(a, stream);
   return stream_blocks<WIDE, 2, EPI, false>(a, stream);
 }
 

@@ -660,8 +660,8 @@ def _stream_wins(M: int, N: int, K: int, swiglu: bool = False) -> bool:
 
 def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
     """Inference: ``x2 W^T`` for a few rows and e4m3 weights.  A long K on stream_gemm.hip where X fits its LDS (us,
-    fp8_gemm.hip -> there: 4096 x 14336, 1 / 4 rows 16.8 / 18.2 -> 15.2 / 16.9; 2048 x 8192, 8 rows 10.9 -> 10.1; but
-    4096 x 4096, 4 rows 6.5 -> 7.2)."""
+    fp8_gemm.hip -> there: 4096 x 14336, 1 / 4 rows 14.5 / 15.9 -> 12.9 / 14.3; 2048 x 8192, 1 row 7.8 -> 7.2; but 4096 x
+    4096, 1 row 5.3 -> 5.9; from 3 rows on w8_linear goes there by itself)."""
     M, K = x2.shape
     if K >= 8192 and _stream_fits(M, K) and _rows_ok(x2, q, scale):
         return native().stream_linear(x2, None, None, 0.0, q, scale, False)[0]

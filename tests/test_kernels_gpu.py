@@ -1055,3 +1055,16 @@ def test_skinny_linear_fragments(gpu, M, N, K):
     y = _ops().skinny_linear(x, w)
     assert rel_err(y, x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
     assert torch.equal(_ops().skinny_linear_swiglu(x, w), ops.swiglu(y))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 16, 512), (2, 48, 4608), (2, 4112, 4096), (3, 48, 2048), (8, 4112, 4096), (8, 48, 14336),
+                                   (5, 16, 1024), (9, 48, 4096)])
+def test_w8_linear_fragments(gpu, M, N, K):
+    """The e4m3 decode GEMM's ways to read (blocks of 8 and of 16 rows, K's rest by smaller blocks, the kernel that stays)
+    against fp64 on the same codes: one bf16 rounding."""
+    torch.manual_seed(M + N + K)
+    x = torch.randn(M, K + 64, device=gpu, dtype=torch.bfloat16)[:, :K]
+    q, s = _stream_weight(torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05, True)
+    ref = x.double() @ (q.view(torch.float8_e4m3fn).double() * s.double()[:, None]).t()
+    assert rel_err(_ops().w8_linear(x, q, s), ref) < 2 ** -8
