@@ -413,6 +413,249 @@ __global__ void __launch_bounds__(D) decode_combine_kernel(const float* __restri
   out[bh * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
 }
 
+// ---------------------------------------------------------------------------
+// Decode attention, heads of 128, of more 256-key splits than the CUs have places for (kEvenPlaces): the
+// keys of all sequences, in units of 16, are dealt evenly to one turn of workgroups.
+//
+// decode_attn_mfma_kernel gives every 256 keys of a sequence a workgroup.  16 sequences of 100 to 2,000 keys
+// are 540 of them on 512 places, and the 28 of the second turn cost nearly what the 512 of the first do.
+// Here a workgroup walks its equal share of the row of sequences of one KV head, segment by segment; a
+// segment's keys are shared by its four waves.  K and V both come straight into registers (a lane takes 8
+// neighbouring channels of 8 keys, and puts halves of its words together to the operand that the product
+// reads), so no LDS holds a tile and three workgroups fit a CU, whose loads hide each other's products.  Loads of
+// the next 32 keys issued ahead of the products of the last lose (29 us: 220 registers, two workgroups a CU), and
+// so do more than two shares a CU (more segments, and parts to merge).
+//
+// Time alone, 32 heads of 8 (merge apart, 4.7 us as before), us: 16 sequences of 100 to 2,000 keys 26.4 -> 23.9,
+// 48 of 60 to 600 21.4 -> 18.8, 32 of 100 to 1,000 25.5 -> 20.6, 7 of 2,500 21.7 -> 18.8.  Heads of 64, at
+// half the bytes a key, do not gain (14.1 -> 14.1, 11.4 -> 13.6) and keep their splits.
+//
+// Scores, weights and sums are those of decode_split_body; a wave keeps a running maximum.
+constexpr int kEvenD = 128, kEvenPlaces = 512;  // two workgroups a CU
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+
+struct EvenState {  // of one wave
+  float m, l;  // of head c; l: this lane's keys
+  f32x4 o[8];  // [e][i]: channel 8 (4 g + i) + e of head c
+
+  __device__ __forceinline__ void clear() {
+    m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // keys key0 .. key0 + 31 below hi (key0 a multiple of 16); k0, v0 / k1, v1: rows of the first / second 16 keys,
+  // l0, l1: the last row of them that is read
+  __device__ __forceinline__ void take(const uint16_t* __restrict__ k0, const uint16_t* __restrict__ k1,
+                                       const uint16_t* __restrict__ v0, const uint16_t* __restrict__ v1, int l0, int l1,
+                                       const u16x8 (&qf)[4], int key0, int hi, float sl, int c, int g) {
+    u32x4_t k[2][4], v[8];  // v: slot s is key 16 (s >> 2) + 4 g + (s & 3), channels 8 c ..
+    const uint32_t r0 = min(c, l0) * kEvenD + 8 * g, r1 = min(c, l1) * kEvenD + 8 * g;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) k[0][s] = *reinterpret_cast<const u32x4_t*>(k0 + (r0 + 32 * s));
+#pragma unroll
+    for (int s = 0; s < 4; ++s) k[1][s] = *reinterpret_cast<const u32x4_t*>(k1 + (r1 + 32 * s));
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      v[s] = *reinterpret_cast<const u32x4_t*>(v0 + (uint32_t)(min(4 * g + s, l0) * kEvenD + 8 * c));
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      v[4 + s] = *reinterpret_cast<const u32x4_t*>(v1 + (uint32_t)(min(4 * g + s, l1) * kEvenD + 8 * c));
+    __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
+    f32x4 sc[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      sc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) sc[j] = mfma16(__builtin_bit_cast(u16x8, k[j][s]), qf[s], sc[j]);
+    }
+    float mx = m;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = key0 + 16 * j + 4 * g + i < hi ? sc[j][i] * sl : -INFINITY;
+        sc[j][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mref = mx == -INFINITY ? 0.f : mx, f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mref);
+    m = mx;
+    l *= f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] *= f;
+    u16x8 pb;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p = __builtin_amdgcn_exp2f(sc[j][i] - mref);
+        l += p;
+        pb[4 * j + i] = f2bf(p);
+      }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      u32x4_t a;  // channel e of the 8 keys: one half of a word of each
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a[i] = __builtin_amdgcn_perm(v[2 * i + 1][e >> 1], v[2 * i][e >> 1], e & 1 ? 0x07060302u : 0x05040100u);
+      o[e] = mfma16(__builtin_bit_cast(u16x8, a), pb, o[e]);
+    }
+  }
+};
+
+// units of 16 keys that row b has; cap: positions that the buffers are sized for
+__device__ __forceinline__ int even_units(const int32_t* lens, int len_off, int cap, int b) {
+  return (min(max(lens[b] + len_off, 0), cap) + 15) >> 4;
+}
+// units of a workgroup: an equal share of all, at least 128 keys
+__device__ __forceinline__ int even_share(int total, int W) { return max((total + W - 1) / W, 8); }
+
+__global__ void __launch_bounds__(256, 3)
+    decode_even_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+                       const int32_t* __restrict__ lens, int len_off, const int32_t* __restrict__ slots,
+                       float* __restrict__ part_ml, float* __restrict__ part_o, uint16_t* __restrict__ out, int B, int Hq,
+                       int Hkv, int max_seq, int cap, int nparts, float sl, const int32_t* __restrict__ bt, int maxb) {
+  constexpr int D = kEvenD;
+  __shared__ float so[4][D][17];
+  __shared__ float mls[4][2][16];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4, hk = blockIdx.y, rep = Hq / Hkv, x = blockIdx.x;
+  int total = 0;
+  for (int i = lane; i < B; i += 64) total += even_units(lens, len_off, cap, i);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+  total = __builtin_amdgcn_readfirstlane(total);
+  const int share = even_share(total, gridDim.x);
+  int at = x * share;
+  const int end = min(total, at + share);
+  if (at >= end) return;
+  int b = 0, start = 0;  // the row that holds unit `at`: start <= at < start + n
+  for (int i0 = 0;; i0 += 64) {
+    const int n = i0 + lane < B ? even_units(lens, len_off, cap, i0 + lane) : 0;
+    int upto = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      if (lane >= o) upto += v;
+    }
+    const uint64_t past = __ballot(start + upto > at);
+    if (past) {
+      const int first = __ffsll((unsigned long long)past) - 1;
+      b = __builtin_amdgcn_readfirstlane(i0 + first);
+      start = __builtin_amdgcn_readlane(start + upto - n, first);
+      break;
+    }
+    start = __builtin_amdgcn_readlane(start + upto, 63);
+  }
+  while (true) {
+    const int len = min(max(lens[b] + len_off, 0), cap), n = (len + 15) >> 4;
+    if (n == 0) {  // (units are left, so a later row has them)
+      ++b;
+      continue;
+    }
+    const int u0 = at - start, u1 = min(end - start, n), per = (u1 - u0 + 3) >> 2;
+    const int k_lo = 16 * (u0 + per * w), hi = min(len, 16 * min(u1, u0 + per * (w + 1)));
+    const int slot = slots ? slots[b] : b;
+    u16x8 qf[4];
+    const uint16_t* qrow = q + ((int64_t)b * Hq + hk * rep + min(c, rep - 1)) * D;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      qf[s] = *reinterpret_cast<const u16x8*>(qrow + 32 * s + 8 * g);
+      if (c >= rep) qf[s] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    EvenState st;
+    st.clear();
+    const int past = (hi - 1) & ~15;  // the last 16 keys that have one
+    for (int k = k_lo; k < hi; k += 32) {
+      const int a1 = min(k + 16, past);  // 16 keys lie in one block: blocks are multiples of 256
+      const int64_t b0 = kv_row(bt, maxb, max_seq, slot, Hkv, hk, k) * D, b1 = kv_row(bt, maxb, max_seq, slot, Hkv, hk, a1) * D;
+      st.take(kc + b0, kc + b1, vc + b0, vc + b1, hi - 1 - k, hi - 1 - a1, qf, k, hi, sl, c, g);
+    }
+    st.l += __shfl_xor(st.l, 16, 64);
+    st.l += __shfl_xor(st.l, 32, 64);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) so[w][8 * (4 * g + i) + e][c] = st.o[e][i];
+    if (g == 0) mls[w][0][c] = st.m, mls[w][1][c] = st.l;
+    __syncthreads();
+    const int part = x - start / share, last = (start + n - 1) / share - start / share;
+    for (int idx = tid; idx < rep * D; idx += 256) {
+      const int h = idx / D, d = idx % D;
+      float M = -INFINITY, L = 0.f, acc = 0.f;
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) M = fmaxf(M, mls[ww][0][h]);
+#pragma unroll
+      for (int ww = 0; ww < 4; ++ww) {
+        const float mw = mls[ww][0][h], f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+        L += f * mls[ww][1][h];
+        acc += f * so[ww][d][h];
+      }
+      const int64_t bh = (int64_t)b * Hq + hk * rep + h;
+      if (last == 0) {  // the row's only part is its output
+        out[bh * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
+      } else {
+        part_o[(bh * nparts + part) * D + d] = acc;
+        if (d == 0) part_ml[(bh * nparts + part) * 2] = M, part_ml[(bh * nparts + part) * 2 + 1] = L;
+      }
+    }
+    at = start += n;
+    if (at >= end) return;
+    ++b;
+    __syncthreads();  // the sums are read
+  }
+}
+
+// merge of decode_even_kernel's parts, of the rows that have several; W: its workgroups of a KV head
+__global__ void __launch_bounds__(kEvenD)
+    decode_even_merge_kernel(const float* __restrict__ part_ml, const float* __restrict__ part_o,
+                             const int32_t* __restrict__ lens, int len_off, uint16_t* __restrict__ out, int B, int Hq,
+                             int W, int cap, int nparts) {
+  const int64_t bh = blockIdx.x;
+  const int b = (int)(bh / Hq), d = threadIdx.x, lane = d & 63;
+  const float* ml = part_ml + bh * nparts * 2;
+  const float* po = part_o + bh * nparts * kEvenD + d;
+  // the first parts' loads go out with those of the lengths; what is no part is not looked at
+  float mv[8], lv[8], ov[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const int p = min(s, nparts - 1);
+    mv[s] = ml[2 * p], lv[s] = ml[2 * p + 1], ov[s] = po[(int64_t)p * kEvenD];
+  }
+  int total = 0, start = 0;
+  const int n = even_units(lens, len_off, cap, b);
+  for (int i = lane; i < B; i += 64) {
+    const int u = even_units(lens, len_off, cap, i);
+    total += u;
+    if (i < b) start += u;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64), start += __shfl_xor(start, o, 64);
+  const int share = even_share(total, W);
+  const int parts = n ? (start + n - 1) / share - start / share + 1 : 0;
+  if (parts == 1) return;  // written by its workgroup
+  float M = -INFINITY, L = 0.f, acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) M = s < parts ? fmaxf(M, mv[s]) : M;
+  for (int s = 8; s < parts; ++s) M = fmaxf(M, ml[2 * s]);
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    if (s >= parts || mv[s] == -INFINITY) continue;
+    const float wgt = __builtin_amdgcn_exp2f(mv[s] - M);
+    L += wgt * lv[s];
+    acc += wgt * ov[s];
+  }
+#pragma unroll 4
+  for (int s = 8; s < parts; ++s) {
+    const float m = ml[2 * s], ls = ml[2 * s + 1], os = po[(int64_t)s * kEvenD];
+    const float wgt = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);
+    L += wgt * ls;
+    acc += wgt * os;
+  }
+  out[bh * kEvenD + d] = f2bf(L > 0.f ? acc / L : 0.f);
+}
+
 __device__ __forceinline__ uint32_t hash3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t h = a * 0x9E3779B1u ^ (b + 0x7F4A7C15u) * 0x85EBCA77u ^ (c + 0x165667B1u) * 0xC2B2AE3Du;
   h ^= h >> 15; h *= 0x2C1B3C6Du; h ^= h >> 12; h *= 0x297A2D39u; h ^= h >> 15;
@@ -541,6 +784,16 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
   const char* pe = getenv("MXLLM_DECODE_HANDOFF");
   const int proto = pe && *pe ? atoi(pe) : 4;
   const bool fused = out && cnt && D == 128 && proto >= 1 && proto <= 4;
+  // Heads of 128, more splits than places: dealt evenly.  What the caller's `nsplit` counts is the longest that the step
+  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.  The buffers have
+  // 2 nsplit + 1 parts a row (a row of n units touches at most (n + share - 2) / share + 1 shares of 8 units or more).
+  if (out && D == kEvenD && (int64_t)nsplit * Hkv * B > kEvenPlaces) {
+    const int W = std::max(1, kEvenPlaces / Hkv), cap = nsplit * kSplit, nparts = 2 * nsplit + 1;
+    decode_even_kernel<<<dim3(W, Hkv), 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, out, B, Hq, Hkv,
+                                                         max_seq, cap, nparts, sl, bt, maxb);
+    decode_even_merge_kernel<<<B * Hq, kEvenD, 0, stream>>>(part_ml, part_o, lens, len_off, out, B, Hq, W, cap, nparts);
+    return (int)hipGetLastError();
+  }
 #define DA(DD)                                                                                                      \
   decode_attn_mfma_kernel<DD><<<grid, 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, Hq, Hkv, \
                                                         max_seq, nsplit, sl, bt, maxb, fused || nsplit == 1 ? out : nullptr, \

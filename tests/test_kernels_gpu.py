@@ -993,6 +993,51 @@ def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,lens,room", [(32, 8, [1, 15, 16, 17, 255, 256, 257, 0] + [1, 33, 700, 90] * 6, 700),
+                                              (16, 1, [3000, 0, 1, 2600], 65536), (8, 8, [4000, 4096], 8448),
+                                              (6, 2, [5] * 300, 256), (64, 8, [2000, 64, 65, 1999, 1, 1900], 3000)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_decode_attn_dealt_evenly(gpu, Hq, Hkv, lens, room, paged):
+    """More splits than the chip has places for: workgroups that take several sequences, sequences of many parts, of none
+    (zeros) and of one, shares that end inside a block, more rows than a wave has lanes; stale rows are NaN.  Softmax
+    weights are rounded to bf16 (2^-9 each) and so is the output: within 2^-7 of f64."""
+    D, B, blk = 128, len(lens), 256
+    torch.manual_seed(B + Hq)
+    assert -(-room // blk) * Hkv * B > 512
+    n_max = max(lens)
+    nb = -(-n_max // blk)
+    if paged:
+        bt = torch.randperm(B * nb, device=gpu).to(torch.int32).view(B, nb)
+        bt = torch.nn.functional.pad(bt, (0, -(-room // blk) - nb))  # blocks past a sequence's end are not read
+        kc = torch.full((B * nb, Hkv, blk, D), float("nan"), device=gpu, dtype=torch.bfloat16)
+    else:
+        bt = None
+        kc = torch.full((B, Hkv, room, D), float("nan"), device=gpu, dtype=torch.bfloat16)
+    vc = kc.clone()
+    q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+    want = torch.zeros(B, Hq, D, dtype=torch.float64, device=gpu)
+    for b, n in enumerate(lens):
+        k, v = (torch.randn(Hkv, n, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        if paged:
+            for j in range(0, n, blk):
+                kc[int(bt[b, j // blk]), :, :min(blk, n - j)] = k[:, j:j + blk]
+                vc[int(bt[b, j // blk]), :, :min(blk, n - j)] = v[:, j:j + blk]
+        else:
+            kc[b, :, :n], vc[b, :, :n] = k, v
+        if n:
+            qd = q[b].double().view(Hkv, Hq // Hkv, D)
+            s = (qd[:, :, None] * k.double()[:, None]).sum(-1) * D ** -0.5
+            want[b] = (torch.softmax(s, -1)[..., None] * v.double()[:, None]).sum(2).view(Hq, D)
+    pos = torch.tensor(lens, dtype=torch.int32, device=gpu)
+    out = _ops().decode_attn(q, kc, vc, pos, None, room, D ** -0.5, 0, bt, None).view(B, Hq, D)
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert not out[b].any()
+        else:
+            assert rel_err(out[b], want[b]) < 2 ** -7, (b, n)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,Hq,Hkv", [(32, 4, 2), (64, 32, 8), (128, 8, 1)])
 @pytest.mark.parametrize("lens", [[1], [127, 1, 129], [256, 65, 700, 128, 3]])
 def test_prompt_attention(gpu, D, Hq, Hkv, lens):
