@@ -6,6 +6,7 @@
 //                      among the choices and streams 16-channel slices of the weights past them; the
 //                      shared expert's slices run in the same launch.  Weights are read once for up to 64
 //                      rows; experts nobody chose are not read.
+#include "e4m3.h"
 #include "gemm8_core.h"
 #include "hybrid.h"
 #include "moe_route.h"
@@ -76,19 +77,24 @@ __global__ void __launch_bounds__(512) moe_route_mfma_kernel(const uint16_t* __r
 // ------------------------------------------------------------------ few tokens
 constexpr int kFewTokens = 64, kFewPairs = 1024;
 
-// What bounds them: weights read once (67 MB up, 34 MB down for 32 tokens at 1B sizes), and behind one another the
-// choices, the list of an expert's pairs, its rows and its weights; several workgroups a CU hide each other's waits,
-// so more loads in flight a wave, which cost registers, lose (blocks of 4 chunks issued ahead of the choices: up
-// 22.5 -> 33.9 us).
+// What bounds them: weights read once (67 MB up, 34 MB down for 32 tokens at 1B sizes: 3.2 and 2.9 TB/s), and behind one another
+// the choices, the list of an expert's pairs, its rows and its weights.  An expert has 8 rows on average there: a block of
+// 16 rows instead of two is a quarter of the loads (up 22.6 -> 21.1 us, 48 tokens 26.4 -> 24.2; 8B sizes 60.7 -> 57.1,
+// 70.5 -> 65.3).  Weights of an expert known by its place, asked for before the choices, gain little by themselves: several
+// workgroups a CU hide each other's waits.
 // One slice set: 16 weight rows a slice, 8 gate and the 8 matching up rows where GLU; KW of the 8 waves share the K
-// of NC slices (a fragment of the rows feeds NC products), 8 / KW such sets a workgroup.
+// of NC slices (a fragment of the rows feeds NC products), 8 / KW such sets a workgroup.  16 rows x 64 B a load: for many
+// rows, whose fragments and sums are then what lasts.
 template <bool GLU, int KW, int NC>
 struct FewSlices {
   static constexpr int SL = 8 / KW * NC, CH = GLU ? 8 : 16, U = 2;
+  typedef int64_t Off;  // of X's rows
+  static constexpr int places(int rows) { return 8 * NC * 64 * ((rows + 15) / 16); }
   const uint16_t* wr[NC];
   int n0, k0, k1, ks;
 
-  __device__ __forceinline__ FewSlices(const uint16_t* W, int bx, int N, int K, int w, int c) {
+  __device__ __forceinline__ FewSlices(const uint16_t* W, int bx, int N, int K, int w, int lane) {
+    const int c = lane & 15;
     ks = w % KW;
     n0 = (bx * SL + w / KW * NC) * CH;
     const int steps = (K + 63) / 64, per = (steps + KW - 1) / KW;
@@ -97,15 +103,21 @@ struct FewSlices {
     for (int j = 0; j < NC; ++j)
       wr[j] = W + ((int64_t)(GLU && c >= 8 ? N : 0) + min(n0 + j * CH + (GLU ? c & 7 : c), N - 1)) * K;
   }
-  // n rows: xrow(r) reads, yrow(r) is the output's; limit of the unit
-  template <int MB, typename X, typename Y>
-  __device__ __forceinline__ void run(int n, int N, X xrow, Y yrow, uint16_t* y, float limit, f32x4* red, int w, int lane,
-                                      int c, int g) {
+  __device__ __forceinline__ void ahead() {}
+  __device__ __forceinline__ void move(int64_t by) {
+#pragma unroll
+    for (int j = 0; j < NC; ++j) wr[j] += by;
+  }
+  // n rows: xrow(r) reads, yrow(r) is the output's; limit of the unit; ROWS at a time; fresh: after ahead()
+  template <int ROWS, typename X, typename Y>
+  __device__ __forceinline__ void run(bool fresh, int n, int N, const uint16_t* xb, X xoff, Y yrow, uint16_t* y, float limit,
+                                      f32x4* red, int w, int lane, int c, int g) {
+    constexpr int MB = (ROWS + 15) / 16;
     auto slot = [&](int wv, int j, int mb) -> f32x4& { return red[((wv * NC + j) * MB + mb) * 64 + lane]; };
     for (int r0 = 0; r0 < n; r0 += 16 * MB) {
       const uint16_t* xr[MB];
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) xr[mb] = xrow(min(r0 + 16 * mb + c, n - 1));
+      for (int mb = 0; mb < MB; ++mb) xr[mb] = xb + xoff(min(r0 + 16 * mb + c, n - 1));
       f32x4 acc[NC][MB];
 #pragma unroll
       for (int j = 0; j < NC; ++j)
@@ -170,34 +182,182 @@ struct FewSlices {
   }
 };
 
+// The same slices for a few rows each, in the fragments of skinny_core.h: loads of 8 rows x 128 B, nontemporal, products of 8
+// token rows with two useful blocks.  K in blocks of as many chunks as a wave's part has or twice that: loads past its end,
+// repeated ones, cost as others do (down, 6 chunks in two parts, blocks of 4 13.6 us, of 3 11.8).  The first U chunks of a wave's part are
+// asked for before the rows are known.  K a multiple of 64, offsets of 32 bits.
+template <bool GLU, int KW, int NC, int UC>
+struct FewLines {
+  static constexpr int SL = 8 / KW * NC, CH = GLU ? 8 : 16, RB = 2 * NC, U = UC;  // block 2 j: gate rows, or rows 0 .. 7
+  static constexpr int places(int rows) { return 8 * RB * 16 * ((rows + 7) / 8); }
+  typedef uint32_t Off;  // of X's rows
+  typedef u32x4 Frag[U][RB];  // (as vectors of 16 bits they come apart where paths join)
+  const char* W;
+  uint32_t wo[RB];
+  int n0, c0, c1, cl, ks;  // chunks of 64 k: this wave's, the last of all
+  Frag pre;
+
+  __device__ __forceinline__ FewLines(const uint16_t* w_, int bx, int N, int K, int w, int lane) {
+    const int c = lane & 15, g = lane >> 4;
+    W = reinterpret_cast<const char*>(w_);
+    ks = w % KW;
+    n0 = (bx * SL + w / KW * NC) * CH;
+    const int steps = K / 64, per = (steps + KW - 1) / KW;
+    c0 = ks * per, c1 = min(steps, c0 + per), cl = steps - 1;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const int ch = n0 + (rb >> 1) * CH + (GLU ? 0 : 8 * (rb & 1)) + (c & 7);
+      wo[rb] = ((uint32_t)((GLU && (rb & 1) ? N : 0) + min(ch, N - 1)) * (uint32_t)K + (uint32_t)sk_lane_k(c, g)) * 2;
+    }
+  }
+  __device__ __forceinline__ void load(Frag& f, int c) const {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const char* p = W + 128 * (int64_t)min(c + u, cl);
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) f[u][rb] = sk_weights<u32x4>(p + wo[rb]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void ahead() { load(pre, c0); }
+  __device__ __forceinline__ void move(int64_t by) { W += 2 * by; }
+  // xoff(r): offset of row r from X, in elements
+  template <int ROWS, typename X, typename Y>
+  __device__ __forceinline__ void run(bool fresh, int n, int N, const uint16_t* xb, X xoff, Y yrow, uint16_t* y, float limit,
+                                      f32x4* red, int w, int lane, int c, int g) {
+    constexpr int TB = (ROWS + 7) / 8, MB = (TB + 1) / 2, UX = TB == 1 || U < 4 ? U : U / 2;  // chunks of rows in flight
+    auto at = [&](int wv, int rb, int tb) { return ((wv * RB + rb) * TB + tb) * 16; };
+    // (the first rows apart: ahead()'s weights are then no longer held)
+    auto rows = [&](int r0, auto first) __attribute__((always_inline)) {
+      uint32_t xo[TB];
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb) xo[tb] = (xoff(min(r0 + 8 * tb + (c & 7), n - 1)) + (uint32_t)sk_lane_k(c, g)) * 2;
+      f32x4 acc[RB][TB];
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+      auto step = [&](const Frag& f, int cb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += UX) {
+          u32x4 fb[UX][TB];
+#pragma unroll
+          for (int u = 0; u < UX; ++u) {
+            const int cu = cb + u0 + u;
+            const char* p = reinterpret_cast<const char*>(xb) + 128 * (int64_t)min(cu, cl);
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) {
+              fb[u][tb] = *reinterpret_cast<const u32x4*>(p + xo[tb]);
+              if (cu >= c1) fb[u][tb] = u32x4{0, 0, 0, 0};
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int u = 0; u < UX; ++u)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+              for (int tb = 0; tb < TB; ++tb)
+                acc[rb][tb] = mfma16_sk(__builtin_bit_cast(u16x8, f[u0 + u][rb]), __builtin_bit_cast(u16x8, fb[u][tb]),
+                                        acc[rb][tb]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      };
+      int cb = c0;
+      if constexpr (first) {
+        step(pre, cb);
+        cb += U;
+      }
+      for (; cb < c1; cb += U) {
+        Frag f;
+        load(f, cb);
+        step(f, cb);
+      }
+      if (r0) __syncthreads();  // the previous rows' sums are read
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+          const f32x4 s = sk_both_halves(acc[rb][tb]);
+          if (c < 8 && g < 2) red[at(w, rb, tb) + 8 * g + c] = s;
+        }
+      __syncthreads();
+      for (int jm = ks; jm < NC * MB; jm += KW) {  // the K parts' waves share the sums
+        const int j = jm % NC, mb = jm / NC, tb = 2 * mb + (c >> 3);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < KW; ++i)
+          s += red[at(w - ks + i, 2 * j + (g >> 1), min(tb, TB - 1)) + 8 * (g & 1) + (c & 7)];
+        const int r = r0 + 16 * mb + c, ch = n0 + j * CH + 4 * g;
+        u16x4 o;
+        if constexpr (GLU) {  // gate in groups 0 and 1, up in 2 and 3
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float up = __shfl_xor(s[i], 32, 64);
+            o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, limit));
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+        }
+        if (tb < TB && r < n && ch < N && (!GLU || g < 2)) *reinterpret_cast<u16x4*>(y + (int64_t)yrow(r) * N + ch) = o;
+      }
+    };
+    int r0 = 0;
+    if (fresh) {
+      rows(0, std::true_type{});
+      r0 = 8 * TB;
+    }
+    for (; r0 < n; r0 += 8 * TB) rows(r0, std::false_type{});
+  }
+};
+
 // GLU: y[pair] = clipped unit of x[token] through [gate | up]; else y[pair] = W x[pair].
 // Workgroups: the shared expert's slices (its rows are the tokens), then those of every expert, or - fewer pairs
-// than experts - of every pair whose expert no earlier pair has chosen.  KW, NC, MB: the experts' slices (MB blocks
-// of 16 rows at a time); SKW, SNC, SMB the shared one's, whose K is longer and whose rows are all tokens.
-// a.logits (GLU): the choices are made here from the router's logits; one workgroup stores them.
-template <bool GLU, int KW, int NC, int MB, int SKW, int SNC, int SMB>
-__global__ void __launch_bounds__(512) moe_few_kernel(MoeFew a) {
-  using Own = FewSlices<GLU, KW, NC>;
-  using Shared = FewSlices<GLU, SKW, SNC>;
+// than experts - of every pair whose expert no earlier pair has chosen.  Own, ROWS: the experts' slices (up to ROWS rows at a
+// time; LESS: up to so many of them, fewer products); Shared, SROWS the shared one's, whose K is longer and whose rows are all
+// tokens.  a.logits (GLU): the choices are made here from the router's logits; one workgroup stores them.  TMAX: most tokens.
+template <bool GLU, typename Own, int ROWS, int LESS, typename Shared, int SROWS, int TMAX>
+__global__ void __launch_bounds__(512, TMAX <= 32 ? 4 : 2) moe_few_kernel(MoeFew a) {
   __shared__ int16_t sel[kFewPairs], list[kFewPairs];
   __shared__ int count;
-  __shared__ f32x4 red[8 * 64 * (NC * MB > SNC * SMB ? NC * MB : SNC * SMB)];
+  __shared__ f32x4 red[Own::places(ROWS) > Shared::places(SROWS) ? Own::places(ROWS) : Shared::places(SROWS)];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
+  typedef typename Own::Off Off;
   constexpr int SCOLS = Shared::SL * Shared::CH, COLS = Own::SL * Own::CH;
   const int snx = a.sw ? (a.sN + SCOLS - 1) / SCOLS : 0, nx = (a.N + COLS - 1) / COLS, P = a.T * a.top;
   if ((int)blockIdx.x < snx) {
-    Shared s(a.sw, blockIdx.x, a.sN, a.sK, w, c);
-    s.template run<SMB>(
-        a.T, a.sN, [&](int r) { return GLU ? a.x + (int64_t)r * a.ldx : a.sx + (int64_t)r * a.sK; },
+    Shared s(a.sw, blockIdx.x, a.sN, a.sK, w, lane);
+    s.ahead();
+    s.template run<SROWS>(
+        true, a.T, a.sN, GLU ? a.x : a.sx, [&](int r) { return GLU ? r * (Off)a.ldx : r * (Off)a.sK; },
         [](int r) { return r; }, a.sy, a.slimit, red, w, lane, c, g);
     return;
   }
   const int bx = (blockIdx.x - snx) % nx, unit = (blockIdx.x - snx) / nx;
+  // What the choices are made of is asked for first, all of it at once, and the weights of an expert known by its place behind
+  // it: the choices do not wait for them (no barrier here drains the loads), and they do not wait for the choices.
+  constexpr int TW = (TMAX + 7) / 8;  // tokens of a wave
+  float z[TW];
   if (GLU && a.logits) {
-    for (int t = w; t < a.T; t += 8) {
+#pragma unroll
+    for (int i = 0; i < TW; ++i) z[i] = a.logits[(int64_t)min(w + 8 * i, a.T - 1) * a.E + min(lane, a.E - 1)];
+  } else {
+    for (int i = tid; i < P; i += 512) sel[i] = (int16_t)min(max(a.ids[i], 0), a.E - 1);
+  }
+  const int64_t wsize = (int64_t)(GLU ? 2 : 1) * a.N * a.K;
+  const bool known = P > a.E;
+  __builtin_amdgcn_sched_barrier(0);
+  Own s(a.w + (known ? unit : 0) * wsize, bx, a.N, a.K, w, lane);
+  if (known) s.ahead();
+  if (GLU && a.logits) {
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+      const int t = w + 8 * i;
+      if (t >= a.T) break;
       const int store = (int)blockIdx.x == snx;
-      moe_choose64(lane < a.E ? a.logits[(int64_t)t * a.E + lane] : 0.f, a.E, a.top, lane, [&](int k, float wt) {
+      moe_choose64(z[i], a.E, a.top, lane, [&](int k, float wt) {
         sel[t * a.top + k] = (int16_t)lane;
         if (store) {
           a.ids_out[t * a.top + k] = lane;
@@ -205,11 +365,9 @@ __global__ void __launch_bounds__(512) moe_few_kernel(MoeFew a) {
         }
       });
     }
-  } else {
-    for (int i = tid; i < P; i += 512) sel[i] = (int16_t)min(max(a.ids[i], 0), a.E - 1);
   }
-  __syncthreads();
-  const int expert = P <= a.E ? sel[unit] : unit;
+  lds_barrier();
+  const int expert = known ? unit : __builtin_amdgcn_readfirstlane(sel[unit]);
   if (w == 0) {  // pairs whose choice this expert is
     int at = 0, first = P;
     for (int i0 = 0; i0 < P; i0 += 64) {
@@ -219,14 +377,16 @@ __global__ void __launch_bounds__(512) moe_few_kernel(MoeFew a) {
       if (m && first == P) first = i0 + __ffsll((unsigned long long)m) - 1;
       at += __popcll(m);
     }
-    if (lane == 0) count = P <= a.E && first < unit ? 0 : at;
+    if (lane == 0) count = !known && first < unit ? 0 : at;
   }
-  __syncthreads();
-  if (count == 0) return;
-  Own s(a.w + (int64_t)expert * (GLU ? 2 : 1) * a.N * a.K, bx, a.N, a.K, w, c);
-  s.template run<MB>(
-      count, a.N, [&](int r) { return a.x + (int64_t)(GLU ? list[r] / a.top : list[r]) * a.ldx; },
-      [&](int r) { return list[r]; }, a.y, a.limit, red, w, lane, c, g);
+  lds_barrier();
+  const int n = __builtin_amdgcn_readfirstlane(count);
+  if (n == 0) return;
+  if (!known) s.move(expert * wsize);
+  auto xoff = [&](int r) { return (Off)(GLU ? list[r] / a.top : list[r]) * (Off)a.ldx; };
+  auto yrow = [&](int r) { return list[r]; };
+  if (LESS < ROWS && n <= LESS) s.template run<LESS>(known, n, a.N, a.x, xoff, yrow, a.y, a.limit, red, w, lane, c, g);
+  else s.template run<ROWS>(known, n, a.N, a.x, xoff, yrow, a.y, a.limit, red, w, lane, c, g);
 }
 
 }  // namespace mx
@@ -285,28 +445,46 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
   // down 64, for a few pairs 32 with K in four parts; the shared expert's down, whose K is the longest, 16 with K in
   // eight (its few workgroups were the last to end: K 2048 in two parts are 16 waits for memory one after another;
   // 32 tokens, 1B sizes 30.5 -> 16.1 us, 4 tokens 15.6 -> 10.3; 8B sizes 38.4 -> 33.1, 22.2 -> 18.7)
-  const bool split = !glu && a.T * a.top <= 8;
   const int64_t units = a.T * a.top <= a.E ? a.T * a.top : a.E;
-#define MF(GLU, KW, NC, MB, SKW, SNC, SMB)                                                                       \
+#define MF(GLU, OWN, ROWS, LESS, SHARED, SROWS, TMAX)                                                            \
   do {                                                                                                           \
-    const int64_t cols = 8 / KW * NC * (GLU ? 8 : 16), sc = 8 / SKW * SNC * (GLU ? 8 : 16);                      \
+    typedef OWN Own;                                                                                             \
+    typedef SHARED Shared;                                                                                       \
+    const int64_t cols = Own::SL * Own::CH, sc = Shared::SL * Shared::CH;                                        \
     const int64_t gr = units * ((a.N + cols - 1) / cols) + (a.sw ? (a.sN + sc - 1) / sc : 0);                    \
     if (gr > INT32_MAX) return -1;                                                                               \
-    moe_few_kernel<GLU, KW, NC, MB, SKW, SNC, SMB><<<(unsigned)gr, 512, 0, stream>>>(a);                         \
+    moe_few_kernel<GLU, Own, ROWS, LESS, Shared, SROWS, TMAX><<<(unsigned)gr, 512, 0, stream>>>(a);              \
   } while (0)
+#define FS(...) FewSlices<__VA_ARGS__>
+#define FL(...) FewLines<__VA_ARGS__>
+  // Down: FewLines, which reads a part of K in blocks of 3 chunks, where it was the faster one: a short K but for 5 to 8 pairs
+  // (four K parts; 2048 x 384, 4 / 8 / 32 / 128 pairs, us: 5.2 / 7.8 / 10.4 (16 tokens) / 11.8 by it, 5.7 / 7.1 / 11.8 / 15.4
+  // by FewSlices), a longer one up to 8 pairs and past 16 tokens (4096 x 768, 2 / 8 / 16 / 32 tokens 14.6 / 23.8 / 25.8 /
+  // 29.4, 15.7 / 23.4 / 25.6 / 33.0).  Up stays with FewSlices (2 x 384 x 2048, 32 tokens 21.1 us, 23.3 by FewLines; 768 x 4096
+  // 57.1, 62.4).
+  const int pairs = a.T * a.top;
+  const bool lines = !glu && a.K % 64 == 0 && (!a.sw || a.sK % 64 == 0) &&
+                     (a.K < 512 ? pairs <= 4 || pairs > 8 : pairs <= 8 || a.T > 16) &&
+                     std::max(std::max((int64_t)a.N * a.K, (int64_t)a.sN * a.sK),
+                              pairs * std::max(a.ldx, (int64_t)a.sK)) < (1ll << 31) - 4096;
   if (glu) {
-    if (a.T <= 16) MF(true, 8, 2, 1, 8, 2, 1);
-    else if (a.T <= 32) MF(true, 8, 2, 2, 8, 2, 2);
-    else MF(true, 8, 4, 4, 8, 4, 4);
-  } else if (split) {
-    MF(false, 4, 1, 1, 8, 1, 1);
-  } else if (a.T <= 16) {
-    MF(false, 2, 1, 1, 8, 1, 1);
-  } else if (a.T <= 32) {
-    MF(false, 2, 1, 2, 8, 1, 2);
+    if (a.T <= 16) MF(true, FS(true, 8, 2), 16, 16, FS(true, 8, 2), 16, 16);
+    else if (a.T <= 32) MF(true, FS(true, 8, 2), 32, 16, FS(true, 8, 2), 32, 32);
+    else MF(true, FS(true, 8, 4), 64, 16, FS(true, 8, 4), 64, 64);
+  } else if (pairs <= 8 && !lines) {
+    MF(false, FS(false, 4, 1), 16, 16, FS(false, 8, 1), 16, 16);
+  } else if (lines) {
+    if (a.T <= 8) MF(false, FL(false, 2, 1, 3), 8, 8, FL(false, 8, 1, 4), 8, 8);
+    else if (a.T <= 16) MF(false, FL(false, 2, 1, 3), 16, 8, FL(false, 8, 1, 4), 16, 16);
+    else if (a.T <= 32) MF(false, FL(false, 2, 1, 3), 16, 8, FS(false, 8, 1), 32, 32);
+    else MF(false, FL(false, 2, 1, 3), 32, 16, FS(false, 8, 1), 64, 64);
   } else {
-    MF(false, 2, 1, 4, 8, 1, 4);
+    if (a.T <= 16) MF(false, FS(false, 2, 1), 16, 16, FS(false, 8, 1), 16, 16);
+    else if (a.T <= 32) MF(false, FS(false, 2, 1), 32, 16, FS(false, 8, 1), 32, 32);
+    else MF(false, FS(false, 2, 1), 64, 16, FS(false, 8, 1), 64, 64);
   }
+#undef FL
+#undef FS
 #undef MF
   return (int)hipGetLastError();
 }

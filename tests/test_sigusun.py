@@ -21,6 +21,7 @@ from mxllm.ops import latent as lops  # noqa: E402
 from mxllm.ops import moe as mops  # noqa: E402
 from mxllm.ops import retention as rops  # noqa: E402
 from mxllm.ops import sublayer as sops  # noqa: E402
+from mxllm.ops import native  # noqa: E402
 from mxllm.serve.engine import Engine  # noqa: E402
 from mxllm.serve.kvcache import KVCache  # noqa: E402
 
@@ -148,6 +149,30 @@ def test_experts_chosen_from_logits(gpu, T, experts, top):
     assert sh is None
     close(wts2, wts, torch.float32, 20)
     close(y2, y, bf)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ff,shared", [(64, 64), (192, 0), (384, 2048), (448, 128), (768, 192)])
+@pytest.mark.parametrize("T", [1, 3, 8, 9, 16, 17, 32, 33, 64])
+def test_down_products_of_few_rows(gpu, T, ff, shared):
+    """Whole-line fragments of the experts' down products: K parts of none, some and all of a block of chunks, a remainder of
+    channels, an expert with nearly every row (several turns of them), ones with a few and one that nobody chose."""
+    bf, N, E, top = torch.bfloat16, 144, 6, 3
+    w = (rnd(E, N, ff, seed=1) / ff ** 0.5).to(bf)
+    g = torch.Generator().manual_seed(T + ff)
+    z = torch.randn(T, E, generator=g)
+    z[:, 1] += 3.0
+    z[:, 4] -= 100.0
+    ids = z.topk(top, 1).indices
+    x = rnd(T * top, ff, seed=2, dt=bf)
+    sw = (rnd(N, shared, seed=3) / shared ** 0.5).to(bf) if shared else None
+    sx = rnd(T, shared, seed=4, dt=bf) if shared else None
+    y, sy, _, _ = native().moe_few(x.to(gpu), ids.int().to(gpu), None, top, w.to(gpu), False, 0.0,
+                                   sw.to(gpu) if shared else None, sx.to(gpu) if shared else None, 0.0)
+    want = torch.stack([w[e].double() @ r.double() for e, r in zip(ids.flatten().tolist(), x)])
+    close(y.view(T * top, N), want, bf, 0.3)  # f32 sums, one rounding to bf16 (2^-9)
+    if shared:
+        close(sy, sx.double() @ sw.double().T, bf, 0.3)
 
 
 @on_devices
