@@ -656,6 +656,149 @@ __global__ void __launch_bounds__(kEvenD)
   out[bh * kEvenD + d] = f2bf(L > 0.f ? acc / L : 0.f);
 }
 
+// ---------------------------------------------------------------------------
+// Decode attention of up to 512 keys: eight waves take a whole (sequence, KV head), 64 keys each, so that nothing is left
+// to merge in a launch of its own.  K and V in registers as in EvenState; each wave leaves its maximum, sum and outputs
+// in LDS, where they are added as decode_split_body adds four waves and decode_combine_kernel two splits, so the bits
+// are those of the splits.
+//
+// Both launches against this one, 32 heads of 8, us: heads of 64, 1 / 4 / 32 sequences of up to 300 / 400 / 400 keys
+// 6.5 / 7.1 / 11.0 -> 5.2 / 6.0 / 7.1; of 128, 8.6 / 9.0 / 15.7 -> 6.5 / 7.4 / 10.5.  Past 512 keys a CU to a sequence is too
+// little (16 waves of 64 keys, one sequence of 700 keys, heads of 64: 7.2 in splits, 7.6 so; 2,048 keys 7.6, 16.9).
+constexpr int kShortSplits = 2, kShortRep = 8;  // q-heads of a KV head: 34 KB of LDS at heads of 128
+
+template <int D>
+__global__ void __launch_bounds__(512)
+    decode_short_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
+                        const int32_t* __restrict__ lens, int len_off, const int32_t* __restrict__ slots,
+                        uint16_t* __restrict__ out, int Hq, int Hkv, int max_seq, float sl,
+                        const int32_t* __restrict__ bt, int maxb) {
+  constexpr int KS = D / 32, E = D / 16, NP = D == 128 ? 1 : 3, TILES = 4 * kShortSplits;
+  typedef uint32_t vrow_t __attribute__((ext_vector_type(E / 2)));
+  typedef float orow_t __attribute__((ext_vector_type(E)));
+  __shared__ float mls[TILES][2][16];
+  __shared__ __attribute__((aligned(16))) float so[TILES * kShortRep * D];
+  const int tid = threadIdx.x, lane = tid & 63, t = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4, hk = blockIdx.x, b = blockIdx.y, rep = Hq / Hkv;
+  const int len = min(max(lens[b] + len_off, 0), kShortSplits * kSplit), slot = slots ? slots[b] : b;
+  const int lim = len - 1 - 64 * t;  // the last row of the wave's tile that is read
+  if (lim < 0) {
+    if (g == 0) mls[t][0][c] = -INFINITY, mls[t][1][c] = 0.f;
+  } else {
+    u16x8 qf[KS];
+    const uint16_t* qrow = q + ((int64_t)b * Hq + hk * rep + min(c, rep - 1)) * D;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      qf[s] = *reinterpret_cast<const u16x8*>(qrow + 32 * s + 8 * g);
+      if (c >= rep) qf[s] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+    const int64_t base = kv_row(bt, maxb, max_seq, slot, Hkv, hk, 64 * t) * D;  // a tile lies in one block
+    const uint16_t *kb = kc + base, *vb = vc + base;
+    u32x4_t k[4][KS];
+    vrow_t v[16];  // slot s: key 16 (s >> 2) + 4 g + (s & 3), channels E c ..
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t r = min(16 * j + c, lim) * D + 8 * g;
+#pragma unroll
+      for (int s = 0; s < KS; ++s) k[j][s] = *reinterpret_cast<const u32x4_t*>(kb + (r + 32 * s));
+    }
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      v[s] = *reinterpret_cast<const vrow_t*>(vb + (uint32_t)(min(16 * (s >> 2) + 4 * g + (s & 3), lim) * D + E * c));
+    __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
+    f32x4 sc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      sc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) sc[j] = mfma16(__builtin_bit_cast(u16x8, k[j][s]), qf[s], sc[j]);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = 16 * j + 4 * g + i <= lim ? sc[j][i] * sl : -INFINITY;
+        sc[j][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float mref = mx == -INFINITY ? 0.f : mx;
+    float ls = 0.f;
+    u16x8 pb[NP][2];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float p = __builtin_amdgcn_exp2f(sc[j][i] - mref);
+        ls += p;
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+          pb[n][j >> 1][4 * (j & 1) + i] = f2bf(p);
+          p -= bf2f(pb[n][j >> 1][4 * (j & 1) + i]);
+        }
+      }
+    ls += __shfl_xor(ls, 16, 64);
+    ls += __shfl_xor(ls, 32, 64);
+    if (g == 0) mls[t][0][c] = mx, mls[t][1][c] = ls;
+    f32x4 o[E];  // [e][i]: channel E (4 g + i) + e of head c
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        u32x4_t a;  // channel e of 8 keys: one half of a word of each
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t hi, lo;
+          if constexpr (E == 2) hi = v[8 * h + 2 * i + 1][0], lo = v[8 * h + 2 * i][0];
+          else hi = v[8 * h + 2 * i + 1][e >> 1], lo = v[8 * h + 2 * i][e >> 1];
+          a[i] = __builtin_amdgcn_perm(hi, lo, e & 1 ? 0x07060302u : 0x05040100u);
+        }
+#pragma unroll
+        for (int n = NP - 1; n >= 0; --n) o[e] = mfma16(__builtin_bit_cast(u16x8, a), pb[n][h], o[e]);
+      }
+    }
+    if (c < rep) {
+      float* const dst = so + (t * rep + c) * D + 4 * E * g;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        orow_t y;
+#pragma unroll
+        for (int e = 0; e < E; ++e) y[e] = o[e][i];
+        *reinterpret_cast<orow_t*>(dst + E * i) = y;
+      }
+    }
+  }
+  __syncthreads();
+  for (int idx = tid; idx < rep * D; idx += 512) {
+    const int h = idx / D, d = idx % D;
+    float M = -INFINITY, L = 0.f, acc = 0.f;
+#pragma unroll
+    for (int w = 0; w < TILES; ++w) M = fmaxf(M, mls[w][0][h]);
+#pragma unroll
+    for (int s = 0; s < kShortSplits; ++s) {
+      float m = -INFINITY, lv = 0.f, ov = 0.f;
+#pragma unroll
+      for (int w = 4 * s; w < 4 * s + 4; ++w) m = fmaxf(m, mls[w][0][h]);
+#pragma unroll
+      for (int w = 4 * s; w < 4 * s + 4; ++w) {
+        const float mw = mls[w][0][h];
+        if (mw == -INFINITY) continue;  // (its outputs may not have been written)
+        const float f = __builtin_amdgcn_exp2f(mw - m);
+        lv += f * mls[w][1][h];
+        ov += f * so[(w * rep + h) * D + d];
+      }
+      if (m == -INFINITY) continue;
+      const float wgt = __builtin_amdgcn_exp2f(m - M);
+      L += wgt * lv;
+      acc += wgt * ov;
+    }
+    out[((int64_t)b * Hq + hk * rep + h) * D + d] = f2bf(L > 0.f ? acc / L : 0.f);
+  }
+}
+
 __device__ __forceinline__ uint32_t hash3(uint32_t a, uint32_t b, uint32_t c) {
   uint32_t h = a * 0x9E3779B1u ^ (b + 0x7F4A7C15u) * 0x85EBCA77u ^ (c + 0x165667B1u) * 0xC2B2AE3Du;
   h ^= h >> 15; h *= 0x2C1B3C6Du; h ^= h >> 12; h *= 0x297A2D39u; h ^= h >> 15;
@@ -784,6 +927,14 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
   const char* pe = getenv("MXLLM_DECODE_HANDOFF");
   const int proto = pe && *pe ? atoi(pe) : 4;
   const bool fused = out && cnt && D == 128 && proto >= 1 && proto <= 4;
+  // up to 512 keys: one launch (B: the grid's second dimension)
+  if (out && nsplit == kShortSplits && Hq / Hkv <= kShortRep && B <= 65535) {
+#define DS(DD) \
+  decode_short_kernel<DD><<<dim3(Hkv, B), 512, 0, stream>>>(q, kc, vc, lens, len_off, slots, out, Hq, Hkv, max_seq, sl, bt, maxb)
+    if (D == 128) DS(128); else if (D == 64) DS(64); else if (D == 32) DS(32); else return -1;
+#undef DS
+    return (int)hipGetLastError();
+  }
   // Heads of 128, more splits than places: dealt evenly.  What the caller's `nsplit` counts is the longest that the step
   // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.  The buffers have
   // 2 nsplit + 1 parts a row (a row of n units touches at most (n + share - 2) / share + 1 shares of 8 units or more).

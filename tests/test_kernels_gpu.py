@@ -993,6 +993,36 @@ def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("Hq,Hkv", [(16, 2), (4, 4), (7, 1), (9, 1)])
+def test_decode_attn_up_to_512_keys(gpu, D, Hq, Hkv):
+    """Both splits of a sequence in one workgroup (up to 8 query heads of a KV head; 9 take two launches): lengths at the
+    edges of waves and splits, none (zeros); stale rows are NaN.  Softmax weights of heads of 128 and every output are rounded to
+    bf16 (2^-9 each): within 2^-7 of f64."""
+    lens = [512, 0, 1, 63, 64, 65, 255, 256, 257, 320, 321, 511]
+    B = len(lens)
+    torch.manual_seed(D + Hq)
+    kc = torch.full((B, Hkv, 600, D), float("nan"), device=gpu, dtype=torch.bfloat16)
+    vc = kc.clone()
+    q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+    slots = torch.randperm(B, device=gpu).to(torch.int32)
+    want = torch.zeros(B, Hq, D, dtype=torch.float64, device=gpu)
+    for b, n in enumerate(lens):
+        k, v = (torch.randn(Hkv, n, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        kc[int(slots[b]), :, :n], vc[int(slots[b]), :, :n] = k, v
+        if n:
+            s = (q[b].double().view(Hkv, Hq // Hkv, 1, D) * k.double()[:, None]).sum(-1) * D ** -0.5
+            want[b] = (torch.softmax(s, -1)[..., None] * v.double()[:, None]).sum(2).view(Hq, D)
+    pos = torch.tensor(lens, dtype=torch.int32, device=gpu) - 1
+    out = _ops().decode_attn(q, kc, vc, pos, slots, 512, D ** -0.5, 1, None, None).view(B, Hq, D)
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert not out[b].any()
+        else:
+            assert rel_err(out[b], want[b]) < 2 ** -7, (b, n)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv,lens,room", [(32, 8, [1, 15, 16, 17, 255, 256, 257, 0] + [1, 33, 700, 90] * 6, 700),
                                               (16, 1, [3000, 0, 1, 2600], 65536), (8, 8, [4000, 4096], 8448),
                                               (6, 2, [5] * 300, 256), (64, 8, [2000, 64, 65, 1999, 1, 1900], 3000)])
