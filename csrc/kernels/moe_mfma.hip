@@ -433,6 +433,8 @@ extern "C" int mx_moe_grouped(const MoeGemm* pa, int64_t xrows, hipStream_t stre
   return (int)hipGetLastError();
 }
 
+extern "C" int mx_moe_stream(const MoeFew* pa, hipStream_t stream);
+
 extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
   const MoeFew& a = *pa;
   if (a.T <= 0) return 0;
@@ -441,7 +443,12 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
       (a.logits && (!glu || a.E > 64 || a.top > a.E)) || (!a.logits && !a.ids) || a.N <= 0 || a.N % 4 || a.K <= 0 || a.K % 16 || a.ldx % 8 || a.ldx < a.K || (al & 15) ||
       (a.sw && (a.sN <= 0 || a.sN % 4 || a.sK <= 0 || a.sK % 16)))
     return -1;
-  // channels of a workgroup: up 16, from 33 tokens on 32 (the rows' fragments are then most of the traffic);
+  if (glu) {
+    const int r = mx_moe_stream(pa, stream);
+    if (r != -1) return r;
+  }
+  // channels of a workgroup: up 16, from 33 tokens on 32 (the rows' fragments are then most of the traffic; first
+  // moe_stream.hip, more pairs than experts);
   // down 64, for a few pairs 32 with K in four parts; the shared expert's down, whose K is the longest, 16 with K in
   // eight (its few workgroups were the last to end: K 2048 in two parts are 16 waits for memory one after another;
   // 32 tokens, 1B sizes 30.5 -> 16.1 us, 4 tokens 15.6 -> 10.3; 8B sizes 38.4 -> 33.1, 22.2 -> 18.7)

@@ -1,5 +1,5 @@
-// The walk of the decode GEMMs over few workgroups that stay (stream_gemm.hip, hybrid_stream.hip): a workgroup of 8
-// waves holds its token rows X in LDS and goes over channel groups grp = blockIdx.x, + gridDim.x, ..., only weights in its
+// The walk of the decode GEMMs over few workgroups that stay (stream_gemm.hip, moe_stream.hip): a workgroup of 8
+// waves holds its token rows X in LDS and goes over channel groups grp = first, + step, ... < groups, only weights in its
 // load queue, two blocks of U 64-k chunks in flight.
 //   row(grp): weight row of channel 0 of a group; off(ch): rows from there to channel ch's, the same in every group (a
 //     scalar base and 32-bit offsets: as 64-bit addresses a lane's two rows spilled registers);
@@ -90,8 +90,8 @@ constexpr int kStreamRed = kStreamPlaces<KIND, TB, KP> * kStreamImages<KIND, TB,
 
 // TB blocks of 8 (lines) or 16 tokens, KP K parts (kStF8Lines: 4, without lines: 8)
 template <int KIND, int TB, int KP, int NL, typename Row, typename Off, typename Stage, typename Finish>
-__device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const float* scale, int M, int K, int groups,
-                                            char* smem, const Row& row, const Off& off, const Stage& stage,
+__device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const float* scale, int M, int K, int first,
+                                            int step, int groups, char* smem, const Row& row, const Off& off, const Stage& stage,
                                             const Finish& finish) {
   constexpr bool F8 = KIND == kStF8 || KIND == kStF8Lines, LINES = KIND == kStLines || KIND == kStF8Lines;
   static_assert(KIND != kStF8Lines || KP == 4, "one block of codes a wave");
@@ -108,7 +108,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
   uint16_t* xs = reinterpret_cast<uint16_t*>(smem + kStreamRed<KIND, TB, KP>);
   const int k0 = sk_part<KP>(w) * kq + (F8 && LINES ? 2 * sk_lane_k(c, g) : LINES ? sk_lane_k(c, g) : F8 ? 16 * g : 8 * g);
   // the block to load next: group lg, block lb
-  int lg = blockIdx.x, lb = 0;
+  int lg = first, lb = 0;
   uint32_t lo[RB];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
@@ -120,7 +120,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
     lp += CH * CK * WB;
     if (++lb == nblk) {
       lb = 0;
-      lg += gridDim.x;
+      lg += step;
       lp = reinterpret_cast<const char*>(W) + row(min(lg, groups - 1)) * ldw * WB;
     }
   };
@@ -138,7 +138,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
       for (int tb = 0; tb < TB; ++tb) acc[rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
   };
   clear();
-  int cg = blockIdx.x, cb = 0, turn = 0;
+  int cg = first, cb = 0, turn = 0;
   auto multiply = [&](const WFrag<KIND, NL, RB>& f) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
@@ -197,9 +197,9 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
     }
     if constexpr (NRED == 1) lds_barrier();  // one image: its sum is read before the next group's parts
     ++turn;
-    cg += gridDim.x;
+    cg += step;
   };
-  const int steps = (groups - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x * nblk;
+  const int steps = (groups - first + step - 1) / step * nblk;
   if (steps == 1) {
     multiply(f0);
     return;

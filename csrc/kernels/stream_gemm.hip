@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm
       *reinterpret_cast<u16x4*>(a.Y + (int64_t)m * a.ldy + (int64_t)cg * 16 + 4 * g) = o;
     }
   };
-  stream_walk<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, a.groups, smem, row, off, stage, finish);
+  stream_walk<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, (int)blockIdx.x, (int)gridDim.x, a.groups, smem, row, off, stage, finish);
 }
 
 constexpr int kTwoLds = 80 * 1024;  // LDS up to which two workgroups share a CU

@@ -36,7 +36,7 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
               ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
-               "mingru", "moe", "moe_mfma", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
+               "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
                "stream_gemm"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),
 }

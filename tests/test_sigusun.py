@@ -152,6 +152,31 @@ def test_experts_chosen_from_logits(gpu, T, experts, top):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,K,ff,shared", [(5, 4, 1, 2048, 8, 0), (9, 8, 2, 2048, 24, 40), (32, 3, 2, 2048, 56, 2048),
+                                                 (32, 6, 3, 4096, 72, 64), (17, 16, 4, 4096, 768, 264), (20, 5, 4, 8192, 16, 16),
+                                                 (33, 8, 2, 2048, 64, 64), (8, 9, 2, 4096, 1024, 0)])
+def test_up_products_past_rows_in_lds(gpu, T, E, top, K, ff, shared):
+    """Workgroups that stay with an expert: rows of one and two blocks and of two turns (experts with nearly every token, the
+    shared one), an expert that nobody chose, runs of channel groups with a shorter end; and sizes left to the other kernel."""
+    bf = torch.bfloat16
+    x = rnd(T, K, seed=1, dt=bf)
+    wgu = (rnd(E, 2 * ff, K, seed=2) * 1.5 / K ** 0.5).to(bf)
+    sgu = (rnd(2 * shared, K, seed=3) * 1.5 / K ** 0.5).to(bf) if shared else None
+    z = torch.randn(T, E, generator=torch.Generator().manual_seed(T + K))
+    z[:, 1] += 3.0
+    z[:, 2] -= 100.0
+    y, sy, ids, wts = native().moe_few(x.to(gpu), None, z.to(gpu), top, wgu.to(gpu), True, 1.2,
+                                       sgu.to(gpu) if shared else None, None, 0.9)
+    val, at = z.topk(top, 1)
+    assert torch.equal(ids.cpu().long(), at)
+    close(wts, torch.softmax(val.double(), 1), torch.float32)
+    want = torch.stack([glu_oracle(x[t].double() @ wgu[e].double().T, 1.2) for t in range(T) for e in at[t].tolist()])
+    close(y.view(T * top, ff), want, bf, 0.3)  # f32 sums, one rounding to bf16 (2^-9)
+    if shared:
+        close(sy, glu_oracle(x.double() @ sgu.double().T, 0.9), bf, 0.3)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ff,shared", [(64, 64), (192, 0), (384, 2048), (448, 128), (768, 192)])
 @pytest.mark.parametrize("T", [1, 3, 8, 9, 16, 17, 32, 33, 64])
 def test_down_products_of_few_rows(gpu, T, ff, shared):
