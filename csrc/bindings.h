@@ -128,6 +128,12 @@ int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, c
                    float eps, uint16_t* h_out, const float* cosb, const float* sinb, const int32_t* pos,
                    const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq, int Hkv, int max_seq,
                    const int32_t* bt, int maxb, hipStream_t stream);
+// stream_parts.hip
+int mx_stream_parts_segments(int M, int N, int K);
+int mx_stream_parts(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, float* parts, int M, int N, int K,
+                    hipStream_t stream);
+int mx_parts_norm(const float* parts, int S, const uint16_t* res, const uint16_t* w, uint16_t* y, uint16_t* h_out, int M,
+                  int H, float eps, hipStream_t stream);
 }
 
 extern "C" {
@@ -162,7 +168,7 @@ int mx_lora_xtg(const int64_t* desc, int np, int T, float alpha, int accumulate,
 // hybrid.hip / mingru.hip / chunk_attn.hip / attn_fwd.hip SEG: f32 != 0 = float activations, else bf16
 int mx_embed_rows(const int64_t* ids, const void* w, int f32, float* out, int64_t T, int W, int V, hipStream_t stream);
 int mx_group_norm(const void* delta, int64_t ldd, float* h, const float* w, void* y, int64_t ldy, int f32, int64_t T,
-                  int W, int groups, float eps, hipStream_t stream);
+                  int W, int groups, float eps, const float* parts, int S, hipStream_t stream);
 int mx_conv_rope_prefill(const mx::ConvRope* a, int f32, const int32_t* rows, int T, hipStream_t stream);
 int mx_conv_rope_decode(const mx::ConvRope* a, int f32, const int32_t* pos, const int32_t* slots, int B,
                         hipStream_t stream);

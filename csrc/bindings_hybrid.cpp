@@ -58,7 +58,23 @@ at::Tensor group_norm(const c10::optional<at::Tensor>& delta, at::Tensor h, cons
     dp = d.data_ptr();
   }
   MX_OK(mx_group_norm(dp, ldd, h.data_ptr<float>(), w.data_ptr<float>(), y.data_ptr(), W, f32, T, (int)W, (int)groups,
-                      (float)eps, cur_stream()));
+                      (float)eps, nullptr, 0, cur_stream()));
+  return y;
+}
+
+// the same of h += the sum of parts [S, T, W] (f32) rounded to bf16
+at::Tensor group_norm_parts(const at::Tensor& parts, at::Tensor h, const at::Tensor& w, int64_t groups, double eps) {
+  check_f32(h, "h");
+  check_f32(w, "w");
+  check_f32(parts, "parts");
+  MX_CHECK(h.dim() == 2 && w.numel() == h.size(1) && groups > 0 && h.size(1) % groups == 0 && parts.dim() == 3 &&
+               parts.size(0) > 0 && parts.size(1) == h.size(0) && parts.size(2) == h.size(1) && parts.device() == h.device(),
+           "group_norm_parts shapes");
+  DevGuard g(h.device());
+  const int64_t T = h.size(0), W = h.size(1);
+  auto y = at::empty({T, W}, h.options().dtype(at::kBFloat16));
+  MX_OK(mx_group_norm(nullptr, 0, h.data_ptr<float>(), w.data_ptr<float>(), y.data_ptr(), W, 0, T, (int)W, (int)groups, (float)eps,
+                      parts.data_ptr<float>(), (int)parts.size(0), cur_stream()));
   return y;
 }
 
@@ -382,6 +398,7 @@ at::Tensor poly_norm(const at::Tensor& z, const at::Tensor& coef, double eps) {
 
 TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("embed_rows(Tensor ids, Tensor w) -> Tensor");
+  m.def("group_norm_parts(Tensor parts, Tensor(a!) h, Tensor w, int groups, float eps) -> Tensor");
   m.def("group_norm(Tensor? delta, Tensor(a!) h, Tensor w, int groups, float eps, bool f32) -> Tensor");
   m.def("conv_rope_prefill(Tensor x, Tensor w, Tensor cos, Tensor sin, int rd, int H, int G, int D, int E, int Dp, int Ep, Tensor rows, int chunk, Tensor(a!)? kc=None, Tensor(b!)? vc=None, Tensor? bt=None, Tensor(c!)? ring=None) -> (Tensor, Tensor, Tensor)");
   m.def("conv_rope_decode(Tensor x, Tensor w, Tensor cos, Tensor sin, int rd, int H, int G, int D, int E, Tensor pos, Tensor slots, int chunk, Tensor(a!) kc, Tensor(b!) vc, Tensor bt, Tensor(c!) ring) -> Tensor");
@@ -399,6 +416,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
 
 TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("embed_rows", &embed_rows);
+  m.impl("group_norm_parts", &group_norm_parts);
   m.impl("group_norm", &group_norm);
   m.impl("conv_rope_prefill", &conv_rope_prefill);
   m.impl("conv_rope_decode", &conv_rope_decode);

@@ -188,6 +188,42 @@ std::tuple<at::Tensor, at::Tensor> stream_linear(const at::Tensor& x, const c10:
   return {y, o.h_out};
 }
 
+// x . w^T as f32 sums over segments of K, [segments, M, N] (rows for parts_norm; stream_parts.hip)
+int64_t stream_parts_segments(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || N < 1 || K < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
+  return mx_stream_parts_segments((int)M, (int)N, (int)K);
+}
+at::Tensor stream_parts(const at::Tensor& x, const at::Tensor& w) {
+  MX_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device() && x.scalar_type() == at::kBFloat16 &&
+               w.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.stride(1) == 1 &&
+               w.stride(1) == 1,
+           "stream_parts: bf16 rows [M, K] and [N, K] on one device");
+  DevGuard g(x.device());
+  const int64_t M = x.size(0), N = w.size(0), K = x.size(1), S = stream_parts_segments(M, N, K);
+  MX_CHECK(S > 0, "stream_parts: sizes not taken");
+  auto y = at::empty({S, M, N}, x.options().dtype(at::kFloat));
+  const int rc = mx_stream_parts(bf(x), x.stride(0), bf(w), w.stride(0), y.data_ptr<float>(), (int)M, (int)N, (int)K, cur_stream());
+  MX_CHECK(rc != -1, "stream_parts: stride or alignment not taken");
+  MX_OK(rc);
+  return y;
+}
+
+// (rmsnorm(h) * w, h) of h = res + the parts' sum, rounded to bf16 first
+std::tuple<at::Tensor, at::Tensor> parts_norm(const at::Tensor& parts, const at::Tensor& res, const at::Tensor& w, double eps) {
+  check_bf16(res, "res");
+  check_bf16(w, "w");
+  MX_CHECK(parts.is_cuda() && parts.scalar_type() == at::kFloat && parts.dim() == 3 && parts.is_contiguous(), "parts f32 [S, M, N]");
+  const int64_t M = parts.size(1), H = parts.size(2);
+  MX_CHECK(res.dim() == 2 && res.size(0) == M && res.size(1) == H && w.numel() == H && res.device() == parts.device() &&
+               w.device() == parts.device(),
+           "parts_norm: shapes");
+  DevGuard g(parts.device());
+  auto y = at::empty({M, H}, res.options()), h = at::empty({M, H}, res.options());
+  MX_OK(mx_parts_norm(parts.data_ptr<float>(), (int)parts.size(0), bf(res), bf(w), bfm(y), bfm(h), (int)M, (int)H, (float)eps,
+                      cur_stream()));
+  return {y, h};
+}
+
 // the QKV projection with RoPE and the cache append in the epilogue, heads of 64 or 128: (q [M, Hq, D], h + delta)
 std::tuple<at::Tensor, at::Tensor> stream_qkv_rope(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
                                                    const c10::optional<at::Tensor>& gamma, double eps,
@@ -439,6 +475,9 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
         "Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, "
         "Tensor? block_table) -> (Tensor, Tensor)");
+  m.def("stream_parts_segments(int M, int N, int K) -> int", &stream_parts_segments);
+  m.def("stream_parts(Tensor x, Tensor w) -> Tensor");
+  m.def("parts_norm(Tensor parts, Tensor res, Tensor w, float eps) -> (Tensor, Tensor)");
   m.def("sample(Tensor logits, float temperature, int seed, int step) -> Tensor");
   m.def("sample_rows(Tensor logits, Tensor temps, Tensor top_p, Tensor top_k, Tensor seeds, Tensor steps) -> Tensor");
   m.def("sample_list(Tensor logits, float[] temps, float[] top_p, int[] top_k, int[] seeds, int[] steps) -> Tensor");
@@ -457,6 +496,8 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn", &decode_attn);
   m.impl("gemm8_rows", &gemm8_rows);
   m.impl("stream_linear", &stream_linear);
+  m.impl("stream_parts", &stream_parts);
+  m.impl("parts_norm", &parts_norm);
   m.impl("stream_qkv_rope", &stream_qkv_rope);
   m.impl("sample", &sample);
   m.impl("sample_rows", &sample_rows);

@@ -32,11 +32,13 @@ __global__ void __launch_bounds__(256) embed_rows_kernel(const int64_t* __restri
 
 // ------------------------------------------------------------------ grouped RMS norm
 // The norm of a row in G equal parts is an RMS norm of G rows: one unit = one (row, part), held in
-// registers by TPU threads (a wave or a workgroup).  h (f32, row stride W) += delta when given.
-template <typename T, int TPU, int VEC>
+// registers by TPU threads (a wave or a workgroup).  h (f32, row stride W) += delta when given, or (PARTS) the sum of
+// `parts`, S of seg elements, rounded to bf16.
+template <typename T, int TPU, int VEC, bool PARTS>
 __global__ void __launch_bounds__(TPU < 256 ? 256 : TPU)
     group_norm_kernel(const T* __restrict__ delta, int64_t ldd, float* __restrict__ h, const float* __restrict__ w,
-                      T* __restrict__ y, int64_t ldy, int64_t units, int groups, int gs, float eps) {
+                      T* __restrict__ y, int64_t ldy, int64_t units, int groups, int gs, float eps,
+                      const float* __restrict__ parts, int S, int64_t seg) {
   constexpr int ITERS = 16 / VEC;
   __shared__ float scratch[16];
   const int64_t unit = TPU < 256 ? (int64_t)blockIdx.x * (256 / TPU) + threadIdx.x / TPU : (int64_t)blockIdx.x;
@@ -58,6 +60,23 @@ __global__ void __launch_bounds__(TPU < 256 ? 256 : TPU)
         ldv<VEC>(dp + c, d);
 #pragma unroll
         for (int j = 0; j < VEC; ++j) v[it][j] += d[j];
+        stv<VEC>(hp + c, v[it]);
+      } else if constexpr (PARTS) {
+        const float* pp = parts + row * (int64_t)groups * gs + g0 + c;
+        float d[VEC];
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) d[j] = 0.f;
+        for (int s0 = 0; s0 < S; s0 += 8) {  // eight loads in flight
+          float q[8][VEC];
+#pragma unroll
+          for (int s = 0; s < 8; ++s) ldv<VEC>(pp + min(s0 + s, S - 1) * seg, q[s]);
+#pragma unroll
+          for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int j = 0; j < VEC; ++j) d[j] += s0 + s < S ? q[s][j] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[it][j] += bf2f(f2bf(d[j]));
         stv<VEC>(hp + c, v[it]);
       }
 #pragma unroll
@@ -458,21 +477,30 @@ extern "C" int mx_embed_rows(const int64_t* ids, const void* w, int f32, float* 
 }
 
 extern "C" int mx_group_norm(const void* delta, int64_t ldd, float* h, const float* w, void* y, int64_t ldy, int f32,
-                             int64_t T, int W, int groups, float eps, hipStream_t stream) {
+                             int64_t T, int W, int groups, float eps, const float* parts, int S, hipStream_t stream) {
   if (T <= 0) return 0;
-  if (groups <= 0 || W % groups) return -1;
+  if (groups <= 0 || W % groups || (parts && (delta || f32 || S < 1))) return -1;
+  const int64_t seg = T * W;
   const int gs = W / groups;
   if (gs > 16384) return -1;
   const int64_t units = T * groups;
   const bool v4 = gs % 4 == 0 && (!delta || ldd % 4 == 0) && ldy % 4 == 0;
 #define GN(TT, TPU, VV)                                                                                      \
-  group_norm_kernel<TT, TPU, VV>                                                                             \
+  group_norm_kernel<TT, TPU, VV, false>                                                                      \
       <<<(unsigned)(TPU == 64 ? (units + 3) / 4 : units), TPU == 64 ? 256 : TPU, 0, stream>>>(               \
-          (const TT*)delta, ldd, h, w, (TT*)y, ldy, units, groups, gs, eps)
+          (const TT*)delta, ldd, h, w, (TT*)y, ldy, units, groups, gs, eps, parts, S, seg)
 #define GNT(TT)                                                                                              \
   if (v4) { if (gs <= 512) GN(TT, 64, 4); else if (gs <= 4096) GN(TT, 256, 4); else GN(TT, 1024, 4); }       \
   else { if (gs <= 1024) GN(TT, 64, 1); else if (gs <= 4096) GN(TT, 256, 1); else GN(TT, 1024, 1); }
-  if (f32) { GNT(float) } else { GNT(uint16_t) }
+#define GNP(TPU)                                                                                             \
+  group_norm_kernel<uint16_t, TPU, 4, true>                                                                  \
+      <<<(unsigned)(TPU == 64 ? (units + 3) / 4 : units), TPU == 64 ? 256 : TPU, 0, stream>>>(               \
+          nullptr, 0, h, w, (uint16_t*)y, ldy, units, groups, gs, eps, parts, S, seg)
+  if (parts) {
+    if (!v4) return -1;
+    if (gs <= 512) GNP(64); else if (gs <= 4096) GNP(256); else GNP(1024);
+  } else if (f32) { GNT(float) } else { GNT(uint16_t) }
+#undef GNP
 #undef GNT
 #undef GN
   return (int)hipGetLastError();

@@ -36,8 +36,9 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
               ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
-               "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk", "sampling", "skinny_gemm",
-               "stream_gemm"),
+               "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk",
+               "sampling", "skinny_gemm",
+               "stream_gemm", "stream_parts"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),
 }
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")

@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from ..ops import hybrid as hops
-from ..ops import linear
+from ..ops import linear, linear_parts
 from ..ops.hybrid import AttnShape, PromptRows, RopeTables
 from .config import PRESETS
 from .llama import FusedLinear, plain_weight
@@ -207,10 +207,17 @@ class Revesun(nn.Module):
                 layer.conv_t()
 
     # ------------------------------------------------------------------ the layer stack
+    def _sub_output(self, lin, x):
+        """Output of a sub-block's last projection; for a few rows of a long K the sums of its segments, which the norm
+        behind it adds (parts of whole vectors)."""
+        w = plain_weight(lin) if self.cfg.hidden // self.cfg.norm_groups % 4 == 0 else None
+        parts = linear_parts(x, w) if w is not None else None
+        return lin(x) if parts is None else parts
+
     def _norm_proj(self, delta, h, gamma, lin, fused: bool = False):
         """(lin(norm(h + delta)), h + delta)."""
         c = self.cfg
-        if fused:
+        if fused and (delta is None or delta.dim() == 2):
             r = hops.norm_linear(delta, h, gamma, c.norm_groups, c.norm_eps, plain_weight(lin))
             if r is not None:
                 return r
@@ -239,7 +246,7 @@ class Revesun(nn.Module):
             r = hops.poly_linear(z, layer.act, self.cfg.norm_eps, plain_weight(layer.wdown))
             if r is not None:
                 return r
-        return layer.wdown(hops.poly_norm(z, layer.act, self.cfg.norm_eps))
+        return self._sub_output(layer.wdown, hops.poly_norm(z, layer.act, self.cfg.norm_eps))
 
     def rows(self, ids: torch.Tensor, rows, tap=None) -> torch.Tensor:
         """Final normed hidden rows of token ``ids`` [T] laid out as ``rows``.  ``tap(i, h)``: the
@@ -249,12 +256,12 @@ class Revesun(nn.Module):
         delta = None  # sub-block output not yet added to h
         for i, layer in enumerate(self.layers):
             y, h = self._mixer(i, delta, h, rows, n)
-            delta = layer.wo(y)
+            delta = self._sub_output(layer.wo, y)
             if layer.spec.ff:
                 z, h = self._norm_proj(delta, h, layer.norm2, layer.wup, rows.decode)
                 delta = self._down(z, layer, rows.decode)
             if tap is not None:
-                tap(i, h + delta.float())
+                tap(i, h + (delta if delta.dim() == 2 else delta.sum(0)).float())
         return hops.group_norm(delta, h, self.final_norm, self.cfg.norm_groups, self.cfg.norm_eps, self.dtype)
 
     @torch.no_grad()

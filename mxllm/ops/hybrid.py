@@ -212,8 +212,11 @@ def embed_rows(ids: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def group_norm(delta: torch.Tensor | None, h: torch.Tensor, w: torch.Tensor, groups: int, eps: float,
                dtype: torch.dtype) -> torch.Tensor:
-    """h (f32, in place) += delta; returns the RMS norm of h in ``groups`` equal parts, times w."""
+    """h (f32, in place) += delta; returns the RMS norm of h in ``groups`` equal parts, times w.  ``delta`` f32 [S, T, W]:
+    the sums of S segments of a projection (``linear_parts``), added and rounded to bf16 first."""
     if use_native(h):
+        if delta is not None and delta.dim() == 3:
+            return native().group_norm_parts(delta, h, w, groups, eps)
         return native().group_norm(delta, h, w, groups, eps, dtype == torch.float32)
     if delta is not None:
         h += delta.float()

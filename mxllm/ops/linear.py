@@ -734,6 +734,33 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w) if y is None else y
 
 
+# Projections in front of a norm whose X is too long for LDS: csrc/kernels/stream_parts.hip, K in segments whose f32 sums the
+# norm adds.  With the norm, us, 9 / 16 / 24 / 32 rows: 4096 x 14336 29.1 / 30.7 / 33.7 / 35.5 -> 25.1 / 26.5 / 30.9 / 31.8; 2048 x
+# 8192 16.0 / 16.1 / 16.8 / 19.0 -> 12.8 / 13.6 / 14.9 / 15.6; 2048 x 12288 22.0 / 21.7 / 21.9 / 26.2 -> 15.3 / 15.6 / 17.2 / 17.4; 8192 x
+# 28672, 9 / 16 rows 97.0 / 98.7 -> 80.8 / 82.7, but 24 101.9 -> 105.2.  A K of 4096 past 16 rows, where it is too long as
+# well: 4096 x 4096, 17 / 32 rows 16.9 / 17.1 -> 14.7 / 16.3, not before (16 rows 13.3 -> 14.2).
+def _parts_wins(M: int, N: int, K: int) -> bool:
+    if not 8 < M <= min(32, _DECODE_M) or K % 512 or N % 64 or N > 8192:
+        return False
+    return (K >= 8192 and (M <= 16 or N * K <= 1 << 27)) if K != 4096 else M > 16 and N <= 4096
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    """Inference, decode rows: f32 ``parts`` [segments of K, M, N] whose sum is ``x w^T``, for :func:`parts_norm` and
+    ``hybrid.group_norm``; None where the sizes go elsewhere."""
+    if not x.is_cuda or x.dim() != 2 or w.dim() != 2:
+        return None
+    (M, K), N = x.shape, w.shape[0]
+    if not _parts_wins(M, N, K) or not _plain(x, w) or not _rows_ok(x, w) or not native().stream_parts_segments(M, N, K):
+        return None
+    return native().stream_parts(x, w)
+
+
+def parts_norm(parts: torch.Tensor, h: torch.Tensor, gamma: torch.Tensor, eps: float):
+    """``add_rms_norm`` of what :func:`linear_parts` returned: (normed, h + the sum rounded to bf16)."""
+    return native().parts_norm(parts, h.contiguous(), gamma, float(eps))
+
+
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
     """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch, with
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,

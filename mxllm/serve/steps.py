@@ -109,20 +109,36 @@ class LlamaSteps:
             return lin.q, lin.scale
         return None, None
 
+    @staticmethod
+    def _in_parts(delta) -> bool:
+        """Whether a sub-block's output came as the sums of segments (``ops.linear_parts``), which a norm adds."""
+        return delta is not None and delta.dim() == 3
+
+    def _sub_output(self, lin, x):
+        """Output of a sub-block's last projection, on its way to a norm."""
+        if self.eng.tp is None and type(lin) is FusedLinear and lin.lora_r == 0:
+            parts = ops.linear_parts(x, lin.weight)
+            if parts is not None:
+                return parts
+        return lin(x)
+
+    def _add_norm(self, delta, h, gamma):
+        """(rmsnorm(h + delta) * gamma, h + delta)"""
+        if delta is None:
+            return ops.rms_norm(h, gamma, self.cfg.norm_eps), h
+        return (ops.parts_norm if self._in_parts(delta) else ops.add_rms_norm)(delta, h, gamma, self.cfg.norm_eps)
+
     def _norm_proj(self, delta, h, gamma, lin, swiglu: bool):
         """(proj(rmsnorm(h + delta) * gamma), h + delta); ``swiglu``: proj = swiglu(lin(.)).
         Decode rows of a plain bf16 or e4m3 projection run as ONE launch (RMSNorm in the GEMM
         prologue, SwiGLU in its epilogue: csrc/kernels/skinny_gemm.hip)."""
         eps = self.cfg.norm_eps
         w, scale = self._stream_weight(lin, h.shape[0])
-        if _NORM_FUSED and w is not None:
+        if _NORM_FUSED and w is not None and not self._in_parts(delta):
             r = ops.norm_linear(delta, h, gamma, eps, w, swiglu, scale)
             if r is not None:
                 return r
-        if delta is None:
-            xn = ops.rms_norm(h, gamma, eps)
-        else:
-            xn, h = ops.add_rms_norm(delta, h, gamma, eps)
+        xn, h = self._add_norm(delta, h, gamma)
         if not swiglu:
             return lin(xn), h
         mid = None
@@ -151,18 +167,15 @@ class LlamaSteps:
             if isinstance(o, tuple):  # split-K partials: merged in the o-projection's prologue
                 a = ops.native().skinny_merge_linear(o[0], o[1], layer.wo.weight)
             else:
-                a = layer.wo(o)
+                a = self._sub_output(layer.wo, o)
             if tp is not None:  # row-parallel Wo: sum the heads' partial outputs
                 tp.all_reduce_(a)
             mid, h = self._norm_proj(a, h, layer.mlp_norm, layer.wgu, True)
-            d = layer.wd(mid)
+            d = self._sub_output(layer.wd, mid)
             if tp is not None:  # row-parallel Wdown
                 tp.all_reduce_(d)
             delta, gamma = d, (m.layers[i + 1].attn_norm if i + 1 < len(m.layers) else m.final_norm)
-        if delta is None:
-            return ops.rms_norm(h, gamma, c.norm_eps)
-        xn, h = ops.add_rms_norm(delta, h, gamma, c.norm_eps)
-        return xn
+        return self._add_norm(delta, h, gamma)[0]
 
     def decode_logits(self, inp: torch.Tensor, max_len: int) -> torch.Tensor:
         """inp int64 [3, B] = (token, position of the new token, cache slot)."""
@@ -217,16 +230,13 @@ class LlamaSteps:
                 return None
             rope = (w, m.rope_cos, m.rope_sin, pos, sl, self.eng.kv.k[i], self.eng.kv.v[i],
                     c.n_heads, c.n_kv_heads, bt, scale)
-            if _NORM_FUSED:
+            if _NORM_FUSED and not self._in_parts(delta):
                 r = ops.qkv_rope_linear(delta, h, gamma, c.norm_eps, *rope)
                 if r is not None:
                     return r
             if not ops.qkv_rope_ok(h, rope[0], rope[1], rope[2], rope[5], rope[6], rope[7], rope[8], False, scale):
                 return None
-            if delta is None:
-                xn = ops.rms_norm(h, gamma, c.norm_eps)
-            else:
-                xn, h = ops.add_rms_norm(delta, h, gamma, c.norm_eps)
+            xn, h = self._add_norm(delta, h, gamma)
             q, _ = ops.qkv_rope_linear(None, xn, None, c.norm_eps, *rope)
             return q, h
 

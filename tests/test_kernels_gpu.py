@@ -993,6 +993,38 @@ def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(16, 1536), (48, 8192), (4112, 3584), (2048, 12288), (4096, 14336), (272, 21504), (8192, 4096)])
+def test_stream_parts(gpu, M, N, K):
+    """Products in segments of K (every length of block; few and uneven channel groups; strided rows): the sum is x w^T to f32
+    (K products of f32 sums: 2^-24 sqrt(K) < 1e-5), and the norms that add it do what they do behind its rounding to
+    bf16, to one rounding of a sum in another order (2^-8)."""
+    torch.manual_seed(N + K + M)
+    x = torch.randn(M, K + 8, device=gpu).bfloat16()[:, :K]
+    w = (torch.randn(N, K, device=gpu) * K ** -0.5).bfloat16()
+    if not _ops().stream_parts_segments(M, N, K):  # no segment fits LDS
+        assert (M, K) == (32, 3584)
+        with pytest.raises(RuntimeError):
+            _ops().stream_parts(x, w)
+        return
+    parts = _ops().stream_parts(x, w)
+    assert parts.shape == (_ops().stream_parts_segments(M, N, K), M, N)
+    want = x.double() @ w.double().t()
+    assert rel_err(parts.double().sum(0), want) < 1e-5
+    h, g = torch.randn(M, N, device=gpu).bfloat16(), torch.randn(N, device=gpu).bfloat16()
+    y, h2 = _ops().parts_norm(parts, h, g, 1e-5)
+    hw = (h.double() + want.bfloat16().double())
+    yw = hw * torch.rsqrt(hw.pow(2).mean(-1, keepdim=True) + 1e-5) * g.double()
+    assert rel_err(h2, hw) < 2 ** -8 and rel_err(y, yw) < 2 ** -7
+    r, gf = torch.randn(M, N, device=gpu), torch.randn(N, device=gpu)
+    r2 = r.double() + want.bfloat16().double()
+    y = _ops().group_norm_parts(parts, r, gf, 4, 1e-5)
+    assert rel_err(r, r2) < 2 ** -8
+    p = r2.view(M, 4, -1)
+    assert rel_err(y, (p * torch.rsqrt(p.pow(2).mean(-1, keepdim=True) + 1e-5)).view(M, N) * gf.double()) < 2 ** -7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Hq,Hkv", [(16, 2), (4, 4), (7, 1), (9, 1)])
 def test_decode_attn_up_to_512_keys(gpu, D, Hq, Hkv):
