@@ -5,6 +5,7 @@
 //   * side_act    : gelu_tanh(z) times the token's row of a second embedding;
 //   * post_dots   : decode rows, the residual step with the products that read the new h next: the router's
 //                   logits, or the second embedding's gate (with its activation);
+//   * post_side   : decode rows, the second embedding's projection with the residual step behind it;
 //   * clipped_glu : min(g, L) sigmoid(1.702 min(g, L)) (clamp(u, -L, L) + 1).
 // Storage type T: bf16 (uint16_t) or float; every reduction and product is f32.
 #include "hybrid.h"
@@ -163,6 +164,63 @@ __global__ void __launch_bounds__(256) post_dots_kernel(PostDots a) {
   }
 }
 
+// decode rows (W <= 4096): h += rms(P g) * w and its copy, P [W, R] the second embedding's projection, g [T, R] its gated
+// rows.  The product and the norm behind it were two launches that wait for each other, 4.7 us each; a workgroup of 16 waves
+// reads P itself (256 KB at W 2048) out of L2.  R / 8 lanes take a row of P, whose products go to LDS rounded as the
+// product's were.
+template <int R>
+__global__ void __launch_bounds__(1024) post_side_kernel(PostNorm a, const uint16_t* __restrict__ gs,
+                                                         const uint16_t* __restrict__ P) {
+  constexpr int LPR = R / 8, RPI = 64 / LPR, U = 16;
+  __shared__ float scratch[16];
+  __shared__ __attribute__((aligned(16))) float ybuf[4096];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, W = a.W, c = min(4 * t, W - 4);
+  const int64_t row = blockIdx.x;
+  const u16x8 gr = *reinterpret_cast<const u16x8*>(gs + row * R + 8 * (lane % LPR));
+  float* hp = a.h + row * W + c;
+  float o[4], w[4], v[4], g[8];
+  ldv<4>(hp, o);
+  ldv<4>(a.w + c, w);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) g[j] = bf2f(gr[j]);
+  const int per = W / 16, n = per / RPI;  // rows of P a wave, loads of RPI of them
+  const int first = wv * per + lane / LPR;
+  const uint16_t* p0 = P + (int64_t)first * R + 8 * (lane % LPR);
+  for (int i0 = 0; i0 < n; i0 += U) {
+    u16x8 m[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) m[u] = *reinterpret_cast<const u16x8*>(p0 + min(i0 + u, n - 1) * (RPI * R));
+    __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += g[j] * bf2f(m[u][j]);
+#define MX_ADD_LANES(CTRL) \
+  s += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(s), CTRL, 0xF, 0xF, true))
+      MX_ADD_LANES(0xB1);                           // lane ^ 1
+      MX_ADD_LANES(0x4E);                           // lane ^ 2
+      if constexpr (LPR >= 8) MX_ADD_LANES(0x141);  // the other quad of eight
+      if constexpr (LPR >= 16) MX_ADD_LANES(0x140); // the other half of sixteen
+#undef MX_ADD_LANES
+      if (i0 + u < n && lane % LPR == 0) ybuf[first + (i0 + u) * RPI] = bf2f(f2bf(s));
+    }
+  }
+  __syncthreads();
+  float ss = 0.f;
+  const bool on = 4 * t < W;
+  ldv<4>(ybuf + c, v);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) ss += on ? v[j] * v[j] : 0.f;
+  ss = block_sum(ss, scratch);
+  if (!on) return;
+  const float rs = 1.f / sqrtf(ss / (float)W + a.eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] += v[j] * rs * w[j];
+  stv<4>(hp, o);
+  stv<4>(reinterpret_cast<uint16_t*>(a.y) + row * W + c, o);
+}
+
 template <typename T, int VEC>
 __global__ void __launch_bounds__(256) side_act_kernel(const T* __restrict__ z, int64_t ldz, const T* __restrict__ emb,
                                                        int64_t lde, const int64_t* __restrict__ ids, int V,
@@ -247,6 +305,21 @@ extern "C" int mx_post_dots(const PostDots* pa, hipStream_t stream) {
     if (a.side) post_dots_kernel<PostNorm::kMix, true><<<g, 256, 0, stream>>>(a);
     else post_dots_kernel<PostNorm::kMix, false><<<g, 256, 0, stream>>>(a);
   }
+  return (int)hipGetLastError();
+}
+
+// bf16 rows g [T, R] and P [W, R], both dense; -1 (nothing launched): sizes it does not take
+extern "C" int mx_post_side(const PostNorm* pa, const uint16_t* g, const uint16_t* P, int R, hipStream_t stream) {
+  const PostNorm& a = *pa;
+  if (a.T <= 0) return 0;
+  if (a.T > 65535 || (R != 32 && R != 64 && R != 128) || a.W <= 0 || a.W > 4096 || a.W % (16 * 512 / R) || !a.h || !a.w || !a.y ||
+      !al16(a.h) || !al16(a.w) || !al16(a.y) || !al16(g) || !al16(P))
+    return -1;
+#define PS(RR) post_side_kernel<RR><<<(unsigned)a.T, 1024, 0, stream>>>(a, g, P)
+  if (R == 32) PS(32);
+  else if (R == 64) PS(64);
+  else PS(128);
+#undef PS
   return (int)hipGetLastError();
 }
 

@@ -373,7 +373,9 @@ class Sigusun(nn.Module):
                 if layer.spec.moe:
                     x = self._mixture(layer, x, h)
                 g = sops.side_act(layer.side_gate(x), self.side_emb, ids, off)
-            x = sops.post_norm(layer.side_proj(g), h, layer.side_norm, eps)
+            x = sops.side_post(g, plain_weight(layer.side_proj), h, layer.side_norm, eps) if rows.decode else None
+            if x is None:
+                x = sops.post_norm(layer.side_proj(g), h, layer.side_norm, eps)
             if tap is not None:
                 tap(i, h.clone())
         return hops.group_norm(None, h, self.final_norm, 1, eps, self.dtype)
