@@ -126,6 +126,17 @@ std::tuple<at::Tensor, at::Tensor> hs_norm_linear(const c10::optional<at::Tensor
   return {y, i.hn};
 }
 
+// the same by the workgroups that stay, up to 4 rows in 8 parts
+std::tuple<at::Tensor, at::Tensor> stream_group_norm(const c10::optional<at::Tensor>& delta, const at::Tensor& h,
+                                                     const at::Tensor& gamma, double eps, const at::Tensor& w) {
+  DevGuard g(w.device());
+  HsIn i = hs_in(h, delta, gamma, w);
+  auto y = at::empty({i.M, w.size(0)}, w.options());
+  MX_OK(mx_stream_group_norm(i.h, i.delta, i.ldd, i.gamma, (float)eps, i.h_out, bf(w), w.stride(0), bfm(y), (int)i.M,
+                             (int)w.size(0), (int)i.K, cur_stream()));
+  return {y, i.hn};
+}
+
 at::Tensor hs_poly_linear(const at::Tensor& z, const at::Tensor& coef, double eps, const at::Tensor& w) {
   DevGuard g(w.device());
   check_f32(coef, "coef");
@@ -408,6 +419,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("mingru_scan(Tensor x, Tensor bias, Tensor chunks, Tensor seqs, bool multi, Tensor(a!)? state=None) -> Tensor");
   m.def("mingru_step(Tensor x, Tensor bias, Tensor slots, Tensor(a!) state) -> Tensor");
   m.def("hs_norm_linear(Tensor? delta, Tensor h, Tensor gamma, int groups, float eps, Tensor w) -> (Tensor, Tensor)");
+  m.def("stream_group_norm(Tensor? delta, Tensor h, Tensor gamma, float eps, Tensor w) -> (Tensor, Tensor)");
   m.def("hs_poly_linear(Tensor z, Tensor coef, float eps, Tensor w) -> Tensor");
   m.def("hs_gru_linear(Tensor? delta, Tensor x, Tensor? gamma, int groups, float eps, Tensor w, Tensor bias, Tensor slots, Tensor(a!) state) -> (Tensor, Tensor)");
   m.def("hs_conv_linear(Tensor? delta, Tensor x, Tensor? gamma, int groups, float eps, Tensor w, Tensor cw, Tensor cos, Tensor sin, int rd, int H, int G, int D, int E, Tensor pos, Tensor slots, int chunk, Tensor(a!) kc, Tensor(b!) vc, Tensor bt, Tensor(c!) ring) -> (Tensor, Tensor, Tensor)");
@@ -426,6 +438,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("mingru_scan", &mingru_scan);
   m.impl("mingru_step", &mingru_step);
   m.impl("hs_norm_linear", &hs_norm_linear);
+  m.impl("stream_group_norm", &stream_group_norm);
   m.impl("hs_poly_linear", &hs_poly_linear);
   m.impl("hs_gru_linear", &hs_gru_linear);
   m.impl("hs_conv_linear", &hs_conv_linear);

@@ -45,6 +45,15 @@ struct StreamArgs {
   SkRope rp;
 };
 
+struct StreamGroups {  // of stream_group_norm_kernel
+  const float* h;
+  const uint16_t* delta;  // or nullptr
+  int64_t ldd;
+  const float* gamma;
+  float* h_out;
+  float eps;
+};
+
 // workgroups of up to 128 registers: two a CU where LDS allows it (X of 9 rows and more of a K over 2048 does not)
 template <int KIND, int TB, int KP, int NL>
 constexpr int kStWaves = KIND >= kStF8 ? (TB == 1 ? 4 : 2) : NL == 8 && (TB == 1 || KP == 4) ? 4 : 2;
@@ -130,9 +139,92 @@ static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
   return stream_blocks<WIDE, 2, EPI, false>(a, stream);
 }
 
+// The same with a grouped RMS norm of an f32 residual (+ delta) in front, up to 4 rows: Y = (rms(h + delta) gamma) . W^T, parts of
+// K / 8 elements, one a wave, so that its sum needs no barrier.  EPT: elements of a row a thread.  Every workgroup does the
+// norm, for all its channels; workgroup 0 stores the sum.  1 / 2 / 4 rows, us: 12288 x 2048 in hybrid_skinny.hip's prologue (every
+// 16 channels) 13.4 / 14.3 / 18.7, norm and product apart 12.5 / 12.9 / 13.3, here 10.5 / 10.9 / 12.2; 21504 x 4096 33.6 / 38.6 /
+// 47.4, 35.3 / 35.0 / 35.4, here 33.0 / 33.3 / 35.0.
+template <int KP, int EPT>
+__global__ void __launch_bounds__(512, 4) stream_group_norm_kernel(StreamArgs a, StreamGroups n) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, c = tid & 15, g = tid >> 4 & 3, M = a.M;
+  constexpr int K = 512 * EPT, Q = EPT / 4;
+  auto row = [&](int grp) __attribute__((always_inline)) -> int64_t { return (int64_t)grp * 16; };
+  auto off = [&](int ch) __attribute__((always_inline)) -> int { return ch; };
+  auto stage = [&](uint16_t* xs, int ldx, auto ahead) __attribute__((always_inline)) {
+    const int cc = tid * EPT;
+    f32x4 h[4][Q], gm[Q];
+    u16x4 d[4][Q];
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      gm[i] = *reinterpret_cast<const f32x4*>(n.gamma + cc + 4 * i);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int mm = min(m, M - 1);
+        h[m][i] = *reinterpret_cast<const f32x4*>(n.h + (int64_t)mm * K + cc + 4 * i);
+        d[m][i] = n.delta ? *reinterpret_cast<const u16x4*>(n.delta + (int64_t)mm * n.ldd + cc + 4 * i) : u16x4{0, 0, 0, 0};
+      }
+    }
+    ahead();
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      if (m >= M) break;
+      float ss = 0.f;
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (n.delta) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) h[m][i][j] += bf2f(d[m][i][j]);
+          if (blockIdx.x == 0) *reinterpret_cast<f32x4*>(n.h_out + (int64_t)m * K + cc + 4 * i) = h[m][i];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss += h[m][i][j] * h[m][i][j];
+      }
+      const float rs = 1.f / sqrtf(wave_sum(ss) / (float)(K / 8) + n.eps);
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        u16x4 o;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = f2bf(h[m][i][j] * rs * gm[i][j]);
+        *reinterpret_cast<u16x4*>(xs + m * ldx + cc + 4 * i) = o;
+      }
+    }
+    lds_barrier();
+  };
+  auto finish = [&](const f32x4& s, int mb, int cg) __attribute__((always_inline)) {
+    const int m = mb * 16 + c;
+    if (m >= M) return;
+    u16x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+    *reinterpret_cast<u16x4*>(a.Y + (int64_t)m * a.ldy + (int64_t)cg * 16 + 4 * g) = o;
+  };
+  stream_walk<kStLines, 1, KP, 8>(a.W, a.ldw, nullptr, M, K, (int)blockIdx.x, (int)gridDim.x, a.groups, smem, row, off, stage,
+                                  finish);
+}
+
 }  // namespace mx
 
 using namespace mx;
+
+// y [M, N] = (grouped rmsnorm of h + delta in 8 parts, times gamma) . w^T, h [M, K] f32 dense, K 2048 or 4096, up to 4 rows;
+// h_out gets h + delta where delta is given.  -1: not taken, nothing launched
+extern "C" int mx_stream_group_norm(const float* h, const uint16_t* delta, int64_t ldd, const float* gamma, float eps,
+                                    float* h_out, const uint16_t* w, int64_t ldw, uint16_t* y, int M, int N, int K,
+                                    hipStream_t stream) {
+  if (M <= 0) return 0;
+  if (M > 4 || (K != 2048 && K != 4096) || N <= 0 || N % 16 || ldw % 8 || ldw < K || ldw * 512 >> 32 ||
+      (delta && (!h_out || ldd % 4 || ldd < K)) ||
+      (((uintptr_t)h | (uintptr_t)gamma | (uintptr_t)h_out | (uintptr_t)w | (uintptr_t)delta | (uintptr_t)y) & 15))
+    return -1;
+  const StreamArgs a{nullptr, 0, w, ldw, nullptr, y, N, M, K, 0, N / 16};
+  const StreamGroups n{h, delta, ldd, gamma, h_out, eps};
+  const unsigned grid = std::min(N / 16, 512);
+  const size_t x = (size_t)M * (K + 8) * 2;  // both below the 64 KB that need no leave
+  if (K == 2048) stream_group_norm_kernel<4, 4><<<grid, 512, kStreamRed<kStLines, 1, 4> + x, stream>>>(a, n);
+  else stream_group_norm_kernel<8, 8><<<grid, 512, kStreamRed<kStLines, 1, 8> + x, stream>>>(a, n);
+  return (int)hipGetLastError();
+}
 
 // Whether mx_stream_gemm takes M rows of K: X and the partial sums in 160 KB of LDS, whole blocks a wave.
 extern "C" int mx_stream_ok(int M, int K, int norm) {

@@ -993,6 +993,28 @@ def test_decode_attn_partials_precision(gpu, D, Hq, Hkv, lens):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 4])
+@pytest.mark.parametrize("N,K", [(16, 2048), (8208, 2048), (12288, 4096)])
+@pytest.mark.parametrize("add", [False, True])
+def test_stream_group_norm(gpu, M, N, K, add):
+    """The grouped norm in the prologue of the GEMM that stays against the norm and the product one after the other: the
+    residual's bits, and the product to two roundings to bf16 (the norm's sum is in another order); parts of unlike size."""
+    torch.manual_seed(N + M)
+    h = torch.randn(M, K, device=gpu) * torch.logspace(-2, 2, 8, device=gpu).repeat_interleave(K // 8)
+    g = torch.randn(K, device=gpu)
+    delta = torch.randn(M, K + 8, device=gpu).bfloat16()[:, :K] if add else None
+    w = (torch.randn(N, K, device=gpu) * K ** -0.5).bfloat16()
+    keep = h.clone()
+    y, h2 = _ops().stream_group_norm(delta, h, g, 1e-3, w)
+    assert torch.equal(h, keep)
+    want_h = h + delta.float() if add else h
+    assert torch.equal(h2, want_h)
+    p = want_h.double().view(M, 8, -1)
+    x = (p * torch.rsqrt(p.pow(2).mean(-1, keepdim=True) + 1e-3)).view(M, K) * g.double()
+    assert rel_err(y, x @ w.double().t()) < 2 ** -7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 9, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 1536), (48, 8192), (4112, 3584), (2048, 12288), (4096, 14336), (272, 21504), (8192, 4096)])
 def test_stream_parts(gpu, M, N, K):
