@@ -177,20 +177,22 @@ def test_up_products_past_rows_in_lds(gpu, T, E, top, K, ff, shared):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("R,W", [(32, 256), (32, 4096), (64, 128), (64, 1920), (64, 2048), (128, 64), (128, 1024)])
+@pytest.mark.parametrize("R,W", [(32, 256), (64, 2048), (64, 4096), (128, 768)])
 @pytest.mark.parametrize("T", [1, 5, 64])
 def test_side_projection_with_its_norm(gpu, T, R, W):
-    """The projection and the residual step in one launch: waves of one load and of several blocks, threads past the
-    row's end; eps that counts."""
+    """The projection and the residual step in one launch, columns that are nearly alike (sums of squares out of large terms
+    that cancel); eps that counts."""
     bf = torch.bfloat16
     g, P, h, w = rnd(T, R, seed=1, dt=bf), (rnd(W, R, seed=2) / R ** 0.5).to(bf), rnd(T, W, seed=3), 1 + 0.3 * rnd(W, seed=4)
+    P[:, 1] = P[:, 0]
+    P[3, 1] += 0.5
+    g[:, 0], g[:, 1] = 30.0, -30.0
     y = (g.double() @ P.double().T).to(bf).double()
     want = h.double() + orc.rms(y, 1e-2) * w.double()
     res = h.clone().to(gpu)
-    x = sops.side_post(g.to(gpu), P.to(gpu), res, w.to(gpu), 1e-2)
+    x = sops.side_post(g.to(gpu), P.to(gpu), sops.side_gram(P.to(gpu)), res, w.to(gpu), 1e-2)
     close(res, want, bf, 0.1)  # a product's f32 sum at a rounding boundary: one step of bf16 of few elements
     assert torch.equal(x, res.to(bf))
-    assert sops.side_post(g.to(gpu), torch.empty(4096, 64, device=gpu, dtype=bf), torch.empty(T, 4096, device=gpu), w, 1e-2) is None
 
 
 @pytest.mark.gpu
