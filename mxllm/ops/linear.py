@@ -603,7 +603,7 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 # Weights from memory in a chain of launches:
 #  * Up to 8 rows (us, skinny -> stream): a K of 4096s, whose blocks are long, from 6144 channels on (6144 x 4096, 1 / 8 rows
 #    12.1 / 14.0 -> 12.0 / 13.0; 28672 39.8 / 42.8 -> 39.4 / 41.1; 4096 x 4096, 8 rows 8.4 -> 9.5), an LM head from 2 rows on
-#    (128256 x 4096), of 2048 past the 5 that skinny has (128256 x 2048, 6 rows hipBLASLt 117.5, stream 86.4).  Else by rows x width, the X that the other reads beside 16 channels of weights: 8192 x 6144, 8 rows
+#    (128256 x 4096).  Else by rows x width, the X that the other reads beside 16 channels of weights: 8192 x 6144, 8 rows
 #    24.4 -> 22.3.
 #  * Past 8 rows (hipBLASLt -> stream): a K of 2048 at any width (2048 x 2048, 12 / 32 rows 11.0 / 11.3 -> 5.6 / 7.7; 16384, 16
 #    rows 17.9 -> 16.3), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 18.0 / 18.1 -> 17.9 / 18.6;
@@ -655,8 +655,6 @@ def _stream_wins(M: int, N: int, K: int, swiglu: bool = False) -> bool:
         return N >= 2048 and (swiglu or M <= 16 or not 12288 < N < 20480)
     if K % 4096 == 0 and N >= _STREAM_N4:
         return M > 1 or N < _STREAM_N2
-    if K == 2048 and M > 5 and N * K > _SKINNY_SMALL_W:
-        return True
     return M * K >= _STREAM_MK and N >= (8192 if K > 2048 else 10240 if swiglu else 20480)
 
 
