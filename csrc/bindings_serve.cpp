@@ -35,7 +35,8 @@ at::Tensor decode_attn(const at::Tensor& q, const at::Tensor& k_cache, const at:
   DevGuard g(q.device());
   // counters: int32 [>= B * Hkv], zero, owned by the caller (a decode engine): the split
   // partials are merged in-launch by the last workgroup of each (seq, kv-head), which
-  // resets its counter -> no combine launch (head_dim 128)
+  // resets its counter -> no combine launch (head_dim 128; not of up to 512 keys, which take one launch anyway, nor
+  // where the keys are dealt evenly)
   unsigned int* cnt = nullptr;
   if (counters.has_value() && D == 128) {
     MX_CHECK(counters->scalar_type() == at::kInt && counters->is_contiguous() && counters->numel() >= B * Hkv &&
