@@ -62,7 +62,8 @@ def post_dots(src: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float, m
 
 def side_gram(p: torch.Tensor) -> torch.Tensor:
     """``p^T p`` in f32, which :func:`side_post` has the sum of squares of a row ``p g`` from."""
-    return (p.double().t() @ p.double()).float().contiguous()
+    p = p.float()
+    return p.t() @ p
 
 
 def side_post(g: torch.Tensor, p: torch.Tensor | None, gram: torch.Tensor | None, h: torch.Tensor, w: torch.Tensor,
