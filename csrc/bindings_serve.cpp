@@ -47,9 +47,9 @@ at::Tensor decode_attn(const at::Tensor& q, const at::Tensor& k_cache, const at:
   const KvPages pg = kv_pages(block_table, k_cache);
   const int64_t cap = pg.bt ? (int64_t)pg.maxb * max_seq : max_seq;  // positions a sequence can hold
   const int64_t nsplit = std::max<int64_t>(1, (std::min(max_len, cap) + 255) / 256);
-  // parts a row: one per 256 keys, and at most 2 nsplit + 1 where the keys are dealt evenly (decode.hip)
-  auto ml = at::empty({B, Hq, 2 * nsplit + 1, 2}, q.options().dtype(at::kFloat));
-  auto po = at::empty({B, Hq, 2 * nsplit + 1, D}, q.options().dtype(at::kFloat));
+  const int64_t nparts = mx_decode_attn_parts((int)Hkv, (int)nsplit);
+  auto ml = at::empty({B, Hq, nparts, 2}, q.options().dtype(at::kFloat));
+  auto po = at::empty({B, Hq, nparts, D}, q.options().dtype(at::kFloat));
   auto out = at::empty({B, Hq * D}, q.options());
   const int32_t* sl = nullptr;
   if (slots.has_value()) sl = slots->data_ptr<int32_t>();

@@ -912,6 +912,14 @@ extern "C" int mx_rope_append(const uint16_t* qkv, const float* cosb, const floa
   return (int)hipGetLastError();
 }
 
+// workgroups of a KV head, and the most parts of a row, where the keys are dealt evenly: a row of n units touches at most
+// (n + share - 2) / share + 1 shares of 8 units or more, and no more than there are
+static int even_groups(int Hkv) { return std::max(1, kEvenPlaces / std::max(1, Hkv)); }
+static int even_parts(int Hkv, int nsplit) { return std::min(2 * nsplit + 1, even_groups(Hkv)); }
+
+// parts a row that the buffers of mx_decode_attn have room for
+extern "C" int mx_decode_attn_parts(int Hkv, int nsplit) { return std::max(nsplit, even_parts(Hkv, nsplit)); }
+
 extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint16_t* vc, const int32_t* lens,
                               int len_off, const int32_t* slots, float* part_ml, float* part_o, uint16_t* out, int B,
                               int Hq, int Hkv, int D, int max_seq, int nsplit, float scale, const int32_t* bt,
@@ -936,10 +944,9 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
     return (int)hipGetLastError();
   }
   // Heads of 128, more splits than places: dealt evenly.  What the caller's `nsplit` counts is the longest that the step
-  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.  The buffers have
-  // 2 nsplit + 1 parts a row (a row of n units touches at most (n + share - 2) / share + 1 shares of 8 units or more).
+  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.
   if (out && D == kEvenD && (int64_t)nsplit * Hkv * B > kEvenPlaces) {
-    const int W = std::max(1, kEvenPlaces / Hkv), cap = nsplit * kSplit, nparts = 2 * nsplit + 1;
+    const int W = even_groups(Hkv), cap = nsplit * kSplit, nparts = even_parts(Hkv, nsplit);
     decode_even_kernel<<<dim3(W, Hkv), 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, out, B, Hq, Hkv,
                                                          max_seq, cap, nparts, sl, bt, maxb);
     decode_even_merge_kernel<<<B * Hq, kEvenD, 0, stream>>>(part_ml, part_o, lens, len_off, out, B, Hq, W, cap, nparts);
