@@ -6,7 +6,7 @@
 
 extern "C" {
 int mx_post_norm(const mx::PostNorm* a, int f32, hipStream_t stream);
-int mx_post_side(const mx::PostNorm* a, const uint16_t* g, const uint16_t* P, const float* gram, int R, hipStream_t stream);
+int mx_post_side(const mx::PostNorm* a, const uint16_t* g, const uint16_t* P, int R, hipStream_t stream);
 int mx_side_act(const void* z, int64_t ldz, const void* emb, int64_t lde, const int64_t* ids, int V, void* y, int f32,
                 int64_t T, int dim, hipStream_t stream);
 int mx_clipped_glu(const void* z, int64_t ldz, void* y, int f32, int64_t T, int F, float limit, hipStream_t stream);
@@ -95,19 +95,16 @@ at::Tensor post_norm(const at::Tensor& src, at::Tensor h, const at::Tensor& w, d
   a.src = src.data_ptr();
   return pn_run(a, h, f);
 }
-// bf16 decode rows: h += rms(P g) * w, the copy of h returned; g [T, R], P [W, R], gram = P^T P f32
-at::Tensor post_side(const at::Tensor& gs, const at::Tensor& P, const at::Tensor& gram, at::Tensor h, const at::Tensor& w, double eps) {
+// bf16 decode rows: h += rms(P g) * w, the copy of h returned; g [T, R], P [W, R]
+at::Tensor post_side(const at::Tensor& gs, const at::Tensor& P, at::Tensor h, const at::Tensor& w, double eps) {
   DevGuard g(h.device());
   mx::PostNorm a = pn_args(h, w, eps);
   MX_CHECK(!is_f32(gs, "g") && !is_f32(P, "P") && gs.dim() == 2 && P.dim() == 2 && gs.is_contiguous() && P.is_contiguous() &&
                gs.size(0) == a.T && P.size(0) == a.W && gs.size(1) == P.size(1),
            "post_side: g [T, R], P [W, R] bf16");
-  check_f32(gram, "gram");
-  MX_CHECK(gram.dim() == 2 && gram.size(0) == P.size(1) && gram.size(1) == P.size(1), "post_side: gram [R, R]");
   auto y = at::empty({a.T, (int64_t)a.W}, h.options().dtype(at::kBFloat16));
   a.y = y.data_ptr();
-  MX_OK(mx_post_side(&a, (const uint16_t*)gs.data_ptr(), (const uint16_t*)P.data_ptr(), gram.data_ptr<float>(),
-                     (int)P.size(1), cur_stream()));
+  MX_OK(mx_post_side(&a, (const uint16_t*)gs.data_ptr(), (const uint16_t*)P.data_ptr(), (int)P.size(1), cur_stream()));
   return y;
 }
 // bf16 decode rows: (new h, its bf16 copy, its dot products with the rows of m) - src a sublayer's rows, or with
@@ -533,7 +530,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> moe_few(
 TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("post_norm(Tensor src, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("embed_norm(Tensor ids, Tensor table, Tensor w, float eps) -> (Tensor, Tensor)");
-  m.def("post_side(Tensor g, Tensor P, Tensor gram, Tensor(a!) h, Tensor w, float eps) -> Tensor");
+  m.def("post_side(Tensor g, Tensor P, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("mix_post_norm(Tensor src, Tensor? inv, Tensor wts, Tensor? shared, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("side_act(Tensor z, Tensor emb, Tensor ids, int off) -> Tensor");
   m.def("clipped_glu(Tensor z, float limit) -> Tensor");

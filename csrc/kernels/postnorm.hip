@@ -165,59 +165,63 @@ __global__ void __launch_bounds__(256) post_dots_kernel(PostDots a) {
   }
 }
 
-// decode rows: h += rms(P g) * w and its copy, P [W, R] the second embedding's projection, g [T, R] its gated rows.  The
-// product and the norm behind it were two launches that wait for each other, 4.7 us each.  A workgroup takes 256 channels of a
-// row; the row's sum of squares, |P g|^2 = g^T (P^T P) g, it has from the small matrix gram [R, R] (f32, laid out once), in
-// f32.  (One workgroup a row, which reads all of P: 8.5 us, 256 KB from memory by one CU.)  R / 8 lanes take a row of P.
-constexpr int kSideCols = 256;
+// decode rows (W <= 4096): h += rms(P g) * w and its copy, P [W, R] the second embedding's projection, g [T, R] its gated
+// rows.  The product and the norm behind it were two launches that wait for each other, 4.7 us each; a workgroup of 16 waves
+// reads P itself (256 KB at W 2048, 8.5 us).  R / 8 lanes take a row of P, whose products go to LDS rounded as the product's
+// were.  The row's sum of squares is that of these products: as g^T (P^T P) g out of a matrix laid out before, several workgroups
+// could share a row (65 us less in a step of 32 sequences, 1B size), but terms cancel (two columns alike to 1 in 256: the norm
+// off by 2 to 4 %), and weights written later would meet the norm of the old ones.
 template <int R>
-__global__ void __launch_bounds__(256) post_side_kernel(PostNorm a, const uint16_t* __restrict__ gs,
-                                                        const uint16_t* __restrict__ P, const float* __restrict__ gram) {
-  constexpr int LPR = R / 8, RPI = 64 / LPR, U = 64 / RPI, GE = R * R / 256;  // loads of a wave's 64 channels; gram a thread
+__global__ void __launch_bounds__(1024) post_side_kernel(PostNorm a, const uint16_t* __restrict__ gs,
+                                                         const uint16_t* __restrict__ P) {
+  constexpr int LPR = R / 8, RPI = 64 / LPR, U = 16;
   __shared__ float scratch[16];
-  __shared__ float gf[R], ybuf[kSideCols];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, W = a.W;
-  const int64_t row = blockIdx.y, c = (int64_t)blockIdx.x * kSideCols + t;
+  __shared__ __attribute__((aligned(16))) float ybuf[4096];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, W = a.W, c = min(4 * t, W - 4);
+  const int64_t row = blockIdx.x;
   const u16x8 gr = *reinterpret_cast<const u16x8*>(gs + row * R + 8 * (lane % LPR));
-  const int first = 64 * wv + lane / LPR;
-  const uint16_t* p0 = P + ((int64_t)blockIdx.x * kSideCols + first) * R + 8 * (lane % LPR);
-  u16x8 m[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) m[u] = *reinterpret_cast<const u16x8*>(p0 + u * (RPI * R));
-  f32x4 q[GE / 4];
-#pragma unroll
-  for (int i = 0; i < GE / 4; ++i) q[i] = *reinterpret_cast<const f32x4*>(gram + t * GE + 4 * i);
   float* hp = a.h + row * W + c;
-  const float h = *hp, w = a.w[c];
-  __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
-  if (t < R) gf[t] = bf2f(gs[row * R + t]);
-  float g[8];
+  float o[4], w[4], v[4], g[8];
+  ldv<4>(hp, o);
+  ldv<4>(a.w + c, w);
 #pragma unroll
   for (int j = 0; j < 8; ++j) g[j] = bf2f(gr[j]);
+  const int per = W / 16, n = per / RPI;  // rows of P a wave, loads of RPI of them
+  const int first = wv * per + lane / LPR;
+  const uint16_t* p0 = P + (int64_t)first * R + 8 * (lane % LPR);
+  for (int i0 = 0; i0 < n; i0 += U) {
+    u16x8 m[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    float s = 0.f;
+    for (int u = 0; u < U; ++u) m[u] = *reinterpret_cast<const u16x8*>(p0 + min(i0 + u, n - 1) * (RPI * R));
+    __builtin_amdgcn_sched_barrier(0);  // every load is in flight before the first product waits
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += g[j] * bf2f(m[u][j]);
+    for (int u = 0; u < U; ++u) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) s += g[j] * bf2f(m[u][j]);
 #define MX_ADD_LANES(CTRL) \
   s += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(s), CTRL, 0xF, 0xF, true))
-    MX_ADD_LANES(0xB1);                            // lane ^ 1
-    MX_ADD_LANES(0x4E);                            // lane ^ 2
-    if constexpr (LPR >= 8) MX_ADD_LANES(0x141);   // the other quad of eight
-    if constexpr (LPR >= 16) MX_ADD_LANES(0x140);  // the other half of sixteen
+      MX_ADD_LANES(0xB1);                           // lane ^ 1
+      MX_ADD_LANES(0x4E);                           // lane ^ 2
+      if constexpr (LPR >= 8) MX_ADD_LANES(0x141);  // the other quad of eight
+      if constexpr (LPR >= 16) MX_ADD_LANES(0x140); // the other half of sixteen
 #undef MX_ADD_LANES
-    if (lane % LPR == 0) ybuf[first + u * RPI] = bf2f(f2bf(s));
+      if (i0 + u < n && lane % LPR == 0) ybuf[first + (i0 + u) * RPI] = bf2f(f2bf(s));
+    }
   }
   __syncthreads();
-  const int at = t * GE;  // the thread's elements lie in one row of gram: GE divides R
   float ss = 0.f;
+  const bool on = 4 * t < W;
+  ldv<4>(ybuf + c, v);
 #pragma unroll
-  for (int i = 0; i < GE; ++i) ss += q[i / 4][i % 4] * gf[at % R + i];
-  ss = block_sum(ss * gf[at / R], scratch);
-  const float rs = 1.f / sqrtf(fmaxf(ss, 0.f) / (float)W + a.eps);
-  const float o = h + ybuf[t] * rs * w;
-  *hp = o;
-  reinterpret_cast<uint16_t*>(a.y)[row * W + c] = f2bf(o);
+  for (int j = 0; j < 4; ++j) ss += on ? v[j] * v[j] : 0.f;
+  ss = block_sum(ss, scratch);
+  if (!on) return;
+  const float rs = 1.f / sqrtf(ss / (float)W + a.eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) o[j] += v[j] * rs * w[j];
+  stv<4>(hp, o);
+  stv<4>(reinterpret_cast<uint16_t*>(a.y) + row * W + c, o);
 }
 
 template <typename T, int VEC>
@@ -307,15 +311,14 @@ extern "C" int mx_post_dots(const PostDots* pa, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-// bf16 rows g [T, R] and P [W, R], gram [R, R] f32, all dense; -1 (nothing launched): sizes it does not take
-extern "C" int mx_post_side(const PostNorm* pa, const uint16_t* g, const uint16_t* P, const float* gram, int R, hipStream_t stream) {
+// bf16 rows g [T, R] and P [W, R], both dense; -1 (nothing launched): sizes it does not take
+extern "C" int mx_post_side(const PostNorm* pa, const uint16_t* g, const uint16_t* P, int R, hipStream_t stream) {
   const PostNorm& a = *pa;
   if (a.T <= 0) return 0;
-  if (a.T > 65535 || (R != 32 && R != 64 && R != 128) || a.W <= 0 || a.W % kSideCols || !a.h || !a.w || !a.y || !al16(g) ||
-      !al16(P) || !al16(gram))
+  if (a.T > 65535 || (R != 32 && R != 64 && R != 128) || a.W <= 0 || a.W > 4096 || a.W % (16 * 512 / R) || !a.h || !a.w || !a.y ||
+      !al16(a.h) || !al16(a.w) || !al16(a.y) || !al16(g) || !al16(P))
     return -1;
-  const dim3 grid(a.W / kSideCols, (unsigned)a.T);
-#define PS(RR) post_side_kernel<RR><<<grid, 256, 0, stream>>>(a, g, P, gram)
+#define PS(RR) post_side_kernel<RR><<<(unsigned)a.T, 1024, 0, stream>>>(a, g, P)
   if (R == 32) PS(32);
   else if (R == 64) PS(64);
   else PS(128);

@@ -230,7 +230,6 @@ class SigusunLayer(nn.Module):
         self.side_gate = FusedLinear(h, [side], **kw)
         self.side_proj = FusedLinear(side, [h], **kw)
         self.side_norm = f32(h, value=1.0)
-        self.side_gram = None  # side_gram(side_proj), Sigusun.prepare
 
 
 class Sigusun(nn.Module):
@@ -293,14 +292,11 @@ class Sigusun(nn.Module):
 
     def prepare(self, max_seq: int) -> None:
         """Build what decoding derives once (its storage must not move under a captured graph): rotation tables,
-        and in bf16 the key weights transposed and the products of the side projection's columns."""
+        and in bf16 the key weights transposed."""
         for s, layer in zip(self.cfg.layers, self.layers):
             self.tables.get(*s.rot, max_seq)
             if s.lat and layer.wuk_t is None and layer.wkv.is_cuda and self.dtype == torch.bfloat16:
                 layer.wuk_t = lops.key_weight(layer.wkv.data, s.lat)
-            side = plain_weight(layer.side_proj)
-            if layer.side_gram is None and side is not None and side.is_cuda and self.dtype == torch.bfloat16:
-                layer.side_gram = sops.side_gram(side.data)
 
     # ------------------------------------------------------------------ the layer stack
     def _mixer(self, i: int, x: torch.Tensor, rows, n: int, latents: dict) -> torch.Tensor:
@@ -377,9 +373,7 @@ class Sigusun(nn.Module):
                 if layer.spec.moe:
                     x = self._mixture(layer, x, h)
                 g = sops.side_act(layer.side_gate(x), self.side_emb, ids, off)
-            x = None
-            if rows.decode:
-                x = sops.side_post(g, plain_weight(layer.side_proj), layer.side_gram, h, layer.side_norm, eps)
+            x = sops.side_post(g, plain_weight(layer.side_proj), h, layer.side_norm, eps) if rows.decode else None
             if x is None:
                 x = sops.post_norm(layer.side_proj(g), h, layer.side_norm, eps)
             if tap is not None:

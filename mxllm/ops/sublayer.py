@@ -60,21 +60,17 @@ def post_dots(src: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float, m
     return native().post_dots(src, h, w, eps, m, wts, shared, emb, ids, off)
 
 
-def side_gram(p: torch.Tensor) -> torch.Tensor:
-    """``p^T p`` in f32, which :func:`side_post` has the sum of squares of a row ``p g`` from."""
-    p = p.float()
-    return p.t() @ p
-
-
-def side_post(g: torch.Tensor, p: torch.Tensor | None, gram: torch.Tensor | None, h: torch.Tensor, w: torch.Tensor,
-              eps: float) -> torch.Tensor | None:
-    """Decode rows, one launch: ``post_norm(g p^T, h, w, eps)`` of the few columns of a second embedding, ``gram``
-    :func:`side_gram` of ``p``; None: sizes or types that it does not take."""
-    if not (p is not None and gram is not None and FUSED and use_native(g) and g.dtype == p.dtype == torch.bfloat16
-            and g.shape[0] <= DECODE_ROWS and g.shape[1] in (32, 64, 128) and h.shape[1] % 256 == 0 and g.is_contiguous()
+def side_post(g: torch.Tensor, p: torch.Tensor | None, h: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor | None:
+    """Decode rows, one launch: ``post_norm(g p^T, h, w, eps)`` of the few columns of a second embedding; None: sizes
+    or types that it does not take.  A workgroup a row reads all of ``p``: 256 KB are worth the launch (steps of the 1B size, 8 / 16 /
+    32 sequences 1242 / 1333 / 1572 -> 1216 / 1314 / 1556 us, 1 to 4 as before), 512 KB are not (8B, 1 / 8 sequences 3386 / 4549 ->
+    3458 / 4608)."""
+    W = h.shape[1]
+    if not (p is not None and p.numel() <= 1 << 17 and FUSED and use_native(g) and g.dtype == p.dtype == torch.bfloat16 and g.shape[0] <= DECODE_ROWS
+            and g.shape[1] in (32, 64, 128) and W <= 4096 and W % (16 * 512 // g.shape[1]) == 0 and g.is_contiguous()
             and p.is_contiguous() and p.data_ptr() % 16 == 0):
         return None
-    return native().post_side(g, p, gram, h, w, eps)
+    return native().post_side(g, p, h, w, eps)
 
 
 def mix_post_norm(src: torch.Tensor, inv: torch.Tensor | None, wts: torch.Tensor, shared: torch.Tensor | None,

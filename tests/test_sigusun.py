@@ -177,11 +177,11 @@ def test_up_products_past_rows_in_lds(gpu, T, E, top, K, ff, shared):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("R,W", [(32, 256), (64, 2048), (64, 4096), (128, 768)])
+@pytest.mark.parametrize("R,W", [(32, 256), (32, 4096), (64, 128), (64, 1920), (64, 2048), (128, 64), (128, 768), (128, 1024)])
 @pytest.mark.parametrize("T", [1, 5, 64])
 def test_side_projection_with_its_norm(gpu, T, R, W):
-    """The projection and the residual step in one launch, columns that are nearly alike (sums of squares out of large terms
-    that cancel); eps that counts."""
+    """The projection and the residual step in one launch: waves of one load and of several blocks, threads past the row's
+    end; columns that are nearly alike (products out of large terms that cancel); eps that counts."""
     bf = torch.bfloat16
     g, P, h, w = rnd(T, R, seed=1, dt=bf), (rnd(W, R, seed=2) / R ** 0.5).to(bf), rnd(T, W, seed=3), 1 + 0.3 * rnd(W, seed=4)
     P[:, 1] = P[:, 0]
@@ -190,9 +190,30 @@ def test_side_projection_with_its_norm(gpu, T, R, W):
     y = (g.double() @ P.double().T).to(bf).double()
     want = h.double() + orc.rms(y, 1e-2) * w.double()
     res = h.clone().to(gpu)
-    x = sops.side_post(g.to(gpu), P.to(gpu), sops.side_gram(P.to(gpu)), res, w.to(gpu), 1e-2)
+    x = sops.side_post(g.to(gpu), P.to(gpu), res, w.to(gpu), 1e-2)
     close(res, want, bf, 0.1)  # a product's f32 sum at a rounding boundary: one step of bf16 of few elements
     assert torch.equal(x, res.to(bf))
+    big = torch.empty(4096, 64, device=gpu, dtype=bf)
+    assert sops.side_post(g.to(gpu), big, torch.empty(T, 4096, device=gpu), w, 1e-2) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [512, 2048])
+def test_side_projection_of_columns_nearly_dependent(gpu, W):
+    """Two large columns that differ in their last bits: the terms' squares are about 1e5 times the row's sum of squares, which
+    has to come from the products.  A product sums terms of up to 2048 x 0.5 in f32, at most 2^10 x 2^-23 off beside elements
+    of about 1: the sum of squares to 1e-3 at the worst, the step to half of that and its bf16 rounding."""
+    bf, T, R = torch.bfloat16, 5, 64
+    g, P, h, w = rnd(T, R, seed=1, dt=bf), (rnd(W, R, seed=2) / R ** 0.5).to(bf), torch.zeros(T, W), torch.ones(W)
+    P[:, 1] = (P[:, 0].float() * (1 + rnd(W, seed=5) / 256)).to(bf)
+    g[:, 0], g[:, 1] = 2048.0, -2048.0
+    y = g.double() @ P.double().T
+    assert 2e4 < float((2 * (2048 * P[:, 0].double()).pow(2).sum() / y.pow(2).sum(1)).min()) < 4e5
+    res = h.to(gpu)
+    sops.side_post(g.to(gpu), P.to(gpu), res, w.to(gpu), 1e-5)
+    got, want = res.double().cpu(), orc.rms(y, 1e-5)
+    assert float((got * want).sum() / want.pow(2).sum() - 1) == pytest.approx(0, abs=1e-3)
+    close(got, want, bf, 0.2)
 
 
 @pytest.mark.gpu
@@ -598,6 +619,9 @@ CONFIGS = {
         R(2, 64, 64, 64, 1e4, (0.98, 0.999), M(4, 2, 128, 2.0)),
         A(4, 32, 32, 48, 96, 1e4, 0.15, window=70, mlp=M(8, 4, 64, 2.0, 64)),
         A(2, 64, 32, 32, 96, 1e4, 0.13, window=33, kv_from=2, mlp=M(4, 1, 192, 2.0, 64))]),
+    # a second embedding wide enough for its projection's decode kernel
+    "side": orc.config(256, 128, 32, [A(4, 64, 32, 64, 128, 1e4, 0.12, sink=True, mlp=M(8, 2, 64, 3.0, 128)),
+                                      R(2, 64, 64, 64, 1e4, (0.98, 0.999), M(4, 2, 128, 2.0))]),
 }
 
 
@@ -864,6 +888,37 @@ def test_graphed_decode_equals_eager(built, gpu, batch):
         outs.append(torch.stack(got))
     rel = (outs[0] - outs[1]).pow(2).mean(-1).sqrt() / outs[1].pow(2).mean().sqrt()
     assert float(rel.median()) < 1.5e-2, float(rel.median())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [False, True])
+def test_decode_follows_a_side_projection_written_in_place(built, gpu, graphs):
+    """New values of ``side_proj`` in the storage that decode steps read: the next steps are those of a model that had them from
+    the start (the same kernels on the same values: the same bits)."""
+    prompts, feed = [tokens(9, 128, 1), tokens(40, 128, 2)], [[5, 6], [7, 8], [9, 1], [2, 3]]
+
+    def write(model):
+        for i, layer in enumerate(model.layers):
+            layer.side_proj.weight.mul_(3.0).add_(rnd(*layer.side_proj.weight.shape, seed=i, dt=torch.bfloat16).to(gpu), alpha=0.1)
+
+    def steps(model, late):
+        if not late:
+            write(model)
+        eng = Engine(model, max_batch=2, max_seq=128, use_graphs=graphs, kv_pool_tokens=512)
+        slots = [eng.acquire() for _ in prompts]
+        for s, p in zip(slots, prompts):
+            eng.extend(s, len(p) + 8)
+        eng.prefill_batch(slots, prompts)
+        if late:  # steps with the old values (and a graph of them), then the prompt again
+            for t in feed:
+                eng.decode(slots, torch.tensor(t))
+            write(model)
+            eng.prefill_batch(slots, prompts)
+        return torch.stack([eng.decode(slots, torch.tensor(t)).float().clone() for t in feed])
+
+    want, got = (steps(built("side", gpu, torch.bfloat16)[2], late) for late in (False, True))
+    rel = float((got - want).pow(2).mean().sqrt() / want.pow(2).mean().sqrt())
+    assert rel < 1e-6, rel
 
 
 @pytest.mark.gpu
