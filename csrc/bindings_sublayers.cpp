@@ -100,8 +100,9 @@ at::Tensor post_side(const at::Tensor& gs, const at::Tensor& P, at::Tensor h, co
   DevGuard g(h.device());
   mx::PostNorm a = pn_args(h, w, eps);
   MX_CHECK(!is_f32(gs, "g") && !is_f32(P, "P") && gs.dim() == 2 && P.dim() == 2 && gs.is_contiguous() && P.is_contiguous() &&
-               gs.size(0) == a.T && P.size(0) == a.W && gs.size(1) == P.size(1),
-           "post_side: g [T, R], P [W, R] bf16");
+               gs.size(0) == a.T && P.size(0) == a.W && gs.size(1) == P.size(1) && gs.device() == h.device() &&
+               P.device() == h.device() && w.device() == h.device(),
+           "post_side: g [T, R], P [W, R] bf16, all on one device");
   auto y = at::empty({a.T, (int64_t)a.W}, h.options().dtype(at::kBFloat16));
   a.y = y.data_ptr();
   MX_OK(mx_post_side(&a, (const uint16_t*)gs.data_ptr(), (const uint16_t*)P.data_ptr(), (int)P.size(1), cur_stream()));

@@ -66,9 +66,9 @@ def side_post(g: torch.Tensor, p: torch.Tensor | None, h: torch.Tensor, w: torch
     32 sequences 1242 / 1333 / 1572 -> 1216 / 1314 / 1556 us, 1 to 4 as before), 512 KB are not (8B, 1 / 8 sequences 3386 / 4549 ->
     3458 / 4608)."""
     W = h.shape[1]
-    if not (p is not None and p.numel() <= 1 << 17 and FUSED and use_native(g) and g.dtype == p.dtype == torch.bfloat16 and g.shape[0] <= DECODE_ROWS
-            and g.shape[1] in (32, 64, 128) and W <= 4096 and W % (16 * 512 // g.shape[1]) == 0 and g.is_contiguous()
-            and p.is_contiguous() and p.data_ptr() % 16 == 0):
+    if not (p is not None and p.numel() <= 1 << 17 and FUSED and use_native(g) and g.dtype == p.dtype == torch.bfloat16
+            and g.shape[0] <= DECODE_ROWS and g.shape[1] in (32, 64, 128) and W <= 4096 and W % (16 * 512 // g.shape[1]) == 0
+            and g.is_contiguous() and p.is_contiguous() and all(t.data_ptr() % 16 == 0 for t in (g, p, h, w))):
         return None
     return native().post_side(g, p, h, w, eps)
 

@@ -198,6 +198,31 @@ def test_side_projection_with_its_norm(gpu, T, R, W):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("odd", ["g", "p", "h", "w"])
+def test_side_projection_leaves_operands_that_are_not_aligned(gpu, odd):
+    """A tensor whose storage starts between two 16-byte pieces goes to the parts instead of an error."""
+    T, R, W, bf = 3, 64, 256, torch.bfloat16
+    t = dict(g=rnd(T, R, seed=1, dt=bf), p=rnd(W, R, seed=2, dt=bf), h=rnd(T, W, seed=3), w=rnd(W, seed=4))
+    at = {}
+    for k, v in t.items():
+        room = torch.empty(v.numel() + 8, device=gpu, dtype=v.dtype)
+        at[k] = room[1 if k == odd else 0:][:v.numel()].view(v.shape)
+        at[k].copy_(v)
+    assert sops.side_post(at["g"], at["p"], at["h"], at["w"], 1e-3) is None
+    assert torch.equal(at["h"].cpu(), t["h"])
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two GPUs")
+def test_side_projection_refuses_another_device(gpu):
+    t = [torch.zeros(3, 64, device=gpu, dtype=torch.bfloat16), torch.zeros(256, 64, device=gpu, dtype=torch.bfloat16),
+         torch.zeros(3, 256, device=gpu), torch.zeros(256, device=gpu)]
+    for i in (0, 1, 3):
+        with pytest.raises(RuntimeError):
+            native().post_side(*(x.to("cuda:1") if j == i else x for j, x in enumerate(t)), 1e-3)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W", [512, 2048])
 def test_side_projection_of_columns_nearly_dependent(gpu, W):
     """Two large columns that differ in their last bits: the terms' squares are about 1e5 times the row's sum of squares, which
