@@ -140,8 +140,7 @@ __global__ void __launch_bounds__(256) post_dots_kernel(PostDots a) {
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        // a close choice of experts follows the residual itself, not its rounding (which is most of the logits' error)
-        const float x = SIDE ? bf2f(f2bf(o[it][j])) : o[it][j];
+        const float x = bf2f(f2bf(o[it][j]));
 #pragma unroll
         for (int r = 0; r < kDotRows; ++r) s[r] += x * bf2f(m[r][it][j]);
       }

@@ -127,6 +127,11 @@ def test_residual_step_with_its_next_products(gpu, T, width, rows, top):
     close(y, y2, torch.float32, 200)
     want = y2.double().cpu() @ m.double().cpu().T
     close(z, want, torch.float32, 100)
+    # of the copy, which prompt passes and the separate kernels route by, and not of the residual: f32 sums of up to 4096 products
+    # (2^-24 sqrt(4096) = 4e-6), where the residual's would be a rounding to bf16 apart (2^-9 = 2e-3)
+    zy, m2 = y.double().cpu() @ m.double().cpu().T, m.double().cpu().T
+    assert float((z.double().cpu() - zy).norm() / zy.norm()) < 2e-5
+    assert float((hn.double().cpu() @ m2 - zy).norm() / zy.norm()) > 2e-4
     hn, _, g = sops.post_dots(src, h, w, 1e-4, m, wts, sh, emb, ids, rows)
     close(hn, h2, torch.float32)
     close(g, orc.gelu_tanh(want) * emb.double().cpu()[ids.cpu(), rows:2 * rows], bf)
