@@ -1015,6 +1015,31 @@ def test_stream_group_norm(gpu, M, N, K, add):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 4, 5, 8])
+@pytest.mark.parametrize("K", [2048, 4096])
+@pytest.mark.parametrize("limit", [None, 3, 8])
+def test_group_norm_prologue_by_the_rows_asked_for(gpu, monkeypatch, M, K, limit):
+    """MXLLM_NORM_FUSED_M past what the GEMM that stays takes (4 rows): the other prologue or the parts, never an error."""
+    from mxllm.ops import hybrid as hops
+
+    if limit is not None:
+        monkeypatch.setattr(hops, "NORM_M", limit)
+        monkeypatch.setattr(hops, "_NORM_STREAM_M", limit)
+    torch.manual_seed(M)
+    h, delta, g = torch.randn(M, K, device=gpu), torch.randn(M, K, device=gpu).bfloat16(), torch.rand(K, device=gpu) + 0.5
+    w = (torch.randn(6144, K, device=gpu) * K ** -0.5).bfloat16()
+    r = hops.norm_linear(delta, h, g, 8, 1e-5, w)
+    want = h.double() + delta.double()
+    if r is None:
+        assert M > (limit or 4) or M * K > 16384
+        h2 = h.clone()
+        r = hops.group_norm(delta, h2, g, 8, 1e-5, torch.bfloat16) @ w.t(), h2
+    p = want.view(M, 8, -1)
+    x = (p * torch.rsqrt(p.pow(2).mean(-1, keepdim=True) + 1e-5)).view(M, K) * g.double()
+    assert rel_err(r[1], want) < 1e-6 and rel_err(r[0], x @ w.double().t()) < 2 ** -7  # the norm's rounding and the product's
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 9, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 1536), (48, 8192), (4112, 3584), (2048, 12288), (4096, 14336), (272, 21504), (8192, 4096)])
 def test_stream_parts(gpu, M, N, K):
