@@ -328,8 +328,9 @@ def norm_linear(delta, h, gamma, groups: int, eps: float, w):
     if not _fusable(h, w):
         return None
     M, K = h.shape
-    if (M <= min(4, _NORM_STREAM_M) and groups == 8 and K in (2048, 4096) and w.shape[0] >= 6144 and w.data_ptr() % 16 == 0
-            and (delta is None or delta.stride(0) % 8 == 0)):
+    if (M <= min(4, _NORM_STREAM_M) and groups == 8 and K in (2048, 4096) and w.shape[0] >= 6144
+            and all(t.data_ptr() % 16 == 0 for t in (h, gamma, w))
+            and (delta is None or (delta.stride(0) % 8 == 0 and delta.data_ptr() % 16 == 0))):
         return native().stream_group_norm(delta, h, gamma, eps, w)
     if not _norm_fits(h, groups):
         return None

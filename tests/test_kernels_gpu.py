@@ -1039,6 +1039,35 @@ def test_group_norm_prologue_by_the_rows_asked_for(gpu, monkeypatch, M, K, limit
     assert rel_err(r[1], want) < 1e-6 and rel_err(r[0], x @ w.double().t()) < 2 ** -7  # the norm's rounding and the product's
 
 
+def _off16(t):
+    """t in storage that starts between two 16-byte pieces."""
+    room = torch.empty(t.numel() + 8, device=t.device, dtype=t.dtype)
+    room[1:t.numel() + 1].copy_(t.flatten())
+    return room[1:t.numel() + 1].view(t.shape)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3])
+@pytest.mark.parametrize("odd", ["gamma", "h", "delta"])
+def test_group_norm_prologue_leaves_operands_that_are_not_aligned(gpu, M, odd):
+    """A norm weight off 16 bytes goes to the other prologue; past its rows everything goes to the parts, without an error."""
+    from mxllm.ops import hybrid as hops
+
+    K = 2048
+    torch.manual_seed(M)
+    t = dict(delta=torch.randn(M, K, device=gpu).bfloat16(), h=torch.randn(M, K, device=gpu), gamma=torch.rand(K, device=gpu) + 0.5)
+    w = (torch.randn(6144, K, device=gpu) * K ** -0.5).bfloat16()
+    if odd != "gamma" and M <= hops.NORM_M:
+        return  # that prologue reads rows in 16-byte pieces and says so
+    t[odd] = _off16(t[odd])
+    r = hops.norm_linear(t["delta"], t["h"], t["gamma"], 8, 1e-5, w)
+    assert (r is None) == (M > hops.NORM_M)
+    if r is not None:
+        h2 = t["h"].clone()
+        y = hops.group_norm(t["delta"], h2, t["gamma"], 8, 1e-5, torch.bfloat16)
+        assert torch.equal(r[1], h2) and rel_err(r[0], y.double() @ w.double().t()) < 2 ** -7
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 9, 16, 17, 32])
 @pytest.mark.parametrize("N,K", [(16, 1536), (48, 8192), (4112, 3584), (2048, 12288), (4096, 14336), (272, 21504), (8192, 4096)])
