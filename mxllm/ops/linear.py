@@ -36,6 +36,7 @@ from torch.autograd import forward_ad
 from ..parallel.grad_ready import direct_grad, direct_grad32, mark_ready
 from . import gemm
 from ._ext import native, use_native
+from .norm import add_rms_norm
 
 
 class _LoRALinearFn(torch.autograd.Function):
@@ -756,9 +757,21 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     return native().stream_parts(x, w)
 
 
+def parts_sum(parts: torch.Tensor) -> torch.Tensor:
+    """The product that :func:`linear_parts` returned in parts, as the norms that add them have it: f32 sums, one part after the
+    other, rounded to bf16."""
+    y = parts[0].clone()
+    for p in parts[1:]:
+        y += p
+    return y.bfloat16()
+
+
 def parts_norm(parts: torch.Tensor, h: torch.Tensor, gamma: torch.Tensor, eps: float):
     """``add_rms_norm`` of what :func:`linear_parts` returned: (normed, h + the sum rounded to bf16)."""
-    return native().parts_norm(parts, h.contiguous(), gamma, float(eps))
+    h = h.contiguous()
+    if h.data_ptr() % 16 or gamma.data_ptr() % 16:  # (the kernel reads both in 16-byte pieces)
+        return add_rms_norm(parts_sum(parts), h, gamma, eps)
+    return native().parts_norm(parts, h, gamma, float(eps))
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:

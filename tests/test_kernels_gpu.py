@@ -1101,6 +1101,22 @@ def test_stream_parts(gpu, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("odd", ["gamma", "h"])
+def test_parts_norm_of_operands_that_are_not_aligned(gpu, odd):
+    """They go to the norm that takes them, behind the parts' sum: the residual's bits, the norm to two roundings to bf16."""
+    from mxllm import ops
+
+    torch.manual_seed(3)
+    M, N, K = 12, 2048, 8192
+    t = dict(h=torch.randn(M, N, device=gpu).bfloat16(), gamma=torch.randn(N, device=gpu).bfloat16())
+    parts = ops.linear_parts(torch.randn(M, K, device=gpu).bfloat16(), (torch.randn(N, K, device=gpu) * K ** -0.5).bfloat16())
+    want = ops.parts_norm(parts, t["h"], t["gamma"], 1e-5)
+    t[odd] = _off16(t[odd])
+    y, h = ops.parts_norm(parts, t["h"], t["gamma"], 1e-5)
+    assert torch.equal(h, want[1]) and rel_err(y, want[0]) < 2 ** -8
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D", [32, 64, 128])
 @pytest.mark.parametrize("Hq,Hkv", [(16, 2), (4, 4), (7, 1), (9, 1)])
 def test_decode_attn_up_to_512_keys(gpu, D, Hq, Hkv):
