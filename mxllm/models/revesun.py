@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from ..ops import hybrid as hops
-from ..ops import linear, linear_parts
+from ..ops import linear, linear_parts, parts_sum
 from ..ops.hybrid import AttnShape, PromptRows, RopeTables
 from .config import PRESETS
 from .llama import FusedLinear, plain_weight
@@ -261,7 +261,7 @@ class Revesun(nn.Module):
                 z, h = self._norm_proj(delta, h, layer.norm2, layer.wup, rows.decode)
                 delta = self._down(z, layer, rows.decode)
             if tap is not None:
-                tap(i, h + (delta if delta.dim() == 2 else delta.sum(0)).float())
+                tap(i, h + (delta if delta.dim() == 2 else parts_sum(delta)).float())
         return hops.group_norm(delta, h, self.final_norm, self.cfg.norm_groups, self.cfg.norm_eps, self.dtype)
 
     @torch.no_grad()

@@ -340,6 +340,22 @@ def test_residual_stream_layer_by_layer(built, dev, dt):
         close(a, b, dt, 2)
 
 
+def parts_model(gpu, last_ff=8192):
+    """Down projections of a K that goes in parts at 9 to 32 rows."""
+    cfg = RevesunConfig.from_json(orc.config(512, 128, 4, [M(68, 8192), A(4, 2, 36, 20, 3, 21, 1e4, 12, 0.2, 8192), M(512, last_ff)]))
+    return Revesun(cfg, device=gpu, seed=1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [8, 9, 16])
+def test_the_residual_that_a_tap_sees_is_the_next_norms(gpu, n):
+    """Sub-blocks whose output comes in parts: the norm of the last tapped residual is the model's output, bit for bit."""
+    model, got = parts_model(gpu), []
+    y = model.hidden_states(torch.tensor([tokens(n, 128, n)], device=gpu), tap=lambda i, h: got.append(h.clone()))
+    c = model.cfg
+    assert torch.equal(hops.group_norm(None, got[-1], model.final_norm, c.norm_groups, c.norm_eps, model.dtype), y)
+
+
 @pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
 @pytest.mark.parametrize("name", ["mixed", "mingru_only", "attention_only"])
 def test_greedy_generation_through_the_scheduler(built, name, dev):
