@@ -347,8 +347,8 @@ def poly_linear(z, coef, eps: float, w):
 
 
 def _normed(delta, h, gamma, groups, eps):
-    """(delta, x, gamma) of a fused projection: the norm in its prologue, or run ahead of it."""
-    if _norm_fits(h, groups):
+    """(delta, x, gamma) of a fused projection: the norm in its prologue, or run ahead of it (a delta in parts is added there)."""
+    if _norm_fits(h, groups) and (delta is None or delta.dim() == 2):
         return delta, h, gamma
     return None, group_norm(delta, h, gamma, groups, eps, torch.bfloat16), None
 

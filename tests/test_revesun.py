@@ -356,6 +356,25 @@ def test_the_residual_that_a_tap_sees_is_the_next_norms(gpu, n):
     assert torch.equal(hops.group_norm(None, got[-1], model.final_norm, c.norm_groups, c.norm_eps, model.dtype), y)
 
 
+@pytest.mark.gpu
+def test_parts_go_past_the_norm_prologues(gpu, monkeypatch):
+    """MXLLM_SKINNY_M and MXLLM_NORM_FUSED_M of 16: projections with the norm in their prologue behind outputs in parts, against
+    the steps without the settings (other kernels, so to rounding)."""
+    model, prompts = parts_model(gpu), [tokens(3 + i, 128, i) for i in range(12)]
+    feed = torch.randint(0, 128, (4, 12), generator=torch.Generator().manual_seed(1))
+    outs = []
+    for rows in (None, 16):
+        if rows:
+            monkeypatch.setattr(hops, "SKINNY_M", rows)
+            monkeypatch.setattr(hops, "NORM_M", rows)
+        eng = Engine(model, max_batch=12, max_seq=256, kv_pool_tokens=4096)
+        slots = [eng.acquire() for _ in prompts]
+        eng.prefill_batch(slots, prompts)
+        outs.append(torch.stack([eng.decode(slots, t).float().clone() for t in feed]))
+    rel = (outs[0] - outs[1]).pow(2).mean().sqrt() / outs[0].pow(2).mean().sqrt()
+    assert float(rel) < 1.5e-2, float(rel)
+
+
 @pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
 @pytest.mark.parametrize("name", ["mixed", "mingru_only", "attention_only"])
 def test_greedy_generation_through_the_scheduler(built, name, dev):
