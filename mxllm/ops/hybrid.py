@@ -19,7 +19,7 @@ import numpy as np
 import torch
 
 from ._ext import native, use_native
-from .linear import NORM_M, SKINNY_M, _NORM_STREAM_M, _SKINNY_SMALL_W
+from .linear import NORM_M, SKINNY_M, _NORM_STREAM_M, _SKINNY_SMALL_W, _near
 
 MFMA_MAX_DIM = 128  # widest head of the MFMA attention kernels
 MFMA_MAX_REP = 16   # query heads per key head in the split-K decode kernels
@@ -329,7 +329,7 @@ def norm_linear(delta, h, gamma, groups: int, eps: float, w):
         return None
     M, K = h.shape
     if (M <= min(4, _NORM_STREAM_M) and groups == 8 and K in (2048, 4096) and w.shape[0] >= 6144
-            and all(t.data_ptr() % 16 == 0 for t in (h, gamma, w))
+            and _near(w) and all(t.data_ptr() % 16 == 0 for t in (h, gamma, w))
             and (delta is None or (delta.stride(0) % 8 == 0 and delta.data_ptr() % 16 == 0))):
         return native().stream_group_norm(delta, h, gamma, eps, w)
     if not _norm_fits(h, groups):

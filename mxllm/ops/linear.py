@@ -640,6 +640,12 @@ def _rows_ok(x2: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = Non
             and (scale is None or scale.data_ptr() % 16 == 0) and use_native(x2))
 
 
+def _near(w: torch.Tensor, swiglu: bool = False) -> bool:
+    """Weights that the workgroups that stay take: their offsets inside a channel group have 32 bits (csrc/kernels/stream_core.h),
+    over 256 rows or, with SwiGLU, from the gate's rows to the up rows.  skinny_gemm.hip has 64-bit addresses."""
+    return (w.shape[0] // 2 + 16 if swiglu else 256) * w.stride(0) * w.element_size() < 1 << 32
+
+
 def _stream_fits(M: int, K: int, norm: bool = False) -> bool:
     """Rows of K that csrc/kernels/stream_gemm.hip holds in LDS beside its partial sums (``norm``: and norms)."""
     return 0 < M <= min(4 if norm else 32, _DECODE_M) and K % 2048 == 0 and 16384 + 2 * M * (K + 8) <= 158 * 1024
@@ -664,7 +670,7 @@ def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Ten
     fp8_gemm.hip -> there: 4096 x 14336, 1 / 4 rows 14.5 / 15.9 -> 12.9 / 14.3; 2048 x 8192, 1 row 7.8 -> 7.2; but 4096 x
     4096, 1 row 5.3 -> 5.9; from 3 rows on w8_linear goes there by itself)."""
     M, K = x2.shape
-    if K >= 8192 and _stream_fits(M, K) and _rows_ok(x2, q, scale):
+    if K >= 8192 and _stream_fits(M, K) and _near(q) and _rows_ok(x2, q, scale):
         return native().stream_linear(x2, None, None, 0.0, q, scale, False)[0]
     return native().w8_linear(x2, q, scale)
 
@@ -713,7 +719,7 @@ def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
         x2 = x.reshape(M, K)
         if not _rows_ok(x2, w):
             return None
-        if route == "stream":
+        if route == "stream" and _near(w):
             y = native().stream_linear(x2, None, None, 0.0, w, None, False)[0]
         else:
             y = (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
@@ -752,7 +758,9 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     if not x.is_cuda or x.dim() != 2 or w.dim() != 2:
         return None
     (M, K), N = x.shape, w.shape[0]
-    if not _parts_wins(M, N, K) or not _plain(x, w) or not _rows_ok(x, w) or not native().stream_parts_segments(M, N, K):
+    if not _parts_wins(M, N, K) or not _near(w) or not _plain(x, w) or not _rows_ok(x, w):
+        return None
+    if not native().stream_parts_segments(M, N, K):
         return None
     return native().stream_parts(x, w)
 
@@ -783,11 +791,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
         return None
     (M, K), N = x.shape, w.shape[0]
     if scale is not None:
-        if not (_stream_fits(M, K) and _plain(x, w) and _rows_ok(x, w, scale)):
+        if not (_stream_fits(M, K) and _near(w, True) and _plain(x, w) and _rows_ok(x, w, scale)):
             return None
         return native().stream_linear(x, None, None, 0.0, w, scale, True)[0]
     if _stream_wins(M, N, K, True) and _plain(x, w) and _rows_ok(x, w):
-        return native().stream_linear(x, None, None, 0.0, w, None, True)[0]
+        return native().stream_linear(x, None, None, 0.0, w, None, True)[0] if _near(w, True) else native().skinny_linear_swiglu(x, w)
     if M <= SKINNY_M and _plain(x, w) and _skinny_ok(x, w):
         return native().skinny_linear_swiglu(x, w)
     parts = gemm.rows_gain(M, N, K, True, True)  # a prompt pass
@@ -835,7 +843,7 @@ def qkv_rope_ok(h: torch.Tensor, w: torch.Tensor, cos, sin, k_cache, v_cache, Hq
             and v_cache.is_contiguous()):
         return False
     if _qkv_stream(M, K, norm, D, scale is not None):
-        return _rows_ok(h, w, scale)
+        return _near(w) and _rows_ok(h, w, scale)
     if scale is not None or D != 128 or not 0 < M <= (min(NORM_M, SKINNY_M) if norm else SKINNY_M):
         return False
     return bool((not norm or M * K <= 32768) and _skinny_ok(h, w))
@@ -886,7 +894,7 @@ def norm_linear(delta: torch.Tensor | None, h: torch.Tensor, gamma: torch.Tensor
         return None
     if w.shape[1] != K or w.shape[0] % 16 or not (_plain(delta, h, gamma, w) and _norm_operands(delta, h, gamma)):
         return None
-    if not (_rows_ok(h, w, scale) if stream else _skinny_ok(h, w)):
+    if not (_near(w, swiglu) and _rows_ok(h, w, scale) if stream else _skinny_ok(h, w)):
         return None
     if stream:
         return native().stream_linear(h, delta, gamma, float(eps), w, scale, bool(swiglu))

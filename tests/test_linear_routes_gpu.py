@@ -111,6 +111,29 @@ def test_odd_layouts_take_the_library(gpu, kind, M):
         assert ops.linear_swiglu(_bf16(gpu, M, K), q, s) is None
 
 
+@pytest.mark.parametrize("M", [2, 12])
+def test_weights_whose_rows_lie_far_apart(gpu, monkeypatch, M):
+    """Rows past the 32-bit offsets of the workgroups that stay (every one of whose rules is made to ask for them): the kernel with
+    64-bit addresses, or the parts; one bf16 rounding, with SwiGLU that of its two operands too."""
+    lin = sys.modules["mxllm.ops.linear"]
+    for rule in ("_stream_wins", "_norm_wins", "_parts_wins"):
+        monkeypatch.setattr(lin, rule, lambda *a: True)
+    N, gamma = 64, torch.ones(2048, device=gpu).bfloat16()
+
+    def far(K, stride):
+        w = torch.empty_strided((N, K), (stride, 1), device=gpu, dtype=torch.bfloat16)
+        w.copy_(_bf16(gpu, N, K, seed=2, std=0.03))
+        return w
+
+    x, w = _bf16(gpu, M, 2048, seed=1), far(2048, 1 << 23)
+    want = x.double() @ w.double().t()
+    _close(ops.linear(x, w), want, 2 ** -8)
+    assert ops.linear_parts(_bf16(gpu, 12, 8192), far(8192, 1 << 23)) is None
+    assert M > 4 or ops.norm_linear(None, x, gamma, 1e-5, w) is None
+    w = far(2048, 1 << 26)
+    _close(ops.linear_swiglu(x, w), torch.nn.functional.silu(want[:, :32]) * want[:, 32:], 3 * 2 ** -8)
+
+
 @pytest.mark.parametrize("M", [1, 16, 64])
 def test_switch_off_is_the_library(gpu, M, monkeypatch):
     """MXLLM_SKINNY_M=0: no forward GEMM of inference runs on a kernel of ours."""
