@@ -944,8 +944,10 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
     return (int)hipGetLastError();
   }
   // Heads of 128, more splits than places: dealt evenly.  What the caller's `nsplit` counts is the longest that the step
-  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.
-  if (out && D == kEvenD && (int64_t)nsplit * Hkv * B > kEvenPlaces) {
+  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.  Not of one split (no merge
+  // to wait for: 32 heads of 8, us, split -> dealt: 80 sequences of 60 to 256 keys 16.0 -> 20.8, 256 36.3 -> 42.8; 72 of 10 to
+  // 64 10.2 -> 19.0) nor of two where the kernel above does not take them (32 heads of 2, 256 of 20 to 200 keys 29.0 -> 31.5).
+  if (out && D == kEvenD && nsplit > kShortSplits && (int64_t)nsplit * Hkv * B > kEvenPlaces) {
     const int W = even_groups(Hkv), cap = nsplit * kSplit, nparts = even_parts(Hkv, nsplit);
     decode_even_kernel<<<dim3(W, Hkv), 256, 0, stream>>>(q, kc, vc, lens, len_off, slots, part_ml, part_o, out, B, Hq, Hkv,
                                                          max_seq, cap, nparts, sl, bt, maxb);

@@ -1147,9 +1147,25 @@ def test_decode_attn_up_to_512_keys(gpu, D, Hq, Hkv):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,room", [(32, 8, 256), (16, 1, 512)])
+def test_decode_attn_of_few_splits_is_not_dealt(gpu, Hq, Hkv, room):
+    """Many sequences of one split, or of two past 8 heads of a KV head, keep a workgroup a split (dealt evenly they took up to
+    twice as long): a row's bits are those it has alone."""
+    D, B = 128, 80 if room == 256 else 300
+    torch.manual_seed(B)
+    kc, vc = (torch.randn(B, Hkv, room, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+    pos = torch.randint(40, room + 1, (B,), device=gpu).to(torch.int32)
+    out = _ops().decode_attn(q, kc, vc, pos, None, room, D ** -0.5, 0, None, None)
+    for b in range(0, B, 9):
+        one = _ops().decode_attn(q[b:b + 1], kc[b:b + 1], vc[b:b + 1], pos[b:b + 1], None, room, D ** -0.5, 0, None, None)
+        assert torch.equal(out[b], one[0])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv,lens,room", [(32, 8, [1, 15, 16, 17, 255, 256, 257, 0] + [1, 33, 700, 90] * 6, 700),
                                               (16, 1, [3000, 0, 1, 2600], 65536), (8, 8, [4000, 4096], 8448),
-                                              (6, 2, [5] * 300, 256), (64, 8, [2000, 64, 65, 1999, 1, 1900], 3000)])
+                                              (6, 2, [5] * 300, 256), (6, 2, [5] * 300, 700), (64, 8, [2000, 64, 65, 1999, 1, 1900], 3000)])
 @pytest.mark.parametrize("paged", [False, True])
 def test_decode_attn_dealt_evenly(gpu, Hq, Hkv, lens, room, paged):
     """More splits than the chip has places for: workgroups that take several sequences, sequences of many parts, of none
