@@ -464,21 +464,23 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
   } while (0)
 #define FS(...) FewSlices<__VA_ARGS__>
 #define FL(...) FewLines<__VA_ARGS__>
-  // Down: FewLines, which reads a part of K in blocks of 3 chunks, where it was the faster one: a short K but for 5 to 8 pairs
-  // (four K parts; 2048 x 384, 4 / 8 / 32 / 128 pairs, us: 5.2 / 7.8 / 10.4 (16 tokens) / 11.8 by it, 5.7 / 7.1 / 11.8 / 15.4
-  // by FewSlices), a longer one up to 8 pairs and past 16 tokens (4096 x 768, 2 / 8 / 16 / 32 tokens 14.6 / 23.8 / 25.8 /
-  // 29.4, 15.7 / 23.4 / 25.6 / 33.0).  Up stays with FewSlices (2 x 384 x 2048, 32 tokens 21.1 us, 23.3 by FewLines; 768 x 4096
-  // 57.1, 62.4).
+  // Down: FewLines for more than 8 pairs where both K parts are whole blocks of 3 chunks, past one block each from 17 tokens on
+  // (and up to 16 tokens with the shared expert's eight in whole blocks of 4): loads past a part's end cost as others do.  us,
+  // FewSlices -> FewLines: 2048 x 384, 16 / 64 / 128 pairs 8.2 -> 6.9, 8.7 -> 7.0, 10.0 -> 8.3; 4096 x 768 with a shared expert of
+  // 2048, 128 pairs 28.5 -> 27.5; 2048 x 1152, 128 pairs 19.3 -> 17.5.  Elsewhere it loses: 1024 x 512, 2 to 8 pairs half as much
+  // again, 2048 x 256, 256 pairs a third, 2 to 8 pairs of any K, where four K parts hide more, up to two thirds; 4096 x 768 with
+  // few tokens' uneven choices, 20 pairs 18.0 -> 23.4, 48 22.8 -> 24.7.  Up stays with FewSlices (2 x 384 x 2048, 32 tokens
+  // 21.1 us, 23.3 by FewLines; 768 x 4096 57.1, 62.4).
   const int pairs = a.T * a.top;
-  const bool lines = !glu && a.K % 64 == 0 && (!a.sw || a.sK % 64 == 0) &&
-                     (a.K < 512 ? pairs <= 4 || pairs > 8 : pairs <= 8 || a.T > 16) &&
+  const bool lines = !glu && a.K % 384 == 0 && pairs > 8 &&
+                     (a.T > 16 || (a.K <= 384 && (!a.sw || a.sK % 2048 == 0))) &&
                      std::max(std::max((int64_t)a.N * a.K, (int64_t)a.sN * a.sK),
                               pairs * std::max(a.ldx, (int64_t)a.sK)) < (1ll << 31) - 4096;
   if (glu) {
     if (a.T <= 16) MF(true, FS(true, 8, 2), 16, 16, FS(true, 8, 2), 16, 16);
     else if (a.T <= 32) MF(true, FS(true, 8, 2), 32, 16, FS(true, 8, 2), 32, 32);
     else MF(true, FS(true, 8, 4), 64, 16, FS(true, 8, 4), 64, 64);
-  } else if (pairs <= 8 && !lines) {
+  } else if (pairs <= 8) {
     MF(false, FS(false, 4, 1), 16, 16, FS(false, 8, 1), 16, 16);
   } else if (lines) {
     if (a.T <= 8) MF(false, FL(false, 2, 1, 3), 8, 8, FL(false, 8, 1, 4), 8, 8);

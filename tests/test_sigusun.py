@@ -247,7 +247,7 @@ def test_side_projection_of_columns_nearly_dependent(gpu, W):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("ff,shared", [(64, 64), (192, 0), (384, 2048), (448, 128), (768, 192)])
+@pytest.mark.parametrize("ff,shared", [(64, 64), (192, 0), (384, 2048), (448, 128), (768, 192), (384, 0), (768, 2048), (1152, 4096)])
 @pytest.mark.parametrize("T", [1, 3, 8, 9, 16, 17, 32, 33, 64])
 def test_down_products_of_few_rows(gpu, T, ff, shared):
     """Whole-line fragments of the experts' down products: K parts of none, some and all of a block of chunks, a remainder of
