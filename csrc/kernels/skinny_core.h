@@ -35,8 +35,10 @@ constexpr int kSkWaves = 8;
 constexpr int sk_parts(int M, int K) { return K == 2048 && M <= 16 ? 4 : 8; }
 // Whether fragments of 16 rows x 64 B and 16 tokens, without the halves, are the better ones: past 16 token rows, and past 8 of a
 // K under 2048, the products and sums of each 8 tokens show beside the few bytes (4096 x 1024, 12 / 32 rows 4.8 / 7.2 us in
-// blocks of 8, 4.6 / 5.9 so; stream_gemm.hip, 16384 x 2048, 32 rows 20.0, 18.6 so).
-constexpr bool sk_wide(int M, int K) { return M > 16 || (M > 8 && K < 2048); }
+// blocks of 8, 4.6 / 5.9 so; stream_gemm.hip, 16384 x 2048, 32 rows 20.0, 18.6 so).  So do they where a wave's part is 6 or 7
+// chunks, whose loads go out in two or three turns either way (2048 x 3072, 9 / 16 rows 7.7 / 8.7, 7.4 / 8.1 so; 2048 x 3584, 16
+// rows 9.7, 9.3 so; of 5 chunks, 2048 x 2560, 6.7 / 7.7, 6.9 / 7.7 so; of 9, 2048 x 4608, 9.7 / 11.1, 10.3 / 11.9 so).
+constexpr bool sk_wide(int M, int K) { return M > 16 || (M > 8 && (K < 2048 || (K > 2560 && K < 4096))); }
 // 8-row blocks of a wave for NC groups of 16 channels
 template <int KP, int NC>
 constexpr int kSkBlocks = NC * KP / 4;
