@@ -135,7 +135,13 @@ static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
   constexpr int LINES = F8 ? kStF8Lines : kStLines, WIDE = F8 ? kStF8 : kStWide;
   if (norm) return stream_blocks<LINES, 1, EPI, true>(a, stream);
   if (a.M <= 8) return stream_blocks<LINES, 1, EPI, false>(a, stream);
-  if (a.M <= 16) return F8 ? stream_blocks<kStF8, 1, EPI, false>(a, stream) : stream_blocks<LINES, F8 ? 1 : 2, EPI, false>(a, stream);
+  // 9 to 16 rows: whole lines, but for a K of 4096 of up to one and a half groups a CU, where the first bytes and the rows in LDS
+  // are what lasts (us, lines -> 16 rows, 9 / 16 rows: 1024 x 4096 8.3 / 9.1 -> 8.2 / 8.8, 2048 8.7 / 9.5 -> 8.4 / 9.1, 6144 14.2 / 15.0
+  // -> 14.2 / 14.7; but 12288 20.8 / 21.8 -> 21.4 / 22.0; 2048 x 2048 5.4 / 6.1 -> 5.6 / 6.0).  Between 192 and 256 groups they are
+  // level, and skinny_gemm.hip has these sizes with the bits of whole lines.
+  const bool few = a.groups <= 192 || (a.groups > 256 && a.groups <= 384);
+  if (a.M <= 16 && (F8 || (a.K == 4096 && few))) return stream_blocks<WIDE, 1, EPI, false>(a, stream);
+  if (a.M <= 16) return stream_blocks<LINES, F8 ? 1 : 2, EPI, false>(a, stream);
   return stream_blocks<WIDE, 2, EPI, false>(a, stream);
 }
 

@@ -1259,7 +1259,7 @@ def test_prefill_attention_runs_the_kernels(gpu, D, Hq, Hkv, S):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1, 48, 2048), (2, 8208, 2048), (3, 48, 2048), (8, 8208, 3072), (7, 16, 512), (9, 32, 1536),
                                    (12, 1040, 3072), (16, 3088, 4096), (16, 48, 2048), (17, 48, 2560), (31, 16, 512), (9, 48, 2560),
-                                   (9, 16, 3072), (13, 2064, 3584), (16, 48, 4608)])
+                                   (9, 16, 3072), (13, 2064, 3584), (16, 48, 4608), (13, 48, 4096), (16, 3072, 4096), (9, 4112, 4096)])
 def test_skinny_linear_fragments(gpu, M, N, K):
     """The decode GEMM's ways to read (4 and 8 K parts, all loads of a block ahead or not, blocks of 8 and of 16 rows and tokens,
     the kernel that stays) against fp64, plain and with SwiGLU; row-strided x, rows and groups at their edges."""
