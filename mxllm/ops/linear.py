@@ -609,8 +609,8 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 #  * Past 8 rows (hipBLASLt -> stream): a K of 2048 at any width (2048 x 2048, 12 / 32 rows 11.0 / 11.3 -> 5.6 / 7.7; 16384, 16
 #    rows 17.9 -> 16.3), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 18.0 / 18.1 -> 17.9 / 18.6;
 #    14336 15.8 / 15.7 -> 16.7 / 17.7; 20480 22.0 / 22.1 -> 20.4 / 21.1), which gain with SwiGLU only (19.2 -> 18.0).  A K of 4096 up
-#    to 16 rows (6144, 16 rows 14.7 -> 14.6; 28672 61 -> 41), but for one group a CU (4096, 9 / 16 rows skinny 9.0 / 10.2
-#    against 10.1 / 10.5), a 17th only where there is much to stream (16384 30.7 -> 29.2, 12288 22.2 -> 24.1).  Longer ones
+#    to 16 rows (6144, 16 rows 14.7 -> 14.6; 28672 61 -> 41), but for one group a CU without SwiGLU (4096, 9 / 16 rows skinny
+#    9.0 / 10.2 against 10.1 / 10.5; with it 12 / 16 rows 11.0 / 11.1, in two launches 11.8 / 12.6), a 17th only where there is much to stream (16384 30.7 -> 29.2, 12288 22.2 -> 24.1).  Longer ones
 #    from 12288 channels on (12288 x 6144, 9 rows 35.5 -> 32.2, 6144 18.4 -> 20.2).
 _STREAM_MK, _STREAM_N4, _STREAM_N2 = 16384, 6144, 32768
 
@@ -658,7 +658,7 @@ def _stream_wins(M: int, N: int, K: int, swiglu: bool = False) -> bool:
         if K > 4096:
             return N >= 12288
         if K == 4096:
-            return N >= 2048 and not 3072 < N <= 4096 if M <= 16 else N >= 16384
+            return N >= 2048 and (swiglu or not 3072 < N <= 4096) if M <= 16 else N >= 16384
         return N >= 2048 and (swiglu or M <= 16 or not 12288 < N < 20480)
     if K % 4096 == 0 and N >= _STREAM_N4:
         return M > 1 or N < _STREAM_N2

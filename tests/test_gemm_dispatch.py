@@ -98,6 +98,7 @@ def test_swiglu_route_of_decode_rows():
     wins = sys.modules["mxllm.ops.linear"]._stream_wins
     assert wins(8, 10240, 2048, True) and not wins(8, 8192, 2048, True) and not wins(8, 10240, 2048)
     assert wins(32, 16384, 2048, True) and not wins(32, 16384, 2048) and not wins(33, 16384, 2048, True)
+    assert wins(12, 4096, 4096, True) and wins(16, 3584, 4096, True) and not wins(12, 4096, 4096)
 
 
 def test_qkv_route_of_decode_rows():
