@@ -187,6 +187,11 @@ extern "C" int mx_skinny_rope_gemm(const uint16_t* h, int64_t ldh, int norm, con
   if (M > (norm ? 4 : 16) || (norm && (int64_t)M * K > 32768) || K % 512 || ldh % 8 || ldd % 8 || ldw % 8 ||
       ldh < K || ldw < K || (norm && delta && (ldd < K || !h_out)))
     return -1;
+  // Past 4 rows of 2048 X is in LDS (us, 3072 channels, 6 / 8 rows 6.2 / 6.6 -> 5.9 / 6.1; 4 rows 5.9), with the same bits.
+  if (!norm && K == 2048 && M > 4 &&
+      mx_stream_gemm(h, ldh, w, ldw, nullptr, nullptr, 0, M, N, K, 2, nullptr, 0, nullptr, 0.f, nullptr, cosb, sinb, pos, slots, q,
+                     kc, vc, Hq, Hkv, max_seq, bt, maxb, stream) == 0)
+    return 0;
   const SkRope rp{cosb, sinb, pos, slots, q, kc, vc, Hq, Hkv, max_seq, bt, maxb};
   if (norm) {
     const SkNorm na{delta, ldd, gamma, h_out, eps};

@@ -610,8 +610,9 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 #    rows 17.9 -> 16.3), but for 16384 channels and their neighbours past 16 rows (24 / 32 rows 18.0 / 18.1 -> 17.9 / 18.6;
 #    14336 15.8 / 15.7 -> 16.7 / 17.7; 20480 22.0 / 22.1 -> 20.4 / 21.1), which gain with SwiGLU only (19.2 -> 18.0).  A K of 4096 up
 #    to 16 rows (6144, 16 rows 14.7 -> 14.6; 28672 61 -> 41), but for one group a CU without SwiGLU (4096, 9 / 16 rows skinny
-#    9.0 / 10.2 against 10.1 / 10.5; with it 12 / 16 rows 11.0 / 11.1, in two launches 11.8 / 12.6), a 17th only where there is much to stream (16384 30.7 -> 29.2, 12288 22.2 -> 24.1).  Longer ones
-#    from 12288 channels on (12288 x 6144, 9 rows 35.5 -> 32.2, 6144 18.4 -> 20.2).
+#    9.0 / 10.2 against 10.1 / 10.5; with it 12 / 16 rows 11.0 / 11.1, in two launches 11.8 / 12.6), a 17th only where there is
+#    much to stream (16384 30.7 -> 29.2, 12288 22.2 -> 24.1).  Longer ones from 12288 channels on (12288 x 6144, 9 rows 35.5 ->
+#    32.2, 6144 18.4 -> 20.2).
 _STREAM_MK, _STREAM_N4, _STREAM_N2 = 16384, 6144, 32768
 
 

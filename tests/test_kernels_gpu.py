@@ -704,7 +704,8 @@ def test_skinny_norm_linear(gpu, M, N, K, resid, swiglu):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,Hq,Hkv,K,norm,resid", [(1, 32, 8, 4096, True, True), (2, 8, 2, 1024, True, False),
-                                                   (2, 64, 8, 8192, True, True), (5, 16, 4, 2048, False, False)])
+                                                   (2, 64, 8, 8192, True, True), (5, 16, 4, 2048, False, False),
+                                                   (4, 16, 4, 2048, False, False)])
 def test_skinny_qkv_rope(gpu, M, Hq, Hkv, K, norm, resid):
     """Decode QKV projection with RoPE + KV-cache append in the GEMM epilogue (and the RMSNorm
     in its prologue): the same q, cache rows and residual as RMSNorm + decode GEMM + rope_append."""
