@@ -202,6 +202,12 @@ def plain_weight(lin) -> torch.Tensor | None:
     return lin.weight if type(lin) is FusedLinear else None
 
 
+def hooked(lin: nn.Module) -> bool:
+    """Whether forward hooks, of the module or of all modules, are to see its call."""
+    m = torch.nn.modules.module
+    return bool(lin._forward_hooks or lin._forward_pre_hooks or m._global_forward_hooks or m._global_forward_pre_hooks)
+
+
 class Llama(nn.Module):
     def __init__(self, cfg: LlamaConfig, *, device=None, dtype=torch.bfloat16, lora_r: int = 0,
                  lora_alpha: float = 16.0, seed: int = 0, init: bool = True,

@@ -24,7 +24,7 @@ from ..ops import hybrid as hops
 from ..ops import linear, linear_parts, parts_sum
 from ..ops.hybrid import AttnShape, PromptRows, RopeTables
 from .config import PRESETS
-from .llama import FusedLinear, plain_weight
+from .llama import FusedLinear, hooked, plain_weight
 
 
 @dataclass(frozen=True)
@@ -210,7 +210,7 @@ class Revesun(nn.Module):
     def _sub_output(self, lin, x):
         """Output of a sub-block's last projection; for a few rows of a long K the sums of its segments, which the norm
         behind it adds (parts of whole vectors)."""
-        w = plain_weight(lin) if self.cfg.hidden // self.cfg.norm_groups % 4 == 0 else None
+        w = plain_weight(lin) if self.cfg.hidden // self.cfg.norm_groups % 4 == 0 and not hooked(lin) else None
         parts = linear_parts(x, w) if w is not None else None
         return lin(x) if parts is None else parts
 

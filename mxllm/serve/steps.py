@@ -20,7 +20,7 @@ import weakref
 import torch
 
 from .. import ops
-from ..models.llama import FusedLinear, Llama
+from ..models.llama import FusedLinear, Llama, hooked
 from ..models.revesun import Revesun
 from ..models.sigusun import Sigusun
 from ..ops import decode as dops
@@ -116,7 +116,7 @@ class LlamaSteps:
 
     def _sub_output(self, lin, x):
         """Output of a sub-block's last projection, on its way to a norm."""
-        if self.eng.tp is None and type(lin) is FusedLinear and lin.lora_r == 0:
+        if self.eng.tp is None and type(lin) is FusedLinear and lin.lora_r == 0 and not hooked(lin):
             parts = ops.linear_parts(x, lin.weight)
             if parts is not None:
                 return parts

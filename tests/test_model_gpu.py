@@ -647,3 +647,26 @@ def test_swiglu_recompute_bitwise_gpu(gpu, monkeypatch):
         assert l0 == l1
         for k in g0:
             assert torch.equal(g0[k], g1[k]), (ck, k)
+
+
+@pytest.mark.parametrize("batch", [4, 12])
+def test_decode_calls_the_hooks_of_output_projections(gpu, batch):
+    """Forward hooks on wo and wd, at batches whose down projection comes in parts without them and at others; the logits are
+    those without hooks to rounding."""
+    from mxllm.models import Llama, get_config
+    from mxllm.serve.engine import Engine
+
+    cfg = get_config("tiny").replace(hidden=512, ffn=8192, n_heads=8, head_dim=64)
+    m, calls, outs = Llama(cfg, device=gpu, seed=3).eval(), [], []
+    for hooks in (False, True):
+        if hooks:
+            for layer in m.layers:
+                for lin in (layer.wo, layer.wd):
+                    lin.register_forward_pre_hook(lambda mod, x: calls.append(mod))
+        eng = Engine(m, max_batch=batch, max_seq=256, use_graphs=False)
+        slots = [eng.acquire() for _ in range(batch)]
+        eng.prefill_batch(slots, [[1, 2, 3 + i] for i in range(batch)])
+        del calls[:]
+        outs.append(eng.decode(slots, torch.arange(batch)).float().clone())
+    assert len(calls) == 2 * cfg.n_layers
+    assert float((outs[0] - outs[1]).norm() / outs[0].norm()) < 2e-2

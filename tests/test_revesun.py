@@ -357,6 +357,18 @@ def test_the_residual_that_a_tap_sees_is_the_next_norms(gpu, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [3, 12])
+def test_hooks_of_output_projections_see_every_call(gpu, n):
+    """Forward hooks on wo and wdown, at rows whose outputs come in parts and at others."""
+    model, calls = parts_model(gpu), []
+    for layer in model.layers[1:]:
+        for lin in (layer.wo, layer.wdown):
+            lin.register_forward_hook(lambda m, x, y: calls.append(y.shape))
+    want = model.hidden_states(torch.tensor([tokens(n, 128, n)], device=gpu))
+    assert calls == [(n, 512)] * 4 and torch.isfinite(want).all()
+
+
+@pytest.mark.gpu
 def test_parts_go_past_the_norm_prologues(gpu, monkeypatch):
     """MXLLM_SKINNY_M and MXLLM_NORM_FUSED_M of 16: projections with the norm in their prologue behind outputs in parts, against
     the steps without the settings (other kernels, so to rounding)."""
