@@ -232,6 +232,10 @@ class SigusunLayer(nn.Module):
         self.side_norm = f32(h, value=1.0)
 
 
+def _refresh_loaded(model, incompatible) -> None:
+    model.refresh()
+
+
 class Sigusun(nn.Module):
     serves_float32 = True  # every kernel has an f32 form
     native_component = "serve"  # the part of the native library it needs (mxllm/_build.py)
@@ -264,6 +268,7 @@ class Sigusun(nn.Module):
         if init:
             self.reset_parameters(seed)
         self.requires_grad_(False)
+        self.register_load_state_dict_post_hook(_refresh_loaded)
 
     @torch.no_grad()
     def reset_parameters(self, seed: int = 0):
@@ -285,6 +290,7 @@ class Sigusun(nn.Module):
                     fan_in(getattr(layer, name))
             if getattr(layer, "sink", None) is not None:
                 layer.sink.normal_(0.0, 1.0, generator=gen)
+        self.refresh()
 
     @property
     def head_weight(self) -> torch.Tensor:
@@ -293,10 +299,22 @@ class Sigusun(nn.Module):
     def prepare(self, max_seq: int) -> None:
         """Build what decoding derives once (its storage must not move under a captured graph): rotation tables,
         and in bf16 the key weights transposed."""
-        for s, layer in zip(self.cfg.layers, self.layers):
+        for s in self.cfg.layers:
             self.tables.get(*s.rot, max_seq)
-            if s.lat and layer.wuk_t is None and layer.wkv.is_cuda and self.dtype == torch.bfloat16:
-                layer.wuk_t = lops.key_weight(layer.wkv.data, s.lat)
+        self.refresh(True)
+
+    @torch.no_grad()
+    def refresh(self, make: bool = False) -> None:
+        """Derive the transposed key weights again, in their storage: after the parameters were written (loading a state dict,
+        ``reset_parameters`` and ``prepare`` do it themselves).  ``make``: those that are not there yet too."""
+        for s, layer in zip(self.cfg.layers, self.layers):
+            if not s.lat or not layer.wkv.is_cuda or self.dtype != torch.bfloat16 or (layer.wuk_t is None and not make):
+                continue
+            t = lops.key_weight(layer.wkv.data, s.lat)
+            if layer.wuk_t is None or layer.wuk_t.device != t.device:
+                layer.wuk_t = t
+            else:
+                layer.wuk_t.copy_(t)
 
     # ------------------------------------------------------------------ the layer stack
     def _mixer(self, i: int, x: torch.Tensor, rows, n: int, latents: dict) -> torch.Tensor:

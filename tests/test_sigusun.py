@@ -952,6 +952,42 @@ def test_decode_follows_a_side_projection_written_in_place(built, gpu, graphs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("way", ["load_state_dict", "reset_parameters", "second engine"])
+def test_decode_follows_new_weights(built, gpu, graphs, way):
+    """All weights new in their storage, after steps (and a graph of them) with the old: decode's transposed key weights are the
+    new ones', and the steps have the bits of a model that had these weights from the start."""
+    prompts, feed = [tokens(9, 128, 1), tokens(40, 128, 2)], [[5, 6], [7, 8], [9, 1]]
+    model, other = (built("wide", gpu, torch.bfloat16)[2] for _ in range(2))
+    other.reset_parameters(5)
+
+    def engine(m):
+        eng = Engine(m, max_batch=2, max_seq=128, use_graphs=graphs, kv_pool_tokens=512)
+        slots = [eng.acquire() for _ in prompts]
+        for s, p in zip(slots, prompts):
+            eng.extend(s, len(p) + 8)
+        return eng, slots
+
+    def steps(eng, slots):
+        eng.prefill_batch(slots, prompts)
+        return torch.stack([eng.decode(slots, torch.tensor(t)).float().clone() for t in feed])
+
+    want = steps(*engine(other))
+    run = engine(model)
+    before = steps(*run)
+    if way == "load_state_dict":
+        model.load_state_dict(other.state_dict())
+    elif way == "reset_parameters":
+        model.reset_parameters(5)
+    else:
+        for p, q in zip(model.parameters(), other.parameters()):
+            p.copy_(q)
+        engine(model)
+    got = steps(*run)
+    assert not torch.equal(before, want) and torch.equal(got, want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16], ids=str)
 def test_large_decode_batches(built, gpu, dt):
     """More sequences than the decode kernels of the experts take at once, against the oracle."""
