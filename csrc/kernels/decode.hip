@@ -430,7 +430,13 @@ __global__ void __launch_bounds__(D) decode_combine_kernel(const float* __restri
 // 48 of 60 to 600 21.4 -> 18.8, 32 of 100 to 1,000 25.5 -> 20.6, 7 of 2,500 21.7 -> 18.8.  Heads of 64, at
 // half the bytes a key, do not gain (14.1 -> 14.1, 11.4 -> 13.6) and keep their splits.
 //
-// Scores, weights and sums are those of decode_split_body; a wave keeps a running maximum.
+// Level or slower where the sequences are alike and end with a split, over four turns and more, where nothing is uneven: 64 of 1,024
+// keys 60.5 -> 64.2, of 2,048 116 -> 127, 128 of 1,024 117 -> 126; but 32 of 2,080 67 -> 61, 64 of 1,000 to 2,048 105 -> 96.  Long
+// ones gain most, whose merge is then of as many parts as shares (1 of 32,768 78 -> 42, 8 of 16,384 144 -> 111).
+//
+// Scores, weights and sums are those of decode_split_body; a wave keeps a running maximum.  Where a row is cut follows from the
+// lengths of all rows and its place among them, so the order of its sums, and with it the last bits of its outputs, may differ
+// from batch to batch (the same call has the same bits; a row of fixed splits has its own whatever the others are).
 constexpr int kEvenD = 128, kEvenPlaces = 512;  // two workgroups a CU
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 

@@ -1148,6 +1148,31 @@ def test_decode_attn_up_to_512_keys(gpu, D, Hq, Hkv):
 
 
 @pytest.mark.gpu
+def test_decode_attn_dealt_evenly_among_other_rows(gpu):
+    """A row's cuts depend on the rows beside it: moved among them, and with others of other lengths, its output differs by
+    the rounding of the softmax weights to bf16 against another maximum (2^-9 of each) and the output's own (2^-9), and
+    the same call has the same bits."""
+    torch.manual_seed(11)
+    Hq, Hkv, D, B, room = 32, 8, 128, 24, 2048
+    kc, vc = (torch.randn(B, Hkv, room, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+    lens = torch.randint(200, room + 1, (B,), device=gpu).to(torch.int32)
+
+    def run(rows, n):
+        r = rows.long()
+        return _ops().decode_attn(q[r], kc, vc, n[r].contiguous(), rows, room, D ** -0.5, 0, None, None).view(-1, Hq, D)
+
+    rows = torch.arange(B, device=gpu, dtype=torch.int32)
+    want = run(rows, lens)
+    assert torch.equal(run(rows, lens), want)
+    moved = rows[torch.randperm(B, device=gpu)]
+    other = lens.clone()
+    other[::2] = torch.randint(1, room + 1, (B // 2,), device=gpu).to(torch.int32)
+    assert rel_err(run(moved, lens), want[moved.long()]) < 2 ** -7
+    assert rel_err(run(rows, other)[1::2], want[1::2]) < 2 ** -7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("Hq,Hkv,room", [(32, 8, 256), (16, 1, 512)])
 def test_decode_attn_of_few_splits_is_not_dealt(gpu, Hq, Hkv, room):
     """Many sequences of one split, or of two past 8 heads of a KV head, keep a workgroup a split (dealt evenly they took up to
