@@ -865,6 +865,8 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attn_bwd_ablate(const at::Tensor&
 // M <= 32: the fused weight-streaming kernel; otherwise dequantise to bf16 and run the
 // hipBLASLt GEMM.  mxllm/serve/quant.py calls this only up to SMALL_M (8) tokens and
 // routes larger calls to the fp8 x fp8 hipBLASLt GEMM.
+// whether w8_linear of these sizes runs on stream_gemm.hip
+bool w8_stays(int64_t M, int64_t K) { return M >= 1 && K >= 1 && M <= INT32_MAX && K <= INT32_MAX && mx_w8_stays((int)M, (int)K); }
 at::Tensor w8_linear(const at::Tensor& x, const at::Tensor& q, const at::Tensor& scale) {
   MX_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && x.dim() == 2 && x.stride(1) == 1, "x: bf16 [M, K] rows");
   MX_CHECK(q.is_cuda() && q.scalar_type() == at::kByte && q.dim() == 2 && q.is_contiguous(), "q: uint8 [N, K]");
@@ -1003,6 +1005,7 @@ TORCH_LIBRARY(mxllm, m) {
   m.def("rope_merge_bwd(Tensor dq, Tensor dkp, Tensor dvp, Tensor cos, Tensor sin, int B, int S, int Hq, int Hkv, int D, int out_pad=0) -> Tensor");
   m.def("attn_fwd(Tensor q, Tensor k, Tensor v, bool causal, float scale, int out_pad=0) -> (Tensor, Tensor)");
   m.def("w8_linear(Tensor x, Tensor q, Tensor scale) -> Tensor");
+  m.def("w8_stays(int M, int K) -> bool", &w8_stays);
   m.def("w8_dequant(Tensor q, Tensor scale) -> Tensor");
   m.def("quant_rows_e4m3(Tensor x) -> (Tensor, Tensor)");
   m.def("lora_xwt(Tensor x, Tensor v, Tensor(a!) out, float alpha, int rows=0) -> ()");

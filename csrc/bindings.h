@@ -131,6 +131,8 @@ int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, c
                    const int32_t* bt, int maxb, hipStream_t stream);
 int mx_stream_group_norm(const float* h, const uint16_t* delta, int64_t ldd, const float* gamma, float eps, float* h_out,
                          const uint16_t* w, int64_t ldw, uint16_t* y, int M, int N, int K, hipStream_t stream);
+int mx_skinny_stays(int M, int N, int K);
+int mx_w8_stays(int M, int K);
 // stream_parts.hip
 int mx_stream_parts_segments(int M, int N, int K);
 int mx_stream_parts(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, float* parts, int M, int N, int K,

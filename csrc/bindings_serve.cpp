@@ -194,6 +194,10 @@ int64_t stream_parts_segments(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
   return mx_stream_parts_segments((int)M, (int)N, (int)K);
 }
+// whether skinny_linear (skinny_linear_swiglu: N = 2 F) of these sizes runs on stream_gemm.hip
+bool skinny_stays(int64_t M, int64_t N, int64_t K) {
+  return M >= 1 && N >= 1 && K >= 1 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX && mx_skinny_stays((int)M, (int)N, (int)K);
+}
 at::Tensor stream_parts(const at::Tensor& x, const at::Tensor& w) {
   MX_CHECK(x.is_cuda() && w.is_cuda() && x.device() == w.device() && x.scalar_type() == at::kBFloat16 &&
                w.scalar_type() == at::kBFloat16 && x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.stride(1) == 1 &&
@@ -476,6 +480,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
         "Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, "
         "Tensor? block_table) -> (Tensor, Tensor)");
+  m.def("skinny_stays(int M, int N, int K) -> bool", &skinny_stays);
   m.def("stream_parts_segments(int M, int N, int K) -> int", &stream_parts_segments);
   m.def("stream_parts(Tensor x, Tensor w) -> Tensor");
   m.def("parts_norm(Tensor parts, Tensor res, Tensor w, float eps) -> (Tensor, Tensor)");

@@ -223,6 +223,9 @@ extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int
                               const int32_t* pos, const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq,
                               int Hkv, int max_seq, const int32_t* bt, int maxb, hipStream_t stream);
 
+// whether mx_w8a16_gemm hands rows of these sizes on to stream_gemm.hip
+extern "C" int mx_w8_stays(int M, int K) { return M > 2 && M <= 8 && mx_stream_ok(M, K, 0); }
+
 // X [M, K] bf16 (row stride ldx), Q [N, K] e4m3 codes, scale [N] f32 (per output channel),
 // Y [M, N] bf16 (row stride ldy).  Requires M in 1..32, N % 16 == 0, K % 512 == 0,
 // ldx a multiple of 8, ldy of 4.
@@ -247,12 +250,11 @@ extern "C" int mx_w8a16_gemm(const uint16_t* x, int64_t ldx, const uint8_t* q, c
   // 31.5 / 34.1 -> 25.3 / 34.3 / 33.0 -> 22.2 / 22.4 / 22.8).  Else the 16-row fragments, which read X half as often (4096 x 14336,
   // 8 rows 18.3 -> 21.5).
   if (!force && M <= 8) {
-    const bool fits = mx_stream_ok(M, K, 0) != 0;
-    if (fits && M > 2 &&
+    if (mx_w8_stays(M, K) &&
         mx_stream_gemm(x, ldx, q, K, scale, y, ldy, M, N, K, 0, nullptr, 0, nullptr, 0.f, nullptr, nullptr, nullptr, nullptr,
                        nullptr, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0, stream) == 0)
       return 0;
-    if (fits || M <= 2) {
+    if (M <= 2 || mx_stream_ok(M, K, 0)) {
       w8_lines_kernel<<<N / 16, 512, 0, stream>>>(x, ldx, q, scale, y, ldy, M, K);
       return (int)hipGetLastError();
     }

@@ -152,13 +152,15 @@ extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int
                               const uint16_t* gamma, float eps, uint16_t* h_out, const float* cosb, const float* sinb,
                               const int32_t* pos, const int32_t* slots, uint16_t* q, uint16_t* kc, uint16_t* vc, int Hq,
                               int Hkv, int max_seq, const int32_t* bt, int maxb, hipStream_t stream);
-static bool sk_stays(int M, int N, int K) {
-  return K == 2048 ? M > 2 : K == 4096 && M > 8 && M <= 16 && !(N > 3072 && N <= 4096);
+extern "C" int mx_stream_ok(int M, int K, int norm);
+// whether mx_skinny_gemm and mx_skinny_gemm_swiglu (N = 2 F) hand rows of these sizes on to it
+extern "C" int mx_skinny_stays(int M, int N, int K) {
+  return mx_stream_ok(M, K, 0) && (K == 2048 ? M > 2 : K == 4096 && M > 8 && M <= 16 && !(N > 3072 && N <= 4096));
 }
 // epi 0: plain, 1: SwiGLU (N = 2 F); -1: not taken
 static int sk_stream_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, uint16_t* y, int64_t ldy, int M, int N,
                           int K, int epi, hipStream_t stream) {
-  if (!sk_stays(M, N, K)) return -1;
+  if (!mx_skinny_stays(M, N, K)) return -1;
   return mx_stream_gemm(x, ldx, w, ldw, nullptr, y, ldy, M, N, K, epi, nullptr, 0, nullptr, 0.f, nullptr, nullptr, nullptr,
                         nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0, stream);
 }

@@ -599,9 +599,9 @@ def _skinny_ok(x2: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 # Where a projection goes to the workgroups that stay (csrc/kernels/stream_gemm.hip: X in LDS once a CU instead of
-# once 16 channels), as far as X fits the LDS (32 rows of 2048, 17 of 4096, 11 of 6144, 8 of 8192, 5 of 14336).  (skinny_linear
-# itself goes there too where that has the same bits and takes less time: a K of 2048 from 3 rows on, one of 4096 from 9.)
-# Weights from memory in a chain of launches:
+# once 16 channels), as far as X fits the LDS (32 rows of 2048, 17 of 4096, 11 of 6144, 8 of 8192, 5 of 14336).  (Callers of
+# skinny_linear that ask no rule get it too where it takes less time: csrc/kernels/skinny_gemm.hip mx_skinny_stays, a K of 2048
+# from 3 rows on, one of 4096 from 9.)  Weights from memory in a chain of launches:
 #  * Up to 8 rows (us, skinny -> stream): a K of 4096s, whose blocks are long, from 6144 channels on (6144 x 4096, 1 / 8 rows
 #    12.1 / 14.0 -> 12.0 / 13.0; 28672 39.8 / 42.8 -> 39.4 / 41.1; 4096 x 4096, 8 rows 8.4 -> 9.5), an LM head from 2 rows on
 #    (128256 x 4096).  Else by rows x width, the X that the other reads beside 16 channels of weights: 8192 x 6144, 8 rows
@@ -677,8 +677,9 @@ def w8_rows(x2: torch.Tensor, q: torch.Tensor, scale: torch.Tensor) -> torch.Ten
 
 
 def _decode_route(M: int, N: int, K: int) -> str:
-    """The decode GEMM of M rows of K times [N, K]: "stream" (stream_gemm.hip), "half" or "skinny" (skinny_gemm.hip, 8 or
-    16 channels a workgroup), or "" (hipBLASLt)."""
+    """The entry point of M rows of K times [N, K]: "stream" (stream_linear), "half" or "skinny" (skinny_linear_half and
+    skinny_linear, 8 or 16 channels a workgroup), or "" (hipBLASLt).  skinny_linear itself hands the sizes of
+    ``native().skinny_stays`` on to stream_gemm.hip, and w8_linear those of ``w8_stays``."""
     if _stream_wins(M, N, K):
         return "stream"
     if K % 512:

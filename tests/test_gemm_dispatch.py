@@ -93,6 +93,17 @@ def test_decode_routes(route, M, N, K):
     assert lin._decode_route(M, N, K) == route
 
 
+def test_what_the_skinny_entry_points_hand_on():
+    """Behind the routes above: sizes that skinny_linear and w8_linear run on the GEMM that stays, both sides of each line."""
+    from mxllm.ops import native
+
+    on = [(3, 48, 2048), (8, 16384, 2048), (32, 3072, 2048), (9, 48, 4096), (16, 3072, 4096), (16, 4112, 4096)]
+    off = [(2, 16384, 2048), (8, 3072, 4096), (9, 3088, 4096), (16, 4096, 4096), (17, 1024, 4096), (8, 3072, 3072), (12, 2048, 8192)]
+    assert [s for s in on if not native().skinny_stays(*s)] == [] and [s for s in off if native().skinny_stays(*s)] == []
+    assert all(native().w8_stays(*s) for s in ((3, 2048), (8, 4096), (5, 14336)))
+    assert not any(native().w8_stays(*s) for s in ((2, 4096), (9, 2048), (4, 4608), (6, 14336)))
+
+
 def test_swiglu_route_of_decode_rows():
     """With SwiGLU in the epilogue the GEMM that stays gains from fewer channels on, and past 16 rows at any."""
     wins = sys.modules["mxllm.ops.linear"]._stream_wins
