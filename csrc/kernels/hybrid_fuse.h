@@ -1,5 +1,4 @@
-// Operands and epilogues of the fused decode GEMMs of the recurrent / chunked-attention decoders (hybrid_skinny.hip,
-// hybrid_stream.hip).
+// Operands and epilogues of the fused decode GEMMs of the recurrent / chunked-attention decoders (hybrid_skinny.hip).
 #pragma once
 
 #include "conv_rope.h"

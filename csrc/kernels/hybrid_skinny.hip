@@ -185,14 +185,15 @@ struct HsRun {
   int64_t ldy;
   int M, K;
 };
-template <int PRO, int EPI>
+template <int PRO, int EPI, int ROWS = 16>
 static void hs_launch(const HsRun& r, const HsNorm& na, const HsPoly& pp, const HsGru& gr, const HsConv& cv, hipStream_t stream) {
-#define HS_RUN(TB, KP) \
-  hybrid_skinny_kernel<PRO, EPI, TB, KP><<<r.groups, 512, r.lds, stream>>>(r.x, r.ldx, r.w, r.ldw, r.y, r.ldy, r.M, r.K, na, pp, gr, cv)
+  constexpr int TB = ROWS > 8 ? 2 : 1;
+#define HS_RUN(TBV, KP) \
+  hybrid_skinny_kernel<PRO, EPI, TBV, KP><<<r.groups, 512, r.lds, stream>>>(r.x, r.ldx, r.w, r.ldw, r.y, r.ldy, r.M, r.K, na, pp, gr, cv)
   if (sk_parts(r.M, r.K) == 4) {
-    if (r.M <= 8) HS_RUN(1, 4); else HS_RUN(2, 4);
+    if (r.M <= 8) HS_RUN(1, 4); else HS_RUN(TB, 4);
   } else {
-    if (r.M <= 8) HS_RUN(1, 8); else HS_RUN(2, 8);
+    if (r.M <= 8) HS_RUN(1, 8); else HS_RUN(TB, 8);
   }
 #undef HS_RUN
 }
@@ -227,12 +228,12 @@ extern "C" int mx_hs_norm_gemm(const uint16_t* delta, int64_t ldd, const float* 
   return (int)hipGetLastError();
 }
 
-// y [M, N] = poly_norm(z) . w^T
+// y [M, N] = poly_norm(z) . w^T, up to 8 rows
 extern "C" int mx_hs_poly_gemm(const uint16_t* z, int64_t ldz, const float* coef, float eps, const uint16_t* w,
                                int64_t ldw, uint16_t* y, int64_t ldy, int M, int N, int K, hipStream_t stream) {
   if (M <= 0) return 0;
-  if (hs_check(z, ldz, ldw, M, K, N) || (int64_t)M * K > 32768 || N % 16 || ldy % 4 || ldy < N) return -1;
-  hs_launch<kProPoly, kEpiPlain>({N / 16, (size_t)M * K * 2, z, ldz, w, ldw, y, ldy, M, K}, {}, HsPoly{coef, eps}, {}, {}, stream);
+  if (M > 8 || hs_check(z, ldz, ldw, M, K, N) || (int64_t)M * K > 32768 || N % 16 || ldy % 4 || ldy < N) return -1;
+  hs_launch<kProPoly, kEpiPlain, 8>({N / 16, (size_t)M * K * 2, z, ldz, w, ldw, y, ldy, M, K}, {}, HsPoly{coef, eps}, {}, {}, stream);
   return (int)hipGetLastError();
 }
 

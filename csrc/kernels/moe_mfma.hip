@@ -5,7 +5,8 @@
 //   * moe_few_up / moe_few_down : up to 64 tokens (decode steps): every workgroup finds its expert's pairs
 //                      among the choices and streams 16-channel slices of the weights past them; the
 //                      shared expert's slices run in the same launch.  Weights are read once for up to 64
-//                      rows; experts nobody chose are not read.
+//                      rows; experts nobody chose are not read, but for the first chunks of their down weights where
+//                      these are asked for before the choices (FewLines).
 #include "e4m3.h"
 #include "gemm8_core.h"
 #include "hybrid.h"
@@ -183,18 +184,18 @@ struct FewSlices {
 };
 
 // The same slices for a few rows each, in the fragments of skinny_core.h: loads of 8 rows x 128 B, nontemporal, products of 8
-// token rows with two useful blocks.  K in blocks of as many chunks as a wave's part has or twice that: loads past its end,
-// repeated ones, cost as others do (down, 6 chunks in two parts, blocks of 4 13.6 us, of 3 11.8).  The first U chunks of a wave's part are
-// asked for before the rows are known.  K a multiple of 64, offsets of 32 bits.
-template <bool GLU, int KW, int NC, int UC>
+// token rows with two useful blocks.  A wave's part of K is whole blocks of U chunks (loads past its end would cost as others do:
+// 6 chunks in two parts, blocks of 4 13.6 us, of 3 11.8); the first is asked for before the rows are known.  Down products alone;
+// offsets of 32 bits.
+template <int KW, int NC, int UC>
 struct FewLines {
-  static constexpr int SL = 8 / KW * NC, CH = GLU ? 8 : 16, RB = 2 * NC, U = UC;  // block 2 j: gate rows, or rows 0 .. 7
+  static constexpr int SL = 8 / KW * NC, CH = 16, RB = 2 * NC, U = UC;
   static constexpr int places(int rows) { return 8 * RB * 16 * ((rows + 7) / 8); }
   typedef uint32_t Off;  // of X's rows
   typedef u32x4 Frag[U][RB];  // (as vectors of 16 bits they come apart where paths join)
   const char* W;
   uint32_t wo[RB];
-  int n0, c0, c1, cl, ks;  // chunks of 64 k: this wave's, the last of all
+  int n0, c0, c1, ks;  // this wave's chunks of 64 k
   Frag pre;
 
   __device__ __forceinline__ FewLines(const uint16_t* w_, int bx, int N, int K, int w, int lane) {
@@ -202,18 +203,19 @@ struct FewLines {
     W = reinterpret_cast<const char*>(w_);
     ks = w % KW;
     n0 = (bx * SL + w / KW * NC) * CH;
-    const int steps = K / 64, per = (steps + KW - 1) / KW;
-    c0 = ks * per, c1 = min(steps, c0 + per), cl = steps - 1;
+    const int per = K / 64 / KW;
+    c0 = ks * per, c1 = c0 + per;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
-      const int ch = n0 + (rb >> 1) * CH + (GLU ? 0 : 8 * (rb & 1)) + (c & 7);
-      wo[rb] = ((uint32_t)((GLU && (rb & 1) ? N : 0) + min(ch, N - 1)) * (uint32_t)K + (uint32_t)sk_lane_k(c, g)) * 2;
+      const int ch = n0 + (rb >> 1) * CH + 8 * (rb & 1) + (c & 7);
+      wo[rb] = ((uint32_t)min(ch, N - 1) * (uint32_t)K + (uint32_t)sk_lane_k(c, g)) * 2;
     }
   }
+  // (readfirstlane: a scalar base and 32-bit offsets; left alone the loop keeps 64-bit addresses a lane, 12 registers and a wave less)
   __device__ __forceinline__ void load(Frag& f, int c) const {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const char* p = W + 128 * (int64_t)min(c + u, cl);
+      const char* p = W + 128 * (int64_t)__builtin_amdgcn_readfirstlane(c + u);
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) f[u][rb] = sk_weights<u32x4>(p + wo[rb]);
     }
@@ -243,13 +245,9 @@ struct FewLines {
           u32x4 fb[UX][TB];
 #pragma unroll
           for (int u = 0; u < UX; ++u) {
-            const int cu = cb + u0 + u;
-            const char* p = reinterpret_cast<const char*>(xb) + 128 * (int64_t)min(cu, cl);
+            const char* p = reinterpret_cast<const char*>(xb) + 128 * (int64_t)__builtin_amdgcn_readfirstlane(cb + u0 + u);
 #pragma unroll
-            for (int tb = 0; tb < TB; ++tb) {
-              fb[u][tb] = *reinterpret_cast<const u32x4*>(p + xo[tb]);
-              if (cu >= c1) fb[u][tb] = u32x4{0, 0, 0, 0};
-            }
+            for (int tb = 0; tb < TB; ++tb) fb[u][tb] = *reinterpret_cast<const u32x4*>(p + xo[tb]);
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -290,17 +288,9 @@ struct FewLines {
           s += red[at(w - ks + i, 2 * j + (g >> 1), min(tb, TB - 1)) + 8 * (g & 1) + (c & 7)];
         const int r = r0 + 16 * mb + c, ch = n0 + j * CH + 4 * g;
         u16x4 o;
-        if constexpr (GLU) {  // gate in groups 0 and 1, up in 2 and 3
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float up = __shfl_xor(s[i], 32, 64);
-            o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, limit));
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
-        }
-        if (tb < TB && r < n && ch < N && (!GLU || g < 2)) *reinterpret_cast<u16x4*>(y + (int64_t)yrow(r) * N + ch) = o;
+        for (int i = 0; i < 4; ++i) o[i] = f2bf(s[i]);
+        if (tb < TB && r < n && ch < N) *reinterpret_cast<u16x4*>(y + (int64_t)yrow(r) * N + ch) = o;
       }
     };
     int r0 = 0;
@@ -483,10 +473,10 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
   } else if (pairs <= 8) {
     MF(false, FS(false, 4, 1), 16, 16, FS(false, 8, 1), 16, 16);
   } else if (lines) {
-    if (a.T <= 8) MF(false, FL(false, 2, 1, 3), 8, 8, FL(false, 8, 1, 4), 8, 8);
-    else if (a.T <= 16) MF(false, FL(false, 2, 1, 3), 16, 8, FL(false, 8, 1, 4), 16, 16);
-    else if (a.T <= 32) MF(false, FL(false, 2, 1, 3), 16, 8, FS(false, 8, 1), 32, 32);
-    else MF(false, FL(false, 2, 1, 3), 32, 16, FS(false, 8, 1), 64, 64);
+    if (a.T <= 8) MF(false, FL(2, 1, 3), 8, 8, FL(8, 1, 4), 8, 8);
+    else if (a.T <= 16) MF(false, FL(2, 1, 3), 16, 8, FL(8, 1, 4), 16, 16);
+    else if (a.T <= 32) MF(false, FL(2, 1, 3), 16, 8, FS(false, 8, 1), 32, 32);
+    else MF(false, FL(2, 1, 3), 32, 16, FS(false, 8, 1), 64, 64);
   } else {
     if (a.T <= 16) MF(false, FS(false, 2, 1), 16, 16, FS(false, 8, 1), 16, 16);
     else if (a.T <= 32) MF(false, FS(false, 2, 1), 32, 16, FS(false, 8, 1), 32, 32);

@@ -279,9 +279,9 @@ extern "C" int mx_skinny_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w,
   while (nc > 1 && (N % (16 * nc) || N / (16 * nc) < 128)) nc >>= 1;
 #define SKG(TBV, NCV, KPV) \
   skinny_gemm_kernel<TBV, NCV, KPV><<<N / (16 * NCV), 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K)
-#define SKT(NCV, KPV) \
+#define SKT(NCV, KPV) /* 4 K parts: up to 16 rows */ \
   do { \
-    if (M <= 8) SKG(1, NCV, KPV); else if (M <= 16) SKG(2, NCV, KPV); else SKG(4, NCV, KPV); \
+    if (M <= 8) SKG(1, NCV, KPV); else if (M <= 16) SKG(2, NCV, KPV); else SKG(KPV == 4 ? 2 : 4, NCV, KPV); \
   } while (0)
   // up to two workgroups a CU (us, compiler's order -> DEEP, one row: 4096 x 4096 7.7 -> 7.6, 4096 x 14336 23.1 -> 21.9; 128256 x
   // 2048 82 -> 88)
@@ -294,7 +294,7 @@ extern "C" int mx_skinny_gemm(const uint16_t* x, int64_t ldx, const uint16_t* w,
   }
 #define SKC(KPV) \
   do { \
-    if (nc >= 4) SKT(4, KPV); else if (nc == 2) SKT(2, KPV); else SKT(1, KPV); \
+    if (nc >= 4) SKT(4, KPV); else if (nc == 2) SKT(2, KPV); else if (M <= 8) SKG(1, 1, KPV); else SKG(2, 1, KPV); \
   } while (0)
   if (sk_wide(M, K) && nc == 1) {
     if (M <= 16) skinny_gemm_kernel<1, 1, 8, false, false, false, false, false, true><<<N / 16, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
@@ -335,7 +335,7 @@ extern "C" int mx_skinny_gemm_swiglu(const uint16_t* x, int64_t ldx, const uint1
 #define SKS(TBV, KPV) skinny_gemm_kernel<TBV, 1, KPV, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F)
 #define SKT(KPV) \
   do { \
-    if (M <= 8) SKS(1, KPV); else if (M <= 16) SKS(2, KPV); else SKS(4, KPV); \
+    if (M <= 8) SKS(1, KPV); else SKS(2, KPV); \
   } while (0)
   if (sk_wide(M, K)) {
     if (M <= 16) skinny_gemm_kernel<1, 1, 8, true, false, false, false, false, true><<<F / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K, F);
