@@ -13,8 +13,8 @@
 //
 // Split form (vocabularies of kSplitV and more): three launches over (chunk, row), so a step's few rows fill the
 // chip.  One workgroup a row kept 32 of 256 CUs on six to nine passes whose LDS atomics and logarithms bound it:
-// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the three launches take 35 us (stats 6, hist
-// 11, pick 17; all top-p 33, all top-k 25, temperature alone 20).  What bounds them now: dependent steps inside each
+// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the three launches take 35 us by themselves (profiled:
+// stats 6, hist 11, pick 17; all top-p 33, all top-k 25, temperature alone 20) and 31 us a call behind one another.  What bounds them now: dependent steps inside each
 // launch (row parameters, the chunks' partials, scans over bins, the counter of a row), and for few rows the host's
 // three launches (22 - 25 us a call).
 //  * stats: a chunk's largest (with its index) and smallest logit;

@@ -747,7 +747,9 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # norm adds.  With the norm, us, 9 / 16 / 24 / 32 rows: 4096 x 14336 29.1 / 30.7 / 33.7 / 35.5 -> 25.1 / 26.5 / 30.9 / 31.8; 2048 x
 # 8192 16.0 / 16.1 / 16.8 / 19.0 -> 12.8 / 13.6 / 14.9 / 15.6; 2048 x 12288 22.0 / 21.7 / 21.9 / 26.2 -> 15.3 / 15.6 / 17.2 / 17.4; 8192 x
 # 28672, 9 / 16 rows 97.0 / 98.7 -> 80.8 / 82.7, but 24 101.9 -> 105.2.  A K of 4096 past 16 rows, where it is too long as
-# well: 4096 x 4096, 17 / 32 rows 16.9 / 17.1 -> 14.7 / 16.3, not before (16 rows 13.3 -> 14.2).
+# well: 4096 x 4096, 17 / 32 rows 16.9 / 17.1 -> 14.7 / 16.3, not before (16 rows 13.3 -> 14.2).  Not in between, though up to 5120
+# channels most of it gains as well (9 / 32 rows, 4096 x 4608 21.5 / 18.2 -> 14.7 / 16.6, 4096 x 6144 26.7 / 22.1 -> 16.1 / 17.7, 4096 x
+# 7680 18.9 / 22.8 -> 19.5 / 21.4; 8192 x 4608 22.7 / 24.0 -> 22.5 / 25.0).
 def _parts_wins(M: int, N: int, K: int) -> bool:
     if not 8 < M <= min(32, _DECODE_M) or K % 512 or N % 64 or N > 8192:
         return False
