@@ -175,6 +175,33 @@ at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool 
   return out;
 }
 
+// a b^T (bf16) for any number of rows, a [M, K], b [N, K], or silu(gate) up [M, N / 2] of b = [gate; up]: tile `tile` with K in
+// `parts` (mx_gemm_tile; callers ask gemm_tile_plan and mxllm/ops/gemm.py rows_ok first).
+at::Tensor gemm_tile(const at::Tensor& a, const at::Tensor& b, bool swiglu, int64_t tile, int64_t parts) {
+  MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm_tile: GPU tensors of one device");
+  MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm_tile: bf16 operands");
+  MX_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == b.size(1), "gemm_tile: a [M, K], b [N, K]");
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(0);
+  MX_CHECK(a.stride(1) == 1 && b.stride(1) == 1 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX,
+           "gemm_tile: row-major operands");
+  MX_CHECK(parts >= 1 && (parts == 1 || parts <= K / 64), "gemm_tile: parts of at least 64 of K");
+  DevGuard g(a.device());
+  auto out = at::empty({M, swiglu ? N / 2 : N}, a.options());
+  at::Tensor ws;
+  if (parts > 1) ws = at::empty({parts * M * N}, a.options().dtype(at::kFloat));
+  const int rc = mx_gemm_tile(bf(a), a.stride(0), bf(b), b.stride(0), bfm(out), out.stride(0), (int)M, (int)N, (int)K, swiglu ? 1 : 0,
+                              (int)tile, (int)parts, parts > 1 ? ws.data_ptr<float>() : nullptr, cur_stream());
+  MX_CHECK(rc != -1, "gemm_tile: shape, stride or alignment not taken");
+  MX_OK(rc);
+  return out;
+}
+
+// (tile, parts) of K for a product as 64 tile + parts; -1: not a size for gemm_tile
+int64_t gemm_tile_plan(int64_t M, int64_t N, int64_t K, bool swiglu) {
+  if (M < 1 || N < 1 || K < 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return -1;
+  return mx_gemm_tile_plan((int)M, (int)N, (int)K, swiglu ? 1 : 0);
+}
+
 // y = [swiglu](x . w^T); with gamma x = rmsnorm(h + delta), up to 4 rows.  Returns (y, h + delta).
 std::tuple<at::Tensor, at::Tensor> stream_linear(const at::Tensor& x, const c10::optional<at::Tensor>& delta,
                                                  const c10::optional<at::Tensor>& gamma, double eps, const at::Tensor& w,
@@ -476,6 +503,8 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("decode_attn_partials(Tensor q, Tensor k_cache, Tensor v_cache, Tensor lens, Tensor? slots, int max_len, float scale, int len_off=0, Tensor? block_table=None) -> (Tensor, Tensor)");
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
   m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
+  m.def("gemm_tile(Tensor a, Tensor b, bool swiglu, int tile, int parts) -> Tensor");
+  m.def("gemm_tile_plan(int M, int N, int K, bool swiglu) -> int", &gemm_tile_plan);
   m.def("stream_linear(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, bool swiglu) -> (Tensor, Tensor)");
   m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
         "Tensor sin, Tensor pos, Tensor? slots, Tensor(a!) k_cache, Tensor(b!) v_cache, int Hq, int Hkv, "
@@ -501,6 +530,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("skinny_merge_linear", &skinny_merge_linear);
   m.impl("decode_attn", &decode_attn);
   m.impl("gemm8_rows", &gemm8_rows);
+  m.impl("gemm_tile", &gemm_tile);
   m.impl("stream_linear", &stream_linear);
   m.impl("stream_parts", &stream_parts);
   m.impl("parts_norm", &parts_norm);

@@ -2,43 +2,6 @@
 // training batches.
 #include "gemm8_core.h"
 
-namespace mx {
-
-// Sum of the S fp32 part images [M][N] of P in their order -> bf16 C [M][N]; GLU: N = 2F, C [M][F] = silu(gate) up of
-// the sums rounded to bf16.  Bound by the images' bytes (the last level cache holds them: at most one 256 x 256 tile a CU).
-template <bool GLU>
-__global__ void __launch_bounds__(256) g8_parts_kernel(const float* __restrict__ P, int64_t part, int S, int N,
-                                                       uint16_t* __restrict__ C, int64_t ldc, int64_t units) {
-  const int F = GLU ? N / 2 : N, per = F / 8;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < units; i += (int64_t)gridDim.x * 256) {
-    const int64_t m = i / per;
-    const int n = (int)(i - m * per) * 8;
-    const float* p = P + m * N + n;
-    f32x4 a[GLU ? 4 : 2];
-#pragma unroll
-    for (int h = 0; h < (GLU ? 4 : 2); ++h) a[h] = *reinterpret_cast<const f32x4*>(p + 4 * (h & 1) + (h >> 1) * F);
-#pragma unroll 4
-    for (int s = 1; s < S; ++s) {
-#pragma unroll
-      for (int h = 0; h < (GLU ? 4 : 2); ++h)
-        a[h] += *reinterpret_cast<const f32x4*>(p + s * part + 4 * (h & 1) + (h >> 1) * F);
-    }
-    u16x8 o;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float v = a[j >> 2][j & 3];
-      if constexpr (GLU) {
-        const float g = g8_rbf(v);
-        v = g * g8_sigmoid(g) * g8_rbf(a[2 + (j >> 2)][j & 3]);
-      }
-      o[j] = f2bf(v);
-    }
-    *reinterpret_cast<u16x8*>(C + m * ldc + n) = o;
-  }
-}
-
-}  // namespace mx
-
 using namespace mx;
 
 // Any number of rows: C[M, N] = A op(B) with A [M][K] and B [N][K] (b_kc) or [K][N], or, swiglu (B = [gate; up], b_kc),

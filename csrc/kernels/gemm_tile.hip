@@ -1,0 +1,320 @@
+// bf16 GEMMs whose output is one turn of tiles: C[M, N] = A[M, K] . B[N, K]^T, any number of rows, f32 sums; with SwiGLU (B =
+// [gate; up], F rows each) C[M, F] = silu(gate) up.  Projections of prompt passes past the decode GEMMs' 32 rows.
+//
+// What bounds these products is not the matrix cores' rate but how many CUs have a tile and how long a tile waits: gemm8's 256 x
+// 256 tiles leave most CUs of a short prompt without one, and a long walk over K behind one tile is as long as its
+// loads' latency.  Here the tile fits the output (64 x 64 to 192 x 192, at most one a CU, two of the smallest), and where even that
+// leaves CUs idle K is cut in parts, whose f32 images a second launch adds in order.  mx_gemm_tile_plan picks both.
+//  * A and B by LDS-DMA (gemm8_core.h: images of 128-B rows, their 16-B chunks XOR-permuted at the source, so that the
+//    MFMA-operand reads are free of bank conflicts), S K-tiles of 64 in LDS;
+//  * a wave's fragments are read one step of 32 k ahead of their MFMAs, in two register sets, between the MFMAs of the step before
+//    (counted lgkmcnt waits: a row of MFMAs waits for its own fragments only); so are the DMA pieces, spread over both steps;
+//  * one barrier a K-tile, a quarter into its second step, when the reads of that stage are long done: behind it the next
+//    tile is read and tile kt + S asked for.  Wherever LDS allows it is asked for S - 1 tiles ahead of its use; past K the
+//    loads are out of the descriptor's range and write zeros into a stage that nobody reads, so every wait has one count;
+//  * 8 waves (two a SIMD) where the tile can be dealt to them, 4 where it cannot: 128 x 256, K 4096, few tiles: 36.8 against 39.6 us.
+// us, weights from memory, hipBLASLt (or gemm8, K in parts, marked *) -> here:
+//   2048 x 2048 at 48 / 330 / 1024 / 2709 / 4096 rows 8.7 / 11.1 / 17.4 / 27.8 / 33.4 -> 7.8 / 8.9 / 15.9 / 23.8 / 30.3
+//   3072 x 2048 at 48 / 256 / 1024 / 2709 11.7 / 13.2 / 24.5 / 42 -> 9.2 / 11.8 / 21.1 / 32
+//   2048 x 8192 at 64 / 330 / 1024 / 2709 23.1 / 31.9 / 55.1 / 95 -> 13.2 / 26.5 / 42.7 / 82
+//   4096 x 4096 at 48 / 128 / 1024 / 2048 13.8 / 24.8 / 42.1 / 60 -> 12.0 / 16.7 / 38.9 / 54
+//   4096 x 14336 at 48 / 64 / 256 36.9 / 35.0* / 60.3* -> 27.8 / 28.3 / 47.6;  8192 x 512 at 128 / 1024 1.8 and 1.2 times as fast.
+// Left: 2709 rows of 2048 x 8192 run at 1.1 PF/s.  A CU alone has its 128 x 192 x 64 step in 0.44 us, 242 of them at once in 0.6: the
+// L2's 15 TB/s (40 KB a step and CU) and the clock under load.
+#include <algorithm>
+
+#include "gemm8_core.h"
+
+namespace mx {
+
+constexpr int kGtPlain = 0, kGtSwiglu = 1, kGtPart = 2;
+
+template <int N>
+__device__ __forceinline__ void gt_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+
+// row of B behind virtual column v of tile pn: with SwiGLU a wave's first half of columns are gate's, the second the same
+// channels of up
+template <int TN, int WN, int EPI>
+__device__ __forceinline__ int gt_row(int v, int pn, int F) {
+  if constexpr (EPI != kGtSwiglu) return pn * TN + v;
+  constexpr int HW = TN / WN / 2;
+  const int q = v % (2 * HW);
+  return (q < HW ? 0 : F) + pn * (TN / 2) + v / (2 * HW) * HW + q % HW;
+}
+
+// TM x TN tile by WM x WN waves, S stages of LDS, OCC workgroups a CU (a launch bound: 256 registers a wave at 2).  kGtPart: C is
+// f32 [parts][M][N].
+template <int TM, int TN, int WM, int WN, int S, int OCC, int EPI>
+__global__ void __launch_bounds__(64 * WM * WN, OCC)
+gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, void* __restrict__ C,
+                 int64_t ldc, int M, int N, int K, int parts) {
+  constexpr int NW = WM * WN, BI = TM / WM / 16, BJ = TN / WN / 16, STG = (TM + TN) * 128;
+  constexpr int QA = TM / 8 / NW, QB = TN / 8 / NW, P = QA + QB;  // DMA pieces of 8 rows of a wave: of A, of B
+  constexpr int NM = BI * BJ, NR = BI + BJ;                      // MFMAs and fragments of a step
+  constexpr int NB = NM / 4 < NM - NR ? NM / 4 : NM - NR;        // MFMAs of the second step ahead of the barrier
+  constexpr int R0 = NM >= 2 * NR ? 2 : 1, R1 = NM - NB >= 2 * NR ? 2 : 1;         // MFMAs from one fragment read to the next
+  constexpr int D0 = NM / (P - P / 2), D1 = (NM - NB) / (P / 2);  // and from one DMA piece to the next
+  static_assert(TM % (8 * NW) == 0 && TN % (8 * NW) == 0 && BJ % 2 == 0 && S >= 3 && NB >= 0 && D0 > 0 && D1 > 0, "tile");
+  __shared__ __attribute__((aligned(1024))) char smem[S * STG];
+  const int nM = (M + TM - 1) / TM, nN = (N + TN - 1) / TN, F = N / 2;
+  int pm, pn, nk = K / 64;
+  {
+    int L = xcd_remap(blockIdx.x, gridDim.x);
+    if constexpr (EPI == kGtPart) {  // parts after each other: an XCD's tiles share the panels of one part of K
+      const int kp = L / (nM * nN), t0 = nk * kp / parts, t1 = nk * (kp + 1) / parts;
+      L -= kp * nM * nN;
+      A += t0 * 64;
+      B += t0 * 64;
+      K -= t0 * 64;
+      nk = t1 - t0;
+      C = reinterpret_cast<float*>(C) + (int64_t)kp * M * N;
+    }
+    constexpr int GM = 8;  // a band of 8 tiles down, then across: an XCD's tiles share their panels in its L2
+    const int per = GM * nN, grp = L / per, first = grp * GM;
+    const int rows = min(GM, nM - first), in = L - grp * per;
+    pm = first + in % rows;
+    pn = in / rows;
+  }
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w / WN, wn = w % WN;
+  // rows past M and N read the last one again: their products are not stored
+  const int mrem = M - pm * TM;
+  const uint16_t* ab = A + (int64_t)pm * TM * lda;
+  const uint16_t* bb = B + (EPI == kGtSwiglu ? 0 : (int64_t)pn * TN * ldb);
+  const int brows = EPI == kGtSwiglu ? N : min(N - pn * TN, TN);
+  const __amdgpu_buffer_rsrc_t ars =
+      __builtin_amdgcn_make_buffer_rsrc((void*)ab, 0, (uint32_t)(((min(mrem, TM) - 1) * lda + K) * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t brs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)bb, 0, (uint32_t)(((brows - 1) * ldb + K) * 2), 0x00020000);
+  uint32_t off[P];
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    const int r = 8 * (j < QA ? w * QA + j : w * QB + j - QA) + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    if (j < QA) {
+      off[j] = (uint32_t)((min(r, mrem - 1) * lda + 8 * c) * 2);
+    } else {
+      const int b = min(gt_row<TN, WN, EPI>(r, pn, F), N - 1) - (EPI == kGtSwiglu ? 0 : pn * TN);
+      off[j] = (uint32_t)((b * ldb + 8 * c) * 2);
+    }
+  }
+  auto piece = [&](int j, uint32_t ko, char* dst) __attribute__((always_inline)) {
+    const uint32_t so = off[j] + ko;
+    char* d = dst + (j < QA ? (w * QA + j) * 1024 : TM * 128 + (w * QB + j - QA) * 1024);
+    if (j < QA) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (g8lptr_t)d, 16, so, 0, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (g8lptr_t)d, 16, so, 0, 0, 0);
+    }
+  };
+  const uint32_t lds0 = lds_addr(smem);
+  uint32_t al[2], bl[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    al[s] = lds0 + g8_kc_lane(lane, s) + wm * (TM / WM) * 128;
+    bl[s] = lds0 + g8_kc_lane(lane, s) + TM * 128 + wn * (TN / WN) * 128;
+  }
+  u16x8 fa[2][BI], fb[2][BJ];
+  f32x4 acc[BI][BJ];
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // fragment r of set s: B's first, then A's
+  auto read = [&](int s, int r, uint32_t a, uint32_t b) __attribute__((always_inline)) {
+    if (r < BJ) fb[s][r] = rd128_off(b, r * 2048);
+    else fa[s][r - BJ] = rd128_off(a, (r - BJ) * 2048);
+  };
+  // A's fragment i of set s, and with the first all of B's, are there once at most `left` younger LDS reads are not
+  auto have = [&](int s, int i, int left) __attribute__((always_inline)) {
+    lds_wait_le(left > 15 ? 15 : left);
+    pin(fa[s][i]);
+    if (i == 0) {
+#pragma unroll
+      for (int j = 0; j < BJ; ++j) pin(fb[s][j]);
+    }
+  };
+
+#pragma unroll
+  for (int t = 0; t < S; ++t)
+#pragma unroll
+    for (int j = 0; j < P; ++j) piece(j, t < nk ? (uint32_t)t * 128 : G8_OOB, smem + t * STG);
+  gt_vm_wait<(S - 1) * P>();
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) read(0, r, al[0], bl[0]);
+  int st = 0;  // stage of kt
+  for (int kt = 0; kt < nk; ++kt) {
+    const int nx = st + 1 == S ? 0 : st + 1;
+    {  // step 0: multiply set 0, read set 1; the second half of tile kt + S - 1's pieces
+      const uint32_t a1 = al[1] + st * STG, b1 = bl[1] + st * STG;
+      char* dst = smem + (st == 0 ? S - 1 : st - 1) * STG;
+      const uint32_t ko = kt > 0 && kt + S - 1 < nk ? (uint32_t)(kt + S - 1) * 128 : G8_OOB;
+#pragma unroll
+      for (int n = 0; n < NM; ++n) {
+        const int i = n / BJ, j = n % BJ, r = n / R0, d = n / D0;
+        if (j == 0) have(0, i, BI - 1 - i + min((n + R0 - 1) / R0, NR));
+        acc[i][j] = g8_mfma(fb[0][j], fa[0][i], acc[i][j]);
+        if (n % R0 == 0 && r < NR) read(1, r, a1, b1);
+        if (n % D0 == D0 - 1 && d < P - P / 2 && kt > 0) piece(P / 2 + d, ko, dst);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    {  // step 1: multiply set 1; behind the barrier read set 0 of the next tile, and the first half of tile kt + S's pieces
+      const uint32_t a0 = al[0] + nx * STG, b0 = bl[0] + nx * STG;
+      char* dst = smem + st * STG;
+      const uint32_t ko = kt + S < nk ? (uint32_t)(kt + S) * 128 : G8_OOB;
+#pragma unroll
+      for (int n = 0; n < NM; ++n) {
+        const int i = n / BJ, j = n % BJ, q = n - NB, r = q / R1, d = q / D1;
+        if (q == 0) {  // this wave's reads of stage st are done, its pieces of tile kt + 1 landed
+          lds_wait();
+          gt_vm_wait<(S - 2) * P>();
+          __builtin_amdgcn_s_barrier();
+        }
+        if (j == 0) have(1, i, q < 0 ? BI - 1 - i : 15);
+        acc[i][j] = g8_mfma(fb[1][j], fa[1][i], acc[i][j]);
+        if (q >= 0 && q % R1 == 0 && r < NR) read(0, r, a0, b0);  // (behind the last tile: bytes that are not multiplied)
+        if (q >= 0 && q % D1 == D1 - 1 && d < P / 2) piece(d, ko, dst);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    st = nx;
+  }
+  // the reads behind the last tile own their registers, and the DMA behind K its LDS, until here
+#pragma unroll
+  for (int i = 0; i < BI; ++i) have(0, i, 0);
+  gt_vm_wait<0>();
+  const int ml = pm * TM + wm * (TM / WM) + (lane & 15);
+  if constexpr (EPI == kGtPart) {
+    float* c = reinterpret_cast<float*>(C);
+    const int n0 = pn * TN + wn * (TN / WN) + 4 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+        if (ml + 16 * i < M && n0 + 16 * j < N)
+          *reinterpret_cast<f32x4*>(c + (int64_t)(ml + 16 * i) * N + n0 + 16 * j) = acc[i][j];
+  } else if constexpr (EPI == kGtSwiglu) {
+    uint16_t* c = reinterpret_cast<uint16_t*>(C);
+    const int n0 = pn * (TN / 2) + wn * (TN / WN / 2) + 4 * (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ / 2; ++j) {
+        u16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = g8_rbf(acc[i][j][e]), u = g8_rbf(acc[i][BJ / 2 + j][e]);
+          o[e] = f2bf(g * g8_sigmoid(g) * u);
+        }
+        if (ml + 16 * i < M && n0 + 16 * j < F) *reinterpret_cast<u16x4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o;
+      }
+  } else {
+    uint16_t* c = reinterpret_cast<uint16_t*>(C);
+    const int n0 = pn * TN + wn * (TN / WN) + 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; j += 2) {
+        const uint4 o = g8_pack8(acc[i][j], acc[i][j + 1]);  // lanes exchange: outside the row test
+        if (ml + 16 * i < M && n0 + 16 * j < N) *reinterpret_cast<uint4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o;
+      }
+  }
+}
+
+// The tiles, and what one of them takes (us; fitted to 10,800 runs of 29 sizes of weights at 9 to 4096 rows, 6 to 7 % off in the mean,
+// the tile so chosen 2 % behind the best one): start + steps of 64 k (step + load units / 256 + two, where two share a CU) + memory MB
+// of weights + with K in parts, sum + image MB of f32 images.
+struct GtTile {
+  int tm, tn, most;
+  float start, step, load, two, memory, sum, image;
+};
+constexpr GtTile kGtTiles[] = {
+    {64, 64, 512, 2.70f, .166f, .069f, .133f, .078f, 2.83f, .477f}, {64, 128, 256, 3.24f, .209f, .132f, 0, .093f, 2.56f, .390f},
+    {128, 128, 256, 3.48f, .333f, .199f, 0, .053f, 2.36f, .467f},   {128, 192, 256, 4.28f, .438f, .210f, 0, .059f, 1.85f, .444f},
+    {128, 256, 256, 5.54f, .537f, .210f, 0, .075f, 1.13f, .366f},   {160, 192, 256, 6.15f, .536f, .172f, 0, .044f, .62f, .413f},
+    {192, 192, 256, 5.81f, .529f, .277f, 0, .037f, 1.36f, .402f}};
+constexpr int kGtCount = sizeof(kGtTiles) / sizeof(GtTile);
+
+static int64_t gt_units(const GtTile& t, int64_t M, int64_t N) { return (M + t.tm - 1) / t.tm * ((N + t.tn - 1) / t.tn); }
+
+template <int EPI>
+static void gt_launch(int tile, int grid, const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, void* C, int64_t ldc,
+                      int M, int N, int K, int parts, hipStream_t s) {
+#define GT(I, TM, TN, WM, WN, S, O) \
+  case I: gemm_tile_kernel<TM, TN, WM, WN, S, O, EPI><<<grid, 64 * WM * WN, 0, s>>>(A, lda, B, ldb, C, ldc, M, N, K, parts); break
+  switch (tile) {
+    GT(0, 64, 64, 2, 2, 4, 2);
+    GT(1, 64, 128, 2, 2, 4, 1);
+    GT(2, 128, 128, 4, 2, 3, 1);
+    GT(3, 128, 192, 4, 2, 3, 1);
+    GT(4, 128, 256, 2, 4, 3, 1);
+    GT(5, 160, 192, 2, 2, 3, 1);
+    GT(6, 192, 192, 4, 2, 3, 1);
+  }
+#undef GT
+}
+
+}  // namespace mx
+
+using namespace mx;
+
+// Tile and parts of K for a product, as 64 tile + parts, by the modelled time; -1: it is not one turn of tiles, or another kernel
+// has it faster.  Where the lines lie (us, hipBLASLt, or gemm8 marked * -> here):
+//  * more than 44 M weights (12288 x 4096 and up) are read at the rate of memory by the library as well, from 256 rows (K of 8192:
+//    128) on it falls behind: 12288 x 4096 at 64 / 256 / 700 rows 26.7 / 1.21 / 1.23 times as fast here (26.8 at 64), 16384 x 4096 at
+//    128 37.3 -> 41.8, 8192 x 8192 at 64 / 128 / 256 33.6 / 50.9 / 1.66 times (39.0, 43.0);
+//  * a K of 12288 and more: up to 2^20 outputs, then gemm8 in parts of K (4096 x 14336 at 256 / 512 / 1024 rows 60.3* / 68.5* /
+//    103.6* -> 47.6 / 68.4 / 119; 2048 x 12288 at 512 / 1400 1.18 and .87 times as fast).
+extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 16 || K % 64) return -1;
+  const int64_t weights = (int64_t)N * K;
+  if (K >= 12288 ? (int64_t)M * N > (1 << 20) : swiglu ? weights > 128000000 : weights > 44000000 && M < (K >= 8192 ? 128 : 256))
+    return -1;
+  const int nk = K / 64;
+  float best = INFINITY;
+  int plan = -1;
+  for (int i = 0; i < kGtCount; ++i) {
+    const GtTile& t = kGtTiles[i];
+    const int64_t tiles = gt_units(t, M, N);
+    for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      const int64_t u = tiles * S;
+      if (u > t.most || (S > 1 && nk < 4 * S)) break;
+      float us = t.start + (float)nk / S * (t.step + t.load * u / 256 + (u > 256 ? t.two : 0.f)) + t.memory * weights * 2e-6f;
+      if (S > 1) us += t.sum + t.image * ((float)S * M * N * 4e-6f);
+      if (us < best) {
+        best = us;
+        plan = 64 * i + S;
+      }
+    }
+  }
+  return plan;
+}
+
+// C[M, N] = A . B^T, or C[M, N / 2] = silu(gate) up, by tile `tile` with K in `parts`; parts > 1: ws holds parts * M * N floats.
+// -1 (nothing launched) for shapes, strides and addresses that are not taken.
+extern "C" int mx_gemm_tile(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc, int M, int N,
+                            int K, int swiglu, int tile, int parts, float* ws, hipStream_t stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 16 || K % 64 || tile < 0 || tile >= kGtCount || parts < 1 || parts > K / 64) return -1;
+  if (lda % 8 || ldb % 8 || ldc % 8 || lda < K || ldb < K || ldc < (swiglu ? N / 2 : N)) return -1;
+  if ((((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) || (parts > 1 && (!ws || ((uintptr_t)ws & 15)))) return -1;
+  const GtTile& t = kGtTiles[tile];
+  // offsets of 31 bits: the 32nd marks those past K
+  if (t.tm * lda >= 1 << 30 || (swiglu ? N : t.tn) * ldb >= 1 << 30) return -1;
+  const int64_t grid = gt_units(t, M, N) * parts;
+  if (grid > INT32_MAX) return -1;
+  if (parts > 1) {
+    gt_launch<kGtPart>(tile, (int)grid, A, lda, B, ldb, ws, N, M, N, K, parts, stream);
+    const int64_t units = (int64_t)M * (swiglu ? N / 2 : N) / 8;
+    const int blocks = (int)std::min<int64_t>((units + 255) / 256, 4096);
+    if (swiglu) g8_parts_kernel<true><<<blocks, 256, 0, stream>>>(ws, (int64_t)M * N, parts, N, C, ldc, units);
+    else g8_parts_kernel<false><<<blocks, 256, 0, stream>>>(ws, (int64_t)M * N, parts, N, C, ldc, units);
+  } else if (swiglu) {
+    gt_launch<kGtSwiglu>(tile, (int)grid, A, lda, B, ldb, C, ldc, M, N, K, 1, stream);
+  } else {
+    gt_launch<kGtPlain>(tile, (int)grid, A, lda, B, ldb, C, ldc, M, N, K, 1, stream);
+  }
+  return (int)hipGetLastError();
+}

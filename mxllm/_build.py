@@ -35,7 +35,7 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 # component -> (library, kernel files, op binding files)
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
-              ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
+              ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "gemm_tile", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
                "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk",
                "sampling", "skinny_gemm",
                "stream_gemm", "stream_parts"),

@@ -20,6 +20,7 @@ the step is bitwise reproducible; vendor stream-K solutions are not, archive/pro
 """
 from __future__ import annotations
 
+import functools
 import json
 import os
 
@@ -158,17 +159,30 @@ def _gains_nn(tiles: int) -> bool:
     return _wave_fill(tiles) >= 0.68
 
 
-def rows_ok(a: torch.Tensor, b: torch.Tensor, b_kc: bool, swiglu: bool = False) -> bool:
-    """What mx_gemm8_rows (csrc/kernels/gemm8_rows.hip) takes: any number of rows of ``a`` [M, K]."""
+def rows_ok(a: torch.Tensor, b: torch.Tensor, b_kc: bool, swiglu: bool = False, cols: int = 256) -> bool:
+    """What mx_gemm8_rows (csrc/kernels/gemm8_rows.hip) takes: any number of rows of ``a`` [M, K].  ``cols`` 16: what
+    mx_gemm_tile (csrc/kernels/gemm_tile.hip) does (``b_kc``)."""
     if not (use_native(a) and a.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16):
         return False
     K, N = a.shape[1], b.shape[0 if b_kc else 1]
     ldb = b.stride(0)
-    return bool(a.shape[0] > 0 and K % 64 == 0 and K > 0 and N % 256 == 0 and N > 0
+    return bool(a.shape[0] > 0 and K % 64 == 0 and K > 0 and N % cols == 0 and N > 0
                 and a.stride(1) == 1 and b.stride(1) == 1 and a.stride(0) % 8 == 0 and ldb % 8 == 0
                 and a.stride(0) >= K and ldb >= (K if b_kc else N)
                 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
                 and 256 * a.stride(0) < 1 << 30 and (N if swiglu else 256 if b_kc else K) * ldb < 1 << 30)
+
+
+@functools.lru_cache(maxsize=4096)  # (of sizes alone)
+def _tile_plan(M: int, N: int, K: int, swiglu: bool) -> tuple[int, int] | None:
+    plan = native().gemm_tile_plan(M, N, K, swiglu)
+    return None if plan < 0 else divmod(plan, 64)
+
+
+def tile_plan(M: int, N: int, K: int, swiglu: bool = False) -> tuple[int, int] | None:
+    """(tile, parts of K) of a projection that csrc/kernels/gemm_tile.hip has faster than the library and gemm8 (the rule is
+    beside the kernel: mx_gemm_tile_plan); None: not."""
+    return None if _policy() == "0" else _tile_plan(M, N, K, swiglu)
 
 
 def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:

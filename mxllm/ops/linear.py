@@ -714,9 +714,9 @@ def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     M = x.numel() // max(K, 1)
     if x.shape[-1] != K or M == 0:
         return None
-    if M <= _DECODE_M:
-        route = _decode_route(M, N, K)
-        if not route or not _plain(x, w):
+    route = _decode_route(M, N, K) if M <= _DECODE_M else ""
+    if route:
+        if not _plain(x, w):
             return None
         x2 = x.reshape(M, K)
         if not _rows_ok(x2, w):
@@ -726,13 +726,16 @@ def _inference_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
         else:
             y = (native().skinny_linear_half if route == "half" else native().skinny_linear)(x2, w)
     else:
-        parts = gemm.rows_gain(M, N, K, True) if SKINNY_M > 0 and x.dim() > 1 else 0
-        if not parts or not _plain(x, w):
+        if SKINNY_M <= 0 or x.dim() < 2 or M <= 8 or not _plain(x, w):
+            return None
+        plan = gemm.tile_plan(M, N, K)
+        parts = 0 if plan or M <= _DECODE_M else gemm.rows_gain(M, N, K, True)
+        if not (plan or parts):
             return None
         x2 = x.reshape(M, K)
-        if not gemm.rows_ok(x2, w, True):
+        if not gemm.rows_ok(x2, w, True, cols=16 if plan else 256):
             return None
-        y = native().gemm8_rows(x2, w, True, False, parts)
+        y = native().gemm_tile(x2, w, False, *plan) if plan else native().gemm8_rows(x2, w, True, False, parts)
     return y.view(*x.shape[:-1], N)
 
 
@@ -789,7 +792,7 @@ def parts_norm(parts: torch.Tensor, h: torch.Tensor, gamma: torch.Tensor, eps: f
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
     """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch, with
     ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
-    stream_gemm.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
+    stream_gemm.hip, gemm_tile.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
     if SKINNY_M <= 0 or x.dim() != 2 or x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
         return None
@@ -805,6 +808,9 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     parts = gemm.rows_gain(M, N, K, True, True)  # a prompt pass
     if parts and _plain(x, w) and gemm.rows_ok(x, w, True, True):
         return native().gemm8_rows(x, w, True, True, parts)
+    plan = gemm.tile_plan(M, N, K, True) if M > 8 and not parts and _plain(x, w) else None
+    if plan and gemm.rows_ok(x, w, True, True, 16):
+        return native().gemm_tile(x, w, True, *plan)
     return None
 
 

@@ -152,3 +152,34 @@ def test_ragged_row_rules():
            (371, 28672, 8192, "nn"), (560, 8192, 57344, "nn"), (64, 128256, 8192, "tn"), (4013, 4096, 21504, "swiglu"), (1792, 10240, 4096, "swiglu"), (1105, 8192, 8192, "swiglu"),
            (3328, 10240, 8192, "swiglu"), (5120, 4096, 21504, "swiglu"), (512, 16384, 2048, "swiglu")]
     assert [s for s in on if not gain(*s)] == [] and [s for s in off if gain(*s)] == []
+
+
+# (M, N, K): both sides of the lines of csrc/kernels/gemm_tile.hip mx_gemm_tile_plan
+TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (17, 10240, 4096), (256, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
+           (1, 64, 4096), (40, 3360, 2048)]
+TILE_OFF = [(192 * 16 + 1, 192 * 16, 2048), (255, 12288, 4096), (127, 8192, 8192), (257, 4096, 14336), (513, 2048, 12288), (40, 3368, 2048), (40, 2048, 2080),
+            (6, 128256, 2048), (2709, 16384, 2048)]
+
+
+def test_tile_plan():
+    from mxllm.ops import native
+
+    assert [s for s in TILE_ON if gemm.tile_plan(*s) is None] == [] and [s for s in TILE_OFF if gemm.tile_plan(*s) is not None] == []
+    assert gemm.tile_plan(48, 28672, 4096, True) and not gemm.tile_plan(48, 28672, 4096) and not gemm.tile_plan(48, 57344, 8192, True)
+    assert native().gemm_tile_plan(0, 64, 64, False) == native().gemm_tile_plan(1 << 40, 64, 64, False) == -1
+
+
+def test_tile_plan_is_one_turn():
+    """Whatever the sizes: tiles and parts of K that the CUs hold at once, four 64s of K a part and more."""
+    import random
+
+    tiles = [(64, 64, 512), (64, 128, 256), (128, 128, 256), (128, 192, 256), (128, 256, 256), (160, 192, 256), (192, 192, 256)]
+    r, seen = random.Random(0), set()
+    for _ in range(4000):
+        M, N, K = int(2 ** r.uniform(0, 13)), 16 * int(2 ** r.uniform(0, 11)), 64 * int(2 ** r.uniform(0, 9))
+        plan = gemm.tile_plan(M, N, K)
+        if plan:
+            tm, tn, most = tiles[plan[0]]
+            assert -(-M // tm) * -(-N // tn) * plan[1] <= most and (plan[1] == 1 or K // 64 >= 4 * plan[1]), (M, N, K, plan)
+            seen.add(plan[0])
+    assert seen == set(range(7))
