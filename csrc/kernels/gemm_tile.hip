@@ -266,6 +266,8 @@ using namespace mx;
 //  * more than 44 M weights (12288 x 4096 and up) are read at the rate of memory by the library as well, from 256 rows (K of 8192:
 //    128) on it falls behind: 12288 x 4096 at 64 / 256 / 700 rows 26.7 / 1.21 / 1.23 times as fast here (26.8 at 64), 16384 x 4096 at
 //    128 37.3 -> 41.8, 8192 x 8192 at 64 / 128 / 256 33.6 / 50.9 / 1.66 times (39.0, 43.0);
+//    So they are by a step of up to 32 sequences from 20 M weights on (6144 x 4096 at 17 / 24 / 32 rows .89, .99, 1.0 times as fast, 16384 x
+//    2048 1.03, .97, .96; but 4096 x 4096 1.18, 1.16, 1.16, 2048 x 8192 1.16, 1.14, 1.33);
 //  * a K of 12288 and more: up to 2^20 outputs, then gemm8 in parts of K (4096 x 14336 at 256 / 512 / 1024 rows 60.3* / 68.5* /
 //    103.6* -> 47.6 / 68.4 / 119; 2048 x 12288 at 512 / 1400 1.18 and .87 times as fast).
 extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
@@ -273,6 +275,7 @@ extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
   const int64_t weights = (int64_t)N * K;
   if (K >= 12288 ? (int64_t)M * N > (1 << 20) : swiglu ? weights > 128000000 : weights > 44000000 && M < (K >= 8192 ? 128 : 256))
     return -1;
+  if (M <= 32 && weights > 20000000 && K < 12288 && !swiglu) return -1;
   const int nk = K / 64;
   float best = INFINITY;
   int plan = -1;
