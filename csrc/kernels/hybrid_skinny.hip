@@ -15,6 +15,14 @@
 #include "hybrid_fuse.h"
 #include "skinny_core.h"
 
+extern "C" int mx_stream_gru(const uint16_t* x, int64_t ldx, const uint16_t* delta, int64_t ldd, const float* h, const float* gamma,
+                             float* h_out, int groups, float eps, const uint16_t* w, int64_t ldw, const float* bias,
+                             const int32_t* slots, float* state, uint16_t* y, int M, int W, int K, hipStream_t stream);
+extern "C" int mx_stream_conv(const uint16_t* x, int64_t ldx, const uint16_t* delta, int64_t ldd, const float* h,
+                              const float* gamma, float* h_out, int groups, float eps, const uint16_t* w, int64_t ldw,
+                              const mx::ConvRope* pa, const int32_t* pos, const int32_t* slots, uint16_t* gate, int M, int K,
+                              hipStream_t stream);
+
 namespace mx {
 
 enum { kProNone, kProNorm, kProPoly };
@@ -243,6 +251,8 @@ extern "C" int mx_hs_gru_gemm(const uint16_t* x, int64_t ldx, int norm, const ui
                               const uint16_t* w, int64_t ldw, const float* bias, const int32_t* slots, float* state,
                               uint16_t* y, int M, int W, int K, hipStream_t stream) {
   if (M <= 0) return 0;
+  const int rc = mx_stream_gru(x, ldx, delta, ldd, norm ? h : nullptr, gamma, h_out, groups, eps, w, ldw, bias, slots, state, y, M, W, K, stream);
+  if (rc != -1) return rc;
   const HsNorm na{delta, ldd, h, gamma, h_out, groups, eps};
   if (hs_check(norm ? nullptr : x, ldx, ldw, M, K, W) || W % 4 || (norm && hs_norm_check(na, M, K)) || (!norm && !x))
     return -1;
@@ -260,6 +270,8 @@ extern "C" int mx_hs_conv_gemm(const uint16_t* x, int64_t ldx, int norm, const u
                                const uint16_t* w, int64_t ldw, const ConvRope* pa, const int32_t* pos,
                                const int32_t* slots, uint16_t* gate, int M, int K, hipStream_t stream) {
   if (M <= 0) return 0;
+  const int rc = mx_stream_conv(x, ldx, delta, ldd, norm ? h : nullptr, gamma, h_out, groups, eps, w, ldw, pa, pos, slots, gate, M, K, stream);
+  if (rc != -1) return rc;
   const HsNorm na{delta, ldd, h, gamma, h_out, groups, eps};
   const ConvRope& a = *pa;
   const int N = hs_conv_rows(a);

@@ -26,7 +26,7 @@
 #include <algorithm>
 
 #include "decode_fuse.h"
-#include "stream_core.h"
+#include "stream_groups.h"
 
 namespace mx {
 
@@ -43,15 +43,6 @@ struct StreamArgs {
   int M, K, F, groups;
   SkNorm na;
   SkRope rp;
-};
-
-struct StreamGroups {  // of stream_group_norm_kernel
-  const float* h;
-  const uint16_t* delta;  // or nullptr
-  int64_t ldd;
-  const float* gamma;
-  float* h_out;
-  float eps;
 };
 
 // workgroups of up to 128 registers: two a CU where LDS allows it (X of 9 rows and more of a K over 2048 does not)
@@ -154,48 +145,11 @@ template <int KP, int EPT>
 __global__ void __launch_bounds__(512, 4) stream_group_norm_kernel(StreamArgs a, StreamGroups n) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, c = tid & 15, g = tid >> 4 & 3, M = a.M;
-  constexpr int K = 512 * EPT, Q = EPT / 4;
+  constexpr int K = 512 * EPT;
   auto row = [&](int grp) __attribute__((always_inline)) -> int64_t { return (int64_t)grp * 16; };
   auto off = [&](int ch) __attribute__((always_inline)) -> int { return ch; };
   auto stage = [&](uint16_t* xs, int ldx, auto ahead) __attribute__((always_inline)) {
-    const int cc = tid * EPT;
-    f32x4 h[4][Q], gm[Q];
-    u16x4 d[4][Q];
-#pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      gm[i] = *reinterpret_cast<const f32x4*>(n.gamma + cc + 4 * i);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int mm = min(m, M - 1);
-        h[m][i] = *reinterpret_cast<const f32x4*>(n.h + (int64_t)mm * K + cc + 4 * i);
-        d[m][i] = n.delta ? *reinterpret_cast<const u16x4*>(n.delta + (int64_t)mm * n.ldd + cc + 4 * i) : u16x4{0, 0, 0, 0};
-      }
-    }
-    ahead();
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      if (m >= M) break;
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        if (n.delta) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) h[m][i][j] += bf2f(d[m][i][j]);
-          if (blockIdx.x == 0) *reinterpret_cast<f32x4*>(n.h_out + (int64_t)m * K + cc + 4 * i) = h[m][i];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ss += h[m][i][j] * h[m][i][j];
-      }
-      const float rs = 1.f / sqrtf(wave_sum(ss) / (float)(K / 8) + n.eps);
-#pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        u16x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = f2bf(h[m][i][j] * rs * gm[i][j]);
-        *reinterpret_cast<u16x4*>(xs + m * ldx + cc + 4 * i) = o;
-      }
-    }
-    lds_barrier();
+    stream_groups_in<EPT>(n, M, xs, ldx, ahead);
   };
   auto finish = [&](const f32x4& s, int mb, int cg) __attribute__((always_inline)) {
     const int m = mb * 16 + c;

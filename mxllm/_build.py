@@ -38,7 +38,7 @@ COMPONENTS = {
               ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "gemm_tile", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
                "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk",
                "sampling", "skinny_gemm",
-               "stream_gemm", "stream_parts"),
+               "stream_gemm", "stream_hybrid", "stream_parts"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),
 }
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")

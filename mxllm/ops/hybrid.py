@@ -19,7 +19,7 @@ import numpy as np
 import torch
 
 from ._ext import native, use_native
-from .linear import NORM_M, SKINNY_M, _NORM_STREAM_M, _SKINNY_SMALL_W, _near
+from .linear import NORM_M, SKINNY_M, _DECODE_M, _NORM_STREAM_M, _SKINNY_SMALL_W, _near
 
 MFMA_MAX_DIM = 128  # widest head of the MFMA attention kernels
 MFMA_MAX_REP = 16   # query heads per key head in the split-K decode kernels
@@ -311,9 +311,9 @@ FUSED = os.environ.get("MXLLM_HYBRID_FUSED", "1") != "0"
 _NORM_MAX, _POLY_MAX = 16384, 32768  # rows x width held in LDS by a prologue
 
 
-def _fusable(t: torch.Tensor, w: torch.Tensor | None, mult: int = 16) -> bool:
+def _fusable(t: torch.Tensor, w: torch.Tensor | None, mult: int = 16, rows: int = SKINNY_M) -> bool:
     M, K = t.shape
-    return bool(FUSED and w is not None and use_native(t) and w.dtype == torch.bfloat16 and 0 < M <= min(SKINNY_M, 16)
+    return bool(FUSED and w is not None and use_native(t) and w.dtype == torch.bfloat16 and 0 < M <= min(rows, 16)
                 and K % 512 == 0 and w.shape[0] % mult == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0
                 and (M == 1 or w.numel() <= _SKINNY_SMALL_W))
 
@@ -330,10 +330,7 @@ def norm_linear(delta, h, gamma, groups: int, eps: float, w):
     14.0 / 17.0, 8192 x 4096 16.8 / 17.3 -> 15.4 / 17.5; fewer would gain as well, 2048 x 2048 6.3 / 6.6 -> 4.9 / 6.1)."""
     if not _fusable(h, w):
         return None
-    M, K = h.shape
-    if (M <= min(4, _NORM_STREAM_M) and groups == 8 and K in (2048, 4096) and w.shape[0] >= 6144
-            and _near(w) and all(t.data_ptr() % 16 == 0 for t in (h, gamma, w))
-            and (delta is None or (delta.stride(0) % 8 == 0 and delta.data_ptr() % 16 == 0))):
+    if w.shape[0] >= 6144 and _norm_stays(delta, h, gamma, groups, w):
         return native().stream_group_norm(delta, h, gamma, eps, w)
     if not _norm_fits(h, groups):
         return None
@@ -349,27 +346,42 @@ def poly_linear(z, coef, eps: float, w):
     return native().hs_poly_linear(z, coef, eps, w)
 
 
-def _normed(delta, h, gamma, groups, eps):
+def _norm_stays(delta, h, gamma, groups: int, w) -> bool:
+    """Whether the workgroups that stay do the norm: 8 parts, one to each of their waves, rows of 512 threads x 4 or 8 elements, up to 4
+    rows (csrc/kernels/stream_groups.h)."""
+    return bool(h.shape[0] <= min(4, _NORM_STREAM_M) and groups == 8 and h.shape[1] in (2048, 4096) and _near(w)
+                and all(t.data_ptr() % 16 == 0 for t in (h, gamma, w))
+                and (delta is None or (delta.dim() == 2 and delta.stride(0) % 8 == 0 and delta.data_ptr() % 16 == 0)))
+
+
+def _mixer_rows(h: torch.Tensor) -> int:
+    """Rows up to which a mixer's projection runs with its epilogue: past SKINNY_M for a width of 2048 (csrc/kernels/stream_hybrid.hip;
+    steps of 9 / 12 / 16 sequences of the 1B size 998 / 1034 / 1057 us apart, 959 / 995 / 1021 so; of 4096, 8B size, 3945 / 4088 /
+    4181 apart, 3960 / 4117 / 4214)."""
+    return _DECODE_M if h.shape[1] == 2048 else SKINNY_M
+
+
+def _normed(delta, h, gamma, groups, eps, w):
     """(delta, x, gamma) of a fused projection: the norm in its prologue, or run ahead of it (a delta in parts is added there)."""
-    if _norm_fits(h, groups) and (delta is None or delta.dim() == 2):
+    if (_norm_stays(delta, h, gamma, groups, w) or _norm_fits(h, groups)) and (delta is None or delta.dim() == 2):
         return delta, h, gamma
     return None, group_norm(delta, h, gamma, groups, eps, torch.bfloat16), None
 
 
 def gru_linear(delta, h, gamma, groups: int, eps: float, w, bias, rows, layer: int):
     """Decode: (minGRU output of the normed rows, new residual), state advanced; w = [z; u; gate]."""
-    if not (rows.decode and _fusable(h, w, 12)):
+    if not (rows.decode and _fusable(h, w, 12, _mixer_rows(h))):
         return None
-    d, x, g = _normed(delta, h, gamma, groups, eps)
+    d, x, g = _normed(delta, h, gamma, groups, eps, w)
     y, hn = native().hs_gru_linear(d, x, g, groups, eps, w, bias, rows.slots, rows.caches.rec[layer])
     return y, (hn if g is not None else h)
 
 
 def conv_linear(delta, h, gamma, groups: int, eps: float, w, conv, cos, sin, sh: AttnShape, rows, layer: int):
     """Decode: (gated attention output of the normed rows, new residual); w = [q; k; v; gate]."""
-    if not (rows.decode and _fusable(h, w) and sh.dim % 4 == 0 and sh.vdim % 4 == 0):
+    if not (rows.decode and _fusable(h, w, 16, _mixer_rows(h)) and sh.dim % 4 == 0 and sh.vdim % 4 == 0):
         return None
-    d, x, g = _normed(delta, h, gamma, groups, eps)
+    d, x, g = _normed(delta, h, gamma, groups, eps, w)
     c = rows.caches
     q, gate, hn = native().hs_conv_linear(d, x, g, groups, eps, w, conv, cos, sin, sh.rot_dims, sh.heads, sh.kv_heads,
                                           sh.dim, sh.vdim, rows.pos, rows.slots, sh.chunk, c.k[layer], c.v[layer],
