@@ -57,15 +57,117 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 // for them)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Folds over a wave's lanes in the vector ALU.  A shuffle (ds_bpermute) queues in the LDS pipe and its answer is waited
+// for: the six dependent ones of a fold, by every wave of a workgroup at once, cost a launch of a decode step or of the
+// sampler 0.3 to 1.2 us, where these take a tenth.  Same pairs in the same order as a butterfly of __shfl_xor (32, 16,
+// .. 1), so sums keep their bits.  Every lane of the wave has to be on.
+template <int CTRL>
+__device__ __forceinline__ uint32_t lane_dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+struct LanePair {
+  uint32_t a, b;
+};
+// The values of a lane and of lane ^ O, in either order.  O 4: where lanes i and i ^ 8 hold the same (after O 8).
+// O 16, 32: a is that of the lower lane of the two.
+template <int O>
+__device__ __forceinline__ LanePair lane_pair(uint32_t v) {
+  static_assert(O == 32 || O == 16 || O == 8 || O == 4 || O == 2 || O == 1, "a power of two");
+  if constexpr (O == 32) {
+    const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return {s[0], s[1]};
+  } else if constexpr (O == 16) {
+    const auto s = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return {s[0], s[1]};
+  } else {
+    // row_ror:8, row_ror:4, quad_perm [2, 3, 0, 1] and [1, 0, 3, 2]
+    return {v, lane_dpp<O == 8 ? 0x128 : O == 4 ? 0x124 : O == 2 ? 0x4E : 0xB1>(v)};
+  }
+}
+template <int O>
+__device__ __forceinline__ float lane_sum(float v) {
+  const LanePair p = lane_pair<O>(__float_as_uint(v));
+  return __uint_as_float(p.a) + __uint_as_float(p.b);
+}
+template <int O>
+__device__ __forceinline__ float lane_max(float v) {
+  const LanePair p = lane_pair<O>(__float_as_uint(v));
+  return fmaxf(__uint_as_float(p.a), __uint_as_float(p.b));
+}
+template <int O>
+__device__ __forceinline__ int lane_sum(int v) {
+  const LanePair p = lane_pair<O>((uint32_t)v);
+  return (int)(p.a + p.b);
+}
+// the larger value, of equal ones the lower index (values are numbers)
+template <int O>
+__device__ __forceinline__ void lane_pick(float& v, int& i) {
+  const LanePair p = lane_pair<O>(__float_as_uint(v)), q = lane_pair<O>((uint32_t)i);
+  const float x = __uint_as_float(p.a), y = __uint_as_float(p.b);
+  const bool other = y > x || (y == x && (int)q.b < (int)q.a);
+  v = other ? y : x;
+  i = (int)(other ? q.b : q.a);
+}
+// lanes 0 .. 15 of each sixteen
+__device__ __forceinline__ float row_sum(float v) { return lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(v)))); }
+__device__ __forceinline__ float row_max(float v) { return lane_max<1>(lane_max<2>(lane_max<4>(lane_max<8>(v)))); }
+__device__ __forceinline__ float wave_sum(float v) { return row_sum(lane_sum<16>(lane_sum<32>(v))); }
+__device__ __forceinline__ float wave_max(float v) { return row_max(lane_max<16>(lane_max<32>(v))); }
+__device__ __forceinline__ int wave_sum(int v) {
+  return lane_sum<1>(lane_sum<2>(lane_sum<4>(lane_sum<8>(lane_sum<16>(lane_sum<32>(v))))));
+}
+__device__ __forceinline__ int row_min(int v) {
+  v = min(v, (int)lane_pair<8>((uint32_t)v).b);
+  v = min(v, (int)lane_pair<4>((uint32_t)v).b);
+  v = min(v, (int)lane_pair<2>((uint32_t)v).b);
+  return min(v, (int)lane_pair<1>((uint32_t)v).b);
+}
+__device__ __forceinline__ int wave_min(int v) {
+  LanePair p = lane_pair<32>((uint32_t)v);
+  p = lane_pair<16>((uint32_t)min((int)p.a, (int)p.b));
+  return row_min(min((int)p.a, (int)p.b));
+}
+__device__ __forceinline__ void row_pick(float& v, int& i) {
+  lane_pick<8>(v, i);
+  lane_pick<4>(v, i);
+  lane_pick<2>(v, i);
+  lane_pick<1>(v, i);
+}
+__device__ __forceinline__ void wave_pick(float& v, int& i) {
+  lane_pick<32>(v, i);
+  lane_pick<16>(v, i);
+  row_pick(v, i);
+}
+// what lane - n of a prefix sum's n-th step gives (zero where it has none): the steps 1, 2, 4, 8 within sixteen lanes,
+// then the sums of the sixteen and the thirty-two ahead
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t lane_ahead(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+template <typename F>
+__device__ __forceinline__ void wave_scan_steps(F&& f) {
+  f(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xF>{});  // row_shr:1
+  f(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xF>{});
+  f(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xF>{});
+  f(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xF>{});
+  f(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast:15
+  f(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // row_bcast:31
+}
+// the value of lane l (the same l in every lane)
+__device__ __forceinline__ unsigned long long lane_value(unsigned long long v, int l) {
+  return ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+// sums over lanes 0 .. this one
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+  wave_scan_steps([&](auto c, auto r) { v += lane_ahead<c.value, r.value>(v); });
   return v;
 }
-
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long v) {
+  wave_scan_steps([&](auto c, auto r) {
+    const uint32_t lo = lane_ahead<c.value, r.value>((uint32_t)v), hi = lane_ahead<c.value, r.value>((uint32_t)(v >> 32));
+    v += ((unsigned long long)hi << 32) | lo;
+  });
   return v;
 }
 
@@ -79,7 +181,8 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   if (lane == 0) scratch[wid] = v;
   __syncthreads();
   float r = 0.f;
-  for (int i = 0; i < nw; ++i) r += scratch[i];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r += i < nw ? scratch[i] : 0.f;  // (all on their way at once)
   return r;
 }
 
@@ -91,7 +194,8 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
   if (lane == 0) scratch[wid] = v;
   __syncthreads();
   float r = -INFINITY;
-  for (int i = 0; i < nw; ++i) r = fmaxf(r, scratch[i]);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) r = fmaxf(r, i < nw ? scratch[i] : -INFINITY);
   return r;
 }
 

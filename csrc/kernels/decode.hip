@@ -199,8 +199,7 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
       sacc[j][i] = x;
       mx = fmaxf(mx, x);
     }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = lane_max<32>(lane_max<16>(mx));
   const float mref = mx == -INFINITY ? 0.f : mx;  // wave with no valid key: all p = 0
   float ls = 0.f;
   u16x8 pb[NP][2];
@@ -216,8 +215,7 @@ __device__ __forceinline__ void decode_split_body(const uint16_t* __restrict__ q
         p -= bf2f(pb[n][j >> 1][4 * (j & 1) + i]);
       }
     }
-  ls += __shfl_xor(ls, 16, 64);
-  ls += __shfl_xor(ls, 32, 64);
+  ls = lane_sum<32>(lane_sum<16>(ls));
 
   // O^T[d][head] += V^T . P; k-step t covers keys 32 t + {16 h + 4 g + i}
   f32x4 oacc[DB];
@@ -483,8 +481,7 @@ struct EvenState {  // of one wave
         sc[j][i] = x;
         mx = fmaxf(mx, x);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_max<32>(lane_max<16>(mx));
     const float mref = mx == -INFINITY ? 0.f : mx, f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mref);
     m = mx;
     l *= f;
@@ -529,9 +526,7 @@ __global__ void __launch_bounds__(256, 3)
   const int c = lane & 15, g = lane >> 4, hk = blockIdx.y, rep = Hq / Hkv, x = blockIdx.x;
   int total = 0;
   for (int i = lane; i < B; i += 64) total += even_units(lens, len_off, cap, i);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
-  total = __builtin_amdgcn_readfirstlane(total);
+  total = __builtin_amdgcn_readfirstlane(wave_sum(total));
   const int share = even_share(total, gridDim.x);
   int at = x * share;
   const int end = min(total, at + share);
@@ -539,12 +534,7 @@ __global__ void __launch_bounds__(256, 3)
   int b = 0, start = 0;  // the row that holds unit `at`: start <= at < start + n
   for (int i0 = 0;; i0 += 64) {
     const int n = i0 + lane < B ? even_units(lens, len_off, cap, i0 + lane) : 0;
-    int upto = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(upto, o, 64);
-      if (lane >= o) upto += v;
-    }
+    const int upto = (int)wave_scan((uint32_t)n);
     const uint64_t past = __ballot(start + upto > at);
     if (past) {
       const int first = __ffsll((unsigned long long)past) - 1;
@@ -578,8 +568,7 @@ __global__ void __launch_bounds__(256, 3)
       const int64_t b0 = kv_row(bt, maxb, max_seq, slot, Hkv, hk, k) * D, b1 = kv_row(bt, maxb, max_seq, slot, Hkv, hk, a1) * D;
       st.take(kc + b0, kc + b1, vc + b0, vc + b1, hi - 1 - k, hi - 1 - a1, qf, k, hi, sl, c, g);
     }
-    st.l += __shfl_xor(st.l, 16, 64);
-    st.l += __shfl_xor(st.l, 32, 64);
+    st.l = lane_sum<32>(lane_sum<16>(st.l));
 #pragma unroll
     for (int e = 0; e < 8; ++e)
 #pragma unroll
@@ -636,8 +625,7 @@ __global__ void __launch_bounds__(kEvenD)
     total += u;
     if (i < b) start += u;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64), start += __shfl_xor(start, o, 64);
+  total = wave_sum(total), start = wave_sum(start);
   const int share = even_share(total, W);
   const int parts = n ? (start + n - 1) / share - start / share + 1 : 0;
   if (parts == 1) return;  // written by its workgroup
@@ -728,8 +716,7 @@ __global__ void __launch_bounds__(512)
         sc[j][i] = x;
         mx = fmaxf(mx, x);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = lane_max<32>(lane_max<16>(mx));
     const float mref = mx == -INFINITY ? 0.f : mx;
     float ls = 0.f;
     u16x8 pb[NP][2];
@@ -745,8 +732,7 @@ __global__ void __launch_bounds__(512)
           p -= bf2f(pb[n][j >> 1][4 * (j & 1) + i]);
         }
       }
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
+    ls = lane_sum<32>(lane_sum<16>(ls));
     if (g == 0) mls[t][0][c] = mx, mls[t][1][c] = ls;
     f32x4 o[E];  // [e][i]: channel E (4 g + i) + e of head c
 #pragma unroll
@@ -873,8 +859,7 @@ __global__ void __launch_bounds__(256) sample_kernel(const T* __restrict__ logit
       if (w > best) { best = w; bi = c; }
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) samp_pick(best, bi, __shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
+  wave_pick(best, bi);
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = best; si[threadIdx.x >> 6] = bi; }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -895,8 +880,7 @@ __global__ void __launch_bounds__(64) sample_final_kernel(int64_t* __restrict__ 
     best = g_samp_val[lrow * kSampMaxChunks + l];
     bi = g_samp_idx[lrow * kSampMaxChunks + l];
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) samp_pick(best, bi, __shfl_xor(best, o, 64), __shfl_xor(bi, o, 64));
+  wave_pick(best, bi);
   if (l == 0) out[(int64_t)row0 + lrow] = bi == 0x7fffffff ? 0 : bi;
 }
 

@@ -42,8 +42,8 @@ __device__ __forceinline__ void hs_gru_store(const f32x4& v, int lane, int M, in
   f32x4 u, gt;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    u[i] = __shfl(v[i], (lane & 15) + 16, 64);
-    gt[i] = __shfl(v[i], (lane & 15) + 32, 64);
+    u[i] = __uint_as_float(lane_pair<16>(__float_as_uint(v[i])).b);  // lanes 0 .. 15: of lane + 16, of lane + 32
+    gt[i] = __uint_as_float(lane_pair<32>(__float_as_uint(v[i])).b);
   }
   const int m = lane & 15, c = blk * 4;
   if (lane < 16 && m < M) {

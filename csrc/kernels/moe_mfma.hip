@@ -170,7 +170,7 @@ struct FewSlices {
         if constexpr (GLU) {  // rows 4 g .. of the slice: gate in groups 0 and 1, up in 2 and 3
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float up = __shfl_xor(s[i], 32, 64);
+            const float up = __uint_as_float(lane_pair<32>(__float_as_uint(s[i])).b);
             o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, limit));
           }
         } else {

@@ -15,12 +15,7 @@ __device__ __forceinline__ void moe_select(float* z, int E, int top, int lane, i
     int at = E;
     for (int e = lane; e < E; e += 64)
       if (z[e] > best) best = z[e], at = e;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oa = __shfl_xor(at, o, 64);
-      if (ob > best || (ob == best && oa < at)) best = ob, at = oa;
-    }
+    wave_pick(best, at);
     if (at >= E) at = 0;  // logits that are not numbers: some expert of the table
     if (k == 0) zmax = best;
     const float w = exp_t<float>(best - zmax);

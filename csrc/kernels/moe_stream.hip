@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(512, 2) moe_stream_kernel(MoeWalk p) {
       u16x4 o;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float up = __shfl_xor(s[i], 32, 64);
+        const float up = __uint_as_float(lane_pair<32>(__float_as_uint(s[i])).b);
         o[i] = f2bf(clipped_glu<uint16_t>(s[i], up, limit));
       }
       if (m < rows && g < 2) {

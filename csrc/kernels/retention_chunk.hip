@@ -342,8 +342,7 @@ __global__ void __launch_bounds__(512, DP <= 128 && EP <= 128 ? 4 : 2) retention
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < EB; ++j) ss += acc[j][i] * acc[j][i];  // columns past E are zero
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    ss = row_sum(ss);
     const float rs = 1.f / sqrtf(ss / (float)a.E + a.eps);
     const int r = 16 * w + 4 * g + i;
     if (r < rows) {

@@ -197,12 +197,7 @@ __device__ __forceinline__ int topkp_row(const T* __restrict__ x, int V, const S
     if (v > best || (v == best && idx < bi)) { best = v; bi = idx; }
   });
   auto argmax_reduce = [&](float& b, int& i) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(b, o, 64);
-      const int oi = __shfl_xor(i, o, 64);
-      if (ov > b || (ov == b && oi < i)) { b = ov; i = oi; }
-    }
+    wave_pick(b, i);
     __syncthreads();
     if (lane == 0) { red[wv] = b; redi[wv] = i; }
     __syncthreads();
@@ -238,8 +233,7 @@ __device__ __forceinline__ int topkp_row(const T* __restrict__ x, int V, const S
     rd.each([&](int, float v) {
       if (okey(v) >= t0) z += __builtin_amdgcn_exp2f((v - mx) * c);
     });
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) z += __shfl_xor(z, o, 64);
+    z = wave_sum(z);
     __syncthreads();
     if (lane == 0) red[wv] = z;
     __syncthreads();
@@ -308,10 +302,6 @@ struct SampWs {
 
 __device__ __forceinline__ void pick(float& b, int& i, float ov, int oi) {
   if (ov > b || (ov == b && oi < i)) { b = ov; i = oi; }
-}
-__device__ __forceinline__ void wave_pick(float& b, int& i) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) pick(b, i, __shfl_xor(b, o, 64), __shfl_xor(i, o, 64));
 }
 
 // [c0, c1) of a row by 16-B loads, two pieces of 8 a thread and turn; rows of any alignment (an odd vocabulary
