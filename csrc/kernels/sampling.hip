@@ -13,10 +13,13 @@
 //
 // Split form (vocabularies of kSplitV and more): three launches over (chunk, row), so a step's few rows fill the
 // chip.  One workgroup a row kept 32 of 256 CUs on six to nine passes whose LDS atomics and logarithms bound it:
-// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the three launches take 35 us by themselves (profiled:
-// stats 6, hist 11, pick 17; all top-p 33, all top-k 25, temperature alone 20) and 31 us a call behind one another.  What bounds them now: dependent steps inside each
-// launch (row parameters, the chunks' partials, scans over bins, the counter of a row), and for few rows the host's
-// three launches (22 - 25 us a call).
+// 253 us for 32 rows of 128,256 bf16 logits of mixed parameters, where the three launches take 27 us a call behind one
+// another (all top-p 28, all top-k 23, temperature alone 20.5; one row 19 - 21), of which the host's part is 21.  With
+// lane shuffles for folds and scans, the last bin's atomics on one address, and the kept tokens scored on the lanes
+// that hold them it was 32 (32 / 26 / 20.5; one row 23 - 25): see each.  What bounds them now (us within a call, stamped): stats
+// 2.5, of which loads 0.8; a launch's gap 1.3 - 2; hist 8, of which parameters and partials 1.6, LDS atomics of 64 bits on
+// random banks 3.7, the sums to memory 2; pick 12.5: loads 1.6, scan of bins and cuts 2.1, tokens 2.4, the row's list
+// and counter 2.7, and its last workgroup's comparisons 3.
 //  * stats: a chunk's largest (with its index) and smallest logit;
 //  * hist: masses exp2((x - max) log2e / T) and counts in 2048 bins, linear in the exponent (64 bins a power of
 //    two, finer where the row's whole range is under 32 of them).  A bin holds all tokens of a value, so bins
@@ -280,6 +283,7 @@ constexpr int kMBins = 2048;
 constexpr int kMaxCh = 64;         // chunks a row (= one wave over their partials)
 constexpr int kListCap = 1024;     // listed tokens a row
 constexpr int kChThreads = 1024;
+constexpr int kNearCap = 2048;     // tokens of a chunk above its row's cut that are dealt out evenly
 
 // A token that only exact sums decide about, with the mass and count of the bins ahead of its own.
 struct Listed {
@@ -379,9 +383,10 @@ __device__ __forceinline__ void group_pick(float& b, int& i, float* sv, int* si)
   if ((threadIdx.x & 63) == 0) { sv[threadIdx.x >> 6] = b; si[threadIdx.x >> 6] = i; }
   __syncthreads();
   if (threadIdx.x < 64) {
-    b = threadIdx.x < kChThreads / 64 ? sv[threadIdx.x] : -INFINITY;
-    i = threadIdx.x < kChThreads / 64 ? si[threadIdx.x] : 0x7fffffff;
-    wave_pick(b, i);
+    static_assert(kChThreads / 64 == 16, "a wave's best each: one row of lanes");
+    b = sv[threadIdx.x & 15];
+    i = si[threadIdx.x & 15];
+    row_pick(b, i);
   }
 }
 
@@ -397,17 +402,37 @@ __global__ void __launch_bounds__(kChThreads) samp_stats_kernel(const T* __restr
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) ws.nlist[row] = ws.done[row] = 0;
   const int c0 = blockIdx.x * chunk;
+  const Chunk<T> ch(logits + (size_t)row * V, c0, min(V, c0 + chunk));
+  const typename Chunk<T>::P first = ch.first();
+  // two comparisons a token: where the largest lies is looked for by the waves that hold it, and the smallest finite one
+  // again by those that have an infinity
   float b = -INFINITY, m = INFINITY;
-  int bi = 0x7fffffff;
-  Chunk<T>(logits + (size_t)row * V, c0, min(V, c0 + chunk)).each([&](int i, float v) {
-    pick(b, bi, v, i);
-    if (v > -INFINITY) m = fminf(m, v);
+  ch.each(first, [&](int, float v) {
+    b = v > b ? v : b;
+    m = v < m ? v : m;
   });
+  if (__ballot(m == -INFINITY)) {
+    m = INFINITY;
+    ch.each(first, [&](int, float v) { m = v < m && v > -INFINITY ? v : m; });
+  }
+  b = wave_max(b);
   m = -wave_max(-m);
-  if (lane == 0) sm[wv] = m;
-  group_pick(b, bi, sv, si);
+  if (lane == 0) sv[wv] = b, sm[wv] = m;
+  __syncthreads();
+  const float top = row_max(sv[lane & 15]);
+  int bi = 0x7fffffff;
+  if (b == top) {
+    ch.each(first, [&](int i, float v) { bi = v == top && i < bi ? i : bi; });
+    bi = wave_min(bi);
+  }
+  if (lane == 0) si[wv] = bi;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    bi = row_min(si[lane & 15]);
+    m = -row_max(-sm[lane & 15]);
+  }
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kChThreads / 64; ++w) m = fminf(m, sm[w]);
+    b = top;
     ws.mx[row * kMaxCh + blockIdx.x] = b;
     ws.mi[row * kMaxCh + blockIdx.x] = bi;
     ws.mn[row * kMaxCh + blockIdx.x] = m;
@@ -416,25 +441,33 @@ __global__ void __launch_bounds__(kChThreads) samp_stats_kernel(const T* __restr
 
 // what the bins of a row are made of; every lane of a wave calls it
 struct RowScale {
-  float mx, c, scale;
+  float mx, c, cs;
   int mi;
-  __device__ __forceinline__ int bin(float v) const {  // not-a-numbers: the first
-    return (int)fminf(fmaxf((mx - v) * c * scale, 0.f), (float)(kMBins - 1));
+  __device__ __forceinline__ int bin(float v) const {  // not-a-numbers: the first (med3 is the least of the others then)
+    return (int)__builtin_amdgcn_fmed3f((mx - v) * cs, 0.f, (float)(kMBins - 1));
   }
-  __device__ __forceinline__ unsigned long long weight(float v) const {  // in 2^-42
-    const float w = fminf(fmaxf(__builtin_amdgcn_exp2f((v - mx) * c), 0.f), 1.f) * 2097152.f;
-    const uint32_t hi = (uint32_t)w;
-    return ((unsigned long long)hi << 21) + (uint32_t)((w - (float)hi) * 2097152.f);
+  // exp2((v - mx) c) in 2^-42, cut off: the power's mantissa where 1 has its own, moved down by its exponent (32 top-p
+  // rows are bound by these instructions: a float's two conversions and their difference are half as many again).  What
+  // is not a number has the largest exponent, and like zero moves past the end.
+  __device__ __forceinline__ unsigned long long weight(float v) const {
+    const uint32_t b = __float_as_uint(__builtin_amdgcn_exp2f((v - mx) * c));
+    const uint32_t down = min(127u - (b >> 23), 63u);  // (no sign)
+    return ((unsigned long long)((b & 0x7fffffu) | 0x800000u) << 19) >> down;
   }
 };
-__device__ __forceinline__ RowScale row_scale(const SampWs& ws, int row, int nch, float temp) {
-  const int lane = threadIdx.x & 63;
-  float b = lane < nch ? ws.mx[row * kMaxCh + lane] : -INFINITY, m = lane < nch ? ws.mn[row * kMaxCh + lane] : INFINITY;
-  int bi = lane < nch ? ws.mi[row * kMaxCh + lane] : 0x7fffffff;
-  for (int o = 1; o < nch; o <<= 1) {  // lane 0's; few chunks, few turns
-    pick(b, bi, __shfl_xor(b, o, 64), __shfl_xor(bi, o, 64));
-    m = fminf(m, __shfl_xor(m, o, 64));
+struct RowParts {  // its chunks' statistics, one a lane
+  float b, m;
+  int bi;
+  __device__ __forceinline__ RowParts(const SampWs& ws, int row, int nch) {
+    const int lane = threadIdx.x & 63, at = row * kMaxCh + min(lane, nch - 1);  // (the last again: it changes nothing)
+    b = ws.mx[at], m = ws.mn[at], bi = ws.mi[at];
   }
+};
+__device__ __forceinline__ RowScale row_scale(RowParts p, float temp) {
+  float b = p.b, m = p.m;
+  int bi = p.bi;
+  wave_pick(b, bi);
+  m = -wave_max(-m);
   b = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(b)));
   m = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m)));
   bi = __builtin_amdgcn_readfirstlane(bi);
@@ -443,7 +476,7 @@ __device__ __forceinline__ RowScale row_scale(const SampWs& ws, int row, int nch
   r.mi = bi;
   r.c = 1.4426950408889634f / temp;  // exp2 domain
   const float range = (b - m) * r.c;
-  r.scale = range > 0.f && range < 31.9f ? (kMBins - 1) / range : 64.f;
+  r.cs = r.c * (range > 0.f && range < 31.9f ? (kMBins - 1) / range : 64.f);
   return r;
 }
 
@@ -455,16 +488,19 @@ __global__ void __launch_bounds__(kChThreads) samp_hist_kernel(const T* __restri
   __shared__ float sv[kChThreads / 64];
   __shared__ int si[kChThreads / 64];
   const int row = blockIdx.y;
+  const int c0 = blockIdx.x * chunk;
+  const Chunk<T> ch(logits + (size_t)row * V, c0, min(V, c0 + chunk));
+  const typename Chunk<T>::P first = ch.first();  // on its way, like the statistics, with the row's parameters
+  const RowParts parts(ws, row, gridDim.x);
+  __builtin_amdgcn_sched_barrier(0);
   const SampRow rp = samp_row(a, row0 + row);
   const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f;
   if (!(rp.temp > 0.f)) return;
-  const int c0 = blockIdx.x * chunk;
-  const Chunk<T> ch(logits + (size_t)row * V, c0, min(V, c0 + chunk));
   if (!(hk || hp)) {  // every token competes: nothing to wait for
     const float inv_t = 1.f / rp.temp;
     float gb = -INFINITY;
     int gi = 0x7fffffff;
-    ch.each([&](int i, float v) { pick(gb, gi, gumbel_score(v, inv_t, rp.seed, rp.step, i), i); });
+    ch.each(first, [&](int i, float v) { pick(gb, gi, gumbel_score(v, inv_t, rp.seed, rp.step, i), i); });
     group_pick(gb, gi, sv, si);
     if (threadIdx.x == 0) {
       ws.gv[row * kMaxCh + blockIdx.x] = gb;
@@ -472,15 +508,32 @@ __global__ void __launch_bounds__(kChThreads) samp_hist_kernel(const T* __restri
     }
     return;
   }
-  const typename Chunk<T>::P first = ch.first();  // on its way while the row's scale is found
   for (int i = threadIdx.x; i < kMBins; i += kChThreads) { mass[i] = 0; cnt[i] = 0; }
-  const RowScale rs = row_scale(ws, row, gridDim.x, rp.temp);
+  const RowScale rs = row_scale(parts, rp.temp);
   __syncthreads();
+  // the last bin holds all that lies further away than it: a sixth of a row at a low temperature, whose atomics on one
+  // address held a workgroup up for 5 us.  Its sums are the threads' own first.
+  unsigned long long fm = 0;
+  uint32_t fc = 0;
   ch.each(first, [&](int, float v) {
     const int b = rs.bin(v);
-    if (hp) atomicAdd(&mass[b], rs.weight(v));
-    if (hk) atomicAdd(&cnt[b], 1u);
+    const unsigned long long w = hp ? rs.weight(v) : 0;
+    if (b == kMBins - 1) {
+      fm += w;
+      ++fc;
+    } else {
+      if (hp) atomicAdd(&mass[b], w);
+      if (hk) atomicAdd(&cnt[b], 1u);
+    }
   });
+  if (__ballot(fc != 0)) {
+    fm = wave_scan(fm);
+    fc = wave_scan(fc);
+    if ((threadIdx.x & 63) == 63) {
+      if (hp) atomicAdd(&mass[kMBins - 1], fm);
+      if (hk) atomicAdd(&cnt[kMBins - 1], fc);
+    }
+  }
   __syncthreads();
   for (int i = threadIdx.x; i < kMBins; i += kChThreads) {
     if (mass[i]) atomicAdd(&ws.mass[row * kMBins + i], mass[i]);
@@ -499,11 +552,11 @@ struct Bins {
   static constexpr int PER = kMBins / kChThreads;
   unsigned long long m[PER];
   uint32_t n[PER];
-  __device__ __forceinline__ Bins(const SampWs& ws, int row, bool hk, bool hp) {
+  __device__ __forceinline__ Bins(const SampWs& ws, int row) {  // (zero where the row has no such cut)
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      m[i] = hp ? ws.mass[row * kMBins + threadIdx.x * PER + i] : 0;
-      n[i] = hk ? ws.cnt[row * kMBins + threadIdx.x * PER + i] : 0;
+      m[i] = ws.mass[row * kMBins + threadIdx.x * PER + i];
+      n[i] = ws.cnt[row * kMBins + threadIdx.x * PER + i];
     }
   }
 };
@@ -512,35 +565,23 @@ __device__ __forceinline__ RowCut row_cut(const Bins& bins, const SampRow& rp, b
                                           unsigned long long* pm, uint32_t* pc, unsigned long long* wm, uint32_t* wc,
                                           RowCut* out, unsigned long long& tot) {
   constexpr int PER = Bins::PER, NW = kChThreads / 64;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const auto &m = bins.m;
   const auto &n = bins.n;
   unsigned long long sm = 0;
   uint32_t sn = 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) sm += m[i], sn += n[i];
-  unsigned long long im = sm;
-  uint32_t in = sn;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const unsigned long long y = __shfl_up(im, o, 64);
-    const uint32_t z = __shfl_up(in, o, 64);
-    if (lane >= o) { im += y; in += z; }
-  }
+  const unsigned long long im = wave_scan(sm);
+  const uint32_t in = wave_scan(sn);
   if (lane == 63) { wm[wv] = im; wc[wv] = in; }
   if (t == 0) *out = RowCut{0, 0, hk ? kMBins - 1 : kMBins, 0, 0};
   __syncthreads();
-  unsigned long long vm = lane < NW ? wm[lane] : 0;
-  uint32_t vn = lane < NW ? wc[lane] : 0;
-#pragma unroll
-  for (int o = 1; o < NW; o <<= 1) {
-    const unsigned long long y = __shfl_up(vm, o, 64);
-    const uint32_t z = __shfl_up(vn, o, 64);
-    if (lane >= o) { vm += y; vn += z; }
-  }
-  tot = __shfl(vm, NW - 1, 64);
-  unsigned long long bm = im - sm + (wv ? __shfl(vm, wv - 1, 64) : 0);
-  uint32_t bn = in - sn + (wv ? __shfl(vn, wv - 1, 64) : 0);
+  const unsigned long long vm = wave_scan(lane < NW ? wm[lane] : 0ull);
+  const uint32_t vn = wave_scan(lane < NW ? wc[lane] : 0u);
+  tot = lane_value(vm, NW - 1);
+  unsigned long long bm = im - sm + (wv ? lane_value(vm, wv - 1) : 0);
+  uint32_t bn = in - sn + (wv ? (uint32_t)__builtin_amdgcn_readlane((int)vn, wv - 1) : 0);
   const unsigned long long bm0 = bm;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -655,26 +696,28 @@ __global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restri
     struct {
       unsigned long long pm[kMBins], wm[kChThreads / 64], own[kListCap];
       uint32_t pc[kMBins], wc[kChThreads / 64];
+      uint2 near[kNearCap];
       RowCut cut;
     } c;
     FinalScratch f;
     SampScratch slow;
   } sh;
   static_assert(kSampThreads == kChThreads && kListCap == kChThreads, "one workgroup shape; a thread a listed token");
-  __shared__ uint32_t nown, at0, last;
+  __shared__ uint32_t nown, nnear, at0, last;
   __shared__ float sv[kChThreads / 64];
   __shared__ int si[kChThreads / 64];
   const int row = blockIdx.y, nch = gridDim.x, t = threadIdx.x, lane = t & 63;
-  const SampRow rp = samp_row(a, row0 + row);
-  const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f, cutting = rp.temp > 0.f && (hk || hp);
   const T* x = logits + (size_t)row * V;
-  if (!cutting && blockIdx.x) return;
-  const Bins bins(ws, row, cutting && hk, cutting && hp);
   const int c0 = blockIdx.x * chunk;
   const Chunk<T> ch(x, c0, min(V, c0 + chunk));
-  typename Chunk<T>::P p = {};
-  if (cutting) p = ch.first();  // on its way while the cut is found
-  const RowScale rs = row_scale(ws, row, nch, rp.temp);
+  const Bins bins(ws, row);  // on their way, like the statistics and the first logits, with the row's parameters
+  const RowParts parts(ws, row, nch);
+  typename Chunk<T>::P p = ch.first();
+  __builtin_amdgcn_sched_barrier(0);
+  const SampRow rp = samp_row(a, row0 + row);
+  const bool hk = rp.k > 0 && rp.k < V, hp = rp.p < 1.f, cutting = rp.temp > 0.f && (hk || hp);
+  if (!cutting && blockIdx.x) return;
+  const RowScale rs = row_scale(parts, rp.temp);
   auto end = [&](float gb, int gi) {  // thread 0
     out[row] = gi < V ? gi : (rs.mi < V ? rs.mi : 0);
   };
@@ -685,7 +728,7 @@ __global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restri
     if (t == 0) end(gb, gi);
     return;
   }
-  if (t == 0) nown = 0;
+  if (t == 0) nown = nnear = 0;
   RowInfo info;
   const RowCut r = row_cut(bins, rp, hk, hp, sh.c.pm, sh.c.pc, sh.c.wm, sh.c.wc, &sh.c.cut, info.tot);
   info.pmk = r.klo;
@@ -703,17 +746,31 @@ __global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restri
     }
   };
   // Most tokens lie further from the largest than the last bin that counts reaches: a difference and a comparison
-  // mark the others (and not-a-numbers), which then go one a lane and turn.  With bins for all, and a score at each of
-  // a wave's 16 places that any lane keeps, 32 top-p rows took 36 us, now 33.
+  // mark the others (and not-a-numbers).  Those are few and uneven, three or four on one lane of a wave and none on
+  // most: they are gathered, and then scored by all threads alike.  What does not fit goes one a lane and turn.
   const int lim = max(max(r.last, hk ? r.bk : 0), r.all - 1);
-  const float far = lim >= kMBins - 1 ? INFINITY : (float)(lim + 1) / (rs.c * rs.scale) * 1.0001f + 1e-30f;
+  const float far = lim >= kMBins - 1 ? INFINITY : (float)(lim + 1) / rs.cs * 1.0001f + 1e-30f;
   ch.ends(token);
-  for (int at = ch.start(); at < ch.ve; at += 2 * ch.S) {
-    if (at != ch.start()) p = ch.load(at);
+  for (int at = ch.start(); at - lane * 8 < ch.ve; at += 2 * ch.S) {  // whole waves, for the sums over lanes
+    if (at != ch.start() && at < ch.ve) p = ch.load(at);
     uint32_t near = 0;
 #pragma unroll
     for (int j = 0; j < 16; ++j) near |= !(rs.mx - p.at(j) > far) ? 1u << j : 0u;
-    if (at + ch.S >= ch.ve) near &= 0xffu;
+    near &= at >= ch.ve ? 0u : at + ch.S >= ch.ve ? 0xffu : 0xffffu;
+    const uint32_t c = __builtin_popcount(near), upto = wave_scan(c);
+    const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+    if (!all) continue;
+    uint32_t from = 0;
+    if (lane == 0) from = atomicAdd(&nnear, all);
+    from = (uint32_t)__builtin_amdgcn_readfirstlane((int)from);
+    if (from + all <= kNearCap) {
+      uint2* q = sh.c.near + from + upto - c;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (near >> j & 1) *q++ = {__float_as_uint(p.at(j)), (uint32_t)(at + (j & 7) + (j & 8 ? ch.S : 0))};
+      continue;
+    }
+    for (uint32_t q = from + lane; q < kNearCap; q += 64) sh.c.near[q] = {0u, ~0u};  // (asked for, and not used)
     for (; near; near &= near - 1) {
       const int j = __builtin_ctz(near);
       float v = p.at(0);
@@ -721,6 +778,11 @@ __global__ void __launch_bounds__(kChThreads) samp_pick_kernel(const T* __restri
       for (int k = 1; k < 16; ++k) v = j == k ? p.at(k) : v;
       token(at + (j & 7) + (j & 8 ? ch.S : 0), v);
     }
+  }
+  __syncthreads();
+  for (uint32_t q = t, n = min(nnear, (uint32_t)kNearCap); q < n; q += kChThreads) {
+    const uint2 e = sh.c.near[q];
+    if (e.y != ~0u) token((int)e.y, __uint_as_float(e.x));
   }
   group_pick(gb, gi, sv, si);  // its barrier: the workgroup's list is whole
   const uint32_t mine = nown;

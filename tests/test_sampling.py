@@ -205,6 +205,29 @@ def test_gpu_split_sampler_draws(gpu, V, dtype, shape):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kept", [1, 63, 2047, 2048, 2049, 6000])
+def test_gpu_split_sampler_kept_tokens_of_one_chunk(gpu, kept, dtype):
+    """Kept tokens are gathered up to 2,048 a chunk, the rest scored where they lie: as many about that, all in the first
+    8,192 of 16,384 (a chunk of a 64-row call), the others far below them, in the histogram's last bin."""
+    V, B = 16384, 64
+    g = torch.Generator().manual_seed(kept)
+    x = torch.full((B, V), -300.0)
+    for i in range(B):
+        x[i, torch.randperm(8192, generator=g)[:kept]] = 1.0
+    x = x.to(dtype)
+    seeds = [7 * i for i in range(B)]
+    got = dops.sample_rows(x.to(gpu), [0.7] * B, [0.9, 1.0] * (B // 2), [0, kept] * (B // 2), seeds, [3] * B).tolist()
+    for i in range(B):
+        noise, err = _scores(V, seeds[i], 3)
+        s = torch.where(x[i] > 0, noise, float("-inf"))
+        best = int((s - err).argmax())
+        rest = s + err
+        rest[best] = float("-inf")
+        assert x[i, got[i]] > 0 and (got[i] == best or (s - err)[best] <= rest.max())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("V", [1000, 16384, 50257])
 @pytest.mark.parametrize("temp,p,k", [(0.8, 1.0, 0), (0.8, 0.9, 0), (0.8, 1.0, 40), (0.8, 0.9, 40), (0.0, 1.0, 0)])
 def test_gpu_sampler_without_numbers(gpu, V, temp, p, k):
