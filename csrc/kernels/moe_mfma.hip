@@ -379,6 +379,48 @@ __global__ void __launch_bounds__(512, TMAX <= 32 ? 4 : 2) moe_few_kernel(MoeFew
   else s.template run<ROWS>(known, n, a.N, a.x, xoff, yrow, a.y, a.limit, red, w, lane, c, g);
 }
 
+// The gated products of more pairs than experts, chosen from the router's logits: y[pair] = clipped unit of x[token] through
+// [gate | up].  Workgroups: the shared expert's slices (its rows are the tokens), those of every expert, and one that
+// stores the choices, behind all others.  A wave finds its expert's tokens by itself (moe_route.h, moe_place): with all
+// choices made by every workgroup and two barriers, the weights of half of them began 10 us into the launch (stamped; 32
+// tokens, 1B sizes), now 7; steps of 24 / 32 / 48 sequences 1480 / 1567 / 1890 -> 1452 / 1525 / 1782 us, 8B sizes of
+// 48 7190 -> 6781.  The other half's logits wait in their CU's queue behind the
+// first half's weights: 67 MB come at 4.5 TB/s whatever is asked for first (half or all of a wave's weights ahead of the
+// choices: within 0.4 %).
+template <typename Own, int ROWS, int LESS, typename Shared, int SROWS, int TMAX>
+__global__ void __launch_bounds__(512, TMAX <= 32 ? 4 : 2) moe_up_kernel(MoeFew a) {
+  __shared__ int16_t list[kFewTokens];
+  __shared__ f32x4 red[Own::places(ROWS) > Shared::places(SROWS) ? Own::places(ROWS) : Shared::places(SROWS)];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  typedef typename Own::Off Off;
+  constexpr int SCOLS = Shared::SL * Shared::CH, COLS = Own::SL * Own::CH;
+  const int snx = a.sw ? (a.sN + SCOLS - 1) / SCOLS : 0, nx = (a.N + COLS - 1) / COLS;
+  if ((int)blockIdx.x < snx) {
+    Shared s(a.sw, blockIdx.x, a.sN, a.sK, w, lane);
+    s.template run<SROWS>(
+        false, a.T, a.sN, a.x, [&](int r) { return r * (Off)a.ldx; }, [](int r) { return r; }, a.sy, a.slimit, red, w, lane,
+        c, g);
+    return;
+  }
+  if (blockIdx.x == gridDim.x - 1) {
+    for (int t = w; t < a.T; t += 8)
+      moe_choose64(a.logits[(int64_t)t * a.E + min(lane, a.E - 1)], a.E, a.top, lane, [&](int k, float wt) {
+        a.ids_out[t * a.top + k] = lane;
+        a.wts_out[t * a.top + k] = wt;
+      });
+    return;
+  }
+  const int bx = (blockIdx.x - snx) % nx, expert = (blockIdx.x - snx) / nx;
+  const int n = moe_list(moe_place(a.logits, a.E, a.top, a.T, expert, lane), a.top, lane, list);
+  if (n == 0) return;
+  Own s(a.w + expert * (2 * (int64_t)a.N * a.K), bx, a.N, a.K, w, lane);
+  auto xoff = [&](int r) { return (Off)(list[r] / a.top) * (Off)a.ldx; };
+  auto yrow = [&](int r) { return list[r]; };
+  if (LESS < ROWS && n <= LESS) s.template run<LESS>(false, n, a.N, a.x, xoff, yrow, a.y, a.limit, red, w, lane, c, g);
+  else s.template run<ROWS>(false, n, a.N, a.x, xoff, yrow, a.y, a.limit, red, w, lane, c, g);
+}
+
 }  // namespace mx
 
 using namespace mx;
@@ -466,7 +508,20 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
                      (a.T > 16 || (a.K <= 384 && (!a.sw || a.sK % 2048 == 0))) &&
                      std::max(std::max((int64_t)a.N * a.K, (int64_t)a.sN * a.sK),
                               pairs * std::max(a.ldx, (int64_t)a.sK)) < (1ll << 31) - 4096;
-  if (glu) {
+#define MU(OWN, ROWS, LESS, SHARED, SROWS, TMAX)                                                                 \
+  do {                                                                                                           \
+    typedef OWN Own;                                                                                             \
+    typedef SHARED Shared;                                                                                       \
+    const int64_t cols = Own::SL * Own::CH, sc = Shared::SL * Shared::CH;                                        \
+    const int64_t gr = a.E * ((a.N + cols - 1) / cols) + (a.sw ? (a.sN + sc - 1) / sc : 0) + 1;                  \
+    if (gr > INT32_MAX) return -1;                                                                               \
+    moe_up_kernel<Own, ROWS, LESS, Shared, SROWS, TMAX><<<(unsigned)gr, 512, 0, stream>>>(a);                    \
+  } while (0)
+  if (glu && a.logits && pairs > a.E) {
+    if (a.T <= 16) MU(FS(true, 8, 2), 16, 16, FS(true, 8, 2), 16, 16);
+    else if (a.T <= 32) MU(FS(true, 8, 2), 32, 16, FS(true, 8, 2), 32, 32);
+    else MU(FS(true, 8, 4), 64, 16, FS(true, 8, 4), 64, 64);
+  } else if (glu) {
     if (a.T <= 16) MF(true, FS(true, 8, 2), 16, 16, FS(true, 8, 2), 16, 16);
     else if (a.T <= 32) MF(true, FS(true, 8, 2), 32, 16, FS(true, 8, 2), 32, 32);
     else MF(true, FS(true, 8, 4), 64, 16, FS(true, 8, 4), 64, 64);
@@ -485,5 +540,6 @@ extern "C" int mx_moe_few(const MoeFew* pa, int glu, hipStream_t stream) {
 #undef FL
 #undef FS
 #undef MF
+#undef MU
   return (int)hipGetLastError();
 }

@@ -34,7 +34,7 @@ struct MoeWalk {
 template <int KP, int NL>
 __global__ void __launch_bounds__(512, 2) moe_stream_kernel(MoeWalk p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  __shared__ int16_t slot[64], list[64];  // a token's pair with this expert or -1; those that have one
+  __shared__ int16_t list[64];  // the pairs of the tokens that chose this expert
   const MoeFew& a = p.a;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
   const bool shared = (int)blockIdx.x < p.ws;
@@ -43,31 +43,23 @@ __global__ void __launch_bounds__(512, 2) moe_stream_kernel(MoeWalk p) {
   const int first = (shared ? unit : unit % p.we) * per, groups = min(F / 8, first + per);
   int n = a.T;
   if (!shared) {
-    constexpr int TW = kMoeStreamTokens / 8;  // tokens of a wave, their logits asked for together
-    float z[TW];
+    if (unit == p.we - 1) {  // the last of the first expert, whose run may be the shorter one, stores the choices
+      constexpr int TW = kMoeStreamTokens / 8;  // tokens of a wave, their logits asked for together
+      float z[TW];
 #pragma unroll
-    for (int i = 0; i < TW; ++i) z[i] = a.logits[(int64_t)min(w + 8 * i, a.T - 1) * a.E + min(lane, a.E - 1)];
-    const bool store = unit == 0;
-    if (lane < TW) slot[w + 8 * lane] = -1;
+      for (int i = 0; i < TW; ++i) z[i] = a.logits[(int64_t)min(w + 8 * i, a.T - 1) * a.E + min(lane, a.E - 1)];
 #pragma unroll
-    for (int i = 0; i < TW; ++i) {
-      const int t = w + 8 * i;
-      if (t >= a.T) break;
-      moe_choose64(z[i], a.E, a.top, lane, [&](int k, float wt) {
-        if (lane == expert) slot[t] = (int16_t)(t * a.top + k);
-        if (store) {
+      for (int i = 0; i < TW; ++i) {
+        const int t = w + 8 * i;
+        if (t >= a.T) break;
+        moe_choose64(z[i], a.E, a.top, lane, [&](int k, float wt) {
           a.ids_out[t * a.top + k] = lane;
           a.wts_out[t * a.top + k] = wt;
-        }
-      });
+        });
+      }
     }
-    lds_barrier();
-    const int mine = lane < kMoeStreamTokens ? slot[lane] : -1;  // every wave writes the list
-    const uint64_t on = __ballot(mine >= 0);
-    n = __popcll(on);
+    n = moe_list(moe_place(a.logits, a.E, a.top, a.T, expert, lane), a.top, lane, list);
     if (n == 0) return;
-    if (mine >= 0) list[__popcll(on & ((1ull << lane) - 1))] = (int16_t)mine;
-    lds_barrier();
   }
   const uint16_t* W = shared ? a.sw : a.w + (int64_t)expert * 2 * a.N * a.K;
   uint16_t* const y = shared ? a.sy : a.y;

@@ -182,6 +182,28 @@ def test_up_products_past_rows_in_lds(gpu, T, E, top, K, ff, shared):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,K", [(2, 3, 2, 192), (17, 16, 4, 192), (33, 18, 4, 192), (64, 33, 5, 192), (64, 64, 2, 192),
+                                       (9, 6, 6, 2048), (16, 18, 2, 2048), (32, 35, 4, 4096)])
+def test_choices_seen_from_one_expert(gpu, T, E, top, K):
+    """A workgroup finds its expert's tokens from the logits alone: equal logits (the lower index first), infinities and
+    what is not a number (last), rows of logits that are no whole 16 B.  The products are those of given choices."""
+    bf, F = torch.bfloat16, 40
+    gen = torch.Generator().manual_seed(T * E)
+    z = torch.randint(-3, 4, (T, E), generator=gen).float()
+    z[torch.rand(T, E, generator=gen) < 0.1] = float("-inf")
+    z[torch.rand(T, E, generator=gen) < 0.05] = float("nan")
+    z[:, T % E] = 2.0
+    z[0] = 1.0
+    at = torch.sort(torch.where(z.isnan(), float("-inf"), z), dim=1, descending=True, stable=True).indices[:, :top]
+    x, w = rnd(T, K, seed=1, dt=bf).to(gpu), (rnd(E, 2 * F, K, seed=2) / K ** 0.5).to(bf).to(gpu)
+    y, _, ids, wts = native().moe_few(x, None, z.to(gpu), top, w, True, 1.2, None, None, 0.0)
+    assert torch.equal(ids.cpu().long(), at)
+    close(wts, torch.softmax(torch.where(z.isnan(), float("-inf"), z).double().gather(1, at), 1), torch.float32)
+    given, _, _, _ = native().moe_few(x, at.int().to(gpu), None, top, w, True, 1.2, None, None, 0.0)
+    close(y, given, bf, 0.3)  # f32 sums in two orders, one rounding to bf16 (2^-9)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("R,W", [(32, 256), (32, 4096), (64, 128), (64, 1920), (64, 2048), (128, 64), (128, 768), (128, 1024)])
 @pytest.mark.parametrize("T", [1, 5, 64])
 def test_side_projection_with_its_norm(gpu, T, R, W):
