@@ -507,9 +507,16 @@ struct EvenState {  // of one wave
   }
 };
 
-// units of 16 keys that row b has; cap: positions that the buffers are sized for
+// What a row costs a workgroup beside its keys, in units of 16: its length, slot, block and q asked for one after another,
+// the sums of its waves, and waves' turns of 32 keys that are not full.  Dealt by their keys alone, workgroups with the end
+// of one row and the start of another ended 22 us into the launch, those within a row at 15 (16 sequences of 100 to 2,000
+// keys).  A step of them, us, with 0 / 3 / 6 / 9 / 13: 4060 / 4008 / 4001 / 4013 / 4043; 32 of 250 to 1,000 4738 / 4710 /
+// 4696 / 4753 / 4768; 24 of 225 to 900 4515 / 4497 / 4498 / 4510 / 4526; 8 of 750 to 3,000 3800 / 3791 / 3799 / 3844 / 3828.
+constexpr int kEvenPad = 6;
+// units that row b is dealt as, the first kEvenPad of which hold no keys; cap: positions that the buffers are sized for
 __device__ __forceinline__ int even_units(const int32_t* lens, int len_off, int cap, int b) {
-  return (min(max(lens[b] + len_off, 0), cap) + 15) >> 4;
+  const int n = (min(max(lens[b] + len_off, 0), cap) + 15) >> 4;
+  return n ? n + kEvenPad : 0;
 }
 // units of a workgroup: an equal share of all, at least 128 keys
 __device__ __forceinline__ int even_share(int total, int W) { return max((total + W - 1) / W, 8); }
@@ -550,7 +557,9 @@ __global__ void __launch_bounds__(256, 3)
       ++b;
       continue;
     }
-    const int u0 = at - start, u1 = min(end - start, n), per = (u1 - u0 + 3) >> 2;
+    const int from = start + kEvenPad;  // of its keys
+    const int u0 = max(at - from, 0), u1 = min(end - from, n), per = (u1 - u0 + 3) >> 2;
+    if (u1 <= 0) return;  // its keys begin in the next share
     const int k_lo = 16 * (u0 + per * w), hi = min(len, 16 * min(u1, u0 + per * (w + 1)));
     const int slot = slots ? slots[b] : b;
     u16x8 qf[4];
@@ -575,7 +584,7 @@ __global__ void __launch_bounds__(256, 3)
       for (int i = 0; i < 4; ++i) so[w][8 * (4 * g + i) + e][c] = st.o[e][i];
     if (g == 0) mls[w][0][c] = st.m, mls[w][1][c] = st.l;
     __syncthreads();
-    const int part = x - start / share, last = (start + n - 1) / share - start / share;
+    const int part = x - from / share, last = (from + n - 1) / share - from / share;
     for (int idx = tid; idx < rep * D; idx += 256) {
       const int h = idx / D, d = idx % D;
       float M = -INFINITY, L = 0.f, acc = 0.f;
@@ -595,7 +604,7 @@ __global__ void __launch_bounds__(256, 3)
         if (d == 0) part_ml[(bh * nparts + part) * 2] = M, part_ml[(bh * nparts + part) * 2 + 1] = L;
       }
     }
-    at = start += n;
+    at = start = from + n;
     if (at >= end) return;
     ++b;
     __syncthreads();  // the sums are read
@@ -619,15 +628,15 @@ __global__ void __launch_bounds__(kEvenD)
     mv[s] = ml[2 * p], lv[s] = ml[2 * p + 1], ov[s] = po[(int64_t)p * kEvenD];
   }
   int total = 0, start = 0;
-  const int n = even_units(lens, len_off, cap, b);
+  const int n = even_units(lens, len_off, cap, b) - kEvenPad;
   for (int i = lane; i < B; i += 64) {
     const int u = even_units(lens, len_off, cap, i);
     total += u;
     if (i < b) start += u;
   }
   total = wave_sum(total), start = wave_sum(start);
-  const int share = even_share(total, W);
-  const int parts = n ? (start + n - 1) / share - start / share + 1 : 0;
+  const int share = even_share(total, W), from = start + kEvenPad;
+  const int parts = n > 0 ? (from + n - 1) / share - from / share + 1 : 0;
   if (parts == 1) return;  // written by its workgroup
   float M = -INFINITY, L = 0.f, acc = 0.f;
 #pragma unroll

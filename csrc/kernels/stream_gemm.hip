@@ -49,8 +49,9 @@ struct StreamArgs {
 template <int KIND, int TB, int KP, int NL>
 constexpr int kStWaves = KIND >= kStF8 ? (TB == 1 ? 4 : 2) : NL == 8 && (TB == 1 || KP == 4) ? 4 : 2;
 
-template <int KIND, int TB, int KP, int EPI, bool NORM, int NL>
-__global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm_kernel(StreamArgs a) {
+// HALF: 256 workgroups, of which each has a group and, in front of the last groups' count, half of one of those
+template <int KIND, int TB, int KP, int EPI, bool NORM, int NL, bool HALF = false>
+__global__ void __launch_bounds__(512, (HALF ? 2 : kStWaves<KIND, TB, KP, NL>)) stream_gemm_kernel(StreamArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, c = tid & 15, g = tid >> 4 & 3;
   const int M = a.M, K = a.K;
@@ -74,8 +75,8 @@ __global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm
       stream_rows_in<KIND < kStF8 && NL == 16 ? 16 : 8>(a.X, a.ldx, M, K, xs, ldx, ahead);
     }
   };
-  auto finish = [&](const f32x4& s, int mb, int cg) __attribute__((always_inline)) {
-    const int m = mb * 16 + c;
+  auto finish = [&](const f32x4& s, int mb, int cg, bool on = true) __attribute__((always_inline)) {
+    const int m = on ? mb * 16 + c : M;
     if constexpr (EPI == kStRope128) {
       dfuse_rope_store<64>(s, g, m, M, cg, a.rp);
     } else if constexpr (EPI == kStRope64) {
@@ -89,17 +90,22 @@ __global__ void __launch_bounds__(512, (kStWaves<KIND, TB, KP, NL>)) stream_gemm
       *reinterpret_cast<u16x4*>(a.Y + (int64_t)m * a.ldy + (int64_t)cg * 16 + 4 * g) = o;
     }
   };
-  stream_walk<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, (int)blockIdx.x, (int)gridDim.x, a.groups, smem, row, off, stage, finish);
+  const int x = blockIdx.x;
+  if constexpr (HALF)
+    stream_and_half<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, x, x < 2 * (a.groups - 256) ? 512 + x : -1, smem, row, off,
+                                      stage, finish);
+  else
+    stream_walk<KIND, TB, KP, NL>(a.W, a.ldw, a.scale, M, K, x, (int)gridDim.x, a.groups, smem, row, off, stage, finish);
 }
 
 constexpr int kTwoLds = 80 * 1024;  // LDS up to which two workgroups share a CU
 
-template <int KIND, int TB, int KP, int EPI, bool NORM, int NL>
+template <int KIND, int TB, int KP, int EPI, bool NORM, int NL, bool HALF = false>
 static int stream_launch(const StreamArgs& a, int per_cu, size_t lds, hipStream_t stream) {
-  static const bool big = hipFuncSetAttribute((const void*)stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL>,
+  static const bool big = hipFuncSetAttribute((const void*)stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL, HALF>,
                                               hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) == hipSuccess;
   if (!big) return -1;
-  stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL><<<std::min(a.groups, 256 * per_cu), 512, lds, stream>>>(a);
+  stream_gemm_kernel<KIND, TB, KP, EPI, NORM, NL, HALF><<<std::min(a.groups, 256 * per_cu), 512, lds, stream>>>(a);
   return (int)hipGetLastError();
 }
 
@@ -110,6 +116,9 @@ static int stream_blocks(const StreamArgs& a, hipStream_t stream) {
   constexpr int KP8 = KIND == kStF8Lines ? 4 : 8;
   const size_t lds = (four ? kStreamRed<KIND, TB, 4> : kStreamRed<KIND, TB, KP8>) + (size_t)a.M * (a.K + 8) * 2;
   const int per_cu = lds <= kTwoLds ? 2 : 1;
+  if constexpr (KIND == kStLines || KIND == kStF8Lines)
+    if (a.K == 4096 && a.groups > 256 && a.groups <= 384)
+      return stream_launch<KIND, TB, KP8, EPI, NORM, KIND == kStLines ? 16 : 8, true>(a, 1, lds, stream);
   if constexpr (KIND >= kStF8) {
     return a.K % 4096 == 0 ? stream_launch<KIND, TB, KP8, EPI, NORM, 8>(a, per_cu, lds, stream)
                            : stream_launch<KIND, TB, KP8, EPI, NORM, 4>(a, per_cu, lds, stream);
@@ -130,7 +139,7 @@ static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
   // are what lasts (us, lines -> 16 rows, 9 / 16 rows: 1024 x 4096 8.3 / 9.1 -> 8.2 / 8.8, 2048 8.7 / 9.5 -> 8.4 / 9.1, 6144 14.2 / 15.0
   // -> 14.2 / 14.7; but 12288 20.8 / 21.8 -> 21.4 / 22.0; 2048 x 2048 5.4 / 6.1 -> 5.6 / 6.0).  Between 192 and 256 groups they are
   // level, and skinny_gemm.hip has these sizes with the bits of whole lines.
-  const bool few = a.groups <= 192 || (a.groups > 256 && a.groups <= 384);
+  const bool few = a.groups <= 192;
   if (a.M <= 16 && (F8 || (a.K == 4096 && few))) return stream_blocks<WIDE, 1, EPI, false>(a, stream);
   if (a.M <= 16) return stream_blocks<LINES, F8 ? 1 : 2, EPI, false>(a, stream);
   return stream_blocks<WIDE, 2, EPI, false>(a, stream);
