@@ -110,9 +110,10 @@ __device__ __forceinline__ void sk_prefetch(const uint16_t* const (&wrow)[RB], i
 // DEEP: a block's loads all go out ahead of its products, at 126 registers; left to itself the compiler keeps half of them
 // back for the sake of more waves, which few workgroups do not have.
 // WIDE: fragments of 16 rows x 64 B and 16 tokens; the two blocks are the halves of a chunk and add up in acc[0].
+// WHOLE: the chunks of a K part, all in flight together.
 // A K part goes by blocks of UNR chunks, then of half as many down to one: whatever K leaves over is in flight
 // together.
-template <int TB, int NC, bool PRE, bool WIDE = false, bool DEEP = false, int RB>
+template <int TB, int NC, bool PRE, bool WIDE = false, bool DEEP = false, int WHOLE = 0, int RB>
 __device__ __forceinline__ void sk_stream(const uint16_t* const (&wrow)[RB], const uint16_t* const (&xr)[TB], int nit,
                                           const u16x8 (&apre)[sk_unr(NC)][RB], f32x4 (&acc)[RB][TB]) {
   constexpr int UNR = sk_unr(NC), XH = WIDE ? 2 : 1;
@@ -148,7 +149,7 @@ __device__ __forceinline__ void sk_stream(const uint16_t* const (&wrow)[RB], con
       for (int rb = 0; rb < RB; ++rb) a[u][rb] = loadw(wrow[rb] + (it + u) * 64);
       loadx((it + u) * 64, b[u]);
     }
-    if constexpr (DEEP) __builtin_amdgcn_sched_barrier(0);
+    if constexpr (DEEP || WHOLE > 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < U; ++u) step(a[u], b[u]);
   };
@@ -161,6 +162,10 @@ __device__ __forceinline__ void sk_stream(const uint16_t* const (&wrow)[RB], con
     for (int u = 0; u < U; ++u) step(apre[u], b[u]);
   };
   using std::integral_constant;
+  if constexpr (WHOLE > 0) {
+    block(integral_constant<int, WHOLE>{}, 0);
+    return;
+  }
   int it = 0;
   if constexpr (PRE) {
     if (nit >= UNR) {

@@ -34,9 +34,9 @@ namespace mx {
 // NC: 16-channel groups per workgroup: each X fragment then feeds NC MFMAs, so X traffic per
 // streamed weight byte drops NC-fold (it equals the weight traffic at 16 tokens with NC = 1).
 // KP: K parts (sk_parts).  HALF: 8 channels a workgroup, 8 K parts, M <= 8.  WIDE: 16-row fragments and TB blocks of 16 tokens
-// (sk_wide).
+// (sk_wide).  WHOLE: chunks of a wave's K part, loaded together.
 template <int TB, int NC, int KP, bool SWO = false, bool NORM = false, bool ROPE = false, bool MERGE = false,
-          bool HALF = false, bool WIDE = false, bool DEEP = false>
+          bool HALF = false, bool WIDE = false, bool DEEP = false, int WHOLE = 0>
 __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __restrict__ X, int64_t ldx,
                                                           const uint16_t* __restrict__ W, int64_t ldw,
                                                           uint16_t* __restrict__ Y, int64_t ldy, int M, int K,
@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
   }
 
   f32x4 acc[RB][TB];
-  sk_stream<TB, NC, LDSX, WIDE, DEEP>(wrow, xr, nit, apre, acc);
+  sk_stream<TB, NC, LDSX, WIDE, DEEP, WHOLE>(wrow, xr, nit, apre, acc);
   if constexpr (HALF) {
     const f32x4 part = sk_both_halves(acc[0][0]);
     if (c < 8 && g < 2) red[w * 16 + 8 * g + c] = part;
@@ -319,6 +319,15 @@ extern "C" int mx_skinny_gemm_half(const uint16_t* x, int64_t ldx, const uint16_
   // DEEP up to where the waves that it leaves are busy (2048 x 2048, one row 3.9 -> 3.7 us, 4096 x 4096 7.7 -> 7.5, 2048 x 8192 8.0 -> 8.4)
   if (K <= 4096)
     skinny_gemm_kernel<1, 1, 8, false, false, false, false, true, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+  // One workgroup a CU has the registers for a whole K part in flight, and nothing beside it to hide its turns of 8 chunks:
+  // 2048 x 12288, a step of revesun-1b with 1 / 2 / 4 / 8 rows 758 / 791 / 838 / 966 -> 740 / 771 / 823 / 953 us.  Rows ahead of
+  // the weights or behind them: as good or worse.  Two turns are level or better left (2048 x 8192, a step of llama3.2-1b of
+  // one row 684 -> 684, beside other processes 686 -> 697).
+#define SKH(U) \
+  else if (N <= 8 * 256 && K == 512 * U) \
+    skinny_gemm_kernel<1, 1, 8, false, false, false, false, true, false, false, U><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
+  SKH(20) SKH(24) SKH(28)
+#undef SKH
   else
     skinny_gemm_kernel<1, 1, 8, false, false, false, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
   return (int)hipGetLastError();

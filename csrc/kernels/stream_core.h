@@ -223,7 +223,7 @@ __device__ __forceinline__ void stream_walk(const void* W, int64_t ldw, const fl
 }
 
 // One group and, more >= 0, half of another (more: twice the group + the half): a wave's loads of both in flight at once.
-// Half h is channels 4 h .. + 3 and 8 + 4 h .. + 3, which an epilogue pairs: 8 rows over eight K parts.  finish has a fourth
+// Half h is channels 4 h .. + 3 and 8 + 4 h .. + 3, which an epilogue pairs: 8 rows.  finish has a fourth
 // argument, whether the lane's four channels are of that half.  For the K whose part is one block (4096: kStLines of 8 parts,
 // NL 16; kStF8Lines, NL 8).
 template <int KIND, int TB, int KP, int NL, typename Row, typename Off, typename Stage, typename Finish>
@@ -233,7 +233,7 @@ __device__ __forceinline__ void stream_and_half(const void* W, int64_t ldw, cons
   constexpr bool F8 = KIND == kStF8Lines;
   static_assert(KIND == kStLines || F8, "blocks of 8 rows");
   constexpr int WB = F8 ? 1 : 2, RB = F8 ? 1 : kSkBlocks<KP, 1>, MB = (TB + 1) / 2;
-  constexpr int CK = F8 ? 128 : 64, CH = NL / RB, HN = CH * KP / 8;  // chunks of a wave's part, of its part of the half
+  constexpr int CK = F8 ? 128 : 64, CH = NL / RB;  // chunks of a wave's part
   static_assert(kStreamImages<KIND, TB, KP> == 2, "sums of both");
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -241,32 +241,33 @@ __device__ __forceinline__ void stream_and_half(const void* W, int64_t ldw, cons
   f32x4* const red = reinterpret_cast<f32x4*>(smem);
   f32x4* const hred = red + kStreamPlaces<KIND, TB, KP>;
   uint16_t* const xs = reinterpret_cast<uint16_t*>(smem + kStreamRed<KIND, TB, KP>);
-  const int kl = F8 ? 2 * sk_lane_k(c, g) : sk_lane_k(c, g), k0 = sk_part<KP>(w) * (K / KP) + kl, kh = w * (K / 8) + kl;
+  const int kl = F8 ? 2 * sk_lane_k(c, g) : sk_lane_k(c, g), k0 = sk_part<KP>(w) * (K / KP) + kl;
   const int hg = more >> 1, h = more & 1, hc = 4 * h + (c & 3) + 8 * (c >> 2 & 1);
   WFrag<KIND, NL, RB> f;
-  WFrag<KIND, HN, 1> f2;
+  WFrag<KIND, CH, 1> f2;
+  const bool extra = more >= 0 && w < KP;  // (the same parts and sums as a whole group's: the same bits)
   stage(xs, ldx, [&]() __attribute__((always_inline)) {
     uint32_t o[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
       o[rb] = (uint32_t)(off(8 * sk_half<KP>(w, rb) + (c & 7)) * (uint32_t)ldw + (uint32_t)k0) * WB;
     f.load(reinterpret_cast<const char*>(W) + row(grp) * ldw * WB, o);
-    if (more >= 0) {
-      const uint32_t o2[1] = {(uint32_t)(off(hc) * (uint32_t)ldw + (uint32_t)kh) * WB};
+    if (extra) {
+      const uint32_t o2[1] = {(uint32_t)(off(hc) * (uint32_t)ldw + (uint32_t)k0) * WB};
       f2.load(reinterpret_cast<const char*>(W) + row(hg) * ldw * WB, o2);
     }
   });
-  auto products = [&](const auto& fr, int chunks, int k, auto& acc) __attribute__((always_inline)) {
+  auto products = [&](const auto& fr, auto& acc) __attribute__((always_inline)) {
     constexpr int R = std::extent<std::remove_reference_t<decltype(acc)>>::value;
     const uint16_t* xr[TB];
 #pragma unroll
-    for (int tb = 0; tb < TB; ++tb) xr[tb] = xs + min(tb * 8 + (c & 7), M - 1) * ldx + k;
+    for (int tb = 0; tb < TB; ++tb) xr[tb] = xs + min(tb * 8 + (c & 7), M - 1) * ldx + k0;
 #pragma unroll
     for (int rb = 0; rb < R; ++rb)
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb) acc[rb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int u = 0; u < chunks; ++u) {
+    for (int u = 0; u < CH; ++u) {
       if constexpr (F8) {
         u16x8 a0, a1;
         fr.get(u, a0, a1);
@@ -288,12 +289,12 @@ __device__ __forceinline__ void stream_and_half(const void* W, int64_t ldw, cons
   const SkSum<TB, 1, KP> sum{red};
   {
     f32x4 acc[RB][TB];
-    products(f, CH, k0, acc);
+    products(f, acc);
     sum.put(w, c, g, acc);
   }
-  if (more >= 0) {
+  if (extra) {
     f32x4 acc[1][TB];
-    products(f2, HN, kh, acc);
+    products(f2, acc);
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) {
       const f32x4 s = sk_both_halves(acc[0][tb]);
@@ -314,7 +315,7 @@ __device__ __forceinline__ void stream_and_half(const void* W, int64_t ldw, cons
       s = f32x4{0.f, 0.f, 0.f, 0.f};
       const int e = min(2 * mb + (c >> 3), TB - 1) * 16 + 8 * (g >> 1) + (c & 7);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) s += hred[i * TB * 16 + e];
+      for (int i = 0; i < KP; ++i) s += hred[i * TB * 16 + e];
     }
     if constexpr (F8) s *= sc;
     finish(s, mb, cg, w == 0 || (g & 1) == h);

@@ -21,8 +21,11 @@
 // 43.7 / 44.4) against skinny_gemm's 39.8 / 41.0 / 42.8 / 54.6 and hipBLASLt's 61 to 64; 16384 x 2048 (67 MB), 4 / 8 / 16 rows 12.9 /
 // 13.4 / 15.4 (15.8 / 16.4 / 16.5); in e4m3, 28672 x 4096, rows 1 / 4 / 8: 22.2 / 22.4 / 22.8 (24.6 / 25.4 / 25.7 in
 // 16 rows x 64 B) against fp8_gemm's 27.1 / 31.5 / 34.1; 4096 x 14336, 1 / 4 rows 12.9 / 14.3 (14.3 / 16.1).
-// Left: the last groups' uneven end (6144 x 4096 is 384 groups on 256 workgroups: 13.0 us for 50 MB; the last 128 as
-// 256 halves: no change, a half's loads take a whole one's turns), and the launch's own 2 us before the first bytes arrive.
+// 6144 x 4096 is 384 groups on 256 CUs: half of the CUs had two and ended at 9.2 us where the others did at 6.7 (e4m3, 4 rows,
+// in a step). 257 to 384 groups go as one and a half a workgroup, all loads in flight (stream_and_half): steps of
+// llama3.1-8b with 1 / 4 / 8 / 16 rows 2990 / 3183 / 3520 / 3760 -> 2913 / 3106 / 3434 / 3752 us, in e4m3 1 / 4 / 8 rows 2048 /
+// 2289 / 2619 -> 2041 / 2275 / 2585 (eight parts of K for a half: other bits, and no faster).
+// Left: the launch's own 2 us before the first bytes arrive.
 #include <algorithm>
 
 #include "decode_fuse.h"
@@ -135,10 +138,10 @@ static int stream_rows(const StreamArgs& a, bool norm, hipStream_t stream) {
   constexpr int LINES = F8 ? kStF8Lines : kStLines, WIDE = F8 ? kStF8 : kStWide;
   if (norm) return stream_blocks<LINES, 1, EPI, true>(a, stream);
   if (a.M <= 8) return stream_blocks<LINES, 1, EPI, false>(a, stream);
-  // 9 to 16 rows: whole lines, but for a K of 4096 of up to one and a half groups a CU, where the first bytes and the rows in LDS
-  // are what lasts (us, lines -> 16 rows, 9 / 16 rows: 1024 x 4096 8.3 / 9.1 -> 8.2 / 8.8, 2048 8.7 / 9.5 -> 8.4 / 9.1, 6144 14.2 / 15.0
-  // -> 14.2 / 14.7; but 12288 20.8 / 21.8 -> 21.4 / 22.0; 2048 x 2048 5.4 / 6.1 -> 5.6 / 6.0).  Between 192 and 256 groups they are
-  // level, and skinny_gemm.hip has these sizes with the bits of whole lines.
+  // 9 to 16 rows: whole lines, but for a K of 4096 of few groups, where the first bytes and the rows in LDS are what lasts (us,
+  // lines -> 16 rows, 9 / 16 rows: 1024 x 4096 8.3 / 9.1 -> 8.2 / 8.8, 2048 8.7 / 9.5 -> 8.4 / 9.1; but 12288 20.8 / 21.8 -> 21.4 /
+  // 22.0; 2048 x 2048 5.4 / 6.1 -> 5.6 / 6.0).  Between 192 and 256 groups they are level, and skinny_gemm.hip has these
+  // sizes with the bits of whole lines.
   const bool few = a.groups <= 192;
   if (a.M <= 16 && (F8 || (a.K == 4096 && few))) return stream_blocks<WIDE, 1, EPI, false>(a, stream);
   if (a.M <= 16) return stream_blocks<LINES, F8 ? 1 : 2, EPI, false>(a, stream);

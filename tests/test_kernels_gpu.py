@@ -886,6 +886,16 @@ def test_skinny_linear_half(gpu, M, N, K):
     assert y.shape == (M, N) and rel_err(y, x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 6144), (8, 2048, 8192), (3, 72, 10240), (5, 2048, 12288), (2, 1024, 14336), (8, 64, 16384)])
+def test_skinny_linear_half_whole_parts(gpu, M, N, K):
+    """A wave's whole K part in flight (12 to 28 chunks) and the sizes beside them."""
+    torch.manual_seed(M + N)
+    x = torch.randn(M, K, device=gpu, dtype=torch.bfloat16)
+    w = torch.randn(N, K + 8, device=gpu, dtype=torch.bfloat16)[:, :K] * 0.05
+    assert rel_err(_ops().skinny_linear_half(x, w), x.double() @ w.double().t()) < 2 ** -8  # one bf16 rounding
+
+
 def _stream_weight(w, f8):
     from mxllm.serve.quant import quantize_e4m3
 
@@ -919,6 +929,42 @@ def test_stream_linear(gpu, M, N, K, f8):
                 got, h2 = _ops().stream_linear(x, d, gamma, 1e-5, w, s, sw)
                 assert torch.equal(h2, hn)
                 assert torch.equal(got, _ops().stream_linear(xn, None, None, 0.0, w, s, sw)[0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f8", [False, True])
+@pytest.mark.parametrize("M", [1, 4, 7, 8, 9, 16])
+@pytest.mark.parametrize("groups", [257, 300, 384])
+def test_stream_group_and_half(gpu, groups, M, f8):
+    """257 to 384 groups of a K of 4096: a workgroup's group and half of another, one of them to every CU; plain, SwiGLU and
+    QKV epilogues (a half has both channels of a pair), with the norm up to 4 rows."""
+    from mxllm import ops
+
+    torch.manual_seed(M + groups)
+    K, N, D = 4096, 16 * groups, 128
+    x = torch.randn(M, K, device=gpu, dtype=torch.bfloat16)
+    w, s = _stream_weight(torch.randn(N, K, device=gpu, dtype=torch.bfloat16) * 0.05, f8)
+    y = _ops().stream_linear(x, None, None, 0.0, w, s, False)[0]
+    wd = w.view(torch.float8_e4m3fn).double() * s.double()[:, None] if f8 else w.double()
+    assert rel_err(y, x.double() @ wd.t()) < 2 ** -8  # one bf16 rounding
+    assert torch.equal(y, _ops().w8_linear(x, w, s) if f8 else _ops().skinny_linear(x, w))
+    assert torch.equal(_ops().stream_linear(x, None, None, 0.0, w, s, True)[0], ops.swiglu(y))
+    d, gamma = torch.randn_like(x), (1.0 + 0.1 * torch.randn(K, device=gpu)).to(torch.bfloat16)
+    if M <= 4:
+        xn, hn = ops.add_rms_norm(d, x, gamma, 1e-5)
+        got, h2 = _ops().stream_linear(x, d, gamma, 1e-5, w, s, False)
+        y = _ops().stream_linear(xn, None, None, 0.0, w, s, False)[0]
+        assert torch.equal(h2, hn) and torch.equal(got, y)
+    if groups == 384:
+        Hq, Hkv, norm = 32, 8, M <= 4
+        cos, sin = ref.rope_tables(64, D, 500000.0, None, gpu)
+        slots, pos = torch.randperm(M, device=gpu).to(torch.int32), torch.randint(0, 64, (M,), device=gpu, dtype=torch.int32)
+        kc, vc = (torch.randn(M, Hkv, 64, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        kc2, vc2 = kc.clone(), vc.clone()
+        q, _ = _ops().stream_qkv_rope(x, d if norm else None, gamma if norm else None, 1e-5, w, s, cos, sin, pos, slots, kc, vc,
+                                      Hq, Hkv, None)
+        q_ref = _ops().rope_append(y, cos, sin, pos, slots, kc2, vc2, Hq, Hkv, D, None)
+        assert torch.equal(q.view(M, -1), q_ref.reshape(M, -1)) and torch.equal(kc, kc2) and torch.equal(vc, vc2)
 
 
 @pytest.mark.gpu
