@@ -269,7 +269,10 @@ using namespace mx;
 //    So they are by a step of up to 32 sequences from 20 M weights on (6144 x 4096 at 17 / 24 / 32 rows .89, .99, 1.0 times as fast, 16384 x
 //    2048 1.03, .97, .96; but 4096 x 4096 1.18, 1.16, 1.16, 2048 x 8192 1.16, 1.14, 1.33);
 //  * a K of 12288 and more: up to 2^20 outputs, then gemm8 in parts of K (4096 x 14336 at 256 / 512 / 1024 rows 60.3* / 68.5* /
-//    103.6* -> 47.6 / 68.4 / 119; 2048 x 12288 at 512 / 1400 1.18 and .87 times as fast).
+//    103.6* -> 47.6 / 68.4 / 119; 2048 x 12288 at 512 / 1400 1.18 and .87 times as fast);
+//  * up to 256 channels of a prompt are not cut along K: a gate of 128 x 4096 at 2048 rows takes 13 us for 20, 1 % of sigusun-8b's
+//    pass, but f32 sums in parts round otherwise than one sum in order, and where an expert's choice is close that shows in
+//    a pass' outputs (one of 17 differed by 3 %; the other way round as often). In one part the library has it faster.
 extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 16 || K % 64) return -1;
   const int64_t weights = (int64_t)N * K;
@@ -293,7 +296,7 @@ extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
       }
     }
   }
-  return plan;
+  return N <= 256 && M >= 512 && plan % 64 > 1 ? -1 : plan;
 }
 
 // C[M, N] = A . B^T, or C[M, N / 2] = silu(gate) up, by tile `tile` with K in `parts`; parts > 1: ws holds parts * M * N floats.

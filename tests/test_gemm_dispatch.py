@@ -158,7 +158,7 @@ def test_ragged_row_rules():
 TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (33, 10240, 4096), (32, 4096, 4096), (17, 4096, 14336), (256, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
            (1, 64, 4096), (40, 3360, 2048)]
 TILE_OFF = [(192 * 16 + 1, 192 * 16, 2048), (255, 12288, 4096), (127, 8192, 8192), (257, 4096, 14336), (513, 2048, 12288), (40, 3368, 2048), (40, 2048, 2080),
-            (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048)]
+            (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048), (2048, 128, 4096), (512, 256, 4096)]
 
 
 def test_tile_plan():
