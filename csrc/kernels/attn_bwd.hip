@@ -788,10 +788,10 @@ __device__ __forceinline__ void vm_wait_le(int n) {
 }
 
 // ============================================================================================
-// Measured-slower backward variant (VERDICT r5 weak 2): compiled only with -DMXLLM_ATTN_EXPERIMENTS.
+// Measured-slower backward variant: compiled only with -DMXLLM_ATTN_EXPERIMENTS.
 // The default build has ONE D = 128 backward family: attn_bwd8_kernel + attn_bwd_dq_kernel.
 #ifdef MXLLM_ATTN_EXPERIMENTS
-// Staggered split-mode key-block kernel (MXLLM_ATTN_BWD8=2; VERDICT r4 item 4).  Same work split
+// Staggered split-mode key-block kernel (MXLLM_ATTN_BWD8=2).  Same work split
 // as attn_bwd8_kernel (8 waves = 4 key groups x 2 q halves, 128 keys of one q head per workgroup),
 // but the two q halves run HALF A TILE apart: each tile is two phases -- A: S = Q K^T, dP = dO V^T
 // and the softmax, B: dV^T += dO^T P, dK^T += Q^T dS -- separated by a barrier, and waves 4-7 start

@@ -514,7 +514,7 @@ attn_fwd_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, 
 }
 
 // ============================================================================================
-// Measured-slower forward variants (VERDICT r5 weak 2): compiled only with
+// Measured-slower forward variants: compiled only with
 // -DMXLLM_ATTN_EXPERIMENTS (python -m mxllm._build with MXLLM_FILE_FLAGS="attn_fwd.hip=-DMXLLM_ATTN_EXPERIMENTS").
 // The default build has ONE forward family, attn_fwd_kernel<D, CAUSAL, 4>.
 #ifdef MXLLM_ATTN_EXPERIMENTS

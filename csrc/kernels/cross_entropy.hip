@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(256) ce_fwd_bwd_kernel(uint16_t* __restrict__ 
 }
 
 // fp32-logits form: the head GEMM wrote fp32 logits (no bf16 rounding of the scores the loss is
-// computed from, VERDICT r3 missing 4); the loss uses them as they are and the gradient
+// computed from); the loss uses them as they are and the gradient
 // (softmax - onehot) * inv_n is written in bf16 to `dl` (the operand of the backward GEMMs).
 __global__ void __launch_bounds__(256) ce_fwd_bwd_f32_kernel(const float* __restrict__ logits,
                                                              uint16_t* __restrict__ dl,

@@ -15,7 +15,7 @@ __device__ __forceinline__ int g8_lane() {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Persistent 4-phase variant (VERDICT r4 item 3): min(tiles, CUs) workgroups, each walking output
+// Persistent 4-phase variant: min(tiles, CUs) workgroups, each walking output
 // tiles t = L, L + G, ... (L = the XCD-contiguous remap of its id, so the G tiles in flight at a
 // time form 8 contiguous ranges, one per XCD / L2).  Between two tiles the NEXT tile's prologue
 // DMA (K-tile 0 and K-tile 1's B images) is issued BEFORE the current tile's epilogue stores, so

@@ -241,7 +241,7 @@ int launch(int mode, char* const* bases, const void* in, void* out, int64_t n, i
 }
 
 // ============================================================================================
-// CU-light schedule (VERDICT r5 Missing 4): no workgroup waits on a peer except ONE wave.
+// CU-light schedule: no workgroup waits on a peer except ONE wave.
 // The resident kernel above keeps `wgs` workgroups spinning on peer flags for the whole call
 // (24.5 % off a concurrent GEMM at 32 WGs, profiles/r5j).  Here a call is cut into segments of
 // at most `cap` bytes per peer, and each segment with host epoch e (identical on every rank:
