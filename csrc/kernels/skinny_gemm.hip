@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(512) skinny_gemm_kernel(const uint16_t* __rest
 }  // namespace mx
 
 // Where the kernel whose workgroups stay (stream_gemm.hip: X in LDS once a CU) takes less time, with the same bits but for its
-// 16-row fragments of a K of 4096 and up to 6144 channels, which go there as long as the addresses allow (us, here ->
+// 16-row fragments of a K of 4096 and up to 3072 channels, which go there as long as the addresses allow (us, here ->
 // there: K 2048, 3 / 8 / 32 rows: 3072 channels 5.2 / 6.1 / 8.8 -> 5.1 / 5.3 / 8.5, 16384 13.8 / 17.0 / 29.7 -> 13.0 / 13.4 / 18.6,
 // 2 rows 12.8 -> 13.0; K 4096, 16 rows: 1024 channels 9.7 -> 9.1, 4096, one group a CU, 10.2 -> 10.5).
 extern "C" int mx_stream_gemm(const uint16_t* x, int64_t ldx, const void* w, int64_t ldw, const float* scale, uint16_t* y,
