@@ -181,8 +181,10 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
   if (lane == 0) scratch[wid] = v;
   __syncthreads();
   float r = 0.f;
+  for (int i = 0; i < nw; i += 4) {  // (four on their way at once)
 #pragma unroll
-  for (int i = 0; i < 16; ++i) r += i < nw ? scratch[i] : 0.f;  // (all on their way at once)
+    for (int j = 0; j < 4; ++j) r += i + j < nw ? scratch[i + j] : 0.f;
+  }
   return r;
 }
 
@@ -194,8 +196,10 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
   if (lane == 0) scratch[wid] = v;
   __syncthreads();
   float r = -INFINITY;
+  for (int i = 0; i < nw; i += 4) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) r = fmaxf(r, i < nw ? scratch[i] : -INFINITY);
+    for (int j = 0; j < 4; ++j) r = fmaxf(r, i + j < nw ? scratch[i + j] : -INFINITY);
+  }
   return r;
 }
 
