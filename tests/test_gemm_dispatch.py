@@ -155,10 +155,14 @@ def test_ragged_row_rules():
 
 
 # (M, N, K): both sides of the lines of csrc/kernels/gemm_tile.hip mx_gemm_tile_plan
-TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (33, 10240, 4096), (32, 4096, 4096), (17, 4096, 14336), (256, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
-           (1, 64, 4096), (40, 3360, 2048)]
+TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (33, 2560, 4096), (32, 2048, 8192), (17, 4096, 14336), (430, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
+           (1, 64, 4096), (40, 3360, 2048),
+           (370, 3072, 2048), (290, 2048, 2048), (549, 2048, 8192), (150, 6144, 4096)]
 TILE_OFF = [(192 * 16 + 1, 192 * 16, 2048), (255, 12288, 4096), (127, 8192, 8192), (257, 4096, 14336), (513, 2048, 12288), (40, 3368, 2048), (40, 2048, 2080),
-            (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048), (2048, 128, 4096), (512, 256, 4096)]
+            (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048), (2048, 128, 4096), (512, 256, 4096),
+            # (the library was quicker by 4 to 18 %)
+            (386, 6144, 4096), (430, 6144, 4096), (290, 4096, 4096), (370, 4096, 4096), (687, 4096, 4096), (290, 16384, 4096), (370, 16384, 4096),
+            (370, 8192, 8192), (600, 8192, 8192), (370, 16384, 2048), (506, 5376, 4096), (10, 4096, 14336), (22, 6144, 16384)]
 
 
 def test_tile_plan():
@@ -166,6 +170,8 @@ def test_tile_plan():
 
     assert [s for s in TILE_ON if gemm.tile_plan(*s) is None] == [] and [s for s in TILE_OFF if gemm.tile_plan(*s) is not None] == []
     assert gemm.tile_plan(48, 28672, 4096, True) and not gemm.tile_plan(48, 28672, 4096) and not gemm.tile_plan(48, 57344, 8192, True)
+    assert not gemm.tile_plan(130, 28672, 4096, True) and gemm.tile_plan(200, 28672, 4096, True) and gemm.tile_plan(135, 21504, 4096, True) and not gemm.tile_plan(16, 7168, 16384, True)
+    assert gemm.tile_plan(9, 1024, 4096, True)[1] <= 8  # (in 16 parts the sum and its activation are what lasts)
     assert native().gemm_tile_plan(0, 64, 64, False) == native().gemm_tile_plan(1 << 40, 64, 64, False) == -1
 
 
@@ -173,7 +179,7 @@ def test_tile_plan_is_one_turn():
     """Whatever the sizes: tiles and parts of K that the CUs hold at once, four 64s of K a part and more."""
     import random
 
-    tiles = [(64, 64, 512), (64, 128, 256), (128, 128, 256), (128, 192, 256), (128, 256, 256), (160, 192, 256), (192, 192, 256)]
+    tiles = [(64, 64, 256), (64, 128, 256), (128, 128, 256), (128, 192, 256), (128, 256, 256), (160, 192, 256), (192, 192, 256)]
     r, seen = random.Random(0), set()
     for _ in range(4000):
         M, N, K = int(2 ** r.uniform(0, 13)), 16 * int(2 ** r.uniform(0, 11)), 64 * int(2 ** r.uniform(0, 9))
