@@ -224,10 +224,10 @@ gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __
   }
 }
 
-// The tiles, and what a turn of them takes, us: start + steps of 64 k (step + load units / 256) + memory MB of weights + with K in
-// parts, sum + part parts (part + glu with SwiGLU) + image MB of f32 images.  Fitted to 89,000 runs of 350 sizes of weights at 9 to 4,200 rows,
-// weights from memory: 4 to 6 % off in the mean, the tile so chosen 1 % behind the best one.  One tile a CU at most: two of 64 x 64 on a
-// CU take 1.8 times as long.
+// The tiles, and what a turn of them takes, us: start + steps of 64 k (step + load units / 256) + memory MB of weights + with K
+// in parts, sum + part parts (part + glu with SwiGLU) + image MB of f32 images.  Fitted to 89,000 runs of 350 sizes of weights
+// at 9 to 4,200 rows, weights from memory: 4 to 6 % off in the mean, the tile so chosen 1 % behind the best one.  One tile a CU
+// at most: two of 64 x 64 on a CU take 1.8 times as long.
 struct GtTile {
   int tm, tn;
   float start, step, load, sum, part, image, memory, glu;
@@ -241,9 +241,9 @@ constexpr GtTile kGtTiles[] = {{64, 64, 2.55f, .169f, .065f, 1.90f, .152f, .497f
                                {192, 192, 6.97f, .547f, .202f, 1.14f, .093f, .316f, .056f, .138f}};
 constexpr int kGtCount = sizeof(kGtTiles) / sizeof(GtTile), kGtPlaces = 256;
 
-// What the library takes where it has a good kernel, us: the quickest tenth of the same sizes.  Its tiles are not known; it is as quick as
-// the best of these would be, in as many turns as they need.  It is slower by 16 % in the mean, and by half and more between the
-// sizes that it is tuned for.
+// What the library takes where it has a good kernel, us: the quickest tenth of the same sizes.  Its tiles are not known; it is
+// as quick as the best of these would be, in as many turns as they need.  It is slower by 16 % in the mean, and by half and
+// more between the sizes that it is tuned for.
 static float gt_library(int64_t M, int64_t N, int64_t K) {
   constexpr int edge[] = {32, 64, 96, 128, 160, 192, 224, 256};
   float step = INFINITY;
@@ -279,45 +279,51 @@ static void gt_launch(int tile, int grid, const uint16_t* A, int64_t lda, const 
 
 using namespace mx;
 
-// Tile and parts of K for a product, as 64 tile + parts, by the modelled time; -1: it is not one turn of tiles, or the library, or
-// another kernel, may have it faster.  Where the lines lie (us, hipBLASLt, or gemm8 marked * -> here):
-//  * K in one part of more than 1,024: tiles past 64 x 64 only where 7 of 8 CUs have one. With fewer the library's kernels are as quick
-//    or quicker at one size of seven (6144 x 4096 at 386 rows, 192 tiles, 30.9 -> 36.8; 4096 x 4096 at 687, 192, 32.3 -> 36.5), with as many at
-//    one of fifty (4096 x 4096 at 1024, 256 tiles, 42.1 -> 38.9). A K up to 1,024 is over before it matters (8192 x 512 at 181 rows,
-//    192 tiles, 9.3 -> 5.9);
-//  * not where the library at its best (gt_library, with SwiGLU and its activation's launch) would be faster. The model may be longer than
-//    that by 3 % (2048 x 8192 at 290 / 549 rows, by 1 % longer, 32.3 / 44.4 -> 25.1 / 33.7); up to 32 rows by 5 % (12 with SwiGLU of more
-//    than 44 M weights); up to 192 rows, where the library is seldom at its best, by 12 % (6144 x 4096 at 150 39.6 -> 24.9); in one part of
-//    filled turns or of the smallest tile by 10 % (2048 x 8192 at 2709 91 -> 84). Past each of these lines more than one size of 50
-//    is slower here; of 3,100 sizes of 139 weights that go here and the fit had not seen, 16 are by more than 3 %, the worst by 13 %, and 24
-//    more of those of the next line (profiles/gemm_routes/tile.txt);
-//  * past 32 rows, which no step's graph holds, what is over in 17 us (24 with SwiGLU) is taken all the same: the library's call costs the
-//    host 21 us, this one 11, in parts 15. A prompt of 290 / 370 / 430 tokens of llama3.2-1b takes 2.85 / 2.83 / 2.82 ms with the
-//    library's products and 1.94 / 1.98 / 2.00 with these, though 370 rows of 3072 x 2048 alone are 15.1 us there and 16.1 here;
-//  * more than 44 M weights (12288 x 4096 and up) are read at the rate of memory by the library as well, from 256 rows (K of 8192:
-//    128) on it falls behind: 12288 x 4096 at 64 / 256 / 700 rows 26.7 / 1.21 / 1.23 times as fast here (26.8 at 64), 16384 x 4096 at
-//    128 37.3 -> 41.8, 8192 x 8192 at 64 / 128 / 256 33.6 / 50.9 / 1.66 times (39.0, 43.0);
-//    So they are by a step of up to 32 sequences from 20 M weights on (6144 x 4096 at 17 / 24 / 32 rows .89, .99, 1.0 times as fast, 16384 x
-//    2048 1.03, .97, .96; but 4096 x 4096 1.18, 1.16, 1.16, 2048 x 8192 1.16, 1.14, 1.33), but for a K of 12288 and more of up to 4096
-//    channels past 16 rows (4096 x 14336 at 10 / 17 / 32 26.3 / 28.6 / 32.6 -> 27.1 / 26.0 / 26.4; 6144 x 16384 at 22 42.2 -> 50.7). With SwiGLU, whose launch is saved, up to 128 M
-//    (28672 x 4096 at 22 / 37 / 110 rows 54.2 / 51.0 / 54.7 -> 46.3 / 46.7 / 50.7; 57344 x 8192 is gemm8's), from 129 to 192 rows 100 M
-//    (28672 x 4096 at 130 / 157 / 205 61.4 / 60.5 / 73.7 -> 63.3 / 61.8 / 68.0, 21504 x 4096 at 135 61.1 -> 52.5), and a K of 12288 and more from 33 rows on (7168 x 16384
-//    at 16 51.5 -> 66.9);
+// Tile and parts of K for a product, as 64 tile + parts, by the modelled time; -1: it is not one turn of tiles, or the library,
+// or another kernel, may have it faster.  Where the lines lie (us, hipBLASLt, or gemm8 marked * -> here):
+//  * K in one part of more than 1,024: tiles past 64 x 64 only where 7 of 8 CUs have one. With fewer the library's kernels are
+//    as quick or quicker at one size of seven (6144 x 4096 at 386 rows, 192 tiles, 30.9 -> 36.8; 4096 x 4096 at 687, 192, 32.3
+//    -> 36.5), with as many at one of fifty (4096 x 4096 at 1024, 256 tiles, 42.1 -> 38.9). A K up to 1,024 is over before it
+//    matters (8192 x 512 at 181 rows, 192 tiles, 9.3 -> 5.9);
+//  * not where the library at its best (gt_library, with SwiGLU and its activation's launch) would be faster. The model may be
+//    longer than that by 3 % (2048 x 8192 at 290 / 549 rows, by 1 % longer, 32.3 / 44.4 -> 25.1 / 33.7); up to 32 rows by 5 %
+//    (12 with SwiGLU of more than 44 M weights); up to 192 rows, where the library is seldom at its best, by 12 % (6144 x 4096
+//    at 150 39.6 -> 24.9); in one part of filled turns or of the smallest tile by 10 % (2048 x 8192 at 2709 91 -> 84). Past
+//    each of these lines more than one size of 50 is slower here; of 3,000 sizes of 139 weights that go here and the fit had
+//    not seen, 15 are by more than 3 %, the worst by 13 %, and 22 more of those of the next line
+//    (profiles/gemm_routes/tile.txt);
+//  * past 32 rows, which no step's graph holds, what is over in 17 us (24 with SwiGLU) is taken all the same: the library's
+//    call costs the host 21 us, this one 11, in parts 15. A prompt of 290 / 370 / 430 tokens of llama3.2-1b takes 2.85 / 2.83 /
+//    2.82 ms with the library's products and 1.94 / 1.98 / 2.00 with these, though 370 rows of 3072 x 2048 alone are 15.1 us
+//    there and 16.1 here;
+//  * more than 44 M weights (12288 x 4096 and up) are read at the rate of memory by the library as well, from 256 rows (K of
+//    8192: 128) on it falls behind: 12288 x 4096 at 64 / 256 / 700 rows 26.7 / 1.21 / 1.23 times as fast here (26.8 at 64),
+//    16384 x 4096 at 128 37.3 -> 41.8, 8192 x 8192 at 64 / 128 / 256 33.6 / 50.9 / 1.66 times (39.0, 43.0). So they are by a
+//    step of up to 32 sequences from 20 M weights on (6144 x 4096 at 17 / 24 / 32 rows .89, .99, 1.0 times as fast, 16384 x
+//    2048 1.03, .97, .96; but 4096 x 4096 1.18, 1.16, 1.16, 2048 x 8192 1.16, 1.14, 1.33), but for a K of 12288 and more of up
+//    to 4096 channels past 16 rows (4096 x 14336 at 10 / 17 / 32 26.3 / 28.6 / 32.6 -> 27.1 / 26.0 / 26.4; 6144 x 16384 at 22
+//    42.2 -> 50.7). With SwiGLU, whose launch is saved, up to 128 M (28672 x 4096 at 22 / 37 / 110 rows 54.2 / 51.0 / 54.7 ->
+//    46.3 / 46.7 / 50.7; 57344 x 8192 is gemm8's), from 129 to 192 rows 100 M (28672 x 4096 at 130 / 157 / 205 61.4 / 60.5 /
+//    73.7 -> 63.3 / 61.8 / 68.0, 21504 x 4096 at 135 61.1 -> 52.5), and a K of 12288 and more from 33 rows on (7168 x 16384 at
+//    16 51.5 -> 66.9);
 //  * a K of 12288 and more: up to 2^20 outputs, then gemm8 in parts of K (4096 x 14336 at 256 / 512 / 1024 rows 60.3* / 68.5* /
 //    103.6* -> 47.6 / 68.4 / 119; 2048 x 12288 at 512 / 1400 1.18 and .87 times as fast);
-//  * up to 256 channels of a prompt are not cut along K: a gate of 128 x 4096 at 2048 rows takes 13 us for 20, 1 % of sigusun-8b's
-//    pass, but f32 sums in parts round otherwise than one sum in order, and where an expert's choice is close that shows in
-//    a pass' outputs (one of 17 differed by 3 %; the other way round as often). In one part the library has it faster.
+//  * up to 256 channels, which are gates and routers, are not cut along K, whatever the rows: the side gate of sigusun-8b, 64 x
+//    4096, takes 8 us for the library's 11 at 48 to 400 rows and 13 for 20 at 2048, 1 % of the pass, but f32 sums in parts
+//    round otherwise than one sum in order, and where an expert's choice is close that shows in a pass' outputs (one of 17
+//    differed by 3 %; the other way round as often). In one part, of which no line above is stretched for them, the library
+//    mostly has it faster.
 extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 16 || K % 64) return -1;
   const int64_t weights = (int64_t)N * K;
   const bool lengthy = K >= 12288;
   if (lengthy && (int64_t)M * N > (1 << 20)) return -1;
   if (swiglu ? weights > (M <= 128 || M > 192 ? 128000000 : 100000000) || (lengthy && M <= 32)
-             : (!lengthy && weights > 44000000 && M < (K >= 8192 ? 128 : 256)) || (M <= 32 && weights > 20000000 && (!lengthy || M <= 16 || N > 4096)))
+             : (!lengthy && weights > 44000000 && M < (K >= 8192 ? 128 : 256)) ||
+                   (M <= 32 && weights > 20000000 && (!lengthy || M <= 16 || N > 4096)))
     return -1;
   const int nk = K / 64;
-  const float quick = M <= 32 ? 0.f : swiglu ? 24.f : 17.f;
+  const float quick = M <= 32 || N <= 256 ? 0.f : swiglu ? 24.f : 17.f;
   float best = INFINITY;
   int plan = -1;
   for (int i = 0; i < kGtCount; ++i) {
@@ -325,7 +331,7 @@ extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
     const int64_t tiles = gt_units(t, M, N);
     for (int S : {1, 2, 3, 4, 6, 8, 12, 16}) {
       const int64_t u = tiles * S;
-      if (u > kGtPlaces || (S > 1 && nk < 4 * S)) break;
+      if (u > kGtPlaces || (S > 1 && (nk < 4 * S || N <= 256))) break;
       float us = t.start + (float)nk / S * (t.step + t.load * u / kGtPlaces) + t.memory * weights * 2e-6f;
       if (S > 1) us += t.sum + (t.part + (swiglu ? t.glu : 0.f)) * S + t.image * ((float)S * M * N * 4e-6f);
       if (S == 1 && i && !swiglu && K > 1024 && 8 * u < 7 * kGtPlaces && us > quick) continue;
@@ -338,8 +344,8 @@ extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
   const bool steady = !swiglu && plan % 64 == 1 && (plan / 64 < 1 || plan / 64 > 2 || K <= 1024);
   float most = gt_library(M, N, K);
   if (swiglu) most += 1.5f + .3f * ((float)M * N * 3e-6f);  // (its bytes: N in, N / 2 out)
-  most *= M <= 32 && !(swiglu && weights > 44000000) ? 1.05f : M <= 192 ? 1.12f : steady ? 1.1f : 1.03f;
-  return best < std::max(most, quick) && !(N <= 256 && M >= 512 && plan % 64 > 1) ? plan : -1;
+  if (N > 256) most *= M <= 32 && !(swiglu && weights > 44000000) ? 1.05f : M <= 192 ? 1.12f : steady ? 1.1f : 1.03f;
+  return best < std::max(most, quick) ? plan : -1;
 }
 
 // C[M, N] = A . B^T, or C[M, N / 2] = silu(gate) up, by tile `tile` with K in `parts`; parts > 1: ws holds parts * M * N floats.

@@ -156,13 +156,13 @@ def test_ragged_row_rules():
 
 # (M, N, K): both sides of the lines of csrc/kernels/gemm_tile.hip mx_gemm_tile_plan
 TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (33, 2560, 4096), (32, 2048, 8192), (17, 4096, 14336), (430, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
-           (1, 64, 4096), (40, 3360, 2048),
+           (40, 3360, 2048),
            (370, 3072, 2048), (290, 2048, 2048), (549, 2048, 8192), (150, 6144, 4096)]
 TILE_OFF = [(192 * 16 + 1, 192 * 16, 2048), (255, 12288, 4096), (127, 8192, 8192), (257, 4096, 14336), (513, 2048, 12288), (40, 3368, 2048), (40, 2048, 2080),
             (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048), (2048, 128, 4096), (512, 256, 4096),
             # (the library was quicker by 4 to 18 %)
             (386, 6144, 4096), (430, 6144, 4096), (290, 4096, 4096), (370, 4096, 4096), (687, 4096, 4096), (290, 16384, 4096), (370, 16384, 4096),
-            (370, 8192, 8192), (600, 8192, 8192), (370, 16384, 2048), (506, 5376, 4096), (10, 4096, 14336), (22, 6144, 16384)]
+            (370, 8192, 8192), (600, 8192, 8192), (370, 16384, 2048), (506, 5376, 4096), (10, 4096, 14336), (22, 6144, 16384), (48, 64, 4096), (300, 64, 4096)]
 
 
 def test_tile_plan():
@@ -173,6 +173,16 @@ def test_tile_plan():
     assert not gemm.tile_plan(130, 28672, 4096, True) and gemm.tile_plan(200, 28672, 4096, True) and gemm.tile_plan(135, 21504, 4096, True) and not gemm.tile_plan(16, 7168, 16384, True)
     assert gemm.tile_plan(9, 1024, 4096, True)[1] <= 8  # (in 16 parts the sum and its activation are what lasts)
     assert native().gemm_tile_plan(0, 64, 64, False) == native().gemm_tile_plan(1 << 40, 64, 64, False) == -1
+
+
+@pytest.mark.parametrize("N,K", [(64, 4096), (128, 4096), (256, 4096), (64, 2048), (128, 2048), (256, 8192)])
+def test_gates_are_not_cut_along_k(N, K):
+    """A gate's or a router's sums are one sum in order at any number of rows: short prompts and long ones round alike."""
+    for M in (9, 17, 32, 33, 48, 300, 511, 512, 700, 2048, 4096):
+        for swiglu in (False, True):
+            plan = gemm.tile_plan(M, N, K, swiglu)
+            assert plan is None or plan[1] == 1, (M, swiglu, plan)
+    assert gemm.tile_plan(48, N + 256, 8192)[1] > 1  # (past them they are)
 
 
 def test_tile_plan_is_one_turn():
