@@ -311,8 +311,10 @@ FUSED = os.environ.get("MXLLM_HYBRID_FUSED", "1") != "0"
 _NORM_MAX, _POLY_MAX = 16384, 32768  # rows x width held in LDS by a prologue
 
 
-def _fusable(t: torch.Tensor, w: torch.Tensor | None, mult: int = 16, rows: int = SKINNY_M) -> bool:
+def _fusable(t: torch.Tensor, w: torch.Tensor | None, mult: int = 16, rows: int | None = None) -> bool:
+    """``rows``: the most that the kernel is for (SKINNY_M)."""
     M, K = t.shape
+    rows = SKINNY_M if rows is None else rows
     return bool(FUSED and w is not None and use_native(t) and w.dtype == torch.bfloat16 and 0 < M <= min(rows, 16)
                 and K % 512 == 0 and w.shape[0] % mult == 0 and w.stride(1) == 1 and w.stride(0) % 8 == 0
                 and (M == 1 or w.numel() <= _SKINNY_SMALL_W))

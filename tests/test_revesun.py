@@ -368,14 +368,32 @@ def test_hooks_of_output_projections_see_every_call(gpu, n):
     assert calls == [(n, 512)] * 4 and torch.isfinite(want).all()
 
 
+def test_row_limits_are_read_at_each_call(monkeypatch):
+    """A limit set after the import holds for the fused projections."""
+    x, w = torch.zeros(12, 512, dtype=torch.bfloat16), torch.zeros(64, 512, dtype=torch.bfloat16)
+    monkeypatch.setattr(hops, "use_native", lambda t: True)
+    assert not hops._fusable(x, w) and hops._fusable(x, w, rows=12)
+    monkeypatch.setattr(hops, "SKINNY_M", 16)
+    assert hops._fusable(x, w)
+
+
 @pytest.mark.gpu
 def test_parts_go_past_the_norm_prologues(gpu, monkeypatch):
     """MXLLM_SKINNY_M and MXLLM_NORM_FUSED_M of 16: projections with the norm in their prologue behind outputs in parts, against
     the steps without the settings (other kernels, so to rounding)."""
     model, prompts = parts_model(gpu), [tokens(3 + i, 128, i) for i in range(12)]
     feed = torch.randint(0, 128, (4, 12), generator=torch.Generator().manual_seed(1))
-    outs = []
+    outs, seen, lib = [], [], hops.native()
+
+    class Seen:
+        def __getattr__(self, name):
+            if name == "hs_norm_linear":
+                seen.append(name)
+            return getattr(lib, name)
+
+    monkeypatch.setattr(hops, "native", Seen)
     for rows in (None, 16):
+        assert not seen
         if rows:
             monkeypatch.setattr(hops, "SKINNY_M", rows)
             monkeypatch.setattr(hops, "NORM_M", rows)
@@ -383,6 +401,7 @@ def test_parts_go_past_the_norm_prologues(gpu, monkeypatch):
         slots = [eng.acquire() for _ in prompts]
         eng.prefill_batch(slots, prompts)
         outs.append(torch.stack([eng.decode(slots, t).float().clone() for t in feed]))
+    assert seen  # the prologue's kernel ran in the second pass
     rel = (outs[0] - outs[1]).pow(2).mean().sqrt() / outs[0].pow(2).mean().sqrt()
     assert float(rel) < 1.5e-2, float(rel)
 
