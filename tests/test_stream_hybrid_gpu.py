@@ -95,3 +95,11 @@ def test_conv(gpu, M, K, groups, parts, add, H, G, D):
         _near(a, b)
     # what no row wrote is as it was
     assert int((c != kv).any(-1).sum()) <= 2 * M * G and int((r != ring).any(-1).sum()) <= M
+
+
+@pytest.mark.parametrize("M", [8, 9, 16])
+def test_rows_past_the_kernels_of_a_width(gpu, monkeypatch, M):
+    """A limit of 16 rows of a width of 4096: what the workgroups that stay leave to csrc/kernels/hybrid_skinny.hip."""
+    monkeypatch.setattr(hops, "SKINNY_M", 16)
+    test_gru(gpu, M, 4096, 8, False, True, 36)
+    test_conv(gpu, M, 4096, 8, False, True, 4, 2, 32)
