@@ -512,13 +512,16 @@ struct EvenState {  // of one wave
 // of one row and the start of another ended 22 us into the launch, those within a row at 15 (16 sequences of 100 to 2,000
 // keys).  A step of them, us, with 0 / 3 / 6 / 9 / 13: 4060 / 4008 / 4001 / 4013 / 4043; 32 of 250 to 1,000 4738 / 4710 /
 // 4696 / 4753 / 4768; 24 of 225 to 900 4515 / 4497 / 4498 / 4510 / 4526; 8 of 750 to 3,000 3800 / 3791 / 3799 / 3844 / 3828.
+// Short rows in a step built for long ones, the attention alone, us, with 0 / 6: 12 of 32 keys 14.6 / 7.0, 64 of 100 15.3 / 10.9, 128 of up
+// to 256 26.3 / 22.1; rows that share by share were whole before are the worst, 40 of 128 9.7 / 11.0, 100 of 64 15.6 / 16.2.
 constexpr int kEvenPad = 6;
 // units that row b is dealt as, the first kEvenPad of which hold no keys; cap: positions that the buffers are sized for
 __device__ __forceinline__ int even_units(const int32_t* lens, int len_off, int cap, int b) {
   const int n = (min(max(lens[b] + len_off, 0), cap) + 15) >> 4;
   return n ? n + kEvenPad : 0;
 }
-// units of a workgroup: an equal share of all, at least 128 keys
+// units of a workgroup: an equal share of all, at least 8 (128 keys, or the first 32 of a row: with 14, so that a row's first 128 stay
+// together, 64 rows of 100 keys 10.9 -> 14.0 us, 20 of up to 192 9.2 -> 12.3; alike only for rows of 128, 9.4 -> 8.3)
 __device__ __forceinline__ int even_share(int total, int W) { return max((total + W - 1) / W, 8); }
 
 __global__ void __launch_bounds__(256, 3)
@@ -943,7 +946,7 @@ extern "C" int mx_decode_attn(const uint16_t* q, const uint16_t* kc, const uint1
     return (int)hipGetLastError();
   }
   // Heads of 128, more splits than places: dealt evenly.  What the caller's `nsplit` counts is the longest that the step
-  // was built for; where the sequences of a call are shorter, the shares are, down to 128 keys.  Not of one split (no merge
+  // was built for; where the sequences of a call are shorter, the shares are (even_share).  Not of one split (no merge
   // to wait for: 32 heads of 8, us, split -> dealt: 80 sequences of 60 to 256 keys 16.0 -> 20.8, 256 36.3 -> 42.8; 72 of 10 to
   // 64 10.2 -> 19.0) nor of two where the kernel above does not take them (32 heads of 2, 256 of 20 to 200 keys 29.0 -> 31.5).
   if (out && D == kEvenD && nsplit > kShortSplits && (int64_t)nsplit * Hkv * B > kEvenPlaces) {

@@ -1280,6 +1280,32 @@ def test_decode_attn_dealt_evenly(gpu, Hq, Hkv, lens, room, paged):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("filler", [[], [700] * 5])
+def test_decode_attn_dealt_evenly_at_the_edges_of_shares(gpu, filler):
+    """A row is dealt as six units without keys and one for every 16: the first row's length moves the second's keys past the end of
+    a share (of 8 units, and of more where the others are long), one unit at a time: shares that end ahead of a row's keys, at
+    them and behind their first unit, empty rows between, and the parts that the merge counts.  Within 2^-7 of f64, as above."""
+    Hq, Hkv, D, room = 32, 8, 128, 2048
+    for units in range(1, 30):
+        lens = [16 * units, 0, 40, 0, 0, 16 * (units % 5) + 1, 129, 0, 15, 300, *filler]
+        B = len(lens)
+        assert room // 256 * Hkv * B > 512
+        torch.manual_seed(units)
+        kc, vc = (torch.full((B, Hkv, room, D), float("nan"), device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        q = torch.randn(B, Hq, D, device=gpu, dtype=torch.bfloat16)
+        for b, n in enumerate(lens):
+            kc[b, :, :n], vc[b, :, :n] = (torch.randn(Hkv, n, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+        out = _ops().decode_attn(q, kc, vc, torch.tensor(lens, dtype=torch.int32, device=gpu), None, room, D ** -0.5, 0, None, None).view(B, Hq, D)
+        for b, n in enumerate(lens):
+            if n == 0:
+                assert not out[b].any()
+                continue
+            s = (q[b].double().view(Hkv, -1, 1, D) * kc[b, :, None, :n].double()).sum(-1) * D ** -0.5
+            want = (torch.softmax(s, -1)[..., None] * vc[b, :, None, :n].double()).sum(2).view(Hq, D)
+            assert rel_err(out[b], want) < 2 ** -7, (units, b, n)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,Hq,Hkv", [(32, 4, 2), (64, 32, 8), (128, 8, 1)])
 @pytest.mark.parametrize("lens", [[1], [127, 1, 129], [256, 65, 700, 128, 3]])
 def test_prompt_attention(gpu, D, Hq, Hkv, lens):
