@@ -319,14 +319,16 @@ extern "C" int mx_skinny_gemm_half(const uint16_t* x, int64_t ldx, const uint16_
   // DEEP up to where the waves that it leaves are busy (2048 x 2048, one row 3.9 -> 3.7 us, 4096 x 4096 7.7 -> 7.5, 2048 x 8192 8.0 -> 8.4)
   if (K <= 4096)
     skinny_gemm_kernel<1, 1, 8, false, false, false, false, true, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
-  // One workgroup a CU has the registers for a whole K part in flight, and nothing beside it to hide its turns of 8 chunks:
-  // 2048 x 12288, a step of revesun-1b with 1 / 2 / 4 / 8 rows 758 / 791 / 838 / 966 -> 740 / 771 / 823 / 953 us.  Rows ahead of
-  // the weights or behind them: as good or worse.  Two turns are level or better left (2048 x 8192, a step of llama3.2-1b of
-  // one row 684 -> 684, beside other processes 686 -> 697).
+  // One workgroup a CU has the registers for a whole K part of up to 30 chunks in flight (231; scratch at 32), and nothing
+  // beside it to hide its turns of 8 chunks.  Weights from memory, 1 / 4 / 8 rows, turns -> whole, us: 2048 x 9216 8.9 / 10.0 / 10.9 -> 7.9 /
+  // 9.0 / 10.4, x 11264 11.4 / 12.6 / 13.1 -> 10.0 / 11.4 / 12.2, x 12288 12.0 / 13.6 / 14.0 -> 10.8 / 12.2 / 13.2, x 15360 14.6 / 16.3 / 16.8 ->
+  // 12.7 / 14.9 / 16.0; 1024 x 10240 8.9 / 10.2 / 11.9 -> 7.8 / 9.5 / 11.1.  2048 x 12288 in a step of revesun-1b with 1 / 2 / 4 / 8 rows
+  // 758 / 791 / 838 / 966 -> 740 / 771 / 823 / 953.  Rows ahead of the weights or behind them: as good or worse.  Two turns are level or
+  // better left (2048 x 8192, a step of llama3.2-1b of one row 684 -> 684, beside other processes 686 -> 697).
 #define SKH(U) \
   else if (N <= 8 * 256 && K == 512 * U) \
     skinny_gemm_kernel<1, 1, 8, false, false, false, false, true, false, false, U><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);
-  SKH(20) SKH(24) SKH(28)
+  SKH(18) SKH(20) SKH(22) SKH(24) SKH(26) SKH(28) SKH(30)
 #undef SKH
   else
     skinny_gemm_kernel<1, 1, 8, false, false, false, false, true><<<N / 8, 512, 0, stream>>>(x, ldx, w, ldw, y, ldy, M, K);

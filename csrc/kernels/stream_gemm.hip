@@ -119,6 +119,8 @@ static int stream_blocks(const StreamArgs& a, hipStream_t stream) {
   constexpr int KP8 = KIND == kStF8Lines ? 4 : 8;
   const size_t lds = (four ? kStreamRed<KIND, TB, 4> : kStreamRed<KIND, TB, KP8>) + (size_t)a.M * (a.K + 8) * 2;
   const int per_cu = lds <= kTwoLds ? 2 : 1;
+  // (A K of 2048 has two workgroups a CU, so 512 groups are one turn; of a longer one a part is more than one block, and the registers
+  // do not hold two of those.)
   if constexpr (KIND == kStLines || KIND == kStF8Lines)
     if (a.K == 4096 && a.groups > 256 && a.groups <= 384)
       return stream_launch<KIND, TB, KP8, EPI, NORM, KIND == kStLines ? 16 : 8, true>(a, 1, lds, stream);

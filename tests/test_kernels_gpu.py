@@ -887,9 +887,10 @@ def test_skinny_linear_half(gpu, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(1, 8, 6144), (8, 2048, 8192), (3, 72, 10240), (5, 2048, 12288), (2, 1024, 14336), (8, 64, 16384)])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 6144), (8, 2048, 8192), (3, 72, 10240), (5, 2048, 12288), (2, 1024, 14336), (8, 64, 16384),
+                                   (2, 2048, 9216), (1, 1024, 11264), (8, 2048, 13312), (4, 8, 15360), (8, 2048, 15360), (8, 2056, 13312)])
 def test_skinny_linear_half_whole_parts(gpu, M, N, K):
-    """A wave's whole K part in flight (12 to 28 chunks) and the sizes beside them."""
+    """A wave's whole K part in flight (18 to 30 chunks) and the sizes beside them."""
     torch.manual_seed(M + N)
     x = torch.randn(M, K, device=gpu, dtype=torch.bfloat16)
     w = torch.randn(N, K + 8, device=gpu, dtype=torch.bfloat16)[:, :K] * 0.05
