@@ -6,6 +6,8 @@ GPU: the batched HIP sampler (csrc/kernels/sampling.hip) draws from exactly
 that distribution (empirical frequencies vs the oracle), keeps greedy rows
 greedy in a mixed batch, and reproduces the temperature-only kernel's draws.
 """
+import math
+
 import pytest
 import torch
 
@@ -209,22 +211,29 @@ def test_gpu_split_sampler_draws(gpu, V, dtype, shape):
 @pytest.mark.parametrize("kept", [1, 63, 2047, 2048, 2049, 6000])
 def test_gpu_split_sampler_kept_tokens_of_one_chunk(gpu, kept, dtype):
     """Kept tokens are gathered up to 2,048 a chunk, the rest scored where they lie: as many about that, all in the first
-    8,192 of 16,384 (a chunk of a 64-row call), the others far below them, in the histogram's last bin."""
-    V, B = 16384, 64
+    8,192 of 16,384 (a chunk of a 64-row call) and in the histogram's first bin.  The cut of mass or count falls among 30 tokens
+    131 bins lower, in the other chunk: what is ahead of them is scored and not listed.  The others lie in the last bin."""
+    V, B, T, low = 16384, 64, 0.7, 30
     g = torch.Generator().manual_seed(kept)
     x = torch.full((B, V), -300.0)
     for i in range(B):
         x[i, torch.randperm(8192, generator=g)[:kept]] = 1.0
+        x[i, 8192 + torch.randperm(8192, generator=g)[:low]] = 0.0
     x = x.to(dtype)
-    seeds = [7 * i for i in range(B)]
-    got = dops.sample_rows(x.to(gpu), [0.7] * B, [0.9, 1.0] * (B // 2), [0, kept] * (B // 2), seeds, [3] * B).tolist()
-    for i in range(B):
-        noise, err = _scores(V, seeds[i], 3)
-        s = torch.where(x[i] > 0, noise, float("-inf"))
-        best = int((s - err).argmax())
-        rest = s + err
-        rest[best] = float("-inf")
-        assert x[i, got[i]] > 0 and (got[i] == best or (s - err)[best] <= rest.max())
+    below = low * math.exp(-1.0 / T)
+    p, seeds = (kept + below / 2) / (kept + below), [7 * i for i in range(B)]
+    wins = 0
+    for step in (3, 4, 5, 6):
+        got = dops.sample_rows(x.to(gpu), [T] * B, [p, 1.0] * (B // 2), [0, kept + low // 3] * (B // 2), seeds, [step] * B).tolist()
+        for i in range(B):
+            noise, err = _scores(V, seeds[i], step)
+            s = torch.where(x[i] >= 0, x[i].double() / T + noise, float("-inf"))
+            best = int((s - err).argmax())
+            rest = s + err
+            rest[best] = float("-inf")
+            assert x[i, got[i]] >= 0 and (got[i] == best or (s - err)[best] <= rest.max()), (i, step)
+            wins += got[i] < 8192
+    assert wins > 3 * B if kept > 1 else 0 < wins < 4 * B  # the gathered ones hold most of the mass, or an eighth of it
 
 
 @pytest.mark.gpu
