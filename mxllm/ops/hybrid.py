@@ -356,11 +356,13 @@ def _norm_stays(delta, h, gamma, groups: int, w) -> bool:
                 and (delta is None or (delta.dim() == 2 and delta.stride(0) % 8 == 0 and delta.data_ptr() % 16 == 0)))
 
 
-def _mixer_rows(h: torch.Tensor) -> int:
+def _mixer_rows(h: torch.Tensor, width: int = 0) -> int:
     """Rows up to which a mixer's projection runs with its epilogue: past SKINNY_M for a width of 2048 (csrc/kernels/stream_hybrid.hip;
     steps of 9 / 12 / 16 sequences of the 1B size 998 / 1034 / 1057 us apart, 959 / 995 / 1021 so; of 4096, 8B size, 3945 / 4088 /
-    4181 apart, 3960 / 4117 / 4214)."""
-    return _DECODE_M if h.shape[1] == 2048 else SKINNY_M
+    4181 apart, 3960 / 4117 / 4214).  A minGRU's up to a state of 2048 (``width``; norm and projection, 9 / 16 rows: 2048 14.0 / 14.7 ->
+    12.3 / 12.8, 2560 14.1 / 14.9 -> 14.9 / 15.7, 4096 16.8 / 18.0 -> 17.6 / 18.6); the convolution's at any size (640 / 768 / 1024 groups of
+    channels, 16 rows: 26.5 / 27.3 / 32.7 -> 24.4 / 25.2 / 31.6)."""
+    return _DECODE_M if h.shape[1] == 2048 and width <= 2048 else SKINNY_M
 
 
 def _normed(delta, h, gamma, groups, eps, w):
@@ -372,7 +374,7 @@ def _normed(delta, h, gamma, groups, eps, w):
 
 def gru_linear(delta, h, gamma, groups: int, eps: float, w, bias, rows, layer: int):
     """Decode: (minGRU output of the normed rows, new residual), state advanced; w = [z; u; gate]."""
-    if not (rows.decode and _fusable(h, w, 12, _mixer_rows(h))):
+    if not (rows.decode and _fusable(h, w, 12, _mixer_rows(h, bias.numel() // 2))):
         return None
     d, x, g = _normed(delta, h, gamma, groups, eps, w)
     y, hn = native().hs_gru_linear(d, x, g, groups, eps, w, bias, rows.slots, rows.caches.rec[layer])

@@ -377,6 +377,13 @@ def test_row_limits_are_read_at_each_call(monkeypatch):
     assert hops._fusable(x, w)
 
 
+def test_rows_of_the_mixers_projections():
+    """Past SKINNY_M rows for a width of 2048, of a minGRU with a state of up to as many channels."""
+    x, y = torch.zeros(12, 2048), torch.zeros(12, 4096)
+    assert hops._mixer_rows(x) == hops._mixer_rows(x, 2048) == hops._DECODE_M > hops.SKINNY_M
+    assert hops._mixer_rows(x, 2052) == hops._mixer_rows(y) == hops._mixer_rows(y, 64) == hops.SKINNY_M
+
+
 @pytest.mark.gpu
 def test_parts_go_past_the_norm_prologues(gpu, monkeypatch):
     """MXLLM_SKINNY_M and MXLLM_NORM_FUSED_M of 16: projections with the norm in their prologue behind outputs in parts, against
