@@ -270,11 +270,13 @@ __device__ __forceinline__ void dfuse_swiglu_store(const f32x4& v, int g, int m,
   }
 }
 
-template <int HD = 64>
+// SWAP: the pairs by lane swaps.  Beside other groups' products those cost more than shuffles (12288 x 4096 with the norm 20.9 us for
+// 20.2); where a workgroup's one group and a half end it, less (a step of llama3.1-8b with 16 sequences 3977 us for 3994).
+template <int HD = 64, bool SWAP = false>
 __device__ __forceinline__ void dfuse_rope_store(const f32x4& v, int g, int m, int M, int blk, const SkRope& rp) {
   f32x4 hi;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) hi[i] = __shfl_xor(v[i], 32, 64);  // (swapped in the vector ALU 12288 x 4096 takes 20.9 us for 20.2)
+  for (int i = 0; i < 4; ++i) hi[i] = SWAP ? __uint_as_float(lane_pair<32>(__float_as_uint(v[i])).b) : __shfl_xor(v[i], 32, 64);
   if (g < 2 && m < M) {
     constexpr int PH = HD / 8;
     const int head = blk / PH, i0 = (blk % PH) * 8 + 4 * g;

@@ -81,9 +81,9 @@ __global__ void __launch_bounds__(512, (HALF ? 2 : kStWaves<KIND, TB, KP, NL>)) 
   auto finish = [&](const f32x4& s, int mb, int cg, bool on = true) __attribute__((always_inline)) {
     const int m = on ? mb * 16 + c : M;
     if constexpr (EPI == kStRope128) {
-      dfuse_rope_store<64>(s, g, m, M, cg, a.rp);
+      dfuse_rope_store<64, HALF>(s, g, m, M, cg, a.rp);
     } else if constexpr (EPI == kStRope64) {
-      dfuse_rope_store<32>(s, g, m, M, cg, a.rp);
+      dfuse_rope_store<32, HALF>(s, g, m, M, cg, a.rp);
     } else if constexpr (EPI == kStSwiglu) {
       dfuse_swiglu_store(s, g, m, M, a.Y, a.ldy, cg);
     } else if (m < M) {
