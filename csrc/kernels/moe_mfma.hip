@@ -383,8 +383,8 @@ __global__ void __launch_bounds__(512, TMAX <= 32 ? 4 : 2) moe_few_kernel(MoeFew
 // [gate | up].  Workgroups: the shared expert's slices (its rows are the tokens), those of every expert, and one that
 // stores the choices, behind all others.  A wave finds its expert's tokens by itself (moe_route.h, moe_place): with all
 // choices made by every workgroup and two barriers, the weights of half of them began 10 us into the launch (stamped; 32
-// tokens, 1B sizes), now 7; steps of 24 / 32 / 48 sequences 1480 / 1567 / 1890 -> 1452 / 1525 / 1782 us, 8B sizes of
-// 48 7190 -> 6781.  The other half's logits wait in their CU's queue behind the
+// tokens, 1B sizes), now 7; steps of 24 / 32 / 48 sequences 1480 / 1567 / 1890 -> 1455 / 1528 / 1813 us, 8B sizes of
+// 48 7190 -> 6760.  The other half's logits wait in their CU's queue behind the
 // first half's weights: 67 MB come at 4.5 TB/s whatever is asked for first (half or all of a wave's weights ahead of the
 // choices: within 0.4 %).
 template <typename Own, int ROWS, int LESS, typename Shared, int SROWS, int TMAX>

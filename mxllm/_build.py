@@ -48,7 +48,8 @@ ARCH = os.environ.get("MXLLM_ARCH", "gfx950")
 # per-kernel-file compiler options (A/B experiments: MXLLM_FILE_FLAGS="file.hip=-opt1 -opt2;other.hip=...")
 # Decode kernels whose arguments are plain values get the first of them in registers at the start instead of by a load
 # that all else waits for: steps of llama3.1-8b with 16 sequences 4004 -> 3972 us, with 4 in e4m3 2218 -> 2206, of revesun-1b
-# with 4 833 -> 825, of llama3.2-1b with one 684 -> 685.  (Arguments in a struct stay in memory; for all files, steps of
+# with 4 833 -> 825, of llama3.2-1b with one 684 -> 685; skinny_gemm.hip alone 5 % past 8 rows and 1 % up to 8, but 16 channels a
+# workgroup of a K of 8192 4096 x 8192 13.7 -> 14.2.  (Arguments in a struct stay in memory; for all files, steps of
 # sigusun-1b with 32 1540 -> 1546.)
 _PRELOAD = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 PER_FILE_HIP_FLAGS: dict[str, list[str]] = {
