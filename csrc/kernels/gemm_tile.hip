@@ -292,10 +292,12 @@ using namespace mx;
 //    each of these lines more than one size of 50 is slower here; of 3,000 sizes of 139 weights that go here and the fit had
 //    not seen, 15 are by more than 3 %, the worst by 13 %, and 22 more of those of the next line
 //    (profiles/gemm_routes/tile.txt);
-//  * past 32 rows, which no step's graph holds, what is over in 17 us (24 with SwiGLU) is taken all the same: the library's
-//    call costs the host 21 us, this one 11, in parts 15. A prompt of 290 / 370 / 430 tokens of llama3.2-1b takes 2.85 / 2.83 /
-//    2.82 ms with the library's products and 1.94 / 1.98 / 2.00 with these, though 370 rows of 3072 x 2048 alone are 15.1 us
-//    there and 16.1 here;
+//  * past 32 rows what is over in 17 us (24 with SwiGLU) is taken all the same: the library's call costs the host 21 us, this
+//    one 11, in parts 15. A prompt of 290 / 370 / 430 tokens of llama3.2-1b takes 2.85 / 2.83 / 2.82 ms with the library's
+//    products and 1.94 / 1.98 / 2.00 with these, though 370 rows of 3072 x 2048 alone are 15.1 us there and 16.1 here. A
+//    step of 33 and more sequences is replayed without the host, but there these are the quicker ones too: 38 sizes of 33 to 256
+//    rows that this line decides take .87 of the library's time in the mean (10240 x 2048 at 65 rows 21.6 -> 15.6), one is slower
+//    by more than 3 % (20480 x 1536 at 64 19.3 -> 21.1);
 //  * more than 44 M weights (12288 x 4096 and up) are read at the rate of memory by the library as well, from 256 rows (K of
 //    8192: 128) on it falls behind: 12288 x 4096 at 64 / 256 / 700 rows 26.7 / 1.21 / 1.23 times as fast here (26.8 at 64),
 //    16384 x 4096 at 128 37.3 -> 41.8, 8192 x 8192 at 64 / 128 / 256 33.6 / 50.9 / 1.66 times (39.0, 43.0). So they are by a
