@@ -1,4 +1,4 @@
-// Inference-side kernels for gfx950 (SURVEY §2.4 K14, K15):
+// Inference-side kernels for gfx950:
 //   * rope_append : decode-step q/k RoPE at per-sequence positions + KV-cache append
 //   * decode_attn : single-token GQA attention over a per-slot KV cache,
 //                   split over the sequence (flash-decoding), memory-bound:

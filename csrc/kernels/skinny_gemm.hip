@@ -1,5 +1,5 @@
 // bf16 weight-streaming GEMM for decode on gfx950: Y[M, N] = X[M, K] . W[N, K]^T with M <= 32
-// tokens (serving path, SURVEY §2.4 K14 neighbourhood).  A decode step reads every weight once;
+// tokens (serving path).  A decode step reads every weight once;
 // for the small projections of an 8B model (34-117 MB) hipBLASLt's skinny solutions stream at
 // 1.7-4.5 TB/s (archive/profiles/r2x_skinny_gemm.md), latency-bound: too few bytes in flight per CU.
 //

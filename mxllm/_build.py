@@ -96,7 +96,7 @@ def _check_loadable(path: str) -> None:
 
 
 def _attn_bwd_counted_wait_ok(asm: str) -> tuple[bool, str]:
-    """ISA invariant of the attention backward's counted end-of-tile wait (ADVICE r4): every
+    """ISA invariant of the attention backward's counted end-of-tile wait: every
     ``s_waitcnt vmcnt(4) lgkmcnt(0)`` in front of an ``s_barrier`` must have at least 4 vector-memory
     instructions (the dS^T stores) between it and the last LDS-DMA issue before it -- then, with
     in-order retirement, vmcnt(4) implies the DMA landed.  Returns (ok, detail)."""
@@ -121,7 +121,7 @@ def _attn_bwd_counted_wait_ok(asm: str) -> tuple[bool, str]:
     if found == 0:
         # the counted-wait schedule is compiled in (the check runs only on that build) but no
         # ``vmcnt(4) lgkmcnt(0)`` + barrier pair survived codegen (merged / reordered by the waitcnt
-        # pass): nothing was verified, so take the safe schedule (ADVICE r5)
+        # pass): nothing was verified, so take the safe schedule
         return False, "no counted wait found in the attn_bwd8 kernels (nothing verified)"
     return True, f"{found} counted waits checked"
 
