@@ -281,16 +281,20 @@ using namespace mx;
 
 // Tile and parts of K for a product, as 64 tile + parts, by the modelled time; -1: it is not one turn of tiles, or the library,
 // or another kernel, may have it faster.  Where the lines lie (us, hipBLASLt, or gemm8 marked * -> here):
-//  * K in one part of more than 1,024: tiles past 64 x 64 only where 7 of 8 CUs have one. With fewer the library's kernels are
-//    as quick or quicker at one size of seven (6144 x 4096 at 386 rows, 192 tiles, 30.9 -> 36.8; 4096 x 4096 at 687, 192, 32.3
-//    -> 36.5), with as many at one of fifty (4096 x 4096 at 1024, 256 tiles, 42.1 -> 38.9). A K up to 1,024 is over before it
-//    matters (8192 x 512 at 181 rows, 192 tiles, 9.3 -> 5.9);
+//  * K in one part of more than 1,024: a tile past 64 x 64 only where enough of the CUs have one. The share, and the mean time
+//    against the library's at 256 to 4,400 rows below it and at it: 64 x 128 13/16, past a K of 2,048 7/8 (K 2048 at 12/16 .99, a
+//    quarter of the sizes slower by more than 3 %, at 13/16 .91; K 3072 at 13/16 1.10); 128 x 128 13/16 (K 4096 1.08, .92), up to a K of
+//    2,048 1/2 (.85; 2048 x 2048 at 1,045 to 1,628 rows 19 -> 15); 128 x 192 5/8 (.98); larger ones 13/16 (1.05 - 1.1, .95); past a
+//    K of 4,096 7/8 (.98 at 13/16, but a quarter slower). Below them the library's kernels are as quick (6144 x 4096 at 386 rows,
+//    192 tiles, 30.9 -> 36.8; 4096 x 4096 at 687, 192, 32.3 -> 36.5). A K up to 1,024 is over before it matters (8192 x 512 at 181
+//    rows, 192 tiles, 9.3 -> 5.9);
 //  * not where the library at its best (gt_library, with SwiGLU and its activation's launch) would be faster. The model may be
-//    longer than that by 3 % (2048 x 8192 at 290 / 549 rows, by 1 % longer, 32.3 / 44.4 -> 25.1 / 33.7); up to 32 rows by 5 %
-//    (12 with SwiGLU of more than 44 M weights); up to 192 rows, where the library is seldom at its best, by 12 % (6144 x 4096
-//    at 150 39.6 -> 24.9); in one part of filled turns or of the smallest tile by 10 % (2048 x 8192 at 2709 91 -> 84). Past
-//    each of these lines more than one size of 50 is slower here; of 3,000 sizes of 139 weights that go here and the fit had
-//    not seen, 15 are by more than 3 %, the worst by 13 %, and 22 more of those of the next line
+//    longer than that by 3 % (64 x 128; in parts that leave CUs idle); up to 32 rows by 5 % (12 with SwiGLU of more than 44 M
+//    weights); up to 192 rows, where the library is seldom at its best, by 12 % (6144 x 4096 at 150 39.6 -> 24.9); in one part of
+//    the smallest or the larger tiles by 10 % (2048 x 8192 at 2709 91 -> 84), in parts for 7 of 8 CUs by 9 (1,800 sizes past 3
+//    .87; past 9 6144 x 4096 at 386 31.3 -> 34.1); of 128 x 128 and a K up to 2,048 by 18 % (3072 x 2048 at 643 to 768 rows .86). Past each of these lines more than one size of 50 is
+//    slower here; of 20,000 sizes of 760 weights at 33 rows and more that go here and that neither lines nor model were fitted to,
+//    2.6 % are by more than 3 %, most of them by the next line, and all together take .82 of the library's time
 //    (profiles/gemm_routes/tile.txt);
 //  * past 32 rows what is over in 17 us (24 with SwiGLU) is taken all the same: the library's call costs the host 21 us, this
 //    one 11, in parts 15. A prompt of 290 / 370 / 430 tokens of llama3.2-1b takes 2.85 / 2.83 / 2.82 ms with the library's
@@ -336,17 +340,24 @@ extern "C" int mx_gemm_tile_plan(int M, int N, int K, int swiglu) {
       if (u > kGtPlaces || (S > 1 && (nk < 4 * S || N <= 256))) break;
       float us = t.start + (float)nk / S * (t.step + t.load * u / kGtPlaces) + t.memory * weights * 2e-6f;
       if (S > 1) us += t.sum + (t.part + (swiglu ? t.glu : 0.f)) * S + t.image * ((float)S * M * N * 4e-6f);
-      if (S == 1 && i && !swiglu && K > 1024 && 8 * u < 7 * kGtPlaces && us > quick) continue;
+      const int least = i == 3 && K <= 4096 ? 10 : i == 2 && K <= 2048 ? 8 : K <= (i == 1 ? 2048 : 4096) ? 13 : 14;  // sixteenths
+      if (S == 1 && i && !swiglu && K > 1024 && 16 * u < least * kGtPlaces && us > quick) continue;
       if (us < best) {
         best = us;
         plan = 64 * i + S;
       }
     }
   }
-  const bool steady = !swiglu && plan % 64 == 1 && (plan / 64 < 1 || plan / 64 > 2 || K <= 1024);
+  if (plan < 0) return -1;
+  const int tile = plan / 64, S = plan % 64;
+  const bool filled = 8 * gt_units(kGtTiles[tile], M, N) * S >= 7 * kGtPlaces;
+  const bool flat = !swiglu && S == 1 && tile == 2 && K <= 2048;
+  const bool steady = !swiglu && (S == 1 ? tile < 1 || tile > 2 || K <= 1024 : filled && !lengthy);
   float most = gt_library(M, N, K);
   if (swiglu) most += 1.5f + .3f * ((float)M * N * 3e-6f);  // (its bytes: N in, N / 2 out)
-  if (N > 256) most *= M <= 32 && !(swiglu && weights > 44000000) ? 1.05f : M <= 192 ? 1.12f : steady ? 1.1f : 1.03f;
+  if (N > 256)
+    most *= M <= 32 ? (swiglu && weights > 44000000 ? 1.12f : 1.05f)
+                    : flat ? 1.18f : M <= 192 ? 1.12f : steady ? (S == 1 ? 1.1f : 1.09f) : 1.03f;
   return best < std::max(most, quick) ? plan : -1;
 }
 

@@ -157,7 +157,9 @@ def test_ragged_row_rules():
 # (M, N, K): both sides of the lines of csrc/kernels/gemm_tile.hip mx_gemm_tile_plan
 TILE_ON = [(9, 2048, 64), (33, 2048, 2048), (2709, 3072, 2048), (192 * 16, 192 * 16, 2048), (33, 2560, 4096), (32, 2048, 8192), (17, 4096, 14336), (430, 12288, 4096), (128, 8192, 8192), (256, 4096, 14336), (512, 2048, 12288),
            (40, 3360, 2048),
-           (370, 3072, 2048), (290, 2048, 2048), (549, 2048, 8192), (150, 6144, 4096)]
+           (370, 3072, 2048), (290, 2048, 2048), (549, 2048, 8192), (150, 6144, 4096),
+           # (too few tiles for most CUs, but .77 to .92 of the library's time)
+           (1045, 2048, 2048), (1600, 2048, 2048), (2237, 2048, 2048), (667, 3072, 2048), (1079, 4096, 4096), (700, 6144, 4096), (540, 5120, 5120)]
 TILE_OFF = [(192 * 16 + 1, 192 * 16, 2048), (255, 12288, 4096), (127, 8192, 8192), (257, 4096, 14336), (513, 2048, 12288), (40, 3368, 2048), (40, 2048, 2080),
             (32, 6144, 4096), (6, 128256, 2048), (2709, 16384, 2048), (2048, 128, 4096), (512, 256, 4096),
             # (the library was quicker by 4 to 18 %)
