@@ -745,7 +745,7 @@ std::tuple<at::Tensor, at::Tensor> attn_fwd(const at::Tensor& q, const at::Tenso
 }
 
 // dq_mode: 1 = f32 atomics, 2 = deterministic per-key-block partials + ordered reduce,
-// 3 = split (dS^T to HBM + separate dQ kernel; default, deterministic)
+// 3 = split (dS^T to HBM + separate dQ kernel, heads of 64: a pass of its own for dQ; default, deterministic)
 // outs (optional, split mode only): preallocated f32 dq [B, Hq, S, D] and dK / dV partials
 // [B, P, Sk, D] to write into (e.g. head-range views of larger tensors: the chunked long-context
 // backward, mxllm/ops/attention.py) instead of fresh tensors.
@@ -797,7 +797,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attn_bwd_impl(const at::Tensor& d
   auto delta = at::empty({B, Hq, S}, q.options().dtype(at::kFloat));
   if (causal >= 0 && dq_mode != 1) {
     at::Tensor work = dq_mode == 2 ? at::empty({nkb, B, Hq, S_pad, D}, q.options().dtype(at::kFloat))
-                                   : at::empty({B * Hq, nkb * 128, S_pad}, q.options());
+                                   : at::empty({D == 64 ? 0 : B * Hq, nkb * 128, S_pad}, q.options());
     // dqkv: the dQ kernel writes d(q) into it; no fp32 dQ at all
     auto dq = outs ? *dq_out
                    : at::empty({dqkv ? 0 : B, Hq, S, D}, q.options().dtype(at::kFloat));
@@ -825,7 +825,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> attn_bwd(const at::Tensor& dout, 
   return attn_bwd_impl(dout, q, k, v, o, lse, causal ? 1 : 0, scale, dq_mode, dq_out, dk_out, dv_out);
 }
 
-// The attention backward straight into d(qkv) [B*S, (Hq+2Hkv)*D (+out_pad)] bf16 (D = 128, split mode):
+// The attention backward straight into d(qkv) [B*S, (Hq+2Hkv)*D (+out_pad)] bf16 (D = 64 and 128, split mode):
 // the dQ kernel writes the q columns with the inverse RoPE applied, rope_merge_bwd only the k / v
 // columns from the dK / dV partials -- the fp32 dQ never reaches HBM (mxllm/ops/attention.py).
 at::Tensor attn_bwd_rope(const at::Tensor& dout, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
@@ -833,7 +833,7 @@ at::Tensor attn_bwd_rope(const at::Tensor& dout, const at::Tensor& q, const at::
                          const at::Tensor& sin, int64_t out_pad) {
   const int64_t B = q.size(0), Hq = q.size(1), S = q.size(2), D = q.size(3);
   const int64_t Hkv = k.size(1), Sk = k.size(2);
-  MX_CHECK(D == 128 && Sk == S, "attn_bwd_rope: D = 128 self-attention");
+  MX_CHECK((D == 128 || D == 64) && Sk == S, "attn_bwd_rope: D = 64 or 128, self-attention");
   check_f32(cos, "cos");
   check_f32(sin, "sin");
   MX_CHECK(cos.is_contiguous() && sin.is_contiguous() && cos.numel() >= S * (D / 2) && sin.numel() >= S * (D / 2),

@@ -1388,7 +1388,8 @@ using namespace mx;
 // dq_mode 2 (deterministic): work = ceil(Sk/128) * B*Hq*ceil(S/64)*64*D floats (no
 //   zeroing); dq receives the result unpadded [B,Hq,S,D], reduced in a fixed order.
 // dq_mode 3 (split, default): work = B*Hq * ceil(Sk/128)*128 * ceil(S/64)*64 bf16 (dS^T,
-//   no zeroing); dq receives [B,Hq,S,D] from attn_bwd_dq_kernel.  Deterministic.
+//   no zeroing); dq receives [B,Hq,S,D] from attn_bwd_dq_kernel.  Deterministic.  At D = 64
+//   attn_bwd64.hip's two passes instead, which need no work.
 // delta: workspace [B,Hq,S].
 // q-heads per workgroup of the 8-wave backward (split mode, D = 128): the largest of 4 / 2 / 1
 // that divides the GQA group and still leaves >= 2 workgroups per CU (512) for the causal
@@ -1424,6 +1425,12 @@ extern "C" int mx_attn_bwd_partial_heads(int B, int Hq, int Hkv, int S, int Sk, 
   return Hq / attn_bwd8_hpw(B, Hq, Hkv, S, Sk, D, dq_mode);
 }
 
+// attn_bwd64.hip
+int mx_attn_bwd64(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* o, const uint16_t* dout,
+                  const float* lse, float* delta, float* dq, float* dkp, float* dvp, int B, int Hq, int Hkv, int S, int Sk,
+                  bool causal, float scale, int64_t ldo, uint16_t* dqkv, int64_t ldq, const float* cosb,
+                  const float* sinb, hipStream_t stream);
+
 extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* o,
                            const uint16_t* dout, const float* lse, float* delta, float* dq, float* dkp, float* dvp,
                            int B, int Hq, int Hkv, int S, int Sk, int D, int causal, float scale, int dq_mode,
@@ -1431,9 +1438,13 @@ extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t*
                            const float* cosb, const float* sinb) {
   if (B <= 0 || S <= 0 || Sk <= 0) return 0;
   if (Hkv <= 0 || Hq % Hkv) return -1;
-  if (dq_mode < 1 || dq_mode > 3 || (dq_mode > 1 && !work)) return -1;
-  // dqkv: the split dQ kernel writes d(q) with the inverse RoPE into it (D = 128, split mode only)
-  if (dqkv && (dq_mode != 3 || D != 128 || !cosb || !sinb || ldq % 8 || causal < 0)) return -1;
+  const bool two_pass = dq_mode == 3 && D == 64;
+  if (dq_mode < 1 || dq_mode > 3 || (dq_mode > 1 && !work && !two_pass)) return -1;
+  // dqkv: the split dQ kernel writes d(q) with the inverse RoPE into it (D = 64 and 128, split mode only)
+  if (dqkv && (dq_mode != 3 || (D != 128 && D != 64) || !cosb || !sinb || ldq % 8 || causal < 0)) return -1;
+  if (two_pass && causal >= 0)
+    return mx_attn_bwd64(q, k, v, o, dout, lse, delta, dq, dkp, dvp, B, Hq, Hkv, S, Sk, causal != 0, scale, ldo, dqkv, ldq,
+                         cosb, sinb, stream);
   const int64_t rows = (int64_t)B * S * Hq;
   const int64_t dthreads = rows * (D / 8);
   const unsigned dgrid = (unsigned)((dthreads + 255) / 256);
@@ -1524,17 +1535,19 @@ extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t*
       attn_bwd8_kernel<false><<<grid8, 512, 0, stream>>>(q, k, v, dout, lse, delta, dst, dkp, dvp, B, Hq, Hkv, S, Sk,
                                                          off, sl, scale, S_pad, bwd8_prio, hpw);
   } else {
-#define BWD(DD, C)                                                                                                  \
-  do {                                                                                                              \
-    if (dq_mode == 3)                                                                                               \
-      attn_bwd_kernel<DD, C, 3><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S,  \
-                                                          Sk, off, sl, scale, S_pad);                               \
-    else if (dq_mode == 2)                                                                                          \
-      attn_bwd_kernel<DD, C, 2><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S,  \
-                                                          Sk, off, sl, scale, S_pad);                               \
-    else                                                                                                            \
-      attn_bwd_kernel<DD, C, 1><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S,  \
-                                                          Sk, off, sl, scale, S_pad);                               \
+#define BWD(DD, C)                                                                                                   \
+  do {                                                                                                               \
+    if (dq_mode == 3) {                                                                                              \
+      if constexpr (DD != 64) /* (D = 64 left above) */                                                              \
+        attn_bwd_kernel<DD, C, 3><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S, \
+                                                            Sk, off, sl, scale, S_pad);                              \
+    } else if (dq_mode == 2) {                                                                                       \
+      attn_bwd_kernel<DD, C, 2><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S,   \
+                                                          Sk, off, sl, scale, S_pad);                                \
+    } else {                                                                                                         \
+      attn_bwd_kernel<DD, C, 1><<<grid, 256, 0, stream>>>(q, k, v, dout, lse, delta, dqk, dkp, dvp, B, Hq, Hkv, S,   \
+                                                          Sk, off, sl, scale, S_pad);                                \
+    }                                                                                                                \
   } while (0)
   if (D == 128) { if (causal) BWD(128, true); else BWD(128, false); }
   else if (D == 64) { if (causal) BWD(64, true); else BWD(64, false); }
@@ -1556,7 +1569,7 @@ extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t*
     else RED(32);
 #undef RED
   } else if (dq_mode == 3) {
-    // 128 q rows per workgroup (every K tile feeds two 64-row sub-blocks); D=32 keeps 64
+    // 256 q rows per workgroup (every K tile feeds four 64-row sub-blocks); D=32 keeps 64
     // MXLLM_ATTN_DQ_QB=2 (experiment): D = 128 with 128 q rows per workgroup and a 4-deep ring
 #ifdef MXLLM_ATTN_EXPERIMENTS
     static const int qb128 = [] {
@@ -1566,12 +1579,12 @@ extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t*
 #else
     constexpr int qb128 = 4;
 #endif
-    const int qbs = D == 128 ? qb128 : (D == 64 ? 2 : 1);
+    const int qbs = D == 128 ? qb128 : 1;
     const int qgrid = ((S + 64 * qbs - 1) / (64 * qbs)) * B * Hq;
     const uint16_t* dst = reinterpret_cast<const uint16_t*>(work);
 #define DQK(DD)                                                                                                   \
   do {                                                                                                            \
-    constexpr int QB = DD == 128 ? 4 : (DD == 64 ? 2 : 1);                                                        \
+    constexpr int QB = DD == 128 ? 4 : 1;                                                                         \
     if (causal)                                                                                                   \
       attn_bwd_dq_kernel<DD, true, QB><<<qgrid, 256 * QB, 0, stream>>>(dst, k, dq, B, Hq, Hkv, S, Sk, off, S_pad,  \
                                                                        nkb * 128, scale, dqkv, ldq, cosb, sinb);  \
@@ -1590,7 +1603,6 @@ extern "C" int mx_attn_bwd(const uint16_t* q, const uint16_t* k, const uint16_t*
     } else
 #endif
     if (D == 128) DQK(128);
-    else if (D == 64) DQK(64);
     else DQK(32);
 #undef DQK
   }
