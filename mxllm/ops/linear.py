@@ -424,9 +424,10 @@ def param_weight_grad(wp: torch.Tensor | None, dy: torch.Tensor, x: torch.Tensor
         return weight_grad_(None, dy, x, dy_scale=dy_scale)
     fresh = getattr(wp, "_mx_grad_fresh", False)
     # the trainer's fused clip norm (mxllm/train/trainer.py): a first write (beta 0) of a gradient
-    # whose owner armed `_mx_sq` also leaves the per-tile sums of squares of the stored values
+    # whose owner armed `_mx_sq` also leaves the per-tile sums of squares of the stored values (not where another
+    # use of the parameter writes after it)
     armed = getattr(wp, "_mx_sq_done", None)
-    sq = getattr(wp, "_mx_sq", None) if fresh and armed is False else None
+    sq = getattr(wp, "_mx_sq", None) if fresh and armed is False and not getattr(wp, "_mx_two_uses", False) else None
     if sq is not None and g.dtype == dy.dtype == x.dtype == torch.bfloat16 and gemm.mm_sq(
             "tt", dy, x, g, sq, None if dy_scale is None else dy_scale.reshape(1).float()):
         wp._mx_sq_done = True

@@ -2,9 +2,12 @@
 themselves (e.g. the fused LoRA backward writes dA/dB straight into the flat
 grad buffer with beta=1 GEMMs instead of returning them to autograd).
 Such ops call ``mark_ready(p)``; DDP registers ``p._mx_on_grad_ready``."""
+import contextlib
 
 
 def mark_ready(p) -> None:
+    if getattr(p, "_mx_two_uses", False):
+        return  # one write of several (two_uses): the owner takes it once the backward is through
     h = getattr(p, "_mx_on_grad_ready", None)
     if h is not None:
         h(p)
@@ -12,8 +15,8 @@ def mark_ready(p) -> None:
 
 def direct_grad(p):
     """The preallocated .grad of ``p`` if it can be accumulated into in place
-    (never for a parameter used twice in the graph, e.g. a tied embedding/head:
-    its gradient is complete only after autograd summed both uses)."""
+    (for a parameter used twice in the graph, e.g. a tied embedding/head, only under
+    :func:`two_uses`: its gradient is complete only after both uses)."""
     if getattr(p, "_mx_no_direct", False):
         return None
     g = p.grad
@@ -31,6 +34,26 @@ def direct_grad32(p):
     if getattr(p, "_mx_no_direct", False):
         return None
     return getattr(p, "_mx_grad32", None)
+
+
+def hook_count(p) -> int:
+    return len(p._backward_hooks or ()) + len(getattr(p, "_post_accumulate_grad_hooks", None) or ())
+
+
+@contextlib.contextmanager
+def two_uses(params):
+    """While a backward runs whose owner looks at gradients only after it: parameters used twice in the graph
+    (tied embedding and head) take the gradients of both uses in place too.  ``params``: (parameter, the
+    :func:`hook_count` its owner left it with); one that has got hooks since, which want the sum that autograd makes,
+    stays with autograd."""
+    on = [p for p, n in params if getattr(p, "_mx_no_direct", False) and hook_count(p) == n]
+    for p in on:
+        p._mx_no_direct, p._mx_two_uses = False, True
+    try:
+        yield
+    finally:
+        for p in on:
+            p._mx_no_direct, p._mx_two_uses = True, False
 
 
 def grad_slot(p):

@@ -18,6 +18,7 @@ import torch
 from .. import ops
 from ..parallel.ddp import DDP
 from ..parallel.flat import FlatParams, production_order
+from ..parallel.grad_ready import hook_count, two_uses
 from ..parallel.runtime import DistEnv
 from ..utils.profiling import range_
 
@@ -151,10 +152,9 @@ class Trainer:
         # itself (2-4 B/param less HBM traffic per step); under ZeRO-1 the full
         # gradient buffer is then not cleared behind each reduce-scatter either (8B:
         # a 16 GB memset per step).  GPU kernels only; not with LoRA (its kernels
-        # accumulate).  A parameter used twice (tied embeddings) is summed by autograd, whose one
-        # addition finds the slot zeroed by _fresh_guard: 0.1 ms for 128256 x 2048, against AdamW
-        # clearing every gradient (1.2 B parameters: 0.5 ms), a full pass for the clip norm (0.44)
-        # and weight gradients that read what they are added to (0.3)
+        # accumulate).  Both gradients of a parameter used twice (tied embedding and head) are written in place
+        # too (grad_ready.two_uses): the head's over last step's, the embedding's rows onto it.  Summed by autograd,
+        # 128256 x 2048 cost two passes and two fills more, 0.7 ms of a step of 37
         self.fresh_grads = (os.environ.get("MXLLM_FRESH_GRADS", "1") != "0" and self.flat.device.type == "cuda"
                             and not getattr(model, "lora", False))
         if self.zero1 is not None:
@@ -189,6 +189,8 @@ class Trainer:
             for p in self.flat.param_list:
                 if p.requires_grad:
                     p.register_hook(_fresh_guard(p))
+        self._two_uses = [(p, hook_count(p)) for p in self.flat.param_list
+                          if self.flat.device.type == "cuda" and getattr(p, "_mx_no_direct", False)]
         # ---- gradient-norm overlap: each DDP bucket's sum of squares is taken on a side
         # stream as soon as the bucket is final (after its all-reduce), under the rest of
         # the backward, instead of one pass over the whole gradient after it (8B full:
@@ -421,7 +423,7 @@ class Trainer:
             with ctx:
                 with range_("forward"):
                     loss = self.model(ids, labels)
-                with range_("backward"):
+                with range_("backward"), two_uses(self._two_uses):
                     (loss / n if n > 1 else loss).backward()
             total = loss.detach() if total is None else total + loss.detach()
         if self._deferred:  # a forward that skipped parameter groups: nothing may stay un-updated
