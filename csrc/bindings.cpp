@@ -158,6 +158,30 @@ bool gemm8(const at::Tensor& a, bool a_kc, const at::Tensor& b, bool b_kc, at::T
   return true;
 }
 
+// out[M, N] (bf16) = a b, a [M, K], or, tt, a^T b (beta 1: + out), a [K, M]; b [K, N]: by tile `tile` of gemm_tile_form_plan.
+// Returns false (nothing launched) for sizes, strides and addresses it does not take.
+bool gemm_tile_form(const at::Tensor& a, const at::Tensor& b, at::Tensor& out, bool tt, double beta, int64_t tile) {
+  MX_CHECK(a.is_cuda() && b.device() == a.device() && out.device() == a.device(), "gemm_tile_form: tensors of one GPU");
+  MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16 && out.scalar_type() == at::kBFloat16,
+           "gemm_tile_form: bf16 tensors");
+  MX_CHECK(a.dim() == 2 && b.dim() == 2 && out.dim() == 2, "gemm_tile_form: 2-D tensors");
+  const int64_t K = b.size(0), N = b.size(1), M = out.size(0);
+  MX_CHECK(out.size(1) == N && a.size(tt ? 0 : 1) == K && a.size(tt ? 1 : 0) == M, "gemm_tile_form: shape mismatch");
+  if (a.stride(1) != 1 || b.stride(1) != 1 || out.stride(1) != 1 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX ||
+      (beta != 0.0 && beta != 1.0))
+    return false;
+  DevGuard g(a.device());
+  const int rc = mx_gemm_tile_form(bf(a), a.stride(0), bf(b), b.stride(0), bfm(out), out.stride(0), (int)M, (int)N, (int)K,
+                                   tt ? 1 : 0, beta != 0.0, (int)tile, cur_stream());
+  if (rc == -1) return false;
+  MX_OK(rc);
+  return true;
+}
+
+int64_t gemm_tile_form_plan(bool tt, int64_t M, int64_t N, int64_t K) {
+  return M > INT32_MAX || N > INT32_MAX || K > INT32_MAX ? -1 : mx_gemm_tile_form_plan(tt ? 1 : 0, (int)M, (int)N, (int)K);
+}
+
 // out[M, N] (bf16, beta 0) = alpha op(a) op(b) that also writes one fp32 sum of squares of the stored
 // values per 256 x 256 output tile into sq (>= (M / 256) * (N / 256) elements, row-major tile order):
 // the gradient-clip norm's partials straight from the weight-gradient GEMMs.  False: nothing launched.
@@ -984,6 +1008,8 @@ TORCH_LIBRARY(mxllm, m) {
   m.def("gemm8_rope(Tensor x, Tensor w, Tensor cos, Tensor sin, int B, int S, int Hq, int Hkv, Tensor(a!) q, Tensor(b!) k, Tensor(c!) v) -> bool");
   m.def("gemm8_rope_tail(Tensor x, Tensor w, Tensor cos, Tensor sin, int B, int S, int Hq, int Hkv, Tensor(a!) q, Tensor(b!) k, Tensor(c!) v, int at) -> bool");
   m.def("gemm8_swiglu(Tensor x, Tensor w, Tensor(a!) gu, Tensor(b!) m) -> bool");
+  m.def("gemm_tile_form(Tensor a, Tensor b, Tensor(a!) out, bool tt, float beta, int tile) -> bool");
+  m.def("gemm_tile_form_plan(bool tt, int M, int N, int K) -> int", &gemm_tile_form_plan);
   m.def("gemm8_sq(Tensor a, bool a_kc, Tensor b, bool b_kc, Tensor(a!) out, Tensor(b!) sq, Tensor? alpha_t=None, float alpha=1.0) -> bool");
   m.def("gemm8_swiglu_bwd(Tensor dy, Tensor w, Tensor gu, Tensor(a!) dgu, Tensor(b!)? m=None) -> bool");
   m.def("sqnorm(Tensor x) -> Tensor");
@@ -1027,6 +1053,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("gemm8_rope", &gemm8_rope);
   m.impl("gemm8_rope_tail", &gemm8_rope_tail);
   m.impl("gemm8_swiglu", &gemm8_swiglu);
+  m.impl("gemm_tile_form", &gemm_tile_form);
   m.impl("gemm8_sq", &gemm8_sq);
   m.impl("gemm8_swiglu_bwd", &gemm8_swiglu_bwd);
   m.impl("ce_inv_count", &ce_inv_count);

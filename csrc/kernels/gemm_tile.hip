@@ -23,206 +23,9 @@
 // L2's 15 TB/s (40 KB a step and CU) and the clock under load.
 #include <algorithm>
 
-#include "gemm8_core.h"
+#include "gemm_tile_core.h"
 
 namespace mx {
-
-constexpr int kGtPlain = 0, kGtSwiglu = 1, kGtPart = 2;
-
-template <int N>
-__device__ __forceinline__ void gt_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
-// row of B behind virtual column v of tile pn: with SwiGLU a wave's first half of columns are gate's, the second the same
-// channels of up
-template <int TN, int WN, int EPI>
-__device__ __forceinline__ int gt_row(int v, int pn, int F) {
-  if constexpr (EPI != kGtSwiglu) return pn * TN + v;
-  constexpr int HW = TN / WN / 2;
-  const int q = v % (2 * HW);
-  return (q < HW ? 0 : F) + pn * (TN / 2) + v / (2 * HW) * HW + q % HW;
-}
-
-// TM x TN tile by WM x WN waves, S stages of LDS, OCC workgroups a CU (a launch bound: 256 registers a wave at 2).  kGtPart: C is
-// f32 [parts][M][N].
-template <int TM, int TN, int WM, int WN, int S, int OCC, int EPI>
-__global__ void __launch_bounds__(64 * WM * WN, OCC)
-gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, void* __restrict__ C,
-                 int64_t ldc, int M, int N, int K, int parts) {
-  constexpr int NW = WM * WN, BI = TM / WM / 16, BJ = TN / WN / 16, STG = (TM + TN) * 128;
-  constexpr int QA = TM / 8 / NW, QB = TN / 8 / NW, P = QA + QB;  // DMA pieces of 8 rows of a wave: of A, of B
-  constexpr int NM = BI * BJ, NR = BI + BJ;                      // MFMAs and fragments of a step
-  constexpr int NB = NM / 4 < NM - NR ? NM / 4 : NM - NR;        // MFMAs of the second step ahead of the barrier
-  constexpr int R0 = NM >= 2 * NR ? 2 : 1, R1 = NM - NB >= 2 * NR ? 2 : 1;         // MFMAs from one fragment read to the next
-  constexpr int D0 = NM / (P - P / 2), D1 = (NM - NB) / (P / 2);  // and from one DMA piece to the next
-  static_assert(TM % (8 * NW) == 0 && TN % (8 * NW) == 0 && BJ % 2 == 0 && S >= 3 && NB >= 0 && D0 > 0 && D1 > 0, "tile");
-  __shared__ __attribute__((aligned(1024))) char smem[S * STG];
-  const int nM = (M + TM - 1) / TM, nN = (N + TN - 1) / TN, F = N / 2;
-  int pm, pn, nk = K / 64;
-  {
-    int L = xcd_remap(blockIdx.x, gridDim.x);
-    if constexpr (EPI == kGtPart) {  // parts after each other: an XCD's tiles share the panels of one part of K
-      const int kp = L / (nM * nN), t0 = nk * kp / parts, t1 = nk * (kp + 1) / parts;
-      L -= kp * nM * nN;
-      A += t0 * 64;
-      B += t0 * 64;
-      K -= t0 * 64;
-      nk = t1 - t0;
-      C = reinterpret_cast<float*>(C) + (int64_t)kp * M * N;
-    }
-    constexpr int GM = 8;  // a band of 8 tiles down, then across: an XCD's tiles share their panels in its L2
-    const int per = GM * nN, grp = L / per, first = grp * GM;
-    const int rows = min(GM, nM - first), in = L - grp * per;
-    pm = first + in % rows;
-    pn = in / rows;
-  }
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = w / WN, wn = w % WN;
-  // rows past M and N read the last one again: their products are not stored
-  const int mrem = M - pm * TM;
-  const uint16_t* ab = A + (int64_t)pm * TM * lda;
-  const uint16_t* bb = B + (EPI == kGtSwiglu ? 0 : (int64_t)pn * TN * ldb);
-  const int brows = EPI == kGtSwiglu ? N : min(N - pn * TN, TN);
-  const __amdgpu_buffer_rsrc_t ars =
-      __builtin_amdgcn_make_buffer_rsrc((void*)ab, 0, (uint32_t)(((min(mrem, TM) - 1) * lda + K) * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t brs =
-      __builtin_amdgcn_make_buffer_rsrc((void*)bb, 0, (uint32_t)(((brows - 1) * ldb + K) * 2), 0x00020000);
-  uint32_t off[P];
-#pragma unroll
-  for (int j = 0; j < P; ++j) {
-    const int r = 8 * (j < QA ? w * QA + j : w * QB + j - QA) + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
-    if (j < QA) {
-      off[j] = (uint32_t)((min(r, mrem - 1) * lda + 8 * c) * 2);
-    } else {
-      const int b = min(gt_row<TN, WN, EPI>(r, pn, F), N - 1) - (EPI == kGtSwiglu ? 0 : pn * TN);
-      off[j] = (uint32_t)((b * ldb + 8 * c) * 2);
-    }
-  }
-  auto piece = [&](int j, uint32_t ko, char* dst) __attribute__((always_inline)) {
-    const uint32_t so = off[j] + ko;
-    char* d = dst + (j < QA ? (w * QA + j) * 1024 : TM * 128 + (w * QB + j - QA) * 1024);
-    if (j < QA) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ars, (g8lptr_t)d, 16, so, 0, 0, 0);
-    } else {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(brs, (g8lptr_t)d, 16, so, 0, 0, 0);
-    }
-  };
-  const uint32_t lds0 = lds_addr(smem);
-  uint32_t al[2], bl[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    al[s] = lds0 + g8_kc_lane(lane, s) + wm * (TM / WM) * 128;
-    bl[s] = lds0 + g8_kc_lane(lane, s) + TM * 128 + wn * (TN / WN) * 128;
-  }
-  u16x8 fa[2][BI], fb[2][BJ];
-  f32x4 acc[BI][BJ];
-#pragma unroll
-  for (int i = 0; i < BI; ++i)
-#pragma unroll
-    for (int j = 0; j < BJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // fragment r of set s: B's first, then A's
-  auto read = [&](int s, int r, uint32_t a, uint32_t b) __attribute__((always_inline)) {
-    if (r < BJ) fb[s][r] = rd128_off(b, r * 2048);
-    else fa[s][r - BJ] = rd128_off(a, (r - BJ) * 2048);
-  };
-  // A's fragment i of set s, and with the first all of B's, are there once at most `left` younger LDS reads are not
-  auto have = [&](int s, int i, int left) __attribute__((always_inline)) {
-    lds_wait_le(left > 15 ? 15 : left);
-    pin(fa[s][i]);
-    if (i == 0) {
-#pragma unroll
-      for (int j = 0; j < BJ; ++j) pin(fb[s][j]);
-    }
-  };
-
-#pragma unroll
-  for (int t = 0; t < S; ++t)
-#pragma unroll
-    for (int j = 0; j < P; ++j) piece(j, t < nk ? (uint32_t)t * 128 : G8_OOB, smem + t * STG);
-  gt_vm_wait<(S - 1) * P>();
-  __builtin_amdgcn_s_barrier();
-#pragma unroll
-  for (int r = 0; r < NR; ++r) read(0, r, al[0], bl[0]);
-  int st = 0;  // stage of kt
-  for (int kt = 0; kt < nk; ++kt) {
-    const int nx = st + 1 == S ? 0 : st + 1;
-    {  // step 0: multiply set 0, read set 1; the second half of tile kt + S - 1's pieces
-      const uint32_t a1 = al[1] + st * STG, b1 = bl[1] + st * STG;
-      char* dst = smem + (st == 0 ? S - 1 : st - 1) * STG;
-      const uint32_t ko = kt > 0 && kt + S - 1 < nk ? (uint32_t)(kt + S - 1) * 128 : G8_OOB;
-#pragma unroll
-      for (int n = 0; n < NM; ++n) {
-        const int i = n / BJ, j = n % BJ, r = n / R0, d = n / D0;
-        if (j == 0) have(0, i, BI - 1 - i + min((n + R0 - 1) / R0, NR));
-        acc[i][j] = g8_mfma(fb[0][j], fa[0][i], acc[i][j]);
-        if (n % R0 == 0 && r < NR) read(1, r, a1, b1);
-        if (n % D0 == D0 - 1 && d < P - P / 2 && kt > 0) piece(P / 2 + d, ko, dst);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    {  // step 1: multiply set 1; behind the barrier read set 0 of the next tile, and the first half of tile kt + S's pieces
-      const uint32_t a0 = al[0] + nx * STG, b0 = bl[0] + nx * STG;
-      char* dst = smem + st * STG;
-      const uint32_t ko = kt + S < nk ? (uint32_t)(kt + S) * 128 : G8_OOB;
-#pragma unroll
-      for (int n = 0; n < NM; ++n) {
-        const int i = n / BJ, j = n % BJ, q = n - NB, r = q / R1, d = q / D1;
-        if (q == 0) {  // this wave's reads of stage st are done, its pieces of tile kt + 1 landed
-          lds_wait();
-          gt_vm_wait<(S - 2) * P>();
-          __builtin_amdgcn_s_barrier();
-        }
-        if (j == 0) have(1, i, q < 0 ? BI - 1 - i : 15);
-        acc[i][j] = g8_mfma(fb[1][j], fa[1][i], acc[i][j]);
-        if (q >= 0 && q % R1 == 0 && r < NR) read(0, r, a0, b0);  // (behind the last tile: bytes that are not multiplied)
-        if (q >= 0 && q % D1 == D1 - 1 && d < P / 2) piece(d, ko, dst);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    st = nx;
-  }
-  // the reads behind the last tile own their registers, and the DMA behind K its LDS, until here
-#pragma unroll
-  for (int i = 0; i < BI; ++i) have(0, i, 0);
-  gt_vm_wait<0>();
-  const int ml = pm * TM + wm * (TM / WM) + (lane & 15);
-  if constexpr (EPI == kGtPart) {
-    float* c = reinterpret_cast<float*>(C);
-    const int n0 = pn * TN + wn * (TN / WN) + 4 * (lane >> 4);
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ; ++j)
-        if (ml + 16 * i < M && n0 + 16 * j < N)
-          *reinterpret_cast<f32x4*>(c + (int64_t)(ml + 16 * i) * N + n0 + 16 * j) = acc[i][j];
-  } else if constexpr (EPI == kGtSwiglu) {
-    uint16_t* c = reinterpret_cast<uint16_t*>(C);
-    const int n0 = pn * (TN / 2) + wn * (TN / WN / 2) + 4 * (lane >> 4);
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ / 2; ++j) {
-        u16x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float g = g8_rbf(acc[i][j][e]), u = g8_rbf(acc[i][BJ / 2 + j][e]);
-          o[e] = f2bf(g * g8_sigmoid(g) * u);
-        }
-        if (ml + 16 * i < M && n0 + 16 * j < F) *reinterpret_cast<u16x4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o;
-      }
-  } else {
-    uint16_t* c = reinterpret_cast<uint16_t*>(C);
-    const int n0 = pn * TN + wn * (TN / WN) + 16 * ((lane >> 4) & 1) + 8 * (lane >> 5);
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ; j += 2) {
-        const uint4 o = g8_pack8(acc[i][j], acc[i][j + 1]);  // lanes exchange: outside the row test
-        if (ml + 16 * i < M && n0 + 16 * j < N) *reinterpret_cast<uint4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o;
-      }
-  }
-}
 
 // The tiles, and what a turn of them takes, us: start + steps of 64 k (step + load units / 256) + memory MB of weights + with K
 // in parts, sum + part parts (part + glu with SwiGLU) + image MB of f32 images.  Fitted to 89,000 runs of 350 sizes of weights

@@ -16,7 +16,8 @@ twice as many half-K workgroups, e.g. the 16 x 40-tile 70B qkv forward), by the 
 for the sizes that the table does not hold, or for every shape it takes in deterministic mode
 (``MXLLM_DETERMINISTIC=1``: one workgroup per output tile, a fixed K order, no split-K or atomics —
 the step is bitwise reproducible; vendor stream-K solutions are not, archive/profiles/r3aa).
-``MXLLM_GEMM8=0`` disables it, ``=all`` forces it wherever it takes the shape (A/B runs).
+``MXLLM_GEMM8=0`` disables it, ``=all`` forces it wherever it takes the shape (A/B runs).  Gradients whose output is one turn
+of smaller tiles go to csrc/kernels/gemm_tile_forms.hip ahead of both (:func:`form_plan`; one workgroup a tile, K in order).
 """
 from __future__ import annotations
 
@@ -185,6 +186,31 @@ def tile_plan(M: int, N: int, K: int, swiglu: bool = False) -> tuple[int, int] |
     return None if _policy() == "0" else _tile_plan(M, N, K, swiglu)
 
 
+@functools.lru_cache(maxsize=4096)
+def _form_plan(tt: bool, M: int, N: int, K: int) -> int:
+    return native().gemm_tile_form_plan(tt, M, N, K)
+
+
+def form_plan(form: str, M: int, N: int, K: int) -> int:
+    """Tile of a gradient's product ("nn", "tt") that csrc/kernels/gemm_tile_forms.hip has faster than the library and gemm8
+    (the rule is beside the kernel: mx_gemm_tile_form_plan); -1: not, or MXLLM_GEMM8 asks for one of those."""
+    return _form_plan(form == "tt", M, N, K) if _policy() == "table" else -1
+
+
+def form_mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None, beta: float = 0.0):
+    """``out = beta * out + op(a) b`` (bf16; ``out`` None: new) by that kernel; None: it does not take the call."""
+    if not (use_native(a) and a.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16 and a.numel() and b.numel()
+            and (out is None or out.dtype == torch.bfloat16)) or asks_grad(a, b):
+        return None
+    M, N, K = _dims(form, a, b)
+    tile = form_plan(form, M, N, K)
+    if tile < 0:
+        return None
+    if out is None:
+        out, beta = torch.empty(M, N, dtype=a.dtype, device=a.device), 0.0
+    return out if native().gemm_tile_form(a, b, out, form == "tt", float(beta), tile) else None
+
+
 def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
     """Parts of K (1: whole) in which the rows kernel is the faster one, else 0.
 
@@ -267,6 +293,10 @@ def mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = N
     M, N, K = _dims(form, a, b)
     odt = out.dtype if out is not None else (out_dtype or a.dtype)
     asked = asks_grad(a, b)
+    if form in ("nn", "tt") and alpha_t is None and odt == torch.bfloat16 and (form == "tt" or beta == 0.0):
+        y = form_mm(form, a, b, out, beta)
+        if y is not None:
+            return y
     if out is None and not asked and form in ("tn", "nn") and alpha_t is None and odt == torch.bfloat16:
         parts = rows_gain(M, N, K, form == "tn")
         if parts and rows_ok(a, b, form == "tn"):
@@ -306,7 +336,7 @@ def mm_sq(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor, sq: to
     M, N, K = _dims(form, a, b)
     if not (use_native(a) and a.dtype == b.dtype == out.dtype == torch.bfloat16 and M % 256 == 0 and N % 256 == 0):
         return False
-    if schedule(form, M, N, K, torch.bfloat16) != 4:
+    if schedule(form, M, N, K, torch.bfloat16) != 4 or (alpha_t is None and form_plan(form, M, N, K) >= 0):
         return False
     a_kc, b_kc = _KC[form]
     t = _TAIL.get((form, M, N, K, "bf16"), 0)

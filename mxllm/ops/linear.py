@@ -383,6 +383,9 @@ def weight_grad_(out: torch.Tensor | None, dy: torch.Tensor, x: torch.Tensor, be
     if use_native(dy) and dy.dtype == torch.bfloat16 and x.dtype == torch.bfloat16:
         # token-major operands straight into the 8-phase MFMA GEMM (no transposes) where it wins
         odt = out.dtype if out is not None else dy.dtype
+        y = gemm.form_mm("tt", dy, x, out, beta) if dy_scale is None and beta in (0.0, 1.0) else None
+        if y is not None:
+            return y
         if gemm.want("tt", dy.shape[1], x.shape[1], dy.shape[0], odt, not gemm.asks_grad(dy, x)):
             sc = None if dy_scale is None else dy_scale.reshape(1).float()
             return gemm.mm("tt", dy, x, out=out, beta=beta if out is not None else 0.0, alpha_t=sc,

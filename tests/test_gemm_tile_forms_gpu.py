@@ -1,0 +1,71 @@
+"""Gradients by one turn of tiles (csrc/kernels/gemm_tile_forms.hip) at the edges of their tiles and of K, against 64-bit sums of
+the same bf16 operands."""
+import pytest
+import torch
+
+from mxllm.ops import gemm
+
+pytestmark = pytest.mark.gpu
+TILES = [(64, 64), (64, 128), (128, 128), (128, 192), (192, 128), (256, 128), (192, 192)]
+
+
+def _operands(gpu, tt, M, N, K, pad):
+    torch.manual_seed(M + 3 * N + 7 * K)
+    a = torch.randn(K, M + pad, device=gpu).bfloat16()[:, :M] if tt else torch.randn(M, K + pad, device=gpu).bfloat16()[:, :K]
+    b = torch.randn(K, N + pad, device=gpu).bfloat16()[:, :N]
+    x = a.double().t().contiguous() if tt else a.double()
+    return a, b, x @ b.double()
+
+
+def _close(got, want, K, old=None):
+    # f32 sums of K products of unit operands (K 2^-24 of their sizes' sum at most, far less as seen) and one rounding to bf16
+    assert float((got.double() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max()) + 2.0 ** -23 * K
+    assert float((got.double() - want).norm()) <= 2.0 ** -8 * float(want.norm())
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("K,pad", [(64, 0), (128, 8), (192, 0), (448, 64)])
+def test_input_gradients(gpu, tile, K, pad):
+    from mxllm.ops import native
+
+    tm, tn = TILES[tile]
+    for M, N in [(1, 16), (tm, tn), (tm + 1, tn + 16), (2 * tm - 1, 3 * tn - 48)]:
+        a, b, want = _operands(gpu, False, M, N, K, pad)
+        out = torch.full((M, N + 8), 7.0, device=gpu).bfloat16()
+        assert native().gemm_tile_form(a, b, out[:, :N], False, 0.0, tile)
+        _close(out[:, :N], want, K)
+        assert bool((out[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("tile", range(len(TILES)))
+@pytest.mark.parametrize("K,pad", [(1, 0), (63, 8), (64, 0), (65, 0), (200, 16), (449, 0)])
+def test_weight_gradients(gpu, tile, K, pad):
+    from mxllm.ops import native
+
+    tm, tn = TILES[tile]
+    for M, N in [(16, 16), (tm, tn), (tm + 16, tn + 48), (2 * tm - 16, 3 * tn - 16)]:
+        a, b, want = _operands(gpu, True, M, N, K, pad)
+        out = torch.full((M, N), float("nan"), device=gpu).bfloat16()
+        assert native().gemm_tile_form(a, b, out, True, 0.0, tile)
+        _close(out, want, K)
+        old = torch.randn(M, N, device=gpu).bfloat16()
+        out = old.clone()
+        assert native().gemm_tile_form(a, b, out, True, 1.0, tile)
+        _close(out, want + old.double(), K)
+
+
+@pytest.mark.parametrize("form,M,N,K", [("tt", 2048, 512, 1003), ("tt", 768, 768, 256), ("nn", 333, 1024, 512), ("nn", 1000, 512, 8192)])
+def test_route(gpu, form, M, N, K):
+    """``gemm.mm`` takes the kernel for the sizes of its rule, and leaves others and unaligned operands alone."""
+    from mxllm.ops import native
+
+    a, b, want = _operands(gpu, form == "tt", M, N, K, 0)
+    tile = gemm.form_plan(form, M, N, K)
+    assert tile >= 0
+    out = torch.empty(M, N, device=gpu, dtype=torch.bfloat16)
+    assert native().gemm_tile_form(a, b, out, form == "tt", 0.0, tile)
+    assert torch.equal(gemm.mm(form, a, b), out)
+    _close(out, want, K)
+    shifted = torch.empty(b.numel() + 4, device=gpu, dtype=torch.bfloat16)[4:].view_as(b).copy_(b)
+    assert gemm.form_mm(form, a, shifted) is None
+    _close(gemm.mm(form, a, shifted), want, K)
