@@ -60,7 +60,7 @@ int mx_gemm8_epi(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb,
                  int N, int K, int mode, MxG8Epi ep, hipStream_t stream);
 int mx_gemm_tile_plan(int M, int N, int K, int swiglu);
 int mx_gemm_tile(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc, int M, int N, int K,
-                 int swiglu, int tile, int parts, float* ws, hipStream_t stream);
+                 int glu, float limit, int tile, int parts, float* ws, hipStream_t stream);
 int mx_gemm_tile_form_plan(int tt, int M, int N, int K);
 int mx_gemm_tile_form(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, uint16_t* C, int64_t ldc, int M, int N,
                       int K, int tt, int add, int tile, hipStream_t stream);

@@ -177,7 +177,7 @@ at::Tensor gemm8_rows(const at::Tensor& a, const at::Tensor& b, bool b_kc, bool 
 
 // a b^T (bf16) for any number of rows, a [M, K], b [N, K], or silu(gate) up [M, N / 2] of b = [gate; up]: tile `tile` with K in
 // `parts` (mx_gemm_tile; callers ask gemm_tile_plan and mxllm/ops/gemm.py rows_ok first).
-at::Tensor gemm_tile(const at::Tensor& a, const at::Tensor& b, bool swiglu, int64_t tile, int64_t parts) {
+static at::Tensor run_gemm_tile(const at::Tensor& a, const at::Tensor& b, int glu, float limit, int64_t tile, int64_t parts) {
   MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm_tile: GPU tensors of one device");
   MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm_tile: bf16 operands");
   MX_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == b.size(1), "gemm_tile: a [M, K], b [N, K]");
@@ -186,14 +186,23 @@ at::Tensor gemm_tile(const at::Tensor& a, const at::Tensor& b, bool swiglu, int6
            "gemm_tile: row-major operands");
   MX_CHECK(parts >= 1 && (parts == 1 || parts <= K / 64), "gemm_tile: parts of at least 64 of K");
   DevGuard g(a.device());
-  auto out = at::empty({M, swiglu ? N / 2 : N}, a.options());
+  auto out = at::empty({M, glu ? N / 2 : N}, a.options());
   at::Tensor ws;
   if (parts > 1) ws = at::empty({parts * M * N}, a.options().dtype(at::kFloat));
-  const int rc = mx_gemm_tile(bf(a), a.stride(0), bf(b), b.stride(0), bfm(out), out.stride(0), (int)M, (int)N, (int)K, swiglu ? 1 : 0,
+  const int rc = mx_gemm_tile(bf(a), a.stride(0), bf(b), b.stride(0), bfm(out), out.stride(0), (int)M, (int)N, (int)K, glu, limit,
                               (int)tile, (int)parts, parts > 1 ? ws.data_ptr<float>() : nullptr, cur_stream());
   MX_CHECK(rc != -1, "gemm_tile: shape, stride or alignment not taken");
   MX_OK(rc);
   return out;
+}
+
+at::Tensor gemm_tile(const at::Tensor& a, const at::Tensor& b, bool swiglu, int64_t tile, int64_t parts) {
+  return run_gemm_tile(a, b, swiglu ? 1 : 0, 0.f, tile, parts);
+}
+
+// the same for a gated unit of clipped inputs (mx_clipped_glu), K in one part
+at::Tensor gemm_tile_clipped(const at::Tensor& a, const at::Tensor& b, double limit, int64_t tile) {
+  return run_gemm_tile(a, b, 2, (float)limit, tile, 1);
 }
 
 // (tile, parts) of K for a product as 64 tile + parts; -1: not a size for gemm_tile
@@ -504,6 +513,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
   m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
   m.def("gemm_tile(Tensor a, Tensor b, bool swiglu, int tile, int parts) -> Tensor");
+  m.def("gemm_tile_clipped(Tensor a, Tensor b, float limit, int tile) -> Tensor");
   m.def("gemm_tile_plan(int M, int N, int K, bool swiglu) -> int", &gemm_tile_plan);
   m.def("stream_linear(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, bool swiglu) -> (Tensor, Tensor)");
   m.def("stream_qkv_rope(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, Tensor cos, "
@@ -531,6 +541,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn", &decode_attn);
   m.impl("gemm8_rows", &gemm8_rows);
   m.impl("gemm_tile", &gemm_tile);
+  m.impl("gemm_tile_clipped", &gemm_tile_clipped);
   m.impl("stream_linear", &stream_linear);
   m.impl("stream_parts", &stream_parts);
   m.impl("parts_norm", &parts_norm);

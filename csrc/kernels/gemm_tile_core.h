@@ -3,10 +3,12 @@
 #pragma once
 
 #include "gemm8_core.h"
+#include "hybrid.h"
 
 namespace mx {
 
-constexpr int kGtPlain = 0, kGtSwiglu = 1, kGtPart = 2, kGtAdd = 3;
+constexpr int kGtPlain = 0, kGtSwiglu = 1, kGtPart = 2, kGtAdd = 3, kGtClipped = 4;
+constexpr bool gt_glu(int epi) { return epi == kGtSwiglu || epi == kGtClipped; }
 
 template <int N>
 __device__ __forceinline__ void gt_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
@@ -15,7 +17,7 @@ __device__ __forceinline__ void gt_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)
 // channels of up
 template <int TN, int WN, int EPI>
 __device__ __forceinline__ int gt_row(int v, int pn, int F) {
-  if constexpr (EPI != kGtSwiglu) return pn * TN + v;
+  if constexpr (!gt_glu(EPI)) return pn * TN + v;
   constexpr int HW = TN / WN / 2;
   const int q = v % (2 * HW);
   return (q < HW ? 0 : F) + pn * (TN / 2) + v / (2 * HW) * HW + q % HW;
@@ -32,11 +34,12 @@ __device__ __forceinline__ uint32_t gt_mn_lane(int lane, int idx) {
 }
 
 // TM x TN tile by WM x WN waves, S stages of LDS, OCC workgroups a CU (a launch bound: 256 registers a wave at 2).  kGtPart: C is
-// f32 [parts][M][N]; kGtAdd: the product is added to C.  AK, BK: A is [M][K], B is [N][K]; else [K][M], [K][N].
+// f32 [parts][M][N]; kGtAdd: the product is added to C; kGtClipped: as kGtSwiglu, the unit of inputs clipped to `limit` (hybrid.h).
+// AK, BK: A is [M][K], B is [N][K]; else [K][M], [K][N].
 template <int TM, int TN, int WM, int WN, int S, int OCC, int EPI, bool AK = true, bool BK = true>
 __global__ void __launch_bounds__(64 * WM * WN, OCC)
 gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __restrict__ B, int64_t ldb, void* __restrict__ C,
-                 int64_t ldc, int M, int N, int K, int parts) {
+                 int64_t ldc, int M, int N, int K, int parts, float limit = 0.f) {
   constexpr int NW = WM * WN, BI = TM / WM / 16, BJ = TN / WN / 16, STG = (TM + TN) * 128;
   constexpr int QA = TM / 8 / NW, QB = TN / 8 / NW, P = QA + QB;  // DMA pieces of 8 rows of a wave: of A, of B
   constexpr int NM = BI * BJ, NR = BI + BJ;                      // MFMAs and fragments of a step
@@ -71,8 +74,8 @@ gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __
   // rows past M and N read the last one again: their products are not stored
   const int mrem = M - pm * TM;
   const uint16_t* ab = A + (int64_t)pm * TM * (AK ? lda : 1);
-  const uint16_t* bb = B + (EPI == kGtSwiglu ? 0 : (int64_t)pn * TN * (BK ? ldb : 1));
-  const int brows = EPI == kGtSwiglu ? N : min(N - pn * TN, TN);
+  const uint16_t* bb = B + (gt_glu(EPI) ? 0 : (int64_t)pn * TN * (BK ? ldb : 1));
+  const int brows = gt_glu(EPI) ? N : min(N - pn * TN, TN);
   const int64_t arec = AK ? (min(mrem, TM) - 1) * lda + K : (K - 1) * lda + mrem;
   const int64_t brec = BK ? (brows - 1) * ldb + K : (K - 1) * ldb + N - pn * TN;
   const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc((void*)ab, 0, (uint32_t)(arec * 2), 0x00020000);
@@ -89,7 +92,7 @@ gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __
     } else if (j < QA) {
       off[j] = (uint32_t)((min(r, mrem - 1) * lda + 8 * c) * 2);
     } else {
-      const int b = min(gt_row<TN, WN, EPI>(r, pn, F), N - 1) - (EPI == kGtSwiglu ? 0 : pn * TN);
+      const int b = min(gt_row<TN, WN, EPI>(r, pn, F), N - 1) - (gt_glu(EPI) ? 0 : pn * TN);
       off[j] = (uint32_t)((b * ldb + 8 * c) * 2);
     }
   }
@@ -245,7 +248,7 @@ gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __
           *reinterpret_cast<u16x4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o[j];
         }
     }
-  } else if constexpr (EPI == kGtSwiglu) {
+  } else if constexpr (gt_glu(EPI)) {
     uint16_t* c = reinterpret_cast<uint16_t*>(C);
     const int n0 = pn * (TN / 2) + wn * (TN / WN / 2) + 4 * (lane >> 4);
 #pragma unroll
@@ -256,7 +259,7 @@ gemm_tile_kernel(const uint16_t* __restrict__ A, int64_t lda, const uint16_t* __
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const float g = g8_rbf(acc[i][j][e]), u = g8_rbf(acc[i][BJ / 2 + j][e]);
-          o[e] = f2bf(g * g8_sigmoid(g) * u);
+          o[e] = f2bf(EPI == kGtClipped ? clipped_glu<uint16_t>(g, u, limit) : g * g8_sigmoid(g) * u);
         }
         if (ml + 16 * i < M && n0 + 16 * j < F) *reinterpret_cast<u16x4*>(c + (int64_t)(ml + 16 * i) * ldc + n0 + 16 * j) = o;
       }

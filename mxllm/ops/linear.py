@@ -818,6 +818,21 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
     return None
 
 
+def linear_clipped(x: torch.Tensor, w: torch.Tensor, limit: float) -> torch.Tensor | None:
+    """Inference: ``clipped_glu(linear(x, w), limit)`` of a prompt pass in the epilogue of csrc/kernels/gemm_tile.hip, with
+    ``w = [gate; up]`` [2F, K]; None when it does not take the call (the caller then runs the two ops)."""
+    if SKINNY_M <= 0 or not x.is_cuda or x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or x.shape[0] <= _DECODE_M:
+        return None
+    # Both read and write each half of the product once less; the unit costs the tiles what SwiGLU does, so its plan holds (us, two
+    # launches -> one: 4096 x 4096 at 512 / 1024 / 1500 / 2048 rows 30.6 / 40.4 / 53.4 / 60.1 -> 21.0 / 34.2 / 50.1 / 54.3, 4096 x 2048
+    # at 65 / 300 / 2048 10.4 / 14.3 / 36.3 -> 8.5 / 10.9 / 29.9, 1024 x 2048 at 128 / 4096 9.8 / 23.1 -> 8.2 / 18.6).  K in parts keeps
+    # the two: the kernel that adds them knows SwiGLU alone.
+    plan = gemm.tile_plan(x.shape[0], *w.shape, True)
+    if not plan or plan[1] > 1 or not _plain(x, w) or not gemm.rows_ok(x, w, True, True, 16):
+        return None
+    return native().gemm_tile_clipped(x, w, limit, plan[0])
+
+
 # rows up to which the RMSNorm runs in the prologue of skinny_gemm.hip (every workgroup recomputes the
 # rows): measured same box, 8B decode batch 1 3.607 -> 3.479 ms and 70B 26.22 -> 24.98 ms, but batch 4
 # 3.83 -> 4.04 ms (archive/profiles/r2s3_decode_ab/); the kernel takes up to 4.  stream_gemm.hip's workgroups

@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 
 from ._ext import native, use_native
-from .linear import linear
+from .linear import linear, linear_clipped
 from .sublayer import clipped_glu
 
 GENERIC_ROWS = 64  # row tile of the products of any size
@@ -33,7 +33,10 @@ def experts(x: torch.Tensor, ids: torch.Tensor, wgu: torch.Tensor, wdown: torch.
     if use_native(x) and few(x, ids.shape[1], wgu, sgu):
         y, _, sh = _run_few(x, ids, None, ids.shape[1], wgu, wdown, limit, sgu, sdown, slimit)
         return y, None, sh
-    sh = None if sgu is None else linear(clipped_glu(linear(x, sgu), slimit), sdown)
+    sh = None
+    if sgu is not None:
+        mid = linear_clipped(x, sgu, slimit)
+        sh = linear(clipped_glu(linear(x, sgu), slimit) if mid is None else mid, sdown)
     if use_native(x):
         bm = MFMA_ROWS if _grouped(x, wgu) else GENERIC_ROWS
         src, inv, tiles = native().moe_group(ids, wgu.shape[0], bm)
