@@ -9,6 +9,8 @@ int mx_post_norm(const mx::PostNorm* a, int f32, hipStream_t stream);
 int mx_post_side(const mx::PostNorm* a, const uint16_t* g, const uint16_t* P, int R, hipStream_t stream);
 int mx_side_act(const void* z, int64_t ldz, const void* emb, int64_t lde, const int64_t* ids, int V, void* y, int f32,
                 int64_t T, int dim, hipStream_t stream);
+int mx_side_gate(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const uint16_t* emb, int64_t lde,
+                 const int64_t* ids, int V, uint16_t* y, int T, int N, int K, hipStream_t stream);
 int mx_clipped_glu(const void* z, int64_t ldz, void* y, int f32, int64_t T, int F, float limit, hipStream_t stream);
 int mx_latent_rows(const mx::LatentRows* a, int f32, hipStream_t stream);
 int mx_latent_attn(const mx::LatentAttn* a, int f32, hipStream_t stream);
@@ -187,6 +189,26 @@ at::Tensor side_act(const at::Tensor& z, const at::Tensor& emb, const at::Tensor
   auto y = at::empty({T, dim}, z.options());
   MX_OK(mx_side_act(z.data_ptr(), ldz, (const char*)emb.data_ptr() + off * emb.element_size(), emb.size(1), id_ptr(ids, T),
                     (int)emb.size(0), y.data_ptr(), f, T, (int)dim, cur_stream()));
+  return y;
+}
+// side_act(x w^T) of a prompt pass, x [T, K], w [N, K] (bf16): mx_side_gate
+at::Tensor side_gate(const at::Tensor& x, const at::Tensor& w, const at::Tensor& emb, const at::Tensor& ids, int64_t off) {
+  MX_CHECK(x.is_cuda() && w.device() == x.device() && emb.device() == x.device(), "side_gate: tensors of one GPU");
+  MX_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && emb.scalar_type() == at::kBFloat16,
+           "side_gate: bf16 tensors");
+  MX_CHECK(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1) && x.stride(1) == 1 && w.stride(1) == 1,
+           "side_gate: x [T, K], w [N, K]");
+  DevGuard g(x.device());
+  const int64_t T = x.size(0), K = x.size(1), N = w.size(0);
+  MX_CHECK(emb.dim() == 2 && emb.is_contiguous() && off >= 0 && off + N <= emb.size(1) && emb.size(0) <= INT32_MAX,
+           "emb [V, >= off + dim]");
+  MX_CHECK(T <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX, "side_gate: sizes");
+  auto y = at::empty({T, N}, x.options());
+  const int rc = mx_side_gate((const uint16_t*)x.data_ptr(), x.stride(0), (const uint16_t*)w.data_ptr(), w.stride(0),
+                              (const uint16_t*)emb.data_ptr() + off, emb.size(1), id_ptr(ids, T), (int)emb.size(0),
+                              (uint16_t*)y.data_ptr(), (int)T, (int)N, (int)K, cur_stream());
+  MX_CHECK(rc != -1, "side_gate: shape, stride or alignment not taken");
+  MX_OK(rc);
   return y;
 }
 at::Tensor clipped_glu(const at::Tensor& z, double limit) {
@@ -534,6 +556,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("post_side(Tensor g, Tensor P, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("mix_post_norm(Tensor src, Tensor? inv, Tensor wts, Tensor? shared, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("side_act(Tensor z, Tensor emb, Tensor ids, int off) -> Tensor");
+  m.def("side_gate(Tensor x, Tensor w, Tensor emb, Tensor ids, int off) -> Tensor");
   m.def("clipped_glu(Tensor z, float limit) -> Tensor");
   m.def("latent_rows(Tensor x, Tensor w, float eps, Tensor cos, Tensor sin, int rot, Tensor rows, int width, Tensor(a!)? pool=None, Tensor? bt=None, int ring=0) -> Tensor");
   m.def("latent_attn(Tensor q, Tensor kv, Tensor lat, Tensor cos, Tensor sin, Tensor rows, Tensor? blocks, Tensor? sink, int H, int D, int R, int E, int rank, int window, float scale) -> Tensor");
@@ -553,6 +576,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("post_side", &post_side);
   m.impl("mix_post_norm", &mix_post_norm);
   m.impl("side_act", &side_act);
+  m.impl("side_gate", &side_gate);
   m.impl("clipped_glu", &clipped_glu);
   m.impl("latent_rows", &latent_rows);
   m.impl("latent_attn", &latent_attn);

@@ -31,7 +31,7 @@ from ..ops.hybrid import PromptRows, RopeTables
 from ..ops.latent import LatentShape
 from ..ops.retention import RetentionShape, decay_table, retention
 from .config import PRESETS
-from .llama import FusedLinear, plain_weight
+from .llama import FusedLinear, hooked, plain_weight
 
 # latent-attention layer types -> whether the softmax has a sink
 LATENT_TYPES = {"latent_attention": False, "latent_attention_2": True}
@@ -390,7 +390,10 @@ class Sigusun(nn.Module):
                 x = sops.post_norm(y, h, layer.norm1, eps)
                 if layer.spec.moe:
                     x = self._mixture(layer, x, h)
-                g = sops.side_act(layer.side_gate(x), self.side_emb, ids, off)
+                w = plain_weight(layer.side_gate)
+                g = None if w is None or hooked(layer.side_gate) else sops.side_gate(x, w, self.side_emb, ids, off)
+                if g is None:
+                    g = sops.side_act(layer.side_gate(x), self.side_emb, ids, off)
             x = sops.side_post(g, plain_weight(layer.side_proj), h, layer.side_norm, eps) if rows.decode else None
             if x is None:
                 x = sops.post_norm(layer.side_proj(g), h, layer.side_norm, eps)

@@ -10,7 +10,9 @@ import os
 
 import torch
 
+from . import gemm
 from ._ext import native, use_native
+from .linear import _DECODE_M, SKINNY_M, _plain
 
 
 def _rms(x: torch.Tensor, eps: float) -> torch.Tensor:
@@ -94,6 +96,20 @@ def side_act(z: torch.Tensor, emb: torch.Tensor, ids: torch.Tensor, off: int) ->
         return native().side_act(z, emb, ids, off)
     e = emb[ids, off:off + z.shape[1]].float()
     return (torch.nn.functional.gelu(z.float(), approximate="tanh") * e).to(z.dtype)
+
+
+def side_gate(x: torch.Tensor, w: torch.Tensor, emb: torch.Tensor, ids: torch.Tensor, off: int) -> torch.Tensor | None:
+    """:func:`side_act` of ``x w^T`` in one launch (csrc/kernels/side_gate.hip); None where it does not take the call."""
+    # One wave a block of 16 rows x 16 channels: past 2,048 of them the library's larger tiles are the quicker ones (with side_act,
+    # us, 64 x 4096 at 8192 / 16384 rows 19.8 / 26.7 -> 15.5 / 28.5, 64 x 2048 11.5 / 16.1 -> 10.3 / 17.7; 256 x 2048 at 2048 / 3000
+    # 11.3 / 11.9 -> 9.2 / 13.5).  A decode step has it behind post_dots.
+    if not use_native(x) or x.dim() != 2 or x.shape[0] <= _DECODE_M or SKINNY_M <= 0:
+        return None
+    (T, K), N = x.shape, w.shape[0]
+    if (N % 16 or K % 64 or off % 4 or (T + 15) // 16 * (N // 16) > 2048 or emb.dtype != torch.bfloat16 or emb.shape[1] % 4
+            or emb.data_ptr() % 8 or not _plain(x, w, emb) or not gemm.rows_ok(x, w, True, cols=16)):
+        return None
+    return native().side_gate(x, w, emb, ids, off)
 
 
 def clipped_glu(z: torch.Tensor, limit: float) -> torch.Tensor:

@@ -4,7 +4,7 @@ import torch
 
 from mxllm.ops import gemm, moe, sublayer
 from mxllm.ops._ext import native
-from mxllm.ops.linear import linear, linear_clipped
+from mxllm.ops.linear import _DECODE_M, linear, linear_clipped
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +42,36 @@ def test_clipped_epilogue_in_the_experts():
         assert torch.equal(moe.experts(x, ids, wgu, wdown, 7.0, w, down, 3.0)[2], linear(ref, down))
     w.requires_grad_()  # a gradient is asked: the two ops
     assert linear_clipped(x, w, 3.0) is None
+
+
+@pytest.mark.parametrize("T,N,K", [(_DECODE_M + 1, 16, 64), (47, 64, 128), (300, 48, 192), (2048, 64, 4096), (4099, 64, 320), (8192, 64, 64),
+                                   (700, 256, 256)])
+def test_side_gate(T, N, K):
+    """One launch against the product and its activation, over ragged rows, a second block of channels that is not there, K of fewer
+    stages than are in flight, strided rows and ids past the table."""
+    torch.manual_seed(T)
+    x, w = _rand(T, K + 8)[:, :K], _rand(N, K, scale=1 / K**0.5)
+    emb = _rand(100, 4 + N + 12)
+    ids = torch.randint(0, 100, (T,), device="cuda")
+    ids[0], ids[1] = -3, 1000
+    with torch.no_grad():
+        y = sublayer.side_gate(x, w, emb, ids, 4)
+    z = x.double() @ w.double().t()
+    e = emb[ids.clamp(0, 99), 4:4 + N].double()
+    ref = torch.nn.functional.gelu(z, approximate="tanh") * e
+    # the product and the result are rounded to bf16 (2^-9 each; gelu's slope is below 1.13, f32 sums are far below that)
+    bound = 2.0**-8 * (1.2 * z.abs() * e.abs() + ref.abs()) + 2.0**-16 * (1 + e.abs())
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+def test_side_gate_refusals():
+    x, w, emb = _rand(64, 64), _rand(64, 64), _rand(10, 128)
+    ids = torch.zeros(64, device="cuda", dtype=torch.long)
+    with torch.no_grad():
+        assert sublayer.side_gate(x, w, emb, ids, 64) is not None
+        assert sublayer.side_gate(x[:_DECODE_M], w, emb, ids[:_DECODE_M], 64) is None  # a decode step's
+        assert sublayer.side_gate(x, w[:24], emb, ids, 0) is None
+        assert sublayer.side_gate(x, w, emb, ids, 2) is None  # (its columns are not on 8 bytes)
+        assert sublayer.side_gate(x.float(), w.float(), emb.float(), ids, 0) is None
+        assert sublayer.side_gate(x[:, 1:33], w[:, :32], emb, ids, 0) is None
+    assert sublayer.side_gate(x, w.requires_grad_(), emb, ids, 0) is None
