@@ -1,4 +1,5 @@
-// Retention over whole prompts in chunks, f32 matrix cores (gfx950), bf16 or f32 storage.  Everything that
+// Retention over whole prompts in chunks, f32 matrix cores (gfx950), bf16 or f32 storage (bf16 heads of 64 and 128, rotated
+// whole: ends and out are retention_mfma.hip's, at half of the time).  Everything that
 // enters the recurrence - rotated q and k, scores, decay powers, state - is f32, as in retention_seq.
 // Three launches over runs of kRetChunk rows of one sequence:
 //   ends  : U = sum_j decay^(n-1-j) k_j v_j^T of every run;
@@ -358,6 +359,10 @@ __global__ void __launch_bounds__(512, DP <= 128 && EP <= 128 ? 4 : 2) retention
 
 using namespace mx;
 
+extern "C" int mx_retention_mfma_takes(const RetentionChunks* a, int f32);  // retention_mfma.hip
+extern "C" void mx_retention_mfma_ends(const RetentionChunks* a, hipStream_t stream);
+extern "C" void mx_retention_mfma_out(const RetentionChunks* a, hipStream_t stream);
+
 // -1 (nothing launched): heads wider than 256
 extern "C" int mx_retention_chunks(const RetentionChunks* pa, int f32, hipStream_t stream) {
   RetentionChunks a = *pa;
@@ -374,11 +379,14 @@ extern "C" int mx_retention_chunks(const RetentionChunks* pa, int f32, hipStream
 #define RED(TT, DP) do { if (a.E <= 64) RE(TT, DP, 64); else RE(TT, DP, 128); } while (0)
 #define ROD(TT, DP) do { if (a.E <= 64) RO(TT, DP, 64); else if (a.E <= 128) RO(TT, DP, 128); else RO(TT, DP, 256); } while (0)
 #define RT(M, TT) do { if (a.D <= 64) M(TT, 64); else if (a.D <= 128) M(TT, 128); else M(TT, 256); } while (0)
+  const bool split = mx_retention_mfma_takes(&a, f32);
   if (a.carry) {
-    if (f32) RT(RED, float); else RT(RED, uint16_t);
+    if (split) mx_retention_mfma_ends(&a, stream);
+    else if (f32) RT(RED, float); else RT(RED, uint16_t);
     retention_carry_kernel<<<dim3((a.D * a.E + 255) / 256, a.H, a.nseq), 256, 0, stream>>>(a);
   }
-  if (f32) RT(ROD, float); else RT(ROD, uint16_t);
+  if (split) mx_retention_mfma_out(&a, stream);
+  else if (f32) RT(ROD, float); else RT(ROD, uint16_t);
 #undef RT
 #undef ROD
 #undef RED
