@@ -37,13 +37,22 @@ __device__ __forceinline__ int lm_vswz(int row) {
 }
 
 // ------------------------------------------------------------------ prompts
+// What bounds it: a wave's own chain through a tile (products a quarter of the time, the softmax's instructions as much, LDS reads and
+// their waits between), two waves a SIMD.  So a row image's fragments are asked for PF - 1 steps ahead of their products and a value's
+// PV - 1 (more is level), and a tile's sources are pointers that move on by a tile, where all its rows are there, instead of 200 address
+// instructions.  32 heads, causal / a window of 1024, us: 192 + 128 dims, 2048 rows 75.6 / 62.3 -> 67.5 / 57.3, 3000 125.7 / 90.6 ->
+// 117.1 / 83.5, 1024 38.9 -> 33.8; 96 + 64 dims, 2048 rows 47.5 / 38.1 -> 41.4 / 35.2.  Row strides that spread a head's rows over the
+// L2's channels are level.
 template <int DK, int DV>
 __global__ void __launch_bounds__(256, 2) latent_flash_kernel(LatentAttn a) {
-  constexpr int BM = 128, BN = 64, CK = DK / 8, CV = DV / 8, KS = DK / 16, DB = DV / 32, G = lm_group(CK);
+  constexpr int BM = 128, BN = 64, CK = DK / 8, CV = DV / 8, KS = DK / 16, DB = DV / 32, G = lm_group(CK), PF = 3, PV = 4;
   constexpr int KT = BN * CK * 16, VT = BN * CV * 16, LK = CK / 4, LV = CV / 4;  // DMA pieces per wave
   __shared__ __attribute__((aligned(1024))) char smem[2 * (KT + VT)];
-  const int bid = blockIdx.x, h = bid % a.H;
-  const int4 sg = reinterpret_cast<const int4*>(a.blocks)[bid / a.H];
+  // Blocks come longest first.  Where all workgroups are on the chip at once, two a CU, nothing is dealt as CUs become free: those of the
+  // second round go shortest first, so that the longest shares its CU with the shortest (2048 rows of 32 heads, 192 + 128 dims, causal
+  // 77.0 -> 75.6 us, 96 + 64 dims 49.1 -> 47.5; a window of 1024 is level).
+  const int bid = blockIdx.x, h = bid % a.H, blk = bid / a.H, ahead = 256 / a.H;
+  const int4 sg = reinterpret_cast<const int4*>(a.blocks)[(int)gridDim.x <= 512 && blk >= ahead ? ahead + a.nblocks - 1 - blk : blk];
   const int64_t row0 = sg.x;
   const int S = sg.y, q0 = sg.z * BM;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -82,26 +91,48 @@ __global__ void __launch_bounds__(256, 2) latent_flash_kernel(LatentAttn a) {
   const char* vb = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(a.kv) + row0 * a.ldkv +
                                                  (int64_t)a.H * a.D + (int64_t)h * a.E);
   const int cd = a.D / 8, cr = DQ / 8, ce = a.E / 8;
+  // this lane's sources in the next whole tile, and the bytes to the tile behind it
+  const char* kp[LK];
+  uint32_t vo[LV], rot = 0;  // rot, bit i: piece i is of the rotated dims
+  const uint32_t kstep = (uint32_t)(BN * 2 * a.ldkv), rstep = (uint32_t)(BN * 2 * a.ldl);
+  auto source = [&](int i, int ln, int64_t t) __attribute__((always_inline)) {
+    const int idx = (w * LK + i) * 64 + ln, row = idx / CK, c = (idx % CK) ^ lm_swz(row, G);
+    const int64_t kr = min(t + row, (int64_t)S - 1);
+    // chunks past the head's dims repeat the first one (their query dims are zero)
+    return c < cd ? kb + kr * (a.ldkv * 2) + 16 * c : c < cr ? rb + kr * (a.ldl * 2) + 16 * (c - cd) : kb + kr * (a.ldkv * 2);
+  };
+  auto vsource = [&](int i, int ln, int last) __attribute__((always_inline)) {
+    const int idx = (w * LV + i) * 64 + ln, row = idx / CV, c = (idx % CV) ^ lm_vswz<CV>(row);
+    return (uint32_t)(min(row, last) * (int)(a.ldkv * 2) + (c < ce ? 16 * c : 0));  // columns past E are not stored
+  };
+#pragma unroll
+  for (int i = 0; i < LK; ++i) {
+    const int idx = (w * LK + i) * 64 + lane, row = idx / CK, c = (idx % CK) ^ lm_swz(row, G);
+    kp[i] = source(i, lane, (int64_t)t0 * BN);
+    rot |= (uint32_t)(c >= cd && c < cr) << i;
+  }
+#pragma unroll
+  for (int i = 0; i < LV; ++i) vo[i] = vsource(i, lane, BN - 1);
   auto issue = [&](int kt, int buf) __attribute__((always_inline)) {
-    char* kd = smem + buf * (KT + VT);
-    char* vd = kd + KT;
+    char* kd = smem + buf * (KT + VT) + w * (LK * 1024);
+    char* vd = smem + buf * (KT + VT) + KT + w * (LV * 1024);
+    const char* vt = vb + (int64_t)kt * (BN * 2) * a.ldkv;
+    if (kt * BN + BN > S) {  // a tile that the sequence ends in: rows past it repeat the last one
+      int ln = lane;
+      asm volatile("" : "+v"(ln));  // (else what this takes is kept in registers through the loop)
+#pragma unroll
+      for (int i = 0; i < LK; ++i) kp[i] = source(i, ln, (int64_t)kt * BN);
+#pragma unroll
+      for (int i = 0; i < LV; ++i) vo[i] = vsource(i, ln, S - 1 - kt * BN);
+    }
 #pragma unroll
     for (int i = 0; i < LK; ++i) {
-      const int seg = w * LK + i, idx = seg * 64 + lane, row = idx / CK;
-      const int c = (idx % CK) ^ lm_swz(row, G);
-      const int64_t kr = min(kt * BN + row, S - 1);
-      // chunks past the head's dims repeat the first one (their query dims are zero)
-      const char* p = c < cd ? kb + kr * (a.ldkv * 2) + 16 * c
-                             : c < cr ? rb + kr * (a.ldl * 2) + 16 * (c - cd) : kb + kr * (a.ldkv * 2);
-      __builtin_amdgcn_global_load_lds((lgptr_t)p, (llptr_t)(kd + seg * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((lgptr_t)kp[i], (llptr_t)(kd + i * 1024), 16, 0, 0);
+      kp[i] += rot >> i & 1 ? rstep : kstep;
     }
 #pragma unroll
     for (int i = 0; i < LV; ++i) {
-      const int seg = w * LV + i, idx = seg * 64 + lane, row = idx / CV;
-      const int c = (idx % CV) ^ lm_vswz<CV>(row);
-      const int64_t kr = min(kt * BN + row, S - 1);
-      const char* p = vb + kr * (a.ldkv * 2) + (c < ce ? 16 * c : 0);  // columns past E are not stored
-      __builtin_amdgcn_global_load_lds((lgptr_t)p, (llptr_t)(vd + seg * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((lgptr_t)(vt + vo[i]), (llptr_t)(vd + i * 1024), 16, 0, 0);
     }
   };
 
@@ -139,19 +170,20 @@ __global__ void __launch_bounds__(256, 2) latent_flash_kernel(LatentAttn a) {
       for (int n = 0; n < 2; ++n)
 #pragma unroll
         for (int j = 0; j < 16; ++j) sacc[n][j] = 0.f;
-      u16x8 kf[2][2];
+      u16x8 kf[PF][2];
       auto ld = [&](int st, u16x8(&x)[2]) __attribute__((always_inline)) {
         const int lo = (2 * st) & (G - 1), hi = (2 * st) & ~(G - 1);
         const uint32_t ad = (kq ^ (uint32_t)(16 * lo)) + bo;
         x[0] = rd128_off(ad, 16 * hi);
         x[1] = rd128_off(ad, 16 * hi + 32 * CK * 16);
       };
-      ld(0, kf[0]);
+#pragma unroll
+      for (int st = 0; st < PF - 1 && st < KS; ++st) ld(st, kf[st]);
 #pragma unroll
       for (int st = 0; st < KS; ++st) {
-        if (st + 1 < KS) ld(st + 1, kf[(st + 1) & 1]);
-        lds_wait_le(st + 1 < KS ? 2 : 0);
-        u16x8(&x)[2] = kf[st & 1];
+        if (st + PF - 1 < KS) ld(st + PF - 1, kf[(st + PF - 1) % PF]);
+        lds_wait_le(2 * (KS - 1 - st < PF - 1 ? KS - 1 - st : PF - 1));
+        u16x8(&x)[2] = kf[st % PF];
         pin(x[0]);
         pin(x[1]);
         sacc[0] = lm_mfma32(x[0], qf[st], sacc[0]);
@@ -201,28 +233,31 @@ __global__ void __launch_bounds__(256, 2) latent_flash_kernel(LatentAttn a) {
           lp[j & 3] += p;
         }
       l_i += (lp[0] + lp[1]) + (lp[2] + lp[3]);
+      // (16 keys, 32 columns) of the values at a time, PV - 1 of them asked for ahead
+      constexpr int NV = 4 * DB;
+      u16x4 fv[PV][2];
+      auto ldv = [&](int i) __attribute__((always_inline)) {
+        fv[i % PV][0] = trd_off(va[i % DB][0] + bo, 16 * (i / DB) * (CV * 16));
+        fv[i % PV][1] = trd_off(va[i % DB][1] + bo, 16 * (i / DB) * (CV * 16));
+      };
 #pragma unroll
-      for (int n = 0; n < 2; ++n)
+      for (int i = 0; i < PV - 1; ++i) ldv(i);
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          u16x8 pb;
+      for (int q = 0; q < 4; ++q) {
+        u16x8 pb;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) pb[j] = f2bf(sacc[n][8 * s2 + j]);
-          u16x4 fv[DB][2];
+        for (int j = 0; j < 8; ++j) pb[j] = f2bf(sacc[q >> 1][8 * (q & 1) + j]);
 #pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            fv[db][0] = trd_off(va[db][0] + bo, (32 * n + 16 * s2) * (CV * 16));
-            fv[db][1] = trd_off(va[db][1] + bo, (32 * n + 16 * s2) * (CV * 16));
-          }
-#pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            lds_wait_le(2 * (DB - 1 - db));
-            pin(fv[db][0]);
-            pin(fv[db][1]);
-            const u16x4 x = fv[db][0], y = fv[db][1];
-            o[db] = lm_mfma32(u16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]}, pb, o[db]);
-          }
+        for (int db = 0; db < DB; ++db) {
+          const int i = q * DB + db;
+          if (i + PV - 1 < NV) ldv(i + PV - 1);
+          lds_wait_le(2 * (NV - 1 - i < PV - 1 ? NV - 1 - i : PV - 1));
+          u16x4(&f)[2] = fv[i % PV];
+          pin(f[0]);
+          pin(f[1]);
+          o[db] = lm_mfma32(u16x8{f[0][0], f[0][1], f[0][2], f[0][3], f[1][0], f[1][1], f[1][2], f[1][3]}, pb, o[db]);
         }
+      }
     }
     lds_wait();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next tile landed
