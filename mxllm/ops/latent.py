@@ -14,6 +14,7 @@ from dataclasses import dataclass
 import torch
 
 from ._ext import native, use_native
+from .linear import linear
 
 
 @dataclass(frozen=True)
@@ -80,7 +81,7 @@ def latent_attention(q: torch.Tensor, lat: torch.Tensor, wkv: torch.Tensor, cos:
     if not use_native(q):
         return _attention_ref(q, lat, wkv, cos, sin, sink, sh, rows, cache)
     sizes = (sh.heads, sh.dim, sh.rot_dim, sh.vdim, sh.rank, sh.window, sh.scale)
-    kv = torch.nn.functional.linear(lat[:, :sh.rank], wkv)
+    kv = linear(lat[:, :sh.rank], wkv)
     return native().latent_attn(q, kv, lat, cos, sin, rows.rowinfo, rows.attn_blocks(max(rows.lens)), sink, *sizes)
 
 
