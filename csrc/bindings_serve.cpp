@@ -196,6 +196,27 @@ static at::Tensor run_gemm_tile(const at::Tensor& a, const at::Tensor& b, int gl
   return out;
 }
 
+// gemm8_rows with swiglu of the first `head` rows, gemm_tile's tile `tile` for the others
+at::Tensor gemm8_rows_rest(const at::Tensor& a, const at::Tensor& b, int64_t head, int64_t tile) {
+  MX_CHECK(a.is_cuda() && b.is_cuda() && a.device() == b.device(), "gemm8_rows_rest: GPU tensors of one device");
+  MX_CHECK(a.scalar_type() == at::kBFloat16 && b.scalar_type() == at::kBFloat16, "gemm8_rows_rest: bf16 operands");
+  MX_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == b.size(1), "gemm8_rows_rest: a [M, K], b [N, K]");
+  const int64_t M = a.size(0), K = a.size(1), N = b.size(0);
+  MX_CHECK(a.stride(1) == 1 && b.stride(1) == 1 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX && head > 0 && head < M,
+           "gemm8_rows_rest: row-major operands, rows on both sides");
+  DevGuard g(a.device());
+  auto out = at::empty({M, N / 2}, a.options());
+  const int r0 = mx_gemm8_rows(bf(a), a.stride(0), bf(b), b.stride(0), 1, bfm(out), out.stride(0), (int)head, (int)N, (int)K, 1,
+                               cur_stream());
+  MX_CHECK(r0 != -1, "gemm8_rows_rest: shape, stride or alignment not taken");
+  MX_OK(r0);
+  const int r1 = mx_gemm_tile(bf(a) + head * a.stride(0), a.stride(0), bf(b), b.stride(0), bfm(out) + head * out.stride(0),
+                              out.stride(0), (int)(M - head), (int)N, (int)K, 1, 0.f, (int)tile, 1, nullptr, cur_stream());
+  MX_CHECK(r1 != -1, "gemm8_rows_rest: shape, stride or alignment not taken");
+  MX_OK(r1);
+  return out;
+}
+
 at::Tensor gemm_tile(const at::Tensor& a, const at::Tensor& b, bool swiglu, int64_t tile, int64_t parts) {
   return run_gemm_tile(a, b, swiglu ? 1 : 0, 0.f, tile, parts);
 }
@@ -513,6 +534,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("skinny_merge_linear(Tensor ml, Tensor po, Tensor w) -> Tensor");
   m.def("gemm8_rows(Tensor a, Tensor b, bool b_kc, bool swiglu, int parts=1) -> Tensor");
   m.def("gemm_tile(Tensor a, Tensor b, bool swiglu, int tile, int parts) -> Tensor");
+  m.def("gemm8_rows_rest(Tensor a, Tensor b, int head, int tile) -> Tensor");
   m.def("gemm_tile_clipped(Tensor a, Tensor b, float limit, int tile) -> Tensor");
   m.def("gemm_tile_plan(int M, int N, int K, bool swiglu) -> int", &gemm_tile_plan);
   m.def("stream_linear(Tensor x, Tensor? delta, Tensor? gamma, float eps, Tensor w, Tensor? scale, bool swiglu) -> (Tensor, Tensor)");
@@ -541,6 +563,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("decode_attn", &decode_attn);
   m.impl("gemm8_rows", &gemm8_rows);
   m.impl("gemm_tile", &gemm_tile);
+  m.impl("gemm8_rows_rest", &gemm8_rows_rest);
   m.impl("gemm_tile_clipped", &gemm_tile_clipped);
   m.impl("stream_linear", &stream_linear);
   m.impl("stream_parts", &stream_parts);

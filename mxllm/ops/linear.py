@@ -794,8 +794,8 @@ def parts_norm(parts: torch.Tensor, h: torch.Tensor, gamma: torch.Tensor, eps: f
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None = None) -> torch.Tensor | None:
-    """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch, with
-    ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
+    """Inference: ``swiglu(linear(x, w))`` for decode-sized row counts and prompt passes as ONE launch (or two, each for
+    its rows: ``gemm.rows_head``), with ``w = [gate; up]`` [2F, K] (the SwiGLU in the epilogue of csrc/kernels/skinny_gemm.hip,
     stream_gemm.hip, gemm_tile.hip or gemm8_rows.hip, bit-identical to the GEMM + SwiGLU kernels); ``scale``: w is e4m3 codes.  None when
     the fused kernels do not take the call (the caller then runs the two ops)."""
     if SKINNY_M <= 0 or x.dim() != 2 or x.shape[1] != w.shape[1] or w.shape[0] % 16 or x.shape[0] < 1:
@@ -811,7 +811,8 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, scale: torch.Tensor | None =
         return native().skinny_linear_swiglu(x, w)
     parts = gemm.rows_gain(M, N, K, True, True)  # a prompt pass
     if parts and _plain(x, w) and gemm.rows_ok(x, w, True, True):
-        return native().gemm8_rows(x, w, True, True, parts)
+        head = gemm.rows_head(M, N, K) if parts == 1 else None
+        return native().gemm8_rows_rest(x, w, *head) if head else native().gemm8_rows(x, w, True, True, parts)
     plan = gemm.tile_plan(M, N, K, True) if M > 8 and not parts and _plain(x, w) else None
     if plan and gemm.rows_ok(x, w, True, True, 16):
         return native().gemm_tile(x, w, True, *plan)
