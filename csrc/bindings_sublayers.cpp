@@ -11,6 +11,7 @@ int mx_side_act(const void* z, int64_t ldz, const void* emb, int64_t lde, const 
                 int64_t T, int dim, hipStream_t stream);
 int mx_side_gate(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const uint16_t* emb, int64_t lde,
                  const int64_t* ids, int V, uint16_t* y, int T, int N, int K, hipStream_t stream);
+int mx_post_route(const mx::PostRoute* a, hipStream_t stream);
 int mx_clipped_glu(const void* z, int64_t ldz, void* y, int f32, int64_t T, int F, float limit, hipStream_t stream);
 int mx_latent_rows(const mx::LatentRows* a, int f32, hipStream_t stream);
 int mx_latent_attn(const mx::LatentAttn* a, int f32, hipStream_t stream);
@@ -96,6 +97,28 @@ at::Tensor post_norm(const at::Tensor& src, at::Tensor h, const at::Tensor& w, d
   a.lds = rows_of(src, "src", f, a.T, a.W);
   a.src = src.data_ptr();
   return pn_run(a, h, f);
+}
+// post_norm of prompt rows and moe_route of its copy (bf16): mx_post_route
+std::tuple<at::Tensor, at::Tensor, at::Tensor> post_route(const at::Tensor& src, at::Tensor h, const at::Tensor& w, double eps,
+                                                          const at::Tensor& m, int64_t top) {
+  DevGuard g(h.device());
+  mx::PostRoute a = {};
+  a.p = pn_args(h, w, eps);
+  a.p.mode = mx::PostNorm::kRows;
+  a.p.lds = rows_of(src, "src", false, a.p.T, a.p.W);
+  a.p.src = src.data_ptr();
+  MX_CHECK(!is_f32(m, "router") && m.dim() == 2 && m.is_contiguous() && m.size(1) == a.p.W && m.device() == h.device() &&
+               src.device() == h.device() && w.device() == h.device(), "router [E, W], all on one device");
+  MX_CHECK(m.size(0) <= 16 && top >= 1 && top <= m.size(0), "post_route: up to 16 experts");
+  a.m = (const uint16_t*)m.data_ptr(), a.E = (int)m.size(0), a.top = (int)top;
+  auto y = at::empty({a.p.T, (int64_t)a.p.W}, src.options());
+  auto ids = at::empty({a.p.T, top}, src.options().dtype(at::kInt));
+  auto wts = at::empty({a.p.T, top}, src.options().dtype(at::kFloat));
+  a.p.y = y.data_ptr(), a.ids = ids.data_ptr<int32_t>(), a.wts = wts.data_ptr<float>();
+  const int rc = mx_post_route(&a, cur_stream());
+  MX_CHECK(rc != -1, "post_route: shape, stride or alignment not taken");
+  MX_OK(rc);
+  return {y, ids, wts};
 }
 // bf16 decode rows: h += rms(P g) * w, the copy of h returned; g [T, R], P [W, R]
 at::Tensor post_side(const at::Tensor& gs, const at::Tensor& P, at::Tensor h, const at::Tensor& w, double eps) {
@@ -555,6 +578,7 @@ TORCH_LIBRARY_FRAGMENT(mxllm, m) {
   m.def("embed_norm(Tensor ids, Tensor table, Tensor w, float eps) -> (Tensor, Tensor)");
   m.def("post_side(Tensor g, Tensor P, Tensor(a!) h, Tensor w, float eps) -> Tensor");
   m.def("mix_post_norm(Tensor src, Tensor? inv, Tensor wts, Tensor? shared, Tensor(a!) h, Tensor w, float eps) -> Tensor");
+  m.def("post_route(Tensor src, Tensor(a!) h, Tensor w, float eps, Tensor m, int top) -> (Tensor, Tensor, Tensor)");
   m.def("side_act(Tensor z, Tensor emb, Tensor ids, int off) -> Tensor");
   m.def("side_gate(Tensor x, Tensor w, Tensor emb, Tensor ids, int off) -> Tensor");
   m.def("clipped_glu(Tensor z, float limit) -> Tensor");
@@ -575,6 +599,7 @@ TORCH_LIBRARY_IMPL(mxllm, CUDA, m) {
   m.impl("embed_norm", &embed_norm);
   m.impl("post_side", &post_side);
   m.impl("mix_post_norm", &mix_post_norm);
+  m.impl("post_route", &post_route);
   m.impl("side_act", &side_act);
   m.impl("side_gate", &side_gate);
   m.impl("clipped_glu", &clipped_glu);

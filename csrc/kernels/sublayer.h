@@ -44,6 +44,15 @@ struct PostDots {
   int V;
 };
 
+// prompt rows: the residual step behind the mixer and the router's choices on the new rows
+struct PostRoute {
+  PostNorm p;            // kRows; y: the copy
+  const uint16_t* m;     // [E, W]
+  int E, top;
+  int32_t* ids;          // [T, top]
+  float* wts;
+};
+
 // the shared latent and rotated key part of latent attention: rows = (position, slot or -1, sequence length, -)
 struct LatentRows {
   const void* x;         // [T, rank + rot] projections

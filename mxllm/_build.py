@@ -36,7 +36,7 @@ LIB_PATH = os.path.join(ROOT, "mxllm", "_C.so")
 COMPONENTS = {
     "serve": (os.path.join(ROOT, "mxllm", "_C_serve.so"),
               ("attn_fwd", "chunk_attn", "decode", "gemm8_rows", "gemm_tile", "hybrid", "hybrid_skinny", "latent", "latent_mfma",
-               "mingru", "moe", "moe_mfma", "moe_stream", "postnorm", "retention", "retention_chunk", "retention_mfma",
+               "mingru", "moe", "moe_mfma", "moe_stream", "post_route", "postnorm", "retention", "retention_chunk", "retention_mfma",
                "sampling", "side_gate", "skinny_gemm",
                "stream_gemm", "stream_hybrid", "stream_parts"),
               ("bindings_hybrid", "bindings_serve", "bindings_sublayers")),

@@ -338,14 +338,20 @@ class Sigusun(nn.Module):
             lat = latents[src]
         return layer.wo(lops.latent_attention(z[:, :a.q_width], lat, layer.wkv, cos, sin, layer.sink, a, rows, cache))
 
-    def _mixture(self, layer: SigusunLayer, x: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
-        m = layer.spec.moe
-        ids, wts = mops.route(x, layer.router, m.top)
+    def _mixture(self, layer: SigusunLayer, y: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
+        """Residual steps of the mixer's output ``y`` and of the feed-forward behind it."""
+        m, eps = layer.spec.moe, self.cfg.norm_eps
+        r = sops.post_route(y, h, layer.norm1, eps, layer.router, m.top)
+        if r is None:
+            x = sops.post_norm(y, h, layer.norm1, eps)
+            ids, wts = mops.route(x, layer.router, m.top)
+        else:
+            x, ids, wts = r
         shared = self._shared(layer)
         y, inv, sh = mops.experts(x, ids, layer.wgu, layer.wdown, m.limit, *(shared or ()))
         if m.shared_ff and shared is None:
             sh = layer.sdown(sops.clipped_glu(layer.sgu(x), m.shared_limit))
-        return sops.mix_post_norm(y, inv, wts, sh, h, layer.norm2, self.cfg.norm_eps)
+        return sops.mix_post_norm(y, inv, wts, sh, h, layer.norm2, eps)
 
     @staticmethod
     def _shared(layer: SigusunLayer):
@@ -387,9 +393,7 @@ class Sigusun(nn.Module):
             if r is not None:
                 h, g = r
             else:
-                x = sops.post_norm(y, h, layer.norm1, eps)
-                if layer.spec.moe:
-                    x = self._mixture(layer, x, h)
+                x = self._mixture(layer, y, h) if layer.spec.moe else sops.post_norm(y, h, layer.norm1, eps)
                 w = plain_weight(layer.side_gate)
                 g = None if w is None or hooked(layer.side_gate) else sops.side_gate(x, w, self.side_emb, ids, off)
                 if g is None:

@@ -41,6 +41,17 @@ def post_norm(src: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float) -
     return _copy(h, src.dtype)
 
 
+def post_route(src: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float, router: torch.Tensor, top: int):
+    """Prompt rows, one launch (csrc/kernels/post_route.hip): (:func:`post_norm`, the experts of each row and their weights as
+    ``moe.route`` has them); None, and nothing done, for calls that it does not take."""
+    T, W = h.shape
+    if (not FUSED or not use_native(h) or src.dtype != torch.bfloat16 or router.dtype != torch.bfloat16 or T <= _DECODE_M or W % 1024
+            or W > 4096 or router.shape[0] > 16 or not all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (h, w, router))
+            or src.stride(0) % 4 or src.data_ptr() % 8 or not _plain(src, h, router)):
+        return None
+    return native().post_route(src, h, w, eps, router, top)
+
+
 DECODE_ROWS = 64  # rows up to which the fused decode kernels run
 FUSED = os.environ.get("MXLLM_SUBLAYER_FUSED", "1") != "0"  # 0: always the parts (A/B)
 
