@@ -9,8 +9,8 @@
 //   TT 2048 x 2048 of 4096 / 2048 / 3001 / 1000 tokens 51.7 / 34.5 / 56.3* / 25.8* -> 34.5 / 19.9 / 26.5 / 12.5
 //      3072 x 2048 63.8 / 41.3 / 56.8* / 26.4* -> 47.4 / 27.0 / 37.2 / 16.8
 //   NN 4096 rows of 2048 x 2048 / 3072 x 2048 37.9 / 50.9 -> 31.6 / 43.4;  2709 rows 39.7 / 39.5 -> 24.9 / 33.8
-//      300 rows of 2048 x 2048 13.6 -> 9.3;  1000 of 4096 x 4096 41 -> 33
-// Over 27,400 random sizes with a tile that fits one turn: TT .52 of the time, NN up to a K of 8192 .79.
+//      300 rows of 2048 x 2048 13.6 -> 9.3
+// Over 27,400 random sizes with a tile that fits one turn: TT .52 of the time, NN (K up to 8192) .79.
 // Left: 0.5 us a step of 64 k where the matrix cores need 0.3 (128 x 128), the L2's rate beside 256 CUs.
 #include "gemm_tile_core.h"
 
@@ -60,13 +60,14 @@ using namespace mx;
 // The tile for a product, -1: more than one turn of the largest, or the other kernels have it faster.  Where the lines lie:
 //  * TT: always, but past 6,144 tokens with fewer than 48 tiles of 64 x 64, where the library's split of K is the quicker one for
 //    a third (.84 in the mean; 256 x 256 of 8192 22.3 -> 28.8, 512 x 512 31.7 -> 37.0; 48 tiles and more .60);
-//  * NN: a K up to 8192.  Of 6,145 to 8192 .91 in the mean, 7 of 100 by more than 3 % slower (120 tiles of 64 x 64 30.2 -> 34.0 the
-//    most); of 14336, .46 to .9 of them are (gemm8 in parts of K).  A K of 1,025 and more from 24 tiles on (16 to 23 tiles 1.1), of
-//    6,145 from 48.
+//  * NN: a K below 4096 (.79 in the mean up to 8192, 1000 rows of 4096 x 4096 41 -> 33).  From there on the library cuts K where it has
+//    few tiles, and one sum in order rounds otherwise: as near to 64 bits (1.3 % of the moments in either), but in the second optimizer
+//    step of six layers of 4096 channels, 1,328 tokens, single elements of the first moment are then .59 of its rms apart.  That is
+//    more than results may move by for 1 % of that step.  A K of 1,025 and more from 24 tiles on (16 to 23 tiles 1.1).
 extern "C" int mx_gemm_tile_form_plan(int tt, int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || N % 16 || (tt ? M % 16 != 0 : K % 64 != 0 || K > 8192)) return -1;
+  if (M <= 0 || N <= 0 || K <= 0 || N % 16 || (tt ? M % 16 != 0 : K % 64 != 0 || K >= 4096)) return -1;
   const int64_t small = gt_form_units(kGtNN[0], M, N);
-  if (tt ? K > 6144 && small < 48 : small < (K > 6144 ? 48 : K > 1024 ? 24 : 1)) return -1;
+  if (tt ? K > 6144 && small < 48 : small < (K > 1024 ? 24 : 1)) return -1;
   const float nk = (float)((K + 63) / 64), mb = (float)M * N * 2e-6f;
   float best = INFINITY;
   int tile = -1;
