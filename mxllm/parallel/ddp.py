@@ -28,6 +28,7 @@ import torch
 import torch.distributed as dist
 
 from .flat import FlatParams
+from .grad_ready import own_hook
 
 log = logging.getLogger("mxllm.ddp")
 
@@ -90,7 +91,7 @@ class DDP:
             return
         for p, bi in zip(self.flat.param_list, self._param_bucket):
             hook = self._make_hook(bi)
-            self._hooks.append(p.register_post_accumulate_grad_hook(hook))
+            self._hooks.append(own_hook(p, p.register_post_accumulate_grad_hook(hook)))
             p._mx_on_grad_ready = hook  # ops that accumulate grads themselves (fused LoRA)
 
     def set_on_ready(self, fn) -> None:

@@ -14,6 +14,8 @@ from dataclasses import dataclass
 
 import torch
 
+from .grad_ready import own_hook
+
 ALIGN = 64
 
 
@@ -82,7 +84,7 @@ class FlatParams:
         self.grad32 = self.grad_dtype == torch.float32 and pdt != torch.float32
         if self.grad32:
             for p in self._plist:
-                p.register_post_accumulate_grad_hook(self._fold_hook)
+                own_hook(p, p.register_post_accumulate_grad_hook(self._fold_hook))
         self.attach_grads()
 
     def _view(self, k: int, buf: torch.Tensor) -> torch.Tensor:

@@ -36,17 +36,24 @@ def direct_grad32(p):
     return getattr(p, "_mx_grad32", None)
 
 
-def hook_count(p) -> int:
-    return len(p._backward_hooks or ()) + len(getattr(p, "_post_accumulate_grad_hooks", None) or ())
+def own_hook(p, handle):
+    """Note ``handle``, a hook that the owner of ``p``'s gradient has put on it; returns it."""
+    p.__dict__.setdefault("_mx_own_hooks", set()).add(handle.id)
+    return handle
+
+
+def callers_hook(p) -> bool:
+    """Whether ``p`` has a hook that no owner has put there (:func:`own_hook`), whenever it was added."""
+    own = getattr(p, "_mx_own_hooks", ())
+    return any(k not in own for d in (p._backward_hooks, getattr(p, "_post_accumulate_grad_hooks", None)) for k in d or ())
 
 
 @contextlib.contextmanager
 def two_uses(params):
     """While a backward runs whose owner looks at gradients only after it: parameters used twice in the graph
-    (tied embedding and head) take the gradients of both uses in place too.  ``params``: (parameter, the
-    :func:`hook_count` its owner left it with); one that has got hooks since, which want the sum that autograd makes,
-    stays with autograd."""
-    on = [p for p, n in params if getattr(p, "_mx_no_direct", False) and hook_count(p) == n]
+    (tied embedding and head) take the gradients of both uses in place too.  One with a hook of the caller's own, which
+    wants the sum that autograd makes and may change it, stays with autograd."""
+    on = [p for p in params if getattr(p, "_mx_no_direct", False) and not callers_hook(p)]
     for p in on:
         p._mx_no_direct, p._mx_two_uses = False, True
     try:

@@ -18,7 +18,7 @@ import torch
 from .. import ops
 from ..parallel.ddp import DDP
 from ..parallel.flat import FlatParams, production_order
-from ..parallel.grad_ready import hook_count, two_uses
+from ..parallel.grad_ready import own_hook, two_uses
 from ..parallel.runtime import DistEnv
 from ..utils.profiling import range_
 
@@ -188,8 +188,8 @@ class Trainer:
             # last step's stale slot -- zero the slot first, once, right before that accumulation
             for p in self.flat.param_list:
                 if p.requires_grad:
-                    p.register_hook(_fresh_guard(p))
-        self._two_uses = [(p, hook_count(p)) for p in self.flat.param_list
+                    own_hook(p, p.register_hook(_fresh_guard(p)))
+        self._two_uses = [p for p in self.flat.param_list
                           if self.flat.device.type == "cuda" and getattr(p, "_mx_no_direct", False)]
         # ---- gradient-norm overlap: each DDP bucket's sum of squares is taken on a side
         # stream as soon as the bucket is final (after its all-reduce), under the rest of
