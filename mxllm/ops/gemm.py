@@ -242,9 +242,11 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
         (3072 x 2048 at 512 26 -> 30); in two or three parts of a K over 24,576 with the last tile's rows not mostly
         padding (57344 x 8192 at 560 524 -> 576, 700 595 -> 591, 1000 738 -> 656).
     Whole, where the library, which is tuned for round numbers of rows, falls behind between them:
-      * projections (``b_kc``) of a K of 256 to 512 from five eighths of the CUs on, behind :func:`tile_plan`: 8192 x 512 at 1400 /
-        1536 / 2048 / 2709 / 4096 33 / 28 / 23.0 / 47 / 41 -> 19 / 19 / 20.7 / 34 / 39, 4096 x 256 at 2816 / 4096 23 / 17.0 -> 15 / 16.0,
-        6144 x 384 at 1900 24 -> 17 (worst of 76 sizes 8192 x 256 at 2200 24.2 -> 24.8; with fewer tiles 4096 x 256 at 2500 13.1 -> 14.4);
+      * projections (``b_kc``) of a K of 256 to 512 and 1,024 rows on, from five eighths of the CUs to two turns: 8192 x 512 at 1400 /
+        1536 / 2048 / 2709 33 / 28 / 23.0 / 47 -> 19 / 19 / 20.7 / 34, 4096 x 256 at 2816 23 -> 15, 6144 x 384 at 1900 24 -> 17; .83 over
+        118 random sizes (worst 5888 x 448 at 1599 17.3 -> 18.7; profiles/gemm_routes/short_k.txt).  With fewer tiles 4096 x 256 at 2500 13.1 ->
+        14.4; with two turns and more 16384 x 256 at 2048 / 4096 31 / 57 -> 33 / 70; with fewer rows, which are wide outputs' or
+        padding, 65536 x 256 at 33 / 64 10.6 / 10.8 -> 12.4 / 13.0, 32768 x 512 at 300 19.5 -> 20.4;
       * projections of K 8192 and more from 500 tiles on: 8192 x 57344 at 700 559 -> 530, 2600 1916 -> 1740;
         8192 x 10240 at 3100 537 -> 456 (at 2600, 440 tiles: 317 -> 321), up to 4096 tiles and from 128 rows on (8192 x
         128256 at 64 414 -> 394 to 454, 158 540 -> 450, 1700 2650 -> 2550, 2210 3378 -> 3555, 4445 6338 -> 6656).  With a
@@ -273,7 +275,8 @@ def rows_gain(M: int, N: int, K: int, b_kc: bool, swiglu: bool = False) -> int:
         fill = 0.0 if K <= 2048 else 0.7 if turns > 2 else 0.6 if K <= 4096 else 0.63
         parts = int(tiles >= CUS * 5 // 8 and dense and useful >= fill and (K <= 8192 or N >= K))
     elif b_kc:
-        parts = int(M >= 128 and M % 256 != 0 and K >= 8192 and 500 <= tiles <= 4096 or 256 <= K <= 512 and CUS * 5 // 8 < tiles <= 4096)
+        parts = int(M >= 128 and M % 256 != 0 and K >= 8192 and 500 <= tiles <= 4096
+                    or M >= 1024 and 256 <= K <= 512 and CUS * 5 // 8 < tiles < 2 * CUS)
     else:
         parts = int(M % 256 != 0 and K >= 128 and _gains_nn(tiles) and dense)
     return parts if parts and _policy() != "0" else 0

@@ -13,6 +13,16 @@ def test_lines():
     assert all(gemm.rows_gain(*s, True) == 1 for s in on) and not any(gemm.rows_gain(*s, True) for s in off)
 
 
+def test_short_products_stay_where_measured():
+    """1,024 rows on, less than two turns; there gemm_tile has no plan that a caller would have to ask for first."""
+    off = [(33, 128256, 512), (64, 65536, 256), (127, 65536, 384), (300, 32768, 512), (1023, 16384, 512), (1024, 32768, 256),
+           (4096, 8192, 512), (2048, 16384, 256), (4096, 16384, 384)]
+    assert not any(gemm.rows_gain(*s, True) for s in off)
+    on = [(M, N, K) for M in (1024, 1100, 1700, 2500, 4090, 5900) for N in range(2048, 20000, 768) for K in (256, 320, 512)
+          if gemm.rows_gain(M, N, K, True)]
+    assert len(on) > 50 and not any(gemm.tile_plan(*s) for s in on)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(1281, 8192, 512), (2709, 4096, 256), (1700, 6144, 384)])
 def test_short_products(M, N, K):
