@@ -18,6 +18,8 @@
 // tile's two blocks are formed ahead of both their exponentials, so that the second block's products can run under the
 // first's exponentials (174 -> 149 us; an order of instructions given by sched_group_barrier 162).  Tiles that need masks are
 // the first or the last ones and have a loop of their own: the other one has no branches.
+#include <algorithm>
+
 #include "common.h"
 
 namespace mx {
@@ -242,8 +244,7 @@ attn_bwd64_kv_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
   const int grow = Hq * kRowB;  // bytes of a row of dO
   const __amdgpu_buffer_rsrc_t qrs =
       __builtin_amdgcn_make_buffer_rsrc((void*)(Q + (size_t)bh * S * kD), 0, S * kRowB, 0x00020000);
-  const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)(dO + ((size_t)b * S * Hq + h) * kD), 0, (int)((size_t)(S - 1) * grow + kRowB), 0x00020000);
+  const uint16_t* gbase = dO + ((size_t)b * S * Hq + h) * kD;
   const float* lsep = LSE + (size_t)bh * S;
   const float* ndp = NDELTA + (size_t)bh * S;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -263,7 +264,10 @@ attn_bwd64_kv_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
   float l0n, l1n, d0n, d1n;  // the lane's row of each 32: lse, -delta
   auto fetch = [&](int it) {
     const int at = (qstart * kRowB) + it * kTile + tid * 16;
-    const int ga = (qstart + it * BQ + srow) * grow + 16 * sch;
+    // (a descriptor a tile: a sequence's dO can be longer than 4 GiB)
+    const int row = qstart + it * BQ, ga = srow * grow + 16 * sch;
+    const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(gbase + (size_t)row * Hq * kD), 0, (min(S - row, BQ) - 1) * grow + kRowB, 0x00020000);
     q0s = load16(qrs, at), g0s = load16(grs, ga);
     q1s = load16(qrs, at + kTile / 2), g1s = load16(grs, ga + 32 * grow);
     const int a = min(lrow + it * BQ, S - 1), c = min(lrow + it * BQ + 32, S - 1);
@@ -361,11 +365,14 @@ attn_bwd64_kv_kernel(const uint16_t* __restrict__ Q, const uint16_t* __restrict_
 
 using namespace mx;
 
-// The arguments of mx_attn_bwd (attn_bwd.hip), which checks them; dq is not written where dqkv is given.
+// The arguments of mx_attn_bwd (attn_bwd.hip), which checks them; dq is not written where dqkv is given.  -1 (nothing launched):
+// more rows of a head, or heads, than the byte offsets of 31 bits within a head's q, k and v and a tile of dO reach.
 int mx_attn_bwd64(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* o, const uint16_t* dout,
                   const float* lse, float* delta, float* dq, float* dkp, float* dvp, int B, int Hq, int Hkv, int S, int Sk,
                   bool causal, float scale, int64_t ldo, uint16_t* dqkv, int64_t ldq, const float* cosb,
                   const float* sinb, hipStream_t stream) {
+  constexpr int kMost = (1 << 24) - 128;  // rows: x 128 B
+  if (S > kMost || Sk > kMost || Hq > (1 << 18) || (int64_t)((std::max(S, Sk) + 127) / 128) * B * Hq > INT32_MAX) return -1;
   const float sl = scale * 1.4426950408889634f;
   const int off = Sk - S, qgrid = (S + 127) / 128 * B * Hq, kgrid = (Sk + 127) / 128 * B * Hq;
 #define MX_BWD64(C)                                                                                                      \

@@ -66,3 +66,21 @@ def test_into_dqkv(gpu, S, pad):
     got = native().attn_bwd_rope(do, q, k, v, o, lse, True, scale, cos, sin, pad)
     n = (Hq + 2 * Hkv) * D
     assert got.stride() == want.stride() and torch.equal(got[:, :n], want[:, :n])
+
+
+def test_long_rows_of_many_heads(gpu):
+    """dO of one sequence past 4 GiB, which no byte offset of 32 bits reaches: the bits of calls of 32 heads each."""
+    from mxllm.ops import native
+
+    Hq, S, Sk = 128, 262_209, 40
+    torch.manual_seed(1)
+    q, o, do = (torch.randn(s, device=gpu, dtype=torch.bfloat16) for s in ((1, Hq, S, D), (1, S, Hq * D), (1, S, Hq * D)))
+    k, v = (torch.randn(1, Hq // 32, Sk, D, device=gpu, dtype=torch.bfloat16) for _ in range(2))
+    lse = torch.full((1, Hq, S), math.log2(Sk) + 1, device=gpu)
+    assert (S - 1) * Hq * D * 2 > 2**32
+    got = native().attn_bwd(do, q, k, v, o, lse, False, 0.125, 3)
+    for i in range(0, Hq, 32):
+        part = [t.view(1, S, Hq, D)[:, :, i:i + 32].reshape(1, S, 32 * D).contiguous() for t in (do, o)]
+        want = native().attn_bwd(part[0], q[:, i:i + 32], k[:, i // 32:i // 32 + 1], v[:, i // 32:i // 32 + 1], part[1],
+                                 lse[:, i:i + 32], False, 0.125, 3)
+        assert all(torch.equal(g[:, i:i + 32], w) and bool(torch.isfinite(w).all()) for g, w in zip(got, want))
