@@ -3,8 +3,9 @@
 // factor is split into three bf16 pieces whose sum it is (8 bits each of the 24), and a product of two is the six of its nine
 // products that are not below 2^-26 of it; v is bf16 as it comes.  The smaller products are added up among themselves or first, so
 // a sum has fewer roundings at its full size than the f32 instruction's: against 64 bits states are off by 1.2e-7 of their size (2.9e-7
-// there), and 0.016 % of the outputs are not the nearest bf16 (0.034 %).  (Of a factor that is infinite the pieces are NaN: what
-// was an infinite or zero product of it is NaN here.)
+// there), and 0.016 % of the outputs are not the nearest bf16 (0.034 %).  A factor that is infinite has NaN for its smaller pieces, and
+// one beside it zeros: a run's sum that is not finite is that of the largest pieces, an output row that comes out NaN is
+// formed again in f32 (rm_row), so that infinite and zero products are what they are.
 // Heads of 128, 32 of them, 2048 tokens, us: ends 62 -> 18, out 104 -> 50; heads of 64 with states and carry 72 -> 39.
 #include "gemm8_core.h"
 #include "hybrid.h"
@@ -210,10 +211,69 @@ __global__ void __launch_bounds__(4 * D, 1) retention_ends_mfma_kernel(Retention
   for (int j = 0; j < EB; ++j)
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      u[(32 * db + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * E + 32 * (eh * EB + j) + (lane & 31)] = acc[j][i] + low[j][i];
+      u[(32 * db + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3)) * E + 32 * (eh * EB + j) + (lane & 31)] =
+          acc[j][i] + (__builtin_isfinite(acc[j][i]) ? low[j][i] : 0.f);
 }
 
 // ------------------------------------------------------------------ outputs
+// Row i of a run by one wave in f32, for rows that hold what is not finite; pw: powers of the decay.  Lane l has dims and channels l and
+// l + 64.  Nothing is stored where all is NaN, as it is already.
+template <int D, int E>
+__device__ __forceinline__ void rm_row(const RetentionChunks& a, const int4& ch, int run, int h, int i, const float* pw, int lane) {
+  constexpr int ND = D / 64, NE = E / 64;
+  const int64_t HD = (int64_t)a.H * D, HE = (int64_t)a.H * E;
+  const uint16_t* x = reinterpret_cast<const uint16_t*>(a.x) + ch.x * a.ldx;
+  auto turned = [&](const uint16_t* xr, int j, float (&o)[ND]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < ND; ++n) {
+      const int d = lane + 64 * n, f = d % (D / 2);
+      const float c = a.cosb[(int64_t)(ch.z + j) * (D / 2) + f], s = a.sinb[(int64_t)(ch.z + j) * (D / 2) + f];
+      const float u = bf2f(xr[d]), v = bf2f(xr[d < D / 2 ? d + D / 2 : d - D / 2]);
+      o[n] = d < D / 2 ? u * c - v * s : u * c + v * s;
+    }
+  };
+  float q[ND], o[NE] = {};
+  turned(x + i * a.ldx + (int64_t)h * D, i, q);
+  auto lost = [&]() __attribute__((always_inline)) {  // sums that are NaN stay so
+    bool all = true;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) all = all && __builtin_isnan(o[e]);
+    return __all(all);
+  };
+  if (ch.z > 0) {
+    const float* S = a.ws + ((int64_t)run * a.H + h) * D * E + lane;
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+      for (int d = 0; d < 64; ++d) {
+        const float w = __shfl(q[n], d);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) o[e] += w * S[(64 * n + d) * E + 64 * e];
+      }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) o[e] *= pw[i + 1];
+    if (lost()) return;
+  }
+  const float ksc = 1.f / sqrtf((float)D);
+  for (int j = 0; j <= i; ++j) {
+    float k[ND], p = 0.f;
+    turned(x + j * a.ldx + HD + (int64_t)h * D, j, k);
+#pragma unroll
+    for (int n = 0; n < ND; ++n) p += q[n] * (k[n] * ksc);
+    p = wave_sum(p) * pw[i - j];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) o[e] += p * bf2f(x[j * a.ldx + 2 * HD + (int64_t)h * E + lane + 64 * e]);
+    if (lost()) return;
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) ss += o[e] * o[e];
+  const float rs = 1.f / sqrtf(wave_sum(ss) / (float)E + a.eps);
+  uint16_t* y = reinterpret_cast<uint16_t*>(a.y) + (ch.x + i) * HE + (int64_t)h * E + lane;
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+    y[64 * e] = f2bf(o[e] * rs * silu_t<uint16_t>(bf2f(x[i * a.ldx + 2 * HD + HE + (int64_t)h * E + lane + 64 * e])));
+}
+
 // A wave has 32 rows of a block of 128, transposed: scores are keys x rows and outputs channels x rows, so that a row is a lane, and
 // the scores of a tile, split, are the next product's operand where they are.  The pieces of q stay in registers (of heads of 128 some
 // in LDS: what was spilled waited, with the loads ahead of it, in every tile), k is split once for the workgroup.
@@ -504,6 +564,10 @@ __global__ void __launch_bounds__(256, 2) retention_out_mfma_kernel(RetentionChu
     const int at = i * 64 + lane, r = at / (E / 8), cc = at % (E / 8);
     if (wr + r < rows) *reinterpret_cast<u16x8*>(y + r * HE + 8 * cc) = *reinterpret_cast<const u16x8*>(gb + rm_along<E>(r, cc));
   }
+  const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));  // (lane: not kept through the kernel for this)
+  uint32_t again = (uint32_t)__ballot(wr + (ln & 31) < rows && __builtin_isnan(ss));
+  if (again) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // those rows are stored a second time
+  for (; again; again &= again - 1) rm_row<D, E>(a, ch, bl.x, h, top + __builtin_ctz(again), pw + PAD, ln);
 }
 
 }  // namespace mx

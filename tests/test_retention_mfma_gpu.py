@@ -83,3 +83,24 @@ def test_rows_do_not_see_later_ones():
     z[200:] = float("inf")
     w, _ = _run(z, decay, cos, sin, H, D, E, [n])
     assert torch.equal(w[:192], y[:192])  # (rows of one tile of 32 keys share its products of zero scores)
+
+
+@pytest.mark.parametrize("D,E", [(64, 64), (64, 128), (128, 64), (128, 128)])
+@pytest.mark.parametrize("what", ["v", "-v", "k", "q", "nan"])
+def test_not_finite(D, E, what):
+    """What is not finite in a row's outputs and in the states, and what is zero or untouched beside it, is as with the f32
+    matrix cores (whose waves take zero products of later keys too: it starts where a tile of 32 keys does)."""
+    H, lens = 3, [300, 40, 700]
+    x, decay, cos, sin = _inputs(H, D, E, lens)
+    bad = float(what.replace("-v", "-inf").replace("v", "inf").replace("k", "inf").replace("q", "inf"))
+    col = {"q": D + 5, "k": H * D + D + 5, "nan": H * D + D + 5}.get(what, 2 * H * D + E + 5)
+    for row in (64, 340 + 352):  # of the first sequence, and of the last one's second run
+        x[row, col] = bad
+    wide = torch.nn.functional.pad(x, (0, 4))[:, :-4]
+    (y, S), (y0, S0) = _run(x, decay, cos, sin, H, D, E, lens), _run(wide, decay, cos, sin, H, D, E, lens)
+    assert 0 < int((~y0.isfinite()).sum()) and int((~y0[:, :E].isfinite()).sum()) == 0  # head 1 alone
+    for a, b in ((y, y0), (S, S0)):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a == 0, b == 0)
+        assert torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()])
+        a, b = a[a.isfinite()].double(), b[b.isfinite()].double()
+        assert float((a - b).norm()) <= 2.0 ** -8 * float(b.norm())
