@@ -15,6 +15,7 @@ import os
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 _LOCK = threading.Lock()
 _LOADED = False
@@ -78,6 +79,13 @@ def use_native(t: torch.Tensor) -> bool:
     if os.environ.get("MXLLM_REFERENCE_OPS") == "1":
         return False
     return t.is_cuda
+
+
+def untransformed() -> bool:
+    """Nothing transforms or records calls at present (forward-mode levels, ``torch.func``, compilers, tracers, dispatch modes),
+    which would not see what a kernel without a batching rule or a shape function does, or keep the choice made for these sizes."""
+    return not (torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                or torch._C._functorch.maybe_current_level() is not None or torch._C._get_tracing_state() is not None)
 
 
 def rows_view(t: torch.Tensor) -> torch.Tensor:

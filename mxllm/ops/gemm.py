@@ -27,7 +27,7 @@ import os
 
 import torch
 
-from ._ext import native, use_native
+from ._ext import native, untransformed, use_native
 
 _TABLE_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tuning",
                            "gemm8_gfx950.json")
@@ -216,13 +216,14 @@ def form_plan(form: str, M: int, N: int, K: int) -> int:
 
 
 def form_mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None, beta: float = 0.0):
-    """``out = beta * out + op(a) b`` (bf16; ``out`` None: new) by that kernel; None: it does not take the call."""
+    """``out = beta * out + op(a) b`` (bf16; ``out`` None: new) by that kernel; None: it does not take the call, or the
+    backward that asks is one of many at once (``is_grads_batched``), traced or recorded."""
     if not (use_native(a) and a.is_cuda and a.device == b.device and a.dtype == b.dtype == torch.bfloat16 and a.numel() and b.numel()
             and (out is None or out.dtype == torch.bfloat16)) or asks_grad(a, b):
         return None
     M, N, K = _dims(form, a, b)
     tile = form_plan(form, M, N, K)
-    if tile < 0:
+    if tile < 0 or not untransformed():
         return None
     if out is None:
         out, beta = torch.empty(M, N, dtype=a.dtype, device=a.device), 0.0

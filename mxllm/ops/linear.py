@@ -31,11 +31,10 @@ from typing import Sequence
 
 import torch
 import torch.nn.functional as F
-from torch.autograd import forward_ad
 
 from ..parallel.grad_ready import direct_grad, direct_grad32, mark_ready
 from . import gemm
-from ._ext import native, use_native
+from ._ext import native, untransformed, use_native
 from .norm import add_rms_norm
 
 
@@ -698,11 +697,9 @@ def _decode_route(M: int, N: int, K: int) -> str:
 
 def _plain(*ts: torch.Tensor | None) -> bool:
     """Tensors that a kernel without a derivative, a batching rule or a shape function may take: no gradient is asked of
-    any, none is a subclass, autocast asks for no other type, and nothing transforms or records the call (forward-mode
-    levels, ``torch.func``, compilers, tracers, dispatch modes), which would not see what the kernel does, or keep the
-    choice made for these sizes.  Asked where a kernel would be taken only: 2 us of host time."""
-    if (torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
-            or torch._C._functorch.maybe_current_level() is not None or torch._C._get_tracing_state() is not None):
+    any, none is a subclass, autocast asks for no other type, and nothing transforms or records the call
+    (:func:`untransformed`).  Asked where a kernel would be taken only: 2 us of host time."""
+    if not untransformed():
         return False
     if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False

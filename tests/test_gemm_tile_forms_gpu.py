@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from mxllm.ops import gemm
+from mxllm.ops.linear import linear
 
 pytestmark = pytest.mark.gpu
 TILES = [(64, 64), (64, 128), (128, 128), (128, 192), (192, 128), (256, 128), (192, 192)]
@@ -69,3 +70,16 @@ def test_route(gpu, form, M, N, K):
     shifted = torch.empty(b.numel() + 4, device=gpu, dtype=torch.bfloat16)[4:].view_as(b).copy_(b)
     assert gemm.form_mm(form, a, shifted) is None
     _close(gemm.mm(form, a, shifted), want, K)
+
+
+@pytest.mark.parametrize("T,N,K", [(2048, 2048, 2048), (64, 64, 64)])
+def test_many_backwards_at_once(gpu, T, N, K):
+    """``is_grads_batched`` runs a backward under vmap, for which the kernel has no rule: such a call goes elsewhere."""
+    torch.manual_seed(T)
+    w = torch.randn(N, K, device=gpu).bfloat16().requires_grad_()
+    x, dy = torch.randn(T, K, device=gpu).bfloat16(), torch.randn(2, T, N, device=gpu).bfloat16()
+    y = linear(x, w)
+    assert gemm.form_plan("tt", N, K, T) >= 0
+    (got,) = torch.autograd.grad(y, [w], dy, is_grads_batched=True, retain_graph=True)
+    for i in range(2):
+        _close(got[i], dy[i].double().t().contiguous() @ x.double(), T)
