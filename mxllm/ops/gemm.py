@@ -187,6 +187,17 @@ def tile_plan(M: int, N: int, K: int, swiglu: bool = False) -> tuple[int, int] |
 
 
 @functools.lru_cache(maxsize=4096)
+def _rows_head(M: int, N: int, K: int) -> tuple[int, int] | None:
+    rows, cols = -(-M // 256), N // 256
+    turns = rows * cols // CUS
+    head = turns * CUS // max(cols, 1)
+    rest = M - 256 * head
+    if K > 2048 or not turns or head >= rows or (rows - head) * cols > CUS // 2 or head * cols < 0.9 * turns * CUS:
+        return None
+    plan = _tile_plan(rest, N, K, True)
+    return (256 * head, plan[0]) if plan and plan[1] == 1 else None
+
+
 def rows_head(M: int, N: int, K: int) -> tuple[int, int] | None:
     """Of a gate-up projection with SwiGLU that :func:`rows_gain` gives to gemm8 whole: (rows of its whole turns, the tile of
     csrc/kernels/gemm_tile.hip for the rows behind them), None: all rows gemm8.  Its last turn takes as long with a few tiles as with
@@ -194,14 +205,7 @@ def rows_head(M: int, N: int, K: int) -> tuple[int, int] | None:
     1500 / 2300 / 3300 / 4400 rows 88 / 88 / 90 / 137 / 188 / 240 -> 67 / 79 / 83 / 123 / 172 / 228; 16384 x 1024 at 1030 / 2560 47 / 76
     -> 36 / 72; 10240 x 2048 at 3584 129 -> 112.  Past half a turn of tiles it is level or loses (16384 x 2048 at 1800 99 -> 105, 2709
     146 -> 153), as past a K of 2048 (28672 x 4096 at 1300 / 1500 254 / 264 -> 259 / 275)."""
-    rows, cols = -(-M // 256), N // 256
-    turns = rows * cols // CUS
-    head = turns * CUS // max(cols, 1)
-    rest = M - 256 * head
-    if K > 2048 or not turns or head >= rows or (rows - head) * cols > CUS // 2 or head * cols < 0.9 * turns * CUS:
-        return None
-    plan = tile_plan(rest, N, K, True)
-    return (256 * head, plan[0]) if plan and plan[1] == 1 else None
+    return None if _policy() == "0" else _rows_head(M, N, K)
 
 
 @functools.lru_cache(maxsize=4096)

@@ -14,6 +14,16 @@ def test_lines():
     assert all(gemm.rows_head(*s) for s in on) and not any(gemm.rows_head(*s) for s in off)
 
 
+def test_lines_follow_the_switch(monkeypatch):
+    """MXLLM_GEMM8 is read at each call: what one answer was under it does not stay for the next."""
+    monkeypatch.setenv("MXLLM_GEMM8", "0")
+    assert gemm.rows_head(1309, 16384, 2048) is None
+    monkeypatch.setenv("MXLLM_GEMM8", "table")
+    assert gemm.rows_head(1309, 16384, 2048)
+    monkeypatch.setenv("MXLLM_GEMM8", "0")
+    assert gemm.rows_head(1309, 16384, 2048) is None
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,F,K", [(1025, 8192, 128), (1300, 8192, 256), (1536, 8192, 64), (2050, 8192, 192), (3073, 4096, 128), (1700, 5120, 128)])
 def test_rest_is_whole(M, F, K):
