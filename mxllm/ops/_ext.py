@@ -81,9 +81,12 @@ def use_native(t: torch.Tensor) -> bool:
     return t.is_cuda
 
 
-def untransformed() -> bool:
+def untransformed(*ts: torch.Tensor | None) -> bool:
     """Nothing transforms or records calls at present (forward-mode levels, ``torch.func``, compilers, tracers, dispatch modes),
-    which would not see what a kernel without a batching rule or a shape function does, or keep the choice made for these sizes."""
+    which would not see what a kernel without a batching rule or a shape function does, or keep the choice made for these sizes;
+    and none of ``ts`` is one of many (``is_grads_batched`` and vectorized jacobians batch without a level)."""
+    if any(t is not None and torch._C._functorch.is_legacy_batchedtensor(t) for t in ts):
+        return False
     return not (torch.compiler.is_compiling() or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
                 or torch._C._functorch.maybe_current_level() is not None or torch._C._get_tracing_state() is not None)
 

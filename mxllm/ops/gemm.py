@@ -227,7 +227,7 @@ def form_mm(form: str, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | Non
         return None
     M, N, K = _dims(form, a, b)
     tile = form_plan(form, M, N, K)
-    if tile < 0 or not untransformed():
+    if tile < 0 or not untransformed(a, b):
         return None
     if out is None:
         out, beta = torch.empty(M, N, dtype=a.dtype, device=a.device), 0.0

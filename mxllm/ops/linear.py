@@ -699,7 +699,7 @@ def _plain(*ts: torch.Tensor | None) -> bool:
     """Tensors that a kernel without a derivative, a batching rule or a shape function may take: no gradient is asked of
     any, none is a subclass, autocast asks for no other type, and nothing transforms or records the call
     (:func:`untransformed`).  Asked where a kernel would be taken only: 2 us of host time."""
-    if not untransformed():
+    if not untransformed(*ts):
         return False
     if torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") != torch.bfloat16:
         return False

@@ -428,3 +428,26 @@ def test_counted_wait_isa_check_fails_closed():
     asm = "_ZN2mx16attn_bwd8_kernelILi1EEEvv:\n s_waitcnt vmcnt(0)\n s_barrier\n.Lfunc_end0:\n"
     ok, detail = _attn_bwd_counted_wait_ok(asm)
     assert not ok and "nothing verified" in detail
+
+
+def test_a_batch_of_backwards_is_seen():
+    """``is_grads_batched`` hands a backward tensors that are many at once, with no level of ``torch.func`` behind them."""
+    from mxllm.ops._ext import untransformed
+
+    seen = []
+
+    class Double(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return 2 * x
+
+        @staticmethod
+        def backward(ctx, g):
+            seen.append(untransformed(g, None))
+            return 2 * g
+
+    x = torch.randn(3, 4, requires_grad=True)
+    y = Double.apply(x)
+    torch.autograd.grad(y, [x], torch.randn(3, 4), retain_graph=True)
+    torch.autograd.grad(y, [x], torch.randn(2, 3, 4), is_grads_batched=True)
+    assert seen == [True, False]
