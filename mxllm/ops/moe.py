@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import torch
 
+from . import sublayer
 from ._ext import native, use_native
 from .linear import linear, linear_clipped
 from .sublayer import clipped_glu
@@ -35,7 +36,7 @@ def experts(x: torch.Tensor, ids: torch.Tensor, wgu: torch.Tensor, wdown: torch.
         return y, None, sh
     sh = None
     if sgu is not None:
-        mid = linear_clipped(x, sgu, slimit)
+        mid = linear_clipped(x, sgu, slimit) if sublayer.FUSED else None
         sh = linear(clipped_glu(linear(x, sgu), slimit) if mid is None else mid, sdown)
     if use_native(x):
         bm = MFMA_ROWS if _grouped(x, wgu) else GENERIC_ROWS

@@ -53,7 +53,7 @@ def post_route(src: torch.Tensor, h: torch.Tensor, w: torch.Tensor, eps: float, 
 
 
 DECODE_ROWS = 64  # rows up to which the fused decode kernels run
-FUSED = os.environ.get("MXLLM_SUBLAYER_FUSED", "1") != "0"  # 0: always the parts (A/B)
+FUSED = os.environ.get("MXLLM_SUBLAYER_FUSED", "1") != "0"  # 0: always the parts, of prompts too (A/B)
 
 
 def fusable(x: torch.Tensor, *mats: torch.Tensor | None) -> bool:
@@ -114,7 +114,7 @@ def side_gate(x: torch.Tensor, w: torch.Tensor, emb: torch.Tensor, ids: torch.Te
     # One wave a block of 16 rows x 16 channels: past 2,048 of them the library's larger tiles are the quicker ones (with side_act,
     # us, 64 x 4096 at 8192 / 16384 rows 19.8 / 26.7 -> 15.5 / 28.5, 64 x 2048 11.5 / 16.1 -> 10.3 / 17.7; 256 x 2048 at 2048 / 3000
     # 11.3 / 11.9 -> 9.2 / 13.5).  A decode step has it behind post_dots.
-    if not use_native(x) or x.dim() != 2 or x.shape[0] <= _DECODE_M or SKINNY_M <= 0:
+    if not FUSED or not use_native(x) or x.dim() != 2 or x.shape[0] <= _DECODE_M or SKINNY_M <= 0:
         return None
     (T, K), N = x.shape, w.shape[0]
     if (N % 16 or K % 64 or off % 4 or (T + 15) // 16 * (N // 16) > 2048 or emb.dtype != torch.bfloat16 or emb.shape[1] % 4

@@ -75,3 +75,24 @@ def test_side_gate_refusals():
         assert sublayer.side_gate(x.float(), w.float(), emb.float(), ids, 0) is None
         assert sublayer.side_gate(x[:, 1:33], w[:, :32], emb, ids, 0) is None
     assert sublayer.side_gate(x, w.requires_grad_(), emb, ids, 0) is None
+
+
+def test_switched_off(monkeypatch):
+    """MXLLM_SUBLAYER_FUSED=0 is the parts in prompts too: none of the launches that join two."""
+    torch.manual_seed(0)
+    x, w, emb = _rand(128, 1024), _rand(64, 1024, scale=1 / 32), _rand(10, 64)
+    ids = torch.zeros(128, device="cuda", dtype=torch.long)
+    sgu, sdown, wgu, wdown = _rand(4096, 1024, scale=1 / 32), _rand(1024, 2048, scale=1 / 45), _rand(4, 128, 1024, scale=0.1), _rand(4, 1024, 64)
+    pick = torch.randint(0, 4, (128, 2), device="cuda", dtype=torch.int32)
+    taken = []
+    monkeypatch.setattr(moe, "linear_clipped", lambda *a: taken.append("unit") or linear_clipped(*a))
+    with torch.no_grad():
+        for fused in (True, False):
+            monkeypatch.setattr(sublayer, "FUSED", fused)
+            for name, r in (("gate", sublayer.side_gate(x, w, emb, ids, 0)),
+                            ("route", sublayer.post_route(x, x.float(), x[0].float(), 1e-6, _rand(4, 1024), 2))):
+                if r is not None:
+                    taken.append(name)
+            moe.experts(x, pick, wgu, wdown, 7.0, sgu, sdown, 3.0)
+            assert taken == (["gate", "route", "unit"] if fused else [])
+            taken.clear()
