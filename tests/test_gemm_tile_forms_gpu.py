@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from mxllm.ops import gemm
-from mxllm.ops.linear import linear
+from mxllm.ops.linear import linear, weight_grad_
 
 pytestmark = pytest.mark.gpu
 TILES = [(64, 64), (64, 128), (128, 128), (128, 192), (192, 128), (256, 128), (192, 192)]
@@ -18,7 +18,7 @@ def _operands(gpu, tt, M, N, K, pad):
     return a, b, x @ b.double()
 
 
-def _close(got, want, K, old=None):
+def _close(got, want, K):
     # f32 sums of K products of unit operands (K 2^-24 of their sizes' sum at most, far less as seen) and one rounding to bf16
     assert float((got.double() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max()) + 2.0 ** -23 * K
     assert float((got.double() - want).norm()) <= 2.0 ** -8 * float(want.norm())
@@ -30,7 +30,7 @@ def test_input_gradients(gpu, tile, K, pad):
     from mxllm.ops import native
 
     tm, tn = TILES[tile]
-    for M, N in [(1, 16), (tm, tn), (tm + 1, tn + 16), (2 * tm - 1, 3 * tn - 48)]:
+    for M, N in [(1, 16), (tm, tn), (tm + 1, tn + 16), (2 * tm - 1, 3 * tn - 48), (10 * tm - 15, 2 * tn)]:  # (bands of 8 tiles down)
         a, b, want = _operands(gpu, False, M, N, K, pad)
         out = torch.full((M, N + 8), 7.0, device=gpu).bfloat16()
         assert native().gemm_tile_form(a, b, out[:, :N], False, 0.0, tile)
@@ -44,7 +44,7 @@ def test_weight_gradients(gpu, tile, K, pad):
     from mxllm.ops import native
 
     tm, tn = TILES[tile]
-    for M, N in [(16, 16), (tm, tn), (tm + 16, tn + 48), (2 * tm - 16, 3 * tn - 16)]:
+    for M, N in [(16, 16), (tm, tn), (tm + 16, tn + 48), (2 * tm - 16, 3 * tn - 16), (10 * tm - 16, 2 * tn)]:  # (bands of 8 tiles down)
         a, b, want = _operands(gpu, True, M, N, K, pad)
         out = torch.full((M, N), float("nan"), device=gpu).bfloat16()
         assert native().gemm_tile_form(a, b, out, True, 0.0, tile)
@@ -55,9 +55,25 @@ def test_weight_gradients(gpu, tile, K, pad):
         _close(out, want + old.double(), K)
 
 
-@pytest.mark.parametrize("form,M,N,K", [("tt", 2048, 512, 1003), ("tt", 768, 768, 256), ("nn", 333, 1024, 512), ("nn", 1000, 512, 4032)])
-def test_route(gpu, form, M, N, K):
-    """``gemm.mm`` takes the kernel for the sizes of its rule, and leaves others and unaligned operands alone."""
+class _Seen:
+    """The native library, noting the tiles that gemm_tile_form ran."""
+
+    def __init__(self, ops):
+        self.ops, self.tiles = ops, []
+
+    def __getattr__(self, name):
+        return getattr(self.ops, name)
+
+    def gemm_tile_form(self, *args):
+        done = self.ops.gemm_tile_form(*args)
+        self.tiles += [args[-1]] if done else []
+        return done
+
+
+@pytest.mark.parametrize("form,M,N,K", [("tt", 2048, 512, 1003), ("tt", 768, 768, 256), ("tt", 336, 1040, 777), ("nn", 333, 1024, 512), ("nn", 1000, 512, 4032)])
+def test_route(gpu, form, M, N, K, monkeypatch):
+    """``gemm.mm`` and, of weights, ``weight_grad_`` take the kernel for the sizes of its rule, and leave others and unaligned
+    operands alone."""
     from mxllm.ops import native
 
     a, b, want = _operands(gpu, form == "tt", M, N, K, 0)
@@ -65,11 +81,20 @@ def test_route(gpu, form, M, N, K):
     assert tile >= 0 and gemm.form_plan("nn", M, N, 4096) < 0
     out = torch.empty(M, N, device=gpu, dtype=torch.bfloat16)
     assert native().gemm_tile_form(a, b, out, form == "tt", 0.0, tile)
-    assert torch.equal(gemm.mm(form, a, b), out)
     _close(out, want, K)
+    seen = _Seen(native())
+    monkeypatch.setattr(gemm, "native", lambda: seen)
+    assert torch.equal(gemm.mm(form, a, b), out) and seen.tiles == [tile]
+    if form == "tt":
+        assert torch.equal(weight_grad_(None, a, b), out) and seen.tiles == [tile] * 2
+        grad = torch.ones_like(out)
+        _close(weight_grad_(grad, a, b, beta=1.0), want + 1, K)
+        assert seen.tiles == [tile] * 3
+    seen.tiles.clear()
     shifted = torch.empty(b.numel() + 4, device=gpu, dtype=torch.bfloat16)[4:].view_as(b).copy_(b)
     assert gemm.form_mm(form, a, shifted) is None
     _close(gemm.mm(form, a, shifted), want, K)
+    assert not seen.tiles
 
 
 @pytest.mark.parametrize("T,N,K", [(2048, 2048, 2048), (64, 64, 64)])
