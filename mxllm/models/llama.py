@@ -231,7 +231,8 @@ class Llama(nn.Module):
         self.final_norm = nn.Parameter(torch.ones(cfg.hidden, dtype=dtype, device=device), requires_grad=train_base)
         if cfg.tie_embeddings:
             self.lm_head = None
-            self.tok_emb._mx_no_direct = True  # two uses (embedding + head): gradient via autograd
+            # two uses (embedding + head): autograd sums them, but in a trainer's backward (grad_ready.two_uses)
+            self.tok_emb._mx_no_direct = True
         else:
             self.lm_head = nn.Parameter(torch.empty(cfg.vocab_size, cfg.hidden, dtype=dtype, device=device),
                                         requires_grad=train_base)

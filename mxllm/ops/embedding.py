@@ -54,7 +54,7 @@ class _EmbeddingFn(torch.autograd.Function):
                 mark_ready(ctx.wp)
                 return None, None
         if ctx.nat and _SPARSE_BWD:
-            # no owner buffer (e.g. tied embeddings: autograd sums this with the head's gradient):
+            # no owner buffer (e.g. tied embeddings outside grad_ready.two_uses: autograd sums this with the head's gradient):
             # the same sorted, fixed-order row sums into a zeroed [V, H] -- deterministic, unlike
             # the atomic accumulator below (its fp32 add order varies run to run).  Each row is one fp32 sum, so
             # where autograd takes it in bf16 it is rounded into bf16 zeros at once (128256 x 2048: the

@@ -394,7 +394,7 @@ def test_fused_grad_norm_matches_full_pass(gpu, monkeypatch):
 
 @pytest.mark.parametrize("gdt,accum", [(None, 1), (None, 2), (torch.float32, 1)])
 def test_tied_fresh_gradients_bitwise(gpu, gdt, accum, monkeypatch):
-    """Tied embeddings, whose gradient autograd sums: slots that hold an earlier step's gradient give the weights of
+    """Tied embeddings, whose two uses write one slot: slots that hold an earlier step's gradient give the weights of
     slots that the optimizer clears."""
     monkeypatch.setenv("MXLLM_FUSED_GRAD_NORM", "0")  # the norm summed in one order on both sides
     cfg = _cfg().replace(tie_embeddings=True)
@@ -416,7 +416,7 @@ def test_tied_fresh_gradients_bitwise(gpu, gdt, accum, monkeypatch):
 
 
 def test_fused_grad_norm_of_tied_embeddings(gpu, monkeypatch):
-    """The default path of models with tied embeddings: their slot, which autograd sums and no GEMM's partials cover, is
+    """The default path of models with tied embeddings: their slot, which both uses write in place and no GEMM's partials cover, is
     read by the direct pass, with nothing of the values that the slots held before the step; the first step's gradients
     and norm are those of the full pass."""
     from mxllm import ops
