@@ -63,11 +63,12 @@ using namespace mx;
 //  * NN: a K below 4096 (.79 in the mean up to 8192, 1000 rows of 4096 x 4096 41 -> 33).  From there on the library cuts K where it has
 //    few tiles, and one sum in order rounds otherwise: as near to 64 bits (1.3 % of the moments in either), but in the second optimizer
 //    step of six layers of 4096 channels, 1,328 tokens, single elements of the first moment are then .59 of its rms apart.  That is
-//    more than results may move by for 1 % of that step.  A K of 1,025 and more from 24 tiles on (16 to 23 tiles 1.1).
+//    more than results may move by for 1 % of that step.  A K of 1,025 and more from 24 tiles on (16 to 23 tiles 1.1),
+//    16 channels below a K of 1024 (.66; from there on .97 and up to 1.44, 2634 rows of 16 x 3584 9.1 -> 13.1).
 extern "C" int mx_gemm_tile_form_plan(int tt, int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || N % 16 || (tt ? M % 16 != 0 : K % 64 != 0 || K >= 4096)) return -1;
   const int64_t small = gt_form_units(kGtNN[0], M, N);
-  if (tt ? K > 6144 && small < 48 : small < (K > 1024 ? 24 : 1)) return -1;
+  if (tt ? K > 6144 && small < 48 : small < (K > 1024 ? 24 : 1) || (N < 32 && K >= 1024)) return -1;
   const float nk = (float)((K + 63) / 64), mb = (float)M * N * 2e-6f;
   float best = INFINITY;
   int tile = -1;

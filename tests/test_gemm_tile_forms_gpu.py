@@ -97,6 +97,14 @@ def test_route(gpu, form, M, N, K, monkeypatch):
     assert not seen.tiles
 
 
+def test_few_channels_stay():
+    """Input gradients of 16 channels leave a K of 1024 and more to the library (the rule beside the kernel)."""
+    for M in (81, 775, 2634, 8000):
+        assert gemm.form_plan("nn", M, 16, 960) >= 0 and gemm.form_plan("tt", M // 16 * 16, 16, M) >= 0
+        assert all(gemm.form_plan("nn", M, 16, K) < 0 for K in (1024, 1088, 3584))
+    assert gemm.form_plan("nn", 2634, 32, 3584) >= 0
+
+
 @pytest.mark.parametrize("T,N,K", [(2048, 2048, 2048), (64, 64, 64)])
 def test_many_backwards_at_once(gpu, T, N, K):
     """``is_grads_batched`` runs a backward under vmap, for which the kernel has no rule: such a call goes elsewhere."""
