@@ -7,9 +7,10 @@
 // With dS^T handed from the key pass to the query pass through memory (as attn_bwd.hip does it for heads of 128) two
 // sequences of 2,048 x 32 heads took 284 us: 290 MB written by a key pass of one wave a SIMD, 201 us, read again in 74, and
 // delta.  At 64 channels a product is cheap next to that: forming S and dP once more is 8 MFMAs of 32 cycles a 32 x 32 block.
-// The two passes take 62 + 78 us (0.61 PF/s of the five products that a backward cannot do without; one sequence of 4,096
-// 480 -> 250, four of 777 113 -> 67, four of 150 24 -> 19).  What bounds them: products and exponentials of a wave follow each
-// other, and two waves a SIMD hide about half of one behind the other (matrix cores busy 45 % of the time, vector ALU 44 %).
+// The two passes take 74 + 88 us there, in a training step as those figures are (0.53 PF/s of the five products that a backward
+// cannot do without).  Replayed alone 158 to 172 from card to card; one sequence of 4,096 480 -> 275, four of 777 113 -> 78, four of 150
+// 24 -> 19.  What bounds them: products and exponentials of a wave follow each other, and two waves a SIMD hide about half of one
+// behind the other (matrix cores busy 45 % of the time, vector ALU 44 %).
 // At 128 channels the products double and the bytes of dS^T stay: there the image is the cheaper one.
 //
 // Both kernels: workgroup = 4 waves, 32 rows (queries or keys) a wave, which sit in registers as B operands of

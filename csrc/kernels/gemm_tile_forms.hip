@@ -10,7 +10,7 @@
 //      3072 x 2048 63.8 / 41.3 / 56.8* / 26.4* -> 47.4 / 27.0 / 37.2 / 16.8
 //   NN 4096 rows of 2048 x 2048 / 3072 x 2048 37.9 / 50.9 -> 31.6 / 43.4;  2709 rows 39.7 / 39.5 -> 24.9 / 33.8
 //      300 rows of 2048 x 2048 13.6 -> 9.3
-// Over 27,400 random sizes with a tile that fits one turn: TT .52 of the time, NN (K up to 8192) .79.
+// Over 480 random sizes that the plan takes: TT .38 of the time, NN .66 (profiles/gemm_routes/forms.txt).
 // Left: 0.5 us a step of 64 k where the matrix cores need 0.3 (128 x 128), the L2's rate beside 256 CUs.
 #include "gemm_tile_core.h"
 
@@ -60,7 +60,7 @@ using namespace mx;
 // The tile for a product, -1: more than one turn of the largest, or the other kernels have it faster.  Where the lines lie:
 //  * TT: always, but past 6,144 tokens with fewer than 48 tiles of 64 x 64, where the library's split of K is the quicker one for
 //    a third (.84 in the mean; 256 x 256 of 8192 22.3 -> 28.8, 512 x 512 31.7 -> 37.0; 48 tiles and more .60);
-//  * NN: a K below 4096 (.79 in the mean up to 8192, 1000 rows of 4096 x 4096 41 -> 33).  From there on the library cuts K where it has
+//  * NN: a K below 4096.  From there on this is the faster one too (1000 rows of 4096 x 4096 41 -> 33), but the library cuts K where it has
 //    few tiles, and one sum in order rounds otherwise: as near to 64 bits (1.3 % of the moments in either), but in the second optimizer
 //    step of six layers of 4096 channels, 1,328 tokens, single elements of the first moment are then .59 of its rms apart.  That is
 //    more than results may move by for 1 % of that step.  A K of 1,025 and more from 24 tiles on (16 to 23 tiles 1.1),

@@ -15,7 +15,8 @@ constexpr int kPrRows = 8;  // rows of a workgroup, one a wave
 // barrier: 128 KB a workgroup for W 4096, which is little beside the rows (the second embedding's
 // matrices, eight times as much, are not: a kernel that had them as well behind the experts' mix was level).  Two launches -> one, replayed,
 // us, 33 / 300 / 1000 / 2048 / 4096 / 8192 rows: W 4096 14.3 / 15.5 / 19.9 / 27.0 / 41.7 / 81.9 -> 11.5 / 12.2 / 14.7 / 19.4 / 36.8 / 75.0,
-// 2048 13.5 / 14.3 / 16.4 / 19.5 / 27.6 / 51.3 -> 7.3 / 7.8 / 8.8 / 11.4 / 19.8 / 35.1.  All of W 4096's stream asked for at once spills
+// 2048 13.5 / 14.3 / 16.4 / 19.5 / 27.6 / 51.3 -> 7.3 / 7.8 / 8.8 / 11.4 / 19.8 / 35.1.  In a prompt pass of 2048 rows of W 4096, whose
+// rows come from further away, 18 + 12 -> 26.5.  All of W 4096's stream asked for at once spills
 // (2048 rows 24.4).
 template <int NIT>
 __global__ void __launch_bounds__(512, 4) post_route_kernel(PostRoute a) {

@@ -10,7 +10,7 @@ __device__ __forceinline__ void sg_vm_wait() { asm volatile("s_waitcnt vmcnt(%0)
 
 // What bounds it: 64 k of a wave, which wait for their DMA, their LDS reads and their products behind one another; the bytes (2048
 // rows of 4096: 16 MB, 2.7 us from memory) come by the side.  The library's product, which has 128 tiles there, takes 19.9 us in a
-// prompt pass, and side_act 4.8.  So tiles are as small as a wave's block, one wave each: nothing is shared, there is no barrier,
+// prompt pass, and side_act 4.8 (this one 13.5).  So tiles are as small as a wave's block, one wave each: nothing is shared, there is no barrier,
 // and S stages of 64 k (a row's 128 bytes are a line) are on their way.  K stays in order, as the library has it: the bits are the
 // same wherever that does not cut K.  With side_act, replayed, 65 / 512 / 2048 / 4096 / 8192 rows of 64 x 4096, us: 12.7 / 13.2 /
 // 18.0 / 19.3 / 19.8 -> 7.9 / 8.6 / 9.3 / 12.0 / 15.5; 64 x 2048 9.7 / 10.5 / 11.4 / 11.9 / 11.5 -> 5.0 / 5.6 / 6.3 / 7.8 / 10.3; 8
